@@ -112,3 +112,21 @@ def ptr(t):
 
 def stream_of(t):
     return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+
+
+class _Native:
+    """The binding in ``_native.so``, loaded at the first use of one of its functions."""
+
+    def __getattr__(self, name):
+        load()   # raises when the library has not been built
+        try:
+            from . import _native
+        except ImportError as e:
+            raise RuntimeError("medvision_amd/_native.so is missing or does not fit this PyTorch: build it with "
+                               f"`python -m medvision_amd.build` ({e})") from e
+        fn = getattr(_native, name)
+        setattr(self, name, fn)   # found without __getattr__ from now on
+        return fn
+
+
+native = _Native()
