@@ -261,6 +261,13 @@ int mv_deform_conv_3d(const void *input, const void *offset, const void *weight,
 int mv_deform_conv_2d(const void *input, const void *offset, const void *weight, const void *bias,
                       void *output, const mv_dcn2d_shape *shape, int dtype, int order, void *stream);
 
+/* ---- small host arrays --------------------------------------------------------------------------
+ * Copies `bytes` (whole 4-byte words, at most MV_UPLOAD_MAX_BYTES) from host to device memory as
+ * kernel arguments: asynchronous on the stream, `host` may be reused as soon as the call returns.
+ * For rois and control grids (aug_cuda/aug_spatial.py builds them on the host for every call).       */
+#define MV_UPLOAD_MAX_BYTES ((size_t)16 << 10)
+int mv_upload(const void *host, void *device, size_t bytes, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -73,6 +73,7 @@ SIGNATURES = {
     "mv_deform_warp_3d": (_i, [_p, _p, _p, _i] + [_i] * 5 + [_i, _p]),
     "mv_deform_conv_3d": (_i, [_p] * 6 + [_i, _i, _p]),
     "mv_deform_conv_2d": (_i, [_p] * 6 + [_i, _i, _p]),
+    "mv_upload": (_i, [_p, _p, _sz, _p]),
 }
 
 _lib = None

@@ -16,17 +16,8 @@ import time
 from datetime import datetime
 
 import numpy as np
-import torch
 
-
-def _peak_mib():
-    """Peak of allocated GPU memory in MiB, as ``torch.cuda.max_memory_allocated`` reports it; read
-    from the nested statistics (that call flattens the whole tree first, tens of microseconds per
-    stage)."""
-    if not torch.cuda.is_available():
-        return 0.0
-    stats = torch.cuda.memory_stats_as_nested_dict()     # {} before the first GPU call
-    return stats.get("allocated_bytes", {}).get("all", {}).get("peak", 0) / 2 ** 20
+from .._lib import native
 
 
 class CudaAugBase:
@@ -131,10 +122,9 @@ class CudaAugBase:
             self._apply_all(result)
         for key in ('history', 'time', 'memory'):
             result.setdefault(key, [])
-        peak = _peak_mib()
         result['history'].append(self.name)
-        result['memory'].append(f"{self.name}-{peak:.02f}MB")
-        started = datetime.fromtimestamp(tic).strftime('%H:%M:%S.%f')
+        result['memory'].append(f"{self.name}-{native.peak_mib():.02f}MB")
+        started = datetime.fromtimestamp(tic).time().isoformat('microseconds')
         result['time'].append(f"{self.name}-{started}-{time.time() - tic:.03f}s")
         return result
 

@@ -22,16 +22,13 @@ def _table(v, cols):
 def window_rois(dim, start_xyz, end_xyz, scales=1.0, shifts=0.0, rotate=0.0, index=None):
     """[n, 6] (2-D: b, cx, cy, w, h, angle) or [n, 10] (3-D: b, cx, cy, cz, w, h, d, 0, 0, angle)
     float32 rows.  Every argument is one value, one row, or n rows; ``index`` defaults to 0..n-1."""
-    cols = {"start": dim, "end": dim, "scales": dim, "shifts": dim, "rotate": 1}
-    tab = {k: _table(v, cols[k]) for k, v in (("start", start_xyz), ("end", end_xyz),
-                                              ("scales", scales), ("shifts", shifts), ("rotate", rotate))}
-    n = max([t.shape[0] for t in tab.values()] + ([len(index)] if index is not None else []))
-    start, end, scales, shifts, rotate = [np.broadcast_to(tab[k], (n, cols[k])) for k in cols]
-    centre = (start + end) / np.float32(2)
+    start, end, scales, shifts = [_table(v, dim) for v in (start_xyz, end_xyz, scales, shifts)]
+    rotate = _table(rotate, 1)
+    n = max(len(start), len(end), len(scales), len(shifts), len(rotate), len(index) if index is not None else 0)
     extent = end - start
     rois = np.zeros((n, 2 * dim + (2 if dim == 2 else 4)), dtype=np.float32)
-    rois[:, 0] = np.arange(n, dtype=np.float32) if index is None else np.asarray(index, dtype=np.float32)
-    rois[:, 1:1 + dim] = centre - extent * shifts / scales
+    rois[:, 0] = np.arange(n, dtype=np.float32) if index is None else index
+    rois[:, 1:1 + dim] = (start + end) / np.float32(2) - extent * shifts / scales
     rois[:, 1 + dim:1 + 2 * dim] = extent / scales
     rois[:, -1:] = rotate          # 3-D: the two leading angles (about x and y) stay 0
     return rois

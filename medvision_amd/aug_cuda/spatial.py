@@ -16,6 +16,7 @@ import numpy as np
 import torch
 
 from ..ops.cuda_fun_tools import affine_2d, affine_3d, apply_offset_2d, apply_offset_3d
+from .._lib import native
 from . import geometry
 from .base import BatchCudaAugBase, CudaAugBase
 
@@ -42,7 +43,7 @@ class _Resampler:
         fn = affine_2d if self.dim == 2 else affine_3d
         rois = getattr(self, '_device_rois', None)
         if rois is None or rois.device != tensor.device:
-            rois = self._device_rois = torch.from_numpy(self._rois()).to(tensor.device)
+            rois = self._device_rois = native.upload(self._rois(), tensor.device)
         batch = tensor if self.batched else tensor.unsqueeze(0)
         out = fn(batch, rois, tuple(int(v) for v in self._out_size()), 1.0, sampling_ratio, True, order)
         return out if self.batched else out.squeeze(0)
@@ -423,13 +424,13 @@ class CudaRandomElasticDeformation(CudaAugBase):
         """[dim, *image_shape] displacements (z, y, x components) -- the batch stage: [batch, dim,
         *image_shape] -- cached per draw."""
         if self.tmp_params is None:
-            coarse = torch.from_numpy(self.params if self.batched else self.params[None])
-            grid = coarse.permute(0, self.dim + 1, *range(1, self.dim + 1)) / 2
-            shape_xyz = list(grid.shape[2:])[::-1]
+            coarse = self.params if self.batched else self.params[None]
+            grid = np.moveaxis(coarse, -1, 1) / 2          # [batch, component, *grid]
+            shape_xyz = grid.shape[2:][::-1]
             roi = geometry.window_rois(self.dim, [1.5] * self.dim, [s - 1.5 for s in shape_xyz],
                                        index=np.arange(grid.shape[0]))
             fn = affine_2d if self.dim == 2 else affine_3d
-            dense = fn(grid.to(device).contiguous(), torch.from_numpy(roi).to(device),
+            dense = fn(native.upload(grid, device), native.upload(roi, device),
                        tuple(self.image_shape), 1, 1, True, self.INTER_ORDER)
             self.tmp_params = dense if self.batched else dense.squeeze(0)
         return self.tmp_params

@@ -8,7 +8,10 @@
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/extension.h>
 
+#include <c10/hip/HIPCachingAllocator.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <pybind11/numpy.h>
 
 #include <optional>
 
@@ -457,6 +460,29 @@ Tensor deform_warp(const Tensor &img_in, const Tensor &offset_in, int order) {
   return out;
 }
 
+// ---- helpers of the augmentation stages ----------------------------------------------------------------------------
+// A host array (rois, a control grid) on the device, without waiting for what is queued there.
+Tensor upload(const py::array_t<float, py::array::c_style | py::array::forcecast> &array, const at::Device &device) {
+  const std::vector<int64_t> shape(array.shape(), array.shape() + array.ndim());
+  const size_t bytes = static_cast<size_t>(array.size()) * sizeof(float);
+  const float *data = array.data();
+  const py::gil_scoped_release no_gil;
+  const at::NoGradGuard no_grad;
+  if (!device.is_cuda() || bytes > MV_UPLOAD_MAX_BYTES)
+    return at::from_blob(const_cast<float *>(data), shape, at::kFloat).to(device, at::kFloat, false, true);
+  const c10::DeviceGuard guard(device);
+  const Tensor out = at::empty(shape, at::TensorOptions().dtype(at::kFloat).device(device));
+  check(mv_upload(data, ptr(out), bytes, stream_of(out)));
+  return out;
+}
+
+// torch.cuda.max_memory_allocated() in MiB, without building the whole tree of statistics (18 us)
+double peak_mib() {
+  auto *allocator = c10::hip::HIPCachingAllocator::get();
+  if (!allocator->initialized()) return 0.0;
+  return allocator->getDeviceStats(c10::hip::current_device()).allocated_bytes[0].peak / 1048576.0;
+}
+
 }  // namespace
 
 PYBIND11_MODULE(_native, m) {
@@ -465,4 +491,6 @@ PYBIND11_MODULE(_native, m) {
   m.def("modulated_deform_conv", &modulated_deform_conv);
   m.def("deform_conv", &deform_conv);
   m.def("deform_warp", &deform_warp);
+  m.def("upload", &upload);
+  m.def("peak_mib", &peak_mib);
 }
