@@ -83,7 +83,8 @@ struct TilePlan {            // 352 bytes
   int roi;                   // roi index
   int batch;                 // feature-map index of the roi
   unsigned vol_lo, vol_hi;   // byte offset of the item's (image, channel) volume in the feature tensor
-  int pad2[3];
+  int shift_b;               // bytes copied ahead of the box in every row (rows that are not aligned)
+  int pad2[2];
   // dword 80: box-relative limits of a clipped box as fp32: coordinates clamp to [0, cmax], the
   // low tap index is at most top = max(n - 2, 0)
   float cmaxf[4], topf[4];
@@ -108,13 +109,14 @@ struct PlanShape {
   int tiles_x, tiles_y, tiles_z;  // spatial tiles per roi
   int tx, ty, tz;                 // tile extent in output voxels
   int vec;                        // elements per aligned 16-byte group (0: rows are not aligned)
+  int loose_vec;                  // elements per 16-byte group of rows that are not aligned (0: rows are aligned, or copied element by element)
   int cap;                        // LDS capacity in elements
   int threads, max_items;         // workgroup size, 16-byte groups one lane holds in registers
   int es;                         // bytes per element
   FastDiv by_per_roi, by_tiles_x, by_tiles_y, by_total, by_slots;
   int halo_lo, halo_hi;           // voxels needed below / above the cell of a sample: 0 / 1, order 3: 1 / 2
   int grids;                      // 1: the kernel takes every sample of a bin (else items with grids above 1 are void)
-  int flat_axis;                  // 1: the middle axis has one cell sampled once whatever the ratio (images as volumes of rows)
+  int flat_axis;                  // 1: the middle axis has one cell sampled once whatever the ratio and the rois are those of images (images as volumes of rows)
   unsigned warm_groups;           // 16-byte groups of the input to pull into the caches during planning (0: none)
   int pad_slices;                 // 1: LDS slices of a box start 32 bytes past a multiple of 128
 };
@@ -145,11 +147,28 @@ __device__ inline void plan_item_lanes(const float *__restrict__ rois, const Roi
   const unsigned chan = p.C > 1 ? ps.by_total.div(it) : 0u;
   const unsigned idx = it - chan * total, n = ps.by_per_roi.div(idx), tile = idx - n * per_roi;
   const int nd = p.ndim, is3d = nd == 3, ax = a < 3 ? a : 0;
-  const float *roi = rois + static_cast<long>(n) * roi_columns(nd, p.rotated);
 
-  // ---- angle `ax`, axis `ax` of the roi -------------------------------------------------------
-  double sn, cs;
-  roi_trig(roi, p, ax, sn, cs);
+  // ---- the roi: centre and extent (plain boxes: corners) of axis `ax`, angle `ax` ---------------
+  // An image resampled as a volume of rows hands in the image's rois: (x, y, w, h, theta) stands for the
+  // volume roi (x, y', y, w, h', h, 0, -theta, 0) whose middle axis has one cell that samples row 0 exactly.
+  const float *roi = rois + static_cast<long>(n) * roi_columns(ps.flat_axis ? 2 : nd, p.rotated);
+  const int rd = ps.flat_axis ? 2 : nd, rax = ps.flat_axis ? (ax == 2 ? 1 : 0) : (ax < nd ? ax : 0);
+  float first_of = roi[1 + rax], second_of = roi[1 + rd + rax], angle = 0.f;
+  if (p.rotated) angle = roi[1 + 2 * rd + (ps.flat_axis || nd == 2 ? 0 : ax)];
+  if (ps.flat_axis) {
+    const float scale = static_cast<float>(p.scale);
+    if (ax == 1) {
+      first_of = p.rotated ? (p.aligned ? 0.5f / scale : 0.f) : -0.5f / scale;
+      second_of = p.rotated ? 1.f / scale : 0.5f / scale;
+      angle = -angle;
+    } else {
+      angle = 0.f;
+    }
+  } else if (nd == 2 && ax > 0) {
+    angle = 0.f;
+  }
+  double sn = 0.0, cs = 1.0;
+  if (p.rotated) sincos_moderate(static_cast<double>(angle), sn, cs);
   const int cells_all[3] = {p.ow, p.oh, p.od}, size_all[3] = {p.W, p.H, p.D}, ext_all[3] = {ps.tx, ps.ty, ps.tz};
   const int out_cells = ax == 0 ? cells_all[0] : (ax == 1 ? cells_all[1] : cells_all[2]);
   const int S = ax == 0 ? size_all[0] : (ax == 1 ? size_all[1] : size_all[2]);
@@ -161,12 +180,12 @@ __device__ inline void plan_item_lanes(const float *__restrict__ rois, const Roi
     const double sc = p.scale;
     double ext;
     if (p.rotated) {
-      ext = static_cast<double>(roi[1 + nd + ax]) * sc;
+      ext = static_cast<double>(second_of) * sc;
       if (!p.aligned) ext = fmax(ext, 1.0);
-      centre = static_cast<double>(roi[1 + ax]) * sc - (p.aligned ? 0.5 : 0.0);
+      centre = static_cast<double>(first_of) * sc - (p.aligned ? 0.5 : 0.0);
       start = -ext / 2.0;
     } else {
-      const double lo = static_cast<double>(roi[1 + ax]) * sc, hi = static_cast<double>(roi[1 + nd + ax]) * sc;
+      const double lo = static_cast<double>(first_of) * sc, hi = static_cast<double>(second_of) * sc;
       ext = fmax(hi - lo, 1.0);
       start = lo;
     }
@@ -238,16 +257,33 @@ __device__ inline void plan_item_lanes(const float *__restrict__ rois, const Roi
   const int ty0 = lane_get(t0, base + 1), tz0 = lane_get(t0, base + 2);
   const int any_empty = lane_get(empty, base) | lane_get(empty, base + 1) | lane_get(empty, base + 2);
   const int any_clip = lane_get(clipped, base) | lane_get(clipped, base + 1) | lane_get(clipped, base + 2);
-  // LDS row pitch: the row's 16-byte groups, or (unaligned rows) the row plus one finite pad
-  const int groups = ps.vec > 0 ? n0 / ps.vec : 0;
-  const int pitch = ps.vec > 0 ? n0 : n0 + 1;
+  // LDS row pitch: the row's 16-byte groups, or the row plus one finite pad.  Rows that start at any element
+  // (row length no multiple of a group, or an unaligned tensor) are copied as groups too: the first group starts
+  // `shift` elements before the box so that the last one ends inside the volume's row, and the LDS tile is read
+  // from `shift` on.  (Memory takes 16-byte loads at any element; one element at a time such boxes took
+  // 2 - 3 times as long as aligned ones.)
   const int es = ps.es;
+  int groups = ps.vec > 0 ? n0 / ps.vec : 0, shift = 0;
+  int pitch = ps.vec > 0 ? n0 : n0 + 1;
   // LDS elements from slice to slice.  The eight taps of a wavefront's 64 samples fall on rows and
   // slices all over the box; with slices 32 bytes past a multiple of 128 a model of the 32 banks
   // counts 3.6 clocks per 2-byte tap read instead of 4.2 and 4.5 instead of 5.1 per 4-byte one (rotations
   // of up to 30 degrees about three axes); other remainders and odd row pitches gave less.
-  int slice_e = n1 * pitch;
-  if (ps.pad_slices && n2 > 1) slice_e = (((slice_e * es - 32 + 127) & ~127) + 32) / es;
+  auto slice_of = [&](int row_pitch) {
+    const int e = n1 * row_pitch;
+    return ps.pad_slices && n2 > 1 ? (((e * es - 32 + 127) & ~127) + 32) / es : e;
+  };
+  int slice_e = slice_of(pitch);
+  if (ps.loose_vec > 0 && n0 > 1) {
+    const int lv = ps.loose_vec == 8 ? 3 : 2, g = (n0 + ps.loose_vec - 1) >> lv, wide = g << lv;
+    const int wide_slice = slice_of(wide);
+    if (wide <= p.W && static_cast<long>(n2) * wide_slice <= ps.cap) {
+      groups = g;
+      pitch = wide;
+      slice_e = wide_slice;
+      shift = max(l0 + wide - p.W, 0);
+    }
+  }
   const long hw = static_cast<long>(p.H) * p.W;
   const long vol = (static_cast<long>(batch < 0 ? 0 : batch) * p.C + chan) * (hw * p.D) * es;
   int span = 0;
@@ -257,7 +293,7 @@ __device__ inline void plan_item_lanes(const float *__restrict__ rois, const Roi
     } else {
       // register staging: a pass copies `span` whole z-slices, one 16-byte group per lane
       int passes = 0;
-      if (ps.vec > 0) {
+      if (groups > 0) {
         const int per_slice = n1 * groups;   // small integers: the float quotients below are exact
         const int sp = min(static_cast<int>(static_cast<float>(ps.threads) / static_cast<float>(per_slice)), n2);
         if (sp >= 1) {
@@ -271,11 +307,12 @@ __device__ inline void plan_item_lanes(const float *__restrict__ rois, const Roi
       else if (!fits) mode = 2;
       else mode = any_clip ? 1 : 3;
       const int rp = span * n1;
-      const long src = vol + ((static_cast<long>(l2) * p.H + l1) * p.W + l0) * es;
+      const long src = vol + ((static_cast<long>(l2) * p.H + l1) * p.W + l0 - shift) * es;
       dst->mode = mode;
       dst->passes = passes;
       dst->src_lo = static_cast<unsigned>(src); dst->src_hi = static_cast<unsigned>(src >> 32);
-      dst->extent = static_cast<int>((((n2 - 1) * hw + static_cast<long>(n1 - 1) * p.W + n0) * es));
+      dst->extent = static_cast<int>((((n2 - 1) * hw + static_cast<long>(n1 - 1) * p.W + (groups > 0 ? pitch : n0)) * es));
+      dst->shift_b = shift * es;
       dst->stride = static_cast<int>(span * hw * es);
       dst->inv_groups = 1.0f / static_cast<float>(max(groups, 1));
       dst->inv_rows = 1.0f / static_cast<float>(n1);
@@ -507,6 +544,7 @@ template <> __device__ __forceinline__ const float *plan_map<float>(const TilePl
 template <> __device__ __forceinline__ const double *plan_map<double>(const TilePlan *r) { return r->map; }
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4_any __attribute__((ext_vector_type(4), aligned(2)));   // at any 16-bit element
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 // One element through a buffer descriptor: offsets beyond the buffer drop the store, so lanes
@@ -869,6 +907,7 @@ __global__ __launch_bounds__(THREADS, 4) void roi_resample_kernel(
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     const f32x4 lim4 = *reinterpret_cast<const f32x4 *>(rec->cmaxf), top4 = *reinterpret_cast<const f32x4 *>(rec->topf);
     const bool staged = (mode & 1) != 0;
+    const T *const box = tile + __builtin_amdgcn_readfirstlane(rec->shift_b) / ES;   // the box's first voxel in LDS
 
     // ---- A: the box into LDS ---------------------------------------------------------------
     // All loads issued for this item have to be back; waiting here on every path (vmcnt(0), other
@@ -891,18 +930,17 @@ __global__ __launch_bounds__(THREADS, 4) void roi_resample_kernel(
       } else {
         // boxes with very long rows, very many slices or unaligned rows: straight from global memory
         const int bx = plan_scalar(&rec->n[0]), by = plan_scalar(&rec->n[1]), bz = plan_scalar(&rec->n[2]);
-        const int vec = ps.vec, pitch = vec > 0 ? bx : bx + 1, rows = by * bz, gap = cpy.y / ES;
+        const int groups = plan_scalar(&rec->groups), vec = 16 / ES, pitch = g.x / ES, rows = by * bz, gap = cpy.y / ES;
         const T *corner = reinterpret_cast<const T *>(
             reinterpret_cast<const char *>(feat) + plan.u64(MV_PLAN_DW(src_lo)));
         const float inv_by = rec->inv_rows;
-        if (vec > 0) {
-          const int groups = bx / vec;
+        if (groups > 0) {
           const float inv_groups = rec->inv_groups;
           for (int i = tid; i < rows * groups; i += THREADS) {
             const int r = div_small(i, inv_groups), gi = i - r * groups;
             const int zz = div_small(r, inv_by), yy = r - zz * by;
             *reinterpret_cast<u32x4 *>(tile + r * pitch + zz * gap + gi * vec) =
-                *reinterpret_cast<const u32x4 *>(corner + (static_cast<long>(zz) * H + yy) * W + gi * vec);
+                *reinterpret_cast<const u32x4_any *>(corner + (static_cast<long>(zz) * H + yy) * W + gi * vec);
           }
         } else {
           int lpr = 1;
@@ -999,21 +1037,21 @@ __global__ __launch_bounds__(THREADS, 4) void roi_resample_kernel(
           const long hw = static_cast<long>(H) * W;
           bins(std::true_type{}, src, W, hw, H > 1 ? W : 0, p.D > 1 ? hw : 0);
         } else {
-          bins(std::false_type{}, tile, g.x / ES, g.y / ES, g.z / ES, g.w / ES);
+          bins(std::false_type{}, box, g.x / ES, g.y / ES, g.z / ES, g.w / ES);
         }
       } else if (mode == 3 && sizeof(CT) == 4) {
         if constexpr (sizeof(CT) == 4)
-          interior_column<T, ORDER, ZPL>(tile, o, b[0], b[1], b[2], st[0], st[1], st[2], g, before);
+          interior_column<T, ORDER, ZPL>(box, o, b[0], b[1], b[2], st[0], st[1], st[2], g, before);
       } else if (mode == 1 && sizeof(CT) == 4) {
         if constexpr (sizeof(CT) == 4) {
           const float cmax[3] = {lim4.x, lim4.y, lim4.z}, top[3] = {top4.x, top4.y, top4.z};
-          clipped_column<T, ORDER, ZPL>(tile, o, b[0], b[1], b[2], st[0], st[1], st[2], g, cmax, top, before);
+          clipped_column<T, ORDER, ZPL>(box, o, b[0], b[1], b[2], st[0], st[1], st[2], g, cmax, top, before);
         }
       } else {
         const int pitch = g.x / ES, slice = g.y / ES, dy = g.z / ES, dz = g.w / ES;
         BoxLimits<CT> lim;
         if (mode == 3) {
-          staged_column<T, CT, true, ORDER, ZPL>(tile, o, b[0], b[1], b[2], st[0], st[1], st[2], lim, pitch, slice, dy, dz, before);
+          staged_column<T, CT, true, ORDER, ZPL>(box, o, b[0], b[1], b[2], st[0], st[1], st[2], lim, pitch, slice, dy, dz, before);
         } else {
           const int size[3] = {W, H, p.D};
 #pragma unroll
@@ -1034,7 +1072,7 @@ __global__ __launch_bounds__(THREADS, 4) void roi_resample_kernel(
             const long dzw = p.D > 1 ? hw : 0;
             staged_column<T, CT, false, ORDER, ZPL, true>(src, o, b[0], b[1], b[2], st[0], st[1], st[2], lim, W, hw, dyw, dzw, before);
           } else {
-            staged_column<T, CT, false, ORDER, ZPL>(tile, o, b[0], b[1], b[2], st[0], st[1], st[2], lim, pitch, slice, dy, dz, before);
+            staged_column<T, CT, false, ORDER, ZPL>(box, o, b[0], b[1], b[2], st[0], st[1], st[2], lim, pitch, slice, dy, dz, before);
           }
         }
       }
@@ -1081,6 +1119,195 @@ __global__ __launch_bounds__(THREADS, 4) void roi_resample_kernel(
   __builtin_amdgcn_s_waitcnt(0);
   MV_TL(10);
 #endif
+}
+
+// ---- taps straight from the caches -----------------------------------------------------------------
+// The persistent kernel above pays ~18 us per launch whatever the size (plans of up to 16 items on one
+// wavefront, a box through registers and LDS, one item after the other).  Small problems run this kernel instead: a
+// workgroup takes 1 / PARTS of one tile, and its lanes read their taps from the L1 / L2, the two x taps of
+// a row in one load.  Items, plans, coordinates (relative to the same box origin), tap rules and blends are those
+// of the kernel above, so the outputs are the same bit for bit.
+// The two x taps of a row: elements `off` and `off` + 1 (bytes) of the buffer.
+template <typename T> struct RowPair { T a, b; };
+template <typename T> __device__ __forceinline__ RowPair<T> load_row_pair(__amdgpu_buffer_rsrc_t rsrc, unsigned off) {
+  static_assert(sizeof(T) == 2 || sizeof(T) == 4, "16- and 32-bit elements");
+  RowPair<T> v;
+  if constexpr (sizeof(T) == 2) {
+    const unsigned w = __builtin_amdgcn_raw_buffer_load_b32(rsrc, off, 0, 0);
+    __builtin_memcpy(&v, &w, 4);
+  } else {
+    const auto w = __builtin_amdgcn_raw_buffer_load_b64(rsrc, off, 0, 0);
+    __builtin_memcpy(&v, &w, 8);
+  }
+  return v;
+}
+template <typename T> __device__ __forceinline__ T load_element(__amdgpu_buffer_rsrc_t rsrc, unsigned off) {
+  T v;
+  if constexpr (sizeof(T) == 2) {
+    const unsigned short w = __builtin_amdgcn_raw_buffer_load_b16(rsrc, off, 0, 0);
+    __builtin_memcpy(&v, &w, 2);
+  } else {
+    const unsigned w = __builtin_amdgcn_raw_buffer_load_b32(rsrc, off, 0, 0);
+    __builtin_memcpy(&v, &w, 4);
+  }
+  return v;
+}
+
+// Position of one sample in its box: byte offset of the low corner, fractions, not void.
+struct Corner {
+  unsigned at;
+  float wx, wy, wz;
+  unsigned pick;   // order 0: offset of the voxel that is picked
+  bool ok;
+};
+struct BoxBytes { unsigned row, slice, dy, dz; };   // dy / dz: 0 when the box is one row / slice thick
+template <typename CT, bool CLIPPED, int ES>
+__device__ __forceinline__ Corner corner_of(CT rx, CT ry, CT rz, const BoxBytes &g, const CT (&cmax)[3], const CT (&top)[3]) {
+  Corner c;
+  c.ok = true;
+  CT lx, ly, lz, fx, fy, fz;
+  if constexpr (CLIPPED) {
+    const CT ux = rx, uy = ry, uz = rz;
+    rx = clamp_ct(rx, CT(0), cmax[0]); ry = clamp_ct(ry, CT(0), cmax[1]); rz = clamp_ct(rz, CT(0), cmax[2]);
+    c.ok = fmax(fmax(fabs(ux - rx), fabs(uy - ry)), fabs(uz - rz)) <= CT(1);
+    lx = fmin(floor(rx), top[0]); ly = fmin(floor(ry), top[1]); lz = fmin(floor(rz), top[2]);
+  } else {
+    lx = floor(rx); ly = floor(ry); lz = floor(rz);
+  }
+  fx = rx - lx; fy = ry - ly; fz = rz - lz;
+  c.at = static_cast<unsigned>(static_cast<int>(lz)) * g.slice + static_cast<unsigned>(static_cast<int>(ly)) * g.row +
+         static_cast<unsigned>(static_cast<int>(lx)) * ES;
+  c.pick = (fz <= CT(0.5) ? 0u : g.dz) + (fy <= CT(0.5) ? 0u : g.dy) + (fx <= CT(0.5) ? 0u : static_cast<unsigned>(ES));
+  c.wx = static_cast<float>(fx); c.wy = static_cast<float>(fy); c.wz = static_cast<float>(fz);
+  return c;
+}
+
+// The lane's column of ZPL voxels: positions first, then every tap of the column in flight, then the blends.
+template <typename T, typename CT, bool CLIPPED, int ORDER, int ZPL>
+__device__ __forceinline__ void direct_column(__amdgpu_buffer_rsrc_t rsrc, float (&o)[ZPL], const CT (&b)[3], const CT (&st)[3],
+                                              const BoxBytes &g, const CT (&cmax)[3], const CT (&top)[3], bool thin) {
+  Corner c[ZPL];
+  if constexpr (sizeof(CT) == 4) {
+    ColumnCoord r;
+    r.start(b[0], b[1], b[2]);
+    column_steps<0, ZPL>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      if constexpr (k > 0) r.template step<k>(st[0], st[1], st[2]);
+      c[k] = corner_of<CT, CLIPPED, sizeof(T)>(r.last[0], r.last[1], r.last[2], g, cmax, top);
+    });
+  } else {
+#pragma unroll
+    for (int k = 0; k < ZPL; k++) {
+      const CT kk = static_cast<CT>(k);
+      c[k] = corner_of<CT, CLIPPED, sizeof(T)>(b[0] + kk * st[0], b[1] + kk * st[1], b[2] + kk * st[2], g, cmax, top);
+    }
+  }
+  if constexpr (ORDER == 0) {
+    T v[ZPL];
+#pragma unroll
+    for (int k = 0; k < ZPL; k++) v[k] = load_element<T>(rsrc, c[k].at + c[k].pick);
+#pragma unroll
+    for (int k = 0; k < ZPL; k++) o[k] = c[k].ok ? load(&v[k]) : 0.f;
+  } else {
+    RowPair<T> v[ZPL][4];
+#pragma unroll
+    for (int k = 0; k < ZPL; k++) {
+      v[k][0] = load_row_pair<T>(rsrc, c[k].at);
+      v[k][1] = load_row_pair<T>(rsrc, c[k].at + g.dy);
+      v[k][2] = load_row_pair<T>(rsrc, c[k].at + g.dz);
+      v[k][3] = load_row_pair<T>(rsrc, c[k].at + g.dz + g.dy);
+    }
+#pragma unroll
+    for (int k = 0; k < ZPL; k++) {
+      // (a box one column wide, on the volume's last column: the pair holds the column before it and itself)
+      if (thin)
+#pragma unroll
+        for (int q = 0; q < 4; q++) v[k][q].a = v[k][q].b;
+      const float x00 = mix(c[k].wx, load(&v[k][0].a), load(&v[k][0].b)), x01 = mix(c[k].wx, load(&v[k][1].a), load(&v[k][1].b));
+      const float x10 = mix(c[k].wx, load(&v[k][2].a), load(&v[k][2].b)), x11 = mix(c[k].wx, load(&v[k][3].a), load(&v[k][3].b));
+      float r;
+      if constexpr (CLIPPED || sizeof(CT) == 8) {
+        r = mix(c[k].wz, mix(c[k].wy, x00, x01), mix(c[k].wy, x10, x11));
+      } else {
+        const float y0 = fmaf(c[k].wy, x01 - x00, x00), y1 = fmaf(c[k].wy, x11 - x10, x10);
+        r = fmaf(c[k].wz, y1 - y0, y0);
+      }
+      o[k] = c[k].ok ? r : 0.f;
+    }
+  }
+}
+
+template <typename T, int TX, int TY, int TZ, int PARTS, int ORDER>
+__global__ __launch_bounds__(512 / PARTS) void roi_resample_direct_kernel(
+    const T *__restrict__ feat, const float *__restrict__ rois, T *__restrict__ out, const RoiProblem p, const PlanShape ps, const unsigned total) {
+  using CT = typename std::conditional<(sizeof(T) == 2), float, double>::type;
+  constexpr int ZPL = TZ / (512 / (TX * TY)), ES = sizeof(T);
+  __shared__ __attribute__((aligned(16))) TilePlan plan;
+  const unsigned wg = xcd_contiguous(blockIdx.x, gridDim.x), item = wg / PARTS, part = wg % PARTS;
+  // (all sixteen groups of four lanes write the same record)
+  if (threadIdx.x < kWave)
+    plan_item_lanes(rois, p, ps, item, total, static_cast<unsigned>(ps.tiles_x) * ps.tiles_y * ps.tiles_z, &plan);
+  __syncthreads();
+  const int tid = threadIdx.x + part * (512 / PARTS);
+  const int lx = tid % TX, ly = (tid / TX) % TY, lz = tid / (TX * TY);
+  const int mode = plan_scalar(&plan.mode);
+  CT b[3], st[3];
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    const CT *m = plan_map<CT>(&plan) + 4 * a;
+    b[a] = m[0] + static_cast<CT>(lx) * m[1] + static_cast<CT>(ly) * m[2] + static_cast<CT>(lz * ZPL) * m[3];
+    st[a] = m[3];
+  }
+  float o[ZPL];
+  auto u64_of = [](const unsigned &lo, const unsigned &hi) {
+    return (static_cast<unsigned long>(static_cast<unsigned>(__builtin_amdgcn_readfirstlane(hi))) << 32) |
+           static_cast<unsigned>(__builtin_amdgcn_readfirstlane(lo));
+  };
+  if (mode == 0) {
+#pragma unroll
+    for (int k = 0; k < ZPL; k++) o[k] = 0.f;
+  } else if (mode == 2) {   // (a box beyond the LDS tile of the kernel above, which then works in coordinates of the volume)
+    const int size[3] = {p.W, p.H, p.D};
+    BoxLimits<CT> lim;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      b[a] += static_cast<CT>(plan_scalar(&plan.lo[a]));
+      lim.cmax[a] = static_cast<CT>(size[a] - 1);
+      lim.top[a] = static_cast<CT>(max(size[a] - 2, 0));
+    }
+    const T *src = reinterpret_cast<const T *>(reinterpret_cast<const char *>(feat) + u64_of(plan.vol_lo, plan.vol_hi));
+    const long hw = static_cast<long>(p.H) * p.W;
+    staged_column<T, CT, false, ORDER, ZPL, true>(src, o, b[0], b[1], b[2], st[0], st[1], st[2], lim, p.W, hw,
+                                                  p.H > 1 ? p.W : 0, p.D > 1 ? hw : 0, [](int) {});
+  } else {
+    const int n0 = plan_scalar(&plan.n[0]), n1 = plan_scalar(&plan.n[1]), n2 = plan_scalar(&plan.n[2]);
+    const int size[3] = {p.W, p.H, p.D}, n[3] = {n0, n1, n2};
+    CT cmax[3], top[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+      cmax[a] = static_cast<CT>(size[a] - 1 - plan_scalar(&plan.lo[a]));
+      top[a] = static_cast<CT>(max(n[a] - 2, 0));
+    }
+    BoxBytes g;
+    g.row = static_cast<unsigned>(p.W) * ES;
+    g.slice = static_cast<unsigned>(p.H) * g.row;
+    g.dy = n1 > 1 ? g.row : 0u;
+    g.dz = n2 > 1 ? g.slice : 0u;
+    const int shift_b = plan_scalar(&plan.shift_b);
+    const bool thin = ORDER != 0 && n0 == 1;   // (the volume is at least two columns wide, checked by the host)
+    const char *base = reinterpret_cast<const char *>(feat) + u64_of(plan.src_lo, plan.src_hi) + (shift_b - (thin ? ES : 0));
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<char *>(base), 0, plan_scalar(&plan.extent) - shift_b + (thin ? ES : 0), 0x00020000);
+    if (mode == 3) direct_column<T, CT, false, ORDER, ZPL>(rsrc, o, b, st, g, cmax, top, thin);
+    else direct_column<T, CT, true, ORDER, ZPL>(rsrc, o, b, st, g, cmax, top, thin);
+  }
+  const int zbytes = p.oh * p.ow * ES;
+  const __amdgpu_buffer_rsrc_t dst = __builtin_amdgcn_make_buffer_rsrc(
+      reinterpret_cast<char *>(out) + u64_of(plan.out_lo, plan.out_hi), 0, p.od * zbytes, 0x00020000);
+  const unsigned voff = (lx < plan_scalar(&plan.xlim) && ly < plan_scalar(&plan.ylim))
+                            ? static_cast<unsigned>(((lz * ZPL * p.oh + ly) * p.ow + lx) * ES + plan_scalar(&plan.tile_off)) : kOutOfRange;
+#pragma unroll
+  for (int k = 0; k < ZPL; k++) store_element<T>(dst, voff, k * zbytes, o[k]);
 }
 
 // Compute units of the current device (workgroups resident at once = units * LDS share).
@@ -1300,8 +1527,8 @@ static unsigned compute_units() {
 // G > 1: `p` is the problem on the finer grid of a fixed sampling grid of G per axis (order 1), `out` the
 // volume of the bins' means.
 template <typename T, int TX, int TY, int TZ, int THREADS, int LDS_BYTES, int KMAX, bool CUBIC = false, int G = 1>
-static int launch_resample(const T *feat, const float *rois, T *out, const RoiProblem &p,
-                           void *workspace, size_t *need, hipStream_t s) {
+static int launch_resample(const T *feat, const float *rois, T *out, const RoiProblem &p, size_t *need,
+                           hipStream_t s) {
   const long tx = (p.ow + TX - 1) / TX, ty = (p.oh + TY - 1) / TY, tz = (p.od + TZ - 1) / TZ;
   const long per_roi = tx * ty * tz, total = per_roi * static_cast<long>(p.R), work = total * p.C;
   if (work >= (1L << 31) || static_cast<long>(p.D) * p.H * p.W * sizeof(T) >= (1L << 31)) return -1;
@@ -1311,6 +1538,7 @@ static int launch_resample(const T *feat, const float *rois, T *out, const RoiPr
   ps.tiles_x = static_cast<int>(tx); ps.tiles_y = static_cast<int>(ty); ps.tiles_z = static_cast<int>(tz);
   ps.tx = TX; ps.ty = TY; ps.tz = TZ;
   ps.vec = ((p.W % V == 0) && (reinterpret_cast<uintptr_t>(feat) % 16 == 0)) ? V : 0;
+  ps.loose_vec = (!CUBIC && ps.vec == 0) ? V : 0;
   ps.cap = LDS_BYTES / sizeof(T);
   ps.threads = THREADS; ps.max_items = KMAX;
   ps.halo_lo = CUBIC ? 1 : 0; ps.halo_hi = CUBIC ? 2 : 1;
@@ -1319,7 +1547,7 @@ static int launch_resample(const T *feat, const float *rois, T *out, const RoiPr
   {
     // inputs that fit the L2s and are read about once (resampling: no more rois than images)
     const long in_bytes = static_cast<long>(p.N) * p.C * p.D * p.H * p.W * static_cast<long>(sizeof(T));
-    ps.warm_groups = (!CUBIC && ps.vec > 0 && p.R <= p.N && in_bytes <= (24L << 20)) ? static_cast<unsigned>(in_bytes / (4 * kWarmStride)) : 0u;
+    ps.warm_groups = (!CUBIC && reinterpret_cast<uintptr_t>(feat) % 16 == 0 && p.R <= p.N && in_bytes <= (24L << 20)) ? static_cast<unsigned>(in_bytes / (4 * kWarmStride)) : 0u;
   }
   ps.es = static_cast<int>(sizeof(T));
   ps.pad_slices = (!CUBIC && sizeof(T) == 2) ? 1 : 0;   // (fp32 tensors: modelled gain 12 %, measured none)
@@ -1327,6 +1555,26 @@ static int launch_resample(const T *feat, const float *rois, T *out, const RoiPr
   ps.by_tiles_x.set(static_cast<unsigned>(tx));
   ps.by_tiles_y.set(static_cast<unsigned>(ty));
   ps.by_total.set(static_cast<unsigned>(total));
+  if constexpr (!CUBIC && G == 1) {
+    // Small outputs: taps straight from the caches.  Fitted over problems of 0.06 - 33 M voxels: that kernel takes
+    // ~4.7 us + 5 - 6 us per million voxels at order 1 (rotated volumes; 4 us at order 0), the persistent one
+    // ~7 us + 2 - 3.3 us, whatever the type.  (32 x 48 x 48 fp32: 20.3 -> 5.1 us.)  Outputs of a sixth of the
+    // image or less are reductions by 1.8 and more per axis, whose boxes are beyond the LDS tile (70 x 211 x 211
+    // fp16 -> 39 x 102 x 102: 32 against 7.7 us), or crops, which lose up to 5 us by this below the limit.
+    const long voxels = static_cast<long>(p.R) * p.C * p.od * p.oh * p.ow;
+    const bool reduced = 6L * p.od * p.oh * p.ow <= static_cast<long>(p.D) * p.H * p.W;
+    if (voxels < (p.order == 0 || reduced ? 2000000L : 700000L) && p.W >= 2) {
+      constexpr int PARTS = 4;   // (512 columns per tile in workgroups of two wavefronts: one volume of 32 x 48 x 48 still gives 144)
+      const dim3 grid(static_cast<unsigned>(work) * PARTS), block(512 / PARTS);
+      if (p.order == 0)
+        hipLaunchKernelGGL((roi_resample_direct_kernel<T, TX, TY, TZ, PARTS, 0>), grid, block, 0, s, feat, rois, out, p,
+                           ps, static_cast<unsigned>(total));
+      else
+        hipLaunchKernelGGL((roi_resample_direct_kernel<T, TX, TY, TZ, PARTS, 1>), grid, block, 0, s, feat, rois, out, p,
+                           ps, static_cast<unsigned>(total));
+      return check_launch("roi_resample_direct_kernel");
+    }
+  }
   unsigned blocks = compute_units() * (160u * 1024u / (LDS_BYTES + sizeof(TilePlan) * kPlanSlots + 64u));
   // As many workgroups as are resident at once, more when that would give one more than
   // kPlanSlots items (the later ones start as the first finish).
@@ -1336,6 +1584,9 @@ static int launch_resample(const T *feat, const float *rois, T *out, const RoiPr
   if (blocks >= kXcds) blocks = blocks / kXcds * kXcds;  // the same number of workgroups on every XCD
   if (by_slots > blocks && work > kPlanSlots) blocks = static_cast<unsigned>(by_slots);
   ps.by_slots.set(blocks >= kXcds ? blocks / kXcds : blocks);
+  // (the warm-up is hidden behind the planning only while a lane has a few loads to issue: with few workgroups it
+  // took 10 us by itself)
+  if (ps.warm_groups > blocks * 6u * (THREADS - kWave)) ps.warm_groups = 0;
   if constexpr (CUBIC)
     hipLaunchKernelGGL((roi_resample_cubic_kernel<T, TX, TY, TZ, THREADS, LDS_BYTES>), dim3(blocks),
                        dim3(THREADS), 0, s, feat, rois, out, p, ps, static_cast<unsigned>(total),
@@ -1399,12 +1650,12 @@ __global__ __launch_bounds__(256) void roi_bin_mean_kernel(const T *__restrict__
 // 0.049 ms).  Returns -1 for what it does not take.  (The workspace query does not know the order and
 // answers for the two passes.)
 static int roi_forward_tiled_image(const void *input, const void *rois, void *output, int dtype, const RoiProblem &p,
-                                   void *workspace, size_t capacity, size_t *need, hipStream_t s, int pool);
+                                   size_t *need, hipStream_t s, int pool);
 
 static int roi_forward_tiled_grid(const void *input, const void *rois, void *output, int dtype,
                                   const RoiProblem &p, void *workspace, size_t capacity, size_t *need, hipStream_t s) {
   const int g = p.sampling_ratio, gz = p.ndim == 3 ? g : 1;
-  // the means inside the kernel: images, grids of 2 and 4 at order 1 (their rewritten rois are in the workspace)
+  // the means inside the kernel: images, grids of 2 and 4 at order 1
   const bool means = p.ndim == 2 && (g == 2 || g == 4) && p.R > 0 && (dtype == MV_F16 || dtype == MV_BF16 || dtype == MV_F32);
   const bool in_kernel = !need && means && p.order == 1;
   if (!need && p.ndim == 3 && p.order != 3) return -1;   // volumes at orders 0 and 1: the loop over the samples
@@ -1421,11 +1672,11 @@ static int roi_forward_tiled_grid(const void *input, const void *rois, void *out
   const long fine = cells * gz * g * g;
   // (32-bit byte offsets inside one finer volume, as in the grid-1 rule)
   if (in_kernel && static_cast<long>(f.od) * f.oh * f.ow * 4 < (1L << 31)) {
-    const int st = roi_forward_tiled_image(input, rois, output, dtype, f, workspace, capacity, nullptr, s, g);
+    const int st = roi_forward_tiled_image(input, rois, output, dtype, f, nullptr, s, g);
     if (st != -1) return st;
   }
   if (dtype != MV_F16 && dtype != MV_F32) {   // bf16: the means inside the kernel or nothing
-    if (need && p.ndim == 2) return roi_forward_tiled_image(nullptr, nullptr, nullptr, dtype, f, nullptr, 0, need, nullptr, g);
+    if (need && p.ndim == 2) return roi_forward_tiled_image(nullptr, nullptr, nullptr, dtype, f, need, nullptr, g);
     return -1;
   }
   if (fine >= (1L << 31) || (cells + 255) / 256 >= (1L << 31)) return -1;
@@ -1456,62 +1707,40 @@ static int roi_forward_tiled_grid(const void *input, const void *rois, void *out
 // the angles (0, -theta, 0) the volume's rotation rows are (cos, 0, -sin) and (sin, 0, cos) with the
 // very values of the image's rotation (sin is odd in the routine used; products with exact 0 and 1 are
 // exact), so the planner forms the same fp64 map as for the image.  Tiles of 64 x 1 x 64 (fp32: 32)
-// outputs, a column of 8 (4) rows per lane.
-__global__ void roi_rows_as_slices_kernel(const float *__restrict__ flat, float *__restrict__ vol, int R, int rotated,
-                                          int aligned, float scale) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= R) return;
-  const float *r = flat + static_cast<long>(i) * (rotated ? 6 : 5);
-  float *o = vol + static_cast<long>(i) * (rotated ? 10 : 7);
-  o[0] = r[0];
-  if (rotated) {
-    o[1] = r[1]; o[2] = aligned ? 0.5f / scale : 0.f; o[3] = r[2];
-    o[4] = r[3]; o[5] = 1.f / scale; o[6] = r[4];
-    o[7] = 0.f; o[8] = -r[5]; o[9] = 0.f;
-  } else {   // corners: the middle axis runs from -0.5 to 0.5, one cell sampled at its centre
-    o[1] = r[1]; o[2] = -0.5f / scale; o[3] = r[2];
-    o[4] = r[3]; o[5] = 0.5f / scale; o[6] = r[4];
-  }
-}
-
+// outputs, a column of 8 (4) rows per lane.  The planner takes the image's rois as they are (PlanShape::flat_axis).
 // pool = 2 or 4: `p` is the problem on the finer grid of a fixed sampling grid (order 1) and `output` takes
 // the bins' means (see roi_forward_tiled_grid).
 static int roi_forward_tiled_image(const void *input, const void *rois, void *output, int dtype, const RoiProblem &p,
-                                   void *workspace, size_t capacity, size_t *need, hipStream_t s, int pool) {
+                                   size_t *need, hipStream_t s, int pool) {
   const long vox = static_cast<long>(p.oh) * p.ow;
   // pool = 0: `p` is the problem asked for, with any sampling grid, and the kernel walks the samples of a bin
   if ((pool != 0 && p.sampling_ratio != 1) || vox < 4096 || p.ow < 16 || p.R == 0) return -1;
   if (pool > 1 && ((!need && p.order != 1) || (pool != 2 && pool != 4))) return -1;   // (a size query is not told the order)
   if (pool == 0 && !need && p.order == 3) return -1;
   if (vox * 4 >= (1L << 31)) return -1;
-  if (dtype != MV_F16 && dtype != MV_BF16 && dtype != MV_F32) return -1;
-  // (the workspace query does not know whether the rois are rotated: room for the wider rows)
+  if (dtype != MV_F16 && dtype != MV_BF16 && dtype != MV_F32 && !(dtype == MV_I32 && pool == 1)) return -1;
+  // (no kernel here uses a workspace any more; callers that size one by the query keep getting the same answer)
   const size_t bytes = (static_cast<size_t>(p.R) * 10 * sizeof(float) + 255) / 256 * 256;
   RoiProblem v = p;
   v.ndim = 3;
   v.D = p.H; v.H = 1; v.W = p.W;
   v.od = p.oh; v.oh = 1; v.ow = p.ow;
-  float *vol_rois = static_cast<float *>(workspace);
-  if (!need) {
-    if (workspace == nullptr || capacity < bytes) return -1;
-    hipLaunchKernelGGL(roi_rows_as_slices_kernel, dim3((p.R + 255) / 256), dim3(256), 0, s, static_cast<const float *>(rois),
-                       vol_rois, p.R, p.rotated, p.aligned, static_cast<float>(p.scale));
-  }
+  const float *vol_rois = static_cast<const float *>(rois);
   int st;
   if (p.order == 3) {
     // (the one cell of the middle axis samples row 0 exactly: its four taps are that row with weights 0, 1, 0, 0)
     switch (dtype) {
       case MV_F16:
         st = launch_resample<__half, 64, 1, 64, 512, 74 * 1024, 8, true>(static_cast<const __half *>(input), vol_rois,
-                                                                          static_cast<__half *>(output), v, nullptr, need, s);
+                                                                          static_cast<__half *>(output), v, need, s);
         break;
       case MV_BF16:
         st = launch_resample<__hip_bfloat16, 64, 1, 64, 512, 74 * 1024, 8, true>(
-            static_cast<const __hip_bfloat16 *>(input), vol_rois, static_cast<__hip_bfloat16 *>(output), v, nullptr, need, s);
+            static_cast<const __hip_bfloat16 *>(input), vol_rois, static_cast<__hip_bfloat16 *>(output), v, need, s);
         break;
       default:
         st = launch_resample<float, 64, 1, 64, 512, 74 * 1024, 6, true>(static_cast<const float *>(input), vol_rois,
-                                                                         static_cast<float *>(output), v, nullptr, need, s);
+                                                                         static_cast<float *>(output), v, need, s);
     }
     if (need && st == MV_OK) *need = bytes;
     return st;
@@ -1520,15 +1749,15 @@ static int roi_forward_tiled_image(const void *input, const void *rois, void *ou
     switch (dtype) {
       case MV_F16:
         st = launch_resample<__half, 64, 1, 64, 512, 74 * 1024, 8, false, 0>(static_cast<const __half *>(input), vol_rois,
-                                                                              static_cast<__half *>(output), v, nullptr, need, s);
+                                                                              static_cast<__half *>(output), v, need, s);
         break;
       case MV_BF16:
         st = launch_resample<__hip_bfloat16, 64, 1, 64, 512, 74 * 1024, 8, false, 0>(
-            static_cast<const __hip_bfloat16 *>(input), vol_rois, static_cast<__hip_bfloat16 *>(output), v, nullptr, need, s);
+            static_cast<const __hip_bfloat16 *>(input), vol_rois, static_cast<__hip_bfloat16 *>(output), v, need, s);
         break;
       default:
         st = launch_resample<float, 64, 1, 32, 512, 74 * 1024, 6, false, 0>(static_cast<const float *>(input), vol_rois,
-                                                                             static_cast<float *>(output), v, nullptr, need, s);
+                                                                             static_cast<float *>(output), v, need, s);
     }
     if (need && st == MV_OK) *need = bytes;
     return st;
@@ -1536,7 +1765,7 @@ static int roi_forward_tiled_image(const void *input, const void *rois, void *ou
   if (pool != 1) {
 #define MV_IMAGE_MEANS(TYPE, TZV, KMAXV, GV)                                                                         \
   launch_resample<TYPE, 64, 1, TZV, 512, 74 * 1024, KMAXV, false, GV>(static_cast<const TYPE *>(input), vol_rois, \
-                                                                       static_cast<TYPE *>(output), v, nullptr, need, s)
+                                                                       static_cast<TYPE *>(output), v, need, s)
     switch (dtype) {
       case MV_F16: st = pool == 2 ? MV_IMAGE_MEANS(__half, 64, 8, 2) : MV_IMAGE_MEANS(__half, 64, 8, 4); break;
       case MV_BF16: st = pool == 2 ? MV_IMAGE_MEANS(__hip_bfloat16, 64, 8, 2) : MV_IMAGE_MEANS(__hip_bfloat16, 64, 8, 4); break;
@@ -1549,19 +1778,19 @@ static int roi_forward_tiled_image(const void *input, const void *rois, void *ou
   switch (dtype) {
     case MV_F16:
       st = launch_resample<__half, 64, 1, 64, 512, 74 * 1024, 8>(static_cast<const __half *>(input), vol_rois,
-                                                                  static_cast<__half *>(output), v, nullptr, need, s);
+                                                                  static_cast<__half *>(output), v, need, s);
       break;
     case MV_BF16:
       st = launch_resample<__hip_bfloat16, 64, 1, 64, 512, 74 * 1024, 8>(static_cast<const __hip_bfloat16 *>(input), vol_rois,
-                                                                          static_cast<__hip_bfloat16 *>(output), v, nullptr, need, s);
+                                                                          static_cast<__hip_bfloat16 *>(output), v, need, s);
       break;
     case MV_I32:
       st = launch_resample<int, 64, 1, 32, 512, 74 * 1024, 6>(static_cast<const int *>(input), vol_rois,
-                                                               static_cast<int *>(output), v, nullptr, need, s);
+                                                               static_cast<int *>(output), v, need, s);
       break;
     default:
       st = launch_resample<float, 64, 1, 32, 512, 74 * 1024, 6>(static_cast<const float *>(input), vol_rois,
-                                                                 static_cast<float *>(output), v, nullptr, need, s);
+                                                                 static_cast<float *>(output), v, need, s);
   }
   if (need && st == MV_OK) *need = bytes;
   return st;
@@ -1584,7 +1813,7 @@ int roi_forward_tiled(const void *input, const void *rois, void *output, int dty
   const bool any_grid = p.sampling_ratio != 1;
   if (any_grid && p.order == 3) return -1;
   // images: rows as slices
-  if (p.ndim == 2) return roi_forward_tiled_image(input, rois, output, dtype, p, workspace, capacity, need, s, any_grid ? 0 : 1);
+  if (p.ndim == 2) return roi_forward_tiled_image(input, rois, output, dtype, p, need, s, any_grid ? 0 : 1);
   const long vox = static_cast<long>(p.od) * p.oh * p.ow;
   if (vox < 4096 || p.ow < 16 || p.R == 0) return -1;
   if (vox * 4 >= (1L << 31)) return -1;   // 32-bit byte offsets inside one output volume
@@ -1593,13 +1822,13 @@ int roi_forward_tiled(const void *input, const void *rois, void *output, int dty
     switch (dtype) {
       case MV_F16:
         return launch_resample<__half, 16, 16, 16, 512, 74 * 1024, 8, false, 0>(
-            static_cast<const __half *>(input), r, static_cast<__half *>(output), p, workspace, need, s);
+            static_cast<const __half *>(input), r, static_cast<__half *>(output), p, need, s);
       case MV_BF16:
         return launch_resample<__hip_bfloat16, 16, 16, 16, 512, 74 * 1024, 8, false, 0>(
-            static_cast<const __hip_bfloat16 *>(input), r, static_cast<__hip_bfloat16 *>(output), p, workspace, need, s);
+            static_cast<const __hip_bfloat16 *>(input), r, static_cast<__hip_bfloat16 *>(output), p, need, s);
       case MV_F32:
         return launch_resample<float, 16, 16, 8, 512, 74 * 1024, 6, false, 0>(
-            static_cast<const float *>(input), r, static_cast<float *>(output), p, workspace, need, s);
+            static_cast<const float *>(input), r, static_cast<float *>(output), p, need, s);
       default:
         return -1;
     }
@@ -1613,14 +1842,14 @@ int roi_forward_tiled(const void *input, const void *rois, void *output, int dty
       switch (dtype) {
         case MV_F16:
           return launch_resample<__half, 16, 16, 32, 512, 20 * 1024, 8, true>(
-              static_cast<const __half *>(input), r, static_cast<__half *>(output), p, workspace, need, s);
+              static_cast<const __half *>(input), r, static_cast<__half *>(output), p, need, s);
         case MV_BF16:
           return launch_resample<__hip_bfloat16, 16, 16, 32, 512, 20 * 1024, 8, true>(
               static_cast<const __hip_bfloat16 *>(input), r, static_cast<__hip_bfloat16 *>(output), p,
-              workspace, need, s);
+              need, s);
         case MV_F32:
           return launch_resample<float, 16, 16, 32, 512, 20 * 1024, 6, true>(
-              static_cast<const float *>(input), r, static_cast<float *>(output), p, workspace, need, s);
+              static_cast<const float *>(input), r, static_cast<float *>(output), p, need, s);
         default:
           return -1;
       }
@@ -1628,14 +1857,14 @@ int roi_forward_tiled(const void *input, const void *rois, void *output, int dty
     switch (dtype) {
       case MV_F16:
         return launch_resample<__half, 16, 16, 8, 512, 74 * 1024, 8, true>(
-            static_cast<const __half *>(input), r, static_cast<__half *>(output), p, workspace, need, s);
+            static_cast<const __half *>(input), r, static_cast<__half *>(output), p, need, s);
       case MV_BF16:
         return launch_resample<__hip_bfloat16, 16, 16, 8, 512, 74 * 1024, 8, true>(
             static_cast<const __hip_bfloat16 *>(input), r, static_cast<__hip_bfloat16 *>(output), p,
-            workspace, need, s);
+            need, s);
       case MV_F32:
         return launch_resample<float, 16, 16, 8, 512, 74 * 1024, 6, true>(
-            static_cast<const float *>(input), r, static_cast<float *>(output), p, workspace, need, s);
+            static_cast<const float *>(input), r, static_cast<float *>(output), p, need, s);
       default:
         return -1;
     }
@@ -1643,17 +1872,17 @@ int roi_forward_tiled(const void *input, const void *rois, void *output, int dty
   switch (dtype) {
     case MV_F16:
       return launch_resample<__half, 16, 16, 16, 512, 74 * 1024, 8>(
-          static_cast<const __half *>(input), r, static_cast<__half *>(output), p, workspace, need, s);
+          static_cast<const __half *>(input), r, static_cast<__half *>(output), p, need, s);
     case MV_BF16:
       return launch_resample<__hip_bfloat16, 16, 16, 16, 512, 74 * 1024, 8>(
           static_cast<const __hip_bfloat16 *>(input), r, static_cast<__hip_bfloat16 *>(output), p,
-          workspace, need, s);
+          need, s);
     case MV_F32:
       return launch_resample<float, 16, 16, 8, 512, 74 * 1024, 6>(
-          static_cast<const float *>(input), r, static_cast<float *>(output), p, workspace, need, s);
+          static_cast<const float *>(input), r, static_cast<float *>(output), p, need, s);
     case MV_I32:
       return launch_resample<int, 16, 16, 8, 512, 74 * 1024, 6>(
-          static_cast<const int *>(input), r, static_cast<int *>(output), p, workspace, need, s);
+          static_cast<const int *>(input), r, static_cast<int *>(output), p, need, s);
     default:
       return -1;
   }
@@ -2073,7 +2302,7 @@ int roi_backward_tiled(const void *grad_output, const void *rois, void *acc, int
   PlanShape ps;
   ps.tiles_x = static_cast<int>(tx); ps.tiles_y = static_cast<int>(ty); ps.tiles_z = static_cast<int>(tz);
   ps.tx = TX; ps.ty = TY; ps.tz = TZ;
-  ps.vec = 0;
+  ps.vec = 0; ps.loose_vec = 0;
   ps.cap = kScatterLds / 4;
   ps.threads = kScatterThreads; ps.max_items = 0;
   ps.halo_lo = 0; ps.halo_hi = 1;
