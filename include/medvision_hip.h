@@ -88,6 +88,14 @@ int mv_roi_align_rotated_3d_backward(const void *grad_output, const void *rois, 
                                      int width, int num_rois, int out_d, int out_h, int out_w,
                                      float spatial_scale, int sampling_ratio, int aligned,
                                      int order, void *workspace, void *stream);
+/* The backward of every head (rois of 5 / 7 columns, `rotated`: 6 / 10; `aligned` read for those only)
+ * that REPLACES grad_input, whatever it held: for callers whose gradient buffer is fresh memory (autograd),
+ * saves the pass that clears it and, where the kernels write every voxel, the one that reads it back.
+ * Images (ndim 2): depth and out_d are ignored.  Same workspace as the others.                   */
+int mv_roi_align_backward_write(const void *grad_output, const void *rois, void *grad_input, int dtype, int ndim,
+                                int rotated, int batch, int channels, int depth, int height, int width, int num_rois,
+                                int out_d, int out_h, int out_w, float spatial_scale, int sampling_ratio, int aligned,
+                                int order, void *workspace, void *stream);
 size_t mv_roi_align_backward_workspace_bytes(int dtype, int batch, int channels, int depth,
                                              int height, int width);
 /* Workspace of the forward entry points (plain, rotated and affine).  0 for a sampling grid of 1 on
@@ -184,6 +192,11 @@ int mv_dcn3d_backward(const void *input, const void *offset, const void *mask, c
                       const void *grad_output, void *grad_input, void *grad_offset,
                       void *grad_mask, void *grad_weight, void *grad_bias,
                       const mv_dcn3d_shape *shape, int dtype, void *workspace, void *stream);
+/* ... with grad_input, grad_weight and grad_bias replaced instead of added to */
+int mv_dcn3d_backward_write(const void *input, const void *offset, const void *mask, const void *weight,
+                            const void *grad_output, void *grad_input, void *grad_offset,
+                            void *grad_mask, void *grad_weight, void *grad_bias,
+                            const mv_dcn3d_shape *shape, int dtype, void *workspace, void *stream);
 
 /* Budget of the backward pass's column buffer in bytes (default 1 GiB, or MV_DCN_COLUMN_BYTES in the
  * environment when the library is first asked).  Changing it changes what
@@ -234,6 +247,10 @@ int mv_dcn2d_backward(const void *input, const void *offset, const void *mask, c
                       const void *grad_output, void *grad_input, void *grad_offset,
                       void *grad_mask, void *grad_weight, void *grad_bias,
                       const mv_dcn2d_shape *shape, int dtype, void *workspace, void *stream);
+int mv_dcn2d_backward_write(const void *input, const void *offset, const void *mask, const void *weight,
+                            const void *grad_output, void *grad_input, void *grad_offset,
+                            void *grad_mask, void *grad_weight, void *grad_bias,
+                            const mv_dcn2d_shape *shape, int dtype, void *workspace, void *stream);
 
 /* ---- displacement-field warp (elastic engine) -----------------------------------------------
  * replaces deform_2d / deform_3d  csrc/deform_2d.h, csrc/deform_3d.h:27 (vision.cpp:71-72) for the

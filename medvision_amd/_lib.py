@@ -48,6 +48,7 @@ SIGNATURES = {
     "mv_roi_align_rotated_2d_backward": (_i, [_p, _p, _p, _i] + [_i] * 7 + [_f, _i, _i, _i, _p, _p]),
     "mv_roi_align_rotated_3d_forward": (_i, [_p, _p, _p, _i] + [_i] * 9 + [_f, _i, _i, _i, _p, _sz, _p]),
     "mv_roi_align_rotated_3d_backward": (_i, [_p, _p, _p, _i] + [_i] * 9 + [_f, _i, _i, _i, _p, _p]),
+    "mv_roi_align_backward_write": (_i, [_p, _p, _p] + [_i] * 12 + [_f, _i, _i, _i, _p, _p]),
     "mv_roi_align_backward_workspace_bytes": (_sz, [_i] * 6),
     "mv_roi_align_forward_workspace_bytes": (_sz, [_i] * 8),
     "mv_roi_align_forward_workspace_bytes_for_input": (_sz, [_i] * 12),
@@ -61,6 +62,7 @@ SIGNATURES = {
     "mv_dcn3d_backward_workspace_bytes": (_sz, [_SHAPE_P, _i]),
     "mv_dcn3d_forward": (_i, [_p] * 6 + [_SHAPE_P, _i, _p, _p]),
     "mv_dcn3d_backward": (_i, [_p] * 10 + [_SHAPE_P, _i, _p, _p]),
+    "mv_dcn3d_backward_write": (_i, [_p] * 10 + [_SHAPE_P, _i, _p, _p]),
     "mv_dcn_set_column_budget": (None, [_sz]),
     "mv_dcn_column_budget": (_sz, []),
     "mv_dcn3d_forward_static": (_i, [_p] * 6 + [_SHAPE_P, _i, _p]),
@@ -69,6 +71,7 @@ SIGNATURES = {
     "mv_dcn2d_backward_workspace_bytes": (_sz, [_SHAPE2_P, _i]),
     "mv_dcn2d_forward": (_i, [_p] * 6 + [_SHAPE2_P, _i, _p, _p]),
     "mv_dcn2d_backward": (_i, [_p] * 10 + [_SHAPE2_P, _i, _p, _p]),
+    "mv_dcn2d_backward_write": (_i, [_p] * 10 + [_SHAPE2_P, _i, _p, _p]),
     "mv_deform_warp_2d": (_i, [_p, _p, _p, _i] + [_i] * 4 + [_i, _p]),
     "mv_deform_warp_3d": (_i, [_p, _p, _p, _i] + [_i] * 5 + [_i, _p]),
     "mv_deform_conv_3d": (_i, [_p] * 6 + [_i, _i, _p]),

@@ -185,24 +185,11 @@ Tensor roi_backward(const RoiCall &c, const Tensor &grad_output, const Tensor &r
   const int code = dtype_code(g);
   const auto d = five_dims(feature_size, c.ndim);
   const int n = static_cast<int>(rois.size(0));
-  const Tensor grad_input = at::zeros(feature_size, g.options());
+  const Tensor grad_input = at::empty(feature_size, g.options());
   const Tensor ws = bytes_on(g, mv_roi_align_backward_workspace_bytes(code, d[0], d[1], d[2], d[3], d[4]));
-  void *const stream = stream_of(g);
-  int status;
-  if (c.kind == kPlain && c.ndim == 2)
-    status = mv_roi_align_2d_backward(ptr(g), ptr(rois), ptr(grad_input), code, d[0], d[1], d[3], d[4], n, c.out[1],
-                                      c.out[2], c.scale, c.ratio, c.order, ptr(ws), stream);
-  else if (c.kind == kPlain)
-    status = mv_roi_align_3d_backward(ptr(g), ptr(rois), ptr(grad_input), code, d[0], d[1], d[2], d[3], d[4], n,
-                                      c.out[0], c.out[1], c.out[2], c.scale, c.ratio, c.order, ptr(ws), stream);
-  else if (c.ndim == 2)
-    status = mv_roi_align_rotated_2d_backward(ptr(g), ptr(rois), ptr(grad_input), code, d[0], d[1], d[3], d[4], n,
-                                              c.out[1], c.out[2], c.scale, c.ratio, c.aligned, c.order, ptr(ws), stream);
-  else
-    status = mv_roi_align_rotated_3d_backward(ptr(g), ptr(rois), ptr(grad_input), code, d[0], d[1], d[2], d[3], d[4], n,
-                                              c.out[0], c.out[1], c.out[2], c.scale, c.ratio, c.aligned, c.order,
-                                              ptr(ws), stream);
-  check(status);
+  check(mv_roi_align_backward_write(ptr(g), ptr(rois), ptr(grad_input), code, c.ndim, c.kind == kRotated, d[0], d[1], d[2],
+                                    d[3], d[4], n, c.out[0], c.out[1], c.out[2], c.scale, c.ratio, c.aligned, c.order,
+                                    ptr(ws), stream_of(g)));
   return grad_input;
 }
 
@@ -349,18 +336,18 @@ DcnGrads dcn_backward(const DcnCall &c, const Tensor &input, const Tensor &offse
   MVB_CHECK(grad.sizes() == at::IntArrayRef(s.out), "Input shape and grad_out shape wont match: (", shape_text(s.out), " vs ",
             shape_text(grad.sizes()), ").");
   DcnGrads g;
-  g.input = at::zeros_like(input);
-  g.weight = at::zeros_like(weight);
-  if (bias.defined()) g.bias = at::zeros_like(bias, at::MemoryFormat::Contiguous);
-  g.offset = at::empty_like(offset);   // (written whole, like grad_mask)
+  g.input = at::empty_like(input);
+  g.weight = at::empty_like(weight);
+  if (bias.defined()) g.bias = at::empty_like(bias, at::MemoryFormat::Contiguous);
+  g.offset = at::empty_like(offset);
   if (mask.defined()) g.mask = at::empty_like(mask);
   const int code = dtype_code(input);
   const Tensor ws = bytes_on(input, c.nd == 3 ? mv_dcn3d_backward_workspace_bytes(&s.v, code)
                                               : mv_dcn2d_backward_workspace_bytes(&s.i, code));
   void *const stream = stream_of(input);
-  check(c.nd == 3 ? mv_dcn3d_backward(ptr(input), ptr(offset), ptr(mask), ptr(weight), ptr(grad), ptr(g.input), ptr(g.offset),
+  check(c.nd == 3 ? mv_dcn3d_backward_write(ptr(input), ptr(offset), ptr(mask), ptr(weight), ptr(grad), ptr(g.input), ptr(g.offset),
                                       ptr(g.mask), ptr(g.weight), ptr(g.bias), &s.v, code, ptr(ws), stream)
-                  : mv_dcn2d_backward(ptr(input), ptr(offset), ptr(mask), ptr(weight), ptr(grad), ptr(g.input), ptr(g.offset),
+                  : mv_dcn2d_backward_write(ptr(input), ptr(offset), ptr(mask), ptr(weight), ptr(grad), ptr(g.input), ptr(g.offset),
                                       ptr(g.mask), ptr(g.weight), ptr(g.bias), &s.i, code, ptr(ws), stream));
   return g;
 }

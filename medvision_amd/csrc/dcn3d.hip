@@ -273,17 +273,11 @@ __global__ __launch_bounds__(256) void dcn_backward_bias_kernel(const T *__restr
   if (threadIdx.x == 0) atomic_add(gb + o, static_cast<G>(part[0] + part[1] + part[2] + part[3]));
 }
 
-__global__ void dcn_fill_zero_kernel(float *p, long n) {
-  for (long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; i < n;
-       i += static_cast<long>(gridDim.x) * blockDim.x)
-    p[i] = 0.f;
-}
-
 template <typename T>
-__global__ void dcn_add_from_f32_kernel(T *dst, const float *src, long n) {
+__global__ void dcn_add_from_f32_kernel(T *dst, const float *src, long n, int accumulate) {
   for (long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; i < n;
        i += static_cast<long>(gridDim.x) * blockDim.x)
-    dst[i] = store_cast<T>(load(dst + i) + src[i]);
+    dst[i] = store_cast<T>(accumulate ? load(dst + i) + src[i] : static_cast<typename Acc<T>::type>(src[i]));
 }
 
 // matrix-core forward for 16-bit tensors (dcn3d_mfma.hip)
@@ -302,10 +296,11 @@ int dcn_mfma_backward(const void *x, const void *off, const void *mask, const vo
                       hipStream_t stream);
 void dcn_set_column_budget(size_t bytes);
 size_t dcn_column_budget();
-int dcn_planar_add(const float *gxt, void *gx, const DcnDims &s, int dtype, hipStream_t stream);
-int dcn_weight_add(const float *acc, void *gw, const DcnDims &s, int dtype, hipStream_t stream);
+int dcn_planar_add(const float *gxt, void *gx, const DcnDims &s, int dtype, bool accumulate, hipStream_t stream);
+int dcn_weight_add(const float *acc, void *gw, const DcnDims &s, int dtype, bool accumulate, hipStream_t stream);
 int dcn_backward_fold(const float *gxt, const float *gw32, const float *gb32, void *grad_input, void *grad_weight,
-                      void *grad_bias, const DcnDims &s, int dtype, hipStream_t stream);
+                      void *grad_bias, const DcnDims &s, int dtype, bool accumulate, hipStream_t stream);
+int fill_zero(void *p, size_t bytes, hipStream_t s);   // roi_align.hip
 
 static inline int blocks_for(long n, int per_block, int cap) {
   return static_cast<int>(std::min<long>((n + per_block - 1) / per_block, cap));
@@ -437,10 +432,11 @@ static int deform_conv_any(const void *input, const void *offset, const void *we
   return check_launch("deform_conv_clamped_kernel");
 }
 
+// `accumulate`: grad_input, grad_weight and grad_bias are added to; otherwise replaced
 static int dcn_backward_any(const void *input, const void *offset, const void *mask,
                             const void *weight, const void *grad_output, void *grad_input,
                             void *grad_offset, void *grad_mask, void *grad_weight, void *grad_bias,
-                            const DcnDims &s, int dtype, void *workspace, void *stream) {
+                            const DcnDims &s, int dtype, void *workspace, void *stream, bool accumulate) {
   int st = MV_OK;
   MV_REQUIRE(input && offset && weight && grad_output && grad_input && grad_offset && grad_weight,
              "null pointer argument");
@@ -473,7 +469,7 @@ static int dcn_backward_any(const void *input, const void *offset, const void *m
     st = dcn_mfma_backward(xp, offset, mask, wsb + l.w, gyp, grad_offset, grad_mask, pad.p, dtype, wsb + l.inner,
                            false, &gx32, &gw32, &gb32, hs);
     if (st) return st;
-    st = dcn_planar_add_padded(gx32, grad_input, s, pad, dtype, hs);
+    st = dcn_planar_add_padded(gx32, grad_input, s, pad, dtype, accumulate, hs);
     if (st) return st;
     MV_DISPATCH(dtype, {
       if (sizeof(T) <= 4) {
@@ -481,11 +477,11 @@ static int dcn_backward_any(const void *input, const void *offset, const void *m
           hipLaunchKernelGGL((dcn_backward_bias_kernel<T, float>), dim3(s.Cout, s.B, static_cast<unsigned>((s.Q + kBiasSlab - 1) / kBiasSlab)), dim3(256), 0, hs,
                              static_cast<const T *>(grad_output), gb32, s);
           hipLaunchKernelGGL((dcn_add_from_f32_kernel<T>), dim3(1), dim3(256), 0, hs,
-                             static_cast<T *>(grad_bias), gb32, static_cast<long>(s.Cout));
+                             static_cast<T *>(grad_bias), gb32, static_cast<long>(s.Cout), accumulate ? 1 : 0);
         }
       }
     });
-    st = dcn_weight_add_padded(gw32, grad_weight, nullptr, nullptr, s, pad, dtype, hs);
+    st = dcn_weight_add_padded(gw32, grad_weight, nullptr, nullptr, s, pad, dtype, accumulate, hs);
     if (st) return st;
     return check_launch("dcn3d backward (padded channels)");
   }
@@ -496,25 +492,30 @@ static int dcn_backward_any(const void *input, const void *offset, const void *m
     st = dcn_mfma_backward(input, offset, mask, weight, grad_output, grad_offset, grad_mask, s, dtype,
                            workspace, grad_bias != nullptr, &gx32, &gw32, &gb32, hs);
     if (st) return st;
-    st = dcn_backward_fold(gx32, gw32, gb32, grad_input, grad_weight, grad_bias, s, dtype, hs);
+    st = dcn_backward_fold(gx32, gw32, gb32, grad_input, grad_weight, grad_bias, s, dtype, accumulate, hs);
     if (st >= 0) return st;   // (one launch for the three folds; -1: not with these tensors)
-    st = dcn_planar_add(gx32, grad_input, s, dtype, hs);
+    st = dcn_planar_add(gx32, grad_input, s, dtype, accumulate, hs);
     if (st) return st;
     MV_DISPATCH(dtype, {
       if (sizeof(T) <= 4) {
         if (grad_bias)   // (the sums of grad_output are in the accumulator already)
           hipLaunchKernelGGL((dcn_add_from_f32_kernel<T>), dim3(1), dim3(256), 0, hs,
-                             static_cast<T *>(grad_bias), gb32, static_cast<long>(s.Cout));
+                             static_cast<T *>(grad_bias), gb32, static_cast<long>(s.Cout), accumulate ? 1 : 0);
       }
     });
-    st = dcn_weight_add(gw32, grad_weight, s, dtype, hs);
+    st = dcn_weight_add(gw32, grad_weight, s, dtype, accumulate, hs);
     if (st) return st;
     return check_launch("dcn3d backward");
   }
   if (narrow) {
     const long n = n_gx + n_gw + s.Cout;
-    hipLaunchKernelGGL(dcn_fill_zero_kernel, dim3(blocks_for(n, 1024, 65536)), dim3(256), 0, hs, ws, n);
+    st = fill_zero(ws, static_cast<size_t>(n) * 4, hs);
+  } else if (!accumulate) {
+    st = fill_zero(grad_input, static_cast<size_t>(n_gx) * dtype_size(dtype), hs);
+    if (!st) st = fill_zero(grad_weight, static_cast<size_t>(n_gw) * dtype_size(dtype), hs);
+    if (!st && grad_bias) st = fill_zero(grad_bias, static_cast<size_t>(s.Cout) * dtype_size(dtype), hs);
   }
+  if (st) return st;
   const long qb = (s.Q + kDcnThreads - 1) / kDcnThreads;
   const long kb = static_cast<long>(s.dg) * s.K;
   const int tiles = (s.opg + kOutTile - 1) / kOutTile;
@@ -543,12 +544,12 @@ static int dcn_backward_any(const void *input, const void *offset, const void *m
                          static_cast<const T *>(grad_output), gb, s);
     if (sizeof(T) == 2) {
       hipLaunchKernelGGL((dcn_add_from_f32_kernel<T>), dim3(blocks_for(n_gx, 1024, 65536)), dim3(256),
-                         0, hs, static_cast<T *>(grad_input), ws, n_gx);
+                         0, hs, static_cast<T *>(grad_input), ws, n_gx, accumulate ? 1 : 0);
       hipLaunchKernelGGL((dcn_add_from_f32_kernel<T>), dim3(blocks_for(n_gw, 1024, 65536)), dim3(256),
-                         0, hs, static_cast<T *>(grad_weight), ws + n_gx, n_gw);
+                         0, hs, static_cast<T *>(grad_weight), ws + n_gx, n_gw, accumulate ? 1 : 0);
       if (grad_bias)
         hipLaunchKernelGGL((dcn_add_from_f32_kernel<T>), dim3(1), dim3(256), 0, hs,
-                           static_cast<T *>(grad_bias), ws + n_gx + n_gw, static_cast<long>(s.Cout));
+                           static_cast<T *>(grad_bias), ws + n_gx + n_gw, static_cast<long>(s.Cout), accumulate ? 1 : 0);
     }
   });
   return check_launch("dcn3d backward");
@@ -593,7 +594,18 @@ int mv_dcn3d_backward(const void *input, const void *offset, const void *mask, c
   const int st = make_dcn_dims(s, shape);
   return st ? st
             : dcn_backward_any(input, offset, mask, weight, grad_output, grad_input, grad_offset,
-                               grad_mask, grad_weight, grad_bias, s, dtype, workspace, stream);
+                               grad_mask, grad_weight, grad_bias, s, dtype, workspace, stream, true);
+}
+
+int mv_dcn3d_backward_write(const void *input, const void *offset, const void *mask, const void *weight,
+                            const void *grad_output, void *grad_input, void *grad_offset,
+                            void *grad_mask, void *grad_weight, void *grad_bias,
+                            const mv_dcn3d_shape *shape, int dtype, void *workspace, void *stream) {
+  DcnDims s;
+  const int st = make_dcn_dims(s, shape);
+  return st ? st
+            : dcn_backward_any(input, offset, mask, weight, grad_output, grad_input, grad_offset,
+                               grad_mask, grad_weight, grad_bias, s, dtype, workspace, stream, false);
 }
 
 // ---- forward without any allocation --------------------------------------------------------
@@ -672,7 +684,18 @@ int mv_dcn2d_backward(const void *input, const void *offset, const void *mask, c
   const int st = make_dcn_dims_2d(s, shape);
   return st ? st
             : dcn_backward_any(input, offset, mask, weight, grad_output, grad_input, grad_offset,
-                               grad_mask, grad_weight, grad_bias, s, dtype, workspace, stream);
+                               grad_mask, grad_weight, grad_bias, s, dtype, workspace, stream, true);
+}
+
+int mv_dcn2d_backward_write(const void *input, const void *offset, const void *mask, const void *weight,
+                            const void *grad_output, void *grad_input, void *grad_offset,
+                            void *grad_mask, void *grad_weight, void *grad_bias,
+                            const mv_dcn2d_shape *shape, int dtype, void *workspace, void *stream) {
+  DcnDims s;
+  const int st = make_dcn_dims_2d(s, shape);
+  return st ? st
+            : dcn_backward_any(input, offset, mask, weight, grad_output, grad_input, grad_offset,
+                               grad_mask, grad_weight, grad_bias, s, dtype, workspace, stream, false);
 }
 
 int mv_deform_conv_3d(const void *input, const void *offset, const void *weight, const void *bias,

@@ -1360,12 +1360,12 @@ __global__ __launch_bounds__(256) void dcn_backward_weight_columns_kernel(
   }
 }
 
-// gxt [B, P, C] fp32 -> gx [B, C, P] T, added to what gx holds; 64 positions x up to kAddChunk
-// channels per workgroup
+// gxt [B, P, C] fp32 -> gx [B, C, P] T, added to what gx holds (`accumulate`) or in its place; 64 positions x up to
+// kAddChunk channels per workgroup
 constexpr int kAddChunk = 64;
 template <typename T>
 __global__ __launch_bounds__(256) void dcn_planar_add_kernel(const float *__restrict__ gxt,
-                                                             T *__restrict__ gx, int C, long P) {
+                                                             T *__restrict__ gx, int C, long P, int accumulate) {
   __shared__ float stagef[64][kAddChunk + 1];
   const int b = blockIdx.y;
   const long p0 = static_cast<long>(blockIdx.x) * 64;
@@ -1381,27 +1381,29 @@ __global__ __launch_bounds__(256) void dcn_planar_add_kernel(const float *__rest
   if (p0 + lp < P)
     for (int c = threadIdx.x / 64; c < cn; c += 4) {
       T *d = gx + (static_cast<long>(b) * C + c0 + c) * P + p0 + lp;
-      *d = store_cast<T>(load(d) + stagef[lp][c]);
+      *d = store_cast<T>(accumulate ? load(d) + stagef[lp][c] : stagef[lp][c]);
     }
 }
 
-// The same move with 16-byte accesses on both sides (whole tiles of 64 positions x 64 channels, P a
-// multiple of 64, 16-byte aligned tensors): a lane reads four channels of one position, then adds
-// V = 16 / sizeof(T) neighbouring positions of one channel to the gradient in one read-modify-write.
-template <typename T>
+// The same move with 16-byte reads (channels in fours, an aligned buffer).  EVEN: P a multiple of 64 and the gradient
+// aligned, so that a lane takes V = 16 / sizeof(T) neighbouring positions of one channel in one write; otherwise a
+// wavefront writes 64 neighbouring elements.  ([4, 256, 38 * 30 * 125] fp16: 431 us through the kernel above.)
+template <typename T, bool EVEN>
 __device__ __forceinline__ void dcn_planar_add_wide_block(const float *__restrict__ gxt, T *__restrict__ gx, int C, long P,
-                                                          const unsigned bx, const int b, const int bz) {
+                                                          const unsigned bx, const int b, const int bz, const int accumulate) {
   constexpr int V = 16 / static_cast<int>(sizeof(T));
+  // (row pitches: 16-byte writes want multiples of four; reads along the positions want an odd multiple of them)
   __shared__ __attribute__((aligned(16))) float stagef[64][kAddChunk + 4];
   const long p0 = static_cast<long>(bx) * 64;
   const int c0 = bz * kAddChunk, cn = min(kAddChunk, C - c0);   // cn: a multiple of 4
+  const int pn = EVEN ? 64 : static_cast<int>(min(64L, P - p0));
   const float *src = gxt + (static_cast<long>(b) * P + p0) * C + c0;
   float4 in[4];
 #pragma unroll
   for (int u = 0; u < 4; u++) {
     const int i = threadIdx.x + u * 256, pp = i / 16, cq = i % 16;
     in[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (cq * 4 < cn) {   // (the accumulation buffer is read once and the result not read here again: nontemporal)
+    if (cq * 4 < cn && (EVEN || pp < pn)) {   // (the accumulation buffer is read once and the result not read here again: nontemporal)
       typedef float f32x4 __attribute__((ext_vector_type(4)));
       const f32x4 t = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(src + static_cast<long>(pp) * C + cq * 4));
       in[u] = make_float4(t.x, t.y, t.z, t.w);
@@ -1413,21 +1415,44 @@ __device__ __forceinline__ void dcn_planar_add_wide_block(const float *__restric
     *reinterpret_cast<float4 *>(&stagef[pp][cq * 4]) = in[u];
   }
   __syncthreads();
-  constexpr int PG = 64 / V;   // position groups per channel
-  for (int i = threadIdx.x; i < cn * PG; i += 256) {
-    const int c = i / PG, pg = i % PG;
-    T *d = gx + (static_cast<long>(b) * C + c0 + c) * P + p0 + pg * V;
-    union { u32x4 u; T e[V]; } piece;
-    piece.u = *reinterpret_cast<const u32x4 *>(d);
+  if constexpr (EVEN) {
+    constexpr int PG = 64 / V;   // position groups per channel
+    for (int i = threadIdx.x; i < cn * PG; i += 256) {
+      const int c = i / PG, pg = i % PG;
+      T *d = gx + (static_cast<long>(b) * C + c0 + c) * P + p0 + pg * V;
+      union { u32x4 u; T e[V]; } piece;
+      if (accumulate) {
+        piece.u = *reinterpret_cast<const u32x4 *>(d);
 #pragma unroll
-    for (int e = 0; e < V; e++) piece.e[e] = store_cast<T>(load(&piece.e[e]) + stagef[pg * V + e][c]);
-    __builtin_nontemporal_store(piece.u, reinterpret_cast<u32x4 *>(d));
+        for (int e = 0; e < V; e++) piece.e[e] = store_cast<T>(load(&piece.e[e]) + stagef[pg * V + e][c]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < V; e++) piece.e[e] = store_cast<T>(stagef[pg * V + e][c]);
+      }
+      __builtin_nontemporal_store(piece.u, reinterpret_cast<u32x4 *>(d));
+    }
+  } else {
+    const int lp = threadIdx.x % 64;
+    if (lp < pn) {
+      T *d = gx + (static_cast<long>(b) * C + c0) * P + p0 + lp;
+      for (int c = threadIdx.x / 64; c < cn; c += 16) {   // (cn is a multiple of four: four channels per turn, reads first)
+        T old[4];
+        if (accumulate)
+#pragma unroll
+          for (int u = 0; u < 4; u++)
+            if (c + 4 * u < cn) old[u] = d[(c + 4 * u) * P];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          if (c + 4 * u < cn)
+            d[(c + 4 * u) * P] = store_cast<T>(accumulate ? load(&old[u]) + stagef[lp][c + 4 * u] : stagef[lp][c + 4 * u]);
+      }
+    }
   }
 }
-template <typename T>
+template <typename T, bool EVEN>
 __global__ __launch_bounds__(256) void dcn_planar_add_wide_kernel(const float *__restrict__ gxt,
-                                                                  T *__restrict__ gx, int C, long P) {
-  dcn_planar_add_wide_block<T>(gxt, gx, C, P, blockIdx.x, blockIdx.y, blockIdx.z);
+                                                                  T *__restrict__ gx, int C, long P, int accumulate) {
+  dcn_planar_add_wide_block<T, EVEN>(gxt, gx, C, P, blockIdx.x, blockIdx.y, blockIdx.z, accumulate);
 }
 
 __device__ __forceinline__ void dcn_zero_f32_block(float *p, long n, const unsigned bid, const unsigned nblocks) {
@@ -1764,108 +1789,109 @@ int dcn_mfma_backward(const void *x, const void *off, const void *mask, const vo
   return backward_run<__hip_bfloat16>(x, off, mask, wt, gy, goff, gmask, s, workspace, gx32, gw32, gb32, dtype, want_bias, stream);
 }
 
-// dst [B, C, P] (element type of `dtype`) += src [B, P, C] fp32
-int planar_add_f32(const float *src, void *dst, int B, int C, long P, int dtype, hipStream_t stream) {
+// dst [B, C, P] (element type of `dtype`) += src [B, P, C] fp32 (= src when not `accumulate`)
+int planar_add_f32(const float *src, void *dst, int B, int C, long P, int dtype, bool accumulate, hipStream_t stream) {
   const long pblocks = (P + 63) / 64;
   MV_REQUIRE(pblocks < (1L << 31) && B <= 65535 && (C + kAddChunk - 1) / kAddChunk <= 65535, "volume too large");
   const dim3 grid(static_cast<unsigned>(pblocks), B, (C + kAddChunk - 1) / kAddChunk);
-  if (P % 64 == 0 && C % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0 &&
-      reinterpret_cast<uintptr_t>(dst) % 16 == 0) {
-    if (dtype == MV_F16)
-      hipLaunchKernelGGL((dcn_planar_add_wide_kernel<__half>), grid, dim3(256), 0, stream, src,
-                         static_cast<__half *>(dst), C, P);
-    else if (dtype == MV_F32)
-      hipLaunchKernelGGL((dcn_planar_add_wide_kernel<float>), grid, dim3(256), 0, stream, src,
-                         static_cast<float *>(dst), C, P);
-    else
-      hipLaunchKernelGGL((dcn_planar_add_wide_kernel<__hip_bfloat16>), grid, dim3(256), 0, stream, src,
-                         static_cast<__hip_bfloat16 *>(dst), C, P);
-    return check_launch("dcn_planar_add_wide_kernel");
-  }
-  if (dtype == MV_F16)
-    hipLaunchKernelGGL((dcn_planar_add_kernel<__half>), grid, dim3(256), 0, stream, src,
-                       static_cast<__half *>(dst), C, P);
-  else if (dtype == MV_F32)
-    hipLaunchKernelGGL((dcn_planar_add_kernel<float>), grid, dim3(256), 0, stream, src,
-                       static_cast<float *>(dst), C, P);
-  else
-    hipLaunchKernelGGL((dcn_planar_add_kernel<__hip_bfloat16>), grid, dim3(256), 0, stream, src,
-                       static_cast<__hip_bfloat16 *>(dst), C, P);
+  const bool wide = C % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0;
+  const bool even = wide && P % 64 == 0 && reinterpret_cast<uintptr_t>(dst) % 16 == 0;
+#define MV_PLANAR_ADD(TYPE)                                                                                           \
+  do {                                                                                                               \
+    if (even)                                                                                                        \
+      hipLaunchKernelGGL((dcn_planar_add_wide_kernel<TYPE, true>), grid, dim3(256), 0, stream, src,                   \
+                         static_cast<TYPE *>(dst), C, P, accumulate ? 1 : 0);                                         \
+    else if (wide)                                                                                                   \
+      hipLaunchKernelGGL((dcn_planar_add_wide_kernel<TYPE, false>), grid, dim3(256), 0, stream, src,                  \
+                         static_cast<TYPE *>(dst), C, P, accumulate ? 1 : 0);                                         \
+    else                                                                                                             \
+      hipLaunchKernelGGL((dcn_planar_add_kernel<TYPE>), grid, dim3(256), 0, stream, src, static_cast<TYPE *>(dst), C, \
+                         P, accumulate ? 1 : 0);                                                                      \
+  } while (0)
+  if (dtype == MV_F16) MV_PLANAR_ADD(__half);
+  else if (dtype == MV_F32) MV_PLANAR_ADD(float);
+  else MV_PLANAR_ADD(__hip_bfloat16);
+#undef MV_PLANAR_ADD
   return check_launch("dcn_planar_add_kernel");
 }
 
 // grad_weight [Cout][cpg][K] += the tap-major fp32 accumulator [K][Cout][cpg] of the weight kernel
 template <typename T>
 __device__ __forceinline__ void dcn_weight_add_block(const float *__restrict__ acc, T *__restrict__ gw, const DcnDims s,
-                                                     const unsigned bid, const unsigned nblocks) {
+                                                     const unsigned bid, const unsigned nblocks, const int accumulate) {
   const long n = static_cast<long>(s.Cout) * s.cpg * s.K;
   for (long i = bid * 256L + threadIdx.x; i < n; i += nblocks * 256L) {
     const long k = i % s.K, oc = i / s.K;
-    gw[i] = store_cast<T>(load(gw + i) + acc[k * s.Cout * s.cpg + oc]);
+    const float v = acc[k * s.Cout * s.cpg + oc];
+    gw[i] = store_cast<T>(accumulate ? load(gw + i) + v : v);
   }
 }
 template <typename T>
 __global__ __launch_bounds__(256) void dcn_weight_add_kernel(const float *__restrict__ acc, T *__restrict__ gw,
-                                                             const DcnDims s) {
-  dcn_weight_add_block<T>(acc, gw, s, blockIdx.x, gridDim.x);
+                                                             const DcnDims s, const int accumulate) {
+  dcn_weight_add_block<T>(acc, gw, s, blockIdx.x, gridDim.x, accumulate);
 }
 
 // The folds behind the backward kernels in one launch: channels-last fp32 grad input -> grad_input,
 // tap-major fp32 grad weight -> grad_weight, the fp32 bias sums -> grad_bias.
-template <typename T>
+template <typename T, bool EVEN>
 __global__ __launch_bounds__(256) void dcn_backward_fold_kernel(const float *__restrict__ gxt, T *__restrict__ gx,
                                                                 const float *__restrict__ gw32, T *__restrict__ gw,
                                                                 const float *__restrict__ gb32, T *__restrict__ gb,
                                                                 const DcnDims s, const unsigned pblocks,
-                                                                const unsigned add_end, const unsigned weight_end) {
+                                                                const unsigned add_end, const unsigned weight_end,
+                                                                const int accumulate) {
   const unsigned id = blockIdx.x;
   if (id < add_end)
-    dcn_planar_add_wide_block<T>(gxt, gx, s.Cin, s.P, id % pblocks, static_cast<int>((id / pblocks) % s.B),
-                                 static_cast<int>(id / (pblocks * s.B)));
+    dcn_planar_add_wide_block<T, EVEN>(gxt, gx, s.Cin, s.P, id % pblocks, static_cast<int>((id / pblocks) % s.B),
+                                       static_cast<int>(id / (pblocks * s.B)), accumulate);
   else if (id < weight_end)
-    dcn_weight_add_block<T>(gw32, gw, s, id - add_end, weight_end - add_end);
+    dcn_weight_add_block<T>(gw32, gw, s, id - add_end, weight_end - add_end, accumulate);
   else
-    for (int o = threadIdx.x; o < s.Cout; o += 256) gb[o] = store_cast<T>(static_cast<float>(load(gb + o)) + gb32[o]);
+    for (int o = threadIdx.x; o < s.Cout; o += 256) gb[o] = store_cast<T>((accumulate ? static_cast<float>(load(gb + o)) : 0.f) + gb32[o]);
 }
 
 // All three folds of a layer on the matrix-core path.  Returns -1 when the tensors do not allow the
 // 16-byte accesses of the one-launch form (the caller then folds one by one).
 int dcn_backward_fold(const float *gxt, const float *gw32, const float *gb32, void *grad_input, void *grad_weight,
-                      void *grad_bias, const DcnDims &s, int dtype, hipStream_t stream) {
+                      void *grad_bias, const DcnDims &s, int dtype, bool accumulate, hipStream_t stream) {
   if (dtype != MV_F16 && dtype != MV_BF16 && dtype != MV_F32) return -1;
   auto aligned16 = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  if (s.P % 64 || s.Cin % 4 || !aligned16(gxt) || !aligned16(grad_input)) return -1;
-  const long pblocks = s.P / 64, add_blocks = pblocks * s.B * ((s.Cin + kAddChunk - 1) / kAddChunk);
+  if (s.Cin % 4 || !aligned16(gxt)) return -1;
+  const bool even = s.P % 64 == 0 && aligned16(grad_input);
+  const long pblocks = (s.P + 63) / 64, add_blocks = pblocks * s.B * ((s.Cin + kAddChunk - 1) / kAddChunk);
   const long n = static_cast<long>(s.Cout) * s.cpg * s.K, weight_blocks = min((n + 255) / 256, 1024L);
   const long bias_blocks = grad_bias ? 1 : 0;
   if (add_blocks + weight_blocks + bias_blocks >= (1L << 31)) return -1;
   const unsigned add_end = static_cast<unsigned>(add_blocks), weight_end = add_end + static_cast<unsigned>(weight_blocks);
-#define MV_FOLD(T)                                                                                                  \
-  hipLaunchKernelGGL((dcn_backward_fold_kernel<T>), dim3(weight_end + static_cast<unsigned>(bias_blocks)), dim3(256), 0, \
+#define MV_FOLD_AS(T, EVENV)                                                                                          \
+  hipLaunchKernelGGL((dcn_backward_fold_kernel<T, EVENV>), dim3(weight_end + static_cast<unsigned>(bias_blocks)), dim3(256), 0, \
                      stream, gxt, static_cast<T *>(grad_input), gw32, static_cast<T *>(grad_weight),               \
                      gb32, static_cast<T *>(grad_bias), s,                                                         \
-                     static_cast<unsigned>(pblocks), add_end, weight_end)
+                     static_cast<unsigned>(pblocks), add_end, weight_end, accumulate ? 1 : 0)
+#define MV_FOLD(T) do { if (even) MV_FOLD_AS(T, true); else MV_FOLD_AS(T, false); } while (0)
   if (dtype == MV_F16) MV_FOLD(__half);
   else if (dtype == MV_BF16) MV_FOLD(__hip_bfloat16);
   else MV_FOLD(float);
 #undef MV_FOLD
+#undef MV_FOLD_AS
   return check_launch("dcn_backward_fold_kernel");
 }
-int dcn_weight_add(const float *acc, void *gw, const DcnDims &s, int dtype, hipStream_t stream) {
+int dcn_weight_add(const float *acc, void *gw, const DcnDims &s, int dtype, bool accumulate, hipStream_t stream) {
   const long n = static_cast<long>(s.Cout) * s.cpg * s.K;
   const dim3 grid(static_cast<unsigned>(min((n + 255) / 256, 4096L)));
   if (dtype == MV_F16)
-    hipLaunchKernelGGL((dcn_weight_add_kernel<__half>), grid, dim3(256), 0, stream, acc, static_cast<__half *>(gw), s);
+    hipLaunchKernelGGL((dcn_weight_add_kernel<__half>), grid, dim3(256), 0, stream, acc, static_cast<__half *>(gw), s, accumulate ? 1 : 0);
   else if (dtype == MV_F32)
-    hipLaunchKernelGGL((dcn_weight_add_kernel<float>), grid, dim3(256), 0, stream, acc, static_cast<float *>(gw), s);
+    hipLaunchKernelGGL((dcn_weight_add_kernel<float>), grid, dim3(256), 0, stream, acc, static_cast<float *>(gw), s, accumulate ? 1 : 0);
   else
     hipLaunchKernelGGL((dcn_weight_add_kernel<__hip_bfloat16>), grid, dim3(256), 0, stream, acc,
-                       static_cast<__hip_bfloat16 *>(gw), s);
+                       static_cast<__hip_bfloat16 *>(gw), s, accumulate ? 1 : 0);
   return check_launch("dcn_weight_add_kernel");
 }
 
-int dcn_planar_add(const float *gxt, void *gx, const DcnDims &s, int dtype, hipStream_t stream) {
-  return planar_add_f32(gxt, gx, s.B, s.Cin, s.P, dtype, stream);
+int dcn_planar_add(const float *gxt, void *gx, const DcnDims &s, int dtype, bool accumulate, hipStream_t stream) {
+  return planar_add_f32(gxt, gx, s.B, s.Cin, s.P, dtype, accumulate, stream);
 }
 
 }  // namespace mv

@@ -130,7 +130,7 @@ int dcn_unpad_channels(const void *src, void *dst, int B, int C, long P, int uni
 // 64 positions x 64 real channels per workgroup through LDS
 template <typename T>
 __global__ __launch_bounds__(256) void dcn_planar_add_padded_kernel(const float *__restrict__ gxt, T *__restrict__ gx,
-                                                                    int C, long P, int unit, int unit_p) {
+                                                                    int C, long P, int unit, int unit_p, int accumulate) {
   __shared__ float stagef[64][65];
   const int Cp = C / unit * unit_p;
   const int b = blockIdx.y;
@@ -148,23 +148,23 @@ __global__ __launch_bounds__(256) void dcn_planar_add_padded_kernel(const float 
   if (p0 + lp < P)
     for (int c = threadIdx.x / 64; c < cn; c += 4) {
       T *d = gx + (static_cast<long>(b) * C + c0 + c) * P + p0 + lp;
-      *d = store_cast<T>(load(d) + stagef[lp][c]);
+      *d = store_cast<T>(accumulate ? load(d) + stagef[lp][c] : stagef[lp][c]);
     }
 }
 
-int dcn_planar_add_padded(const float *gxt, void *gx, const DcnDims &s, const DcnPad &pad, int dtype, hipStream_t stream) {
+int dcn_planar_add_padded(const float *gxt, void *gx, const DcnDims &s, const DcnPad &pad, int dtype, bool accumulate, hipStream_t stream) {
   const long pblocks = (s.P + 63) / 64;
   MV_REQUIRE(pblocks < (1L << 31) && s.B <= 65535 && (s.Cin + 63) / 64 <= 65535, "volume too large");
   const dim3 grid(static_cast<unsigned>(pblocks), s.B, (s.Cin + 63) / 64);
   if (dtype == MV_F16)
     hipLaunchKernelGGL((dcn_planar_add_padded_kernel<__half>), grid, dim3(256), 0, stream, gxt, static_cast<__half *>(gx),
-                       s.Cin, s.P, pad.unit, pad.unit_p);
+                       s.Cin, s.P, pad.unit, pad.unit_p, accumulate ? 1 : 0);
   else if (dtype == MV_F32)
     hipLaunchKernelGGL((dcn_planar_add_padded_kernel<float>), grid, dim3(256), 0, stream, gxt, static_cast<float *>(gx),
-                       s.Cin, s.P, pad.unit, pad.unit_p);
+                       s.Cin, s.P, pad.unit, pad.unit_p, accumulate ? 1 : 0);
   else
     hipLaunchKernelGGL((dcn_planar_add_padded_kernel<__hip_bfloat16>), grid, dim3(256), 0, stream, gxt,
-                       static_cast<__hip_bfloat16 *>(gx), s.Cin, s.P, pad.unit, pad.unit_p);
+                       static_cast<__hip_bfloat16 *>(gx), s.Cin, s.P, pad.unit, pad.unit_p, accumulate ? 1 : 0);
   return check_launch("dcn_planar_add_padded_kernel");
 }
 
@@ -173,7 +173,7 @@ int dcn_planar_add_padded(const float *gxt, void *gx, const DcnDims &s, const Dc
 template <typename T>
 __global__ __launch_bounds__(256) void dcn_weight_add_padded_kernel(const float *__restrict__ acc, T *__restrict__ gw,
                                                                     const float *__restrict__ gb_acc, T *__restrict__ gb,
-                                                                    const DcnDims s, const DcnDims p, int unit, int unit_p) {
+                                                                    const DcnDims s, const DcnDims p, int unit, int unit_p, int accumulate) {
   const long n = static_cast<long>(s.Cout) * s.cpg * s.K;
   for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L) {
     const int k = static_cast<int>(i % s.K);
@@ -181,29 +181,30 @@ __global__ __launch_bounds__(256) void dcn_weight_add_padded_kernel(const float 
     const int cl = static_cast<int>(oc % s.cpg), o = static_cast<int>(oc / s.cpg);
     const int g = o / s.opg, ol = o - g * s.opg;
     const int u = cl / unit, r = cl - u * unit;
-    gw[i] = store_cast<T>(load(gw + i) + acc[(static_cast<long>(k) * p.Cout + g * p.opg + ol) * p.cpg + u * unit_p + r]);
+    const float v = acc[(static_cast<long>(k) * p.Cout + g * p.opg + ol) * p.cpg + u * unit_p + r];
+    gw[i] = store_cast<T>(accumulate ? load(gw + i) + v : v);
   }
   if (gb != nullptr)
     for (long o = blockIdx.x * 256L + threadIdx.x; o < s.Cout; o += gridDim.x * 256L) {
       const int g = static_cast<int>(o) / s.opg, ol = static_cast<int>(o) - g * s.opg;
-      gb[o] = store_cast<T>(load(gb + o) + gb_acc[g * p.opg + ol]);
+      gb[o] = store_cast<T>((accumulate ? load(gb + o) : 0.f) + gb_acc[g * p.opg + ol]);
     }
 }
 
 int dcn_weight_add_padded(const float *acc, void *gw, const float *gb_acc, void *gb, const DcnDims &s,
-                          const DcnPad &pad, int dtype, hipStream_t stream) {
+                          const DcnPad &pad, int dtype, bool accumulate, hipStream_t stream) {
   const long n = static_cast<long>(s.Cout) * s.cpg * s.K;
   const dim3 grid(static_cast<unsigned>(std::min<long>((n + 255) / 256, 4096L)));
   if (dtype == MV_F16)
     hipLaunchKernelGGL((dcn_weight_add_padded_kernel<__half>), grid, dim3(256), 0, stream, acc, static_cast<__half *>(gw),
-                       gb_acc, static_cast<__half *>(gb), s, pad.p, pad.unit, pad.unit_p);
+                       gb_acc, static_cast<__half *>(gb), s, pad.p, pad.unit, pad.unit_p, accumulate ? 1 : 0);
   else if (dtype == MV_F32)
     hipLaunchKernelGGL((dcn_weight_add_padded_kernel<float>), grid, dim3(256), 0, stream, acc, static_cast<float *>(gw),
-                       gb_acc, static_cast<float *>(gb), s, pad.p, pad.unit, pad.unit_p);
+                       gb_acc, static_cast<float *>(gb), s, pad.p, pad.unit, pad.unit_p, accumulate ? 1 : 0);
   else
     hipLaunchKernelGGL((dcn_weight_add_padded_kernel<__hip_bfloat16>), grid, dim3(256), 0, stream, acc,
                        static_cast<__hip_bfloat16 *>(gw), gb_acc, static_cast<__hip_bfloat16 *>(gb), s, pad.p, pad.unit,
-                       pad.unit_p);
+                       pad.unit_p, accumulate ? 1 : 0);
   return check_launch("dcn_weight_add_padded_kernel");
 }
 

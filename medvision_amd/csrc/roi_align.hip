@@ -105,17 +105,39 @@ __global__ __launch_bounds__(kRoiThreads) void roi_backward_kernel(const T *__re
   }
 }
 
-__global__ void fill_zero_kernel(float *p, long n) {
-  for (long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; i < n;
-       i += static_cast<long>(gridDim.x) * blockDim.x)
-    p[i] = 0.f;
+// bytes of zeros, 16 per store but for the ragged ends
+__global__ __launch_bounds__(256) void fill_zero_kernel(unsigned char *p, long head, long quads, long tail) {
+  const long t = blockIdx.x * 256L + threadIdx.x, step = gridDim.x * 256L;
+  uint4 *body = reinterpret_cast<uint4 *>(p + head);
+  for (long i = t; i < quads; i += step) body[i] = make_uint4(0u, 0u, 0u, 0u);
+  if (t < head) p[t] = 0;
+  if (t < tail) p[head + quads * 16 + t] = 0;
+}
+int fill_zero(void *p, size_t bytes, hipStream_t s) {
+  if (bytes == 0) return MV_OK;
+  const long n = static_cast<long>(bytes), head = std::min<long>((16 - reinterpret_cast<uintptr_t>(p) % 16) % 16, n);
+  const long quads = (n - head) / 16;
+  const long blocks = std::min<long>(std::max<long>((quads + 1023) / 1024, 1), 65536);
+  hipLaunchKernelGGL(fill_zero_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, static_cast<unsigned char *>(p),
+                     head, quads, n - head - quads * 16);
+  return check_launch("fill_zero_kernel");
 }
 
+// dst = src, added to what dst holds when `accumulate`
 template <typename T>
-__global__ void add_from_f32_kernel(T *dst, const float *src, long n) {
+__global__ void add_from_f32_kernel(T *dst, const float *src, long n, int accumulate) {
   for (long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x; i < n;
        i += static_cast<long>(gridDim.x) * blockDim.x)
-    dst[i] = store_cast<T>(load(dst + i) + src[i]);
+    dst[i] = store_cast<T>(accumulate ? load(dst + i) + src[i] : src[i]);
+}
+int add_from_f32(void *dst, const float *src, long n, int dtype, bool accumulate, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(std::min<long>((n + 1023) / 1024, 65536)));
+  if (dtype == MV_F16)
+    hipLaunchKernelGGL((add_from_f32_kernel<__half>), grid, dim3(256), 0, s, static_cast<__half *>(dst), src, n, accumulate ? 1 : 0);
+  else
+    hipLaunchKernelGGL((add_from_f32_kernel<__hip_bfloat16>), grid, dim3(256), 0, s, static_cast<__hip_bfloat16 *>(dst), src, n,
+                       accumulate ? 1 : 0);
+  return check_launch("add_from_f32_kernel");
 }
 
 // roi_resample.hip: tiled LDS-staged forward; returns -1 when it does not apply
@@ -141,6 +163,13 @@ int roi_pool_prepare(const void *input, int dtype, const RoiProblem &p, void *pr
 int roi_pool_backward(const void *grad_output, const void *rois, void *acc, int dtype,
                       const RoiProblem &p, hipStream_t s, bool channels_last);
 bool roi_pool_applies(int dtype, const RoiProblem &p);
+// roi_plane.hip: heads on images with plain boxes; -1 (0 parts): not for this problem
+size_t roi_plane_forward_workspace(int dtype, const RoiProblem &p);
+int roi_plane_forward(const void *input, const void *rois, void *output, int dtype, const RoiProblem &p, void *workspace,
+                      size_t capacity, hipStream_t s);
+int roi_plane_backward_parts(int dtype, const RoiProblem &p);
+int roi_plane_backward(const void *grad_output, const void *rois, void *grad, float *acc, int dtype, const RoiProblem &p,
+                       int parts, bool accumulate, hipStream_t s);
 // roi_gather_backward.hip: atomic-free backward for resampling-sized problems; -1 when not applicable
 // roi_box.hip: backward of small outputs that the pooled kernels do not take (rotated boxes, large
 // grids), one workgroup per (roi, channel group) with LDS tiles of the source boxes; -1 when not applicable
@@ -151,9 +180,9 @@ int roi_forward_cl(const void *input, const void *rois, void *output, int dtype,
                    void *workspace, size_t capacity, hipStream_t s);
 
 int roi_backward_gather(const void *grad_output, const void *rois, void *grad_input, int dtype,
-                        const RoiProblem &p, hipStream_t s);
-// dcn3d_mfma_backward.hip: dst [B, C, P] += src [B, P, C] fp32
-int planar_add_f32(const float *src, void *dst, int B, int C, long P, int dtype, hipStream_t stream);
+                        const RoiProblem &p, bool accumulate, hipStream_t s);
+// dcn3d_mfma_backward.hip: dst [B, C, P] += (not `accumulate`: =) src [B, P, C] fp32
+int planar_add_f32(const float *src, void *dst, int B, int C, long P, int dtype, bool accumulate, hipStream_t stream);
 
 static int make_problem(RoiProblem &p, int ndim, int rotated, int batch, int channels, int depth,
                         int height, int width, int num_rois, int out_d, int out_h, int out_w,
@@ -213,12 +242,14 @@ int roi_forward(const void *input, const void *rois, void *output, int dtype, in
   {
     // (a workspace too small for a path selects the kernels that need none)
     const size_t capacity = workspace ? workspace_bytes : 0;
-    if (prepared != nullptr) {   // (a copy the pooled kernels have no use for is left alone)
+    if (prepared != nullptr && p.ndim == 3) {   // (a copy the pooled kernels have no use for is left alone)
       const int pooled = roi_pool_forward(input, rois, output, dtype, p, workspace, capacity, s, prepared);
       if (pooled >= 0) return pooled;
     }
     const int tiled = roi_forward_tiled(input, rois, output, dtype, p, workspace, capacity, nullptr, s);
     if (tiled >= 0) return tiled;
+    const int plane = roi_plane_forward(input, rois, output, dtype, p, workspace, capacity, s);
+    if (plane >= 0) return plane;
     const int pooled = order != 3 ? roi_pool_forward(input, rois, output, dtype, p, workspace, capacity, s) : -1;
     if (pooled >= 0) return pooled;
     const int wide = order != 3 ? roi_forward_cl(input, rois, output, dtype, p, workspace, capacity, s) : -1;
@@ -239,70 +270,79 @@ int roi_forward(const void *input, const void *rois, void *output, int dtype, in
   return check_launch("roi_forward_kernel");
 }
 
+// `accumulate`: the gradient is added to what grad_input holds; otherwise it replaces it (a path that writes every voxel
+// then neither reads nor clears it; the others clear it first)
 int roi_backward(const void *grad_output, const void *rois, void *grad_input, int dtype, int ndim,
                  int rotated, int batch, int channels, int depth, int height, int width,
                  int num_rois, int out_d, int out_h, int out_w, float spatial_scale,
-                 int sampling_ratio, int aligned, int order, void *workspace, void *stream) {
+                 int sampling_ratio, int aligned, int order, void *workspace, void *stream, bool accumulate) {
   RoiProblem p;
   int st = make_problem(p, ndim, rotated, batch, channels, depth, height, width, num_rois, out_d,
                         out_h, out_w, spatial_scale, sampling_ratio, aligned, order);
   if (st) return st;
-  if (num_rois == 0) return MV_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const long total = static_cast<long>(batch) * channels * depth * height * width;
+  auto clear_gradient = [&] {
+    return accumulate ? MV_OK : fill_zero(grad_input, static_cast<size_t>(total) * dtype_size(dtype), s);
+  };
+  if (num_rois == 0) {
+    MV_REQUIRE(accumulate || grad_input, "null pointer argument");
+    return clear_gradient();
+  }
   MV_REQUIRE(grad_output && rois && grad_input, "null pointer argument");
   const bool narrow = dtype == MV_F16 || dtype == MV_BF16;
   MV_REQUIRE(!narrow || workspace, "16-bit backward needs an fp32 workspace");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const long total = static_cast<long>(batch) * channels * depth * height * width;
-  const int fill_blocks = static_cast<int>(std::min<long>((total + 1023) / 1024, 65536));
-  if (roi_backward_tiled_direct(dtype, p, grad_input))
-    return roi_backward_tiled(grad_output, rois, grad_input, dtype, p, s, true);
+  float *const ws = static_cast<float *>(workspace);
+  // sums that several workgroups add to: the fp32 workspace of 16-bit tensors (folded into the gradient afterwards), the
+  // gradient itself otherwise
+  void *const sums = narrow ? workspace : grad_input;
+  auto clear_sums = [&] { return narrow ? fill_zero(ws, static_cast<size_t>(total) * 4, s) : clear_gradient(); };
+  auto fold_sums = [&] { return narrow ? add_from_f32(grad_input, ws, total, dtype, accumulate, s) : MV_OK; };
+  if (roi_backward_tiled_direct(dtype, p, grad_input)) {
+    st = clear_gradient();
+    return st ? st : roi_backward_tiled(grad_output, rois, grad_input, dtype, p, s, true);
+  }
   if (roi_backward_tiled_applies(dtype, p)) {
-    // 16-bit tensors: sums in the fp32 workspace; fp32: sums in grad_input
-    float *ws = static_cast<float *>(workspace);
-    if (narrow) hipLaunchKernelGGL(fill_zero_kernel, dim3(fill_blocks), dim3(256), 0, s, ws, total);
-    st = roi_backward_tiled(grad_output, rois, narrow ? ws : static_cast<float *>(grad_input), dtype, p, s);
-    if (st) return st;
-    if (!narrow) return MV_OK;
-    MV_DISPATCH(dtype, {
-      if constexpr (sizeof(T) == 2)
-        hipLaunchKernelGGL((add_from_f32_kernel<T>), dim3(fill_blocks), dim3(256), 0, s,
-                           static_cast<T *>(grad_input), static_cast<const float *>(workspace), total);
-    });
-    return check_launch("add_from_f32_kernel");
+    st = clear_sums();
+    if (!st) st = roi_backward_tiled(grad_output, rois, sums, dtype, p, s);
+    return st ? st : fold_sums();
   }
-  const int gathered = roi_backward_gather(grad_output, rois, grad_input, dtype, p, s);
+  const int gathered = roi_backward_gather(grad_output, rois, grad_input, dtype, p, accumulate, s);
   if (gathered >= 0) return gathered;
-  const dim3 grid(p.chunks * num_rois), block(kRoiThreads);
-  if (narrow) {
-    hipLaunchKernelGGL(fill_zero_kernel, dim3(fill_blocks), dim3(256), 0, s,
-                       static_cast<float *>(workspace), total);
+  if (const int parts = roi_plane_backward_parts(dtype, p)) {
+    if (parts > 1) {
+      st = clear_sums();
+      if (st) return st;
+    }
+    st = roi_plane_backward(grad_output, rois, grad_input, static_cast<float *>(sums), dtype, p, parts, accumulate, s);
+    if (st >= 0) return st || parts == 1 ? st : fold_sums();
   }
+  st = clear_sums();
+  if (st) return st;
   // 16-bit pooled path: the fp32 workspace is used channels-last and folded in by a transposing add
   const bool channels_last = narrow && roi_pool_applies(dtype, p);
-  const int pooled = roi_pool_backward(grad_output, rois, narrow ? workspace : grad_input, dtype, p, s, channels_last);
+  const int pooled = roi_pool_backward(grad_output, rois, sums, dtype, p, s, channels_last);
   if (pooled > 0) return pooled;
   if (pooled == 0 && channels_last)
-    return planar_add_f32(static_cast<const float *>(workspace), grad_input, batch, channels,
-                          static_cast<long>(depth) * height * width, dtype, s);
-  const int boxed = pooled < 0 ? roi_box_backward(grad_output, rois, static_cast<float *>(narrow ? workspace : grad_input), dtype, p, s) : -1;
+    return planar_add_f32(ws, grad_input, batch, channels, static_cast<long>(depth) * height * width, dtype, accumulate, s);
+  const int boxed = pooled < 0 ? roi_box_backward(grad_output, rois, static_cast<float *>(sums), dtype, p, s) : -1;
   if (boxed > 0) return boxed;
-  MV_DISPATCH(dtype, {
-    using RT = typename std::conditional<std::is_same<T, double>::value, double, float>::type;
-    using G = typename std::conditional<(sizeof(T) == 2), float, T>::type;
-    G *acc = narrow ? static_cast<G *>(workspace) : static_cast<G *>(grad_input);
-    if (pooled == 0 || boxed == 0) {
-      // gradient already accumulated by the pooled / box kernel
-    } else if (rotated)
-      hipLaunchKernelGGL((roi_backward_kernel<T, G, RT, true>), grid, block, 0, s,
-                         static_cast<const T *>(grad_output), static_cast<const RT *>(rois), acc, p);
-    else
-      hipLaunchKernelGGL((roi_backward_kernel<T, G, RT, false>), grid, block, 0, s,
-                         static_cast<const T *>(grad_output), static_cast<const RT *>(rois), acc, p);
-    if (sizeof(T) == 2)
-      hipLaunchKernelGGL((add_from_f32_kernel<T>), dim3(fill_blocks), dim3(256), 0, s,
-                         static_cast<T *>(grad_input), static_cast<const float *>(workspace), total);
-  });
-  return check_launch("roi_backward_kernel");
+  if (pooled < 0 && boxed < 0) {
+    const dim3 grid(p.chunks * num_rois), block(kRoiThreads);
+    MV_DISPATCH(dtype, {
+      using RT = typename std::conditional<std::is_same<T, double>::value, double, float>::type;
+      using G = typename std::conditional<(sizeof(T) == 2), float, T>::type;
+      if (rotated)
+        hipLaunchKernelGGL((roi_backward_kernel<T, G, RT, true>), grid, block, 0, s,
+                           static_cast<const T *>(grad_output), static_cast<const RT *>(rois), static_cast<G *>(sums), p);
+      else
+        hipLaunchKernelGGL((roi_backward_kernel<T, G, RT, false>), grid, block, 0, s,
+                           static_cast<const T *>(grad_output), static_cast<const RT *>(rois), static_cast<G *>(sums), p);
+    });
+    st = check_launch("roi_backward_kernel");
+    if (st) return st;
+  }
+  return fold_sums();
 }
 
 }  // namespace mv
@@ -358,13 +398,24 @@ int mv_roi_align_forward_prepared(const void *input, const void *prepared, const
                      workspace, workspace_bytes, stream, false, prepared);
 }
 
+int mv_roi_align_backward_write(const void *grad_output, const void *rois, void *grad_input, int dtype, int ndim,
+                                int rotated, int batch, int channels, int depth, int height, int width, int num_rois,
+                                int out_d, int out_h, int out_w, float spatial_scale, int sampling_ratio, int aligned,
+                                int order, void *workspace, void *stream) {
+  MV_REQUIRE(ndim == 2 || ndim == 3, "ndim must be 2 or 3");
+  const bool flat = ndim == 2;
+  return roi_backward(grad_output, rois, grad_input, dtype, ndim, rotated ? 1 : 0, batch, channels, flat ? 1 : depth, height,
+                      width, num_rois, flat ? 1 : out_d, out_h, out_w, spatial_scale, sampling_ratio,
+                      rotated ? aligned : 1, order, workspace, stream, false);
+}
+
 int mv_roi_align_2d_backward(const void *grad_output, const void *rois, void *grad_input,
                              int dtype, int batch, int channels, int height, int width,
                              int num_rois, int out_h, int out_w, float spatial_scale,
                              int sampling_ratio, int order, void *workspace, void *stream) {
   return roi_backward(grad_output, rois, grad_input, dtype, 2, 0, batch, channels, 1, height,
                       width, num_rois, 1, out_h, out_w, spatial_scale, sampling_ratio, 1, order,
-                      workspace, stream);
+                      workspace, stream, true);
 }
 
 int mv_roi_align_3d_forward(const void *input, const void *rois, void *output, int dtype,
@@ -382,7 +433,7 @@ int mv_roi_align_3d_backward(const void *grad_output, const void *rois, void *gr
                              int sampling_ratio, int order, void *workspace, void *stream) {
   return roi_backward(grad_output, rois, grad_input, dtype, 3, 0, batch, channels, depth, height,
                       width, num_rois, out_d, out_h, out_w, spatial_scale, sampling_ratio, 1,
-                      order, workspace, stream);
+                      order, workspace, stream, true);
 }
 
 int mv_roi_align_rotated_2d_forward(const void *input, const void *rois, void *output, int dtype,
@@ -401,7 +452,7 @@ int mv_roi_align_rotated_2d_backward(const void *grad_output, const void *rois, 
                                      void *stream) {
   return roi_backward(grad_output, rois, grad_input, dtype, 2, 1, batch, channels, 1, height,
                       width, num_rois, 1, out_h, out_w, spatial_scale, sampling_ratio, aligned,
-                      order, workspace, stream);
+                      order, workspace, stream, true);
 }
 
 int mv_roi_align_rotated_3d_forward(const void *input, const void *rois, void *output, int dtype,
@@ -422,7 +473,7 @@ int mv_roi_align_rotated_3d_backward(const void *grad_output, const void *rois, 
                                      int order, void *workspace, void *stream) {
   return roi_backward(grad_output, rois, grad_input, dtype, 3, 1, batch, channels, depth, height,
                       width, num_rois, out_d, out_h, out_w, spatial_scale, sampling_ratio, aligned,
-                      order, workspace, stream);
+                      order, workspace, stream, true);
 }
 
 size_t mv_roi_align_forward_workspace_bytes(int dtype, int ndim, int channels, int num_rois,
@@ -445,7 +496,7 @@ size_t mv_roi_align_forward_workspace_bytes_for_input(int dtype, int ndim, int b
   p.od = ndim == 2 ? 1 : out_d; p.oh = out_h; p.ow = out_w; p.sampling_ratio = sampling_ratio; p.order = 1;
   if (batch <= 0 || channels <= 0 || p.D <= 0 || height <= 0 || width <= 0 || num_rois <= 0) return basic;
   if (basic || dtype == MV_I32) return basic;   // (the tiled resampler takes the problem; label maps have no other path that wants memory)
-  const size_t pooled = mv::roi_pool_forward_workspace(dtype, p);
+  const size_t pooled = std::max(mv::roi_pool_forward_workspace(dtype, p), mv::roi_plane_forward_workspace(dtype, p));
   return pooled ? pooled : mv::roi_forward_cl_workspace(dtype, p);
 }
 

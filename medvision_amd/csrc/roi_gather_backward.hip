@@ -230,7 +230,7 @@ __device__ __forceinline__ typename Acc<T>::type gather_voxel(const GatherGeo &q
 template <typename T, typename RT, bool EXACT, int PER>
 __device__ __forceinline__ void gather_block(const T *__restrict__ gout, const RT *__restrict__ rois, T *__restrict__ gin,
                                              const RoiProblem &p, const unsigned walk_begin, const unsigned walk_count,
-                                             const unsigned block_x) {
+                                             const unsigned block_x, const int accumulate) {
   using A = typename Acc<T>::type;
   using C = typename std::conditional<EXACT, double, float>::type;
   __shared__ GatherShared sh;
@@ -300,15 +300,15 @@ __device__ __forceinline__ void gather_block(const T *__restrict__ gout, const R
       if (sum != A(0)) sums[k * kGatherThreads + threadIdx.x] += sum;
     }
   }
-  // this thread owns its voxels: plain read-modify-write
+  // this thread owns its voxels: plain read-modify-write, or plain writes of all of them
   for (int k = 0; k < PER; k++) {
     const long vi = first + static_cast<long>(k) * kGatherThreads;
     const A total = sums[k * kGatherThreads + threadIdx.x];
-    if (vi < walk_end && total != A(0)) {
+    if (vi < walk_end && (total != A(0) || !accumulate)) {
       int v[3];
       shell.voxel(static_cast<unsigned>(vi), v);
       T *at = dst + (static_cast<long>(v[2]) * p.H + v[1]) * p.W + v[0];
-      *at = store_cast<T>(load(at) + total);
+      *at = store_cast<T>(accumulate ? load(at) + total : total);
     }
   }
 }
@@ -319,18 +319,18 @@ __device__ __forceinline__ void gather_block(const T *__restrict__ gout, const R
 template <typename T, typename RT>
 __global__ __launch_bounds__(kGatherThreads) __attribute__((amdgpu_waves_per_eu(5))) void roi_backward_gather_kernel(
     const T *__restrict__ gout, const RT *__restrict__ rois, T *__restrict__ gin, const RoiProblem p,
-    const unsigned inner, const unsigned plane, const unsigned exact_blocks) {
+    const unsigned inner, const unsigned plane, const unsigned exact_blocks, const int accumulate) {
   if (blockIdx.x < exact_blocks)
-    gather_block<T, RT, true, 1>(gout, rois, gin, p, inner, plane - inner, blockIdx.x);
+    gather_block<T, RT, true, 1>(gout, rois, gin, p, inner, plane - inner, blockIdx.x, accumulate);
   else
-    gather_block<T, RT, false, kGatherPerThread>(gout, rois, gin, p, 0u, inner, blockIdx.x - exact_blocks);
+    gather_block<T, RT, false, kGatherPerThread>(gout, rois, gin, p, 0u, inner, blockIdx.x - exact_blocks, accumulate);
 }
 
 // Applies when the problem is a resampling: one sample per cell, outputs of at least 4096 voxels
 // that are not much smaller than the image, at most two rois per image on average (every input
 // voxel walks over all rois of its image).  Returns -1 otherwise.
 int roi_backward_gather(const void *grad_output, const void *rois, void *grad_input, int dtype,
-                        const RoiProblem &p, hipStream_t s) {
+                        const RoiProblem &p, bool accumulate, hipStream_t s) {
   const long plane = static_cast<long>(p.D) * p.H * p.W;
   const long ocells = static_cast<long>(p.od) * p.oh * p.ow;
   if (p.sampling_ratio != 1 || (p.order != 0 && p.order != 1)) return -1;
@@ -350,7 +350,7 @@ int roi_backward_gather(const void *grad_output, const void *rois, void *grad_in
     hipLaunchKernelGGL((roi_backward_gather_kernel<T, RT>), grid, block, 0, s,
                        static_cast<const T *>(grad_output), static_cast<const RT *>(rois),
                        static_cast<T *>(grad_input), p, inner, static_cast<unsigned>(plane),
-                       static_cast<unsigned>(exact_blocks));
+                       static_cast<unsigned>(exact_blocks), accumulate ? 1 : 0);
   });
   return check_launch("roi_backward_gather_kernel");
 }

@@ -1,0 +1,42 @@
+"""Heads on images with plain boxes: the matrix-core kernels at the edges of their tiles and lists, forward and
+backward, against the fp64 oracle."""
+import pytest
+import torch
+
+from parity import BWD_TOL, FWD_TOL, assert_close
+import workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("size,channels,rois,cells,ratio,order,reach", [
+    ((33, 47), 37, 9, (7, 7), 0, 1, 40),      # tiles and channels with remainders, boxes over the border
+    ((16, 16), 8, 1, (8, 8), 2, 1, 16),       # one tile, whole cells
+    ((40, 21), 5, 6, (14, 14), 2, 1, 30),     # the 16-cell kernels
+    ((50, 64), 3, 40, (16, 9), 1, 0, 30),     # nearest taps, cells of both sizes
+    ((20, 3), 4, 5, (5, 3), 2, 1, 12),        # rows shorter than a load
+    ((9, 9), 2, 3, (1, 5), 0, 1, 9),          # a single row of cells
+    ((300, 180), 4, 4, (7, 7), 0, 1, 290),    # more rows and columns than the forward lists hold
+    ((24, 24), 16, 1100, (7, 7), 2, 1, 12),   # more rois than one look-through, several workgroups per tile
+    ((260, 260), 64, 300, (7, 7), 2, 1, 60),  # features beyond an L2: rois ordered first
+    ((12, 12), 3, 4, (3, 1), 2, 1, 9),        # too few cells for the matrix cores
+])
+def test_plane_heads(oracle, dtype, size, channels, rois, cells, ratio, order, reach):
+    from medvision_amd.ops.roi_align_nd import roi_align_2d
+    g = wl.gen(sum(size) + rois + channels)
+    batch = 2
+    feat = torch.randn(batch, channels, *size, generator=g).to(dtype)
+    at = torch.rand(rois, 2, generator=g) * torch.tensor(size[::-1]) * 1.2 - 4.0
+    extent = torch.rand(rois, 2, generator=g) * reach
+    image = torch.randint(0, batch, (rois, 1), generator=g).float()
+    boxes = torch.cat([image, at, at + extent], 1)
+    x = feat.to(DEV).requires_grad_()
+    out = roi_align_2d(x, boxes.to(DEV), cells, 0.5, ratio, order)
+    assert_close(out, oracle.roi_align_forward(feat, boxes, cells, 0.5, ratio, True, order, False), FWD_TOL[dtype], "forward")
+    gy = torch.randn(out.shape, generator=g).to(dtype)
+    out.backward(gy.to(DEV))
+    want = oracle.roi_align_backward(gy, boxes, feat.shape, 0.5, ratio, True, order, False)
+    assert_close(x.grad, want, BWD_TOL[dtype], "backward")
