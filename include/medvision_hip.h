@@ -198,9 +198,9 @@ int mv_dcn3d_backward_write(const void *input, const void *offset, const void *m
                             void *grad_mask, void *grad_weight, void *grad_bias,
                             const mv_dcn3d_shape *shape, int dtype, void *workspace, void *stream);
 
-/* Budget of the backward pass's column buffer in bytes (default 1 GiB, or MV_DCN_COLUMN_BYTES in the
- * environment when the library is first asked).  Changing it changes what
- * mv_dcn{2,3}d_backward_workspace_bytes() returns: query again.  No counterpart in the reference
+/* Budget of the column buffer that the backward pass of earlier versions kept (default 1 GiB, or
+ * MV_DCN_COLUMN_BYTES in the environment when the library is first asked).  The pass has no such buffer any
+ * more: the value is stored and returned, and changes nothing.  No counterpart in the reference
  * (its column buffer is a tensor argument, csrc/modulated_deform_conv_3d.h:89).               */
 void mv_dcn_set_column_budget(size_t bytes);
 size_t mv_dcn_column_budget(void);

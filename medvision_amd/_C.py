@@ -363,8 +363,8 @@ def _dcn_backward(input, offset, mask, weight, grad_output, gi, goff, gmask, gw,
 
 
 def set_dcn_column_budget(nbytes):
-    """Budget (bytes) of the column buffer the DCN backward keeps for its weight kernel; layers
-    beyond it gather the input a second time.  Returns the previous budget."""
+    """Budget (bytes) of the column buffer that the DCN backward of earlier versions kept: stored and
+    returned, without effect.  Returns the previous budget."""
     lib = _lib.load()
     old = lib.mv_dcn_column_budget()
     lib.mv_dcn_set_column_budget(int(nbytes))

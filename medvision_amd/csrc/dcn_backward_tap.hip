@@ -1,0 +1,433 @@
+// Backward of the deformable convolution on the matrix cores: gradients of the offsets, the mask and the weight, and the
+// far corners of the gradient of the input (dcn3d_mfma_backward.hip has the equations and the kernels around this one).
+//
+// One workgroup = one TAP, a range of positions and a chunk of input channels.  With the tap fixed,
+//   * its weight block Wt_k [channels x output channels] sits in registers for the whole range,
+//   * the gradient of that block, gw_k = gy col_k^T, stays in accumulators over the range (added to memory once),
+//   * the column values mask * Z(x) go from the lanes that blend them through LDS into that product,
+// so that there is no column buffer and no second gather of x, and a layer of a few thousand positions has taps x ranges
+// workgroups instead of one wavefront per 32 positions.  64 positions at a time, grad_output of them in LDS:
+//   1  gcol = Wt_k^T gy (16 x 16 MFMA, rows = channels), through LDS to the load layout (position l / 4, 16-byte piece
+//      l % 4: a voxel's pieces are one cache look-up);
+//   2  every wavefront samples 16 positions: the corners' pieces are loaded once and used twice, blended into the column
+//      value and multiplied with gcol into one sum per corner, D_c = sum over channels of gcol * x_c.  The trilinear form is
+//      linear in the corners, so value and derivatives come from the eight D once per position instead of from
+//      eight x once per channel (16-bit tensors; fp32 forms the differences per channel, which is kinder to sums of
+//      nearly equal corners);
+//   3  gw_k += gy col_k^T, a quarter of the output channels per wavefront, both operands by transposing LDS reads.
+// Corners that the LDS scatter does not take are listed when the records are made, and their 32 channels are added as
+// 128 contiguous bytes.
+// What bounds it: narrow layers the vector instructions of the samples (128 multiply-adds and as many more for everything
+// else per 16 positions and 32 channels), wide ones the matrix cores and LDS, and everywhere the atomics of the far
+// corners (64 bytes per corner and 16 channels, 21 G of them a second at best).
+//   (bf16 [2, 32 -> 64, 48^3]: 343 us without the far corners; the data and weight kernels before it took 670 us.  fp16
+//   images [8, 256 -> 256, 100 x 152]: 694 us, 4380 us before.  [1, 128 -> 128, 7 x 45 x 18]: 64 us, 790 us before.)
+#include "dcn_scatter.hpp"
+
+namespace mv {
+
+// One 16-byte piece (kPiece neighbouring channels of a position) of an LDS block [piece][position]: rows of 68 pieces, so that
+// both the four pieces of neighbouring positions and one piece of sixteen positions fall on different banks.
+constexpr int kTapTile = 64, kTapPitch = kTapTile + 4;   // positions per turn
+__device__ __forceinline__ int tap_slot(int piece, int position) { return piece * kTapPitch + position; }
+
+// Operand of a product over positions from such a block: row `block * 16 + lane % 16` (a channel), the kPiece positions
+// 4 * kPiece * ks + ... that belong to lane group lane / 16.  16-bit: two transposing reads (lane 4 e + t of a group of sixteen
+// addresses channels 4 t .. 4 t + 3 of position e, lane i gets channel i of the four positions).
+template <typename T> __device__ __forceinline__ u32x4 tap_transposed(const u32x4 *base, int block, int ks, int lane) {
+  const int kc = lane / 16, i = lane % 16;
+  if constexpr (sizeof(T) == 2) {
+    typedef short s16x4 __attribute__((ext_vector_type(4)));
+    typedef __attribute__((address_space(3))) s16x4 *lds_ptr;
+    const int piece = block * 2 + (i % 4) / 2, half = i % 2, position = ks * 32 + kc * 8 + i / 4;
+    const auto at = [&](int add) {
+      return (lds_ptr)(reinterpret_cast<s16x4 *>(const_cast<u32x4 *>(base + tap_slot(piece, position + add))) + half);
+    };
+    union { s16x4 h[2]; u32x4 u; } r;
+    r.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(at(0));
+    r.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(at(4));
+    return r.u;
+  } else {
+    const int piece = block * 4 + i / 4;
+    union { unsigned e[4]; u32x4 u; } r;
+#pragma unroll
+    for (int t = 0; t < 4; t++) r.e[t] = reinterpret_cast<const unsigned *>(base + tap_slot(piece, ks * 16 + kc * 4 + t))[i % 4];
+    return r.u;
+  }
+}
+
+// workgroups per compute unit that the registers should leave room for
+template <typename T, int NC, int OBW, int CBW>
+constexpr int TAP_WAVES = OBW * CBW >= 8 || (NC == 8 && (sizeof(T) == 4 || OBW >= 2)) ? 2 : OBW == 1 && CBW == 2 && sizeof(T) == 2 ? 4 : 3;
+
+// OBW: blocks of 16 output channels per wavefront (every fourth block of the 64 * OBW rows from row0; layers with more rows
+// take several passes, gcol and all that follows from it being sums over them).  CBW: blocks of 16 input channels of a
+// chunk.  NC: corners, 8 for volumes, 4 for images.
+template <typename T, int NC, int OBW, int CBW>
+__global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backward_tap_kernel(
+    const T *__restrict__ xt, const T *__restrict__ off, const T *__restrict__ mask, const T *__restrict__ gyt,
+    const T *__restrict__ wf, float *__restrict__ gxt, T *__restrict__ goff, T *__restrict__ gmask,
+    float *__restrict__ partial, float *__restrict__ gw, const DcnDims s, const unsigned *__restrict__ bounds,
+    const int chunks, const int shares, const int range, const int row0) {
+  using M = Mfma<T>;
+  using P = typename std::conditional<(sizeof(T) == 2), float, double>::type;  // position type
+  using S = typename std::conditional<NC == 8, VolumeBricks, ImageBricks>::type;
+  constexpr int PC = M::kPiece, SL = 4 * PC, ES = sizeof(T), CW = 16 * CBW, ROWS = 64 * OBW;
+  constexpr int BPI = SL / 16, ITEMS = CBW / BPI, KS = kTapTile / SL;   // 16-channel blocks per item; items; K steps of a tile
+  constexpr int STEPS = ROWS / SL, STAGED = ROWS * kTapTile / PC / 256;
+  constexpr int RW = 2 * NC + 4, kRecs = 2 * kTapTile, GP = CW + 4;
+  __shared__ __attribute__((aligned(16))) unsigned rec[kRecs][RW];          // at[NC], mask * w[NC], ld, lh, lw, mask
+  __shared__ u32x4 gyl[ROWS / PC * kTapPitch];                               // grad_output, pieces of output channels
+  __shared__ u32x4 col[CW / PC * kTapPitch];                                 // column values, pieces of input channels
+  __shared__ __attribute__((aligned(16))) float gcol[kTapTile][GP];
+  __shared__ uint2 far_list[2][kTapTile * NC];   // {offset in the gradient buffer | position, mask * weight}
+  __shared__ int far_count[2];
+  const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int j = lane % 16, kc = lane / 16;   // matrix layout
+  const int lj = lane / 4, lk = lane % 4;    // load layout
+  // (taps of one range next to each other, on one XCD: they gather the same part of x and read the same gy)
+  const int id = static_cast<int>(xcd_contiguous(blockIdx.x, gridDim.x)), k = id % s.K;
+  const int dgi = blockIdx.y / chunks, part = blockIdx.y % chunks, b = blockIdx.z;
+  const int c0 = dgi * s.cpd + part * CW, g = c0 / s.cpg;
+  const long q0 = static_cast<long>(id / s.K) * range;
+  const int count = static_cast<int>(min(static_cast<long>(range), s.Q - q0));   // positions of the range
+  const long bg = static_cast<long>(b) * s.dg + dgi;
+  const int rows = min(ROWS, s.opg - row0), steps = rows / SL;
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T *>(xt + static_cast<long>(b) * s.P * s.Cin), 0, static_cast<int>(s.P * s.Cin * ES), kRsrcFlags);
+  const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
+      gxt + static_cast<long>(b) * s.P * s.Cin, 0, static_cast<int>(s.P * s.Cin * 4), kRsrcFlags);
+  const bool split = bounds && scatter_scale(bounds, S::BD * S::BH * S::BW * s.K, mask != nullptr).valid;
+
+  // gcol: wavefront w forms the channels of block w % CBW for CBW blocks of sixteen positions; its rows of the weight stay
+  // in registers for the whole range
+  const int wblock = wave % CBW, wfirst = wave / CBW * CBW;
+  u32x4 wreg[STEPS];
+  {
+    const T *src = wf + (((static_cast<long>(g) * s.K + k) * (s.cpg / 16) + (c0 - g * s.cpg) / 16 + wblock) * (s.opg / SL) + row0 / SL) * (64 * PC) + lane * PC;
+#pragma unroll
+    for (int st = 0; st < STEPS; st++)
+      wreg[st] = st < steps ? *reinterpret_cast<const u32x4 *>(src + st * (64 * PC)) : u32x4{0u, 0u, 0u, 0u};
+  }
+  // grad_output of a tile, loaded a tile ahead where the registers allow it: thread t has piece t % NP of positions t / NP +
+  // u * 256 / NP (positions and rows that do not exist: zeros)
+  constexpr bool AHEAD = STAGED <= 4;
+  constexpr int NP = ROWS / PC;
+  const int cout_bytes = s.Cout * ES, tpiece = tid % NP, tposition = tid / NP;
+  const __amdgpu_buffer_rsrc_t gyr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T *>(gyt + (static_cast<long>(b) * s.Q + q0) * s.Cout), 0, count * cout_bytes, kRsrcFlags);
+  const unsigned stage_at = tpiece * PC < rows ? static_cast<unsigned>(tposition * cout_bytes + tpiece * 16) : kOob;
+  u32x4 *const keep_at = gyl + tap_slot(tpiece, tposition);
+  u32x4 staged[STAGED];
+  auto stage = [&](int tile) {
+#pragma unroll
+    for (int u = 0; u < STAGED; u++)
+      staged[u] = __builtin_amdgcn_raw_buffer_load_b128(gyr, stage_at, (tile * kTapTile + u * (256 / NP)) * cout_bytes + (g * s.opg + row0) * ES, 0);
+  };
+  auto keep = [&] {
+#pragma unroll
+    for (int u = 0; u < STAGED; u++) keep_at[u * (256 / NP)] = staged[u];
+  };
+
+  // ---- records: thread t < 128 works out position t of the next two tiles; its offsets are requested a block ahead -----
+  const int ti = k / (s.kh * s.kw), tj = (k / s.kw) % s.kh, tk = k % s.kw;
+  const T *const ob = off + (bg * s.nd * s.K + s.nd * k) * s.Q, *const mb = mask ? mask + (bg * s.K + k) * s.Q : nullptr;
+  P fd = P(0), fh = P(0), fw = P(0);
+  float fm = 1.f;
+  auto request = [&](int first) {
+    const long q = q0 + min(first + tid, count - 1);
+    dcn_offsets(s, ob + q, fd, fh, fw);
+    if (mb) fm = load(mb + q);
+  };
+  auto publish = [&](int first) {
+    const bool live = first + tid < count;
+    const int qc = static_cast<int>(q0) + min(first + tid, count - 1);
+    const int ow = qc % s.Wo, t = qc / s.Wo, oh = t % s.Ho, od = t / s.Ho;
+    P pd = fd + static_cast<P>(od * s.sd - s.pd + ti * s.dd);
+    const P ph = fh + static_cast<P>(oh * s.sh - s.ph + tj * s.dh), pw = fw + static_cast<P>(ow * s.sw - s.pw + tk * s.dw);
+    if (NC == 4) pd = P(0);   // images: the only slice
+    CornerTaps ct;
+    corner_taps<P>(s, pd, ph, pw, live, static_cast<unsigned>(s.Cin) * ES, 0u, kOob, ct);
+    unsigned *r = rec[tid];
+#pragma unroll
+    for (int c = 0; c < NC; c += 4) {
+      *reinterpret_cast<u32x4 *>(r + c) = u32x4{ct.at[c], ct.at[c + 1], ct.at[c + 2], ct.at[c + 3]};
+      *reinterpret_cast<float4 *>(r + NC + c) = make_float4(fm * ct.w[c], fm * ct.w[c + 1], fm * ct.w[c + 2], fm * ct.w[c + 3]);
+    }
+    *reinterpret_cast<float4 *>(r + 2 * NC) = make_float4(ct.ld, ct.lh, ct.lw, fm);
+    int first_cell;
+    const unsigned local = split ? tile_bits<S>(tile_origin<S>(s, od / S::BD, oh / S::BH, ow / S::BW), static_cast<int>(floor(pd)),
+                                                static_cast<int>(floor(ph)), static_cast<int>(floor(pw)), first_cell) : 0u;
+    int listed = 0;   // (the wavefront is one tile)
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+      const bool is_far = ct.at[c] != kOob && !((local >> c) & 1u);
+      const unsigned long long owners = __ballot(is_far);
+      // (a voxel's channels start at a multiple of 128 bytes: the position fits below)
+      if (is_far)
+        far_list[wave][listed + __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(owners >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(owners), 0u))] =
+            make_uint2(ct.at[c] * (4u / ES) | static_cast<unsigned>(lane), __float_as_uint(fm * ct.w[c]));
+      listed += __popcll(owners);
+    }
+    if (lane == 0) far_count[wave] = listed;
+  };
+
+  float4_t acc[OBW][CBW];
+#pragma unroll
+  for (int o = 0; o < OBW; o++)
+#pragma unroll
+    for (int c = 0; c < CBW; c++) acc[o][c] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+  // lane l % 4 stores component l % 4 of its position (d, h, w, mask)
+  float *pout = nullptr;
+  T *tout = nullptr;
+  {
+    const int p = wave * 16 + lj;
+    if (partial) pout = partial + (((bg * s.K + k) * shares + row0 / ROWS * chunks + part) * s.Q + q0 + p) * 4 + lk;
+    else if (lk == 3) tout = gmask ? gmask + (bg * s.K + k) * s.Q + q0 + p : nullptr;
+    else if (lk + s.nd >= 3) tout = goff + (bg * s.nd * s.K + s.nd * k + lk + s.nd - 3) * s.Q + q0 + p;
+  }
+  if (tid < kRecs) request(0);
+  if (AHEAD) stage(0);
+  const int tiles = (count + kTapTile - 1) / kTapTile;
+  for (int tile = 0; tile < tiles; tile++) {
+    const int half = tile & 1;
+    __syncthreads();   // the tile before has been read
+    if (!AHEAD) stage(tile);
+    keep();
+    if (half == 0 && tid < kRecs) {
+      publish(tile * kTapTile);
+      if (tile + 2 < tiles) request(tile * kTapTile + kRecs);
+    }
+    __syncthreads();
+    // ---- the sampling pieces of this wavefront's sixteen positions are on their way during the product ---------------
+    const int p = wave * 16 + lj;
+    const unsigned *r = rec[half * kTapTile + p];
+    unsigned at[NC];
+    float cw[NC];
+#pragma unroll
+    for (int c = 0; c < NC; c += 4) {
+      const u32x4 a = *reinterpret_cast<const u32x4 *>(r + c);
+      const float4 w = *reinterpret_cast<const float4 *>(r + NC + c);
+      at[c] = a.x + lk * 16u; at[c + 1] = a.y + lk * 16u; at[c + 2] = a.z + lk * 16u; at[c + 3] = a.w + lk * 16u;
+      cw[c] = w.x; cw[c + 1] = w.y; cw[c + 2] = w.z; cw[c + 3] = w.w;
+    }
+    const float4 e = *reinterpret_cast<const float4 *>(r + 2 * NC);   // ld, lh, lw, mask
+    constexpr int SETS = NC == 4 && ITEMS > 1 ? 2 : 1;   // items whose corners are in registers (volumes: one, for occupancy)
+    u32x4 raw[SETS][NC];
+    auto gather = [&](u32x4 (&to)[NC], int item) {
+#pragma unroll
+      for (int c = 0; c < NC; c++) to[c] = __builtin_amdgcn_raw_buffer_load_b128(xr, at[c], (c0 + item * SL) * ES, 0);
+    };
+    gather(raw[0], 0);
+    if (AHEAD) stage(tile + 1);   // (beyond the last one: zeros)
+    {
+      float4_t gc[CBW];
+#pragma unroll
+      for (int n = 0; n < CBW; n++) gc[n] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int st = 0; st < STEPS; st++)
+#pragma unroll
+        for (int n = 0; n < CBW; n++) gc[n] = M::run16(wreg[st], gyl[tap_slot(st * 4 + kc, (wfirst + n) * 16 + j)], gc[n]);
+#pragma unroll
+      for (int n = 0; n < CBW; n++)
+        *reinterpret_cast<float4 *>(&gcol[(wfirst + n) * 16 + j][wblock * 16 + 4 * kc]) = make_float4(gc[n][0], gc[n][1], gc[n][2], gc[n][3]);
+    }
+    __syncthreads();   // gcol is complete
+    float D[NC], t0 = 0.f, t1 = 0.f, t2 = 0.f, t3 = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; c++) D[c] = 0.f;
+#pragma unroll
+    for (int item = 0; item < ITEMS; item++) {
+      if (SETS == 2 && item + 1 < ITEMS) gather(raw[(item + 1) % SETS], item + 1);
+      const u32x4(&x)[NC] = raw[item % SETS];
+      float gv[PC], v[PC];
+#pragma unroll
+      for (int i = 0; i < PC; i += 4) {
+        const float4 t = *reinterpret_cast<const float4 *>(&gcol[p][item * SL + lk * PC + i]);
+        gv[i] = t.x; gv[i + 1] = t.y; gv[i + 2] = t.z; gv[i + 3] = t.w;
+      }
+#pragma unroll
+      for (int i = 0; i < PC; i++) v[i] = 0.f;
+#pragma unroll
+      for (int c = 0; c < NC; c++) {
+        M::fma_piece(v, cw[c], x[c]);
+        if constexpr (ES == 2) D[c] = M::dot_piece(gv, x[c], D[c]);
+      }
+      if constexpr (ES == 4) {
+#pragma unroll
+        for (int i = 0; i < PC; i++) {
+          float u[8];
+#pragma unroll
+          for (int c = 0; c < 8; c++) u[c] = c < NC ? __uint_as_float(x[c < NC ? c : 0][i]) : 0.f;
+          const float x0 = u[1] - u[0], x1 = u[3] - u[2], a0 = fmaf(e.z, x0, u[0]), a1 = fmaf(e.z, x1, u[2]);
+          const float b0 = fmaf(e.y, x1 - x0, x0), y0 = a1 - a0, v0 = fmaf(e.y, y0, a0);
+          float dw = b0, dh = y0, dd = 0.f, val = v0;
+          if constexpr (NC == 8) {
+            const float x2 = u[5] - u[4], x3 = u[7] - u[6], a2 = fmaf(e.z, x2, u[4]), a3 = fmaf(e.z, x3, u[6]);
+            const float b1 = fmaf(e.y, x3 - x2, x2), y1 = a3 - a2, v1 = fmaf(e.y, y1, a2);
+            dw = fmaf(e.x, b1 - b0, b0);
+            dh = fmaf(e.x, y1 - y0, y0);
+            dd = v1 - v0;
+            val = fmaf(e.x, dd, v0);
+          }
+          t0 = fmaf(dd, gv[i], t0); t1 = fmaf(dh, gv[i], t1); t2 = fmaf(dw, gv[i], t2); t3 = fmaf(val, gv[i], t3);
+        }
+      }
+      col[tap_slot(item * 4 + lk, p)] = M::pack(v);
+      if (SETS == 1 && item + 1 < ITEMS) gather(raw[0], item + 1);
+    }
+    if constexpr (ES == 2) {
+      const float x0 = D[1] - D[0], x1 = D[3] - D[2], a0 = fmaf(e.z, x0, D[0]), a1 = fmaf(e.z, x1, D[2]);
+      const float b0 = fmaf(e.y, x1 - x0, x0), y0 = a1 - a0, v0 = fmaf(e.y, y0, a0);
+      t2 = b0; t1 = y0; t3 = v0;
+      if constexpr (NC == 8) {
+        const float x2 = D[5] - D[4], x3 = D[7] - D[6], a2 = fmaf(e.z, x2, D[4]), a3 = fmaf(e.z, x3, D[6]);
+        const float b1 = fmaf(e.y, x3 - x2, x2), y1 = a3 - a2, v1 = fmaf(e.y, y1, a2);
+        t2 = fmaf(e.x, b1 - b0, b0);
+        t1 = fmaf(e.x, y1 - y0, y0);
+        t0 = v1 - v0;
+        t3 = fmaf(e.x, t0, v0);
+      }
+    }
+    // the four pieces of a position: lane l % 4 ends with the sum of component l % 4
+#define MV_QUAD(v, ctrl) __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ctrl, 0xf, 0xf, true))
+    {
+      const bool odd = lk & 1, upper = lk & 2;
+      const float u0 = (odd ? t1 : t0) + MV_QUAD(odd ? t0 : t1, 0xB1);   // xor 1: components 0 | 1
+      const float u1 = (odd ? t3 : t2) + MV_QUAD(odd ? t2 : t3, 0xB1);   // components 2 | 3
+      const float sum = (upper ? u1 : u0) + MV_QUAD(upper ? u0 : u1, 0x4E);
+      const float out = lk < 3 ? e.w * sum : sum;
+      if (tile * kTapTile + p < count) {
+        if (partial) pout[tile * (kTapTile * 4)] = out;
+        else if (tout) tout[tile * kTapTile] = store_cast<T>(out);
+      }
+    }
+#undef MV_QUAD
+    __syncthreads();   // the tile's column values are complete
+    // ---- gw += gy col^T, a quarter of the rows per wavefront -------------------------------------------------------
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      u32x4 a[OBW];
+#pragma unroll
+      for (int o = 0; o < OBW; o++) a[o] = tap_transposed<T>(gyl, o * 4 + wave, ks, lane);
+#pragma unroll
+      for (int c = 0; c < CBW; c++) {
+        const u32x4 bf = tap_transposed<T>(col, c, ks, lane);
+#pragma unroll
+        for (int o = 0; o < OBW; o++) acc[o][c] = M::run16(a[o], bf, acc[o][c]);
+      }
+    }
+    // ---- far corners: 32 lanes add an entry's channels, 32 at a time -------------------------------------------------
+    const int far = __builtin_amdgcn_readfirstlane(far_count[half]), n = tid % 32;
+    for (int i = tid / 32; i < far; i += 8) {
+      const uint2 entry = far_list[half][i];
+      const float w = __uint_as_float(entry.y);
+      const float *src = gcol[entry.x & 63u];
+      const unsigned base = (entry.x & ~127u) + static_cast<unsigned>(c0 + n) * 4u;
+#pragma unroll
+      for (int c = 0; c < CW; c += 32)
+        __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(w * src[c + n], gr, base + c * 4u, 0, 0);
+    }
+  }
+  // accumulator register r of lane l: output channel 4 * (l / 16) + r of its block, input channel l % 16
+#pragma unroll
+  for (int o = 0; o < OBW; o++) {
+    const int row = (o * 4 + wave) * 16;
+    if (row >= rows) continue;
+#pragma unroll
+    for (int c = 0; c < CBW; c++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        atomicAdd(gw + (static_cast<long>(k) * s.Cout + g * s.opg + row0 + row + 4 * kc + i) * s.cpg + c0 - g * s.cpg + c * 16 + j,
+                  acc[o][c][i]);
+  }
+}
+
+// The chunks' shares of the offset and mask gradients, summed.
+template <typename T>
+__global__ __launch_bounds__(256) void dcn_backward_partial_kernel(const float4 *__restrict__ partial, T *__restrict__ goff,
+                                                                   T *__restrict__ gmask, const DcnDims s, const int chunks) {
+  const long q = blockIdx.x * 256L + threadIdx.x, bgk = blockIdx.y + static_cast<long>(blockIdx.z) * s.dg * s.K;
+  if (q >= s.Q) return;
+  float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int c = 0; c < chunks; c++) {
+    const float4 v = partial[(bgk * chunks + c) * s.Q + q];
+    sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
+  }
+  T *go = goff + bgk * s.nd * s.Q + q;
+  if (s.nd == 3) *go = store_cast<T>(sum.x);
+  go[(s.nd - 2) * s.Q] = store_cast<T>(sum.y);
+  go[(s.nd - 1) * s.Q] = store_cast<T>(sum.z);
+  if (gmask) gmask[bgk * s.Q + q] = store_cast<T>(sum.w);
+}
+
+// Chunks of 64 input channels for 16-bit images (four corners; grad_output of a tile then serves twice the channels), 32
+// for volumes and fp32, whose eight corners or wider pieces would leave too few registers for two workgroups on a SIMD,
+// and where a group is no multiple of 64.
+static int tap_chunk(const DcnDims &s, int dtype) {
+  return dtype != MV_F32 && s.nd == 2 && s.cpd % 64 == 0 && s.cpg % 64 == 0 ? 64 : 32;
+}
+static int tap_chunks(const DcnDims &s, int dtype) { return s.cpd / tap_chunk(s, dtype); }
+// rows of a pass: 256 (fp32: 128) output channels keep grad_output of 64 positions within 32 KB of LDS
+static int tap_rows(int dtype) { return dtype == MV_F32 ? 128 : 256; }
+static int tap_shares(const DcnDims &s, int dtype) { return tap_chunks(s, dtype) * ((s.opg + tap_rows(dtype) - 1) / tap_rows(dtype)); }
+
+size_t dcn_tap_partial_bytes(const DcnDims &s, int dtype) {
+  const int shares = tap_shares(s, dtype);
+  return shares > 1 ? static_cast<size_t>(s.B) * s.dg * s.K * shares * s.Q * 16 : 0;
+}
+bool dcn_tap_supported(const DcnDims &s, int dtype) {
+  // (a range of 4096 positions of grad_output within 32-bit byte offsets)
+  return s.Q < (1L << 31) && s.Cout <= 65536 && static_cast<long>(s.dg) * tap_chunks(s, dtype) <= 65535 && static_cast<long>(s.dg) * s.K <= 65535;
+}
+
+template <typename T, int NC, int CBW>
+static int tap_launch(const T *xt, const T *off, const T *mask, const T *gyt, const T *wf, float *gxt, T *goff,
+                      T *gmask, float *partial, float *gw, const DcnDims &s, const unsigned *bounds, int dtype,
+                      hipStream_t stream) {
+  const int chunks = tap_chunks(s, dtype), shares = tap_shares(s, dtype);
+  // Positions of a workgroup: every one adds a block of the weight gradient to memory and fills LDS with a block of the
+  // weight, so as many as leave ~4 workgroups per compute unit.
+  const long others = static_cast<long>(s.K) * s.dg * chunks * s.B, tiles = (s.Q + kTapTile - 1) / kTapTile;
+  const long want = std::max(1L, 1024 / others), per = std::min(std::max(1L, (tiles + want - 1) / want), 64L);
+  const long ranges = (tiles + per - 1) / per;
+  MV_REQUIRE(ranges * s.K < (1L << 31), "grid too large");
+  const dim3 grid(static_cast<unsigned>(ranges * s.K), static_cast<unsigned>(s.dg * chunks), s.B);
+  const int range = static_cast<int>(per * kTapTile);
+#define MV_TAP(OBWV, ROW)                                                                                               \
+  hipLaunchKernelGGL((dcn_backward_tap_kernel<T, NC, OBWV, CBW>), grid, dim3(256), 0, stream, xt, off, mask, gyt, wf, gxt,     \
+                     goff, gmask, partial, gw, s, bounds, chunks, shares, range, ROW)
+  if (s.opg <= 64) {
+    MV_TAP(1, 0);
+  } else if (s.opg <= 128 || sizeof(T) == 4) {
+    for (int row = 0; row < s.opg; row += 128) MV_TAP(2, row);
+  } else if constexpr (sizeof(T) == 2) {
+    for (int row = 0; row < s.opg; row += 256) MV_TAP(4, row);
+  }
+#undef MV_TAP
+  int st = check_launch("dcn_backward_tap_kernel");
+  if (st || !partial) return st;
+  hipLaunchKernelGGL((dcn_backward_partial_kernel<T>), dim3(static_cast<unsigned>((s.Q + 255) / 256), s.dg * s.K, s.B), dim3(256), 0,
+                     stream, reinterpret_cast<const float4 *>(partial), goff, gmask, s, shares);
+  return check_launch("dcn_backward_partial_kernel");
+}
+
+// `bounds` null: no scatter kernel runs, every corner of the gradient of the input is added here
+int dcn_tap_backward(const void *xt, const void *off, const void *mask, const void *gyt, const void *wf,
+                     float *gxt, void *goff, void *gmask, float *partial, float *gw, const DcnDims &s, const unsigned *bounds,
+                     int dtype, hipStream_t stream) {
+  if (tap_shares(s, dtype) == 1) partial = nullptr;
+#define MV_TAP_AS(T, NC, CBW)                                                                                          \
+  tap_launch<T, NC, CBW>(static_cast<const T *>(xt), static_cast<const T *>(off), static_cast<const T *>(mask),           \
+                         static_cast<const T *>(gyt), static_cast<const T *>(wf), gxt, static_cast<T *>(goff),            \
+                         static_cast<T *>(gmask), partial, gw, s, bounds, dtype, stream)
+  const bool wide = tap_chunk(s, dtype) == 64, image = s.nd == 2;
+  if (dtype == MV_F32) return image ? MV_TAP_AS(float, 4, 2) : MV_TAP_AS(float, 8, 2);
+  if (dtype == MV_F16) return wide ? MV_TAP_AS(__half, 4, 4) : image ? MV_TAP_AS(__half, 4, 2) : MV_TAP_AS(__half, 8, 2);
+  return wide ? MV_TAP_AS(__hip_bfloat16, 4, 4) : image ? MV_TAP_AS(__hip_bfloat16, 4, 2) : MV_TAP_AS(__hip_bfloat16, 8, 2);
+#undef MV_TAP_AS
+}
+
+}  // namespace mv

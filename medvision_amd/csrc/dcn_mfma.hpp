@@ -45,6 +45,12 @@ template <> struct Mfma<__half> {
     v[0] += w * lo(r.x); v[1] += w * hi(r.x); v[2] += w * lo(r.y); v[3] += w * hi(r.y);
     v[4] += w * lo(r.z); v[5] += w * hi(r.z); v[6] += w * lo(r.w); v[7] += w * hi(r.w);
   }
+  // d + sum over the piece of g * piece
+  static __device__ __forceinline__ float dot_piece(const float (&g)[8], u32x4 r, float d) {
+    d += g[0] * lo(r.x); d += g[1] * hi(r.x); d += g[2] * lo(r.y); d += g[3] * hi(r.y);
+    d += g[4] * lo(r.z); d += g[5] * hi(r.z); d += g[6] * lo(r.w); d += g[7] * hi(r.w);
+    return d;
+  }
   static __device__ __forceinline__ u32x4 pack(const float (&v)[8]) {
     return u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7])};
   }
@@ -68,6 +74,12 @@ template <> struct Mfma<__hip_bfloat16> {
   static __device__ __forceinline__ void fma_piece(float (&v)[8], float w, u32x4 r) {
     v[0] += w * lo(r.x); v[1] += w * hi(r.x); v[2] += w * lo(r.y); v[3] += w * hi(r.y);
     v[4] += w * lo(r.z); v[5] += w * hi(r.z); v[6] += w * lo(r.w); v[7] += w * hi(r.w);
+  }
+  // d + sum over the piece of g * piece
+  static __device__ __forceinline__ float dot_piece(const float (&g)[8], u32x4 r, float d) {
+    d += g[0] * lo(r.x); d += g[1] * hi(r.x); d += g[2] * lo(r.y); d += g[3] * hi(r.y);
+    d += g[4] * lo(r.z); d += g[5] * hi(r.z); d += g[6] * lo(r.w); d += g[7] * hi(r.w);
+    return d;
   }
   static __device__ __forceinline__ u32x4 pack(const float (&v)[8]) {
     return u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7])};
