@@ -1,6 +1,6 @@
 // 3-D deformable convolution (DCNv1 when mask == nullptr, DCNv2 otherwise): general-shape
 // kernels for every dtype / group configuration, plus the entry points that choose between them
-// and the matrix-core forward for 16-bit tensors (dcn3d_mfma.hip).
+// and the matrix-core forward for 16-bit tensors (dcn_forward_columns.hip).
 //
 // Nothing here materialises the reference's column matrix: the trilinear gather feeds the weight
 // contraction directly, and the 8 corner offsets / weights of a (tap, position) pair are computed
@@ -280,10 +280,10 @@ __global__ void dcn_add_from_f32_kernel(T *dst, const float *src, long n, int ac
     dst[i] = store_cast<T>(accumulate ? load(dst + i) + src[i] : static_cast<typename Acc<T>::type>(src[i]));
 }
 
-// matrix-core forward for 16-bit tensors (dcn3d_mfma.hip)
-bool dcn_mfma_supported(const DcnDims &s, int dtype);
-size_t dcn_mfma_workspace_bytes(const DcnDims &s, int dtype);
-int dcn_mfma_forward(const void *x, const void *off, const void *mask, const void *wt,
+// matrix-core forward for 16-bit tensors (dcn_forward_columns.hip)
+bool dcn_columns_supported(const DcnDims &s, int dtype);
+size_t dcn_columns_workspace_bytes(const DcnDims &s, int dtype);
+int dcn_columns_forward(const void *x, const void *off, const void *mask, const void *wt,
                      const void *bias, void *y, const DcnDims &s, int dtype, void *workspace,
                      hipStream_t stream);
 
@@ -340,19 +340,19 @@ static PadLayout pad_layout(const DcnDims &s, const DcnPad &pad, int dtype, bool
   l.y = at; at += (!backward && l.y_padded) ? align256p(static_cast<size_t>(p.B) * p.Cout * p.Q * es) : 0;
   l.gy = at; at += (backward && l.y_padded) ? align256p(static_cast<size_t>(p.B) * p.Cout * p.Q * es) : 0;
   l.inner = at;
-  at += backward ? dcn_mfma_backward_workspace_bytes(p, dtype) : dcn_mfma_workspace_bytes(p, dtype);
+  at += backward ? dcn_mfma_backward_workspace_bytes(p, dtype) : dcn_columns_workspace_bytes(p, dtype);
   l.total = at;
   return l;
 }
 static bool forward_pads(const DcnDims &s, int dtype, DcnPad &pad) {
-  return !dcn_mfma_supported(s, dtype) && dcn_pad_plan(s, dtype, pad) && dcn_mfma_supported(pad.p, dtype);
+  return !dcn_columns_supported(s, dtype) && dcn_pad_plan(s, dtype, pad) && dcn_columns_supported(pad.p, dtype);
 }
 static bool backward_pads(const DcnDims &s, int dtype, DcnPad &pad) {
   return !dcn_mfma_backward_supported(s, dtype) && dcn_pad_plan(s, dtype, pad) && dcn_mfma_backward_supported(pad.p, dtype);
 }
 
 static size_t forward_workspace(const DcnDims &s, int dtype) {
-  if (dcn_mfma_supported(s, dtype)) return dcn_mfma_workspace_bytes(s, dtype);
+  if (dcn_columns_supported(s, dtype)) return dcn_columns_workspace_bytes(s, dtype);
   DcnPad pad;
   return forward_pads(s, dtype, pad) ? pad_layout(s, pad, dtype, false).total : 0;
 }
@@ -372,9 +372,9 @@ static int dcn_forward_any(const void *input, const void *offset, const void *ma
                            int dtype, void *workspace, void *stream) {
   MV_REQUIRE(input && offset && weight && output, "null pointer argument");
   hipStream_t hs = static_cast<hipStream_t>(stream);
-  if (dcn_mfma_supported(s, dtype)) {
+  if (dcn_columns_supported(s, dtype)) {
     MV_REQUIRE(workspace, "this shape needs a workspace of mv_dcn3d_forward_workspace_bytes()");
-    return dcn_mfma_forward(input, offset, mask, weight, bias, output, s, dtype, workspace, hs);
+    return dcn_columns_forward(input, offset, mask, weight, bias, output, s, dtype, workspace, hs);
   }
   DcnPad pad;
   if (forward_pads(s, dtype, pad)) {
@@ -396,7 +396,7 @@ static int dcn_forward_any(const void *input, const void *offset, const void *ma
       if (st) return st;
     }
     void *yp = l.y_padded ? static_cast<void *>(ws + l.y) : output;
-    st = dcn_mfma_forward(xp, offset, mask, ws + l.w, bias ? ws + l.b : nullptr, yp, pad.p, dtype, ws + l.inner, hs);
+    st = dcn_columns_forward(xp, offset, mask, ws + l.w, bias ? ws + l.b : nullptr, yp, pad.p, dtype, ws + l.inner, hs);
     if (st || !l.y_padded) return st;
     return dcn_unpad_channels(yp, output, s.B, s.Cout, s.Q, s.opg, pad.p.opg, es, hs);
   }

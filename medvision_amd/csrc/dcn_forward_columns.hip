@@ -1,0 +1,359 @@
+// Matrix-core forward of the deformable convolution for fp16 / bf16 / fp32 tensors, images and volumes.
+//
+//   y[b, o, q] = sum_{k, c} Wt[o, c, k] * col[c, k, q] + bias[o],
+//   col[c, k, q] = mask[k, q] * Z(x[b, c], p(k, q))           (zero-padded trilinear / bilinear sample)
+//
+// is a GEMM whose right operand, the column matrix, exists 16 pieces (of 16 bytes: 8 or 4 channels of a position) at a
+// time in LDS.  The contraction runs over the flat sequence of pieces (tap, deformable group, channels), so that any
+// channel count that is a multiple of a piece fills the K steps of the matrix instruction.
+//
+// Layout: x channels-last [B, P, C] (workspace): ONE 16-byte load per corner brings the channels of a piece, and the four
+// lanes of a position fetch four neighbouring pieces, usually one cache line, together.  Weights in fragment order
+// (workspace): a wavefront's operand is one coalesced 16-byte load per lane.
+//
+// Workgroup = PT positions x up to 64 * OBW output channels, four wavefronts:
+//   records   a thread works out one (unit, position): the corners' byte offsets and weights (times the mask) go
+//             to LDS, 256 of them at a time; a unit is a tap of one deformable group.  Their offsets are requested a window ahead.
+//   samples   an item = 16 positions x 4 pieces: load, blend, write the piece to LDS.  The corners of the next item are on
+//             their way while one is blended, also across the product in between.
+//   product   16 pieces of K against the wavefront's rows of the weight, v_mfma_f32_16x16x32 (fp32: 16x16x4).
+// PT: 32 positions use a weight fragment twice; 16 give a layer of a few thousand positions twice the workgroups, whose
+// wavefronts then share the positions and split the pieces.  (64 positions: no faster for wide layers, 165 us against
+// 134 us for bf16 [2, 128 -> 64, 50 x 37 x 13].)
+// What bounds it: narrow layers the blend (a multiply-add per channel and corner) and the cache look-ups of the corners
+// (64 bytes a clock), wide ones the matrix cores; small layers the latency of the chain load - blend - product.
+//   (Images fp16 [8, 256 -> 256, 100 x 152]: 566 us with 16 positions per wavefront and the weights through LDS, 283 us now;
+//   bf16 [4, 256 -> 64, 121 x 21] stride 2: 83 us, 21 us now; bf16 [1, 128 -> 32, 6 x 22 x 34]: 100 us, 30 us now.)
+#include "dcn_mfma.hpp"
+
+namespace mv {
+
+// ---- layouts: x [B, C, P] -> xt [B, P, C] and the weight fragments, one launch --------------------------------------
+// 64 positions x 128 bytes of channels per workgroup through LDS.  Rows of any alignment: 16 bytes at a time all the same.
+constexpr int kMovePos = 64;
+template <typename U>
+__device__ __forceinline__ void dcn_move_block(const U *__restrict__ x, U *__restrict__ xt, const int C, const long P,
+                                               const long bx, const int b, const int bz) {
+  constexpr int V = 16 / sizeof(U), CH = 128 / sizeof(U), PITCH = kMovePos + V, PG = kMovePos / V;
+  typedef unsigned int piece_t __attribute__((ext_vector_type(4), aligned(2)));   // (element alignment: the hardware takes it)
+  __shared__ __attribute__((aligned(16))) U stage[CH * PITCH];
+  const long p0 = bx * kMovePos;
+  const int c0 = bz * CH, cn = min(CH, C - c0), np = static_cast<int>(min(static_cast<long>(kMovePos), P - p0));
+  const U *src = x + (static_cast<long>(b) * C + c0) * P + p0;
+#pragma unroll
+  for (int u = 0; u < CH * PG / 256; u++) {
+    const int i = threadIdx.x + u * 256, c = i / PG, at = i % PG * V;
+    if (c >= cn) continue;
+    const U *from = src + static_cast<long>(c) * P + at;
+    if (at + V <= np) {
+      *reinterpret_cast<u32x4 *>(stage + c * PITCH + at) = *reinterpret_cast<const piece_t *>(from);
+    } else {
+      for (int e = 0; at + e < np; e++) stage[c * PITCH + at + e] = from[e];
+    }
+  }
+  __syncthreads();
+  const int groups = cn / V;
+  for (int i = threadIdx.x; i < np * groups; i += 256) {
+    const int p = i / groups, cg = i - p * groups;
+    U out[V];
+#pragma unroll
+    for (int e = 0; e < V; e++) out[e] = stage[(cg * V + e) * PITCH + p];
+    u32x4 packed;
+    __builtin_memcpy(&packed, out, 16);
+    *reinterpret_cast<u32x4 *>(xt + (static_cast<long>(b) * P + p0 + p) * C + c0 + cg * V) = packed;
+  }
+}
+
+// weight [Cout, cpg, K] -> [group][16-row block][K step][lane][piece]: lane l holds row l % 16 and flat piece 4 * step + l / 16
+// (tap piece / (cpg / PC), channels piece % (cpg / PC)); pieces beyond the last one are zeros
+template <typename U>
+__device__ __forceinline__ void dcn_flat_fragments_block(const U *__restrict__ wt, U *__restrict__ wf, const DcnDims &s, const long id) {
+  constexpr int PC = 16 / sizeof(U);
+  const int per_tap = s.cpg / PC, steps = (s.K * per_tap + 3) / 4, blocks = s.opg / 16;
+  if (id >= static_cast<long>(s.groups) * blocks * steps * 64) return;
+  const int lane = id % 64;
+  long r = id / 64;
+  const int st = r % steps; r /= steps;
+  const int mb = r % blocks, g = static_cast<int>(r / blocks);
+  const int piece = st * 4 + lane / 16, k = piece / per_tap, c = piece % per_tap * PC;
+  const U *src = wt + (static_cast<long>(g * s.opg + mb * 16 + lane % 16) * s.cpg + c) * s.K + k;
+  U out[PC];
+#pragma unroll
+  for (int i = 0; i < PC; i++) out[i] = k < s.K ? src[static_cast<long>(i) * s.K] : U(0);
+  u32x4 packed;
+  __builtin_memcpy(&packed, out, 16);
+  *reinterpret_cast<u32x4 *>(wf + id * PC) = packed;
+}
+
+template <typename U>
+__global__ __launch_bounds__(256) void dcn_columns_layout_kernel(const U *__restrict__ x, U *__restrict__ xt,
+                                                                 const U *__restrict__ wt, U *__restrict__ wf, const DcnDims s,
+                                                                 const unsigned pblocks, const unsigned moves) {
+  if (blockIdx.x < moves) {
+    const unsigned bx = blockIdx.x % pblocks, r = blockIdx.x / pblocks;
+    dcn_move_block<U>(x, xt, s.Cin, s.P, bx, static_cast<int>(r % s.B), static_cast<int>(r / s.B));
+  } else {
+    dcn_flat_fragments_block<U>(wt, wf, s, (blockIdx.x - moves) * 256L + threadIdx.x);
+  }
+}
+
+// ---- the layer ---------------------------------------------------------------------------------------------------------
+constexpr int kColPieces = 16;   // pieces of a product: four K steps
+
+template <typename T, int NC, int PT, int OBW>
+__global__ __launch_bounds__(256, OBW == 4 && (PT == 32 || NC == 8) ? 2 : (OBW == 1 ? 4 : 3)) void dcn_forward_columns_kernel(
+    const T *__restrict__ xt, const T *__restrict__ off, const T *__restrict__ mask, const T *__restrict__ wf,
+    const T *__restrict__ bias, T *__restrict__ y, const DcnDims s) {
+  using M = Mfma<T>;
+  using P = typename std::conditional<(sizeof(T) == 2), float, double>::type;  // position type
+  constexpr int PC = M::kPiece, ES = sizeof(T), PG = PT / 16, TG = 256 / PT;   // position groups; units of a window
+  constexpr int PIECES = kColPieces, KS = PIECES / 4;
+  constexpr int ITEMS = KS * PG / 4;                                           // items of a wavefront per product
+  constexpr unsigned kOutside = 0x80000000u;                                   // beyond the buffer: such loads return zeros
+  constexpr int RW = 2 * NC + 4, PITCH = PT + 4;   // (records 4 dwords further apart than they are long: banks)
+  __shared__ __attribute__((aligned(16))) unsigned rec[TG * PT][RW];           // [unit][position]: at[NC], mask * w[NC]
+  __shared__ u32x4 col[2][PIECES * PITCH];                                 // [piece][position]
+  const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int j = lane % 16, kc = lane / 16;   // matrix layout
+  const int lj = lane / 4, lk = lane % 4;    // load layout
+  const int row_chunks = (s.opg + 64 * OBW - 1) / (64 * OBW);
+  const int g = blockIdx.y / row_chunks, row0 = blockIdx.y % row_chunks * (64 * OBW), b = blockIdx.z;
+  // (an XCD takes a contiguous eighth of the positions: its L2 then holds an eighth of the input and the offsets' reach)
+  const long q0 = static_cast<long>(xcd_contiguous(blockIdx.x, gridDim.x)) * PT;
+  const int dgn = s.cpd < s.cpg ? s.cpg / s.cpd : 1, dg0 = g * s.cpg / s.cpd;
+  const int units = s.K * dgn, up = (dgn == 1 ? s.cpg : s.cpd) / PC;   // pieces per unit
+  const int total = units * up, steps_all = (total + 3) / 4;
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T *>(xt + static_cast<long>(b) * s.P * s.Cin), 0, static_cast<int>(s.P * s.Cin * ES), 0x00020000);
+
+  // ---- records ------------------------------------------------------------------------------------------------------
+  const int ru = tid / PT, rp = tid % PT;   // this thread's unit of a window and position
+  const long rq = min(q0 + rp, s.Q - 1);
+  const bool rlive = q0 + rp < s.Q;
+  int base_d, base_h, base_w;
+  {
+    const int qi = static_cast<int>(rq), ow = qi % s.Wo, t = qi / s.Wo, oh = t % s.Ho, od = t / s.Ho;
+    base_d = od * s.sd - s.pd; base_h = oh * s.sh - s.ph; base_w = ow * s.sw - s.pw;
+  }
+  P fd = P(0), fh = P(0), fw = P(0);
+  float fm = 1.f;
+  auto request = [&](int first) {
+    const int u = min(first + ru, units - 1), k = u / dgn;
+    const long bg = static_cast<long>(b) * s.dg + dg0 + u - k * dgn;
+    dcn_offsets(s, off + (bg * s.K + k) * s.nd * s.Q + rq, fd, fh, fw);
+    if (mask) fm = load(mask + (bg * s.K + k) * s.Q + rq);
+  };
+  auto publish = [&](int first) {
+    const int u = first + ru, k = u / dgn;
+    const int ti = k / (s.kh * s.kw), tj = (k / s.kw) % s.kh, tk = k % s.kw;
+    P pd = fd + static_cast<P>(base_d + ti * s.dd);
+    const P ph = fh + static_cast<P>(base_h + tj * s.dh), pw = fw + static_cast<P>(base_w + tk * s.dw);
+    if (NC == 4) pd = P(0);   // images: the only slice
+    CornerTaps t;
+    corner_taps<P>(s, pd, ph, pw, rlive && u < units, static_cast<unsigned>(s.Cin) * ES, 0u, kOutside, t);
+    unsigned *r = rec[tid];
+#pragma unroll
+    for (int c = 0; c < NC; c += 4) {
+      *reinterpret_cast<u32x4 *>(r + c) = u32x4{t.at[c], t.at[c + 1], t.at[c + 2], t.at[c + 3]};
+      *reinterpret_cast<float4 *>(r + NC + c) = make_float4(fm * t.w[c], fm * t.w[c + 1], fm * t.w[c + 2], fm * t.w[c + 3]);
+    }
+  };
+
+  // ---- samples: item i of a product: slot = wave + 4 i, positions 16 * (slot % PG), quadruple slot / PG of the product's pieces;
+  // a wavefront's items form one sequence over the window, 4 / PG quadruples apart ------------------------------------
+  const int p = wave % PG * 16 + lj;         // (slot % PG is the same for all of them)
+  const bool whole = up % 4 == 0;            // a quadruple belongs to one unit
+  const int quads = up / 4;                  // per unit (`whole`)
+  // (division by the pieces of a unit: the high half of a product, exact while piece * up < 2^32)
+  const unsigned magic = up == 1 ? 0u : 0xffffffffu / static_cast<unsigned>(up) + 1u;
+  u32x4 raw[NC];
+  const unsigned *rnow = nullptr;            // the record of the item on its way
+  int nu = 0, nr = 0;                        // the next item: unit of the window and quadruple of it (`whole`), or quadruple of the window
+  auto gather = [&](int window, int limit) {
+    unsigned add;
+    int scalar_add = g * s.cpg * ES;
+    if (whole) {
+      const int u = min(nu, min(TG, units - window) - 1);   // (past the last one: loaded for nothing)
+      rnow = rec[u * PT + p];
+      add = static_cast<unsigned>(lk) * 16u;
+      scalar_add += nr * 64;
+      if (dgn > 1) scalar_add += (window + u) % dgn * (s.cpd * ES);
+      nr += 4 / PG;
+      while (nr >= quads) { nr -= quads; nu++; }
+    } else {
+      const int piece = min(nr * 4 + lk, limit - 1);
+      const int u = up == 1 ? piece : static_cast<int>(__umulhi(static_cast<unsigned>(piece), magic)), r = piece - u * up;
+      rnow = rec[u * PT + p];
+      add = static_cast<unsigned>((dgn == 1 ? r * PC : (window + u) % dgn * s.cpd + r * PC) * ES);
+      nr += 4 / PG;
+    }
+#pragma unroll
+    for (int c = 0; c < NC; c += 4) {
+      const u32x4 a = *reinterpret_cast<const u32x4 *>(rnow + c);
+#pragma unroll
+      for (int t = 0; t < 4; t++) raw[c + t] = __builtin_amdgcn_raw_buffer_load_b128(xr, a[t] + add, scalar_add, 0);
+    }
+  };
+  // `left`: pieces of the window from this product's first one on
+  auto blend = [&](int left, int i, u32x4 *to) {
+    const int piece = (wave / PG + i * (4 / PG)) * 4 + lk;
+    float v[PC];
+#pragma unroll
+    for (int e = 0; e < PC; e++) v[e] = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; c += 4) {
+      const float4 w = *reinterpret_cast<const float4 *>(rnow + NC + c);
+      M::fma_piece(v, w.x, raw[c]); M::fma_piece(v, w.y, raw[c + 1]);
+      M::fma_piece(v, w.z, raw[c + 2]); M::fma_piece(v, w.w, raw[c + 3]);
+    }
+    // (pieces beyond the last one meet weights that are zero, or the next window's: they must be zero themselves)
+    to[piece * PITCH + p] = piece < left ? M::pack(v) : u32x4{0u, 0u, 0u, 0u};
+  };
+
+  float4_t acc[OBW][PG];
+#pragma unroll
+  for (int o = 0; o < OBW; o++)
+#pragma unroll
+    for (int n = 0; n < PG; n++) acc[o][n] = float4_t{0.f, 0.f, 0.f, 0.f};
+  const int blocks = s.opg / 16;
+  const T *wsrc[OBW];
+#pragma unroll
+  for (int o = 0; o < OBW; o++)   // (blocks beyond the last one repeat it; their products are not used)
+    wsrc[o] = wf + (static_cast<long>(g) * blocks + min(row0 / 16 + o * 4 + wave, blocks - 1)) * steps_all * (64 * PC) + lane * PC;
+
+  request(0);
+  int buf = 0;
+  for (int window = 0; window < units; window += TG) {
+    __syncthreads();   // the records have been read
+    publish(window);
+    if (window + TG < units) request(window + TG);
+    __syncthreads();
+    const int limit = min(TG, units - window) * up, step0 = window * up / 4;   // (TG is a multiple of four)
+    nu = 0;
+    nr = wave / PG;
+    if (whole) while (nr >= quads) { nr -= quads; nu++; }
+    gather(window, limit);
+    for (int first = 0; first < limit; first += PIECES) {
+      u32x4 a[OBW][KS];
+#pragma unroll
+      for (int st = 0; st < KS; st++) {
+        const int step = min(step0 + first / 4 + st, steps_all - 1);
+#pragma unroll
+        for (int o = 0; o < OBW; o++) a[o][st] = *reinterpret_cast<const u32x4 *>(wsrc[o] + static_cast<long>(step) * (64 * PC));
+      }
+#pragma unroll
+      for (int i = 0; i < ITEMS; i++) {
+        blend(limit - first, i, col[buf]);
+        if (i + 1 < ITEMS || first + PIECES < limit) gather(window, limit);
+      }
+      __syncthreads();   // the pieces are complete (and the other buffer has been read)
+#pragma unroll
+      for (int st = 0; st < KS; st++)
+#pragma unroll
+        for (int n = 0; n < PG; n++) {
+          const u32x4 bf = col[buf][(st * 4 + kc) * PITCH + n * 16 + j];
+#pragma unroll
+          for (int o = 0; o < OBW; o++) acc[o][n] = M::run16(a[o][st], bf, acc[o][n]);
+        }
+      buf ^= 1;
+    }
+  }
+  // accumulator register r of lane l: output channel 4 * (l / 16) + r of its block, position l % 16 of its group
+#pragma unroll
+  for (int o = 0; o < OBW; o++) {
+    const int row = row0 + (o * 4 + wave) * 16 + 4 * kc;
+    if (row >= s.opg) continue;
+    float bv[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) bv[r] = bias ? load(bias + g * s.opg + row + r) : 0.f;
+#pragma unroll
+    for (int n = 0; n < PG; n++) {
+      const long q = q0 + n * 16 + j;
+      if (q < s.Q) {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          y[(static_cast<long>(b) * s.Cout + g * s.opg + row + r) * s.Q + q] = store_cast<T>(acc[o][n][r] + bv[r]);
+      }
+    }
+  }
+}
+
+// dcn3d_mfma.hip: large volumes with few channels; -1: not for this layer
+int dcn_shared_taps_forward(const void *xt, const void *off, const void *mask, const void *wf, const void *bias, void *y,
+                            const DcnDims &s, int dtype, hipStream_t stream);
+
+static size_t columns_align(size_t v) { return (v + 255) / 256 * 256; }
+static long columns_steps(const DcnDims &s, int pc) { return (static_cast<long>(s.K) * (s.cpg / pc) + 3) / 4; }
+
+bool dcn_columns_supported(const DcnDims &s, int dtype) {
+  if (dtype != MV_F16 && dtype != MV_BF16 && dtype != MV_F32) return false;
+  const int es = dtype == MV_F32 ? 4 : 2, pc = 16 / es;
+  if (s.cpg % pc || s.cpd % pc || s.opg % 16 || (s.cpd < s.cpg && s.cpg % s.cpd) || (s.cpd > s.cpg && s.cpd % s.cpg)) return false;
+  if (s.B > 65535 || s.Q >= (1L << 31) || s.K > 65536) return false;
+  // 32-bit byte offsets into a sample; pieces of a window below 2^16
+  return static_cast<long>(s.P) * s.Cin * es < (1L << 31) && 16L * (s.cpg / pc) < 65536 && static_cast<long>(s.K) * s.cpg < (1L << 30);
+}
+
+size_t dcn_columns_workspace_bytes(const DcnDims &s, int dtype) {
+  const size_t es = dtype == MV_F32 ? 4 : 2;
+  return columns_align(static_cast<size_t>(s.B) * s.P * s.Cin * es) +
+         columns_align(static_cast<size_t>(s.Cout / 16) * columns_steps(s, static_cast<int>(16 / es)) * 1024);
+}
+
+template <typename T, int NC>
+static int columns_run(const void *x, const void *off, const void *mask, const void *wt, const void *bias, void *y,
+                       const DcnDims &s, void *workspace, hipStream_t stream) {
+  using U = typename std::conditional<(sizeof(T) == 2), unsigned short, unsigned int>::type;
+  T *xt = static_cast<T *>(workspace);
+  T *wf = reinterpret_cast<T *>(static_cast<char *>(workspace) + columns_align(static_cast<size_t>(s.B) * s.P * s.Cin * sizeof(T)));
+  const int ch = 128 / static_cast<int>(sizeof(T));
+  const long pblocks = (s.P + kMovePos - 1) / kMovePos, moves = pblocks * s.B * ((s.Cin + ch - 1) / ch);
+  const long frags = (static_cast<long>(s.Cout / 16) * columns_steps(s, 16 / static_cast<int>(sizeof(T))) * 64 + 255) / 256;
+  MV_REQUIRE(moves + frags < (1L << 31), "volume too large");
+  hipLaunchKernelGGL((dcn_columns_layout_kernel<U>), dim3(static_cast<unsigned>(moves + frags)), dim3(256), 0, stream,
+                     static_cast<const U *>(x), reinterpret_cast<U *>(xt), static_cast<const U *>(wt), reinterpret_cast<U *>(wf), s,
+                     static_cast<unsigned>(pblocks), static_cast<unsigned>(moves));
+  int st = check_launch("dcn_columns_layout_kernel");
+  if (st) return st;
+  if constexpr (sizeof(T) == 2 && NC == 8) {
+    st = dcn_shared_taps_forward(xt, off, mask, wf, bias, y, s, sizeof(T) == 2 && std::is_same<T, __half>::value ? MV_F16 : MV_BF16, stream);
+    if (st >= 0) return st;
+  }
+  // Positions per workgroup: 32 as long as that gives every compute unit two workgroups, otherwise 16; then fewer output
+  // channels per workgroup (each share repeats the samples) until there is one for every compute unit.
+  int pt = 32, obw = s.opg <= 64 ? 1 : (s.opg <= 128 ? 2 : 4);
+  auto groups_of = [&](int p, int o) { return (s.Q + p - 1) / p * s.B * s.groups * ((s.opg + 64 * o - 1) / (64 * o)); };
+  if (groups_of(pt, obw) < 512) pt = 16;
+  while (obw > 1 && groups_of(pt, obw) < 256) obw /= 2;
+  const long qblocks = (s.Q + pt - 1) / pt;
+  const long rows = static_cast<long>(s.groups) * ((s.opg + 64 * obw - 1) / (64 * obw));
+  MV_REQUIRE(qblocks < (1L << 31) && rows <= 65535, "grid too large");
+  const dim3 grid(static_cast<unsigned>(qblocks), static_cast<unsigned>(rows), s.B), block(256);
+#define MV_COLUMNS(PTV, OBWV)                                                                                          \
+  hipLaunchKernelGGL((dcn_forward_columns_kernel<T, NC, PTV, OBWV>), grid, block, 0, stream, xt, static_cast<const T *>(off), \
+                     static_cast<const T *>(mask), wf, static_cast<const T *>(bias), static_cast<T *>(y), s)
+#define MV_COLUMNS_PT(PTV)                                                                                             \
+  do {                                                                                                                 \
+    if (obw == 1) MV_COLUMNS(PTV, 1);                                                                                  \
+    else if (obw == 2) MV_COLUMNS(PTV, 2);                                                                             \
+    else MV_COLUMNS(PTV, 4);                                                                                           \
+  } while (0)
+  if (pt == 32) MV_COLUMNS_PT(32);
+  else MV_COLUMNS_PT(16);
+#undef MV_COLUMNS_PT
+#undef MV_COLUMNS
+  return check_launch("dcn_forward_columns_kernel");
+}
+
+int dcn_columns_forward(const void *x, const void *off, const void *mask, const void *wt, const void *bias, void *y,
+                        const DcnDims &s, int dtype, void *workspace, hipStream_t stream) {
+  const bool image = s.nd == 2 && s.D == 1 && s.kd == 1 && s.pd == 0;
+#define MV_COLUMNS_AS(T) \
+  (image ? columns_run<T, 4>(x, off, mask, wt, bias, y, s, workspace, stream) : columns_run<T, 8>(x, off, mask, wt, bias, y, s, workspace, stream))
+  if (dtype == MV_F16) return MV_COLUMNS_AS(__half);
+  if (dtype == MV_F32) return MV_COLUMNS_AS(float);
+  return MV_COLUMNS_AS(__hip_bfloat16);
+#undef MV_COLUMNS_AS
+}
+
+}  // namespace mv
