@@ -291,15 +291,13 @@ int dcn_columns_forward(const void *x, const void *off, const void *mask, const 
 bool dcn_mfma_backward_supported(const DcnDims &s, int dtype);
 size_t dcn_mfma_backward_workspace_bytes(const DcnDims &s, int dtype);
 int dcn_mfma_backward(const void *x, const void *off, const void *mask, const void *wt,
-                      const void *gy, void *goff, void *gmask, const DcnDims &s, int dtype,
+                      const void *gy, void *goff, void *gmask, const DcnDims &s, const DcnPad &pad, int dtype,
                       void *workspace, bool want_bias, float **gx32, float **gw32, float **gb32,
                       hipStream_t stream);
 void dcn_set_column_budget(size_t bytes);
 size_t dcn_column_budget();
-int dcn_planar_add(const float *gxt, void *gx, const DcnDims &s, int dtype, bool accumulate, hipStream_t stream);
-int dcn_weight_add(const float *acc, void *gw, const DcnDims &s, int dtype, bool accumulate, hipStream_t stream);
 int dcn_backward_fold(const float *gxt, const float *gw32, const float *gb32, void *grad_input, void *grad_weight,
-                      void *grad_bias, const DcnDims &s, int dtype, bool accumulate, hipStream_t stream);
+                      void *grad_bias, const DcnDims &s, const DcnPad &pad, int dtype, bool accumulate, hipStream_t stream);
 int fill_zero(void *p, size_t bytes, hipStream_t s);   // roi_align.hip
 
 static inline int blocks_for(long n, int per_block, int cap) {
@@ -325,10 +323,10 @@ int mv_dcn3d_output_dims(const mv_dcn3d_shape *shape, int *out_d, int *out_h, in
 // of the padded layer.
 static size_t align256p(size_t v) { return (v + 255) / 256 * 256; }
 struct PadLayout {
-  size_t x, w, b, y, gy, inner, total;   // byte offsets (x, w, b / gy, y: padded copies; y only when Cout is padded)
+  size_t x, w, b, y, inner, total;   // byte offsets (x, w, b, y: padded copies; y only when Cout is padded)
   bool x_padded, y_padded;
 };
-static PadLayout pad_layout(const DcnDims &s, const DcnPad &pad, int dtype, bool backward) {
+static PadLayout pad_layout(const DcnDims &s, const DcnPad &pad, int dtype) {
   const size_t es = dtype == MV_F32 ? 4 : 2;
   const DcnDims &p = pad.p;
   PadLayout l;
@@ -337,30 +335,32 @@ static PadLayout pad_layout(const DcnDims &s, const DcnPad &pad, int dtype, bool
   l.x = at; at += l.x_padded ? align256p(static_cast<size_t>(p.B) * p.Cin * p.P * es) : 0;
   l.w = at; at += align256p(static_cast<size_t>(p.Cout) * p.cpg * p.K * es);
   l.b = at; at += align256p(static_cast<size_t>(p.Cout) * es);
-  l.y = at; at += (!backward && l.y_padded) ? align256p(static_cast<size_t>(p.B) * p.Cout * p.Q * es) : 0;
-  l.gy = at; at += (backward && l.y_padded) ? align256p(static_cast<size_t>(p.B) * p.Cout * p.Q * es) : 0;
+  l.y = at; at += l.y_padded ? align256p(static_cast<size_t>(p.B) * p.Cout * p.Q * es) : 0;
   l.inner = at;
-  at += backward ? dcn_mfma_backward_workspace_bytes(p, dtype) : dcn_columns_workspace_bytes(p, dtype);
+  at += dcn_columns_workspace_bytes(p, dtype);
   l.total = at;
   return l;
 }
 static bool forward_pads(const DcnDims &s, int dtype, DcnPad &pad) {
   return !dcn_columns_supported(s, dtype) && dcn_pad_plan(s, dtype, pad) && dcn_columns_supported(pad.p, dtype);
 }
-static bool backward_pads(const DcnDims &s, int dtype, DcnPad &pad) {
-  return !dcn_mfma_backward_supported(s, dtype) && dcn_pad_plan(s, dtype, pad) && dcn_mfma_backward_supported(pad.p, dtype);
+// The layer that the matrix-core backward runs: this one (pad.on false) or the next larger one that it takes; false: neither.
+static bool backward_plan(const DcnDims &s, int dtype, DcnPad &pad) {
+  pad.on = false;
+  pad.p = s;
+  pad.unit = pad.unit_p = std::min(s.cpg, s.cpd);
+  return dcn_mfma_backward_supported(s, dtype) || (dcn_pad_plan(s, dtype, pad) && dcn_mfma_backward_supported(pad.p, dtype));
 }
 
 static size_t forward_workspace(const DcnDims &s, int dtype) {
   if (dcn_columns_supported(s, dtype)) return dcn_columns_workspace_bytes(s, dtype);
   DcnPad pad;
-  return forward_pads(s, dtype, pad) ? pad_layout(s, pad, dtype, false).total : 0;
+  return forward_pads(s, dtype, pad) ? pad_layout(s, pad, dtype).total : 0;
 }
 
 static size_t backward_workspace(const DcnDims &s, int dtype) {
-  if (dcn_mfma_backward_supported(s, dtype)) return dcn_mfma_backward_workspace_bytes(s, dtype);
   DcnPad pad;
-  if (backward_pads(s, dtype, pad)) return pad_layout(s, pad, dtype, true).total;
+  if (backward_plan(s, dtype, pad)) return dcn_mfma_backward_workspace_bytes(pad.p, dtype);
   if (dtype != MV_F16 && dtype != MV_BF16) return 0;
   // fp32 accumulators for grad_input, grad_weight, grad_bias
   const size_t n = static_cast<size_t>(s.B) * s.Cin * s.P + static_cast<size_t>(s.Cout) * s.cpg * s.K + s.Cout;
@@ -379,7 +379,7 @@ static int dcn_forward_any(const void *input, const void *offset, const void *ma
   DcnPad pad;
   if (forward_pads(s, dtype, pad)) {
     MV_REQUIRE(workspace, "this shape needs a workspace of mv_dcn3d_forward_workspace_bytes()");
-    const PadLayout l = pad_layout(s, pad, dtype, false);
+    const PadLayout l = pad_layout(s, pad, dtype);
     const int es = dtype == MV_F32 ? 4 : 2;
     char *ws = static_cast<char *>(workspace);
     const void *xp = input;
@@ -444,69 +444,17 @@ static int dcn_backward_any(const void *input, const void *offset, const void *m
              "grad_mask given without mask");
   const bool narrow = dtype == MV_F16 || dtype == MV_BF16;
   DcnPad pad;
-  const bool padded = backward_pads(s, dtype, pad);
-  MV_REQUIRE((!narrow && !dcn_mfma_backward_supported(s, dtype) && !padded) || workspace,
-             "this backward needs a workspace of mv_dcn3d_backward_workspace_bytes()");
+  const bool cores = backward_plan(s, dtype, pad);
+  MV_REQUIRE((!narrow && !cores) || workspace, "this backward needs a workspace of mv_dcn3d_backward_workspace_bytes()");
   hipStream_t hs = static_cast<hipStream_t>(stream);
-  if (padded) {
-    const PadLayout l = pad_layout(s, pad, dtype, true);
-    const int es = dtype == MV_F32 ? 4 : 2;
-    char *wsb = static_cast<char *>(workspace);
-    const void *xp = input, *gyp = grad_output;
-    if (l.x_padded) {
-      st = dcn_pad_channels(input, wsb + l.x, s.B, s.Cin, s.P, pad.unit, pad.unit_p, es, hs);
-      if (st) return st;
-      xp = wsb + l.x;
-    }
-    st = dcn_pad_weight(weight, wsb + l.w, s, pad, es, hs);
-    if (st) return st;
-    if (l.y_padded) {
-      st = dcn_pad_channels(grad_output, wsb + l.gy, s.B, s.Cout, s.Q, s.opg, pad.p.opg, es, hs);
-      if (st) return st;
-      gyp = wsb + l.gy;
-    }
+  if (cores) {
     float *gx32, *gw32, *gb32;
-    st = dcn_mfma_backward(xp, offset, mask, wsb + l.w, gyp, grad_offset, grad_mask, pad.p, dtype, wsb + l.inner,
-                           false, &gx32, &gw32, &gb32, hs);
-    if (st) return st;
-    st = dcn_planar_add_padded(gx32, grad_input, s, pad, dtype, accumulate, hs);
-    if (st) return st;
-    MV_DISPATCH(dtype, {
-      if (sizeof(T) <= 4) {
-        if (grad_bias) {   // from the real output gradient, into the (zeroed) accumulator of the padded layer
-          hipLaunchKernelGGL((dcn_backward_bias_kernel<T, float>), dim3(s.Cout, s.B, static_cast<unsigned>((s.Q + kBiasSlab - 1) / kBiasSlab)), dim3(256), 0, hs,
-                             static_cast<const T *>(grad_output), gb32, s);
-          hipLaunchKernelGGL((dcn_add_from_f32_kernel<T>), dim3(1), dim3(256), 0, hs,
-                             static_cast<T *>(grad_bias), gb32, static_cast<long>(s.Cout), accumulate ? 1 : 0);
-        }
-      }
-    });
-    st = dcn_weight_add_padded(gw32, grad_weight, nullptr, nullptr, s, pad, dtype, accumulate, hs);
-    if (st) return st;
-    return check_launch("dcn3d backward (padded channels)");
+    st = dcn_mfma_backward(input, offset, mask, weight, grad_output, grad_offset, grad_mask, s, pad, dtype, workspace,
+                           grad_bias != nullptr, &gx32, &gw32, &gb32, hs);
+    return st ? st : dcn_backward_fold(gx32, gw32, gb32, grad_input, grad_weight, grad_bias, s, pad, dtype, accumulate, hs);
   }
   const long n_gx = static_cast<long>(s.B) * s.Cin * s.P, n_gw = static_cast<long>(s.Cout) * s.cpg * s.K;
   float *ws = static_cast<float *>(workspace);
-  if (dcn_mfma_backward_supported(s, dtype)) {
-    float *gx32, *gw32, *gb32;
-    st = dcn_mfma_backward(input, offset, mask, weight, grad_output, grad_offset, grad_mask, s, dtype,
-                           workspace, grad_bias != nullptr, &gx32, &gw32, &gb32, hs);
-    if (st) return st;
-    st = dcn_backward_fold(gx32, gw32, gb32, grad_input, grad_weight, grad_bias, s, dtype, accumulate, hs);
-    if (st >= 0) return st;   // (one launch for the three folds; -1: not with these tensors)
-    st = dcn_planar_add(gx32, grad_input, s, dtype, accumulate, hs);
-    if (st) return st;
-    MV_DISPATCH(dtype, {
-      if (sizeof(T) <= 4) {
-        if (grad_bias)   // (the sums of grad_output are in the accumulator already)
-          hipLaunchKernelGGL((dcn_add_from_f32_kernel<T>), dim3(1), dim3(256), 0, hs,
-                             static_cast<T *>(grad_bias), gb32, static_cast<long>(s.Cout), accumulate ? 1 : 0);
-      }
-    });
-    st = dcn_weight_add(gw32, grad_weight, s, dtype, accumulate, hs);
-    if (st) return st;
-    return check_launch("dcn3d backward");
-  }
   if (narrow) {
     const long n = n_gx + n_gw + s.Cout;
     st = fill_zero(ws, static_cast<size_t>(n) * 4, hs);

@@ -7,34 +7,6 @@
 
 namespace mv {
 
-// x [B, Cin, P] -> xt [B, P, Cin]; one workgroup moves 64 positions of up to kLayoutChunk
-// channels through LDS (U = unsigned short / unsigned int: only the element size matters)
-constexpr int kLayoutChunk = 128;
-template <typename U>
-__global__ void dcn_channels_last_kernel(const U *__restrict__ x, U *__restrict__ xt, int Cin, long P) {
-  __shared__ U stage[64][kLayoutChunk + 2];
-  const int b = blockIdx.y;
-  const long p0 = static_cast<long>(blockIdx.x) * 64;
-  const int c0 = blockIdx.z * kLayoutChunk, cn = min(kLayoutChunk, Cin - c0);
-  const U *src = x + (static_cast<long>(b) * Cin + c0) * P;
-  U *dst = xt + (static_cast<long>(b) * P + p0) * Cin + c0;
-  const int lp = threadIdx.x % 64;
-  for (int c = threadIdx.x / 64; c < cn; c += 4)
-    if (p0 + lp < P) stage[lp][c] = src[static_cast<long>(c) * P + p0 + lp];
-  __syncthreads();
-  const int count = static_cast<int>(min(static_cast<long>(64), P - p0)) * cn;
-  for (int i = threadIdx.x; i < count; i += 256) {
-    const int pp = i / cn, c = i % cn;
-    dst[static_cast<long>(pp) * Cin + c] = stage[pp][c];
-  }
-}
-
-template <typename U>
-__global__ __launch_bounds__(256) void dcn_channels_last_wide_kernel(const U *__restrict__ x, U *__restrict__ xt,
-                                                                     int Cin, long P) {
-  channels_last_wide_block<U>(x, xt, Cin, P, blockIdx.x, blockIdx.y, blockIdx.z);
-}
-
 // A workgroup of four wavefronts owns 64 positions and alternates two phases
 // per group of TG = 4 taps:
 //   G  wavefront w takes tap w of the group with ONE position per lane (the offset planes are read
@@ -246,35 +218,6 @@ __global__ __launch_bounds__(256, 5) void dcn_forward_shared_taps_kernel(
       y[(static_cast<long>(b) * s.Cout + o) * s.Q + qo] = store_cast<T>(acc[m][r] + bv[r]);
     }
   }
-}
-
-// [B, C, P] -> [B, P, C] for elements of 2 or 4 bytes
-int dcn_channels_last(const void *x, void *xt, int B, int C, long P, int elem_bytes, hipStream_t stream) {
-  const int vec = 16 / elem_bytes;
-  const bool aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(xt) % 16 == 0;
-  if (aligned && P % vec == 0 && C % vec == 0) {
-    const long wblocks = (P + kLayoutPos - 1) / kLayoutPos;
-    const int ch = 256 / elem_bytes;
-    MV_REQUIRE(wblocks < (1L << 31) && B <= 65535 && (C + ch - 1) / ch <= 65535, "volume too large");
-    const dim3 wgrid(static_cast<unsigned>(wblocks), B, (C + ch - 1) / ch);
-    if (elem_bytes == 2)
-      hipLaunchKernelGGL((dcn_channels_last_wide_kernel<unsigned short>), wgrid, dim3(256), 0, stream,
-                         static_cast<const unsigned short *>(x), static_cast<unsigned short *>(xt), C, P);
-    else
-      hipLaunchKernelGGL((dcn_channels_last_wide_kernel<unsigned int>), wgrid, dim3(256), 0, stream,
-                         static_cast<const unsigned int *>(x), static_cast<unsigned int *>(xt), C, P);
-    return check_launch("dcn_channels_last_wide_kernel");
-  }
-  const long pblocks = (P + 63) / 64;
-  MV_REQUIRE(pblocks < (1L << 31) && B <= 65535, "volume too large");
-  const dim3 grid(static_cast<unsigned>(pblocks), B, (C + kLayoutChunk - 1) / kLayoutChunk);
-  if (elem_bytes == 2)
-    hipLaunchKernelGGL((dcn_channels_last_kernel<unsigned short>), grid, dim3(256), 0, stream,
-                       static_cast<const unsigned short *>(x), static_cast<unsigned short *>(xt), C, P);
-  else
-    hipLaunchKernelGGL((dcn_channels_last_kernel<unsigned int>), grid, dim3(256), 0, stream,
-                       static_cast<const unsigned int *>(x), static_cast<unsigned int *>(xt), C, P);
-  return check_launch("dcn_channels_last_kernel");
 }
 
 // The layers that this kernel serves: volumes of many bricks (below four workgroups per compute unit the columns

@@ -11,6 +11,7 @@
 // Scatter kernels (unit-stride layers whose taps fit their tile): the corners that land near their
 // position are summed per brick of positions in a fixed-point LDS tile and reach the gradient buffer as one
 // atomic per (voxel, channel) of the tile.
+#include "dcn_pad.hpp"
 #include "dcn_scatter.hpp"
 
 #include <atomic>
@@ -62,10 +63,6 @@ __device__ __forceinline__ void dcn_absmax_block(const T *__restrict__ p, long n
   if (tid < n - tail) take(p[tail + tid]);
   fold_max(bad ? 0x7fc00000u : __float_as_uint(m), out);
 }
-template <typename T>
-__global__ __launch_bounds__(256) void dcn_absmax_kernel(const T *__restrict__ p, long n, unsigned *out) {
-  dcn_absmax_block<T>(p, n, out, blockIdx.x, gridDim.x);
-}
 // max over (group, c, k) of sum_o |Wt[o, c, k]|: a workgroup takes 64 columns, its four wavefronts
 // a quarter of the rows each
 template <typename T>
@@ -82,10 +79,6 @@ __device__ __forceinline__ void dcn_weight_colsum_block(const T *__restrict__ wt
   __syncthreads();
   if (wave == 0) sum = part[0][threadIdx.x] + part[1][threadIdx.x] + part[2][threadIdx.x] + part[3][threadIdx.x];
   fold_max(wave == 0 ? (sum == sum ? __float_as_uint(sum) : 0x7fc00000u) : 0u, out);
-}
-template <typename T>
-__global__ __launch_bounds__(256) void dcn_weight_colsum_kernel(const T *__restrict__ wt, const DcnDims s, unsigned *out) {
-  dcn_weight_colsum_block<T>(wt, s, out, blockIdx.x);
 }
 
 // dcn_backward_tap.hip
@@ -107,12 +100,20 @@ int dcn_tap_backward(const void *xt, const void *off, const void *mask, const vo
 constexpr int kScatterSplit = 2, kScatterWaves = 8 * kScatterSplit, kScatterStride = 9;
 constexpr int kScatterKeep = 4;  // slices of grad_output a wavefront keeps in registers over the taps (all of them)
 
+// Element (output channel o of the padded layer p, channel cl of its group, tap k) of the real layer's weight
+template <typename T>
+__device__ __forceinline__ T padded_weight(const T *__restrict__ wt, const DcnDims &s, const DcnPad &pad, int o, int cl, int k) {
+  const int g = o / pad.p.opg, ol = o - g * pad.p.opg, u = cl / pad.unit_p, r = cl - u * pad.unit_p;
+  return ol < s.opg && r < pad.unit ? wt[(static_cast<long>(g * s.opg + ol) * s.cpg + u * pad.unit + r) * s.K + k] : store_cast<T>(0.f);
+}
+
 // weight [Cout, cpg, K] -> A pieces [group][tap][8-channel block][row step][lane][kPiece]: lane l
 // is MFMA row l % 16 = channel (row / 4) + 4 * (row % 2) of the block (rows 4j + 2, 4j + 3 repeat
 // rows 4j, 4j + 1 and are not used), element i the output channel g*opg + step*4*kPiece +
 // (l/16)*kPiece + i
 template <typename T>
-__device__ __forceinline__ void dcn_weight_afragments8_block(const T *__restrict__ wt, T *__restrict__ wa, const DcnDims s, const unsigned bid) {
+__device__ __forceinline__ void dcn_weight_afragments8_block(const T *__restrict__ wt, T *__restrict__ wa, const DcnDims &real, const DcnPad &pad, const unsigned bid) {
+  const DcnDims &s = pad.p;
   constexpr int PC = Mfma<T>::kPiece;
   const int cblocks = s.cpg / 8, steps = s.opg / (4 * PC);
   const long total = static_cast<long>(s.groups) * s.K * cblocks * steps * 64;
@@ -126,12 +127,8 @@ __device__ __forceinline__ void dcn_weight_afragments8_block(const T *__restrict
   const int g = static_cast<int>(r / s.K);
   const int row = lane % 16, cl = cb * 8 + row / 4 + 4 * (row % 2);
   const int o = g * s.opg + st * 4 * PC + (lane / 16) * PC;
-  for (int i = 0; i < PC; i++) wa[id * PC + i] = wt[(static_cast<long>(o + i) * s.cpg + cl) * s.K + k];
+  for (int i = 0; i < PC; i++) wa[id * PC + i] = padded_weight(wt, real, pad, o + i, cl, k);
 }
-template <typename T>
-__global__ __launch_bounds__(256) void dcn_weight_afragments8_kernel(const T *__restrict__ wt,
-                                                                     T *__restrict__ wa,
-                                                                     const DcnDims s) { dcn_weight_afragments8_block<T>(wt, wa, s, blockIdx.x); }
 
 template <typename T, typename S>
 __global__ __launch_bounds__(kScatterWaves * 64) void dcn_backward_scatter_kernel(
@@ -325,7 +322,8 @@ __host__ __device__ constexpr int scatter32_shift(int terms) {
 // MFMA row l % 16 = channel l % 16 of the block, element i the output channel
 // g*opg + step*4*kPiece + (l/16)*kPiece + i
 template <typename T>
-__device__ __forceinline__ void dcn_weight_afragments16_block(const T *__restrict__ wt, T *__restrict__ wa, const DcnDims s, const unsigned bid) {
+__device__ __forceinline__ void dcn_weight_afragments16_block(const T *__restrict__ wt, T *__restrict__ wa, const DcnDims &real, const DcnPad &pad, const unsigned bid) {
+  const DcnDims &s = pad.p;
   constexpr int PC = Mfma<T>::kPiece;
   const int cblocks = s.cpg / 16, steps = s.opg / (4 * PC);
   const long total = static_cast<long>(s.groups) * s.K * cblocks * steps * 64;
@@ -339,12 +337,8 @@ __device__ __forceinline__ void dcn_weight_afragments16_block(const T *__restric
   const int g = static_cast<int>(r / s.K);
   const int cl = cb * 16 + lane % 16;
   const int o = g * s.opg + st * 4 * PC + (lane / 16) * PC;
-  for (int i = 0; i < PC; i++) wa[id * PC + i] = wt[(static_cast<long>(o + i) * s.cpg + cl) * s.K + k];
+  for (int i = 0; i < PC; i++) wa[id * PC + i] = padded_weight(wt, real, pad, o + i, cl, k);
 }
-template <typename T>
-__global__ __launch_bounds__(256) void dcn_weight_afragments16_kernel(const T *__restrict__ wt,
-                                                                      T *__restrict__ wa,
-                                                                      const DcnDims s) { dcn_weight_afragments16_block<T>(wt, wa, s, blockIdx.x); }
 
 template <typename T, typename S>
 __global__ __launch_bounds__(kScatterWaves * 64) void dcn_backward_scatter32_kernel(
@@ -558,44 +552,43 @@ __global__ __launch_bounds__(kScatterWaves * 64) void dcn_backward_scatter32_ker
   }
 }
 
-// gxt [B, P, C] fp32 -> gx [B, C, P] T, added to what gx holds (`accumulate`) or in its place; 64 positions x up to
-// kAddChunk channels per workgroup
+// gxt [B, P, Cs] fp32 -> gx [B, C, P] T, added to what gx holds (`accumulate`) or in its place; 64 positions x up to
+// kAddChunk channels per workgroup.  The source may hold padded channels: channel c at (c / unit) * unit_p + c % unit.
 constexpr int kAddChunk = 64;
+struct AddShared { __attribute__((aligned(16))) float f[64][kAddChunk + 4]; };   // (16-byte writes; reads along the positions)
 template <typename T>
-__global__ __launch_bounds__(256) void dcn_planar_add_kernel(const float *__restrict__ gxt,
-                                                             T *__restrict__ gx, int C, long P, int accumulate) {
-  __shared__ float stagef[64][kAddChunk + 1];
-  const int b = blockIdx.y;
-  const long p0 = static_cast<long>(blockIdx.x) * 64;
-  const int c0 = blockIdx.z * kAddChunk, cn = min(kAddChunk, C - c0);
+__device__ __forceinline__ void dcn_planar_add_block(AddShared &stage, const float *__restrict__ gxt, T *__restrict__ gx, int C, long P,
+                                                     const unsigned bx, const int b, const int bz, const int accumulate,
+                                                     const int Cs, const int unit, const int unit_p) {
+  const long p0 = static_cast<long>(bx) * 64;
+  const int c0 = bz * kAddChunk, cn = min(kAddChunk, C - c0);
   const int count = static_cast<int>(min(static_cast<long>(64), P - p0)) * cn;
-  const float *src = gxt + (static_cast<long>(b) * P + p0) * C + c0;
+  const float *src = gxt + (static_cast<long>(b) * P + p0) * Cs;
   for (int i = threadIdx.x; i < count; i += 256) {
-    const int pp = i / cn, c = i % cn;
-    stagef[pp][c] = src[static_cast<long>(pp) * C + c];
+    const int pp = i / cn, c = c0 + i % cn;
+    stage.f[pp][c - c0] = src[static_cast<long>(pp) * Cs + c / unit * unit_p + c % unit];
   }
   __syncthreads();
   const int lp = threadIdx.x % 64;
   if (p0 + lp < P)
     for (int c = threadIdx.x / 64; c < cn; c += 4) {
       T *d = gx + (static_cast<long>(b) * C + c0 + c) * P + p0 + lp;
-      *d = store_cast<T>(accumulate ? load(d) + stagef[lp][c] : stagef[lp][c]);
+      *d = store_cast<T>(accumulate ? load(d) + stage.f[lp][c] : stage.f[lp][c]);
     }
 }
 
-// The same move with 16-byte reads (channels in fours, an aligned buffer).  EVEN: P a multiple of 64 and the gradient
+// The same move with 16-byte reads (units and channels in fours, an aligned buffer).  EVEN: P a multiple of 64 and the gradient
 // aligned, so that a lane takes V = 16 / sizeof(T) neighbouring positions of one channel in one write; otherwise a
 // wavefront writes 64 neighbouring elements.  ([4, 256, 38 * 30 * 125] fp16: 431 us through the kernel above.)
 template <typename T, bool EVEN>
-__device__ __forceinline__ void dcn_planar_add_wide_block(const float *__restrict__ gxt, T *__restrict__ gx, int C, long P,
-                                                          const unsigned bx, const int b, const int bz, const int accumulate) {
+__device__ __forceinline__ void dcn_planar_add_wide_block(AddShared &stage, const float *__restrict__ gxt, T *__restrict__ gx, int C, long P,
+                                                          const unsigned bx, const int b, const int bz, const int accumulate,
+                                                          const int Cs, const int unit, const int unit_p) {
   constexpr int V = 16 / static_cast<int>(sizeof(T));
-  // (row pitches: 16-byte writes want multiples of four; reads along the positions want an odd multiple of them)
-  __shared__ __attribute__((aligned(16))) float stagef[64][kAddChunk + 4];
   const long p0 = static_cast<long>(bx) * 64;
   const int c0 = bz * kAddChunk, cn = min(kAddChunk, C - c0);   // cn: a multiple of 4
   const int pn = EVEN ? 64 : static_cast<int>(min(64L, P - p0));
-  const float *src = gxt + (static_cast<long>(b) * P + p0) * C + c0;
+  const float *src = gxt + (static_cast<long>(b) * P + p0) * Cs;
   float4 in[4];
 #pragma unroll
   for (int u = 0; u < 4; u++) {
@@ -603,14 +596,15 @@ __device__ __forceinline__ void dcn_planar_add_wide_block(const float *__restric
     in[u] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (cq * 4 < cn && (EVEN || pp < pn)) {   // (the accumulation buffer is read once and the result not read here again: nontemporal)
       typedef float f32x4 __attribute__((ext_vector_type(4)));
-      const f32x4 t = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(src + static_cast<long>(pp) * C + cq * 4));
+      const int c = c0 + cq * 4, at = unit == unit_p ? c : c / unit * unit_p + c % unit;
+      const f32x4 t = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(src + static_cast<long>(pp) * Cs + at));
       in[u] = make_float4(t.x, t.y, t.z, t.w);
     }
   }
 #pragma unroll
   for (int u = 0; u < 4; u++) {
     const int i = threadIdx.x + u * 256, pp = i / 16, cq = i % 16;
-    *reinterpret_cast<float4 *>(&stagef[pp][cq * 4]) = in[u];
+    *reinterpret_cast<float4 *>(&stage.f[pp][cq * 4]) = in[u];
   }
   __syncthreads();
   if constexpr (EVEN) {
@@ -622,10 +616,10 @@ __device__ __forceinline__ void dcn_planar_add_wide_block(const float *__restric
       if (accumulate) {
         piece.u = *reinterpret_cast<const u32x4 *>(d);
 #pragma unroll
-        for (int e = 0; e < V; e++) piece.e[e] = store_cast<T>(load(&piece.e[e]) + stagef[pg * V + e][c]);
+        for (int e = 0; e < V; e++) piece.e[e] = store_cast<T>(load(&piece.e[e]) + stage.f[pg * V + e][c]);
       } else {
 #pragma unroll
-        for (int e = 0; e < V; e++) piece.e[e] = store_cast<T>(stagef[pg * V + e][c]);
+        for (int e = 0; e < V; e++) piece.e[e] = store_cast<T>(stage.f[pg * V + e][c]);
       }
       __builtin_nontemporal_store(piece.u, reinterpret_cast<u32x4 *>(d));
     }
@@ -642,21 +636,33 @@ __device__ __forceinline__ void dcn_planar_add_wide_block(const float *__restric
 #pragma unroll
         for (int u = 0; u < 4; u++)
           if (c + 4 * u < cn)
-            d[(c + 4 * u) * P] = store_cast<T>(accumulate ? load(&old[u]) + stagef[lp][c + 4 * u] : stagef[lp][c + 4 * u]);
+            d[(c + 4 * u) * P] = store_cast<T>(accumulate ? load(&old[u]) + stage.f[lp][c + 4 * u] : stage.f[lp][c + 4 * u]);
       }
     }
   }
 }
-template <typename T, bool EVEN>
-__global__ __launch_bounds__(256) void dcn_planar_add_wide_kernel(const float *__restrict__ gxt,
-                                                                  T *__restrict__ gx, int C, long P, int accumulate) {
-  dcn_planar_add_wide_block<T, EVEN>(gxt, gx, C, P, blockIdx.x, blockIdx.y, blockIdx.z, accumulate);
+// MODE 0: the plain move, 1: 16-byte reads, 2: 16-byte writes as well
+template <typename T, int MODE>
+__device__ __forceinline__ void dcn_planar_add_mode(AddShared &stage, const float *__restrict__ gxt, T *__restrict__ gx, int C, long P, const unsigned bx,
+                                                    const int b, const int bz, const int accumulate, const int Cs, const int unit,
+                                                    const int unit_p) {
+  if constexpr (MODE == 0) dcn_planar_add_block<T>(stage, gxt, gx, C, P, bx, b, bz, accumulate, Cs, unit, unit_p);
+  else dcn_planar_add_wide_block<T, MODE == 2>(stage, gxt, gx, C, P, bx, b, bz, accumulate, Cs, unit, unit_p);
+}
+static int planar_add_mode(const void *src, const void *dst, int unit, long P) {
+  auto aligned16 = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  return unit % 4 || !aligned16(src) ? 0 : (P % 64 == 0 && aligned16(dst) ? 2 : 1);
+}
+template <typename T, int MODE>
+__global__ __launch_bounds__(256) void dcn_planar_add_kernel(const float *__restrict__ gxt, T *__restrict__ gx, int C, long P,
+                                                             int accumulate) {
+  __shared__ AddShared stage;
+  dcn_planar_add_mode<T, MODE>(stage, gxt, gx, C, P, blockIdx.x, blockIdx.y, blockIdx.z, accumulate, C, C, C);
 }
 
 __device__ __forceinline__ void dcn_zero_f32_block(float *p, long n, const unsigned bid, const unsigned nblocks) {
   for (long i = bid * 256L + threadIdx.x; i < n; i += nblocks * 256L) p[i] = 0.f;
 }
-__global__ __launch_bounds__(256) void dcn_zero_f32_kernel(float *p, long n) { dcn_zero_f32_block(p, n, blockIdx.x, gridDim.x); }
 
 // One pass over a slab of grad_output[b, o, .]: its sum into the fp32 bias accumulator and (`out`
 // given) its largest magnitude as a bit pattern into *out.  Workgroup = (o, b, slab of `slab_len`
@@ -708,39 +714,33 @@ __device__ __forceinline__ void dcn_gy_sum_max_block(const T *__restrict__ gy, f
   else __syncthreads();
   if (threadIdx.x == 0) atomicAdd(gb32 + o, (sums[0] + sums[1]) + (sums[2] + sums[3]));
 }
-template <typename T>
-__global__ __launch_bounds__(256) void dcn_gy_sum_kernel(const T *__restrict__ gy, float *__restrict__ gb32, const DcnDims s,
-                                                         const long slab_len) {
-  dcn_gy_sum_max_block<T>(gy, gb32, nullptr, s, slab_len, blockIdx.x);
-}
 
-// The small jobs in front of the data kernel of a layer with tiles, in two launches instead of eight
-// (a dependent launch costs ~2.7 us before its first instruction, and kernels of a few microseconds do
-// not fill the machine): first the two layout passes, the weight fragments and the zero fill of the
-// accumulators and of the maxima's words; then the maxima, which need those words at zero.
+// The small jobs in front of the tap kernel in two launches (a dependent launch costs ~2.7 us before its first
+// instruction, and kernels of a few microseconds do not fill the machine): first the two layout passes, the weight
+// fragments and the zero fill of the accumulators and of the maxima's words; then the maxima and the bias sums, which need those
+// words at zero.
 struct PrepareJobs {
   unsigned x_end, gy_end, f16_end, fsc_end, zero_end;   // block ranges of the first launch
-  unsigned wbx, wbq;                                    // 128-position blocks of the input / the output
+  unsigned px, pq;                                      // blocks of positions of the input / the output
 };
 template <typename T>
 __global__ __launch_bounds__(256) void dcn_backward_prepare_kernel(const T *__restrict__ x, T *__restrict__ xt,
                                                                    const T *__restrict__ gy, T *__restrict__ gyt,
                                                                    const T *__restrict__ wt, T *__restrict__ wb,
                                                                    T *__restrict__ wa, float *__restrict__ zero,
-                                                                   const long nz, const DcnDims s, const PrepareJobs j) {
+                                                                   const long nz, const DcnDims s, const DcnPad pad, const PrepareJobs j) {
   using U = typename std::conditional<(sizeof(T) == 2), unsigned short, unsigned int>::type;
   const unsigned id = blockIdx.x;
-  if (id < j.x_end) {
-    channels_last_wide_block<U>(reinterpret_cast<const U *>(x), reinterpret_cast<U *>(xt), s.Cin, s.P, id % j.wbx,
-                                static_cast<int>((id / j.wbx) % s.B), static_cast<int>(id / (j.wbx * s.B)));
-  } else if (id < j.gy_end) {
-    const unsigned r = id - j.x_end;
-    channels_last_wide_block<U>(reinterpret_cast<const U *>(gy), reinterpret_cast<U *>(gyt), s.Cout, s.Q, r % j.wbq,
-                                static_cast<int>((r / j.wbq) % s.B), static_cast<int>(r / (j.wbq * s.B)));
+  if (id < j.gy_end) {   // (one body, and one LDS block, for both)
+    const bool first = id < j.x_end;
+    const unsigned r = first ? id : id - j.x_end, pb = first ? j.px : j.pq;
+    dcn_move_block<U>(reinterpret_cast<const U *>(first ? x : gy), reinterpret_cast<U *>(first ? xt : gyt), first ? s.Cin : s.Cout,
+                      first ? pad.p.Cin : pad.p.Cout, first ? pad.unit : s.opg, first ? pad.unit_p : pad.p.opg, first ? s.P : s.Q,
+                      r % pb, static_cast<int>((r / pb) % s.B), static_cast<int>(r / pb / s.B));
   } else if (id < j.f16_end) {
-    dcn_weight_afragments16_block<T>(wt, wb, s, id - j.gy_end);
+    dcn_weight_afragments16_block<T>(wt, wb, s, pad, id - j.gy_end);
   } else if (id < j.fsc_end) {
-    dcn_weight_afragments8_block<T>(wt, wa, s, id - j.f16_end);
+    dcn_weight_afragments8_block<T>(wt, wa, s, pad, id - j.f16_end);
   } else {
     dcn_zero_f32_block(zero, nz, id - j.fsc_end, j.zero_end - j.fsc_end);
   }
@@ -821,8 +821,9 @@ size_t dcn_mfma_backward_workspace_bytes(const DcnDims &s, int dtype) { return b
 
 template <typename T>
 static int backward_run(const void *x, const void *off, const void *mask, const void *wt,
-                        const void *gy, void *goff, void *gmask, const DcnDims &s, void *workspace,
+                        const void *gy, void *goff, void *gmask, const DcnDims &real, const DcnPad &pad, void *workspace,
                         float **gx32, float **gw32, float **gb32, int dtype, bool want_bias, hipStream_t stream) {
+  const DcnDims &s = pad.p;
   const BackwardLayout l = backward_layout(s, dtype);
   char *ws = static_cast<char *>(workspace);
   T *xt = reinterpret_cast<T *>(ws + l.xt), *gyt = reinterpret_cast<T *>(ws + l.gyt), *wb = reinterpret_cast<T *>(ws + l.wb);
@@ -839,62 +840,33 @@ static int backward_run(const void *x, const void *off, const void *mask, const 
   const long frag_lanes = static_cast<long>(s.groups) * s.K * (s.cpg / 16) * (s.opg / (4 * Mfma<T>::kPiece)) * 64;
   const long scatter_lanes = tiles && !narrow ? static_cast<long>(s.groups) * s.K * (s.cpg / 8) * (s.opg / (4 * Mfma<T>::kPiece)) * 64 : 0;
   const long nz = static_cast<long>((l.part - l.gxt) / 4);
-  const long ngy = static_cast<long>(s.B) * s.Cout * s.Q, nmask = static_cast<long>(s.B) * s.dg * s.K * s.Q;
-  const long ncols = static_cast<long>(s.groups) * s.cpg * s.K;
-  constexpr int V = 16 / static_cast<int>(sizeof(T)), CH = 256 / static_cast<int>(sizeof(T));
-  auto aligned16 = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  const long wbx = (s.P + kLayoutPos - 1) / kLayoutPos, wbq = (s.Q + kLayoutPos - 1) / kLayoutPos;
-  const long nx = wbx * s.B * ((s.Cin + CH - 1) / CH), ngyb = wbq * s.B * ((s.Cout + CH - 1) / CH);
+  const long ngy = static_cast<long>(s.B) * real.Cout * s.Q, nmask = static_cast<long>(s.B) * s.dg * s.K * s.Q;
+  const long ncols = static_cast<long>(s.groups) * real.cpg * s.K;
+  constexpr int CH = 128 / static_cast<int>(sizeof(T));   // channels of a move
+  const long px = (s.P + kMovePos - 1) / kMovePos, pq = (s.Q + kMovePos - 1) / kMovePos;
+  const long nx = px * s.B * ((s.Cin + CH - 1) / CH), ngyb = pq * s.B * ((s.Cout + CH - 1) / CH);
   const long nf16 = (frag_lanes + 255) / 256, nfsc = (scatter_lanes + 255) / 256, nzb = min((nz + 1023) / 1024, 4096L);
-  int st = MV_OK;
-  bool bias_summed = false;
-  if (tiles && aligned16(x) && aligned16(xt) && aligned16(gy) && aligned16(gyt) && s.P % V == 0 && s.Q % V == 0 &&
-      s.Cin % V == 0 && s.Cout % V == 0 && nx + ngyb + nf16 + nfsc + nzb < (1L << 31)) {
-    PrepareJobs j;
-    j.x_end = static_cast<unsigned>(nx); j.gy_end = j.x_end + static_cast<unsigned>(ngyb);
-    j.f16_end = j.gy_end + static_cast<unsigned>(nf16); j.fsc_end = j.f16_end + static_cast<unsigned>(nfsc);
-    j.zero_end = j.fsc_end + static_cast<unsigned>(nzb);
-    j.wbx = static_cast<unsigned>(wbx); j.wbq = static_cast<unsigned>(wbq); 
-    hipLaunchKernelGGL((dcn_backward_prepare_kernel<T>), dim3(j.zero_end), dim3(256), 0, stream, static_cast<const T *>(x), xt,
-                       static_cast<const T *>(gy), gyt, static_cast<const T *>(wt), wb, wa, gxt, nz, s, j);
-    const long slab_len = gy_slab_len(s);
-    const long sum_blocks = static_cast<long>(s.Cout) * s.B * ((s.Q + slab_len - 1) / slab_len);
-    const bool sums = want_bias && sum_blocks < (1L << 30);
-    const unsigned gy_blocks = sums ? static_cast<unsigned>(sum_blocks) : static_cast<unsigned>(min((ngy + 8191) / 8192, 256L));
-    const unsigned mask_blocks = mask ? static_cast<unsigned>(min((nmask + 8191) / 8192, 256L)) : 0u;
-    hipLaunchKernelGGL((dcn_backward_maxima_kernel<T>), dim3(gy_blocks + mask_blocks + static_cast<unsigned>((ncols + 63) / 64)),
-                       dim3(256), 0, stream, static_cast<const T *>(gy), ngy, static_cast<const T *>(mask), nmask,
-                       static_cast<const T *>(wt), s, bounds, sums ? *gb32 : nullptr, slab_len, gy_blocks, mask_blocks);
-    bias_summed = sums;
-  } else {
-    st = dcn_channels_last(x, xt, s.B, s.Cin, s.P, sizeof(T), stream);
-    if (st) return st;
-    st = dcn_channels_last(gy, gyt, s.B, s.Cout, s.Q, sizeof(T), stream);
-    if (st) return st;
-    hipLaunchKernelGGL((dcn_weight_afragments16_kernel<T>), dim3(static_cast<unsigned>(nf16)), dim3(256), 0, stream,
-                       static_cast<const T *>(wt), wb, s);
-    hipLaunchKernelGGL(dcn_zero_f32_kernel, dim3(static_cast<unsigned>(min((nz + 1023) / 1024, 65536L))), dim3(256),
-                       0, stream, gxt, nz);
-    if (tiles) {
-      hipLaunchKernelGGL((dcn_absmax_kernel<T>), dim3(static_cast<unsigned>(min((ngy + 8191) / 8192, 256L))), dim3(256),
-                         0, stream, static_cast<const T *>(gy), ngy, bounds);
-      hipLaunchKernelGGL((dcn_weight_colsum_kernel<T>), dim3(static_cast<unsigned>((ncols + 63) / 64)), dim3(256), 0,
-                         stream, static_cast<const T *>(wt), s, bounds + 1);
-      if (mask)
-        hipLaunchKernelGGL((dcn_absmax_kernel<T>), dim3(static_cast<unsigned>(min((nmask + 8191) / 8192, 256L))),
-                           dim3(256), 0, stream, static_cast<const T *>(mask), nmask, bounds + 2);
-      if (!narrow)
-        hipLaunchKernelGGL((dcn_weight_afragments8_kernel<T>), dim3(static_cast<unsigned>(nfsc)), dim3(256), 0, stream,
-                           static_cast<const T *>(wt), wa, s);
-    }
+  MV_REQUIRE(nx + ngyb + nf16 + nfsc + nzb < (1L << 31), "volume too large");
+  PrepareJobs j;
+  j.x_end = static_cast<unsigned>(nx); j.gy_end = j.x_end + static_cast<unsigned>(ngyb);
+  j.f16_end = j.gy_end + static_cast<unsigned>(nf16); j.fsc_end = j.f16_end + static_cast<unsigned>(nfsc);
+  j.zero_end = j.fsc_end + static_cast<unsigned>(nzb);
+  j.px = static_cast<unsigned>(px); j.pq = static_cast<unsigned>(pq);
+  hipLaunchKernelGGL((dcn_backward_prepare_kernel<T>), dim3(j.zero_end), dim3(256), 0, stream, static_cast<const T *>(x), xt,
+                     static_cast<const T *>(gy), gyt, static_cast<const T *>(wt), wb, wa, gxt, nz, real, pad, j);
+  if (tiles || want_bias) {
+    const long slab_len = gy_slab_len(real);
+    const long sum_blocks = static_cast<long>(real.Cout) * s.B * ((s.Q + slab_len - 1) / slab_len);
+    const unsigned gy_blocks = static_cast<unsigned>(want_bias ? sum_blocks : min((ngy + 8191) / 8192, 256L));
+    const unsigned mask_blocks = mask && tiles ? static_cast<unsigned>(min((nmask + 8191) / 8192, 256L)) : 0u;
+    const unsigned col_blocks = tiles ? static_cast<unsigned>((ncols + 63) / 64) : 0u;
+    MV_REQUIRE(sum_blocks < (1L << 30), "grid too large");
+    hipLaunchKernelGGL((dcn_backward_maxima_kernel<T>), dim3(gy_blocks + mask_blocks + col_blocks), dim3(256), 0, stream,
+                       static_cast<const T *>(gy), ngy, static_cast<const T *>(mask), nmask, static_cast<const T *>(wt), real,
+                       tiles ? bounds : nullptr, want_bias ? *gb32 : nullptr, slab_len, gy_blocks, mask_blocks);
   }
-  if (want_bias && !bias_summed) {
-    const long slab_len = gy_slab_len(s);
-    const long sum_blocks = static_cast<long>(s.Cout) * s.B * ((s.Q + slab_len - 1) / slab_len);
-    MV_REQUIRE(sum_blocks < (1L << 31), "grid too large");
-    hipLaunchKernelGGL((dcn_gy_sum_kernel<T>), dim3(static_cast<unsigned>(sum_blocks)), dim3(256), 0, stream,
-                       static_cast<const T *>(gy), *gb32, s, slab_len);
-  }
+  int st = check_launch("dcn_backward_prepare_kernel");
+  if (st) return st;
   st = dcn_tap_backward(xt, off, mask, gyt, wb, gxt, goff, gmask, reinterpret_cast<float *>(ws + l.part), *gw32, s,
                         tiles ? bounds : nullptr, dtype, stream);
   if (st || !tiles) return st;
@@ -919,19 +891,19 @@ static int backward_run(const void *x, const void *off, const void *mask, const 
   return check_launch("dcn_backward_scatter_kernel");
 }
 
-// Runs the data and weight kernels; grad_offset / grad_mask are written, the fp32 gradients of
-// input (channels-last; dcn_planar_add) and weight (tap-major; dcn_weight_add) and the bias
-// accumulator (zero; with `want_bias` the sums of grad_output over samples and positions) are returned
-// for the caller to fold in.
+// Runs the kernels of the layer, padded to channel counts that they take (`pad.p`; the layer itself when it has such):
+// grad_offset / grad_mask are written, the fp32 gradients of input (channels-last) and weight (tap-major) of the padded
+// layer and the bias accumulator (with `want_bias` the sums of grad_output over samples and positions) are
+// returned for the caller to fold in.
 int dcn_mfma_backward(const void *x, const void *off, const void *mask, const void *wt,
-                      const void *gy, void *goff, void *gmask, const DcnDims &s, int dtype,
+                      const void *gy, void *goff, void *gmask, const DcnDims &s, const DcnPad &pad, int dtype,
                       void *workspace, bool want_bias, float **gx32, float **gw32, float **gb32,
                       hipStream_t stream) {
   if (dtype == MV_F16)
-    return backward_run<__half>(x, off, mask, wt, gy, goff, gmask, s, workspace, gx32, gw32, gb32, dtype, want_bias, stream);
+    return backward_run<__half>(x, off, mask, wt, gy, goff, gmask, s, pad, workspace, gx32, gw32, gb32, dtype, want_bias, stream);
   if (dtype == MV_F32)
-    return backward_run<float>(x, off, mask, wt, gy, goff, gmask, s, workspace, gx32, gw32, gb32, dtype, want_bias, stream);
-  return backward_run<__hip_bfloat16>(x, off, mask, wt, gy, goff, gmask, s, workspace, gx32, gw32, gb32, dtype, want_bias, stream);
+    return backward_run<float>(x, off, mask, wt, gy, goff, gmask, s, pad, workspace, gx32, gw32, gb32, dtype, want_bias, stream);
+  return backward_run<__hip_bfloat16>(x, off, mask, wt, gy, goff, gmask, s, pad, workspace, gx32, gw32, gb32, dtype, want_bias, stream);
 }
 
 // dst [B, C, P] (element type of `dtype`) += src [B, P, C] fp32 (= src when not `accumulate`)
@@ -939,104 +911,84 @@ int planar_add_f32(const float *src, void *dst, int B, int C, long P, int dtype,
   const long pblocks = (P + 63) / 64;
   MV_REQUIRE(pblocks < (1L << 31) && B <= 65535 && (C + kAddChunk - 1) / kAddChunk <= 65535, "volume too large");
   const dim3 grid(static_cast<unsigned>(pblocks), B, (C + kAddChunk - 1) / kAddChunk);
-  const bool wide = C % 4 == 0 && reinterpret_cast<uintptr_t>(src) % 16 == 0;
-  const bool even = wide && P % 64 == 0 && reinterpret_cast<uintptr_t>(dst) % 16 == 0;
+  const int mode = planar_add_mode(src, dst, C, P);
+#define MV_PLANAR_ADD_AS(TYPE, MODE)                                                                                  \
+  hipLaunchKernelGGL((dcn_planar_add_kernel<TYPE, MODE>), grid, dim3(256), 0, stream, src, static_cast<TYPE *>(dst), C, P, \
+                     accumulate ? 1 : 0)
 #define MV_PLANAR_ADD(TYPE)                                                                                           \
   do {                                                                                                               \
-    if (even)                                                                                                        \
-      hipLaunchKernelGGL((dcn_planar_add_wide_kernel<TYPE, true>), grid, dim3(256), 0, stream, src,                   \
-                         static_cast<TYPE *>(dst), C, P, accumulate ? 1 : 0);                                         \
-    else if (wide)                                                                                                   \
-      hipLaunchKernelGGL((dcn_planar_add_wide_kernel<TYPE, false>), grid, dim3(256), 0, stream, src,                  \
-                         static_cast<TYPE *>(dst), C, P, accumulate ? 1 : 0);                                         \
-    else                                                                                                             \
-      hipLaunchKernelGGL((dcn_planar_add_kernel<TYPE>), grid, dim3(256), 0, stream, src, static_cast<TYPE *>(dst), C, \
-                         P, accumulate ? 1 : 0);                                                                      \
+    if (mode == 2) MV_PLANAR_ADD_AS(TYPE, 2);                                                                         \
+    else if (mode == 1) MV_PLANAR_ADD_AS(TYPE, 1);                                                                    \
+    else MV_PLANAR_ADD_AS(TYPE, 0);                                                                                   \
   } while (0)
   if (dtype == MV_F16) MV_PLANAR_ADD(__half);
   else if (dtype == MV_F32) MV_PLANAR_ADD(float);
   else MV_PLANAR_ADD(__hip_bfloat16);
 #undef MV_PLANAR_ADD
+#undef MV_PLANAR_ADD_AS
   return check_launch("dcn_planar_add_kernel");
 }
 
 // grad_weight [Cout][cpg][K] += the tap-major fp32 accumulator [K][Cout][cpg] of the weight kernel
 template <typename T>
-__device__ __forceinline__ void dcn_weight_add_block(const float *__restrict__ acc, T *__restrict__ gw, const DcnDims s,
+__device__ __forceinline__ void dcn_weight_add_block(const float *__restrict__ acc, T *__restrict__ gw, const DcnDims &s, const DcnPad &pad,
                                                      const unsigned bid, const unsigned nblocks, const int accumulate) {
+  const DcnDims &p = pad.p;
   const long n = static_cast<long>(s.Cout) * s.cpg * s.K;
   for (long i = bid * 256L + threadIdx.x; i < n; i += nblocks * 256L) {
-    const long k = i % s.K, oc = i / s.K;
-    const float v = acc[k * s.Cout * s.cpg + oc];
+    const int k = static_cast<int>(i % s.K), c = static_cast<int>(i / s.K % s.cpg), o = static_cast<int>(i / s.K / s.cpg);
+    const int g = o / s.opg, u = c / pad.unit;
+    const float v = acc[(static_cast<long>(k) * p.Cout + g * p.opg + o - g * s.opg) * p.cpg + u * pad.unit_p + c - u * pad.unit];
     gw[i] = store_cast<T>(accumulate ? load(gw + i) + v : v);
   }
-}
-template <typename T>
-__global__ __launch_bounds__(256) void dcn_weight_add_kernel(const float *__restrict__ acc, T *__restrict__ gw,
-                                                             const DcnDims s, const int accumulate) {
-  dcn_weight_add_block<T>(acc, gw, s, blockIdx.x, gridDim.x, accumulate);
 }
 
 // The folds behind the backward kernels in one launch: channels-last fp32 grad input -> grad_input,
 // tap-major fp32 grad weight -> grad_weight, the fp32 bias sums -> grad_bias.
-template <typename T, bool EVEN>
+template <typename T, int MODE>
 __global__ __launch_bounds__(256) void dcn_backward_fold_kernel(const float *__restrict__ gxt, T *__restrict__ gx,
                                                                 const float *__restrict__ gw32, T *__restrict__ gw,
                                                                 const float *__restrict__ gb32, T *__restrict__ gb,
-                                                                const DcnDims s, const unsigned pblocks,
+                                                                const DcnDims s, const DcnPad pad, const unsigned pblocks,
                                                                 const unsigned add_end, const unsigned weight_end,
                                                                 const int accumulate) {
+  __shared__ AddShared stage;
   const unsigned id = blockIdx.x;
   if (id < add_end)
-    dcn_planar_add_wide_block<T, EVEN>(gxt, gx, s.Cin, s.P, id % pblocks, static_cast<int>((id / pblocks) % s.B),
-                                       static_cast<int>(id / (pblocks * s.B)), accumulate);
+    dcn_planar_add_mode<T, MODE>(stage, gxt, gx, s.Cin, s.P, id % pblocks, static_cast<int>((id / pblocks) % s.B),
+                                       static_cast<int>(id / (pblocks * s.B)), accumulate, pad.p.Cin, pad.unit, pad.unit_p);
   else if (id < weight_end)
-    dcn_weight_add_block<T>(gw32, gw, s, id - add_end, weight_end - add_end, accumulate);
+    dcn_weight_add_block<T>(gw32, gw, s, pad, id - add_end, weight_end - add_end, accumulate);
   else
     for (int o = threadIdx.x; o < s.Cout; o += 256) gb[o] = store_cast<T>((accumulate ? static_cast<float>(load(gb + o)) : 0.f) + gb32[o]);
 }
 
-// All three folds of a layer on the matrix-core path.  Returns -1 when the tensors do not allow the
-// 16-byte accesses of the one-launch form (the caller then folds one by one).
+// All three folds of a layer on the matrix-core path.
 int dcn_backward_fold(const float *gxt, const float *gw32, const float *gb32, void *grad_input, void *grad_weight,
-                      void *grad_bias, const DcnDims &s, int dtype, bool accumulate, hipStream_t stream) {
-  if (dtype != MV_F16 && dtype != MV_BF16 && dtype != MV_F32) return -1;
-  auto aligned16 = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  if (s.Cin % 4 || !aligned16(gxt)) return -1;
-  const bool even = s.P % 64 == 0 && aligned16(grad_input);
+                      void *grad_bias, const DcnDims &s, const DcnPad &pad, int dtype, bool accumulate, hipStream_t stream) {
+  const int mode = planar_add_mode(gxt, grad_input, pad.unit, s.P);
   const long pblocks = (s.P + 63) / 64, add_blocks = pblocks * s.B * ((s.Cin + kAddChunk - 1) / kAddChunk);
   const long n = static_cast<long>(s.Cout) * s.cpg * s.K, weight_blocks = min((n + 255) / 256, 1024L);
   const long bias_blocks = grad_bias ? 1 : 0;
-  if (add_blocks + weight_blocks + bias_blocks >= (1L << 31)) return -1;
+  MV_REQUIRE(add_blocks + weight_blocks + bias_blocks < (1L << 31), "volume too large");
   const unsigned add_end = static_cast<unsigned>(add_blocks), weight_end = add_end + static_cast<unsigned>(weight_blocks);
-#define MV_FOLD_AS(T, EVENV)                                                                                          \
-  hipLaunchKernelGGL((dcn_backward_fold_kernel<T, EVENV>), dim3(weight_end + static_cast<unsigned>(bias_blocks)), dim3(256), 0, \
+#define MV_FOLD_AS(T, MODE)                                                                                          \
+  hipLaunchKernelGGL((dcn_backward_fold_kernel<T, MODE>), dim3(weight_end + static_cast<unsigned>(bias_blocks)), dim3(256), 0, \
                      stream, gxt, static_cast<T *>(grad_input), gw32, static_cast<T *>(grad_weight),               \
-                     gb32, static_cast<T *>(grad_bias), s,                                                         \
+                     gb32, static_cast<T *>(grad_bias), s, pad,                                                    \
                      static_cast<unsigned>(pblocks), add_end, weight_end, accumulate ? 1 : 0)
-#define MV_FOLD(T) do { if (even) MV_FOLD_AS(T, true); else MV_FOLD_AS(T, false); } while (0)
+#define MV_FOLD(T)                                                                                                    \
+  do {                                                                                                               \
+    if (mode == 2) MV_FOLD_AS(T, 2);                                                                                  \
+    else if (mode == 1) MV_FOLD_AS(T, 1);                                                                             \
+    else MV_FOLD_AS(T, 0);                                                                                            \
+  } while (0)
   if (dtype == MV_F16) MV_FOLD(__half);
   else if (dtype == MV_BF16) MV_FOLD(__hip_bfloat16);
   else MV_FOLD(float);
 #undef MV_FOLD
 #undef MV_FOLD_AS
   return check_launch("dcn_backward_fold_kernel");
-}
-int dcn_weight_add(const float *acc, void *gw, const DcnDims &s, int dtype, bool accumulate, hipStream_t stream) {
-  const long n = static_cast<long>(s.Cout) * s.cpg * s.K;
-  const dim3 grid(static_cast<unsigned>(min((n + 255) / 256, 4096L)));
-  if (dtype == MV_F16)
-    hipLaunchKernelGGL((dcn_weight_add_kernel<__half>), grid, dim3(256), 0, stream, acc, static_cast<__half *>(gw), s, accumulate ? 1 : 0);
-  else if (dtype == MV_F32)
-    hipLaunchKernelGGL((dcn_weight_add_kernel<float>), grid, dim3(256), 0, stream, acc, static_cast<float *>(gw), s, accumulate ? 1 : 0);
-  else
-    hipLaunchKernelGGL((dcn_weight_add_kernel<__hip_bfloat16>), grid, dim3(256), 0, stream, acc,
-                       static_cast<__hip_bfloat16 *>(gw), s, accumulate ? 1 : 0);
-  return check_launch("dcn_weight_add_kernel");
-}
-
-int dcn_planar_add(const float *gxt, void *gx, const DcnDims &s, int dtype, bool accumulate, hipStream_t stream) {
-  return planar_add_f32(gxt, gx, s.B, s.Cin, s.P, dtype, accumulate, stream);
 }
 
 }  // namespace mv

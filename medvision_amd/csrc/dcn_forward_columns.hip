@@ -29,41 +29,6 @@
 namespace mv {
 
 // ---- layouts: x [B, C, P] -> xt [B, P, C] and the weight fragments, one launch --------------------------------------
-// 64 positions x 128 bytes of channels per workgroup through LDS.  Rows of any alignment: 16 bytes at a time all the same.
-constexpr int kMovePos = 64;
-template <typename U>
-__device__ __forceinline__ void dcn_move_block(const U *__restrict__ x, U *__restrict__ xt, const int C, const long P,
-                                               const long bx, const int b, const int bz) {
-  constexpr int V = 16 / sizeof(U), CH = 128 / sizeof(U), PITCH = kMovePos + V, PG = kMovePos / V;
-  typedef unsigned int piece_t __attribute__((ext_vector_type(4), aligned(2)));   // (element alignment: the hardware takes it)
-  __shared__ __attribute__((aligned(16))) U stage[CH * PITCH];
-  const long p0 = bx * kMovePos;
-  const int c0 = bz * CH, cn = min(CH, C - c0), np = static_cast<int>(min(static_cast<long>(kMovePos), P - p0));
-  const U *src = x + (static_cast<long>(b) * C + c0) * P + p0;
-#pragma unroll
-  for (int u = 0; u < CH * PG / 256; u++) {
-    const int i = threadIdx.x + u * 256, c = i / PG, at = i % PG * V;
-    if (c >= cn) continue;
-    const U *from = src + static_cast<long>(c) * P + at;
-    if (at + V <= np) {
-      *reinterpret_cast<u32x4 *>(stage + c * PITCH + at) = *reinterpret_cast<const piece_t *>(from);
-    } else {
-      for (int e = 0; at + e < np; e++) stage[c * PITCH + at + e] = from[e];
-    }
-  }
-  __syncthreads();
-  const int groups = cn / V;
-  for (int i = threadIdx.x; i < np * groups; i += 256) {
-    const int p = i / groups, cg = i - p * groups;
-    U out[V];
-#pragma unroll
-    for (int e = 0; e < V; e++) out[e] = stage[(cg * V + e) * PITCH + p];
-    u32x4 packed;
-    __builtin_memcpy(&packed, out, 16);
-    *reinterpret_cast<u32x4 *>(xt + (static_cast<long>(b) * P + p0 + p) * C + c0 + cg * V) = packed;
-  }
-}
-
 // weight [Cout, cpg, K] -> [group][16-row block][K step][lane][piece]: lane l holds row l % 16 and flat piece 4 * step + l / 16
 // (tap piece / (cpg / PC), channels piece % (cpg / PC)); pieces beyond the last one are zeros
 template <typename U>
@@ -85,13 +50,30 @@ __device__ __forceinline__ void dcn_flat_fragments_block(const U *__restrict__ w
   *reinterpret_cast<u32x4 *>(wf + id * PC) = packed;
 }
 
+// the first of the two alone, for callers outside this file: elements of 2 or 4 bytes, channels in whole 16 bytes
+template <typename U>
+__global__ __launch_bounds__(256) void channels_last_kernel(const U *__restrict__ x, U *__restrict__ xt, const int C, const long P) {
+  dcn_move_block<U>(x, xt, C, C, C, C, P, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+int channels_last(const void *x, void *xt, int B, int C, long P, int elem_bytes, hipStream_t stream) {
+  const long blocks = (P + kMovePos - 1) / kMovePos;
+  const int ch = 128 / elem_bytes;
+  MV_REQUIRE(blocks < (1L << 31) && B <= 65535 && (C + ch - 1) / ch <= 65535, "volume too large");
+  const dim3 grid(static_cast<unsigned>(blocks), B, (C + ch - 1) / ch);
+  if (elem_bytes == 2)
+    hipLaunchKernelGGL((channels_last_kernel<unsigned short>), grid, dim3(256), 0, stream, static_cast<const unsigned short *>(x), static_cast<unsigned short *>(xt), C, P);
+  else
+    hipLaunchKernelGGL((channels_last_kernel<unsigned int>), grid, dim3(256), 0, stream, static_cast<const unsigned int *>(x), static_cast<unsigned int *>(xt), C, P);
+  return check_launch("channels_last_kernel");
+}
+
 template <typename U>
 __global__ __launch_bounds__(256) void dcn_columns_layout_kernel(const U *__restrict__ x, U *__restrict__ xt,
                                                                  const U *__restrict__ wt, U *__restrict__ wf, const DcnDims s,
                                                                  const unsigned pblocks, const unsigned moves) {
   if (blockIdx.x < moves) {
     const unsigned bx = blockIdx.x % pblocks, r = blockIdx.x / pblocks;
-    dcn_move_block<U>(x, xt, s.Cin, s.P, bx, static_cast<int>(r % s.B), static_cast<int>(r / s.B));
+    dcn_move_block<U>(x, xt, s.Cin, s.Cin, s.Cin, s.Cin, s.P, bx, static_cast<int>(r % s.B), static_cast<int>(r / s.B));
   } else {
     dcn_flat_fragments_block<U>(wt, wf, s, (blockIdx.x - moves) * 256L + threadIdx.x);
   }

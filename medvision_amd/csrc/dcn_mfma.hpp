@@ -109,42 +109,53 @@ template <> struct Mfma<float> {
   }
 };
 
-// x [B, C, P] -> xt [B, P, C], elements of `elem_bytes` (2 or 4); defined in dcn3d_mfma.hip
-int dcn_channels_last(const void *x, void *xt, int B, int C, long P, int elem_bytes, hipStream_t stream);
-
-// The same move with 16-byte global accesses: rows of x are read as groups of 16 bytes (V
-// positions of one channel), kept in LDS as [channel][position], and every lane writes V channels
-// of one position.  Needs P and Cin to be multiples of V and 16-byte aligned tensors.
-constexpr int kLayoutPos = 128;
+// x [B, C, P] -> xt [B, P, Cp], channel c at (c / unit) * unit_p + c % unit, zeros elsewhere (Cp = C / unit * unit_p, a multiple of
+// 16 bytes; unit = unit_p: no padding).  64 positions x 128 bytes of channels per workgroup through LDS; rows of any
+// alignment, 16 bytes at a time all the same.  (U: the element as an integer of its size.)
+//   ([8, 256, 100 x 152] fp16: 29 us with 64 positions, 41 us with 128 positions x 256 bytes; [128, 7 x 45 x 18], whose
+//   rows are not aligned: 4 us, 12 us element by element.)
+constexpr int kMovePos = 64;
 template <typename U>
-__device__ __forceinline__ void channels_last_wide_block(const U *__restrict__ x, U *__restrict__ xt, int Cin, long P,
-                                                         unsigned bx, int b, int bz) {
-  constexpr int V = 16 / sizeof(U), CH = 256 / sizeof(U);   // CH channels per workgroup: 128 (2 bytes), 64 (4 bytes)
-  constexpr int PITCH = kLayoutPos + V;
+__device__ __forceinline__ void dcn_move_block(const U *__restrict__ x, U *__restrict__ xt, const int C, const int Cp, const int unit,
+                                               const int unit_p, const long P, const long bx, const int b, const int bz) {
+  constexpr int V = 16 / sizeof(U), CH = 128 / sizeof(U), PITCH = kMovePos + V, PG = kMovePos / V;
+  typedef unsigned int piece_t __attribute__((ext_vector_type(4), aligned(2)));   // (element alignment: the hardware takes it)
   __shared__ __attribute__((aligned(16))) U stage[CH * PITCH];
-  const long p0 = static_cast<long>(bx) * kLayoutPos;
-  const int c0 = bz * CH, cn = min(CH, Cin - c0);
-  const int np = static_cast<int>(min(static_cast<long>(kLayoutPos), P - p0));   // a multiple of V
-  const U *src = x + (static_cast<long>(b) * Cin + c0) * P + p0;
-  U *dst = xt + (static_cast<long>(b) * P + p0) * Cin + c0;
-  constexpr int PG = kLayoutPos / V;
-  for (int i = threadIdx.x; i < cn * PG; i += 256) {
-    const int c = i / PG, pg = i % PG;
-    if (pg * V < np)
-      *reinterpret_cast<u32x4 *>(stage + c * PITCH + pg * V) = *reinterpret_cast<const u32x4 *>(src + static_cast<long>(c) * P + pg * V);
+  const long p0 = bx * kMovePos;
+  const int c0 = bz * CH, cn = min(CH, Cp - c0), np = static_cast<int>(min(static_cast<long>(kMovePos), P - p0));
+#pragma unroll
+  for (int u = 0; u < CH * PG / 256; u++) {
+    const int i = threadIdx.x + u * 256, c = i / PG, at = i % PG * V;
+    if (c >= cn) continue;
+    int from_c = c0 + c;
+    bool real = true;
+    if (unit != unit_p) {
+      const int r = from_c % unit_p;
+      real = r < unit;
+      from_c = from_c / unit_p * unit + r;
+    }
+    const U *from = x + (static_cast<long>(b) * C + from_c) * P + p0 + at;
+    if (!real) {
+      *reinterpret_cast<u32x4 *>(stage + c * PITCH + at) = u32x4{0u, 0u, 0u, 0u};
+    } else if (at + V <= np) {
+      *reinterpret_cast<u32x4 *>(stage + c * PITCH + at) = *reinterpret_cast<const piece_t *>(from);
+    } else {
+      for (int e = 0; at + e < np; e++) stage[c * PITCH + at + e] = from[e];
+    }
   }
   __syncthreads();
-  const int cg_n = cn / V;
-  for (int i = threadIdx.x; i < np * cg_n; i += 256) {
-    const int pp = i / cg_n, cg = i % cg_n;
+  const int groups = cn / V;
+  for (int i = threadIdx.x; i < np * groups; i += 256) {
+    const int p = i / groups, cg = i - p * groups;
     U out[V];
 #pragma unroll
-    for (int e = 0; e < V; e++) out[e] = stage[(cg * V + e) * PITCH + pp];
+    for (int e = 0; e < V; e++) out[e] = stage[(cg * V + e) * PITCH + p];
     u32x4 packed;
     __builtin_memcpy(&packed, out, 16);
-    *reinterpret_cast<u32x4 *>(dst + static_cast<long>(pp) * Cin + cg * V) = packed;
+    *reinterpret_cast<u32x4 *>(xt + (static_cast<long>(b) * P + p0 + p) * Cp + c0 + cg * V) = packed;
   }
 }
+
 // The 8 trilinear corners of one (tap, position), z-major order: `at[c]` = voxel index * scale + add
 // for a corner inside the volume, `outside` otherwise (also when the sample itself is void, i.e.
 // not -1 < p < size on every axis, or the lane is not live); w[c] the trilinear weight; ld/lh/lw

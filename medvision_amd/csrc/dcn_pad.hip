@@ -4,8 +4,8 @@
 // group and per group of output channels (dcn3d_mfma.hip, dcn3d_mfma_backward.hip).  Any other layer
 // (16, 24, 40, 48 ... channels, with any number of groups as long as convolution groups and
 // deformable groups nest) is run as the next larger layer that they do take: the input, the weight
-// and the output gradient are copied with zero channels added, the kernels run on the padded shapes,
-// and outputs and gradients are taken from the real channels only.  Zero inputs, zero weight rows and
+// and the output gradient get zero channels (backward: in the passes that lay them out for the kernels anyway; forward:
+// as copies), the kernels run on the padded shapes, and outputs and gradients are taken from the real channels only.  Zero inputs, zero weight rows and
 // zero weight columns add nothing to any output or gradient, so the results are those of the layer
 // itself.  The copies live in the caller's workspace; they cost one pass over the tensors, against
 // kernels that are 50 - 100 times slower without the matrix cores.
@@ -124,88 +124,6 @@ int dcn_unpad_channels(const void *src, void *dst, int B, int C, long P, int uni
     hipLaunchKernelGGL((dcn_unpad_channels_kernel<unsigned int>), grid, dim3(256), 0, stream,
                        static_cast<const unsigned int *>(src), static_cast<unsigned int *>(dst), C, P, unit, unit_p, n);
   return check_launch("dcn_unpad_channels_kernel");
-}
-
-// gx [B, C, P] (T) += the real channels of gxt [B, P, C / unit * unit_p] (fp32, channels-last);
-// 64 positions x 64 real channels per workgroup through LDS
-template <typename T>
-__global__ __launch_bounds__(256) void dcn_planar_add_padded_kernel(const float *__restrict__ gxt, T *__restrict__ gx,
-                                                                    int C, long P, int unit, int unit_p, int accumulate) {
-  __shared__ float stagef[64][65];
-  const int Cp = C / unit * unit_p;
-  const int b = blockIdx.y;
-  const long p0 = static_cast<long>(blockIdx.x) * 64;
-  const int c0 = blockIdx.z * 64, cn = min(64, C - c0);
-  const int count = static_cast<int>(min(static_cast<long>(64), P - p0)) * cn;
-  const float *src = gxt + (static_cast<long>(b) * P + p0) * Cp;
-  for (int i = threadIdx.x; i < count; i += 256) {
-    const int pp = i / cn, c = c0 + i % cn;
-    const int u = c / unit, r = c - u * unit;
-    stagef[pp][i % cn] = src[static_cast<long>(pp) * Cp + u * unit_p + r];
-  }
-  __syncthreads();
-  const int lp = threadIdx.x % 64;
-  if (p0 + lp < P)
-    for (int c = threadIdx.x / 64; c < cn; c += 4) {
-      T *d = gx + (static_cast<long>(b) * C + c0 + c) * P + p0 + lp;
-      *d = store_cast<T>(accumulate ? load(d) + stagef[lp][c] : stagef[lp][c]);
-    }
-}
-
-int dcn_planar_add_padded(const float *gxt, void *gx, const DcnDims &s, const DcnPad &pad, int dtype, bool accumulate, hipStream_t stream) {
-  const long pblocks = (s.P + 63) / 64;
-  MV_REQUIRE(pblocks < (1L << 31) && s.B <= 65535 && (s.Cin + 63) / 64 <= 65535, "volume too large");
-  const dim3 grid(static_cast<unsigned>(pblocks), s.B, (s.Cin + 63) / 64);
-  if (dtype == MV_F16)
-    hipLaunchKernelGGL((dcn_planar_add_padded_kernel<__half>), grid, dim3(256), 0, stream, gxt, static_cast<__half *>(gx),
-                       s.Cin, s.P, pad.unit, pad.unit_p, accumulate ? 1 : 0);
-  else if (dtype == MV_F32)
-    hipLaunchKernelGGL((dcn_planar_add_padded_kernel<float>), grid, dim3(256), 0, stream, gxt, static_cast<float *>(gx),
-                       s.Cin, s.P, pad.unit, pad.unit_p, accumulate ? 1 : 0);
-  else
-    hipLaunchKernelGGL((dcn_planar_add_padded_kernel<__hip_bfloat16>), grid, dim3(256), 0, stream, gxt,
-                       static_cast<__hip_bfloat16 *>(gx), s.Cin, s.P, pad.unit, pad.unit_p, accumulate ? 1 : 0);
-  return check_launch("dcn_planar_add_padded_kernel");
-}
-
-// grad_weight [Cout][cpg][K] (T) += the real entries of the tap-major fp32 accumulator
-// [K][Cout_p][cpg_p] of the padded layer; grad_bias [Cout] += the real entries of gb [Cout_p]
-template <typename T>
-__global__ __launch_bounds__(256) void dcn_weight_add_padded_kernel(const float *__restrict__ acc, T *__restrict__ gw,
-                                                                    const float *__restrict__ gb_acc, T *__restrict__ gb,
-                                                                    const DcnDims s, const DcnDims p, int unit, int unit_p, int accumulate) {
-  const long n = static_cast<long>(s.Cout) * s.cpg * s.K;
-  for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += gridDim.x * 256L) {
-    const int k = static_cast<int>(i % s.K);
-    const long oc = i / s.K;
-    const int cl = static_cast<int>(oc % s.cpg), o = static_cast<int>(oc / s.cpg);
-    const int g = o / s.opg, ol = o - g * s.opg;
-    const int u = cl / unit, r = cl - u * unit;
-    const float v = acc[(static_cast<long>(k) * p.Cout + g * p.opg + ol) * p.cpg + u * unit_p + r];
-    gw[i] = store_cast<T>(accumulate ? load(gw + i) + v : v);
-  }
-  if (gb != nullptr)
-    for (long o = blockIdx.x * 256L + threadIdx.x; o < s.Cout; o += gridDim.x * 256L) {
-      const int g = static_cast<int>(o) / s.opg, ol = static_cast<int>(o) - g * s.opg;
-      gb[o] = store_cast<T>((accumulate ? load(gb + o) : 0.f) + gb_acc[g * p.opg + ol]);
-    }
-}
-
-int dcn_weight_add_padded(const float *acc, void *gw, const float *gb_acc, void *gb, const DcnDims &s,
-                          const DcnPad &pad, int dtype, bool accumulate, hipStream_t stream) {
-  const long n = static_cast<long>(s.Cout) * s.cpg * s.K;
-  const dim3 grid(static_cast<unsigned>(std::min<long>((n + 255) / 256, 4096L)));
-  if (dtype == MV_F16)
-    hipLaunchKernelGGL((dcn_weight_add_padded_kernel<__half>), grid, dim3(256), 0, stream, acc, static_cast<__half *>(gw),
-                       gb_acc, static_cast<__half *>(gb), s, pad.p, pad.unit, pad.unit_p, accumulate ? 1 : 0);
-  else if (dtype == MV_F32)
-    hipLaunchKernelGGL((dcn_weight_add_padded_kernel<float>), grid, dim3(256), 0, stream, acc, static_cast<float *>(gw),
-                       gb_acc, static_cast<float *>(gb), s, pad.p, pad.unit, pad.unit_p, accumulate ? 1 : 0);
-  else
-    hipLaunchKernelGGL((dcn_weight_add_padded_kernel<__hip_bfloat16>), grid, dim3(256), 0, stream, acc,
-                       static_cast<__hip_bfloat16 *>(gw), gb_acc, static_cast<__hip_bfloat16 *>(gb), s, pad.p, pad.unit,
-                       pad.unit_p, accumulate ? 1 : 0);
-  return check_launch("dcn_weight_add_padded_kernel");
 }
 
 }  // namespace mv

@@ -21,9 +21,5 @@ int dcn_pad_channels(const void *src, void *dst, int B, int C, long P, int unit,
 int dcn_unpad_channels(const void *src, void *dst, int B, int C, long P, int unit, int unit_p, int es, hipStream_t stream);
 // weight [Cout, cpg, K] -> [Cout_p, cpg_p, K]
 int dcn_pad_weight(const void *src, void *dst, const DcnDims &s, const DcnPad &pad, int es, hipStream_t stream);
-// the matrix-core backward's fp32 accumulators of the padded layer, folded into the real gradients
-int dcn_planar_add_padded(const float *gxt, void *gx, const DcnDims &s, const DcnPad &pad, int dtype, bool accumulate, hipStream_t stream);
-int dcn_weight_add_padded(const float *acc, void *gw, const float *gb_acc, void *gb, const DcnDims &s,
-                          const DcnPad &pad, int dtype, bool accumulate, hipStream_t stream);
 
 }  // namespace mv

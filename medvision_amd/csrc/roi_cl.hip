@@ -20,7 +20,7 @@
 namespace mv {
 
 // [B, C, P] -> [B, P, C] for elements of 2 or 4 bytes (dcn3d_mfma.hip)
-int dcn_channels_last(const void *x, void *xt, int B, int C, long P, int elem_bytes, hipStream_t stream);
+int channels_last(const void *x, void *xt, int B, int C, long P, int elem_bytes, hipStream_t stream);
 
 constexpr int kClThreads = 256;
 
@@ -158,7 +158,7 @@ int roi_forward_cl(const void *input, const void *rois, void *output, int dtype,
   if (need == 0 || workspace == nullptr || capacity < need) return -1;
   const int es = dtype == MV_F32 ? 4 : 2, v = 16 / es;
   const long plane = static_cast<long>(p.D) * p.H * p.W;
-  const int st = dcn_channels_last(input, workspace, p.N, p.C, plane, es, s);
+  const int st = channels_last(input, workspace, p.N, p.C, plane, es, s);
   if (st) return st;
   ClShape cs;
   const int pieces = p.C / v;
