@@ -8,7 +8,7 @@
 //
 // Tap kernel (dcn_backward_tap.hip): everything but the gradient of the input, and of that the corners that
 // the scatter kernel leaves.
-// Scatter kernels (unit-stride layers whose taps fit their tile): the corners that land near their
+// Scatter kernel (dcn_backward_scatter.hip; layers whose taps fit its tile): the corners that land near their
 // position are summed per brick of positions in a fixed-point LDS tile and reach the gradient buffer as one
 // atomic per (voxel, channel) of the tile.
 #include "dcn_pad.hpp"
@@ -86,236 +86,22 @@ size_t dcn_tap_partial_bytes(const DcnDims &s, int dtype);
 bool dcn_tap_supported(const DcnDims &s, int dtype);
 int dcn_tap_backward(const void *xt, const void *off, const void *mask, const void *gyt, const void *wf,
                      float *gxt, void *goff, void *gmask, float *partial, float *gw, const DcnDims &s, const unsigned *bounds,
-                     int dtype, hipStream_t stream);
+                     const ScatterShape &shape, int dtype, hipStream_t stream);
+// dcn_backward_scatter.hip
+bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape);
+int dcn_scatter(const void *off, const void *mask, const void *gyt, const void *wf, float *gxt, const DcnDims &s,
+                const ScatterShape &shape, const unsigned *bounds, int dtype, hipStream_t stream);
+// dcn_backward_scatter.hip
+bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape);
+int dcn_scatter(const void *off, const void *mask, const void *gyt, const void *wf, float *gxt, const DcnDims &s,
+                const ScatterShape &shape, const unsigned *bounds, int dtype, hipStream_t stream);
 
-// ---- gradient of the input, local corners: summed in LDS, then added to the buffer ----------------
-// A workgroup owns a brick of positions and eight channels; its sixteen wavefronts are kScatterSplit
-// groups of eight, every group covers the positions of the brick (32 per wavefront at a time) and
-// takes a contiguous share of the taps.  gcol comes from the 16 x 16 MFMA with the channels as
-// rows: lane l holds position l % 16 of a 16-position block and the channels l / 16 and l / 16 + 4,
-// so one LDS add instruction covers 16 positions x 4 adjacent channels; a voxel's 8 sums are 9
-// qwords apart from the next voxel's to spread the banks.  After the taps the tile's non-zero sums are converted and added
-// to the gradient buffer: one global atomic per (voxel, channel) of the tile instead of one per
-// (position, tap, corner, channel).
-constexpr int kScatterSplit = 2, kScatterWaves = 8 * kScatterSplit, kScatterStride = 9;
-constexpr int kScatterKeep = 4;  // slices of grad_output a wavefront keeps in registers over the taps (all of them)
-
+// ---- layouts and folds -----------------------------------------------------------------------------
 // Element (output channel o of the padded layer p, channel cl of its group, tap k) of the real layer's weight
 template <typename T>
 __device__ __forceinline__ T padded_weight(const T *__restrict__ wt, const DcnDims &s, const DcnPad &pad, int o, int cl, int k) {
   const int g = o / pad.p.opg, ol = o - g * pad.p.opg, u = cl / pad.unit_p, r = cl - u * pad.unit_p;
   return ol < s.opg && r < pad.unit ? wt[(static_cast<long>(g * s.opg + ol) * s.cpg + u * pad.unit + r) * s.K + k] : store_cast<T>(0.f);
-}
-
-// weight [Cout, cpg, K] -> A pieces [group][tap][8-channel block][row step][lane][kPiece]: lane l
-// is MFMA row l % 16 = channel (row / 4) + 4 * (row % 2) of the block (rows 4j + 2, 4j + 3 repeat
-// rows 4j, 4j + 1 and are not used), element i the output channel g*opg + step*4*kPiece +
-// (l/16)*kPiece + i
-template <typename T>
-__device__ __forceinline__ void dcn_weight_afragments8_block(const T *__restrict__ wt, T *__restrict__ wa, const DcnDims &real, const DcnPad &pad, const unsigned bid) {
-  const DcnDims &s = pad.p;
-  constexpr int PC = Mfma<T>::kPiece;
-  const int cblocks = s.cpg / 8, steps = s.opg / (4 * PC);
-  const long total = static_cast<long>(s.groups) * s.K * cblocks * steps * 64;
-  const long id = bid * 256L + threadIdx.x;
-  if (id >= total) return;
-  const int lane = id % 64;
-  long r = id / 64;
-  const int st = r % steps; r /= steps;
-  const int cb = r % cblocks; r /= cblocks;
-  const int k = r % s.K;
-  const int g = static_cast<int>(r / s.K);
-  const int row = lane % 16, cl = cb * 8 + row / 4 + 4 * (row % 2);
-  const int o = g * s.opg + st * 4 * PC + (lane / 16) * PC;
-  for (int i = 0; i < PC; i++) wa[id * PC + i] = padded_weight(wt, real, pad, o + i, cl, k);
-}
-
-template <typename T, typename S>
-__global__ __launch_bounds__(kScatterWaves * 64) void dcn_backward_scatter_kernel(
-    const T *__restrict__ off, const T *__restrict__ mask, const T *__restrict__ gyt,
-    const T *__restrict__ wa, float *__restrict__ gxt, const DcnDims s, const int nbh, const int nbw,
-    const unsigned *__restrict__ bounds) {
-  using M = Mfma<T>;
-  using P = typename std::conditional<(sizeof(T) == 2), float, double>::type;
-  constexpr int PC = M::kPiece, SL = 4 * PC;
-  constexpr int VOX = S::TD * S::TH * S::TW;
-  constexpr int GROUPS = S::BD * S::BH * S::BW / 32;  // 32-position groups of the brick
-  static_assert(VOX <= kTileVoxMax && GROUPS % 8 == 0, "brick and tile sizes");
-  __shared__ unsigned long long tile[VOX * kScatterStride];
-  __shared__ __attribute__((aligned(16))) float recs[kScatterWaves][32][8];
-  const ScatterScale scale = scatter_scale(bounds, S::BD * S::BH * S::BW * s.K, mask != nullptr);
-  if (!scale.valid) return;  // every corner went through the data kernel
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const int n = lane % 32, p16 = lane % 16, j = lane / 16;
-  const int tg = wave / 8;
-  const unsigned brick = xcd_contiguous(blockIdx.x, gridDim.x);
-  const int bx = brick % nbw, by = (brick / nbw) % nbh, bz = brick / (nbw * nbh);
-  const int c0 = blockIdx.y * 8, b = blockIdx.z;
-  const int dgi = c0 / s.cpd, g = c0 / s.cpg, cb = (c0 - g * s.cpg) / 8;
-  const long bg = static_cast<long>(b) * s.dg + dgi;
-  const int cblocks = s.cpg / 8, steps = s.opg / SL;
-  const TileOrigin origin = tile_origin<S>(s, bz, by, bx);
-
-  for (int i = threadIdx.x; i < VOX * kScatterStride; i += kScatterWaves * 64) tile[i] = 0ull;
-  __syncthreads();
-
-  // position of brick index i, columns fastest
-  auto position = [&](int i, bool &live) {
-    const int od = bz * S::BD + i / (S::BH * S::BW), oh = by * S::BH + (i / S::BW) % S::BH, ow = bx * S::BW + i % S::BW;
-    live = od < s.Do && oh < s.Ho && ow < s.Wo;
-    return (static_cast<long>(min(od, s.Do - 1)) * s.Ho + min(oh, s.Ho - 1)) * s.Wo + min(ow, s.Wo - 1);
-  };
-  for (int pg = wave % 8; pg < GROUPS; pg += 8) {
-  // the lane's own position for the taps (both halves of the wavefront compute them)
-  bool live;
-  const long q = position(pg * 32 + n, live);
-  const int ow = q % s.Wo, oh = (q / s.Wo) % s.Ho, od = q / (static_cast<long>(s.Wo) * s.Ho);
-  const int bd = od * s.sd - s.pd, bh = oh * s.sh - s.ph, bw = ow * s.sw - s.pw;
-  // grad_output of the lane's column in the two 16-position blocks (MFMA B operand)
-  bool blive[2];
-  const T *grow[2];
-  u32x4 keep[2][kScatterKeep];
-#pragma unroll
-  for (int blk = 0; blk < 2; blk++) {
-    const long qb = position(pg * 32 + blk * 16 + p16, blive[blk]);
-    grow[blk] = gyt + (static_cast<long>(b) * s.Q + qb) * s.Cout + g * s.opg + j * PC;
-#pragma unroll
-    for (int st = 0; st < kScatterKeep; st++)
-      keep[blk][st] = (blive[blk] && st < steps) ? *reinterpret_cast<const u32x4 *>(grow[blk] + st * SL)
-                                                : u32x4{0u, 0u, 0u, 0u};
-  }
-  const int per = (s.K + kScatterSplit - 1) / kScatterSplit, k0 = min(tg * per, s.K), k1 = min(s.K, k0 + per);
-  const T *o = off + (bg * s.nd * s.K + static_cast<long>(s.nd) * k0) * s.Q + q;
-  const T *mk = mask ? mask + (bg * s.K + k0) * s.Q + q : nullptr;
-  float(*rec)[8] = recs[wave];
-
-  int ki = k0 / (s.kh * s.kw), kj = (k0 / s.kw) % s.kh, kk = k0 % s.kw;
-  P fd = P(0), fh = P(0), fw = P(0);
-  float fm = 1.f;
-  if (k0 < k1) {
-    dcn_offsets(s, o, fd, fh, fw);
-    if (mk) fm = load(mk);
-  }
-  // weight pieces of the current tap, loaded one tap ahead
-  const long tap_stride = static_cast<long>(cblocks) * steps * 64 * PC;
-  const T *afrag = wa + (((static_cast<long>(g) * s.K + k0) * cblocks + cb) * steps * 64 + lane) * PC;
-  u32x4 wcur[kScatterKeep];
-#pragma unroll
-  for (int st = 0; st < kScatterKeep; st++)
-    wcur[st] = (k0 < k1 && st < steps) ? *reinterpret_cast<const u32x4 *>(afrag + static_cast<long>(st) * (64 * PC))
-                                       : u32x4{0u, 0u, 0u, 0u};
-  for (int k = k0; k < k1; k++) {
-    u32x4 wnext[kScatterKeep];
-#pragma unroll
-    for (int st = 0; st < kScatterKeep; st++)
-      wnext[st] = (k + 1 < k1 && st < steps)
-                      ? *reinterpret_cast<const u32x4 *>(afrag + tap_stride + static_cast<long>(st) * (64 * PC))
-                      : u32x4{0u, 0u, 0u, 0u};
-    {
-      const P pd = fd + static_cast<P>(bd + ki * s.dd), ph = fh + static_cast<P>(bh + kj * s.dh),
-              pw = fw + static_cast<P>(bw + kk * s.dw);
-      const float m = fm;
-      o += s.nd * s.Q;
-      if (mk) mk += s.Q;
-      if (++kk == s.kw) { kk = 0; if (++kj == s.kh) { kj = 0; ++ki; } }
-      if (k + 1 < k1) {  // the next tap's offsets are in flight during this tap's adds
-        dcn_offsets(s, o, fd, fh, fw);
-        if (mk) fm = load(mk);
-      }
-      CornerTaps t;
-      corner_taps<P>(s, pd, ph, pw, live, 1u, 0u, ~0u, t);
-      int first;
-      unsigned bits = tile_bits<S>(origin, static_cast<int>(floor(pd)), static_cast<int>(floor(ph)),
-                                static_cast<int>(floor(pw)), first);
-      unsigned inside = 0;
-#pragma unroll
-      for (int c = 0; c < 8; c++) inside |= t.at[c] != ~0u ? 1u << c : 0u;
-      bits &= inside;
-      if (lane < 32) {
-        float4 *dst = reinterpret_cast<float4 *>(rec[n]);
-        dst[0] = make_float4(__int_as_float(first), __uint_as_float(bits), m, t.ld);
-        dst[1] = make_float4(t.lh, t.lw, 0.f, 0.f);
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-    float4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-    for (int st = 0; st < kScatterKeep; st++)
-      if (st < steps) {
-        acc[0] = M::run16(wcur[st], keep[0][st], acc[0]);
-        acc[1] = M::run16(wcur[st], keep[1][st], acc[1]);
-      }
-#pragma unroll
-    for (int blk = 0; blk < 2; blk++) {
-      const float4 *src = reinterpret_cast<const float4 *>(rec[blk * 16 + p16]);
-      const float4 ra = src[0], rb = src[1];
-      const int first = __float_as_int(ra.x);
-      const unsigned bits = __float_as_uint(ra.y);
-      // the lane's two channels, times the mask and the fixed-point scale
-      const double gv[2] = {static_cast<double>(acc[blk][0] * ra.z) * scale.up,
-                            static_cast<double>(acc[blk][1] * ra.z) * scale.up};
-      const float wd[2] = {1.f - ra.w, ra.w}, wh[2] = {1.f - rb.x, rb.x}, ww[2] = {1.f - rb.y, rb.y};
-      // the lane's qword of the first corner, as a 32-bit byte offset worked out once: the corners
-      // differ by constants that go into the instructions' offset fields
-      char *const cell0 = reinterpret_cast<char *>(tile) + (static_cast<unsigned>(first) * kScatterStride + j) * 8u;
-#pragma unroll
-      for (int c = 0; c < 8; c++) {
-        const int ca = c >> 2, cb2 = (c >> 1) & 1, ce = c & 1;
-        if ((S::TD > 1 || ca == 0) && ((bits >> c) & 1u)) {  // images have no second slice
-          const float wc = wd[ca] * wh[cb2] * ww[ce];
-          unsigned long long *dst = reinterpret_cast<unsigned long long *>(
-              cell0 + (ca * (S::TH * S::TW) + cb2 * S::TW + ce) * (kScatterStride * 8));
-#pragma unroll
-          for (int r = 0; r < 2; r++)
-            __hip_atomic_fetch_add(dst + 4 * r, fixed_term(wc, gv[r]), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-        }
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    afrag += tap_stride;
-#pragma unroll
-    for (int st = 0; st < kScatterKeep; st++) wcur[st] = wnext[st];
-  }
-  }
-  __syncthreads();
-  // ---- the tile's voxels inside the volume go to the gradient buffer, 8 channels per voxel --------
-  const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
-      gxt + static_cast<long>(b) * s.P * s.Cin, 0, static_cast<int>(s.P * s.Cin * 4), kRsrcFlags);
-  const unsigned cin4 = static_cast<unsigned>(s.Cin) * 4u;
-  const int ch = threadIdx.x % 8;
-  for (int cell = threadIdx.x / 8; cell < VOX; cell += kScatterWaves * 8) {
-    const int zw = cell % S::TW + origin.w, zh = (cell / S::TW) % S::TH + origin.h, zd = cell / (S::TW * S::TH) + origin.d;
-    const unsigned long long sum = tile[cell * kScatterStride + ch];
-    if (zd >= 0 && zd < s.D && zh >= 0 && zh < s.H && zw >= 0 && zw < s.W && sum != 0ull) {
-      const double v = static_cast<double>(static_cast<long long>(sum)) * scale.down;
-      __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(
-          static_cast<float>(v), gr,
-          static_cast<unsigned>((zd * s.H + zh) * s.W + zw) * cin4 + static_cast<unsigned>(c0 + ch) * 4u, 0, 0);
-    }
-  }
-}
-
-// ---- the same sums in 32-bit cells, for 16-bit tensors ---------------------------------------------
-// A workgroup owns a brick and SIXTEEN channels (all 16 rows of the 16 x 16 MFMA): the taps, the
-// records and grad_output serve twice the channels, an LDS add moves 4 bytes instead of 8 and a term
-// costs one fma and one subtraction.  32 bits leave 30 - ceil(log2(positions * taps)) bits for a
-// term (17 for 3 x 3 x 3 taps), so the scale comes from the data: a first sweep over the brick's
-// taps forms gcol alone (matrix cores, no geometry) and takes max |gcol| of the workgroup; every
-// term is then below max |gcol| * max |mask| < 2^ex and is rounded to a multiple of 2^(ex - shift)
-// (adding 1.5 * 2^23 in fp32 leaves round(x) in the low mantissa bits for |x| < 2^22).  The error of
-// a voxel's sum stays below terms * 2^(ex - shift - 1), about 2^-15 of the values it sums for the
-// 3 x 3 x 3 layer — a sixteenth of the last bit of the 16-bit result.
-constexpr int kScatter32Stride = 17;    // dwords between voxels: 16 channels and one to spread the banks
-constexpr int kScatter32MinShift = 14;  // fewer bits per term: the 64-bit kernel takes the layer
-__host__ __device__ constexpr int scatter32_shift(int terms) {
-  int bits = 0;
-  while ((1L << bits) < terms) bits++;
-  return 30 - bits;
 }
 
 // weight [Cout, cpg, K] -> A pieces [group][tap][16-channel block][row step][lane][kPiece]: lane l is
@@ -338,218 +124,6 @@ __device__ __forceinline__ void dcn_weight_afragments16_block(const T *__restric
   const int cl = cb * 16 + lane % 16;
   const int o = g * s.opg + st * 4 * PC + (lane / 16) * PC;
   for (int i = 0; i < PC; i++) wa[id * PC + i] = padded_weight(wt, real, pad, o + i, cl, k);
-}
-
-template <typename T, typename S>
-__global__ __launch_bounds__(kScatterWaves * 64) void dcn_backward_scatter32_kernel(
-    const T *__restrict__ off, const T *__restrict__ mask, const T *__restrict__ gyt,
-    const T *__restrict__ wa, float *__restrict__ gxt, const DcnDims s, const int nbh, const int nbw,
-    const unsigned *__restrict__ bounds) {
-  using M = Mfma<T>;
-  using P = typename std::conditional<(sizeof(T) == 2), float, double>::type;
-  constexpr int PC = M::kPiece, SL = 4 * PC;
-  constexpr int VOX = S::TD * S::TH * S::TW;
-  constexpr int GROUPS = S::BD * S::BH * S::BW / 32;  // 32-position groups of the brick
-  static_assert(VOX <= kTileVoxMax && GROUPS % 8 == 0, "brick and tile sizes");
-  __shared__ int tile[VOX * kScatter32Stride];
-  __shared__ __attribute__((aligned(8))) float recs[kScatterWaves][64][6];
-  __shared__ unsigned wgmax;
-  // (the validity of the data kernel's split: no NaN or infinity anywhere, products finite)
-  if (!scatter_scale(bounds, S::BD * S::BH * S::BW * s.K, mask != nullptr).valid) return;
-  const float mask_max = mask ? __uint_as_float(bounds[2]) : 1.f;
-  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const int n = lane % 32, p16 = lane % 16, j = lane / 16;
-  const int tg = wave / 8;
-  const unsigned brick = xcd_contiguous(blockIdx.x, gridDim.x);
-  const int bx = brick % nbw, by = (brick / nbw) % nbh, bz = brick / (nbw * nbh);
-  const int c0 = blockIdx.y * 16, b = blockIdx.z;
-  const int dgi = c0 / s.cpd, g = c0 / s.cpg, cb = (c0 - g * s.cpg) / 16;
-  const long bg = static_cast<long>(b) * s.dg + dgi;
-  const int cblocks = s.cpg / 16, steps = s.opg / SL;
-  const TileOrigin origin = tile_origin<S>(s, bz, by, bx);
-  const int per = (s.K + kScatterSplit - 1) / kScatterSplit, k0 = min(tg * per, s.K), k1 = min(s.K, k0 + per);
-  const long tap_stride = static_cast<long>(cblocks) * steps * 64 * PC;
-  const T *afrag0 = wa + (((static_cast<long>(g) * s.K + k0) * cblocks + cb) * steps * 64 + lane) * PC;
-
-  for (int i = threadIdx.x; i < VOX * kScatter32Stride; i += kScatterWaves * 64) tile[i] = 0;
-  if (threadIdx.x == 0) wgmax = 0u;
-  __syncthreads();
-
-  // position of brick index i, columns fastest
-  auto position = [&](int i, bool &live) {
-    const int od = bz * S::BD + i / (S::BH * S::BW), oh = by * S::BH + (i / S::BW) % S::BH, ow = bx * S::BW + i % S::BW;
-    live = od < s.Do && oh < s.Ho && ow < s.Wo;
-    return (static_cast<long>(min(od, s.Do - 1)) * s.Ho + min(oh, s.Ho - 1)) * s.Wo + min(ow, s.Wo - 1);
-  };
-  // grad_output of the lane's column in the two 16-position blocks of a group (MFMA B operand)
-  auto load_keep = [&](int pg, u32x4 (&keep)[2][kScatterKeep]) {
-#pragma unroll
-    for (int blk = 0; blk < 2; blk++) {
-      bool blive;
-      const long qb = position(pg * 32 + blk * 16 + p16, blive);
-      const T *grow = gyt + (static_cast<long>(b) * s.Q + qb) * s.Cout + g * s.opg + j * PC;
-#pragma unroll
-      for (int st = 0; st < kScatterKeep; st++)
-        keep[blk][st] = (blive && st < steps) ? *reinterpret_cast<const u32x4 *>(grow + st * SL) : u32x4{0u, 0u, 0u, 0u};
-    }
-  };
-  auto load_weights = [&](const T *afrag, bool on, u32x4 (&w)[kScatterKeep]) {
-#pragma unroll
-    for (int st = 0; st < kScatterKeep; st++)
-      w[st] = (on && st < steps) ? *reinterpret_cast<const u32x4 *>(afrag + static_cast<long>(st) * (64 * PC))
-                                 : u32x4{0u, 0u, 0u, 0u};
-  };
-
-  // ---- first sweep: max |gcol| over the brick's positions, the taps and the 16 channels -----------
-  {
-    float top = 0.f;
-    for (int pg = wave % 8; pg < GROUPS; pg += 8) {
-      u32x4 keep[2][kScatterKeep];
-      load_keep(pg, keep);
-      const T *afrag = afrag0;
-      for (int k = k0; k < k1; k++) {
-        u32x4 w[kScatterKeep];
-        load_weights(afrag, true, w);
-        afrag += tap_stride;
-        float4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-        for (int st = 0; st < kScatterKeep; st++)
-          if (st < steps) {
-            acc[0] = M::run16(w[st], keep[0][st], acc[0]);
-            acc[1] = M::run16(w[st], keep[1][st], acc[1]);
-          }
-#pragma unroll
-        for (int i = 0; i < 4; i++) top = fmaxf(top, fmaxf(fabsf(acc[0][i]), fabsf(acc[1][i])));
-      }
-    }
-    for (int sh = 32; sh > 0; sh >>= 1) top = fmaxf(top, __shfl_xor(top, sh));
-    if (lane == 0 && top > 0.f) atomicMax(&wgmax, __float_as_uint(top));
-  }
-  __syncthreads();
-  const float bound = fmaxf(1.001f * __uint_as_float(wgmax), 1e-30f) * mask_max;
-  if (!(bound > 0.f)) return;  // nothing but zeros to add (the whole workgroup leaves together)
-  const int shift = scatter32_shift(S::BD * S::BH * S::BW * s.K);
-  int ex = 0;
-  frexpf(bound, &ex);  // bound < 2^ex
-  const float up = ldexpf(1.f, shift - ex), down = ldexpf(1.f, ex - shift);
-  constexpr float kMagic = 12582912.f;  // 1.5 * 2^23
-
-  for (int pg = wave % 8; pg < GROUPS; pg += 8) {
-  // the taps are worked out two at a time: the lower half-wavefront takes tap k of the group's 32
-  // positions, the upper half tap k + 1
-  const int hh = lane / 32;
-  bool live;
-  const long q = position(pg * 32 + n, live);
-  const int ow = q % s.Wo, oh = (q / s.Wo) % s.Ho, od = q / (static_cast<long>(s.Wo) * s.Ho);
-  const int bd = od * s.sd - s.pd, bh = oh * s.sh - s.ph, bw = ow * s.sw - s.pw;
-  u32x4 keep[2][kScatterKeep];
-  load_keep(pg, keep);
-  int kt = k0 + hh;  // the lane's own tap
-  const T *o = off + (bg * s.nd * s.K + static_cast<long>(s.nd) * kt) * s.Q + q;
-  const T *mk = mask ? mask + (bg * s.K + kt) * s.Q + q : nullptr;
-  float(*rec)[6] = recs[wave];
-
-  int ki = kt / (s.kh * s.kw), kj = (kt / s.kw) % s.kh, kk = kt % s.kw;
-  P fd = P(0), fh = P(0), fw = P(0);
-  float fm = 1.f;
-  if (kt < k1) {
-    dcn_offsets(s, o, fd, fh, fw);
-    if (mk) fm = load(mk);
-  }
-  const T *afrag = afrag0;
-  for (int k = k0; k < k1; k += 2) {
-    // weight pieces of the two taps (the taps' geometry below hides their latency)
-    u32x4 wpair[2][kScatterKeep];
-    load_weights(afrag, true, wpair[0]);
-    load_weights(afrag + tap_stride, k + 1 < k1, wpair[1]);
-    {
-      const P pd = fd + static_cast<P>(bd + ki * s.dd), ph = fh + static_cast<P>(bh + kj * s.dh),
-              pw = fw + static_cast<P>(bw + kk * s.dw);
-      const float m = fm;
-      const bool tap_on = kt < k1;
-      kt += 2;
-      o += 2 * s.nd * s.Q;
-      if (mk) mk += 2 * s.Q;
-#pragma unroll
-      for (int u = 0; u < 2; u++)
-        if (++kk == s.kw) { kk = 0; if (++kj == s.kh) { kj = 0; ++ki; } }
-      if (kt < k1) {  // the next pair's offsets are in flight during this pair's adds
-        dcn_offsets(s, o, fd, fh, fw);
-        if (mk) fm = load(mk);
-      }
-      CornerTaps t;
-      corner_taps<P>(s, pd, ph, pw, live && tap_on, 1u, 0u, ~0u, t);
-      int first;
-      unsigned bits = tile_bits<S>(origin, static_cast<int>(floor(pd)), static_cast<int>(floor(ph)),
-                                static_cast<int>(floor(pw)), first);
-      unsigned inside = 0;
-#pragma unroll
-      for (int c = 0; c < 8; c++) inside |= t.at[c] != ~0u ? 1u << c : 0u;
-      bits &= inside;
-      float2 *dst = reinterpret_cast<float2 *>(rec[lane]);
-      dst[0] = make_float2(__int_as_float(first), __uint_as_float(bits));
-      dst[1] = make_float2(m * up, t.ld);
-      dst[2] = make_float2(t.lh, t.lw);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-      if (k + u >= k1) break;
-      float4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-      for (int st = 0; st < kScatterKeep; st++)
-        if (st < steps) {
-          acc[0] = M::run16(wpair[u][st], keep[0][st], acc[0]);
-          acc[1] = M::run16(wpair[u][st], keep[1][st], acc[1]);
-        }
-#pragma unroll
-      for (int blk = 0; blk < 2; blk++) {
-        const float2 *src = reinterpret_cast<const float2 *>(rec[u * 32 + blk * 16 + p16]);
-        const float2 ra = src[0], rb = src[1], rc = src[2];
-        const int first = __float_as_int(ra.x);
-        const unsigned bits = __float_as_uint(ra.y);
-        // the lane's four channels 4j .. 4j + 3, times the mask and the fixed-point scale
-        const float gv[4] = {acc[blk][0] * rb.x, acc[blk][1] * rb.x, acc[blk][2] * rb.x, acc[blk][3] * rb.x};
-        const float wd[2] = {1.f - rb.y, rb.y}, wh[2] = {1.f - rc.x, rc.x}, ww[2] = {1.f - rc.y, rc.y};
-        // the lane's first dword of the first corner, as a 32-bit byte offset worked out once: the
-        // corners and channels differ by constants that go into the instructions' offset fields
-        char *const cell0 = reinterpret_cast<char *>(tile) + (static_cast<unsigned>(first) * kScatter32Stride + 4 * j) * 4u;
-#pragma unroll
-        for (int c = 0; c < 8; c++) {
-          const int ca = c >> 2, cb2 = (c >> 1) & 1, ce = c & 1;
-          if ((S::TD > 1 || ca == 0) && ((bits >> c) & 1u)) {  // images have no second slice
-            const float wc = wd[ca] * wh[cb2] * ww[ce];
-            int *dst = reinterpret_cast<int *>(cell0 + (ca * (S::TH * S::TW) + cb2 * S::TW + ce) * (kScatter32Stride * 4));
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-              __hip_atomic_fetch_add(dst + r, __float_as_int(fmaf(wc, gv[r], kMagic)) - 0x4B400000, __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_WORKGROUP);
-          }
-        }
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    afrag += 2 * tap_stride;
-  }
-  }
-  __syncthreads();
-  // ---- the tile's voxels inside the volume go to the gradient buffer, 16 channels per voxel -------
-  const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
-      gxt + static_cast<long>(b) * s.P * s.Cin, 0, static_cast<int>(s.P * s.Cin * 4), kRsrcFlags);
-  const unsigned cin4 = static_cast<unsigned>(s.Cin) * 4u;
-  const int ch = threadIdx.x % 16;
-  for (int cell = threadIdx.x / 16; cell < VOX; cell += kScatterWaves * 4) {
-    const int zw = cell % S::TW + origin.w, zh = (cell / S::TW) % S::TH + origin.h, zd = cell / (S::TW * S::TH) + origin.d;
-    const int sum = tile[cell * kScatter32Stride + ch];
-    if (zd >= 0 && zd < s.D && zh >= 0 && zh < s.H && zw >= 0 && zw < s.W && sum != 0)
-      __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(
-          static_cast<float>(sum) * down, gr,
-          static_cast<unsigned>((zd * s.H + zh) * s.W + zw) * cin4 + static_cast<unsigned>(c0 + ch) * 4u, 0, 0);
-  }
 }
 
 // gxt [B, P, Cs] fp32 -> gx [B, C, P] T, added to what gx holds (`accumulate`) or in its place; 64 positions x up to
@@ -720,14 +294,14 @@ __device__ __forceinline__ void dcn_gy_sum_max_block(const T *__restrict__ gy, f
 // fragments and the zero fill of the accumulators and of the maxima's words; then the maxima and the bias sums, which need those
 // words at zero.
 struct PrepareJobs {
-  unsigned x_end, gy_end, f16_end, fsc_end, zero_end;   // block ranges of the first launch
+  unsigned x_end, gy_end, f16_end, zero_end;   // block ranges of the first launch
   unsigned px, pq;                                      // blocks of positions of the input / the output
 };
 template <typename T>
 __global__ __launch_bounds__(256) void dcn_backward_prepare_kernel(const T *__restrict__ x, T *__restrict__ xt,
                                                                    const T *__restrict__ gy, T *__restrict__ gyt,
                                                                    const T *__restrict__ wt, T *__restrict__ wb,
-                                                                   T *__restrict__ wa, float *__restrict__ zero,
+                                                                   float *__restrict__ zero,
                                                                    const long nz, const DcnDims s, const DcnPad pad, const PrepareJobs j) {
   using U = typename std::conditional<(sizeof(T) == 2), unsigned short, unsigned int>::type;
   const unsigned id = blockIdx.x;
@@ -739,10 +313,8 @@ __global__ __launch_bounds__(256) void dcn_backward_prepare_kernel(const T *__re
                       r % pb, static_cast<int>((r / pb) % s.B), static_cast<int>(r / pb / s.B));
   } else if (id < j.f16_end) {
     dcn_weight_afragments16_block<T>(wt, wb, s, pad, id - j.gy_end);
-  } else if (id < j.fsc_end) {
-    dcn_weight_afragments8_block<T>(wt, wa, s, pad, id - j.f16_end);
   } else {
-    dcn_zero_f32_block(zero, nz, id - j.fsc_end, j.zero_end - j.fsc_end);
+    dcn_zero_f32_block(zero, nz, id - j.f16_end, j.zero_end - j.f16_end);
   }
 }
 template <typename T>
@@ -761,20 +333,6 @@ __global__ __launch_bounds__(256) void dcn_backward_maxima_kernel(const T *__res
   else dcn_weight_colsum_block<T>(wt, s, bounds + 1, id - gy_blocks - mask_blocks);
 }
 
-// The LDS scatter pays when its tile holds the reach of a brick's undeformed taps with a voxel to
-// spare on either side (offsets beyond the tile still work, through the data kernel's atomics).
-template <typename S>
-static bool scatter_tile_applies(const DcnDims &s, int dtype) {
-  // the scatter kernel keeps grad_output of its positions in registers: up to kScatterKeep slices
-  // of 4 * kPiece output channels per group (128 for 16-bit tensors, 64 for fp32); wider layers
-  // would repeat too much per 8-channel workgroup and keep the atomics
-  if (s.opg > kScatterKeep * (dtype == MV_F32 ? 16 : 32)) return false;
-  const int ed = (S::BD - 1) * s.sd + (s.kd - 1) * s.dd + 1, eh = (S::BH - 1) * s.sh + (s.kh - 1) * s.dh + 1,
-            ew = (S::BW - 1) * s.sw + (s.kw - 1) * s.dw + 1;
-  return (S::TD == 1 || ed + 2 <= S::TD) && eh + 2 <= S::TH && ew + 2 <= S::TW &&
-         static_cast<long>(S::BD * S::BH * S::BW) * s.K < (1L << 20);
-}
-
 static size_t align256b(size_t v) { return (v + 255) / 256 * 256; }
 
 bool dcn_mfma_backward_supported(const DcnDims &s, int dtype) {
@@ -785,10 +343,10 @@ bool dcn_mfma_backward_supported(const DcnDims &s, int dtype) {
   return dcn_tap_supported(s, dtype);
 }
 
-// workspace: xt | gyt | weight fragments (16- and 8-channel blocks) | gxt (fp32) | gw (fp32) | gb (fp32) |
+// workspace: xt | gyt | weight fragments | gxt (fp32) | gw (fp32) | gb (fp32) |
 // the three maxima of the scatter scale (gxt .. maxima start at zero) | partial sums of the tap kernel
 struct BackwardLayout {
-  size_t xt, gyt, wb, wa, gxt, gw, gb, bounds, part, total;
+  size_t xt, gyt, wb, gxt, gw, gb, bounds, part, total;
 };
 // (the budget of an earlier design's column buffer, still stored and returned for callers that set it)
 static std::atomic<size_t> &column_budget_cell() {
@@ -807,7 +365,6 @@ static BackwardLayout backward_layout(const DcnDims &s, int dtype) {
   l.xt = at; at += align256b(static_cast<size_t>(s.B) * s.P * s.Cin * es);
   l.gyt = at; at += align256b(static_cast<size_t>(s.B) * s.Q * s.Cout * es);
   l.wb = at; at += align256b(static_cast<size_t>(s.Cout) * s.cpg * s.K * es);
-  l.wa = at; at += align256b(2 * static_cast<size_t>(s.Cout) * s.cpg * s.K * es);  // 16 MFMA rows per 8 channels
   l.gxt = at; at += align256b(static_cast<size_t>(s.B) * s.P * s.Cin * 4);
   l.gw = at; at += align256b(static_cast<size_t>(s.Cout) * s.cpg * s.K * 4);
   l.gb = at; at += align256b(static_cast<size_t>(s.Cout) * 4);
@@ -829,31 +386,25 @@ static int backward_run(const void *x, const void *off, const void *mask, const 
   T *xt = reinterpret_cast<T *>(ws + l.xt), *gyt = reinterpret_cast<T *>(ws + l.gyt), *wb = reinterpret_cast<T *>(ws + l.wb);
   float *gxt = reinterpret_cast<float *>(ws + l.gxt);
   *gx32 = gxt; *gw32 = reinterpret_cast<float *>(ws + l.gw); *gb32 = reinterpret_cast<float *>(ws + l.gb);
-  const bool image = s.nd == 2;
-  const bool tiles = image ? scatter_tile_applies<ImageBricks>(s, dtype) : scatter_tile_applies<VolumeBricks>(s, dtype);
-  // 16-bit tensors: 32-bit cells and 16 channels per workgroup, while a term keeps enough bits
-  const int terms = (image ? ImageBricks::BD * ImageBricks::BH * ImageBricks::BW
-                           : VolumeBricks::BD * VolumeBricks::BH * VolumeBricks::BW) * s.K;
-  const bool narrow = sizeof(T) == 2 && scatter32_shift(terms) >= kScatter32MinShift;
-  T *wa = narrow ? wb : reinterpret_cast<T *>(ws + l.wa);   // (16-channel blocks: those of the tap kernel)
+  ScatterShape shape{};
+  const bool tiles = dcn_scatter_plan(s, dtype, shape);
   unsigned *bounds = reinterpret_cast<unsigned *>(ws + l.bounds);
   const long frag_lanes = static_cast<long>(s.groups) * s.K * (s.cpg / 16) * (s.opg / (4 * Mfma<T>::kPiece)) * 64;
-  const long scatter_lanes = tiles && !narrow ? static_cast<long>(s.groups) * s.K * (s.cpg / 8) * (s.opg / (4 * Mfma<T>::kPiece)) * 64 : 0;
   const long nz = static_cast<long>((l.part - l.gxt) / 4);
   const long ngy = static_cast<long>(s.B) * real.Cout * s.Q, nmask = static_cast<long>(s.B) * s.dg * s.K * s.Q;
   const long ncols = static_cast<long>(s.groups) * real.cpg * s.K;
   constexpr int CH = 128 / static_cast<int>(sizeof(T));   // channels of a move
   const long px = (s.P + kMovePos - 1) / kMovePos, pq = (s.Q + kMovePos - 1) / kMovePos;
   const long nx = px * s.B * ((s.Cin + CH - 1) / CH), ngyb = pq * s.B * ((s.Cout + CH - 1) / CH);
-  const long nf16 = (frag_lanes + 255) / 256, nfsc = (scatter_lanes + 255) / 256, nzb = min((nz + 1023) / 1024, 4096L);
-  MV_REQUIRE(nx + ngyb + nf16 + nfsc + nzb < (1L << 31), "volume too large");
+  const long nf16 = (frag_lanes + 255) / 256, nzb = min((nz + 1023) / 1024, 4096L);
+  MV_REQUIRE(nx + ngyb + nf16 + nzb < (1L << 31), "volume too large");
   PrepareJobs j;
   j.x_end = static_cast<unsigned>(nx); j.gy_end = j.x_end + static_cast<unsigned>(ngyb);
-  j.f16_end = j.gy_end + static_cast<unsigned>(nf16); j.fsc_end = j.f16_end + static_cast<unsigned>(nfsc);
-  j.zero_end = j.fsc_end + static_cast<unsigned>(nzb);
+  j.f16_end = j.gy_end + static_cast<unsigned>(nf16); 
+  j.zero_end = j.f16_end + static_cast<unsigned>(nzb);
   j.px = static_cast<unsigned>(px); j.pq = static_cast<unsigned>(pq);
   hipLaunchKernelGGL((dcn_backward_prepare_kernel<T>), dim3(j.zero_end), dim3(256), 0, stream, static_cast<const T *>(x), xt,
-                     static_cast<const T *>(gy), gyt, static_cast<const T *>(wt), wb, wa, gxt, nz, real, pad, j);
+                     static_cast<const T *>(gy), gyt, static_cast<const T *>(wt), wb, gxt, nz, real, pad, j);
   if (tiles || want_bias) {
     const long slab_len = gy_slab_len(real);
     const long sum_blocks = static_cast<long>(real.Cout) * s.B * ((s.Q + slab_len - 1) / slab_len);
@@ -868,27 +419,8 @@ static int backward_run(const void *x, const void *off, const void *mask, const 
   int st = check_launch("dcn_backward_prepare_kernel");
   if (st) return st;
   st = dcn_tap_backward(xt, off, mask, gyt, wb, gxt, goff, gmask, reinterpret_cast<float *>(ws + l.part), *gw32, s,
-                        tiles ? bounds : nullptr, dtype, stream);
-  if (st || !tiles) return st;
-  MV_REQUIRE(s.Cin / 8 <= 65535, "grid too large");
-#define MV_LAUNCH_SCATTER(S)                                                                                      \
-  {                                                                                                               \
-    const long nbd = (s.Do + S::BD - 1) / S::BD, nbh = (s.Ho + S::BH - 1) / S::BH, nbw = (s.Wo + S::BW - 1) / S::BW; \
-    MV_REQUIRE(nbd * nbh * nbw < (1L << 31), "grid too large");                                                   \
-    if (narrow)                                                                                                   \
-      hipLaunchKernelGGL((dcn_backward_scatter32_kernel<T, S>),                                                   \
-                         dim3(static_cast<unsigned>(nbd * nbh * nbw), s.Cin / 16, s.B), dim3(kScatterWaves * 64), 0, \
-                         stream, static_cast<const T *>(off), static_cast<const T *>(mask), gyt, wa, gxt, s,      \
-                         static_cast<int>(nbh), static_cast<int>(nbw), bounds);                                   \
-    else                                                                                                          \
-      hipLaunchKernelGGL((dcn_backward_scatter_kernel<T, S>),                                                     \
-                         dim3(static_cast<unsigned>(nbd * nbh * nbw), s.Cin / 8, s.B), dim3(kScatterWaves * 64), 0, \
-                         stream, static_cast<const T *>(off), static_cast<const T *>(mask), gyt, wa, gxt, s,      \
-                         static_cast<int>(nbh), static_cast<int>(nbw), bounds);                                   \
-  }
-  if (image) MV_LAUNCH_SCATTER(ImageBricks) else MV_LAUNCH_SCATTER(VolumeBricks)
-#undef MV_LAUNCH_SCATTER
-  return check_launch("dcn_backward_scatter_kernel");
+                        tiles ? bounds : nullptr, shape, dtype, stream);
+  return st || !tiles ? st : dcn_scatter(off, mask, gyt, wb, gxt, s, shape, bounds, dtype, stream);
 }
 
 // Runs the kernels of the layer, padded to channel counts that they take (`pad.p`; the layer itself when it has such):

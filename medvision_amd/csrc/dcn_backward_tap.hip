@@ -68,10 +68,9 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
     const T *__restrict__ xt, const T *__restrict__ off, const T *__restrict__ mask, const T *__restrict__ gyt,
     const T *__restrict__ wf, float *__restrict__ gxt, T *__restrict__ goff, T *__restrict__ gmask,
     float *__restrict__ partial, float *__restrict__ gw, const DcnDims s, const unsigned *__restrict__ bounds,
-    const int chunks, const int shares, const int range, const int row0) {
+    const ScatterShape shape, const int chunks, const int shares, const int range, const int row0) {
   using M = Mfma<T>;
   using P = typename std::conditional<(sizeof(T) == 2), float, double>::type;  // position type
-  using S = typename std::conditional<NC == 8, VolumeBricks, ImageBricks>::type;
   constexpr int PC = M::kPiece, SL = 4 * PC, ES = sizeof(T), CW = 16 * CBW, ROWS = 64 * OBW;
   constexpr int BPI = SL / 16, ITEMS = CBW / BPI, KS = kTapTile / SL;   // 16-channel blocks per item; items; K steps of a tile
   constexpr int STEPS = ROWS / SL, STAGED = ROWS * kTapTile / PC / 256;
@@ -97,7 +96,7 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
       const_cast<T *>(xt + static_cast<long>(b) * s.P * s.Cin), 0, static_cast<int>(s.P * s.Cin * ES), kRsrcFlags);
   const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
       gxt + static_cast<long>(b) * s.P * s.Cin, 0, static_cast<int>(s.P * s.Cin * 4), kRsrcFlags);
-  const bool split = bounds && scatter_scale(bounds, S::BD * S::BH * S::BW * s.K, mask != nullptr).valid;
+  const bool split = bounds && scatter_scale(bounds, shape.terms, mask != nullptr).valid;
 
   // gcol: wavefront w forms the channels of block w % CBW for CBW blocks of sixteen positions; its rows of the weight stay
   // in registers for the whole range
@@ -156,8 +155,8 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
     }
     *reinterpret_cast<float4 *>(r + 2 * NC) = make_float4(ct.ld, ct.lh, ct.lw, fm);
     int first_cell;
-    const unsigned local = split ? tile_bits<S>(tile_origin<S>(s, od / S::BD, oh / S::BH, ow / S::BW), static_cast<int>(floor(pd)),
-                                                static_cast<int>(floor(ph)), static_cast<int>(floor(pw)), first_cell) : 0u;
+    const unsigned local = split ? tile_bits(shape, tile_origin(s, shape, od >> shape.bd, oh >> shape.bh, ow >> shape.bw),
+                                             static_cast<int>(floor(pd)), static_cast<int>(floor(ph)), static_cast<int>(floor(pw)), first_cell) : 0u;
     int listed = 0;   // (the wavefront is one tile)
 #pragma unroll
     for (int c = 0; c < NC; c++) {
@@ -385,7 +384,7 @@ bool dcn_tap_supported(const DcnDims &s, int dtype) {
 
 template <typename T, int NC, int CBW>
 static int tap_launch(const T *xt, const T *off, const T *mask, const T *gyt, const T *wf, float *gxt, T *goff,
-                      T *gmask, float *partial, float *gw, const DcnDims &s, const unsigned *bounds, int dtype,
+                      T *gmask, float *partial, float *gw, const DcnDims &s, const unsigned *bounds, const ScatterShape &shape, int dtype,
                       hipStream_t stream) {
   const int chunks = tap_chunks(s, dtype), shares = tap_shares(s, dtype);
   // Positions of a workgroup: every one adds a block of the weight gradient to memory and fills LDS with a block of the
@@ -398,7 +397,7 @@ static int tap_launch(const T *xt, const T *off, const T *mask, const T *gyt, co
   const int range = static_cast<int>(per * kTapTile);
 #define MV_TAP(OBWV, ROW)                                                                                               \
   hipLaunchKernelGGL((dcn_backward_tap_kernel<T, NC, OBWV, CBW>), grid, dim3(256), 0, stream, xt, off, mask, gyt, wf, gxt,     \
-                     goff, gmask, partial, gw, s, bounds, chunks, shares, range, ROW)
+                     goff, gmask, partial, gw, s, bounds, shape, chunks, shares, range, ROW)
   if (s.opg <= 64) {
     MV_TAP(1, 0);
   } else if (s.opg <= 128 || sizeof(T) == 4) {
@@ -417,12 +416,12 @@ static int tap_launch(const T *xt, const T *off, const T *mask, const T *gyt, co
 // `bounds` null: no scatter kernel runs, every corner of the gradient of the input is added here
 int dcn_tap_backward(const void *xt, const void *off, const void *mask, const void *gyt, const void *wf,
                      float *gxt, void *goff, void *gmask, float *partial, float *gw, const DcnDims &s, const unsigned *bounds,
-                     int dtype, hipStream_t stream) {
+                     const ScatterShape &shape, int dtype, hipStream_t stream) {
   if (tap_shares(s, dtype) == 1) partial = nullptr;
 #define MV_TAP_AS(T, NC, CBW)                                                                                          \
   tap_launch<T, NC, CBW>(static_cast<const T *>(xt), static_cast<const T *>(off), static_cast<const T *>(mask),           \
                          static_cast<const T *>(gyt), static_cast<const T *>(wf), gxt, static_cast<T *>(goff),            \
-                         static_cast<T *>(gmask), partial, gw, s, bounds, dtype, stream)
+                         static_cast<T *>(gmask), partial, gw, s, bounds, shape, dtype, stream)
   const bool wide = tap_chunk(s, dtype) == 64, image = s.nd == 2;
   if (dtype == MV_F32) return image ? MV_TAP_AS(float, 4, 2) : MV_TAP_AS(float, 8, 2);
   if (dtype == MV_F16) return wide ? MV_TAP_AS(__half, 4, 4) : image ? MV_TAP_AS(__half, 4, 2) : MV_TAP_AS(__half, 8, 2);

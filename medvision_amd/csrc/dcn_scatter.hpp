@@ -7,43 +7,40 @@ namespace mv {
 constexpr unsigned kOob = 0x80000000u;  // byte offset beyond every buffer: loads give 0, atomics are dropped
 constexpr int kRsrcFlags = 0x00020000;
 
-// ---- bricks and tiles of the LDS scatter (dcn_backward_scatter_kernel below) ----------------------
-// A brick is BD x BH x BW output positions; its tile the TD x TH x TW input voxels centred on the
+// ---- bricks and tiles of the LDS scatter (dcn_backward_scatter.hip) ---------------------------------
+// A brick is 2^bd x 2^bh x 2^bw output positions; its tile the td x th x tw input voxels centred on the
 // reach of the brick's undeformed taps.  A corner is "local" when its voxel lies in
 // the tile of its position's brick: local corners are summed in LDS by the scatter kernel, all
-// others are added to the gradient buffer by the data kernel, 128 bytes per request.
-// Volumes use 4 x 8 x 8 bricks with 10 x 14 x 14 tiles, images 32 x 32 bricks with 44 x 44 tiles (a
-// workgroup's fixed costs — clearing and flushing the tile — need more than nine taps of 256
-// positions to pay: 16 x 16 bricks gained nothing on 256-channel FPN layers).
-struct VolumeBricks { static constexpr int BD = 4, BH = 8, BW = 8, TD = 10, TH = 14, TW = 14; };
-struct ImageBricks { static constexpr int BD = 1, BH = 32, BW = 32, TD = 1, TH = 44, TW = 44; };
-constexpr int kTileVoxMax = 1960;
+// others are added to the gradient buffer by the tap kernel, 128 bytes per request.
+struct ScatterShape {
+  int bd, bh, bw, td, th, tw;
+  int nbh, nbw;   // bricks per column and row of bricks
+  int terms;      // corners that a voxel of a tile can take: positions of the brick times taps
+};
 struct TileOrigin { int d, h, w; };
-template <typename S>
-__device__ __forceinline__ TileOrigin tile_origin(const DcnDims &s, int bz, int by, int bx) {
-  TileOrigin t;
-  t.d = bz * S::BD * s.sd - s.pd - (S::TD - ((S::BD - 1) * s.sd + (s.kd - 1) * s.dd + 1)) / 2;
-  t.h = by * S::BH * s.sh - s.ph - (S::TH - ((S::BH - 1) * s.sh + (s.kh - 1) * s.dh + 1)) / 2;
-  t.w = bx * S::BW * s.sw - s.pw - (S::TW - ((S::BW - 1) * s.sw + (s.kw - 1) * s.dw + 1)) / 2;
-  return t;
+__device__ __forceinline__ TileOrigin tile_origin(const DcnDims &s, const ScatterShape &t, int bz, int by, int bx) {
+  TileOrigin o;
+  o.d = (bz << t.bd) * s.sd - s.pd - (t.td - (((1 << t.bd) - 1) * s.sd + (s.kd - 1) * s.dd + 1)) / 2;
+  o.h = (by << t.bh) * s.sh - s.ph - (t.th - (((1 << t.bh) - 1) * s.sh + (s.kh - 1) * s.dh + 1)) / 2;
+  o.w = (bx << t.bw) * s.sw - s.pw - (t.tw - (((1 << t.bw) - 1) * s.sw + (s.kw - 1) * s.dw + 1)) / 2;
+  return o;
 }
 // bit c: corner c (z-major) of the sample whose first corner is voxel (id, ih, iw) lies in the tile;
 // `first` its cell index there
-template <typename S>
-__device__ __forceinline__ unsigned tile_bits(const TileOrigin &t, int id, int ih, int iw, int &first) {
-  const int zd = id - t.d, zh = ih - t.h, zw = iw - t.w;
-  const bool fd[2] = {zd >= 0 && zd < S::TD, zd >= -1 && zd < S::TD - 1};
-  const bool fh[2] = {zh >= 0 && zh < S::TH, zh >= -1 && zh < S::TH - 1};
-  const bool fw[2] = {zw >= 0 && zw < S::TW, zw >= -1 && zw < S::TW - 1};
+__device__ __forceinline__ unsigned tile_bits(const ScatterShape &t, const TileOrigin &o, int id, int ih, int iw, int &first) {
+  const int zd = id - o.d, zh = ih - o.h, zw = iw - o.w;
+  const bool fd[2] = {zd >= 0 && zd < t.td, zd >= -1 && zd < t.td - 1};
+  const bool fh[2] = {zh >= 0 && zh < t.th, zh >= -1 && zh < t.th - 1};
+  const bool fw[2] = {zw >= 0 && zw < t.tw, zw >= -1 && zw < t.tw - 1};
   unsigned bits = 0;
 #pragma unroll
   for (int c = 0; c < 8; c++) bits |= (fd[c >> 2] && fh[(c >> 1) & 1] && fw[c & 1]) ? 1u << c : 0u;
-  first = (zd * S::TH + zh) * S::TW + zw;
+  first = (zd * t.th + zh) * t.tw + zw;
   return bits;
 }
 
-// The LDS sums are 64-bit fixed point (LDS float atomics retire one lane at a time, integer ones
-// a wavefront in a few clocks).  Every term is w * mask * gcol with 0 <= w <= 1, so
+// The LDS sums are fixed point (LDS float atomics retire one lane at a time: 0.33 lanes a clock, 64-bit integer ones
+// six to seven).  Every term is w * mask * gcol with 0 <= w <= 1, so
 //   |term| <= max|mask| * max|grad_output| * max_{c,k} sum_o |Wt[o,c,k]|  =: bound < 2^ex,
 // and a voxel takes at most one corner of each (position, tap) of the brick: positions * taps terms.
 // Terms are scaled by 2^(shift - ex), shift = min(50, 62 - ceil(log2(terms))), and rounded to
