@@ -132,7 +132,9 @@ __global__ void add_from_f32_kernel(T *dst, const float *src, long n, int accumu
 }
 int add_from_f32(void *dst, const float *src, long n, int dtype, bool accumulate, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(std::min<long>((n + 1023) / 1024, 65536)));
-  if (dtype == MV_F16)
+  if (dtype == MV_F32)
+    hipLaunchKernelGGL((add_from_f32_kernel<float>), grid, dim3(256), 0, s, static_cast<float *>(dst), src, n, accumulate ? 1 : 0);
+  else if (dtype == MV_F16)
     hipLaunchKernelGGL((add_from_f32_kernel<__half>), grid, dim3(256), 0, s, static_cast<__half *>(dst), src, n, accumulate ? 1 : 0);
   else
     hipLaunchKernelGGL((add_from_f32_kernel<__hip_bfloat16>), grid, dim3(256), 0, s, static_cast<__hip_bfloat16 *>(dst), src, n,
@@ -270,6 +272,19 @@ int roi_forward(const void *input, const void *rois, void *output, int dtype, in
   return check_launch("roi_forward_kernel");
 }
 
+// fp32 volumes whose gradient is better summed in a channels-last workspace than in its own layout: the pooled kernel is bound
+// by its global atomics, which cost by the 64-byte segment (21 G of them a second), and a voxel's sixteen channels are one
+// segment where a row of a box is one or two per channel.  The copy costs clearing and transposing it, 16 bytes of traffic
+// per element, so the rois have to touch the map: below one cell per eight voxels the map's size decides, and the sums
+// stay in the gradient.  Head training steps: [1,32,44,70,59] with 19 rois of 5^3 cells 131 -> 40 us, [4,64,41,66,72] with
+// 66 135 -> 68, [1,32,15,125,34] with 173 of 4^3 135 -> 59, [2,16,12,61,125] with 59 133 -> 55.
+static bool roi_backward_wants_sums(int dtype, const RoiProblem &p) {
+  if (dtype != MV_F32 || p.ndim != 3 || p.C < 8) return false;
+  const long cells = static_cast<long>(p.od) * p.oh * p.ow, plane = static_cast<long>(p.D) * p.H * p.W;
+  if (static_cast<double>(p.R) * cells * 8 < static_cast<double>(p.N) * plane) return false;
+  return !roi_backward_tiled_applies(dtype, p) && roi_pool_applies(dtype, p);
+}
+
 // `accumulate`: the gradient is added to what grad_input holds; otherwise it replaces it (a path that writes every voxel
 // then neither reads nor clears it; the others clear it first)
 int roi_backward(const void *grad_output, const void *rois, void *grad_input, int dtype, int ndim,
@@ -290,8 +305,9 @@ int roi_backward(const void *grad_output, const void *rois, void *grad_input, in
     return clear_gradient();
   }
   MV_REQUIRE(grad_output && rois && grad_input, "null pointer argument");
-  const bool narrow = dtype == MV_F16 || dtype == MV_BF16;
-  MV_REQUIRE(!narrow || workspace, "16-bit backward needs an fp32 workspace");
+  // (fp32: the workspace is there when the caller asked for its size, see roi_backward_wants_sums)
+  const bool narrow = dtype == MV_F16 || dtype == MV_BF16 || (workspace && roi_backward_wants_sums(dtype, p));
+  MV_REQUIRE(dtype == MV_F32 || dtype == MV_F64 || workspace, "16-bit backward needs an fp32 workspace");
   float *const ws = static_cast<float *>(workspace);
   // sums that several workgroups add to: the fp32 workspace of 16-bit tensors (folded into the gradient afterwards), the
   // gradient itself otherwise
@@ -319,7 +335,8 @@ int roi_backward(const void *grad_output, const void *rois, void *grad_input, in
   }
   st = clear_sums();
   if (st) return st;
-  // 16-bit pooled path: the fp32 workspace is used channels-last and folded in by a transposing add
+  // sums in the workspace are kept channels-last and folded in by a transposing add: a voxel's channels are then
+  // neighbours, and atomics cost by the 64 bytes
   const bool channels_last = narrow && roi_pool_applies(dtype, p);
   const int pooled = roi_pool_backward(grad_output, rois, sums, dtype, p, s, channels_last);
   if (pooled > 0) return pooled;
@@ -415,7 +432,7 @@ int mv_roi_align_2d_backward(const void *grad_output, const void *rois, void *gr
                              int sampling_ratio, int order, void *workspace, void *stream) {
   return roi_backward(grad_output, rois, grad_input, dtype, 2, 0, batch, channels, 1, height,
                       width, num_rois, 1, out_h, out_w, spatial_scale, sampling_ratio, 1, order,
-                      workspace, stream, true);
+                      dtype == MV_F32 ? nullptr : workspace, stream, true);
 }
 
 int mv_roi_align_3d_forward(const void *input, const void *rois, void *output, int dtype,
@@ -433,7 +450,7 @@ int mv_roi_align_3d_backward(const void *grad_output, const void *rois, void *gr
                              int sampling_ratio, int order, void *workspace, void *stream) {
   return roi_backward(grad_output, rois, grad_input, dtype, 3, 0, batch, channels, depth, height,
                       width, num_rois, out_d, out_h, out_w, spatial_scale, sampling_ratio, 1,
-                      order, workspace, stream, true);
+                      order, dtype == MV_F32 ? nullptr : workspace, stream, true);
 }
 
 int mv_roi_align_rotated_2d_forward(const void *input, const void *rois, void *output, int dtype,
@@ -452,7 +469,7 @@ int mv_roi_align_rotated_2d_backward(const void *grad_output, const void *rois, 
                                      void *stream) {
   return roi_backward(grad_output, rois, grad_input, dtype, 2, 1, batch, channels, 1, height,
                       width, num_rois, 1, out_h, out_w, spatial_scale, sampling_ratio, aligned,
-                      order, workspace, stream, true);
+                      order, dtype == MV_F32 ? nullptr : workspace, stream, true);
 }
 
 int mv_roi_align_rotated_3d_forward(const void *input, const void *rois, void *output, int dtype,
@@ -473,7 +490,7 @@ int mv_roi_align_rotated_3d_backward(const void *grad_output, const void *rois, 
                                      int order, void *workspace, void *stream) {
   return roi_backward(grad_output, rois, grad_input, dtype, 3, 1, batch, channels, depth, height,
                       width, num_rois, out_d, out_h, out_w, spatial_scale, sampling_ratio, aligned,
-                      order, workspace, stream, true);
+                      order, dtype == MV_F32 ? nullptr : workspace, stream, true);
 }
 
 size_t mv_roi_align_forward_workspace_bytes(int dtype, int ndim, int channels, int num_rois,
@@ -498,6 +515,18 @@ size_t mv_roi_align_forward_workspace_bytes_for_input(int dtype, int ndim, int b
   if (basic || dtype == MV_I32) return basic;   // (the tiled resampler takes the problem; label maps have no other path that wants memory)
   const size_t pooled = std::max(mv::roi_pool_forward_workspace(dtype, p), mv::roi_plane_forward_workspace(dtype, p));
   return pooled ? pooled : mv::roi_forward_cl_workspace(dtype, p);
+}
+
+size_t mv_roi_align_backward_write_workspace_bytes(int dtype, int ndim, int rotated, int batch, int channels, int depth,
+                                                   int height, int width, int num_rois, int out_d, int out_h, int out_w,
+                                                   int sampling_ratio, int order) {
+  mv::RoiProblem p{};
+  const bool flat = ndim == 2;
+  p.ndim = ndim; p.rotated = rotated; p.N = batch; p.C = channels; p.D = flat ? 1 : depth; p.H = height; p.W = width;
+  p.R = num_rois; p.od = flat ? 1 : out_d; p.oh = out_h; p.ow = out_w; p.sampling_ratio = sampling_ratio; p.order = order;
+  const bool any = batch > 0 && channels > 0 && p.D > 0 && height > 0 && width > 0 && num_rois > 0 && p.od > 0 && out_h > 0 && out_w > 0;
+  if (any && mv::roi_backward_wants_sums(dtype, p)) return sizeof(float) * static_cast<size_t>(batch) * channels * p.D * height * width;
+  return mv_roi_align_backward_workspace_bytes(dtype, batch, channels, depth, height, width);
 }
 
 size_t mv_roi_align_backward_workspace_bytes(int dtype, int batch, int channels, int depth,

@@ -1054,8 +1054,8 @@ __device__ inline void pool_backward_mfma(const T *__restrict__ src_any, float *
 }
 
 // G = element type of the accumulation buffer (T for fp32, float for 16-bit T).
-// CL: the accumulation buffer is channels-last [N, D*H*W, C] (the fp32 workspace of the 16-bit
-// path): the lanes of a wavefront then add neighbouring channels of a voxel, contiguous bytes,
+// CL: the accumulation buffer is channels-last [N, D*H*W, C] (a workspace): the lanes of a wavefront
+// then add neighbouring channels of a voxel, contiguous bytes,
 // instead of one element in each of many rows (a scattered atomic moves a whole memory sector).
 template <typename T, typename G, typename RT, bool CL, int CELLS>
 __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
@@ -1527,8 +1527,8 @@ int roi_pool_forward(const void *input, const void *rois, void *output, int dtyp
 
 bool roi_pool_applies(int dtype, const RoiProblem &p) { return pool_applies(dtype, p) && (p.C + 31) / 32 <= 65535; }
 
-// `acc` is the accumulation buffer: grad_input itself for fp32, the fp32 workspace for 16-bit
-// (channels-last [N, D*H*W, C] when `channels_last` is set; 16-bit types only).
+// `acc` is the fp32 accumulation buffer: grad_input itself (fp32 tensors) or the workspace, laid out like grad_input or
+// (`channels_last`) [N, D*H*W, C].
 int roi_pool_backward(const void *grad_output, const void *rois, void *acc, int dtype,
                       const RoiProblem &p, hipStream_t s, bool channels_last) {
   if (!pool_applies(dtype, p)) return -1;
@@ -1543,8 +1543,8 @@ int roi_pool_backward(const void *grad_output, const void *rois, void *acc, int 
          : launch_pool_backward<TYPE, CLV, 16>(grad_output, r, acc, p, cpb, grid, s))
   switch (dtype) {
     case MV_F32:
-      if (channels_last) return fail(MV_INVALID_ARGUMENT, "channels-last accumulation is for 16-bit tensors");
-      MV_POOL_BACKWARD(float, false);
+      if (channels_last) MV_POOL_BACKWARD(float, true);
+      else MV_POOL_BACKWARD(float, false);
       break;
     case MV_F16:
       if (channels_last) MV_POOL_BACKWARD(__half, true);
