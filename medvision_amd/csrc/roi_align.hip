@@ -175,6 +175,10 @@ int roi_plane_backward(const void *grad_output, const void *rois, void *grad, fl
 // roi_gather_backward.hip: atomic-free backward for resampling-sized problems; -1 when not applicable
 // roi_box.hip: backward of small outputs that the pooled kernels do not take (rotated boxes, large
 // grids), one workgroup per (roi, channel group) with LDS tiles of the source boxes; -1 when not applicable
+bool roi_own_applies(int dtype, const RoiProblem &p);
+size_t roi_own_workspace(int dtype, const RoiProblem &p);
+int roi_own_backward(const void *grad_output, const void *rois, void *grad_input, int dtype, const RoiProblem &p, void *workspace,
+                     hipStream_t s);
 int roi_box_backward(const void *grad_output, const void *rois, float *acc, int dtype, const RoiProblem &p, hipStream_t s);
 // Many small outputs over wide feature maps, read from a channels-last copy in the workspace (roi_cl.hip).
 size_t roi_forward_cl_workspace(int dtype, const RoiProblem &p);
@@ -332,6 +336,11 @@ int roi_backward(const void *grad_output, const void *rois, void *grad_input, in
     }
     st = roi_plane_backward(grad_output, rois, grad_input, static_cast<float *>(sums), dtype, p, parts, accumulate, s);
     if (st >= 0) return st || parts == 1 ? st : fold_sums();
+  }
+  // (a gradient to be added to keeps the kernel with atomics, and so does an fp32 one without a workspace)
+  if (!accumulate && workspace && !roi_pool_applies(dtype, p)) {
+    st = roi_own_backward(grad_output, rois, grad_input, dtype, p, workspace, s);
+    if (st >= 0) return st;
   }
   st = clear_sums();
   if (st) return st;
@@ -526,7 +535,9 @@ size_t mv_roi_align_backward_write_workspace_bytes(int dtype, int ndim, int rota
   p.R = num_rois; p.od = flat ? 1 : out_d; p.oh = out_h; p.ow = out_w; p.sampling_ratio = sampling_ratio; p.order = order;
   const bool any = batch > 0 && channels > 0 && p.D > 0 && height > 0 && width > 0 && num_rois > 0 && p.od > 0 && out_h > 0 && out_w > 0;
   if (any && mv::roi_backward_wants_sums(dtype, p)) return sizeof(float) * static_cast<size_t>(batch) * channels * p.D * height * width;
-  return mv_roi_align_backward_workspace_bytes(dtype, batch, channels, depth, height, width);
+  const size_t sums = mv_roi_align_backward_workspace_bytes(dtype, batch, channels, depth, height, width);
+  if (!any || mv::roi_pool_applies(dtype, p)) return sums;
+  return std::max(sums, mv::roi_own_workspace(dtype, p));
 }
 
 size_t mv_roi_align_backward_workspace_bytes(int dtype, int batch, int channels, int depth,
