@@ -4,9 +4,10 @@
 // Both passes use that the samples of a plain box are separable: a pixel's weight in a cell is wy[cell row] *
 // wx[cell column], each the sum over the cell's samples on that axis, so that with G = the 7 x 7 cells of a channel
 //     forward  G = Wy box Wx^T,        backward  box += Wy^T G Wx
-// are two small matrix products per channel each.  (A non-finite pixel or gradient reaches every cell or pixel its
-// product covers: 0 times infinity.)  They run on the fp32 matrix cores (16 x 16 x 4, exact fp32
-// products and sums).  The accumulator of the first product is the right-hand operand of the second as it stands:
+// are two small matrix products per channel each.  They run on the fp32 matrix cores (16 x 16 x 4, exact fp32
+// products and sums).  A dense product gives 0 x infinity for a pixel or gradient that no sample's weight reaches, so
+// sums that come out not finite are formed again without the terms of weight 0 (one test per finished sum; the second
+// pass runs for such channels and tiles alone).  The accumulator of the first product is the right-hand operand of the second as it stands:
 // lane l holds column l % 16 and the four rows 4 (l / 16) + r, and a product's step r takes K = one row per lane
 // group, so a suitable order of the rows (that is: of the lanes' loads) is all the second product needs - no
 // LDS, no exchange between lanes.
@@ -169,6 +170,7 @@ __global__ __launch_bounds__(1024) void roi_plane_order_kernel(const float *__re
 // ---- forward ---------------------------------------------------------------------------------------
 constexpr int kPlaneRows = 128, kPlaneGroups = 32;   // listed rows, groups of four columns
 constexpr int kPlaneAtOnce = 4, kPlaneSteps = 4;     // channels of a step, steps loaded or in flight
+constexpr int kPlaneChannels = 256;                  // of a workgroup at most
 
 template <typename T, int CELLS>
 __global__ __launch_bounds__(kPlaneThreads, 4) void roi_plane_forward_kernel(const T *__restrict__ feat,
@@ -287,6 +289,8 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void roi_plane_forward_kernel(con
     for (int c = 0; c < kPlaneAtOnce; c++) v[c] = plane_load_cells<T, 4>(rsrc, off, c * plane_bytes);
   };
   f32x4_t sum[kPlaneAtOnce], t[kPlaneAtOnce];
+  static_assert(kPlaneChannels <= 32 * kPlaneWaves * kPlaneAtOnce, "a bit for each of the wavefront's groups of channels");
+  unsigned special = 0;   // the groups whose sums are not finite
   unsigned out_off[4];   // the lane's four outputs of a channel
 #pragma unroll
   for (int r = 0; r < 4; r++)
@@ -323,6 +327,15 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void roi_plane_forward_kernel(con
     if (st.yp == 0) row_sums(st, std::true_type{});
     else row_sums(st, std::false_type{});
     if (st.yp + 1 < y_pieces) return;
+    float check = 0.f;   // stays zero unless a sum is infinite or NaN
+#pragma unroll
+    for (int c = 0; c < kPlaneAtOnce; c++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) check = fmaf(sum[c][r], 0.f, check);
+    if (__ballot(!(check == 0.f)) != 0) {
+      special |= 1u << (st.c0 / (kPlaneWaves * kPlaneAtOnce));
+      return;
+    }
     const __amdgpu_buffer_rsrc_t to = __builtin_amdgcn_make_buffer_rsrc(
         dst + static_cast<long>(st.c0) * cells, 0,
         __builtin_amdgcn_readfirstlane(min(kPlaneAtOnce, c_count - st.c0) * cells * ES), 0x00020000);
@@ -346,6 +359,23 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void roi_plane_forward_kernel(con
       issue(v[(u + kPlaneSteps - 1) % kPlaneSteps], step[(u + kPlaneSteps - 1) % kPlaneSteps]);
       if (step[u].c0 < c_count) products(v[u], step[u]);
       step[u] = next_of(step[(u + kPlaneSteps - 1) % kPlaneSteps]);
+    }
+  }
+  for (; special != 0; special &= special - 1) {   // again, output by output, without the pixels of weight 0
+    const int c0 = (__builtin_ctz(special) * kPlaneWaves + wave) * kPlaneAtOnce, outputs = min(kPlaneAtOnce, c_count - c0) * cells;
+    for (int i = lane; i < outputs; i += kWave) {
+      const int c = i / cells, r = i - c * cells, ph = r / p.ow, pw = r - ph * p.ow;
+      const T *from = src + (c0 + c) * plane;
+      float acc = 0.f;
+      for (int k = 0; k < rows; k++) {
+        if (wy[k][ph] == 0.f) continue;
+        const T *row = from + static_cast<long>(row_of[k]) * p.W;
+        float along = 0.f;
+        for (int x = 0; x < 4 * groups; x++)
+          if (wx[x][pw] != 0.f) along = fmaf(wx[x][pw], load(row + column_of[x / 4] + x % 4), along);
+        acc = fmaf(wy[k][ph], along, acc);
+      }
+      dst[c0 * cells + i] = store_cast<T>(acc);
     }
   }
 }
@@ -431,6 +461,30 @@ __global__ __launch_bounds__(kPlaneThreads, CELLS == 8 ? 4 : 2) void roi_plane_b
       for (int c = 0; c < CH; c++) acc[c] = plane_product(wy[s], t[c / PER][c % PER * STEPS + s], acc[c]);
   };
 
+  auto touches = [&](int i) {
+    if (i >= p.R || (SPLIT && i % parts != part)) return false;
+    const float *r = rois + static_cast<long>(i) * 5;
+    const float scale = static_cast<float>(p.scale);
+    const float xl = r[1] * scale, yl = r[2] * scale;
+    const float xh = fmaxf(r[3] * scale, xl + 1.f), yh = fmaxf(r[4] * scale, yl + 1.f);
+    // (a sample touches the pixels within one of it; one more for rounding.  Written so that NaN misses.)
+    return static_cast<int>(r[0]) == image && r[0] > -1.f && xh >= x0 - 2.f && xl <= x0 + kPlaneTile + 1.f && yh >= y0 - 2.f &&
+           yl <= y0 + kPlaneTile + 1.f;
+  };
+  // weights of column (axis 0) or row (axis 1) k of the tile in the cells of roi i
+  auto weigh = [&](int i, int axis, int k, float *w) {
+    const float *r = rois + static_cast<long>(i) * 5;
+    PlaneAxis A;
+    A.set(r[1 + axis], r[3 + axis], p.scale, axis == 0 ? p.ow : p.oh, p.sampling_ratio, axis == 0 ? p.W : p.H);
+    const int x = (axis == 0 ? x0 : y0) + k;
+    if (x < A.size && A.grid > 0) {
+      A.template pixel_weights<CELLS>(x, p.order, w);
+    } else {
+#pragma unroll
+      for (int c = 0; c < CELLS; c++) w[c] = 0.f;
+    }
+  };
+
   for (int base = 0; base < p.R; base += kPlaneQueue) {
     // ---- rois that touch the tile, in order, of the next kPlaneQueue ---------------------------------
     constexpr int kTests = kPlaneQueue / kPlaneThreads;
@@ -438,18 +492,7 @@ __global__ __launch_bounds__(kPlaneThreads, CELLS == 8 ? 4 : 2) void roi_plane_b
     unsigned long long hits[kTests];
 #pragma unroll
     for (int u = 0; u < kTests; u++) {
-      const int i = base + u * kPlaneThreads + tid;
-      bool hit = false;
-      if (i < p.R && (!SPLIT || i % parts == part)) {
-        const float *r = rois + static_cast<long>(i) * 5;
-        const float scale = static_cast<float>(p.scale);
-        const float xl = r[1] * scale, yl = r[2] * scale;
-        const float xh = fmaxf(r[3] * scale, xl + 1.f), yh = fmaxf(r[4] * scale, yl + 1.f);
-        // (a sample touches the pixels within one of it; one more for rounding.  Written so that NaN misses.)
-        hit = static_cast<int>(r[0]) == image && r[0] > -1.f && xh >= x0 - 2.f && xl <= x0 + kPlaneTile + 1.f &&
-              yh >= y0 - 2.f && yl <= y0 + kPlaneTile + 1.f;
-      }
-      hits[u] = __ballot(hit);
+      hits[u] = __ballot(touches(base + u * kPlaneThreads + tid));
       if (lane == 0) wave_count[u * kPlaneWaves + wave] = __popcll(hits[u]);
     }
     __syncthreads();
@@ -475,19 +518,7 @@ __global__ __launch_bounds__(kPlaneThreads, CELLS == 8 ? 4 : 2) void roi_plane_b
       {
         // weights: thread = (roi of the batch, one of the tile's 16 columns or 16 rows)
         const int bi = tid / (2 * kPlaneTile), k = tid % (2 * kPlaneTile), axis = k / kPlaneTile;
-        if (bi < batch) {
-          const float *r = rois + static_cast<long>(queue[q0 + bi]) * 5;
-          PlaneAxis A;
-          A.set(r[1 + axis], r[3 + axis], p.scale, axis == 0 ? p.ow : p.oh, p.sampling_ratio, axis == 0 ? p.W : p.H);
-          const int x = (axis == 0 ? x0 : y0) + k % kPlaneTile;
-          float *w = weights[bi][axis][k % kPlaneTile];
-          if (x < A.size && A.grid > 0) {
-            A.template pixel_weights<CELLS>(x, p.order, w);
-          } else {
-#pragma unroll
-            for (int c = 0; c < CELLS; c++) w[c] = 0.f;
-          }
-        }
+        if (bi < batch) weigh(queue[q0 + bi], axis, k % kPlaneTile, weights[bi][axis][k % kPlaneTile]);
       }
       __syncthreads();
       // The loads of the next kPlaneAhead - 1 rois are in flight while one is added.  (Loads under a condition would make
@@ -501,6 +532,45 @@ __global__ __launch_bounds__(kPlaneThreads, CELLS == 8 ? 4 : 2) void roi_plane_b
         }
       }
     }
+  }
+  __syncthreads();   // the weights are free
+  float check = 0.f;   // stays zero unless a sum is infinite or NaN
+#pragma unroll
+  for (int c = 0; c < CH; c++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) check = fmaf(acc[c][r], 0.f, check);
+  if (__ballot(!(check == 0.f)) != 0) {
+    // this wavefront's channels again, roi by roi, without the terms of weight 0
+    static_assert(kPlaneBatch >= kPlaneWaves, "a slot of weights for each wavefront");
+    float(*mine)[kPlaneTile][PITCH] = weights[wave];
+#pragma unroll
+    for (int c = 0; c < CH; c++) acc[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto wave_sync = [] {   // LDS of one wavefront is in order: only the compiler has to keep it
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    };
+    for (int i0 = 0; i0 < p.R; i0 += kWave)
+      for (unsigned long long hits = __ballot(touches(i0 + lane)); hits != 0; hits &= hits - 1) {
+        const int i = i0 + __builtin_ctzll(hits);
+        wave_sync();
+        if (lane < 2 * kPlaneTile) weigh(i, lane / kPlaneTile, lane % kPlaneTile, mine[lane / kPlaneTile][lane % kPlaneTile]);
+        wave_sync();
+        const T *g = gout + (static_cast<long>(i) * p.C + c0) * cells;
+        for (int k = 0; k < cells; k++) {
+          const int gy = k / p.ow, gx = k - gy * p.ow;
+          const float wx = mine[0][m][gx];
+#pragma unroll
+          for (int c = 0; c < CH; c++) {
+            if (c >= c_count) continue;
+            const float v = load(g + static_cast<long>(c) * cells + k);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+              const float wy = mine[1][4 * q + r][gy];
+              if (wx != 0.f && wy != 0.f) acc[c][r] = fmaf(wy, wx * v, acc[c][r]);
+            }
+          }
+        }
+      }
   }
   const int x = x0 + m;
   if (x >= p.W) return;
@@ -559,7 +629,7 @@ int roi_plane_forward(const void *input, const void *rois, void *output, int dty
     hipLaunchKernelGGL(roi_plane_order_kernel, dim3(1), dim3(1024), 0, s, static_cast<const float *>(rois), order, p, side);
   }
   // Channels per workgroup: the lists cost ~3 us, so as many channels as leave eight workgroups per compute unit.
-  int cpb = 256;
+  int cpb = kPlaneChannels;
   while (cpb > 16 && static_cast<long>(p.R) * ((p.C + cpb - 1) / cpb) < 4096) cpb /= 2;
   const long cblocks = (p.C + cpb - 1) / cpb;
   if (cblocks * p.R >= (1L << 31)) return -1;

@@ -40,3 +40,49 @@ def test_plane_heads(oracle, dtype, size, channels, rois, cells, ratio, order, r
     out.backward(gy.to(DEV))
     want = oracle.roi_align_backward(gy, boxes, feat.shape, 0.5, ratio, True, order, False)
     assert_close(x.grad, want, BWD_TOL[dtype], "backward")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("size,channels,rois,cells,ratio,order,reach", [
+    ((48, 53), 37, 30, (7, 7), 0, 1, 30),     # 8-cell kernels, a group of channels with a remainder
+    ((40, 44), 9, 24, (14, 11), 2, 1, 24),    # 16-cell kernels
+    ((40, 44), 9, 24, (5, 3), 1, 0, 24),      # nearest taps
+    ((24, 24), 16, 1100, (7, 7), 2, 1, 12),   # several workgroups per tile
+])
+def test_plane_heads_non_finite(oracle, dtype, size, channels, rois, cells, ratio, order, reach):
+    """Infinite and NaN pixels and gradients reach what a sample's weight ties them to and nothing else."""
+    from medvision_amd.ops.roi_align_nd import roi_align_2d
+    g = wl.gen(sum(size) + rois + channels)
+    feat = torch.randn(2, channels, *size, generator=g).to(dtype)
+    extent = torch.rand(rois, 2, generator=g) * reach + 1.0
+    at = torch.rand(rois, 2, generator=g) * (torch.tensor(size[::-1]) * 2.0 - extent)   # inside the image: no void samples
+    boxes = torch.cat([torch.randint(0, 2, (rois, 1), generator=g).float(), at, at + extent], 1)
+    centre, half = torch.tensor([size[1] // 2 + 0.3, size[0] // 2 + 0.2]), torch.tensor([cells[1], cells[0]]) / 2.0
+    boxes[0] = torch.cat([torch.zeros(1), 2 * (centre - half), 2 * (centre + half)])   # samples every pixel around the first one
+    bad = feat.clone()
+    bad[0, 0, size[0] // 2, size[1] // 2] = float("inf")
+    bad[1, channels - 1, size[0] // 3, size[1] - 1] = float("nan")    # the last column: its group is moved back into the row
+    x = bad.to(DEV).requires_grad_()
+    out = roi_align_2d(x, boxes.to(DEV), cells, 0.5, ratio, order)
+
+    def compare(got, want, finite, tol, name):
+        got, finite = got.detach().cpu().double(), finite.reshape(got.shape)
+        assert not finite.all() and torch.equal(torch.isfinite(got), finite), name
+        assert_close(torch.where(finite, got, 0.0), torch.where(finite, want.reshape(got.shape), 0.0), tol, name)
+
+    def pooled(x):
+        return oracle.roi_align_forward(x, boxes, cells, 0.5, ratio, True, order, False)
+
+    # (the oracle multiplies nearest neighbours that are not picked by 0: the cells reached come from marks instead)
+    marks = (~torch.isfinite(bad)).to(dtype)
+    compare(out, pooled(torch.where(marks > 0, 0.0, bad)), pooled(marks) == 0, FWD_TOL[dtype], "forward")
+    gy = torch.randn(out.shape, generator=g).to(dtype)
+    gy[0, 0].view(-1)[0] = float("inf")
+    gy[rois - 1, channels - 1].view(-1)[-1] = float("nan")
+    out.backward(gy.to(DEV))
+
+    def spread(t):
+        return oracle.roi_align_backward(t, boxes, feat.shape, 0.5, ratio, True, order, False)
+
+    marks = (~torch.isfinite(gy)).to(dtype)
+    compare(x.grad, spread(torch.where(marks > 0, 0.0, gy)), spread(marks) == 0, BWD_TOL[dtype], "backward")
