@@ -30,6 +30,13 @@ namespace {
   throw py::error_already_set();
 }
 
+// None of the operators has a forward-mode derivative: a dual tensor is refused instead of losing its tangent (it need
+// not require a gradient, so the short ways around the autograd nodes would take it).
+void no_forward_mode(const Tensor &t) {
+  if (t.defined() && t._fw_grad(/*level=*/0).defined())
+    raise(PyExc_NotImplementedError, "forward-mode AD is not implemented for this operator");
+}
+
 // (std::runtime_error becomes RuntimeError without the C++ backtrace that TORCH_CHECK appends)
 #define MVB_CHECK(cond, ...) \
   do {                       \
@@ -220,6 +227,8 @@ Tensor roi_align(int ndim, bool rotated, const Tensor &features, const Tensor &r
                  double spatial_scale, int sampling_ratio, bool aligned, int order, const std::optional<Tensor> &prepared) {
   const RoiCall c{rotated ? kRotated : kPlain, ndim, sampling_ratio, order, aligned, static_cast<float>(spatial_scale),
                   parse_size(output_size, ndim)};
+  no_forward_mode(features);
+  no_forward_mode(rois);
   const py::gil_scoped_release no_gil;
   if (!(at::GradMode::is_enabled() && (features.requires_grad() || rois.requires_grad()))) {
     const at::NoGradGuard no_grad;
@@ -408,6 +417,7 @@ Tensor modulated_deform_conv(int nd, const Tensor &input, const Tensor &offset, 
   if (!input.is_cuda()) raise(PyExc_NotImplementedError, "");
   const int s0 = nd == 3 ? stride : 1, p0 = nd == 3 ? padding : 0, d0 = nd == 3 ? dilation : 1;
   const DcnCall c{nd, groups, dg, {s0, stride, stride}, {p0, padding, padding}, {d0, dilation, dilation}};
+  for (const Tensor &t : {input, offset, mask, weight, bias.value_or(Tensor())}) no_forward_mode(t);
   const py::gil_scoped_release no_gil;
   return DeformConvFunction::apply(input, offset, mask, weight, bias, c);
 }
@@ -417,6 +427,7 @@ Tensor deform_conv(int nd, const Tensor &input, const Tensor &offset, const Tens
                    const py::object &stride, const py::object &padding, const py::object &dilation, int groups, int dg,
                    int64_t im2col_step) {
   const DcnCall c{nd, groups, dg, per_axis(stride, nd, 1), per_axis(padding, nd, 0), per_axis(dilation, nd, 1)};
+  for (const Tensor &t : {input, offset, weight, bias}) no_forward_mode(t);
   const py::gil_scoped_release no_gil;
   MVB_CHECK(input.is_cuda(), "Not implemented on the CPU");
   im2col_step_check(input.size(0), im2col_step);
