@@ -9,13 +9,13 @@
 // integer additions to LDS; afterwards the tile's non-zero sums are added to the gradient buffer, one global atomic per
 // (voxel, channel) of the tile instead of one per (position, tap, corner, channel).
 //
-// NARROW (16-bit tensors): 32-bit sums.  (Two of them per 64-bit addition: 11.3 terms a clock and compute unit
+// NARROW (dense layers of 16-bit tensors, see dcn_scatter_plan): 32-bit sums.  (Two of them per 64-bit addition: 11.3 terms a clock and compute unit
 // against 10.3, and more vector instructions to make the words: 556 us against 504 us.)  They leave 30 - ceil(log2(positions * taps)) bits for a term (17 for 3 x 3 x 3 taps), so the scale comes from the data: a
 // first sweep over the brick's taps forms gcol alone (matrix cores, no geometry) and takes max |gcol| of the workgroup;
 // every term is then below max |gcol| * max |mask| < 2^ex and is rounded to a multiple of 2^(ex - shift) (adding
 // 1.5 * 2^23 in fp32 leaves round(x) in the low mantissa bits for |x| < 2^22).  The error of a voxel's sum stays below
 // terms * 2^(ex - shift - 1), about 2^-15 of the values it sums for the 3 x 3 x 3 layer — a sixteenth of the last bit of the
-// 16-bit result.  Otherwise (fp32, or too many terms): a 64-bit word per channel, scale from the global maxima.
+// 16-bit result.  Otherwise a 64-bit word per channel, scale from the global maxima.
 //
 // What bounds it: the LDS additions (six to seven 64-bit lanes a clock and compute unit) and the 64-byte atomics of the tiles
 // (21 G a second on the whole chip).
@@ -274,20 +274,24 @@ using TileStrided = Tile<12, 12, 13>;   // 4 x 4 x 4 positions: stride 2, dilati
 using TileImage = Tile<1, 44, 44>;      // 32 x 32 positions (16 x 16 at stride 2)
 using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions, two workgroups on a compute unit
 
-static bool scatter_narrow(const DcnDims &s, const ScatterShape &shape, int dtype) {
-  return dtype != MV_F32 && scatter32_shift(shape.terms) >= kScatterMinShift;
-}
-
 // The brick and its tile: the first of the list whose tile holds the reach of the brick's undeformed taps with two voxels to spare
 // on either side, or one, if none has two.  Images with fewer workgroups than compute units take a smaller brick (77 us ->
 // 35 us for [1, 256 -> 128, 27 x 58]); volumes do not (the halo of 4 x 4 x 4 positions is most of their tile: 117 us
 // against 78 us for [2, 16 -> 128, 7 x 19 x 32]).  False: no brick fits.
+//
+// Width of the sums: 32 bits round every term to 14 - 22 bits of the workgroup's largest, which is worth their speed in dense
+// layers alone (16-bit tensors, the first brick fits: unit strides, taps close together; up to 128 output channels).  bf16 training
+// step of [2, 32 -> 64, 48^3]: 1178 us, 1393 us with 64-bit sums.  Strided and wide layers have 64-bit sums, as good as fp32 ones:
+// where the output's gradient is 2^-14 of what it is elsewhere in the brick, 32 bits left them 2 - 20 % off.  Training steps, 32
+// against 64 bits: [8, 256 -> 256, 100 x 152] fp16 2315 / 2337 us; stride 2, [8, 128 -> 128, 100 x 152] 332 / 370 us and
+// [2, 32 -> 64, 48^3] 297 / 345 us.
 bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
   static const int volumes[2][6] = {{2, 3, 3, 10, 14, 14}, {2, 2, 2, 12, 12, 13}};
   static const int images[4][6] = {{0, 5, 5, 1, 44, 44}, {0, 4, 4, 1, 28, 28}, {0, 4, 4, 1, 44, 44}, {0, 3, 3, 1, 28, 28}};
   const bool image = s.nd == 2;
   const int st[3] = {s.sd, s.sh, s.sw}, kn[3] = {s.kd, s.kh, s.kw}, dl[3] = {s.dd, s.dh, s.dw}, on[3] = {s.Do, s.Ho, s.Wo};
   int best = -1;
+  bool dense = false;
   for (int i = 0; i < (image ? 4 : 2); i++) {
     const int *e = image ? images[i] : volumes[i];
     long spare = 1 << 20, bricks = s.B;
@@ -297,12 +301,14 @@ bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
       bricks *= (on[a] + (1 << e[a]) - 1) >> e[a];
     }
     if (spare < 2 || (1L << (e[0] + e[1] + e[2])) * s.K >= (1L << 20)) continue;
+    dense = dense || i == 0;
     const int rank = (spare >= 4 ? 2 : 0) + (image && bricks * (s.Cin / (dtype == MV_F32 ? 8 : 16)) >= 256 ? 1 : 0);
     if (rank <= best) continue;
     best = rank;
-    shape = ScatterShape{e[0], e[1], e[2], e[3], e[4], e[5], 0, 0, (1 << (e[0] + e[1] + e[2])) * s.K};
+    shape = ScatterShape{e[0], e[1], e[2], e[3], e[4], e[5], 0, 0, (1 << (e[0] + e[1] + e[2])) * s.K, 0};
   }
   if (best < 0 || s.Cin / 8 > 65535) return false;
+  shape.narrow = dense && dtype != MV_F32 && s.opg <= 128 && scatter32_shift(shape.terms) >= kScatterMinShift;
   shape.nbh = (s.Ho + (1 << shape.bh) - 1) >> shape.bh;
   shape.nbw = (s.Wo + (1 << shape.bw) - 1) >> shape.bw;
   return static_cast<long>(shape.nbh) * shape.nbw * ((s.Do + (1 << shape.bd) - 1) >> shape.bd) < (1L << 31);
@@ -310,16 +316,16 @@ bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
 
 template <typename T, typename S>
 static int scatter_launch(const void *off, const void *mask, const void *gyt, const void *wf, float *gxt, const DcnDims &s,
-                          const ScatterShape &shape, const unsigned *bounds, bool narrow, hipStream_t stream) {
+                          const ScatterShape &shape, const unsigned *bounds, hipStream_t stream) {
   const int nbd = (s.Do + (1 << shape.bd) - 1) >> shape.bd;
   const bool wide = s.opg > 4 * 64 / static_cast<int>(sizeof(T));
-  const dim3 grid(static_cast<unsigned>(nbd) * shape.nbh * shape.nbw, s.Cin / (narrow ? 16 : 8), s.B);
+  const dim3 grid(static_cast<unsigned>(nbd) * shape.nbh * shape.nbw, s.Cin / (shape.narrow ? 16 : 8), s.B);
 #define MV_SCATTER(NARROWV, KEEPV)                                                                                    \
   hipLaunchKernelGGL((dcn_backward_scatter_kernel<T, NARROWV, S, KEEPV>), grid, dim3(KEEPV == 4 ? 1024 : 512), 0, stream,     \
                      static_cast<const T *>(off), static_cast<const T *>(mask), static_cast<const T *>(gyt),          \
                      static_cast<const T *>(wf), gxt, s, shape, bounds)
-  if (narrow) {
-    if constexpr (sizeof(T) == 2) { if (wide) MV_SCATTER(true, 8); else MV_SCATTER(true, 4); }
+  if (shape.narrow) {
+    if constexpr (sizeof(T) == 2) MV_SCATTER(true, 4);   // (never wide)
   } else {
     if (wide) MV_SCATTER(false, 8); else MV_SCATTER(false, 4);
   }
@@ -329,8 +335,7 @@ static int scatter_launch(const void *off, const void *mask, const void *gyt, co
 
 int dcn_scatter(const void *off, const void *mask, const void *gyt, const void *wf, float *gxt, const DcnDims &s,
                 const ScatterShape &shape, const unsigned *bounds, int dtype, hipStream_t stream) {
-  const bool narrow = scatter_narrow(s, shape, dtype);
-#define MV_SCATTER_TILE(T, S) scatter_launch<T, S>(off, mask, gyt, wf, gxt, s, shape, bounds, narrow, stream)
+#define MV_SCATTER_TILE(T, S) scatter_launch<T, S>(off, mask, gyt, wf, gxt, s, shape, bounds, stream)
 #define MV_SCATTER_AS(T)                                                                                              \
   (shape.th == TileVolume::TH ? MV_SCATTER_TILE(T, TileVolume)                                                          \
    : shape.th == TileStrided::TH ? MV_SCATTER_TILE(T, TileStrided)                                                      \

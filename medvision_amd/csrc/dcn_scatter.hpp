@@ -16,6 +16,7 @@ struct ScatterShape {
   int bd, bh, bw, td, th, tw;
   int nbh, nbw;   // bricks per column and row of bricks
   int terms;      // corners that a voxel of a tile can take: positions of the brick times taps
+  int narrow;     // 32-bit sums instead of 64-bit ones (dcn_scatter_plan)
 };
 struct TileOrigin { int d, h, w; };
 __device__ __forceinline__ TileOrigin tile_origin(const DcnDims &s, const ScatterShape &t, int bz, int by, int bx) {

@@ -39,3 +39,37 @@ def test_matrix_core_layers(oracle, dtype, cin, cout, size, stride, groups, dg):
     want = oracle.dcn3d_backward(x, off, mask, w, gy, True, stride, 1, 1, groups, dg)
     for t, v, name in zip(leaves, want, ("input", "offset", "mask", "weight", "bias")):
         assert_close(t.grad, v, BWD_TOL[dtype], name)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("cin,cout,size,stride,dilation", [
+    (32, 256, (40, 72), 1, 1),        # images with more output channels than 128
+    (32, 64, (44, 80), 2, 1),         # strided
+    (32, 64, (48, 72), 1, 12),        # taps far apart
+    (32, 64, (6, 20, 48), 2, 1),      # volumes, strided
+    (32, 160, (5, 9, 48), 1, 1),
+])
+def test_small_gradients_beside_large_ones(oracle, dtype, cin, cout, size, stride, dilation):
+    """The gradient of the input keeps fp32 sums in strided and wide layers: where the output's gradient is 2^-14 of what it
+    is a few columns further on, in the same brick, the sums are as good as anywhere (rounding of the result: 2^-11 / 2^-8)."""
+    if len(size) == 3:
+        from medvision_amd.ops.modulated_deform_conv_3d import modulated_deform_conv
+    else:
+        from medvision_amd.ops.modulated_deform_conv_2d import modulated_deform_conv
+    g = wl.gen(cin + cout + sum(size))
+    x, off, mask, w, b = wl.dcn_inputs(g, 1, cin, cout, size, 3, 1, 1, dtype, stride, dilation, dilation, offset_std=0.0)
+    off = (torch.rand(off.shape, generator=g) - 0.5).to(dtype)
+    leaves = [t.to(DEV).requires_grad_(True) for t in (x, off, mask, w, b)]
+    y = modulated_deform_conv(*leaves, stride, dilation, dilation, 1, 1)
+    gy = torch.randn(y.shape, generator=g)
+    split = y.shape[-1] // 2 + 1
+    gy[..., :split] *= 2.0 ** -6
+    gy[..., split:] *= 2.0 ** 8
+    gy = gy.to(dtype)
+    y.backward(gy.to(DEV))
+    want = oracle.dcn3d_backward(x, off, mask, w, gy, True, stride, dilation, dilation, 1, 1)[0].reshape(x.shape)
+    edge = split * stride - 2 - dilation       # columns that no position beyond the split reaches
+    got, want = leaves[0].grad.cpu().double()[..., :edge], want[..., :edge]
+    assert float(want.abs().max()) < 1.0       # nothing of the large ones
+    error = float((got - want).norm() / want.norm())
+    assert error < (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8), error
