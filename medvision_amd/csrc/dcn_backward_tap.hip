@@ -10,18 +10,21 @@
 //   1  gcol = Wt_k^T gy (16 x 16 MFMA, rows = channels), through LDS to the load layout (position l / 4, 16-byte piece
 //      l % 4: a voxel's pieces are one cache look-up);
 //   2  every wavefront samples 16 positions: the corners' pieces are loaded once and used twice, blended into the column
-//      value and multiplied with gcol into one sum per corner, D_c = sum over channels of gcol * x_c.  The trilinear form is
-//      linear in the corners, so value and derivatives come from the eight D once per position instead of from
-//      eight x once per channel (16-bit tensors; fp32 forms the differences per channel, which is kinder to sums of
-//      nearly equal corners);
+//      value and differenced against gcol.  The trilinear form is blended axis by axis, which passes the differences that
+//      its derivatives are made of: along w four per channel (images: two), along h two (one), along d one.  Sums over the channels
+//      are taken of these differences, and the blends over the axes that are left are done once per position.  (One sum per
+//      corner, differenced at the end, is 16 instead of 23 vector instructions per channel, images 8 instead of 11, and loses the
+//      digits that nearly equal corners share: 4e-5 of sum |gcol * step| on an input of 64 and 64 + one step of fp16.  That
+//      form took 496 us against 493 us for bf16 [2, 32 -> 64, 48^3], 728 us against 762 us for fp16 images
+//      [8, 256 -> 256, 100 x 152].);
 //   3  gw_k += gy col_k^T, a quarter of the output channels per wavefront, both operands by transposing LDS reads.
 // Corners that the LDS scatter does not take are listed when the records are made, and their 32 channels are added as
 // 128 contiguous bytes.
-// What bounds it: narrow layers the vector instructions of the samples (128 multiply-adds and as many more for everything
-// else per 16 positions and 32 channels), wide ones the matrix cores and LDS, and everywhere the atomics of the far
+// What bounds it: narrow layers the vector instructions of the samples (184 per 16 positions and 32 channels, and as many more
+// for everything else) and the latency of the gathers, wide ones the matrix cores and LDS, and everywhere the atomics of the far
 // corners (64 bytes per corner and 16 channels, 21 G of them a second at best).
-//   (bf16 [2, 32 -> 64, 48^3]: 343 us without the far corners; the data and weight kernels before it took 670 us.  fp16
-//   images [8, 256 -> 256, 100 x 152]: 694 us, 4380 us before.  [1, 128 -> 128, 7 x 45 x 18]: 64 us, 790 us before.)
+//   (bf16 [2, 32 -> 64, 48^3]: 493 us; the data and weight kernels before it took 670 us.  fp16 images
+//   [8, 256 -> 256, 100 x 152]: 762 us, 4380 us before.  [1, 128 -> 128, 7 x 45 x 18]: 64 us, 790 us before.)
 #include "dcn_scatter.hpp"
 
 namespace mv {
@@ -74,8 +77,8 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
   constexpr int PC = M::kPiece, SL = 4 * PC, ES = sizeof(T), CW = 16 * CBW, ROWS = 64 * OBW;
   constexpr int BPI = SL / 16, ITEMS = CBW / BPI, KS = kTapTile / SL;   // 16-channel blocks per item; items; K steps of a tile
   constexpr int STEPS = ROWS / SL, STAGED = ROWS * kTapTile / PC / 256;
-  constexpr int RW = 2 * NC + 4, kRecs = 2 * kTapTile, GP = CW + 4;
-  __shared__ __attribute__((aligned(16))) unsigned rec[kRecs][RW];          // at[NC], mask * w[NC], ld, lh, lw, mask
+  constexpr int RW = 12, kRecs = 2 * kTapTile, GP = CW + 4;
+  __shared__ __attribute__((aligned(16))) unsigned rec[kRecs][RW];          // at[NC], ld, lh, lw, mask (12 words: sixteen rows on different banks)
   __shared__ u32x4 gyl[ROWS / PC * kTapPitch];                               // grad_output, pieces of output channels
   __shared__ u32x4 col[CW / PC * kTapPitch];                                 // column values, pieces of input channels
   __shared__ __attribute__((aligned(16))) float gcol[kTapTile][GP];
@@ -149,11 +152,8 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
     corner_taps<P>(s, pd, ph, pw, live, static_cast<unsigned>(s.Cin) * ES, 0u, kOob, ct);
     unsigned *r = rec[tid];
 #pragma unroll
-    for (int c = 0; c < NC; c += 4) {
-      *reinterpret_cast<u32x4 *>(r + c) = u32x4{ct.at[c], ct.at[c + 1], ct.at[c + 2], ct.at[c + 3]};
-      *reinterpret_cast<float4 *>(r + NC + c) = make_float4(fm * ct.w[c], fm * ct.w[c + 1], fm * ct.w[c + 2], fm * ct.w[c + 3]);
-    }
-    *reinterpret_cast<float4 *>(r + 2 * NC) = make_float4(ct.ld, ct.lh, ct.lw, fm);
+    for (int c = 0; c < NC; c += 4) *reinterpret_cast<u32x4 *>(r + c) = u32x4{ct.at[c], ct.at[c + 1], ct.at[c + 2], ct.at[c + 3]};
+    *reinterpret_cast<float4 *>(r + NC) = make_float4(ct.ld, ct.lh, ct.lw, fm);
     int first_cell;
     const unsigned local = split ? tile_bits(shape, tile_origin(s, shape, od >> shape.bd, oh >> shape.bh, ow >> shape.bw),
                                              static_cast<int>(floor(pd)), static_cast<int>(floor(ph)), static_cast<int>(floor(pw)), first_cell) : 0u;
@@ -204,15 +204,12 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
     const int p = wave * 16 + lj;
     const unsigned *r = rec[half * kTapTile + p];
     unsigned at[NC];
-    float cw[NC];
 #pragma unroll
     for (int c = 0; c < NC; c += 4) {
       const u32x4 a = *reinterpret_cast<const u32x4 *>(r + c);
-      const float4 w = *reinterpret_cast<const float4 *>(r + NC + c);
       at[c] = a.x + lk * 16u; at[c + 1] = a.y + lk * 16u; at[c + 2] = a.z + lk * 16u; at[c + 3] = a.w + lk * 16u;
-      cw[c] = w.x; cw[c + 1] = w.y; cw[c + 2] = w.z; cw[c + 3] = w.w;
     }
-    const float4 e = *reinterpret_cast<const float4 *>(r + 2 * NC);   // ld, lh, lw, mask
+    const float4 e = *reinterpret_cast<const float4 *>(r + NC);   // ld, lh, lw, mask
     constexpr int SETS = NC == 4 && ITEMS > 1 ? 2 : 1;   // items whose corners are in registers (volumes: one, for occupancy)
     u32x4 raw[SETS][NC];
     auto gather = [&](u32x4 (&to)[NC], int item) {
@@ -234,9 +231,12 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
         *reinterpret_cast<float4 *>(&gcol[(wfirst + n) * 16 + j][wblock * 16 + 4 * kc]) = make_float4(gc[n][0], gc[n][1], gc[n][2], gc[n][3]);
     }
     __syncthreads();   // gcol is complete
-    float D[NC], t0 = 0.f, t1 = 0.f, t2 = 0.f, t3 = 0.f;
+    // sums over the lane's channels: differences along w (along h, d), value
+    float sw[NC / 2], sh[NC / 4], sd = 0.f, sv = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; c++) D[c] = 0.f;
+    for (int c = 0; c < NC / 2; c++) sw[c] = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC / 4; c++) sh[c] = 0.f;
 #pragma unroll
     for (int item = 0; item < ITEMS; item++) {
       if (SETS == 2 && item + 1 < ITEMS) gather(raw[(item + 1) % SETS], item + 1);
@@ -248,47 +248,37 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
         gv[i] = t.x; gv[i + 1] = t.y; gv[i + 2] = t.z; gv[i + 3] = t.w;
       }
 #pragma unroll
-      for (int i = 0; i < PC; i++) v[i] = 0.f;
+      for (int i = 0; i < PC; i++) {
+        float row[NC / 2], plane[NC / 4];   // blended along w; along w and h
 #pragma unroll
-      for (int c = 0; c < NC; c++) {
-        M::fma_piece(v, cw[c], x[c]);
-        if constexpr (ES == 2) D[c] = M::dot_piece(gv, x[c], D[c]);
-      }
-      if constexpr (ES == 4) {
-#pragma unroll
-        for (int i = 0; i < PC; i++) {
-          float u[8];
-#pragma unroll
-          for (int c = 0; c < 8; c++) u[c] = c < NC ? __uint_as_float(x[c < NC ? c : 0][i]) : 0.f;
-          const float x0 = u[1] - u[0], x1 = u[3] - u[2], a0 = fmaf(e.z, x0, u[0]), a1 = fmaf(e.z, x1, u[2]);
-          const float b0 = fmaf(e.y, x1 - x0, x0), y0 = a1 - a0, v0 = fmaf(e.y, y0, a0);
-          float dw = b0, dh = y0, dd = 0.f, val = v0;
-          if constexpr (NC == 8) {
-            const float x2 = u[5] - u[4], x3 = u[7] - u[6], a2 = fmaf(e.z, x2, u[4]), a3 = fmaf(e.z, x3, u[6]);
-            const float b1 = fmaf(e.y, x3 - x2, x2), y1 = a3 - a2, v1 = fmaf(e.y, y1, a2);
-            dw = fmaf(e.x, b1 - b0, b0);
-            dh = fmaf(e.x, y1 - y0, y0);
-            dd = v1 - v0;
-            val = fmaf(e.x, dd, v0);
-          }
-          t0 = fmaf(dd, gv[i], t0); t1 = fmaf(dh, gv[i], t1); t2 = fmaf(dw, gv[i], t2); t3 = fmaf(val, gv[i], t3);
+        for (int c = 0; c < NC / 2; c++) {
+          const float first = M::element(x[2 * c], i), step = M::element(x[2 * c + 1], i) - first;
+          sw[c] = fmaf(step, gv[i], sw[c]);
+          row[c] = fmaf(e.z, step, first);
         }
+#pragma unroll
+        for (int c = 0; c < NC / 4; c++) {
+          const float step = row[2 * c + 1] - row[2 * c];
+          sh[c] = fmaf(step, gv[i], sh[c]);
+          plane[c] = fmaf(e.y, step, row[2 * c]);
+        }
+        float value = plane[0];
+        if constexpr (NC == 8) {
+          const float step = plane[1] - plane[0];
+          sd = fmaf(step, gv[i], sd);
+          value = fmaf(e.x, step, plane[0]);
+        }
+        sv = fmaf(value, gv[i], sv);
+        v[i] = e.w * value;
       }
       col[tap_slot(item * 4 + lk, p)] = M::pack(v);
       if (SETS == 1 && item + 1 < ITEMS) gather(raw[0], item + 1);
     }
-    if constexpr (ES == 2) {
-      const float x0 = D[1] - D[0], x1 = D[3] - D[2], a0 = fmaf(e.z, x0, D[0]), a1 = fmaf(e.z, x1, D[2]);
-      const float b0 = fmaf(e.y, x1 - x0, x0), y0 = a1 - a0, v0 = fmaf(e.y, y0, a0);
-      t2 = b0; t1 = y0; t3 = v0;
-      if constexpr (NC == 8) {
-        const float x2 = D[5] - D[4], x3 = D[7] - D[6], a2 = fmaf(e.z, x2, D[4]), a3 = fmaf(e.z, x3, D[6]);
-        const float b1 = fmaf(e.y, x3 - x2, x2), y1 = a3 - a2, v1 = fmaf(e.y, y1, a2);
-        t2 = fmaf(e.x, b1 - b0, b0);
-        t1 = fmaf(e.x, y1 - y0, y0);
-        t0 = v1 - v0;
-        t3 = fmaf(e.x, t0, v0);
-      }
+    const auto mix = [](float f, float a, float b) { return fmaf(f, b - a, a); };
+    float t0 = sd, t1 = sh[0], t2 = mix(e.y, sw[0], sw[1]), t3 = sv;
+    if constexpr (NC == 8) {
+      t1 = mix(e.x, sh[0], sh[1]);
+      t2 = mix(e.x, t2, mix(e.y, sw[2], sw[3]));
     }
     // the four pieces of a position: lane l % 4 ends with the sum of component l % 4
 #define MV_QUAD(v, ctrl) __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ctrl, 0xf, 0xf, true))

@@ -34,6 +34,7 @@ template <> struct Mfma<__half> {
   static __device__ __forceinline__ float hi(unsigned w) {
     return __half2float(__ushort_as_half(static_cast<unsigned short>(w >> 16)));
   }
+  static __device__ __forceinline__ float element(const u32x4 &r, int i) { return i % 2 ? hi(r[i / 2]) : lo(r[i / 2]); }
   // two values rounded to nearest even and packed, in one instruction
   static __device__ __forceinline__ unsigned pack2(float a, float b) {
     unsigned r;
@@ -44,12 +45,6 @@ template <> struct Mfma<__half> {
   static __device__ __forceinline__ void fma_piece(float (&v)[8], float w, u32x4 r) {
     v[0] += w * lo(r.x); v[1] += w * hi(r.x); v[2] += w * lo(r.y); v[3] += w * hi(r.y);
     v[4] += w * lo(r.z); v[5] += w * hi(r.z); v[6] += w * lo(r.w); v[7] += w * hi(r.w);
-  }
-  // d + sum over the piece of g * piece
-  static __device__ __forceinline__ float dot_piece(const float (&g)[8], u32x4 r, float d) {
-    d += g[0] * lo(r.x); d += g[1] * hi(r.x); d += g[2] * lo(r.y); d += g[3] * hi(r.y);
-    d += g[4] * lo(r.z); d += g[5] * hi(r.z); d += g[6] * lo(r.w); d += g[7] * hi(r.w);
-    return d;
   }
   static __device__ __forceinline__ u32x4 pack(const float (&v)[8]) {
     return u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7])};
@@ -65,6 +60,7 @@ template <> struct Mfma<__hip_bfloat16> {
   }
   static __device__ __forceinline__ float lo(unsigned w) { return __uint_as_float(w << 16); }
   static __device__ __forceinline__ float hi(unsigned w) { return __uint_as_float(w & 0xffff0000u); }
+  static __device__ __forceinline__ float element(const u32x4 &r, int i) { return i % 2 ? hi(r[i / 2]) : lo(r[i / 2]); }
   // two values rounded to nearest even and packed, in one instruction
   static __device__ __forceinline__ unsigned pack2(float a, float b) {
     unsigned r;
@@ -74,12 +70,6 @@ template <> struct Mfma<__hip_bfloat16> {
   static __device__ __forceinline__ void fma_piece(float (&v)[8], float w, u32x4 r) {
     v[0] += w * lo(r.x); v[1] += w * hi(r.x); v[2] += w * lo(r.y); v[3] += w * hi(r.y);
     v[4] += w * lo(r.z); v[5] += w * hi(r.z); v[6] += w * lo(r.w); v[7] += w * hi(r.w);
-  }
-  // d + sum over the piece of g * piece
-  static __device__ __forceinline__ float dot_piece(const float (&g)[8], u32x4 r, float d) {
-    d += g[0] * lo(r.x); d += g[1] * hi(r.x); d += g[2] * lo(r.y); d += g[3] * hi(r.y);
-    d += g[4] * lo(r.z); d += g[5] * hi(r.z); d += g[6] * lo(r.w); d += g[7] * hi(r.w);
-    return d;
   }
   static __device__ __forceinline__ u32x4 pack(const float (&v)[8]) {
     return u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7])};
@@ -99,7 +89,7 @@ template <> struct Mfma<float> {
     c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.z), __uint_as_float(b.z), c, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.w), __uint_as_float(b.w), c, 0, 0, 0);
   }
-  static __device__ __forceinline__ float lo(unsigned w) { return __uint_as_float(w); }
+  static __device__ __forceinline__ float element(const u32x4 &r, int i) { return __uint_as_float(r[i]); }
   static __device__ __forceinline__ void fma_piece(float (&v)[4], float w, u32x4 r) {
     v[0] += w * __uint_as_float(r.x); v[1] += w * __uint_as_float(r.y);
     v[2] += w * __uint_as_float(r.z); v[3] += w * __uint_as_float(r.w);

@@ -73,3 +73,33 @@ def test_small_gradients_beside_large_ones(oracle, dtype, cin, cout, size, strid
     assert float(want.abs().max()) < 1.0       # nothing of the large ones
     error = float((got - want).norm() / want.norm())
     assert error < (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8), error
+
+
+@pytest.mark.parametrize("cin,cout,size", [(32, 32, (5, 12, 21)), (64, 32, (24, 40))])
+def test_offset_gradient_of_nearly_equal_corners(oracle, cin, cout, size):
+    """Offset gradients are formed from differences of the corners, channel by channel: an input of 64 and 64 + one step of fp16
+    loses nothing.  Weights and gradients are whole numbers, so that their sums with the differences are exact in fp32 and
+    only the blend over the rows rounds (four operations, 2^-24 each); with one sum per corner, 1000 times as large, what cancels
+    would show in the small results."""
+    nd, delta, dtype = len(size), 1 / 16, torch.float16
+    if nd == 3:
+        from medvision_amd.ops.modulated_deform_conv_3d import modulated_deform_conv
+    else:
+        from medvision_amd.ops.modulated_deform_conv_2d import modulated_deform_conv
+    g = wl.gen(cin + sum(size))
+    taps = 3 ** nd
+    x = (64 + delta * torch.randint(0, 2, (1, cin, *size), generator=g)).to(dtype)
+    w = torch.randint(-128, 129, (cout, cin, *[3] * nd), generator=g).to(dtype)
+    gy = torch.randint(-128, 129, (1, cout, *size), generator=g).to(dtype)
+    off = ((torch.rand(1, nd * taps, *size, generator=g) - 0.5) * 1.5).to(dtype)
+    mask, b = torch.ones(1, taps, *size, dtype=dtype), torch.zeros(cout, dtype=dtype)
+    leaves = [t.to(DEV).requires_grad_(True) for t in (x, off, mask, w, b)]
+    y = modulated_deform_conv(*leaves, 1, 1, 1, 1, 1)
+    got = torch.autograd.grad(y, leaves[1], gy.to(DEV))[0]
+    want = oracle.dcn3d_backward(x, off, mask, w, gy, True, 1, 1, 1, 1, 1)[1].reshape(off.shape)
+    inside = (slice(None), slice(nd - 1, None, nd), *[slice(2, -2)] * nd)     # along w, away from the zeros outside
+    got, want = got.cpu().double()[inside], want[inside]
+    terms = torch.einsum("ock,oq->ckq", w.double().flatten(2), gy.double()[0].flatten(1)).abs().sum(0)   # sum over c of |gcol|
+    largest = (terms.reshape(1, taps, *size) * delta)[(slice(None), slice(None), *inside[2:])]
+    worst = float((((got - want).abs() - 2.0 ** -11 * want.abs()) / largest).max())
+    assert worst <= 2.0 ** -22, worst
