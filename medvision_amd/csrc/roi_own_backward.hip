@@ -4,13 +4,13 @@
 // (csrc/cuda/roi_align_rotated_3d_cuda_kernel.cuh:124-265 and the 2-D twin).
 //
 // A workgroup owns a tile of 64 voxels (8 x 4 x 2, images 8 x 8) and 64 channels and writes their gradient once.  It lists
-// the rois whose samples' bounding box meets the tile; each of its four wavefronts takes rois from the list.  A roi's
+// the rois whose samples' bounding box meets the tile; each of its two wavefronts takes rois from the list.  A roi's
 // contribution is a matrix product, gradient[voxel][channel] = sum over cells of weight[voxel][cell] *
 // grad_output[cell][channel], where weight[voxel][cell] is the mean over the cell's samples of the corner weights that
 // fall on the voxel.  The wavefront picks the cells that reach the tile (32 columns at a time, of several rois where one
 // has fewer), works their samples out once -- for all the channels -- and adds the corner weights to a table of 32-bit
-// fixed-point numbers in LDS (quanta of 2^-30 of a cell's whole weight, so finer than the fp32 product of the three
-// fractions that they are made of); the table then is the left operand of matrix-core products with the
+// fixed-point numbers in LDS (quanta of 2^-30 of a cell's whole weight -- of the part of it that one voxel can get where a
+// cell has many samples -- so finer than the fp32 product of the three fractions that they are made of); the table then is the left operand of matrix-core products with the
 // gradient's rows, which a transposing copy has laid out channels-last.  Products keep the table's precision: 16-bit
 // gradients are exact operands and the weights are split into two fp16 or three bf16 numbers, fp32 ones use the fp32
 // matrix instructions; sums are fp32.
@@ -42,6 +42,7 @@ constexpr int kOwnTried = 2;       // rois that a thread tries at a time: their 
 // map from a tile's middle to the middle of the cells that can reach it, in cells, with half their extent.
 struct OwnBox { float map[3][3], offset[3], reach[3], unused; };
 static_assert(sizeof(OwnBox) == 64 && sizeof(RoiGeom) == 192, "a box record is one cache line, a geometry record 24 doubles");
+constexpr int kOwnPart = 47;   // word of a geometry record, behind its last member: the part of a cell's whole weight that one voxel can get
 struct OwnRois {
   RoiGeom *geom;    // [R]
   OwnBox *box;      // [R]
@@ -76,6 +77,25 @@ __device__ inline void own_geometry(const float *roi, const unsigned n, const Ow
     if (!(c - reach <= c + reach)) empty = true;   // NaN
   }
   out.geom[n] = g;
+  // The part of a cell's whole weight that one voxel can get, as a power of two.  A sample's weight is at most the integral, over
+  // its cell of the sample lattice, of the voxel's weight function widened by half that cell: (b + e) / spacing per axis, e the
+  // lattice cell's extent along the voxel axis, b the function's own integral (1; 1.5 at a border, whose voxel also takes the
+  // samples beyond it; 2 on an axis of one voxel).  (1 down to an eighth: three bits of 30 do not matter, and rois of one part
+  // share tables.)
+  double most = 1.0;
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    if (a >= p.ndim) continue;
+    double e = 0.0;
+#pragma unroll
+    for (int j = 0; j < 3; j++)
+      if (j < p.ndim) e += fabs(g.rot[3 * a + j] * g.sub[j]);
+    most *= (((a == 0 ? p.W : a == 1 ? p.H : p.D) == 1 ? 2.0 : 1.5) + e) / fabs(g.sub[a]);
+  }
+  float part = 1.f;
+  if (most * 1.0001 < g.count)   // (not for NaN)
+    while (part > 1e-9f && 0.5 * part * g.count >= fmax(most * 1.0001, 1.0)) part *= 0.5f;
+  reinterpret_cast<float *>(out.geom + n)[kOwnPart] = part < 0.125f ? part : 1.f;
   out.first[n] = make_float4(empty ? 3e38f : lo[0], lo[1], lo[2], __int_as_float(g.batch));
   out.last[n] = make_float4(hi[0], hi[1], hi[2], 0.f);
   OwnBox box;
@@ -308,8 +328,10 @@ __global__ __launch_bounds__(kOwnThreads, 3) void roi_own_backward_kernel(const 
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[m][n][i] = 0.f;
     int columns = 0;   // of the table in use
+    unsigned part_bits = __float_as_uint(1.f);   // kOwnPart of the rois in the table
 
     auto multiply = [&] {
+      const float unit = S::scale * __uint_as_float(part_bits);
       own_wave_sync();
       if (careful) {
         for (int k = 0; k < columns; k++) {
@@ -321,7 +343,7 @@ __global__ __launch_bounds__(kOwnThreads, 3) void roi_own_backward_kernel(const 
             for (int i = 0; i < 16; i++) {
               const unsigned q = table[(m * 32 + 8 * (i / 4) + 4 * half + i % 4) * kOwnPitch + k];
               if (q != 0) {
-                const float w = static_cast<float>(q) * S::scale;
+                const float w = static_cast<float>(q) * unit;
                 acc[m][0][i] += w * g0;
                 acc[m][1][i] += w * g1;
               }
@@ -349,7 +371,7 @@ __global__ __launch_bounds__(kOwnThreads, 3) void roi_own_backward_kernel(const 
           cell[1] = own_u32x4{0, 0, 0, 0};
           const unsigned q[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
 #pragma unroll
-          for (int e = 0; e < 8; e++) w[m][e] = static_cast<float>(q[e]) * S::scale;
+          for (int e = 0; e < 8; e++) w[m][e] = static_cast<float>(q[e]) * unit;
         }
         if (careful) continue;
         if constexpr (sizeof(T) == 2) {
@@ -387,7 +409,7 @@ __global__ __launch_bounds__(kOwnThreads, 3) void roi_own_backward_kernel(const 
       own_wave_sync();
     };
 
-    auto one_roi = [&](const RoiGeom &g, const unsigned n, const unsigned corner, const unsigned beyond) {
+    auto one_roi = [&](const RoiGeom &g, const unsigned bits, const unsigned n, const unsigned corner, const unsigned beyond) {
       const int first[3] = {static_cast<int>(corner & 1023u), static_cast<int>((corner >> 10) & 1023u), static_cast<int>(corner >> 20)};
       const int num[3] = {static_cast<int>(beyond & 1023u) + 1, static_cast<int>((beyond >> 10) & 1023u) + 1, static_cast<int>(beyond >> 20) + 1};
       double reach[3];   // of a cell's samples along the voxel axes
@@ -400,7 +422,7 @@ __global__ __launch_bounds__(kOwnThreads, 3) void roi_own_backward_kernel(const 
       }
       const int count = g.count, boxed = num[0] * num[1] * num[2];
       const float inv_x = 1.f / static_cast<float>(num[0]), inv_y = 1.f / static_cast<float>(num[1]);
-      const float quanta = 1073741824.f / static_cast<float>(count);
+      const float quanta = 1073741824.f / (__uint_as_float(bits) * static_cast<float>(count));
       const float inv_gx = 1.f / static_cast<float>(g.grid[0]), inv_gy = 1.f / static_cast<float>(g.grid[1]);
       for (int i0 = 0; i0 < boxed; i0 += kWave) {
         // each cell of the box is tried on its own
@@ -426,6 +448,10 @@ __global__ __launch_bounds__(kOwnThreads, 3) void roi_own_backward_kernel(const 
         if (hit) mine[__popcll(hits & ((1UL << lane) - 1))] = static_cast<unsigned>(at[0]) | at[1] << 10 | at[2] << 20;
         own_wave_sync();
         for (int done = 0; left > 0;) {
+          if (columns == kOwnColumns || bits != part_bits) {
+            multiply();
+            part_bits = bits;
+          }
           const int m = min(left, kOwnColumns - columns);
           // lanes: m cells (rounded up to a power of two) times parts of their samples
           const int log_m = m > 1 ? 32 - __clz(m - 1) : 0, parts = kWave >> log_m;
@@ -472,7 +498,6 @@ __global__ __launch_bounds__(kOwnThreads, 3) void roi_own_backward_kernel(const 
             }
           }
           columns += m; done += m; left -= m;
-          if (columns == kOwnColumns) multiply();
         }
       }
     };
@@ -579,9 +604,10 @@ __global__ __launch_bounds__(kOwnThreads, 3) void roi_own_backward_kernel(const 
         for (int a = 0; a < 3; a++) { g.centre[a] = from(9 + a); g.start[a] = from(12 + a); g.bin[a] = from(15 + a); g.sub[a] = from(18 + a); }
         g.grid[0] = __builtin_amdgcn_readlane(rec.x, 21); g.grid[1] = __builtin_amdgcn_readlane(rec.y, 21);
         g.grid[2] = __builtin_amdgcn_readlane(rec.x, 22); g.count = __builtin_amdgcn_readlane(rec.x, 23);
+        const unsigned bits = __builtin_amdgcn_readlane(rec.y, kOwnPart / 2);
         const unsigned n0 = n, corner0 = corner, beyond0 = beyond;
         more = take(n, corner, beyond, rec);
-        one_roi(g, n0, corner0, beyond0);
+        one_roi(g, bits, n0, corner0, beyond0);
       }
     }
     if (!any) break;
