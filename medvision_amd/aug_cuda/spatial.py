@@ -425,6 +425,8 @@ class CudaRandomElasticDeformation(CudaAugBase):
         *image_shape] -- cached per draw."""
         if self.tmp_params is None:
             coarse = self.params if self.batched else self.params[None]
+            if coarse.dtype.kind != 'f':
+                coarse = coarse.astype(np.float32)
             grid = np.moveaxis(coarse, -1, 1) / 2          # [batch, component, *grid]
             shape_xyz = grid.shape[2:][::-1]
             roi = geometry.window_rois(self.dim, [1.5] * self.dim, [s - 1.5 for s in shape_xyz],

@@ -460,17 +460,22 @@ Tensor deform_warp(const Tensor &img_in, const Tensor &offset_in, int order) {
 }
 
 // ---- helpers of the augmentation stages ----------------------------------------------------------------------------
-// A host array (rois, a control grid) on the device, without waiting for what is queued there.
-Tensor upload(const py::array_t<float, py::array::c_style | py::array::forcecast> &array, const at::Device &device) {
+// A host array (rois, a control grid) on the device, without waiting for what is queued there.  float64 stays float64,
+// every other type becomes float32.
+Tensor upload(const py::array &given, const at::Device &device) {
+  const bool wide = py::isinstance<py::array_t<double>>(given);
+  const py::array array = wide ? py::array(py::array_t<double, py::array::c_style | py::array::forcecast>(given))
+                               : py::array(py::array_t<float, py::array::c_style | py::array::forcecast>(given));
+  const auto type = wide ? at::kDouble : at::kFloat;
   const std::vector<int64_t> shape(array.shape(), array.shape() + array.ndim());
-  const size_t bytes = static_cast<size_t>(array.size()) * sizeof(float);
-  const float *data = array.data();
+  const size_t bytes = static_cast<size_t>(array.nbytes());
+  const void *data = array.data();
   const py::gil_scoped_release no_gil;
   const at::NoGradGuard no_grad;
   if (!device.is_cuda() || bytes > MV_UPLOAD_MAX_BYTES)
-    return at::from_blob(const_cast<float *>(data), shape, at::kFloat).to(device, at::kFloat, false, true);
+    return at::from_blob(const_cast<void *>(data), shape, type).to(device, type, false, true);
   const c10::DeviceGuard guard(device);
-  const Tensor out = at::empty(shape, at::TensorOptions().dtype(at::kFloat).device(device));
+  const Tensor out = at::empty(shape, at::TensorOptions().dtype(type).device(device));
   check(mv_upload(data, ptr(out), bytes, stream_of(out)));
   return out;
 }

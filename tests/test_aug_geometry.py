@@ -8,6 +8,7 @@ import random
 
 import numpy as np
 import pytest
+import torch
 
 from medvision_amd.aug_cuda import geometry
 from medvision_amd.aug_cuda import spatial
@@ -100,3 +101,27 @@ def test_elastic_control_grid_and_gate():
     assert out["history"] == ["CudaRandomShift"] and "CudaRandomShift_params" not in out
     with pytest.raises(AssertionError):
         spatial.CudaRandomShift(p=0.0, shift=0.1)({"img": torch.zeros(1, 4, 4), "img_dim": 2})
+
+
+def test_uploads_keep_double():
+    """Control grids and rois that a caller gives in float64 stay float64 (the field is then resampled in float64)."""
+    from medvision_amd._lib import native
+    values = np.random.default_rng(0).standard_normal((2, 3, 5))
+    for array, dtype in ((values, torch.float64), (values.astype(np.float32), torch.float32), (values.T, torch.float64),
+                         (np.arange(6), torch.float32)):
+        out = native.upload(array, torch.device("cpu"))
+        assert out.dtype == dtype and out.is_contiguous()
+        assert torch.equal(out, torch.from_numpy(np.ascontiguousarray(array)).to(dtype))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("grid,dtype", [(np.float64, torch.float64), (np.float32, torch.float32), (np.int64, torch.float32)])
+def test_elastic_field_keeps_the_control_grids_type(grid, dtype):
+    import medvision_amd.aug_cuda as aug
+    params = (np.random.default_rng(1).standard_normal((9, 9, 9, 3)) * 3).astype(grid)   # 17 KB in float64: more than one upload
+    for points in (5, 9):
+        stage = aug.CudaRandomElasticDeformation(1.0, points, 0.8)
+        stage._init_params({"img": torch.zeros(1, 20, 24, 28, device="cuda"), "img_dim": 3})
+        stage.params = params[:points, :points, :points]
+        field = stage.dense_field(torch.device("cuda"))
+        assert field.dtype == dtype and field.shape == (3, 20, 24, 28)
