@@ -185,9 +185,11 @@ typedef struct {
 
 int mv_dcn3d_output_dims(const mv_dcn3d_shape *shape, int *out_d, int *out_h, int *out_w);
 size_t mv_dcn3d_forward_workspace_bytes(const mv_dcn3d_shape *shape, int dtype);
-/* The backward workspace of 16-bit / fp32 layers on the matrix-core path includes a buffer of column
- * values (batch x taps x in_channels x positions elements) while that stays below 1 GiB or the number
- * of bytes set with mv_dcn_set_column_budget() / the environment variable MV_DCN_COLUMN_BYTES. */
+/* The backward workspace of 16-bit / fp32 layers on the matrix-core path includes a buffer of partial
+ * sums (16 bytes x batch x deformable groups x taps x positions x chunks of channels) for layers of more than one
+ * chunk: 32 input channels per deformable group (64 for 16-bit images) and 256 output channels (fp32: 128).  Where
+ * they exceed 1 GiB, or the number of bytes set with mv_dcn_set_column_budget() / the environment variable
+ * MV_DCN_COLUMN_BYTES, the layer runs in several launches that share a buffer of that size. */
 size_t mv_dcn3d_backward_workspace_bytes(const mv_dcn3d_shape *shape, int dtype);
 int mv_dcn3d_forward(const void *input, const void *offset, const void *mask, const void *weight,
                      const void *bias, void *output, const mv_dcn3d_shape *shape, int dtype,
@@ -202,10 +204,11 @@ int mv_dcn3d_backward_write(const void *input, const void *offset, const void *m
                             void *grad_mask, void *grad_weight, void *grad_bias,
                             const mv_dcn3d_shape *shape, int dtype, void *workspace, void *stream);
 
-/* Budget of the column buffer that the backward pass of earlier versions kept (default 1 GiB, or
- * MV_DCN_COLUMN_BYTES in the environment when the library is first asked).  The pass has no such buffer any
- * more: the value is stored and returned, and changes nothing.  No counterpart in the reference
- * (its column buffer is a tensor argument, csrc/modulated_deform_conv_3d.h:89).               */
+/* Limit of those partial sums (default 1 GiB, or MV_DCN_COLUMN_BYTES in the environment when the library is first
+ * asked); a buffer for one tap and 4096 positions is the least, whatever the limit.  Query the workspace size again
+ * after changing it, and do not change it between a query and its backward call (other threads' included).  (Named
+ * after the column buffer that it limited before: the reference's is a tensor argument,
+ * csrc/modulated_deform_conv_3d.h:89.)                                                                       */
 void mv_dcn_set_column_budget(size_t bytes);
 size_t mv_dcn_column_budget(void);
 

@@ -363,8 +363,9 @@ def _dcn_backward(input, offset, mask, weight, grad_output, gi, goff, gmask, gw,
 
 
 def set_dcn_column_budget(nbytes):
-    """Budget (bytes) of the column buffer that the DCN backward of earlier versions kept: stored and
-    returned, without effect.  Returns the previous budget."""
+    """Limit (bytes) of the partial sums that the DCN backward keeps in its workspace (layers of more than 32 or 64
+    input channels per deformable group, or more than 256 output channels): layers beyond it run in several launches.
+    Returns the previous limit.  Not while other threads are in a backward pass."""
     lib = _lib.load()
     old = lib.mv_dcn_column_budget()
     lib.mv_dcn_set_column_budget(int(nbytes))

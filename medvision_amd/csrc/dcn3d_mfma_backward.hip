@@ -82,11 +82,11 @@ __device__ __forceinline__ void dcn_weight_colsum_block(const T *__restrict__ wt
 }
 
 // dcn_backward_tap.hip
-size_t dcn_tap_partial_bytes(const DcnDims &s, int dtype);
+size_t dcn_tap_partial_bytes(const DcnDims &s, int dtype, size_t budget);
 bool dcn_tap_supported(const DcnDims &s, int dtype);
 int dcn_tap_backward(const void *xt, const void *off, const void *mask, const void *gyt, const void *wf,
-                     float *gxt, void *goff, void *gmask, float *partial, float *gw, const DcnDims &s, const unsigned *bounds,
-                     const ScatterShape &shape, int dtype, hipStream_t stream);
+                     float *gxt, void *goff, void *gmask, float *partial, size_t budget, float *gw, const DcnDims &s,
+                     const unsigned *bounds, const ScatterShape &shape, int dtype, hipStream_t stream);
 // dcn_backward_scatter.hip
 bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape);
 int dcn_scatter(const void *off, const void *mask, const void *gyt, const void *wf, float *gxt, const DcnDims &s,
@@ -348,7 +348,7 @@ bool dcn_mfma_backward_supported(const DcnDims &s, int dtype) {
 struct BackwardLayout {
   size_t xt, gyt, wb, gxt, gw, gb, bounds, part, total;
 };
-// (the budget of an earlier design's column buffer, still stored and returned for callers that set it)
+// Bytes that the partial sums may take: layers with more run in pieces (fewer taps or positions per launch).
 static std::atomic<size_t> &column_budget_cell() {
   static std::atomic<size_t> cell{[] {
     const char *e = getenv("MV_DCN_COLUMN_BYTES");
@@ -358,7 +358,7 @@ static std::atomic<size_t> &column_budget_cell() {
 }
 void dcn_set_column_budget(size_t bytes) { column_budget_cell().store(bytes, std::memory_order_relaxed); }
 size_t dcn_column_budget() { return column_budget_cell().load(std::memory_order_relaxed); }
-static BackwardLayout backward_layout(const DcnDims &s, int dtype) {
+static BackwardLayout backward_layout(const DcnDims &s, int dtype, size_t budget) {
   BackwardLayout l;
   const size_t es = dtype == MV_F32 ? 4 : 2;
   size_t at = 0;
@@ -369,19 +369,20 @@ static BackwardLayout backward_layout(const DcnDims &s, int dtype) {
   l.gw = at; at += align256b(static_cast<size_t>(s.Cout) * s.cpg * s.K * 4);
   l.gb = at; at += align256b(static_cast<size_t>(s.Cout) * 4);
   l.bounds = at; at += 256;
-  l.part = at; at += align256b(dcn_tap_partial_bytes(s, dtype));
+  l.part = at; at += align256b(dcn_tap_partial_bytes(s, dtype, budget));
   l.total = at;
   return l;
 }
 
-size_t dcn_mfma_backward_workspace_bytes(const DcnDims &s, int dtype) { return backward_layout(s, dtype).total; }
+size_t dcn_mfma_backward_workspace_bytes(const DcnDims &s, int dtype) { return backward_layout(s, dtype, dcn_column_budget()).total; }
 
 template <typename T>
 static int backward_run(const void *x, const void *off, const void *mask, const void *wt,
                         const void *gy, void *goff, void *gmask, const DcnDims &real, const DcnPad &pad, void *workspace,
                         float **gx32, float **gw32, float **gb32, int dtype, bool want_bias, hipStream_t stream) {
   const DcnDims &s = pad.p;
-  const BackwardLayout l = backward_layout(s, dtype);
+  const size_t budget = dcn_column_budget();
+  const BackwardLayout l = backward_layout(s, dtype, budget);
   char *ws = static_cast<char *>(workspace);
   T *xt = reinterpret_cast<T *>(ws + l.xt), *gyt = reinterpret_cast<T *>(ws + l.gyt), *wb = reinterpret_cast<T *>(ws + l.wb);
   float *gxt = reinterpret_cast<float *>(ws + l.gxt);
@@ -418,7 +419,7 @@ static int backward_run(const void *x, const void *off, const void *mask, const 
   }
   int st = check_launch("dcn_backward_prepare_kernel");
   if (st) return st;
-  st = dcn_tap_backward(xt, off, mask, gyt, wb, gxt, goff, gmask, reinterpret_cast<float *>(ws + l.part), *gw32, s,
+  st = dcn_tap_backward(xt, off, mask, gyt, wb, gxt, goff, gmask, reinterpret_cast<float *>(ws + l.part), budget, *gw32, s,
                         tiles ? bounds : nullptr, shape, dtype, stream);
   return st || !tiles ? st : dcn_scatter(off, mask, gyt, wb, gxt, s, shape, bounds, dtype, stream);
 }

@@ -59,6 +59,10 @@ template <typename T> __device__ __forceinline__ u32x4 tap_transposed(const u32x
   }
 }
 
+// A launch's part of the layer: all of it, unless the shares of the offset and mask gradients (`partial`) are limited
+// to fewer taps or positions at a time.
+struct TapPiece { int k_first, taps, q_first, positions; };
+
 // workgroups per compute unit that the registers should leave room for
 template <typename T, int NC, int OBW, int CBW>
 constexpr int TAP_WAVES = OBW * CBW >= 8 || (NC == 8 && (sizeof(T) == 4 || OBW >= 2)) ? 2 : OBW == 1 && CBW == 2 && sizeof(T) == 2 ? 4 : 3;
@@ -71,7 +75,7 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
     const T *__restrict__ xt, const T *__restrict__ off, const T *__restrict__ mask, const T *__restrict__ gyt,
     const T *__restrict__ wf, float *__restrict__ gxt, T *__restrict__ goff, T *__restrict__ gmask,
     float *__restrict__ partial, float *__restrict__ gw, const DcnDims s, const unsigned *__restrict__ bounds,
-    const ScatterShape shape, const int chunks, const int shares, const int range, const int row0) {
+    const ScatterShape shape, const int chunks, const int shares, const int range, const int row0, const TapPiece piece) {
   using M = Mfma<T>;
   using P = typename std::conditional<(sizeof(T) == 2), float, double>::type;  // position type
   constexpr int PC = M::kPiece, SL = 4 * PC, ES = sizeof(T), CW = 16 * CBW, ROWS = 64 * OBW;
@@ -88,11 +92,12 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
   const int j = lane % 16, kc = lane / 16;   // matrix layout
   const int lj = lane / 4, lk = lane % 4;    // load layout
   // (taps of one range next to each other, on one XCD: they gather the same part of x and read the same gy)
-  const int id = static_cast<int>(xcd_contiguous(blockIdx.x, gridDim.x)), k = id % s.K;
+  const int id = static_cast<int>(xcd_contiguous(blockIdx.x, gridDim.x)), k = piece.k_first + id % piece.taps;
   const int dgi = blockIdx.y / chunks, part = blockIdx.y % chunks, b = blockIdx.z;
   const int c0 = dgi * s.cpd + part * CW, g = c0 / s.cpg;
-  const long q0 = static_cast<long>(id / s.K) * range;
-  const int count = static_cast<int>(min(static_cast<long>(range), s.Q - q0));   // positions of the range
+  const int within = id / piece.taps * range;   // < 2^31: within.. is a range of the piece
+  const long q0 = piece.q_first + static_cast<long>(within);
+  const int count = min(range, piece.positions - within);   // positions of the range
   const long bg = static_cast<long>(b) * s.dg + dgi;
   const int rows = min(ROWS, s.opg - row0), steps = rows / SL;
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
@@ -183,7 +188,8 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
   T *tout = nullptr;
   {
     const int p = wave * 16 + lj;
-    if (partial) pout = partial + (((bg * s.K + k) * shares + row0 / ROWS * chunks + part) * s.Q + q0 + p) * 4 + lk;
+    if (partial)
+      pout = partial + (((bg * piece.taps + k - piece.k_first) * shares + row0 / ROWS * chunks + part) * piece.positions + within + p) * 4 + lk;
     else if (lk == 3) tout = gmask ? gmask + (bg * s.K + k) * s.Q + q0 + p : nullptr;
     else if (lk + s.nd >= 3) tout = goff + (bg * s.nd * s.K + s.nd * k + lk + s.nd - 3) * s.Q + q0 + p;
   }
@@ -337,19 +343,21 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
 // The chunks' shares of the offset and mask gradients, summed.
 template <typename T>
 __global__ __launch_bounds__(256) void dcn_backward_partial_kernel(const float4 *__restrict__ partial, T *__restrict__ goff,
-                                                                   T *__restrict__ gmask, const DcnDims s, const int chunks) {
-  const long q = blockIdx.x * 256L + threadIdx.x, bgk = blockIdx.y + static_cast<long>(blockIdx.z) * s.dg * s.K;
-  if (q >= s.Q) return;
+                                                                   T *__restrict__ gmask, const DcnDims s, const int chunks,
+                                                                   const TapPiece piece) {
+  const long q = blockIdx.x * 256L + threadIdx.x, row = blockIdx.y + static_cast<long>(blockIdx.z) * s.dg * piece.taps;
+  if (q >= piece.positions) return;
   float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
   for (int c = 0; c < chunks; c++) {
-    const float4 v = partial[(bgk * chunks + c) * s.Q + q];
+    const float4 v = partial[(row * chunks + c) * piece.positions + q];
     sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
   }
-  T *go = goff + bgk * s.nd * s.Q + q;
+  const long bgk = row / piece.taps * s.K + piece.k_first + row % piece.taps;
+  T *go = goff + bgk * s.nd * s.Q + piece.q_first + q;
   if (s.nd == 3) *go = store_cast<T>(sum.x);
   go[(s.nd - 2) * s.Q] = store_cast<T>(sum.y);
   go[(s.nd - 1) * s.Q] = store_cast<T>(sum.z);
-  if (gmask) gmask[bgk * s.Q + q] = store_cast<T>(sum.w);
+  if (gmask) gmask[bgk * s.Q + piece.q_first + q] = store_cast<T>(sum.w);
 }
 
 // Chunks of 64 input channels for 16-bit images (four corners; grad_output of a tile then serves twice the channels), 32
@@ -363,9 +371,24 @@ static int tap_chunks(const DcnDims &s, int dtype) { return s.cpd / tap_chunk(s,
 static int tap_rows(int dtype) { return dtype == MV_F32 ? 128 : 256; }
 static int tap_shares(const DcnDims &s, int dtype) { return tap_chunks(s, dtype) * ((s.opg + tap_rows(dtype) - 1) / tap_rows(dtype)); }
 
-size_t dcn_tap_partial_bytes(const DcnDims &s, int dtype) {
-  const int shares = tap_shares(s, dtype);
-  return shares > 1 ? static_cast<size_t>(s.B) * s.dg * s.K * shares * s.Q * 16 : 0;
+constexpr long kTapRange = 64 * kTapTile;   // positions of a workgroup at most
+
+// Taps and positions of a launch (TapPiece): as many as keep the shares of several chunks within `budget` bytes, fewer positions
+// only where a single tap is beyond it, one range of them at least.
+static long tap_share_bytes(const DcnDims &s, int dtype) { return static_cast<long>(s.B) * s.dg * tap_shares(s, dtype) * 16; }
+static void tap_pieces(const DcnDims &s, int dtype, size_t budget, long &taps, long &positions) {
+  taps = s.K;
+  positions = s.Q;
+  if (tap_shares(s, dtype) == 1) return;
+  const long fits = static_cast<long>(std::min(budget, static_cast<size_t>(1) << 62)) / tap_share_bytes(s, dtype);   // taps x positions
+  taps = std::min(std::max(fits / s.Q, 1L), static_cast<long>(s.K));
+  if (fits < s.Q) positions = std::min(std::max(fits / kTapRange, 1L) * kTapRange, s.Q);
+}
+size_t dcn_tap_partial_bytes(const DcnDims &s, int dtype, size_t budget) {
+  if (tap_shares(s, dtype) == 1) return 0;
+  long taps, positions;
+  tap_pieces(s, dtype, budget, taps, positions);
+  return static_cast<size_t>(tap_share_bytes(s, dtype)) * taps * positions;
 }
 bool dcn_tap_supported(const DcnDims &s, int dtype) {
   // (a range of 4096 positions of grad_output within 32-bit byte offsets)
@@ -375,19 +398,19 @@ bool dcn_tap_supported(const DcnDims &s, int dtype) {
 template <typename T, int NC, int CBW>
 static int tap_launch(const T *xt, const T *off, const T *mask, const T *gyt, const T *wf, float *gxt, T *goff,
                       T *gmask, float *partial, float *gw, const DcnDims &s, const unsigned *bounds, const ScatterShape &shape, int dtype,
-                      hipStream_t stream) {
+                      const TapPiece &piece, hipStream_t stream) {
   const int chunks = tap_chunks(s, dtype), shares = tap_shares(s, dtype);
   // Positions of a workgroup: every one adds a block of the weight gradient to memory and fills LDS with a block of the
   // weight, so as many as leave ~4 workgroups per compute unit.
-  const long others = static_cast<long>(s.K) * s.dg * chunks * s.B, tiles = (s.Q + kTapTile - 1) / kTapTile;
-  const long want = std::max(1L, 1024 / others), per = std::min(std::max(1L, (tiles + want - 1) / want), 64L);
+  const long others = static_cast<long>(piece.taps) * s.dg * chunks * s.B, tiles = (piece.positions + static_cast<long>(kTapTile) - 1) / kTapTile;
+  const long want = std::max(1L, 1024 / others), per = std::min(std::max(1L, (tiles + want - 1) / want), kTapRange / kTapTile);
   const long ranges = (tiles + per - 1) / per;
-  MV_REQUIRE(ranges * s.K < (1L << 31), "grid too large");
-  const dim3 grid(static_cast<unsigned>(ranges * s.K), static_cast<unsigned>(s.dg * chunks), s.B);
+  MV_REQUIRE(ranges * piece.taps < (1L << 31), "grid too large");
+  const dim3 grid(static_cast<unsigned>(ranges * piece.taps), static_cast<unsigned>(s.dg * chunks), s.B);
   const int range = static_cast<int>(per * kTapTile);
 #define MV_TAP(OBWV, ROW)                                                                                               \
   hipLaunchKernelGGL((dcn_backward_tap_kernel<T, NC, OBWV, CBW>), grid, dim3(256), 0, stream, xt, off, mask, gyt, wf, gxt,     \
-                     goff, gmask, partial, gw, s, bounds, shape, chunks, shares, range, ROW)
+                     goff, gmask, partial, gw, s, bounds, shape, chunks, shares, range, ROW, piece)
   if (s.opg <= 64) {
     MV_TAP(1, 0);
   } else if (s.opg <= 128 || sizeof(T) == 4) {
@@ -398,25 +421,35 @@ static int tap_launch(const T *xt, const T *off, const T *mask, const T *gyt, co
 #undef MV_TAP
   int st = check_launch("dcn_backward_tap_kernel");
   if (st || !partial) return st;
-  hipLaunchKernelGGL((dcn_backward_partial_kernel<T>), dim3(static_cast<unsigned>((s.Q + 255) / 256), s.dg * s.K, s.B), dim3(256), 0,
-                     stream, reinterpret_cast<const float4 *>(partial), goff, gmask, s, shares);
+  hipLaunchKernelGGL((dcn_backward_partial_kernel<T>), dim3(static_cast<unsigned>((piece.positions + 255L) / 256), s.dg * piece.taps, s.B),
+                     dim3(256), 0, stream, reinterpret_cast<const float4 *>(partial), goff, gmask, s, shares, piece);
   return check_launch("dcn_backward_partial_kernel");
 }
 
-// `bounds` null: no scatter kernel runs, every corner of the gradient of the input is added here
+// `bounds` null: no scatter kernel runs, every corner of the gradient of the input is added here.  `partial`: memory of
+// dcn_tap_partial_bytes(s, dtype, budget).
 int dcn_tap_backward(const void *xt, const void *off, const void *mask, const void *gyt, const void *wf,
-                     float *gxt, void *goff, void *gmask, float *partial, float *gw, const DcnDims &s, const unsigned *bounds,
-                     const ScatterShape &shape, int dtype, hipStream_t stream) {
+                     float *gxt, void *goff, void *gmask, float *partial, size_t budget, float *gw, const DcnDims &s,
+                     const unsigned *bounds, const ScatterShape &shape, int dtype, hipStream_t stream) {
   if (tap_shares(s, dtype) == 1) partial = nullptr;
+  long taps, positions;
+  tap_pieces(s, dtype, budget, taps, positions);
 #define MV_TAP_AS(T, NC, CBW)                                                                                          \
   tap_launch<T, NC, CBW>(static_cast<const T *>(xt), static_cast<const T *>(off), static_cast<const T *>(mask),           \
                          static_cast<const T *>(gyt), static_cast<const T *>(wf), gxt, static_cast<T *>(goff),            \
-                         static_cast<T *>(gmask), partial, gw, s, bounds, shape, dtype, stream)
+                         static_cast<T *>(gmask), partial, gw, s, bounds, shape, dtype, piece, stream)
   const bool wide = tap_chunk(s, dtype) == 64, image = s.nd == 2;
-  if (dtype == MV_F32) return image ? MV_TAP_AS(float, 4, 2) : MV_TAP_AS(float, 8, 2);
-  if (dtype == MV_F16) return wide ? MV_TAP_AS(__half, 4, 4) : image ? MV_TAP_AS(__half, 4, 2) : MV_TAP_AS(__half, 8, 2);
-  return wide ? MV_TAP_AS(__hip_bfloat16, 4, 4) : image ? MV_TAP_AS(__hip_bfloat16, 4, 2) : MV_TAP_AS(__hip_bfloat16, 8, 2);
+  for (long k = 0; k < s.K; k += taps)
+    for (long q = 0; q < s.Q; q += positions) {
+      const TapPiece piece{static_cast<int>(k), static_cast<int>(std::min(taps, s.K - k)), static_cast<int>(q),
+                           static_cast<int>(std::min(positions, s.Q - q))};
+      const int st = dtype == MV_F32 ? (image ? MV_TAP_AS(float, 4, 2) : MV_TAP_AS(float, 8, 2))
+                     : dtype == MV_F16 ? (wide ? MV_TAP_AS(__half, 4, 4) : image ? MV_TAP_AS(__half, 4, 2) : MV_TAP_AS(__half, 8, 2))
+                     : wide ? MV_TAP_AS(__hip_bfloat16, 4, 4) : image ? MV_TAP_AS(__hip_bfloat16, 4, 2) : MV_TAP_AS(__hip_bfloat16, 8, 2);
+      if (st) return st;
+    }
 #undef MV_TAP_AS
+  return MV_OK;
 }
 
 }  // namespace mv

@@ -132,3 +132,29 @@ def test_host_shim_cost_per_call(monkeypatch):
         best = min(best, (time.perf_counter() - t) / 2000 * 1e6)
     print(f"roi_align_rotated_3d_forward shim: {best:.1f} us per call")
     assert best < 2000.0   # (a sanity bound only: ~8 us on an idle core)
+
+
+def test_dcn_backward_workspace_keeps_to_its_limit():
+    """The partial sums of layers with several chunks of channels stay within the limit that the caller sets."""
+    import ctypes
+    from medvision_amd import _C, _lib
+    lib = _lib.load()
+
+    def need(shape, code=_lib.MV_F16):
+        fn = lib.mv_dcn3d_backward_workspace_bytes if isinstance(shape, _lib.DcnShape) else lib.mv_dcn2d_backward_workspace_bytes
+        return fn(ctypes.byref(shape), code)
+
+    volume = _lib.DcnShape(2, 256, 48, 48, 48, 256, 5, 5, 5, 1, 1, 1, 2, 2, 2, 1, 1, 1, 1, 1)     # 3.5 GB of partial sums
+    image = _lib.Dcn2dShape(8, 256, 100, 152, 256, 3, 3, 1, 1, 1, 1, 1, 1, 1, 1)
+    old = _C.set_dcn_column_budget(0)
+    try:
+        least = [need(s) for s in (volume, image)]
+        for budget in (100 << 20, 1 << 30, 2 ** 63):
+            _C.set_dcn_column_budget(budget)
+            for s, low in zip((volume, image), least):
+                assert low <= need(s) <= low + budget
+        assert need(volume) - least[0] > 3 << 30
+        _C.set_dcn_column_budget(1 << 30)
+        assert need(volume) - least[0] > 1 << 29     # ... and use it
+    finally:
+        _C.set_dcn_column_budget(old)

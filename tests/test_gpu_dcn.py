@@ -192,21 +192,28 @@ def test_input_gradient_through_lds_tiles_5x5x5(ops, oracle):
     assert_close(ws.grad, gw, tol, "grad weight")
 
 
-def test_weight_gradient_without_column_buffer(ops, oracle):
-    """Layers whose column values would not fit the buffer's budget gather x a second time in the
-    weight kernel: forced here by a budget of zero bytes."""
+@pytest.mark.parametrize("budget,channels,size", [
+    (0, 32, (7, 9, 11)),          # a single chunk of channels: no partial sums
+    (0, 96, (7, 9, 11)),          # a tap at a time
+    (140000, 96, (7, 9, 11)),     # two taps at a time, one at the end
+    (0, 192, (70, 61)),           # 4096 positions of a tap at a time, and the rest
+])
+def test_weight_gradient_without_column_buffer(ops, oracle, budget, channels, size):
+    """Layers whose partial sums (the shares of several chunks of channels in the offset and mask gradients) exceed the limit
+    run in pieces of fewer taps or positions."""
+    import importlib
     from medvision_amd import _C
-    from medvision_amd.ops.modulated_deform_conv_3d import modulated_deform_conv
-    old = _C.set_dcn_column_budget(0)
+    layer = importlib.import_module(f"medvision_amd.ops.modulated_deform_conv_{len(size)}d")
+    old = _C.set_dcn_column_budget(budget)
     try:
-        _weight_gradient_without_column_buffer(oracle, modulated_deform_conv)
+        _weight_gradient_without_column_buffer(oracle, layer.modulated_deform_conv, channels, size)
     finally:
         _C.set_dcn_column_budget(old)
 
 
-def _weight_gradient_without_column_buffer(oracle, modulated_deform_conv):
+def _weight_gradient_without_column_buffer(oracle, modulated_deform_conv, channels, size):
     g = wl.gen(450)
-    x, off, mask, w, b = wl.dcn_inputs(g, 2, 32, 64, (7, 9, 11), 3, 1, 1, torch.float16, 1, 1, 1, True, 2.0)
+    x, off, mask, w, b = wl.dcn_inputs(g, 2, channels, 64, size, 3, 1, 1, torch.float16, 1, 1, 1, True, 2.0)
     xs, offs, ms, ws, bs = [t.to(DEV).requires_grad_(True) for t in (x, off, mask, w, b)]
     y = modulated_deform_conv(xs, offs, ms, ws, bs, 1, 1, 1, 1, 1)
     gy = torch.randn(y.shape, generator=g).half()
