@@ -91,8 +91,16 @@ int mv_roi_align_rotated_3d_backward(const void *grad_output, const void *rois, 
 /* The backward of every head (rois of 5 / 7 columns, `rotated`: 6 / 10; `aligned` read for those only)
  * that REPLACES grad_input, whatever it held: for callers whose gradient buffer is fresh memory (autograd),
  * saves the pass that clears it and, where the kernels write every voxel, the one that reads it back.
- * Images (ndim 2): depth and out_d are ignored.  Workspace of mv_roi_align_backward_write_workspace_bytes(): the one of
- * the others, and one for fp32 volumes where summing channels-last is the faster way (NULL there: without).   */
+ * Images (ndim 2): depth and out_d are ignored.  Takes the workspace together with its size: no access beyond
+ * `workspace_bytes`, and a path that wants more than that is left for one that does not.  16-bit tensors need
+ * mv_roi_align_backward_workspace_bytes(), as for the others; with mv_roi_align_backward_write_workspace_bytes() bytes
+ * every path can run (fp32 volumes summed channels-last, rotated boxes by the voxels' owners).
+ * mv_roi_align_backward_write: the same without the size, which it takes to be that of
+ * mv_roi_align_backward_workspace_bytes().                                                                      */
+int mv_roi_align_backward_replace(const void *grad_output, const void *rois, void *grad_input, int dtype, int ndim,
+                                  int rotated, int batch, int channels, int depth, int height, int width, int num_rois,
+                                  int out_d, int out_h, int out_w, float spatial_scale, int sampling_ratio, int aligned,
+                                  int order, void *workspace, size_t workspace_bytes, void *stream);
 int mv_roi_align_backward_write(const void *grad_output, const void *rois, void *grad_input, int dtype, int ndim,
                                 int rotated, int batch, int channels, int depth, int height, int width, int num_rois,
                                 int out_d, int out_h, int out_w, float spatial_scale, int sampling_ratio, int aligned,

@@ -48,6 +48,7 @@ SIGNATURES = {
     "mv_roi_align_rotated_2d_backward": (_i, [_p, _p, _p, _i] + [_i] * 7 + [_f, _i, _i, _i, _p, _p]),
     "mv_roi_align_rotated_3d_forward": (_i, [_p, _p, _p, _i] + [_i] * 9 + [_f, _i, _i, _i, _p, _sz, _p]),
     "mv_roi_align_rotated_3d_backward": (_i, [_p, _p, _p, _i] + [_i] * 9 + [_f, _i, _i, _i, _p, _p]),
+    "mv_roi_align_backward_replace": (_i, [_p, _p, _p] + [_i] * 12 + [_f, _i, _i, _i, _p, _sz, _p]),
     "mv_roi_align_backward_write": (_i, [_p, _p, _p] + [_i] * 12 + [_f, _i, _i, _i, _p, _p]),
     "mv_roi_align_backward_write_workspace_bytes": (_sz, [_i] * 14),
     "mv_roi_align_backward_workspace_bytes": (_sz, [_i] * 6),

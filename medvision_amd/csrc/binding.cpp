@@ -193,11 +193,12 @@ Tensor roi_backward(const RoiCall &c, const Tensor &grad_output, const Tensor &r
   const auto d = five_dims(feature_size, c.ndim);
   const int n = static_cast<int>(rois.size(0));
   const Tensor grad_input = at::empty(feature_size, g.options());
-  const Tensor ws = bytes_on(g, mv_roi_align_backward_write_workspace_bytes(code, c.ndim, c.kind == kRotated, d[0], d[1], d[2], d[3], d[4], n,
-                                                                            c.out[0], c.out[1], c.out[2], c.ratio, c.order));
-  check(mv_roi_align_backward_write(ptr(g), ptr(rois), ptr(grad_input), code, c.ndim, c.kind == kRotated, d[0], d[1], d[2],
-                                    d[3], d[4], n, c.out[0], c.out[1], c.out[2], c.scale, c.ratio, c.aligned, c.order,
-                                    ptr(ws), stream_of(g)));
+  const size_t bytes = mv_roi_align_backward_write_workspace_bytes(code, c.ndim, c.kind == kRotated, d[0], d[1], d[2], d[3], d[4], n,
+                                                                   c.out[0], c.out[1], c.out[2], c.ratio, c.order);
+  const Tensor ws = bytes_on(g, bytes);
+  check(mv_roi_align_backward_replace(ptr(g), ptr(rois), ptr(grad_input), code, c.ndim, c.kind == kRotated, d[0], d[1], d[2],
+                                      d[3], d[4], n, c.out[0], c.out[1], c.out[2], c.scale, c.ratio, c.aligned, c.order,
+                                      ptr(ws), bytes, stream_of(g)));
   return grad_input;
 }
 

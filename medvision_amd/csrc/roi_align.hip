@@ -178,7 +178,7 @@ int roi_plane_backward(const void *grad_output, const void *rois, void *grad, fl
 bool roi_own_applies(int dtype, const RoiProblem &p);
 size_t roi_own_workspace(int dtype, const RoiProblem &p);
 int roi_own_backward(const void *grad_output, const void *rois, void *grad_input, int dtype, const RoiProblem &p, void *workspace,
-                     hipStream_t s);
+                     size_t capacity, hipStream_t s);
 int roi_box_backward(const void *grad_output, const void *rois, float *acc, int dtype, const RoiProblem &p, hipStream_t s);
 // Many small outputs over wide feature maps, read from a channels-last copy in the workspace (roi_cl.hip).
 size_t roi_forward_cl_workspace(int dtype, const RoiProblem &p);
@@ -290,11 +290,12 @@ static bool roi_backward_wants_sums(int dtype, const RoiProblem &p) {
 }
 
 // `accumulate`: the gradient is added to what grad_input holds; otherwise it replaces it (a path that writes every voxel
-// then neither reads nor clears it; the others clear it first)
+// then neither reads nor clears it; the others clear it first).  A path that wants more than the workspace's `capacity` is
+// left alone.
 int roi_backward(const void *grad_output, const void *rois, void *grad_input, int dtype, int ndim,
                  int rotated, int batch, int channels, int depth, int height, int width,
                  int num_rois, int out_d, int out_h, int out_w, float spatial_scale,
-                 int sampling_ratio, int aligned, int order, void *workspace, void *stream, bool accumulate) {
+                 int sampling_ratio, int aligned, int order, void *workspace, size_t capacity, void *stream, bool accumulate) {
   RoiProblem p;
   int st = make_problem(p, ndim, rotated, batch, channels, depth, height, width, num_rois, out_d,
                         out_h, out_w, spatial_scale, sampling_ratio, aligned, order);
@@ -309,9 +310,11 @@ int roi_backward(const void *grad_output, const void *rois, void *grad_input, in
     return clear_gradient();
   }
   MV_REQUIRE(grad_output && rois && grad_input, "null pointer argument");
-  // (fp32: the workspace is there when the caller asked for its size, see roi_backward_wants_sums)
-  const bool narrow = dtype == MV_F16 || dtype == MV_BF16 || (workspace && roi_backward_wants_sums(dtype, p));
-  MV_REQUIRE(dtype == MV_F32 || dtype == MV_F64 || workspace, "16-bit backward needs an fp32 workspace");
+  if (!workspace) capacity = 0;
+  const bool holds_sums = capacity >= static_cast<size_t>(total) * sizeof(float);
+  const bool narrow = dtype == MV_F16 || dtype == MV_BF16 || (holds_sums && roi_backward_wants_sums(dtype, p));
+  MV_REQUIRE(dtype == MV_F32 || dtype == MV_F64 || holds_sums,
+             "16-bit backward needs an fp32 workspace (mv_roi_align_backward_workspace_bytes)");
   float *const ws = static_cast<float *>(workspace);
   // sums that several workgroups add to: the fp32 workspace of 16-bit tensors (folded into the gradient afterwards), the
   // gradient itself otherwise
@@ -337,9 +340,9 @@ int roi_backward(const void *grad_output, const void *rois, void *grad_input, in
     st = roi_plane_backward(grad_output, rois, grad_input, static_cast<float *>(sums), dtype, p, parts, accumulate, s);
     if (st >= 0) return st || parts == 1 ? st : fold_sums();
   }
-  // (a gradient to be added to keeps the kernel with atomics, and so does an fp32 one without a workspace)
-  if (!accumulate && workspace && !roi_pool_applies(dtype, p)) {
-    st = roi_own_backward(grad_output, rois, grad_input, dtype, p, workspace, s);
+  // (a gradient to be added to keeps the kernel with atomics, and so does one without the workspace)
+  if (!accumulate && !roi_pool_applies(dtype, p)) {
+    st = roi_own_backward(grad_output, rois, grad_input, dtype, p, workspace, capacity, s);
     if (st >= 0) return st;
   }
   st = clear_sums();
@@ -424,15 +427,26 @@ int mv_roi_align_forward_prepared(const void *input, const void *prepared, const
                      workspace, workspace_bytes, stream, false, prepared);
 }
 
-int mv_roi_align_backward_write(const void *grad_output, const void *rois, void *grad_input, int dtype, int ndim,
-                                int rotated, int batch, int channels, int depth, int height, int width, int num_rois,
-                                int out_d, int out_h, int out_w, float spatial_scale, int sampling_ratio, int aligned,
-                                int order, void *workspace, void *stream) {
+int mv_roi_align_backward_replace(const void *grad_output, const void *rois, void *grad_input, int dtype, int ndim,
+                                  int rotated, int batch, int channels, int depth, int height, int width, int num_rois,
+                                  int out_d, int out_h, int out_w, float spatial_scale, int sampling_ratio, int aligned,
+                                  int order, void *workspace, size_t workspace_bytes, void *stream) {
   MV_REQUIRE(ndim == 2 || ndim == 3, "ndim must be 2 or 3");
   const bool flat = ndim == 2;
   return roi_backward(grad_output, rois, grad_input, dtype, ndim, rotated ? 1 : 0, batch, channels, flat ? 1 : depth, height,
                       width, num_rois, flat ? 1 : out_d, out_h, out_w, spatial_scale, sampling_ratio,
-                      rotated ? aligned : 1, order, workspace, stream, false);
+                      rotated ? aligned : 1, order, workspace, workspace_bytes, stream, false);
+}
+
+int mv_roi_align_backward_write(const void *grad_output, const void *rois, void *grad_input, int dtype, int ndim,
+                                int rotated, int batch, int channels, int depth, int height, int width, int num_rois,
+                                int out_d, int out_h, int out_w, float spatial_scale, int sampling_ratio, int aligned,
+                                int order, void *workspace, void *stream) {
+  // (the size is not known: no more than what every backward entry point may ask for)
+  return mv_roi_align_backward_replace(grad_output, rois, grad_input, dtype, ndim, rotated, batch, channels, depth, height, width,
+                                       num_rois, out_d, out_h, out_w, spatial_scale, sampling_ratio, aligned, order, workspace,
+                                       mv_roi_align_backward_workspace_bytes(dtype, batch, channels, ndim == 2 ? 1 : depth, height, width),
+                                       stream);
 }
 
 int mv_roi_align_2d_backward(const void *grad_output, const void *rois, void *grad_input,
@@ -440,8 +454,8 @@ int mv_roi_align_2d_backward(const void *grad_output, const void *rois, void *gr
                              int num_rois, int out_h, int out_w, float spatial_scale,
                              int sampling_ratio, int order, void *workspace, void *stream) {
   return roi_backward(grad_output, rois, grad_input, dtype, 2, 0, batch, channels, 1, height,
-                      width, num_rois, 1, out_h, out_w, spatial_scale, sampling_ratio, 1, order,
-                      dtype == MV_F32 ? nullptr : workspace, stream, true);
+                      width, num_rois, 1, out_h, out_w, spatial_scale, sampling_ratio, 1, order, workspace,
+                      mv_roi_align_backward_workspace_bytes(dtype, batch, channels, 1, height, width), stream, true);
 }
 
 int mv_roi_align_3d_forward(const void *input, const void *rois, void *output, int dtype,
@@ -458,8 +472,8 @@ int mv_roi_align_3d_backward(const void *grad_output, const void *rois, void *gr
                              int num_rois, int out_d, int out_h, int out_w, float spatial_scale,
                              int sampling_ratio, int order, void *workspace, void *stream) {
   return roi_backward(grad_output, rois, grad_input, dtype, 3, 0, batch, channels, depth, height,
-                      width, num_rois, out_d, out_h, out_w, spatial_scale, sampling_ratio, 1,
-                      order, dtype == MV_F32 ? nullptr : workspace, stream, true);
+                      width, num_rois, out_d, out_h, out_w, spatial_scale, sampling_ratio, 1, order, workspace,
+                      mv_roi_align_backward_workspace_bytes(dtype, batch, channels, depth, height, width), stream, true);
 }
 
 int mv_roi_align_rotated_2d_forward(const void *input, const void *rois, void *output, int dtype,
@@ -477,8 +491,8 @@ int mv_roi_align_rotated_2d_backward(const void *grad_output, const void *rois, 
                                      int sampling_ratio, int aligned, int order, void *workspace,
                                      void *stream) {
   return roi_backward(grad_output, rois, grad_input, dtype, 2, 1, batch, channels, 1, height,
-                      width, num_rois, 1, out_h, out_w, spatial_scale, sampling_ratio, aligned,
-                      order, dtype == MV_F32 ? nullptr : workspace, stream, true);
+                      width, num_rois, 1, out_h, out_w, spatial_scale, sampling_ratio, aligned, order, workspace,
+                      mv_roi_align_backward_workspace_bytes(dtype, batch, channels, 1, height, width), stream, true);
 }
 
 int mv_roi_align_rotated_3d_forward(const void *input, const void *rois, void *output, int dtype,
@@ -498,8 +512,8 @@ int mv_roi_align_rotated_3d_backward(const void *grad_output, const void *rois, 
                                      float spatial_scale, int sampling_ratio, int aligned,
                                      int order, void *workspace, void *stream) {
   return roi_backward(grad_output, rois, grad_input, dtype, 3, 1, batch, channels, depth, height,
-                      width, num_rois, out_d, out_h, out_w, spatial_scale, sampling_ratio, aligned,
-                      order, dtype == MV_F32 ? nullptr : workspace, stream, true);
+                      width, num_rois, out_d, out_h, out_w, spatial_scale, sampling_ratio, aligned, order, workspace,
+                      mv_roi_align_backward_workspace_bytes(dtype, batch, channels, depth, height, width), stream, true);
 }
 
 size_t mv_roi_align_forward_workspace_bytes(int dtype, int ndim, int channels, int num_rois,

@@ -703,10 +703,10 @@ size_t roi_own_workspace(int dtype, const RoiProblem &p) {
   return roi_own_applies(dtype, p) ? own_copy_bytes(dtype, p) + own_partial_bytes(p) + static_cast<size_t>(p.R) * kOwnRoiBytes : 0;
 }
 
-// Writes all of grad_input.  -1: not for these kernels.
+// Writes all of grad_input.  -1: not for these kernels, or a workspace that is too small for them.
 int roi_own_backward(const void *grad_output, const void *rois, void *grad_input, int dtype, const RoiProblem &p, void *workspace,
-                     hipStream_t s) {
-  if (!roi_own_applies(dtype, p)) return -1;
+                     size_t capacity, hipStream_t s) {
+  if (!roi_own_applies(dtype, p) || capacity < roi_own_workspace(dtype, p)) return -1;
   const int es = static_cast<int>(dtype_size(dtype));
   char *const after = static_cast<char *>(workspace) + own_copy_bytes(dtype, p);
   float *const partial = reinterpret_cast<float *>(after);

@@ -94,3 +94,36 @@ def test_cells_of_many_samples(oracle, size, cells, ratio, reach):
     want = oracle.roi_align_backward(gy, boxes, x.shape, 1.0, ratio, True, 1, True)
     error = float((x.grad.cpu().double() - want).norm() / want.norm())
     assert error < 1e-6, error
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("rotated", [False, True])
+@pytest.mark.parametrize("sized", [False, True])
+def test_backward_keeps_to_its_workspace(oracle, dtype, rotated, sized):
+    """The entry points that replace the gradient stay within the workspace they are told of (`sized`), or within the size of the
+    query that all backward entry points share: the paths that want more, the owners' and the channels-last sums, are left."""
+    from medvision_amd import _lib
+    lib, code = _lib.load(), _lib.MV_F16 if dtype == torch.float16 else _lib.MV_F32
+    g = wl.gen(3 + rotated)
+    dims, rois, cells = (2, 64, 9, 11, 13), 60, 7
+    at = torch.rand(rois, 3, generator=g) * torch.tensor(dims[:1:-1])
+    image = torch.randint(0, 2, (rois, 1), generator=g).float()
+    extent = torch.rand(rois, 3, generator=g) * 8 + 1
+    boxes = torch.cat([image, at, extent, torch.rand(rois, 3, generator=g)], 1) if rotated else torch.cat([image, at, at + extent], 1)
+    gy = torch.randn(rois, dims[1], cells, cells, cells, generator=g).to(dtype)
+    want = oracle.roi_align_backward(gy, boxes, dims, 1.0, 2, True, 1, rotated)
+    size = (code, 3, int(rotated), *dims, rois, cells, cells, cells, 2, 1)
+    full, shared = lib.mv_roi_align_backward_write_workspace_bytes(*size), lib.mv_roi_align_backward_workspace_bytes(code, *dims)
+    assert full > shared or (dtype == torch.float16 and not rotated)
+    grad, d_gy, d_rois = torch.full(dims, 7.0, dtype=dtype, device=DEV), gy.to(DEV), boxes.to(DEV)
+    for given in (shared, full) if sized else (shared,):
+        room = torch.full((full + 4096,), 0x5a, dtype=torch.uint8, device=DEV)
+        call = (lib.mv_roi_align_backward_replace if sized else lib.mv_roi_align_backward_write)
+        _lib.check(call(_lib.ptr(d_gy), _lib.ptr(d_rois), _lib.ptr(grad), code, 3, int(rotated), *dims, rois, cells, cells, cells,
+                        1.0, 2, 1, 1, _lib.ptr(room), *([given] if sized else []), _lib.stream_of(grad)))
+        assert bool((room[given:] == 0x5a).all())
+        assert_close(grad, want, BWD_TOL[dtype], f"{given} bytes")
+    if dtype == torch.float16 and sized:
+        with pytest.raises(RuntimeError, match="workspace"):
+            _lib.check(call(_lib.ptr(d_gy), _lib.ptr(d_rois), _lib.ptr(grad), code, 3, int(rotated), *dims, rois, cells, cells, cells,
+                            1.0, 2, 1, 1, _lib.ptr(room), shared - 4, _lib.stream_of(grad)))
