@@ -536,8 +536,9 @@ size_t mv_roi_align_forward_workspace_bytes_for_input(int dtype, int ndim, int b
   p.od = ndim == 2 ? 1 : out_d; p.oh = out_h; p.ow = out_w; p.sampling_ratio = sampling_ratio; p.order = 1;
   if (batch <= 0 || channels <= 0 || p.D <= 0 || height <= 0 || width <= 0 || num_rois <= 0) return basic;
   if (basic || dtype == MV_I32) return basic;   // (the tiled resampler takes the problem; label maps have no other path that wants memory)
-  const size_t pooled = std::max(mv::roi_pool_forward_workspace(dtype, p), mv::roi_plane_forward_workspace(dtype, p));
-  return pooled ? pooled : mv::roi_forward_cl_workspace(dtype, p);
+  // (the query is not told whether the rois are rotated: plain ones take the image kernels, rotated ones the channels-last copy)
+  const size_t pooled = mv::roi_pool_forward_workspace(dtype, p), copy = mv::roi_forward_cl_workspace(dtype, p);
+  return pooled ? pooled : std::max(mv::roi_plane_forward_workspace(dtype, p), copy);
 }
 
 size_t mv_roi_align_backward_write_workspace_bytes(int dtype, int ndim, int rotated, int batch, int channels, int depth,

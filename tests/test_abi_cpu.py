@@ -47,6 +47,18 @@ def test_workspace_queries_and_dims_need_no_gpu():
     assert b"must divide group" in lib.mv_last_error()
 
 
+def test_rotated_image_heads_get_room_for_the_channels_last_copy():
+    """The forward query is not told whether the rois are rotated: what plain heads on images want (an order of the rois) must not
+    take the place of the copy that rotated ones read."""
+    from medvision_amd import _lib
+    lib = _lib.load()
+    for code, size in ((_lib.MV_F32, 4), (_lib.MV_BF16, 2), (_lib.MV_F16, 2)):
+        for rois in (100, 1000):
+            need = lib.mv_roi_align_forward_workspace_bytes_for_input(code, 2, 2, 64, 1, 64, 100, rois, 1, 14, 14, 2)
+            assert need >= 2 * 64 * 64 * 100 * size
+    assert lib.mv_roi_align_forward_workspace_bytes_for_input(_lib.MV_F32, 2, 2, 256, 1, 200, 304, 1000, 1, 7, 7, 2) >= 2 * 256 * 200 * 304 * 4
+
+
 def test_host_shim_rejects_cpu_tensors_and_bad_rois():
     import medvision_amd.ops as ops
     feat = torch.randn(1, 2, 4, 5, 6)
