@@ -139,7 +139,7 @@ size_t mv_roi_align_forward_workspace_bytes_for_input(int dtype, int ndim, int b
 /* Detection heads that pool ONE feature map several times (cascade stages, several batches of rois):
  * the re-ordered copy that mv_roi_align_2d_forward / _3d_forward make in their workspace on every call
  * (fp16 features whose width is a multiple of four) can be made once and handed in.
- * mv_roi_align_prepared_bytes: size of that copy, 0 when the forward pass has no use for one.
+ * mv_roi_align_prepared_bytes: size of that copy, 0 when the forward pass has no use for one (images).
  * mv_roi_align_prepare_features: writes it (8-byte aligned pointers; an error when the size is 0 or
  * `prepared_bytes` is smaller).  mv_roi_align_forward_prepared: mv_roi_align_{2,3}d_forward (plain
  * rois; replaces the same reference functions) reading `prepared`, which must have been written from

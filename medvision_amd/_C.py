@@ -110,7 +110,7 @@ def _roi_forward(fn_name, what, ndim, cols, input, rois, output, out_sizes, spat
 def roi_align_prepare(features):
     """The re-ordered copy of ``features`` that the RoIAlign forward of detection heads reads (made by
     every call in its workspace otherwise), for callers that pool one feature map several times; None
-    when the forward pass has no use for one (other than fp16, width no multiple of four).  No
+    when the forward pass has no use for one (images, other than fp16, width no multiple of four).  No
     counterpart in the reference.  Pass it as ``prepared`` to ``roi_align_{2,3}d_forward`` together with
     the same, unchanged features."""
     _require_cuda(features, "RoIAlign")

@@ -166,6 +166,7 @@ int roi_pool_backward(const void *grad_output, const void *rois, void *acc, int 
                       const RoiProblem &p, hipStream_t s, bool channels_last);
 bool roi_pool_applies(int dtype, const RoiProblem &p);
 // roi_plane.hip: heads on images with plain boxes; -1 (0 parts): not for this problem
+bool roi_plane_applies(int dtype, const RoiProblem &p);
 size_t roi_plane_forward_workspace(int dtype, const RoiProblem &p);
 int roi_plane_forward(const void *input, const void *rois, void *output, int dtype, const RoiProblem &p, void *workspace,
                       size_t capacity, hipStream_t s);
@@ -248,7 +249,7 @@ int roi_forward(const void *input, const void *rois, void *output, int dtype, in
   {
     // (a workspace too small for a path selects the kernels that need none)
     const size_t capacity = workspace ? workspace_bytes : 0;
-    if (prepared != nullptr && p.ndim == 3) {   // (a copy the pooled kernels have no use for is left alone)
+    if (prepared != nullptr) {   // (a copy the pooled kernels have no use for is left alone)
       const int pooled = roi_pool_forward(input, rois, output, dtype, p, workspace, capacity, s, prepared);
       if (pooled >= 0) return pooled;
     }
@@ -394,9 +395,9 @@ int mv_roi_align_2d_forward(const void *input, const void *rois, void *output, i
 }
 
 size_t mv_roi_align_prepared_bytes(int dtype, int ndim, int batch, int channels, int depth, int height, int width) {
-  if ((ndim != 2 && ndim != 3) || batch <= 0 || channels <= 0 || depth <= 0 || height <= 0 || width <= 0) return 0;
+  if (ndim != 3 || batch <= 0 || channels <= 0 || depth <= 0 || height <= 0 || width <= 0) return 0;   // (heads on images read their features as they are)
   mv::RoiProblem p{};
-  p.ndim = ndim; p.N = batch; p.C = channels; p.D = ndim == 2 ? 1 : depth; p.H = height; p.W = width;
+  p.ndim = ndim; p.N = batch; p.C = channels; p.D = depth; p.H = height; p.W = width;
   return mv::roi_pool_prepared_bytes(dtype, p);
 }
 
@@ -407,8 +408,8 @@ int mv_roi_align_prepare_features(const void *input, int dtype, int ndim, int ba
              "feature dims must be positive (got %d,%d,%d,%d,%d)", batch, channels, depth, height, width);
   MV_REQUIRE(input && prepared, "null pointer argument");
   mv::RoiProblem p{};
-  p.ndim = ndim; p.N = batch; p.C = channels; p.D = ndim == 2 ? 1 : depth; p.H = height; p.W = width;
-  const size_t bytes = mv::roi_pool_prepared_bytes(dtype, p);
+  p.ndim = ndim; p.N = batch; p.C = channels; p.D = depth; p.H = height; p.W = width;
+  const size_t bytes = mv_roi_align_prepared_bytes(dtype, ndim, batch, channels, depth, height, width);
   MV_REQUIRE(bytes > 0, "no prepared copy for these features (mv_roi_align_prepared_bytes is 0)");
   MV_REQUIRE(prepared_bytes >= bytes, "prepared buffer too small");
   MV_REQUIRE(reinterpret_cast<uintptr_t>(input) % 8 == 0 && reinterpret_cast<uintptr_t>(prepared) % 8 == 0,
@@ -424,7 +425,7 @@ int mv_roi_align_forward_prepared(const void *input, const void *prepared, const
   MV_REQUIRE(ndim == 2 || ndim == 3, "ndim must be 2 or 3");
   return roi_forward(input, rois, output, dtype, ndim, 0, batch, channels, ndim == 2 ? 1 : depth, height, width,
                      num_rois, ndim == 2 ? 1 : out_d, out_h, out_w, spatial_scale, sampling_ratio, 1, order,
-                     workspace, workspace_bytes, stream, false, prepared);
+                     workspace, workspace_bytes, stream, false, ndim == 3 ? prepared : nullptr);
 }
 
 int mv_roi_align_backward_replace(const void *grad_output, const void *rois, void *grad_input, int dtype, int ndim,
@@ -537,7 +538,9 @@ size_t mv_roi_align_forward_workspace_bytes_for_input(int dtype, int ndim, int b
   if (batch <= 0 || channels <= 0 || p.D <= 0 || height <= 0 || width <= 0 || num_rois <= 0) return basic;
   if (basic || dtype == MV_I32) return basic;   // (the tiled resampler takes the problem; label maps have no other path that wants memory)
   // (the query is not told whether the rois are rotated: plain ones take the image kernels, rotated ones the channels-last copy)
-  const size_t pooled = mv::roi_pool_forward_workspace(dtype, p), copy = mv::roi_forward_cl_workspace(dtype, p);
+  // (images of at least four cells never reach the kernels that read the re-ordered copy)
+  const size_t pooled = mv::roi_plane_applies(dtype, p) ? 0 : mv::roi_pool_forward_workspace(dtype, p);
+  const size_t copy = mv::roi_forward_cl_workspace(dtype, p);
   return pooled ? pooled : std::max(mv::roi_plane_forward_workspace(dtype, p), copy);
 }
 

@@ -602,7 +602,7 @@ __global__ __launch_bounds__(kPlaneThreads, CELLS == 8 ? 4 : 2) void roi_plane_b
   }
 }
 
-static bool plane_applies(int dtype, const RoiProblem &p) {
+bool roi_plane_applies(int dtype, const RoiProblem &p) {
   return p.ndim == 2 && !p.rotated && p.oh * p.ow >= 4 && (p.order == 0 || p.order == 1) && p.oh <= 16 && p.ow <= 16 && p.R > 0 &&
          (dtype == MV_F32 || dtype == MV_F16 || dtype == MV_BF16) && static_cast<long>(p.H) * p.W < (1L << 25);
 }
@@ -611,7 +611,7 @@ static bool plane_small(const RoiProblem &p) { return p.oh <= 8 && p.ow <= 8; }
 // Bytes of workspace that the forward pass can make use of: four per roi where ordering them pays for the ~7 us it takes
 // (features well beyond an L2, enough rois).
 size_t roi_plane_forward_workspace(int dtype, const RoiProblem &p) {
-  if (!plane_applies(dtype, p) || p.R < 256 || p.R > kPlaneOrderMax || p.N > kPlaneBuckets / kPlaneSizes) return 0;
+  if (!roi_plane_applies(dtype, p) || p.R < 256 || p.R > kPlaneOrderMax || p.N > kPlaneBuckets / kPlaneSizes) return 0;
   const long bytes = static_cast<long>(p.N) * p.C * p.H * p.W * static_cast<long>(dtype_size(dtype));
   return bytes >= (16L << 20) ? static_cast<size_t>(p.R) * 4 : 0;
 }
@@ -619,7 +619,7 @@ size_t roi_plane_forward_workspace(int dtype, const RoiProblem &p) {
 // -1: not for this problem
 int roi_plane_forward(const void *input, const void *rois, void *output, int dtype, const RoiProblem &p, void *workspace,
                       size_t capacity, hipStream_t s) {
-  if (!plane_applies(dtype, p)) return -1;
+  if (!roi_plane_applies(dtype, p)) return -1;
   unsigned *order = nullptr;
   const size_t need = roi_plane_forward_workspace(dtype, p);
   if (need > 0 && workspace != nullptr && capacity >= need && reinterpret_cast<uintptr_t>(workspace) % 4 == 0) {
@@ -657,7 +657,7 @@ static int plane_channels(const RoiProblem &p) { return 8; }   // per wavefront 
 
 // Workgroups that share a tile's rois: 1 while the tiles and channels alone fill the chip (0: not for this problem).
 int roi_plane_backward_parts(int dtype, const RoiProblem &p) {
-  if (!plane_applies(dtype, p)) return 0;
+  if (!roi_plane_applies(dtype, p)) return 0;
   const int ch = plane_channels(p) * kPlaneWaves;
   const long groups = static_cast<long>(p.N) * ((p.W + kPlaneTile - 1) / kPlaneTile) * ((p.H + kPlaneTile - 1) / kPlaneTile) *
                       ((p.C + ch - 1) / ch);

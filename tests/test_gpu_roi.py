@@ -617,7 +617,8 @@ def test_pooled_forward_from_blocked_copy(ops, oracle, ndim):
     out3 = out if ndim == 3 else (1, *out)
     in3 = size if ndim == 3 else (1, *size)
     need = _lib.load().mv_roi_align_forward_workspace_bytes_for_input(_lib.MV_F16, ndim, 2, channels, *in3, n, *out3, 2)
-    assert need == feat.numel() * 2 + 4 * n     # the copy (and the launch order of the rois) is in use
+    # volumes: the copy (and the launch order of the rois) is in use; images are read as they are
+    assert need == (feat.numel() * 2 + 4 * n if ndim == 3 else 0)
     got = ops.RoIAlign(out, 1.0, 2)(feat.to(DEV), rois.to(DEV))
     want = oracle.roi_align_forward(feat, rois, out, 1.0, 2)
     assert_close(got, want, FWD_TOL[torch.float16], "pooled forward from the blocked copy")
@@ -626,7 +627,7 @@ def test_pooled_forward_from_blocked_copy(ops, oracle, ndim):
     # made for them inside a call); gradients reach the features
     x = feat.to(DEV).requires_grad_(True)
     kept = ops.PreparedFeatures(x)
-    assert kept.copy is not None and kept.copy.numel() == feat.numel() * 2
+    assert kept.copy.numel() == feat.numel() * 2 if ndim == 3 else kept.copy is None
     again = ops.RoIAlign(out, 1.0, 2)(kept, rois.to(DEV))
     assert torch.equal(again, got)
     few = ops.RoIAlign(out, 1.0, 2)(kept, rois[:5].to(DEV))
