@@ -530,13 +530,15 @@ size_t mv_roi_align_forward_workspace_bytes(int dtype, int ndim, int channels, i
 size_t mv_roi_align_forward_workspace_bytes_for_input(int dtype, int ndim, int batch, int channels, int depth,
                                                       int height, int width, int num_rois, int out_d,
                                                       int out_h, int out_w, int sampling_ratio) {
-  const size_t basic = mv_roi_align_forward_workspace_bytes(dtype, ndim, channels, num_rois, out_d, out_h, out_w,
-                                                            sampling_ratio);
   mv::RoiProblem p = {};
   p.ndim = ndim; p.N = batch; p.C = channels; p.D = ndim == 2 ? 1 : depth; p.H = height; p.W = width; p.R = num_rois;
   p.od = ndim == 2 ? 1 : out_d; p.oh = out_h; p.ow = out_w; p.sampling_ratio = sampling_ratio; p.order = 1;
-  if (batch <= 0 || channels <= 0 || p.D <= 0 || height <= 0 || width <= 0 || num_rois <= 0) return basic;
-  if (basic || dtype == MV_I32) return basic;   // (the tiled resampler takes the problem; label maps have no other path that wants memory)
+  size_t tiled = 0;
+  const bool resampled = mv::roi_forward_tiled(nullptr, nullptr, nullptr, dtype, p, nullptr, 0, &tiled, nullptr) == MV_OK;
+  if (!resampled) tiled = 0;
+  if (batch <= 0 || channels <= 0 || p.D <= 0 || height <= 0 || width <= 0 || num_rois <= 0) return tiled;
+  // (the tiled resampler takes the problem; label maps have no other path that wants memory)
+  if (tiled || dtype == MV_I32 || (resampled && ndim == 2)) return tiled;
   // (the query is not told whether the rois are rotated: plain ones take the image kernels, rotated ones the channels-last copy)
   // (images of at least four cells never reach the kernels that read the re-ordered copy)
   const size_t pooled = mv::roi_plane_applies(dtype, p) ? 0 : mv::roi_pool_forward_workspace(dtype, p);

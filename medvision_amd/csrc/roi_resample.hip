@@ -1719,8 +1719,6 @@ static int roi_forward_tiled_image(const void *input, const void *rois, void *ou
   if (pool == 0 && !need && p.order == 3) return -1;
   if (vox * 4 >= (1L << 31)) return -1;
   if (dtype != MV_F16 && dtype != MV_BF16 && dtype != MV_F32 && !(dtype == MV_I32 && pool == 1)) return -1;
-  // (no kernel here uses a workspace any more; callers that size one by the query keep getting the same answer)
-  const size_t bytes = (static_cast<size_t>(p.R) * 10 * sizeof(float) + 255) / 256 * 256;
   RoiProblem v = p;
   v.ndim = 3;
   v.D = p.H; v.H = 1; v.W = p.W;
@@ -1742,7 +1740,6 @@ static int roi_forward_tiled_image(const void *input, const void *rois, void *ou
         st = launch_resample<float, 64, 1, 64, 512, 74 * 1024, 6, true>(static_cast<const float *>(input), vol_rois,
                                                                          static_cast<float *>(output), v, need, s);
     }
-    if (need && st == MV_OK) *need = bytes;
     return st;
   }
   if (pool == 0) {
@@ -1759,7 +1756,6 @@ static int roi_forward_tiled_image(const void *input, const void *rois, void *ou
         st = launch_resample<float, 64, 1, 32, 512, 74 * 1024, 6, false, 0>(static_cast<const float *>(input), vol_rois,
                                                                              static_cast<float *>(output), v, need, s);
     }
-    if (need && st == MV_OK) *need = bytes;
     return st;
   }
   if (pool != 1) {
@@ -1772,7 +1768,6 @@ static int roi_forward_tiled_image(const void *input, const void *rois, void *ou
       default: st = pool == 2 ? MV_IMAGE_MEANS(float, 32, 6, 2) : MV_IMAGE_MEANS(float, 32, 6, 4);
     }
 #undef MV_IMAGE_MEANS
-    if (need && st == MV_OK) *need = bytes;
     return st;
   }
   switch (dtype) {
@@ -1792,7 +1787,6 @@ static int roi_forward_tiled_image(const void *input, const void *rois, void *ou
       st = launch_resample<float, 64, 1, 32, 512, 74 * 1024, 6>(static_cast<const float *>(input), vol_rois,
                                                                  static_cast<float *>(output), v, need, s);
   }
-  if (need && st == MV_OK) *need = bytes;
   return st;
 }
 

@@ -59,6 +59,15 @@ def test_rotated_image_heads_get_room_for_the_channels_last_copy():
     assert lib.mv_roi_align_forward_workspace_bytes_for_input(_lib.MV_F32, 2, 2, 256, 1, 200, 304, 1000, 1, 7, 7, 2) >= 2 * 256 * 200 * 304 * 4
 
 
+def test_resampled_images_need_no_workspace():
+    """Images of resampling size keep their state in LDS: no tensor is allocated per call."""
+    from medvision_amd import _lib
+    lib = _lib.load()
+    for code in (_lib.MV_F32, _lib.MV_F16, _lib.MV_BF16, _lib.MV_I32):
+        assert lib.mv_roi_align_forward_workspace_bytes(code, 2, 3, 8, 1, 512, 512, 1) == 0
+        assert lib.mv_roi_align_forward_workspace_bytes_for_input(code, 2, 8, 16, 1, 512, 512, 8, 1, 512, 512, 1) == 0
+
+
 def test_host_shim_rejects_cpu_tensors_and_bad_rois():
     import medvision_amd.ops as ops
     feat = torch.randn(1, 2, 4, 5, 6)
