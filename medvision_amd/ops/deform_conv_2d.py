@@ -9,20 +9,41 @@ import math
 
 import torch
 from torch import nn
+from torch.autograd.function import once_differentiable
 from torch.nn import init
 from torch.nn.modules.utils import _pair
 
+from .. import _C
 from .._lib import native
+from ._function import NativeFunction
 
 
-class DeformConv2dFunction:
+class DeformConv2dFunction(NativeFunction):
     @staticmethod
-    def apply(input, offset, weight, bias, stride, padding, dilation, group, deformable_groups, im2col_step):
+    def native(input, offset, weight, bias, stride, padding, dilation, group, deformable_groups, im2col_step):
         return native.deform_conv(2, input, offset, weight, bias, stride, padding, dilation, group, deformable_groups,
                                   im2col_step)
 
+    @staticmethod
+    def forward(ctx, input, offset, weight, bias, stride, padding, dilation, group,
+                deformable_groups, im2col_step):
+        ctx.geometry = (*weight.shape[2:4], *_pair(stride), *_pair(padding), *_pair(dilation),
+                        group, deformable_groups, im2col_step)
+        if offset.dtype in (torch.float16, torch.bfloat16):   # autocast: follow the offset branch
+            input, bias, weight = input.to(offset.dtype), bias.to(offset.dtype), weight.to(offset.dtype)
+        output = _C.deform_conv_2d_forward(input, weight, bias, offset, *ctx.geometry)
+        ctx.save_for_backward(input, offset, weight, bias)
+        return output
 
-deform_conv = DeformConv2dFunction.apply
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad_output):
+        input, offset, weight, bias = ctx.saved_tensors
+        grads = _C.deform_conv_2d_backward(input, weight, bias, offset, grad_output, *ctx.geometry)
+        return (*grads, None, None, None, None, None, None)
+
+
+deform_conv = DeformConv2dFunction.native
 
 
 class DeformConv2d(nn.Module):

@@ -8,20 +8,46 @@ import math
 
 import torch
 from torch import nn
+from torch.autograd.function import once_differentiable
 from torch.nn import init
 from torch.nn.modules.utils import _triple
 
+from .. import _C
 from .._lib import native
+from ._function import NativeFunction
 
 
-class DeformConv3dFunction:
+class DeformConv3dFunction(NativeFunction):
     @staticmethod
-    def apply(input, offset, weight, bias, stride, padding, dilation, group, deformable_groups, im2col_step):
+    def native(input, offset, weight, bias, stride, padding, dilation, group, deformable_groups, im2col_step):
         return native.deform_conv(3, input, offset, weight, bias, stride, padding, dilation, group, deformable_groups,
                                   im2col_step)
 
+    @staticmethod
+    def forward(ctx, input, offset, weight, bias, stride, padding, dilation, group,
+                deformable_groups, im2col_step):
+        ctx.stride, ctx.padding, ctx.dilation = _triple(stride), _triple(padding), _triple(dilation)
+        ctx.kernel_size = tuple(weight.shape[2:5])
+        ctx.group, ctx.deformable_groups, ctx.im2col_step = group, deformable_groups, im2col_step
+        if offset.dtype in (torch.float16, torch.bfloat16):   # autocast: follow the offset branch
+            input, bias, weight = input.to(offset.dtype), bias.to(offset.dtype), weight.to(offset.dtype)
+        output = _C.deform_conv_3d_forward(input, weight, bias, offset, *ctx.kernel_size,
+                                           *ctx.stride, *ctx.padding, *ctx.dilation, group,
+                                           deformable_groups, im2col_step)
+        ctx.save_for_backward(input, offset, weight, bias)
+        return output
 
-deform_conv = DeformConv3dFunction.apply
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad_output):
+        input, offset, weight, bias = ctx.saved_tensors
+        grad_input, grad_offset, grad_weight, grad_bias = _C.deform_conv_3d_backward(
+            input, weight, bias, offset, grad_output, *ctx.kernel_size, *ctx.stride, *ctx.padding,
+            *ctx.dilation, ctx.group, ctx.deformable_groups, ctx.im2col_step)
+        return grad_input, grad_offset, grad_weight, grad_bias, None, None, None, None, None, None
+
+
+deform_conv = DeformConv3dFunction.native
 
 
 class DeformConv3d(nn.Module):

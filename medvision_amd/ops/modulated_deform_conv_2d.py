@@ -10,19 +10,59 @@ import math
 
 import torch
 from torch import nn
+from torch.autograd.function import once_differentiable
 from torch.nn.modules.utils import _pair
 
+from .. import _C
 from .._lib import native
+from ._function import NativeFunction
 
 
-class ModulatedDeformConv2dFunction:
+class ModulatedDeformConv2dFunction(NativeFunction):
     @staticmethod
-    def apply(input, offset, mask, weight, bias=None, stride=1, padding=0, dilation=1, groups=1, deformable_groups=1):
+    def native(input, offset, mask, weight, bias=None, stride=1, padding=0, dilation=1, groups=1, deformable_groups=1):
         return native.modulated_deform_conv(2, input, offset, mask, weight, bias, stride, padding, dilation, groups,
                                             deformable_groups)
 
+    @staticmethod
+    def forward(ctx, input, offset, mask, weight, bias=None, stride=1, padding=0, dilation=1,
+                groups=1, deformable_groups=1):
+        ctx.with_bias = bias is not None
+        if not ctx.with_bias:
+            bias = input.new_empty(1)  # placeholder so that five tensors are always saved
+        if not input.is_cuda:
+            raise NotImplementedError
+        if offset.dtype in (torch.float16, torch.bfloat16):   # autocast: follow the offset branch
+            input, bias, weight = input.to(offset.dtype), bias.to(offset.dtype), weight.to(offset.dtype)
+        ctx.geometry = (*weight.shape[2:4], stride, stride, padding, padding, dilation, dilation,
+                        groups, deformable_groups, ctx.with_bias)
+        spatial = [(size + 2 * padding - (dilation * (k - 1) + 1)) // stride + 1
+                   for size, k in zip(input.shape[2:4], weight.shape[2:4])]
+        output = input.new_empty((input.size(0), weight.size(0), *spatial))
+        _C.modulated_deform_conv_2d_forward(input, weight, bias, None, offset, mask, output, None,
+                                            *ctx.geometry)
+        ctx.save_for_backward(input, offset, mask, weight, bias)
+        return output
 
-modulated_deform_conv = ModulatedDeformConv2dFunction.apply
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad_output):
+        if not grad_output.is_cuda:
+            raise NotImplementedError
+        input, offset, mask, weight, bias = ctx.saved_tensors
+        grad_input = torch.zeros_like(input)
+        grad_offset = torch.zeros_like(offset, dtype=input.dtype)
+        grad_mask = torch.zeros_like(mask, dtype=input.dtype)
+        grad_weight = torch.zeros_like(weight)
+        grad_bias = torch.zeros_like(bias)
+        _C.modulated_deform_conv_2d_backward(input, weight, bias, None, offset, mask, None,
+                                             grad_input, grad_weight, grad_bias, grad_offset,
+                                             grad_mask, grad_output, *ctx.geometry)
+        return (grad_input, grad_offset.to(offset.dtype), grad_mask.to(mask.dtype), grad_weight,
+                grad_bias if ctx.with_bias else None, None, None, None, None, None)
+
+
+modulated_deform_conv = ModulatedDeformConv2dFunction.native
 
 
 class ModulatedDeformConv2d(nn.Module):

@@ -11,19 +11,73 @@ import math
 
 import torch
 from torch import nn
+from torch.autograd.function import once_differentiable
 from torch.nn.modules.utils import _triple
 
+from .. import _C
 from .._lib import native
+from ._function import NativeFunction
 
 
-class ModulatedDeformConv3dFunction:
+class ModulatedDeformConv3dFunction(NativeFunction):
     @staticmethod
-    def apply(input, offset, mask, weight, bias=None, stride=1, padding=0, dilation=1, groups=1, deformable_groups=1):
+    def native(input, offset, mask, weight, bias=None, stride=1, padding=0, dilation=1, groups=1, deformable_groups=1):
         return native.modulated_deform_conv(3, input, offset, mask, weight, bias, stride, padding, dilation, groups,
                                             deformable_groups)
 
+    @staticmethod
+    def forward(ctx, input, offset, mask, weight, bias=None, stride=1, padding=0, dilation=1,
+                groups=1, deformable_groups=1):
+        ctx.stride, ctx.padding, ctx.dilation = stride, padding, dilation
+        ctx.groups, ctx.deformable_groups = groups, deformable_groups
+        ctx.with_bias = bias is not None
+        if not ctx.with_bias:
+            bias = input.new_empty(1)  # placeholder so that five tensors are always saved
+        if not input.is_cuda:
+            raise NotImplementedError
+        if offset.dtype in (torch.float16, torch.bfloat16):   # autocast: follow the offset branch
+            input, bias, weight = input.to(offset.dtype), bias.to(offset.dtype), weight.to(offset.dtype)
+        output = offset.new_empty(ModulatedDeformConv3dFunction._infer_shape(ctx, input, weight),
+                                  dtype=input.dtype)
+        k = weight.shape[2:5]
+        _C.modulated_deform_conv_3d_forward(
+            input, weight, bias, None, offset, mask, output, None, k[0], k[1], k[2],
+            stride, stride, stride, padding, padding, padding, dilation, dilation, dilation,
+            groups, deformable_groups, ctx.with_bias)
+        ctx.save_for_backward(input, offset, mask, weight, bias)
+        return output
 
-modulated_deform_conv = ModulatedDeformConv3dFunction.apply
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad_output):
+        if not grad_output.is_cuda:
+            raise NotImplementedError
+        input, offset, mask, weight, bias = ctx.saved_tensors
+        grad_input = torch.zeros_like(input)
+        grad_offset = torch.zeros_like(offset, dtype=input.dtype)
+        grad_mask = torch.zeros_like(mask, dtype=input.dtype)
+        grad_weight = torch.zeros_like(weight)
+        grad_bias = torch.zeros_like(bias)
+        k = weight.shape[2:5]
+        s, p, d = ctx.stride, ctx.padding, ctx.dilation
+        _C.modulated_deform_conv_3d_backward(
+            input, weight, bias, None, offset, mask, None, grad_input, grad_weight, grad_bias,
+            grad_offset, grad_mask, grad_output, k[0], k[1], k[2], s, s, s, p, p, p, d, d, d,
+            ctx.groups, ctx.deformable_groups, ctx.with_bias)
+        if not ctx.with_bias:
+            grad_bias = None
+        return (grad_input, grad_offset.to(offset.dtype), grad_mask.to(mask.dtype), grad_weight,
+                grad_bias, None, None, None, None, None)
+
+    @staticmethod
+    def _infer_shape(ctx, input, weight):
+        n, channels_out = input.size(0), weight.size(0)
+        spatial = [(size + 2 * ctx.padding - (ctx.dilation * (k - 1) + 1)) // ctx.stride + 1
+                   for size, k in zip(input.shape[2:5], weight.shape[2:5])]
+        return (n, channels_out, *spatial)
+
+
+modulated_deform_conv = ModulatedDeformConv3dFunction.native
 
 
 class ModulatedDeformConv3d(nn.Module):

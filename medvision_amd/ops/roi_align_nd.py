@@ -1,7 +1,7 @@
 """``RoIAlign`` for plain (axis-aligned) boxes, 2-D and 3-D.
 
 Interface of the reference's ``medvision/ops/roi_align_nd.py`` (module :158-198, autograd
-functions :7-155; the nodes themselves are native, ``csrc/binding.cpp``): ``RoIAlign(output_size, spatial_scale, sampling_ratio=-1)(features, rois,
+functions :7-155): ``RoIAlign(output_size, spatial_scale, sampling_ratio=-1)(features, rois,
 order=1)`` with rois ``(n, 5) = (batch_index, x1, y1, x2, y2)`` or ``(n, 7) = (batch_index, x1, y1,
 z1, x2, y2, z2)``.
 """
@@ -9,6 +9,23 @@ import torch.nn as nn
 
 from .. import _C
 from .._lib import native
+from ._function import NativeFunction
+
+
+def _parse_output_size(output_size, ndim):
+    if isinstance(output_size, int):
+        return (output_size,) * ndim
+    if isinstance(output_size, tuple):
+        assert len(output_size) == ndim
+        assert all(isinstance(v, int) for v in output_size)
+        return output_size
+    raise TypeError('"output_size" must be an integer or tuple of integers')
+
+
+def _kernels(ndim):
+    if ndim == 2:
+        return _C.roi_align_2d_forward, _C.roi_align_2d_backward
+    return _C.roi_align_3d_forward, _C.roi_align_3d_backward
 
 
 class PreparedFeatures:
@@ -29,20 +46,62 @@ class PreparedFeatures:
             raise RuntimeError("the features were changed in place after PreparedFeatures was made")
 
 
-class RoIAlign2DFunction:
+def _forward(ndim, ctx, features, rois, output_size, spatial_scale, sampling_ratio, order, prepared=None):
+    out = _parse_output_size(output_size, ndim)
+    ctx.spatial_scale, ctx.sampling_ratio, ctx.order = spatial_scale, sampling_ratio, order
+    ctx.save_for_backward(rois)
+    ctx.feature_size = features.size()
+    # every output element is written by the kernel (zeros where a sample is void): no zero fill
+    output = features.new_empty(rois.size(0), features.size(1), *out)
+    if prepared is not None:
+        _kernels(ndim)[0](features.contiguous(), rois, output, *out, spatial_scale, sampling_ratio, order, prepared)
+    else:
+        _kernels(ndim)[0](features, rois, output, *out, spatial_scale, sampling_ratio, order)
+    return output
+
+
+def _backward(ndim, ctx, grad_output):
+    (rois,) = ctx.saved_tensors
+    grad_input = None
+    if ctx.needs_input_grad[0]:
+        # the reference allocates this with the rois' dtype (roi_align_nd.py:64,139); the
+        # gradient's dtype is used here, which is the same whenever the reference runs at all
+        grad_input = grad_output.new_zeros(ctx.feature_size)
+        _kernels(ndim)[1](grad_output.contiguous(), rois, grad_input, *grad_output.shape[2:],
+                          ctx.spatial_scale, ctx.sampling_ratio, ctx.order)
+    return grad_input, None, None, None, None, None, None
+
+
+class RoIAlign2DFunction(NativeFunction):
     @staticmethod
-    def apply(features, rois, output_size, spatial_scale, sampling_ratio=0, order=1, prepared=None):
+    def native(features, rois, output_size, spatial_scale, sampling_ratio=0, order=1, prepared=None):
         return native.roi_align(2, False, features, rois, output_size, spatial_scale, sampling_ratio, True, order, prepared)
 
-
-class RoIAlign3DFunction:
     @staticmethod
-    def apply(features, rois, output_size, spatial_scale, sampling_ratio=0, order=1, prepared=None):
+    def forward(ctx, features, rois, output_size, spatial_scale, sampling_ratio=0, order=1, prepared=None):
+        return _forward(2, ctx, features, rois, output_size, spatial_scale, sampling_ratio, order, prepared)
+
+    @staticmethod
+    def backward(ctx, grad_output):
+        return _backward(2, ctx, grad_output)
+
+
+class RoIAlign3DFunction(NativeFunction):
+    @staticmethod
+    def native(features, rois, output_size, spatial_scale, sampling_ratio=0, order=1, prepared=None):
         return native.roi_align(3, False, features, rois, output_size, spatial_scale, sampling_ratio, True, order, prepared)
 
+    @staticmethod
+    def forward(ctx, features, rois, output_size, spatial_scale, sampling_ratio=0, order=1, prepared=None):
+        return _forward(3, ctx, features, rois, output_size, spatial_scale, sampling_ratio, order, prepared)
 
-roi_align_2d = RoIAlign2DFunction.apply
-roi_align_3d = RoIAlign3DFunction.apply
+    @staticmethod
+    def backward(ctx, grad_output):
+        return _backward(3, ctx, grad_output)
+
+
+roi_align_2d = RoIAlign2DFunction.native
+roi_align_3d = RoIAlign3DFunction.native
 
 
 class RoIAlign(nn.Module):

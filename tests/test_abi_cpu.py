@@ -179,3 +179,38 @@ def test_dcn_backward_workspace_keeps_to_its_limit():
         assert need(volume) - least[0] > 1 << 29     # ... and use it
     finally:
         _C.set_dcn_column_budget(old)
+
+
+def test_operator_functions_can_be_subclassed():
+    """The ``*Function`` classes are autograd functions with ``forward`` and ``backward``; one that overrides them is run through
+    its own."""
+    import importlib
+    for module, names in (("roi_align_nd", ("RoIAlign2DFunction", "RoIAlign3DFunction")),
+                          ("roi_align_rotated_nd", ("RoIAlignRotated2DFunction", "RoIAlignRotated3DFunction")),
+                          ("deform_conv_2d", ("DeformConv2dFunction",)), ("deform_conv_3d", ("DeformConv3dFunction",)),
+                          ("modulated_deform_conv_2d", ("ModulatedDeformConv2dFunction",)),
+                          ("modulated_deform_conv_3d", ("ModulatedDeformConv3dFunction",))):
+        for name in names:
+            base = getattr(importlib.import_module("medvision_amd.ops." + module), name)
+            assert issubclass(base, torch.autograd.Function)
+
+            class Twice(base):
+                @staticmethod
+                def forward(ctx, x, *rest):
+                    return 2 * x
+
+                @staticmethod
+                def backward(ctx, grad):
+                    return 3 * grad
+
+            class Node(base):
+                native = staticmethod(lambda x, add=1: x + add)
+
+            class Same(Node):
+                pass
+
+            x = torch.ones(2, requires_grad=True)
+            y = Twice.apply(x)
+            y.sum().backward()
+            assert y.tolist() == [2, 2] and x.grad.tolist() == [3, 3]
+            assert Same.apply(1) == 2 and Same.apply(1, add=2) == 3     # nothing overridden: the native node

@@ -41,3 +41,49 @@ def test_dual_tensors_are_refused(name, grad):
     with pytest.raises(RuntimeError):
         torch.func.vmap(lambda t: run(t, second))(x.unsqueeze(0))
     assert torch.isfinite(run(x, second)).all()
+
+
+def _layers():
+    import medvision_amd.ops as ops
+    from medvision_amd.ops import (deform_conv_2d, deform_conv_3d, modulated_deform_conv_2d, modulated_deform_conv_3d,
+                                   roi_align_nd, roi_align_rotated_nd)
+    g = torch.Generator().manual_seed(3)
+    r = lambda *s: torch.randn(*s, generator=g).to(DEV)
+    vol, img = r(2, 4, 7, 8, 9), r(2, 4, 8, 9)
+    plain3, plain2 = torch.tensor([[1, 1, 1, 1, 6, 6, 5.]], device=DEV), torch.tensor([[0, 1, 1, 6, 6.]], device=DEV)
+    turned3 = torch.tensor([[1, 4, 4, 4, 5, 5, 5, .1, .2, .3]], device=DEV)
+    turned2 = torch.tensor([[0, 4, 4, 5, 5, .1]], device=DEV)
+    w3, w2, b = r(6, 4, 3, 3, 3), r(6, 4, 3, 3), r(6)
+    return [
+        (roi_align_nd.RoIAlign3DFunction, [vol], (plain3, (2, 2, 2), 1.0, 2)),
+        (roi_align_nd.RoIAlign2DFunction, [img], (plain2, (2, 2), 1.0, 0, 1)),
+        (roi_align_rotated_nd.RoIAlignRotated3DFunction, [vol], (turned3, (2, 2, 2), 1.0, 2, True, 1)),
+        (roi_align_rotated_nd.RoIAlignRotated2DFunction, [img], (turned2, (2, 2), 1.0, 2)),
+        (deform_conv_3d.DeformConv3dFunction, [vol, r(2, 81, 7, 8, 9), w3, b], (1, 1, 1, 1, 1, 64)),
+        (deform_conv_2d.DeformConv2dFunction, [img, r(2, 18, 8, 9), w2, b], (1, 1, 1, 1, 1, 64)),
+        (modulated_deform_conv_3d.ModulatedDeformConv3dFunction, [vol, r(2, 81, 7, 8, 9), r(2, 27, 7, 8, 9), w3, b], (1, 1)),
+        (modulated_deform_conv_2d.ModulatedDeformConv2dFunction, [img, r(2, 18, 8, 9), r(2, 9, 8, 9), w2, b], (1, 1)),
+    ]
+
+
+@pytest.mark.parametrize("index", range(8))
+def test_functions_and_their_subclasses_agree(index):
+    """``forward`` and ``backward`` of the classes, as a subclass of them is run, against the native node."""
+    base, leaves, rest = _layers()[index]
+
+    class Counted(base):
+        calls = 0
+
+        @staticmethod
+        def backward(ctx, grad):
+            Counted.calls += 1
+            return base.backward(ctx, grad)
+
+    results = []
+    for function in (base, Counted):
+        ins = [t.clone().requires_grad_() for t in leaves]
+        out = function.apply(*ins, *rest)
+        results.append([out, *torch.autograd.grad(out, ins, torch.ones_like(out))])
+    assert Counted.calls == 1
+    for got, want in zip(*results):
+        torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-4 * float(want.abs().max()))
