@@ -1,11 +1,15 @@
 """Base of the operators' autograd functions."""
+import torch
 from torch.autograd import Function
+
+_tracing = torch._C._get_tracing_state     # None outside of torch.jit.trace
 
 
 class NativeFunction(Function):
     """A ``torch.autograd.Function`` whose ``apply`` runs the node of ``csrc/binding.cpp`` (``native``, the same arguments
-    and results without the interpreter in the backward pass).  ``forward`` and ``backward`` do the same through ``_C``: they
-    are there for callers that call them, and a subclass that overrides one of them is run through them."""
+    and results without the interpreter in the backward pass).  ``forward`` and ``backward`` do the same through ``_C``: for
+    callers that call them, for a subclass that overrides one of them, and for ``torch.jit.trace``, which records a Python
+    function as one node but of the native one nothing except the allocation of its result."""
     _direct = False
 
     def __init_subclass__(cls, **kwargs):
@@ -16,4 +20,6 @@ class NativeFunction(Function):
 
     @classmethod
     def apply(cls, *args, **kwargs):
-        return cls.native(*args, **kwargs) if cls._direct else super().apply(*args, **kwargs)
+        if cls._direct and _tracing() is None:
+            return cls.native(*args, **kwargs)
+        return super().apply(*args, **kwargs)

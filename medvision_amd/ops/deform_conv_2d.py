@@ -43,7 +43,7 @@ class DeformConv2dFunction(NativeFunction):
         return (*grads, None, None, None, None, None, None)
 
 
-deform_conv = DeformConv2dFunction.native
+deform_conv = DeformConv2dFunction.apply
 
 
 class DeformConv2d(nn.Module):

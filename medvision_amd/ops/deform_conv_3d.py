@@ -47,7 +47,7 @@ class DeformConv3dFunction(NativeFunction):
         return grad_input, grad_offset, grad_weight, grad_bias, None, None, None, None, None, None
 
 
-deform_conv = DeformConv3dFunction.native
+deform_conv = DeformConv3dFunction.apply
 
 
 class DeformConv3d(nn.Module):

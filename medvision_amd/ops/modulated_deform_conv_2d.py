@@ -62,7 +62,7 @@ class ModulatedDeformConv2dFunction(NativeFunction):
                 grad_bias if ctx.with_bias else None, None, None, None, None, None)
 
 
-modulated_deform_conv = ModulatedDeformConv2dFunction.native
+modulated_deform_conv = ModulatedDeformConv2dFunction.apply
 
 
 class ModulatedDeformConv2d(nn.Module):

@@ -77,7 +77,7 @@ class ModulatedDeformConv3dFunction(NativeFunction):
         return (n, channels_out, *spatial)
 
 
-modulated_deform_conv = ModulatedDeformConv3dFunction.native
+modulated_deform_conv = ModulatedDeformConv3dFunction.apply
 
 
 class ModulatedDeformConv3d(nn.Module):

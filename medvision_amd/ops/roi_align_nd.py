@@ -100,8 +100,8 @@ class RoIAlign3DFunction(NativeFunction):
         return _backward(3, ctx, grad_output)
 
 
-roi_align_2d = RoIAlign2DFunction.native
-roi_align_3d = RoIAlign3DFunction.native
+roi_align_2d = RoIAlign2DFunction.apply
+roi_align_3d = RoIAlign3DFunction.apply
 
 
 class RoIAlign(nn.Module):

@@ -78,8 +78,8 @@ class RoIAlignRotated3DFunction(NativeFunction):
         return _backward(3, ctx, grad_output)
 
 
-roi_align_rotated_2d = RoIAlignRotated2DFunction.native
-roi_align_rotated_3d = RoIAlignRotated3DFunction.native
+roi_align_rotated_2d = RoIAlignRotated2DFunction.apply
+roi_align_rotated_3d = RoIAlignRotated3DFunction.apply
 
 
 class RoIAlignRotated(nn.Module):

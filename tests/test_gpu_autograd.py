@@ -87,3 +87,27 @@ def test_functions_and_their_subclasses_agree(index):
     assert Counted.calls == 1
     for got, want in zip(*results):
         torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-4 * float(want.abs().max()))
+
+
+@pytest.mark.parametrize("index", range(8))
+def test_traced_layers_run_their_operator(index):
+    """torch.jit.trace records the operators as nodes: a traced call computes with the inputs that it is given."""
+    function, leaves, rest = _layers()[index]
+    consts = [a for a in rest if not torch.is_tensor(a)]
+    inputs = [*leaves, *[a for a in rest if torch.is_tensor(a)]]
+
+    def run(*tensors):
+        return function.apply(*tensors, *consts) + 1
+
+    with torch.no_grad():
+        traced = torch.jit.trace(run, tuple(inputs))
+        other = (leaves[0] * 2 + 1, *inputs[1:])
+        torch.testing.assert_close(traced(*other), run(*other))
+        assert not torch.equal(traced(*other), traced(*inputs))
+
+
+def test_function_transforms_are_refused():
+    """torch.func's gradient has no rule for the operators either: an error, as before, not a wrong result."""
+    for function, leaves, rest in _layers():
+        with pytest.raises(RuntimeError):
+            torch.func.grad(lambda t: function.apply(t, *leaves[1:], *rest).sum())(leaves[0])
