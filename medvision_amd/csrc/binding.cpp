@@ -73,6 +73,12 @@ Tensor bytes_on(const Tensor &like, size_t n) {
   return n ? at::empty({static_cast<int64_t>(n)}, like.options().dtype(at::kByte)) : Tensor();
 }
 
+// sampling_ratio, order, im2col_step: any number, as int() takes it
+int64_t whole(double v) {
+  MVB_CHECK(v > -9e18 && v < 9e18, "expected a whole number, got ", v);
+  return static_cast<int64_t>(v);
+}
+
 void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
 
 using Dims = std::array<int, 3>;
@@ -225,8 +231,8 @@ struct RoiAlignFunction : torch::autograd::Function<RoiAlignFunction> {
 
 // features that need no gradient (or a call under no_grad) get no node
 Tensor roi_align(int ndim, bool rotated, const Tensor &features, const Tensor &rois, const py::object &output_size,
-                 double spatial_scale, int sampling_ratio, bool aligned, int order, const std::optional<Tensor> &prepared) {
-  const RoiCall c{rotated ? kRotated : kPlain, ndim, sampling_ratio, order, aligned, static_cast<float>(spatial_scale),
+                 double spatial_scale, double sampling_ratio, bool aligned, double order, const std::optional<Tensor> &prepared) {
+  const RoiCall c{rotated ? kRotated : kPlain, ndim, static_cast<int>(whole(sampling_ratio)), static_cast<int>(whole(order)), aligned, static_cast<float>(spatial_scale),
                   parse_size(output_size, ndim)};
   no_forward_mode(features);
   no_forward_mode(rois);
@@ -239,14 +245,15 @@ Tensor roi_align(int ndim, bool rotated, const Tensor &features, const Tensor &r
 }
 
 Tensor affine(int ndim, const Tensor &features, const Tensor &rois, const py::object &out_size, double spatial_scale,
-              int sampling_ratio, bool aligned, int order) {
-  RoiCall c{kAffine, ndim, sampling_ratio, order, aligned, static_cast<float>(spatial_scale), parse_size(out_size, ndim)};
+              double sampling_ratio, bool aligned, double given_order) {
+  const int order = static_cast<int>(whole(given_order));
+  RoiCall c{kAffine, ndim, static_cast<int>(whole(sampling_ratio)), order, aligned, static_cast<float>(spatial_scale), parse_size(out_size, ndim)};
   const auto t = features.scalar_type();
   // (int32: label maps at order 0, sampled as they are -- the reference resamples a float copy of them)
   if (!(t == at::kFloat || t == at::kHalf || t == at::kBFloat16 || t == at::kDouble || (t == at::kInt && order == 0)))
     raise(PyExc_AssertionError, "input must be a floating tensor but got " + dtype_name(features));
-  if (order != 0 && order != 1 && order != 3)
-    raise(PyExc_AssertionError, "order " + std::to_string(order) + " is not supported!");
+  if ((order != 0 && order != 1 && order != 3) || order != given_order)
+    raise(PyExc_AssertionError, c10::str("order ", given_order, " is not supported!"));
   if (order == 0) c.ratio = 1;   // never average nearest-neighbour samples (reference cuda_fun_tools.py:72-74)
   const py::gil_scoped_release no_gil;
   const at::NoGradGuard no_grad;
@@ -426,17 +433,18 @@ Tensor modulated_deform_conv(int nd, const Tensor &input, const Tensor &offset, 
 // DCNv1: the bias is always added
 Tensor deform_conv(int nd, const Tensor &input, const Tensor &offset, const Tensor &weight, const Tensor &bias,
                    const py::object &stride, const py::object &padding, const py::object &dilation, int groups, int dg,
-                   int64_t im2col_step) {
+                   double im2col_step) {
   const DcnCall c{nd, groups, dg, per_axis(stride, nd, 1), per_axis(padding, nd, 0), per_axis(dilation, nd, 1)};
   for (const Tensor &t : {input, offset, weight, bias}) no_forward_mode(t);
   const py::gil_scoped_release no_gil;
   MVB_CHECK(input.is_cuda(), "Not implemented on the CPU");
-  im2col_step_check(input.size(0), im2col_step);
+  im2col_step_check(input.size(0), whole(im2col_step));
   return DeformConvFunction::apply(input, offset, std::nullopt, weight, bias, c);
 }
 
 // ---- displacement-field warp ------------------------------------------------------------------------------------------
-Tensor deform_warp(const Tensor &img_in, const Tensor &offset_in, int order) {
+Tensor deform_warp(const Tensor &img_in, const Tensor &offset_in, double given_order) {
+  const int order = given_order == 0.0 || given_order == 1.0 || given_order == 3.0 ? static_cast<int>(given_order) : -1;
   const py::gil_scoped_release no_gil;
   const at::NoGradGuard no_grad;
   MVB_CHECK(img_in.is_cuda(), "Not implemented on the CPU");
@@ -450,7 +458,7 @@ Tensor deform_warp(const Tensor &img_in, const Tensor &offset_in, int order) {
   std::vector<int64_t> want = img.sizes().vec();
   if (want.size() > 1) want[1] = ndim;
   MVB_CHECK(offset.sizes() == at::IntArrayRef(want), "offset must have shape [B, ", ndim, ", *spatial]");
-  MVB_CHECK(order == 0 || order == 1 || order == 3, "order ", order, " is not supported (0 nearest, 1 linear, 3 cubic)");
+  MVB_CHECK(order >= 0, "order ", given_order, " is not supported (0 nearest, 1 linear, 3 cubic)");
   const int code = labels ? static_cast<int>(MV_I32) : dtype_code(img);
   const Tensor out = at::empty_like(img);
   const auto d = five_dims(img.sizes(), ndim);

@@ -214,3 +214,20 @@ def test_operator_functions_can_be_subclassed():
             y.sum().backward()
             assert y.tolist() == [2, 2] and x.grad.tolist() == [3, 3]
             assert Same.apply(1) == 2 and Same.apply(1, add=2) == 3     # nothing overridden: the native node
+
+
+def test_whole_numbers_may_be_floats():
+    """sampling_ratio, order and im2col_step go through int(): the calls get as far as the check of the device."""
+    import medvision_amd.ops as ops
+    from medvision_amd.ops.deform_conv_3d import deform_conv
+    vol, plain, turned = torch.randn(1, 4, 6, 6, 6), torch.zeros(1, 7), torch.zeros(1, 10)
+    weight, bias, off = torch.zeros(4, 4, 3, 3, 3), torch.zeros(4), torch.zeros(1, 81, 6, 6, 6)
+    for run in (lambda: ops.roi_align_nd.roi_align_3d(vol, plain, (2, 2, 2), 1.0, 2.0, 1.0),
+                lambda: ops.roi_align_rotated_nd.roi_align_rotated_3d(vol, turned, (2, 2, 2), 1.0, 2.0, True, 1.0),
+                lambda: ops.affine_3d(vol, turned, (2, 2, 2), 1.0, 1.0, True, 1.0),
+                lambda: ops.apply_offset_3d(vol, torch.zeros(1, 3, 6, 6, 6), 1.0),
+                lambda: deform_conv(vol, off, weight, bias, 1, 1, 1, 1, 1, 64.0)):
+        with pytest.raises(RuntimeError, match="CPU"):
+            run()
+    with pytest.raises(AssertionError, match="order 1.5 is not supported"):
+        ops.affine_3d(vol, turned, (2, 2, 2), 1.0, 1, True, 1.5)
