@@ -280,6 +280,7 @@ DcnShape dcn_shape(const DcnCall &c, const Tensor &input, const Tensor &weight) 
   MVB_CHECK(input.dim() == c.nd + 2 && weight.dim() == c.nd + 2, "expected ", c.nd + 2, "-d input and weight tensors");
   const auto x = five_dims(input.sizes(), c.nd), w = five_dims(weight.sizes(), c.nd);
   const int C = x[1], Cout = w[0], ck = w[1];
+  MVB_CHECK(c.groups > 0 && c.dg > 0, "groups must be positive");   // (divided by below)
   MVB_CHECK(C == ck * c.groups, "Input shape and kernel channels wont match: (", C, " vs ", ck * c.groups, ").");
   MVB_CHECK(C % c.groups == 0 && Cout % c.groups == 0, "channels(", C, ") and channels_out(", Cout, ") must divide group(",
             c.groups, ")");

@@ -111,3 +111,15 @@ def test_function_transforms_are_refused():
     for function, leaves, rest in _layers():
         with pytest.raises(RuntimeError):
             torch.func.grad(lambda t: function.apply(t, *leaves[1:], *rest).sum())(leaves[0])
+
+
+@pytest.mark.parametrize("groups,dg", [(0, 1), (1, 0), (-1, 1), (1, -2)])
+def test_groups_that_cannot_be_divided_by_are_refused(groups, dg):
+    from medvision_amd.ops.deform_conv_2d import deform_conv
+    from medvision_amd.ops.modulated_deform_conv_2d import modulated_deform_conv
+    x, off, mask = torch.zeros(1, 4, 6, 6, device=DEV), torch.zeros(1, 18, 6, 6, device=DEV), torch.zeros(1, 9, 6, 6, device=DEV)
+    weight, bias = torch.zeros(4, 4, 3, 3, device=DEV), torch.zeros(4, device=DEV)
+    with pytest.raises(RuntimeError):
+        modulated_deform_conv(x, off, mask, weight, bias, 1, 1, 1, groups, dg)
+    with pytest.raises(RuntimeError):
+        deform_conv(x, off, weight, bias, 1, 1, 1, groups, dg, 64)
