@@ -18,12 +18,13 @@ namespace mv {
 // The offsets of the next group are requested a whole B phase ahead; no barrier separates the samples of a group from
 // its products, and the registers leave room for five wavefronts per SIMD.  One convolution group must lie inside one
 // deformable group, and a tap's weight pieces (SLICES x MB x 1 KB) are kept to 8 KB.
-template <typename T, int MB, int SLICES, int NC>
+template <typename T, int SLICES>
 __global__ __launch_bounds__(256, 5) void dcn_forward_shared_taps_kernel(
     const T *__restrict__ xt, const T *__restrict__ off, const T *__restrict__ mask,
     const T *__restrict__ wf, const T *__restrict__ bias, T *__restrict__ y, const DcnDims s) {
   using M = Mfma<T>;
   constexpr int PC = M::kPiece, SL = 4 * PC, ES = sizeof(T), TG = 4;
+  constexpr int NC = 8, MB = 4;                   // corners; blocks of 16 output channels
   static_assert(sizeof(T) == 2, "16-bit tensors");
   constexpr int REC = 2 * NC;                     // dwords per record: NC corner offsets, NC weights
   constexpr int WT = SLICES * MB * 64;            // 16-byte weight pieces per tap
@@ -70,19 +71,19 @@ __global__ __launch_bounds__(256, 5) void dcn_forward_shared_taps_kernel(
   }
   const int plane_bytes = static_cast<int>(s.Q) * ES;
   const __amdgpu_buffer_rsrc_t offr = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<T *>(off + bg * s.nd * s.K * s.Q), 0, s.nd * s.K * plane_bytes, 0x00020000);
+      const_cast<T *>(off + bg * 3 * s.K * s.Q), 0, 3 * s.K * plane_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t maskr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<T *>(mask ? mask + bg * s.K * s.Q : off), 0, mask ? s.K * plane_bytes : 0, 0x00020000);
   const unsigned q_bytes = static_cast<unsigned>(qgc) * ES;
   auto as_float = [](unsigned short bits) { T t; __builtin_memcpy(&t, &bits, 2); return load(&t); };
-  // (d), h, w offsets and the mask value of tap k, requested one group ahead (a tap beyond the
+  // d, h, w offsets and the mask value of tap k, requested one group ahead (a tap beyond the
   // last one reads zeros: scalar offsets take part in the range check)
   unsigned short rd = 0, rh = 0, rw = 0, rm = 0;
   auto request = [&](int k) {
-    const int first = s.nd * k * plane_bytes;
-    if (s.nd == 3) rd = __builtin_amdgcn_raw_buffer_load_b16(offr, q_bytes, first, 0);
-    rh = __builtin_amdgcn_raw_buffer_load_b16(offr, q_bytes, first + (s.nd - 2) * plane_bytes, 0);
-    rw = __builtin_amdgcn_raw_buffer_load_b16(offr, q_bytes, first + (s.nd - 1) * plane_bytes, 0);
+    const int first = 3 * k * plane_bytes;
+    rd = __builtin_amdgcn_raw_buffer_load_b16(offr, q_bytes, first, 0);
+    rh = __builtin_amdgcn_raw_buffer_load_b16(offr, q_bytes, first + plane_bytes, 0);
+    rw = __builtin_amdgcn_raw_buffer_load_b16(offr, q_bytes, first + 2 * plane_bytes, 0);
     rm = __builtin_amdgcn_raw_buffer_load_b16(maskr, q_bytes, k * plane_bytes, 0);
   };
   // element strides of the channels-last input in bytes, and the corner offsets relative to the first
@@ -118,10 +119,9 @@ __global__ __launch_bounds__(256, 5) void dcn_forward_shared_taps_kernel(
     const int k = k0 + wave;
     if (k < s.K) {
       const float m = mask ? as_float(rm) : 1.f;
-      float pd = base_d + static_cast<float>(ki * s.dd) + as_float(rd);
+      const float pd = base_d + static_cast<float>(ki * s.dd) + as_float(rd);
       const float ph = base_h + static_cast<float>(kj * s.dh) + as_float(rh);
       const float pw = base_w + static_cast<float>(kk * s.dw) + as_float(rw);
-      if (NC == 4) pd = 0.f;   // images: the only slice
       // A corner is inside iff its index is: with f = floor(p) the low one iff 0 <= f < size, the
       // high one iff 0 <= f + 1 < size (a sample at -1 exactly keeps a high corner of weight 0).
       const float fd = floorf(pd), fh = floorf(ph), fw = floorf(pw);
@@ -230,13 +230,13 @@ int dcn_shared_taps_forward(const void *xt, const void *off, const void *mask, c
   // bricks of 8 x 4 x 2 output voxels (8 x 8 of a single slice), one per workgroup
   const int bdz = s.Do > 1 ? 2 : 1, bhy = 8 / bdz;
   const long bricks = static_cast<long>((s.Wo + 7) / 8) * ((s.Ho + bhy - 1) / bhy) * ((s.Do + bdz - 1) / bdz);
-  if (s.cpg % 32 || slices < 1 || slices > 2 || s.cpd % s.cpg || blocks < 4 || bricks * s.B < 1024 || bricks >= (1L << 31) ||
-      static_cast<long>(s.groups) * chunks > 65535 || static_cast<long>(s.nd) * s.K * s.Q * 2 >= (1L << 31) ||
+  if (s.nd != 3 || s.cpg % 32 || slices < 1 || slices > 2 || s.cpd % s.cpg || blocks < 4 || bricks * s.B < 1024 || bricks >= (1L << 31) ||
+      static_cast<long>(s.groups) * chunks > 65535 || 3L * s.K * s.Q * 2 >= (1L << 31) ||
       static_cast<long>(s.K) * slices * blocks * 1024 >= (1L << 31))
     return -1;
   const dim3 grid(static_cast<unsigned>(bricks), s.groups * chunks, s.B), block(256);
 #define MV_SHARED_TAPS(T, SLICES)                                                                                     \
-  hipLaunchKernelGGL((dcn_forward_shared_taps_kernel<T, 4, SLICES, 8>), grid, block, 0, stream, static_cast<const T *>(xt), \
+  hipLaunchKernelGGL((dcn_forward_shared_taps_kernel<T, SLICES>), grid, block, 0, stream, static_cast<const T *>(xt), \
                      static_cast<const T *>(off), static_cast<const T *>(mask), static_cast<const T *>(wf),           \
                      static_cast<const T *>(bias), static_cast<T *>(y), s)
   if (dtype == MV_F16) { if (slices == 1) MV_SHARED_TAPS(__half, 1); else MV_SHARED_TAPS(__half, 2); }

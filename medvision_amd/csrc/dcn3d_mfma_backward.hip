@@ -91,10 +91,6 @@ int dcn_tap_backward(const void *xt, const void *off, const void *mask, const vo
 bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape);
 int dcn_scatter(const void *off, const void *mask, const void *gyt, const void *wf, float *gxt, const DcnDims &s,
                 const ScatterShape &shape, const unsigned *bounds, int dtype, hipStream_t stream);
-// dcn_backward_scatter.hip
-bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape);
-int dcn_scatter(const void *off, const void *mask, const void *gyt, const void *wf, float *gxt, const DcnDims &s,
-                const ScatterShape &shape, const unsigned *bounds, int dtype, hipStream_t stream);
 
 // ---- layouts and folds -----------------------------------------------------------------------------
 // Element (output channel o of the padded layer p, channel cl of its group, tap k) of the real layer's weight

@@ -4,11 +4,11 @@
 // group and per group of output channels (dcn3d_mfma.hip, dcn3d_mfma_backward.hip).  Any other layer
 // (16, 24, 40, 48 ... channels, with any number of groups as long as convolution groups and
 // deformable groups nest) is run as the next larger layer that they do take: the input, the weight
-// and the output gradient get zero channels (backward: in the passes that lay them out for the kernels anyway; forward:
-// as copies), the kernels run on the padded shapes, and outputs and gradients are taken from the real channels only.  Zero inputs, zero weight rows and
+// and the output gradient get zero channels (forward: as copies in the caller's workspace; backward: in the passes that lay them
+// out for the kernels anyway, which also take the gradients from the real channels), the kernels run on the padded shapes, and outputs and gradients are taken from the real channels only.  Zero inputs, zero weight rows and
 // zero weight columns add nothing to any output or gradient, so the results are those of the layer
-// itself.  The copies live in the caller's workspace; they cost one pass over the tensors, against
-// kernels that are 50 - 100 times slower without the matrix cores.
+// itself.  The forward's copies cost one pass over the tensors, against kernels that are 50 - 100 times slower without the
+// matrix cores.
 //
 // Channel map: with unit = min(channels per convolution group, channels per deformable group) (the
 // smaller divides the larger) real input channel c sits at (c / unit) * unit_p + c % unit of the

@@ -173,19 +173,20 @@ int roi_plane_forward(const void *input, const void *rois, void *output, int dty
 int roi_plane_backward_parts(int dtype, const RoiProblem &p);
 int roi_plane_backward(const void *grad_output, const void *rois, void *grad, float *acc, int dtype, const RoiProblem &p,
                        int parts, bool accumulate, hipStream_t s);
-// roi_gather_backward.hip: atomic-free backward for resampling-sized problems; -1 when not applicable
-// roi_box.hip: backward of small outputs that the pooled kernels do not take (rotated boxes, large
-// grids), one workgroup per (roi, channel group) with LDS tiles of the source boxes; -1 when not applicable
+// roi_own_backward.hip: backward of heads that the pooled kernels do not take (rotated boxes, large grids) by the voxels' owners
 bool roi_own_applies(int dtype, const RoiProblem &p);
 size_t roi_own_workspace(int dtype, const RoiProblem &p);
 int roi_own_backward(const void *grad_output, const void *rois, void *grad_input, int dtype, const RoiProblem &p, void *workspace,
                      size_t capacity, hipStream_t s);
+// roi_box.hip: the same heads where the owners do not apply (gradients to be added to, no workspace), one workgroup per (roi,
+// channel group) with LDS tiles of the source boxes; -1 when not applicable
 int roi_box_backward(const void *grad_output, const void *rois, float *acc, int dtype, const RoiProblem &p, hipStream_t s);
 // Many small outputs over wide feature maps, read from a channels-last copy in the workspace (roi_cl.hip).
 size_t roi_forward_cl_workspace(int dtype, const RoiProblem &p);
 int roi_forward_cl(const void *input, const void *rois, void *output, int dtype, const RoiProblem &p,
                    void *workspace, size_t capacity, hipStream_t s);
 
+// roi_gather_backward.hip: atomic-free backward for resampling-sized problems; -1 when not applicable
 int roi_backward_gather(const void *grad_output, const void *rois, void *grad_input, int dtype,
                         const RoiProblem &p, bool accumulate, hipStream_t s);
 // dcn3d_mfma_backward.hip: dst [B, C, P] += (not `accumulate`: =) src [B, P, C] fp32

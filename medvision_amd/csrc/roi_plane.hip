@@ -384,6 +384,7 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void roi_plane_forward_kernel(con
 constexpr int kPlaneAhead = 2;      // rois whose gradients are loaded or in flight
 constexpr int kPlaneBatch = 8;      // rois whose pixel weights are worked out together
 constexpr int kPlaneQueue = 1024;   // rois looked through at a time
+constexpr int kPlaneBackwardChannels = 8;   // of a wavefront
 
 // A wavefront has CH channels of the tile.  SPLIT: several workgroups share a tile's rois (few tiles, many rois) and
 // add to the fp32 buffer `acc`; otherwise a pixel is written once, to `grad` (added to what is there when
@@ -653,12 +654,10 @@ int roi_plane_forward(const void *input, const void *rois, void *output, int dty
   return check_launch("roi_plane_forward_kernel");
 }
 
-static int plane_channels(const RoiProblem &p) { return 8; }   // per wavefront of the backward pass
-
 // Workgroups that share a tile's rois: 1 while the tiles and channels alone fill the chip (0: not for this problem).
 int roi_plane_backward_parts(int dtype, const RoiProblem &p) {
   if (!roi_plane_applies(dtype, p)) return 0;
-  const int ch = plane_channels(p) * kPlaneWaves;
+  const int ch = kPlaneBackwardChannels * kPlaneWaves;
   const long groups = static_cast<long>(p.N) * ((p.W + kPlaneTile - 1) / kPlaneTile) * ((p.H + kPlaneTile - 1) / kPlaneTile) *
                       ((p.C + ch - 1) / ch);
   // (a part should have a few dozen rois to look through)
@@ -668,19 +667,19 @@ int roi_plane_backward_parts(int dtype, const RoiProblem &p) {
 // parts == 1: `grad` is written (added to when `accumulate`); else the sums are added to the fp32 buffer `acc` (zeros).
 int roi_plane_backward(const void *grad_output, const void *rois, void *grad, float *acc, int dtype, const RoiProblem &p,
                        int parts, bool accumulate, hipStream_t s) {
-  const int ch = plane_channels(p) * kPlaneWaves;
+  const int ch = kPlaneBackwardChannels * kPlaneWaves;
   const int tx = (p.W + kPlaneTile - 1) / kPlaneTile, ty = (p.H + kPlaneTile - 1) / kPlaneTile;
   const long tiles = static_cast<long>(p.N) * tx * ty, cblocks = (p.C + ch - 1) / ch;
   if (tiles >= (1L << 31) || cblocks > 65535) return -1;
   const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(cblocks), parts), block(kPlaneThreads);
   const float *r = static_cast<const float *>(rois);
-#define MV_PLANE_BACKWARD(TYPE, CELLSV, CHV, SPLITV)                                                                 \
-  hipLaunchKernelGGL((roi_plane_backward_kernel<TYPE, CELLSV, CHV, SPLITV>), grid, block, 0, s,                       \
+#define MV_PLANE_BACKWARD(TYPE, CELLSV, SPLITV)                                                                      \
+  hipLaunchKernelGGL((roi_plane_backward_kernel<TYPE, CELLSV, kPlaneBackwardChannels, SPLITV>), grid, block, 0, s,                       \
                      static_cast<const TYPE *>(grad_output), r, static_cast<TYPE *>(grad), acc, p, tx, ty, accumulate ? 1 : 0)
 #define MV_PLANE_BACKWARD_OF(TYPE)                                                                                    \
   do {                                                                                                               \
-    if (plane_small(p)) { if (parts > 1) MV_PLANE_BACKWARD(TYPE, 8, 8, true); else MV_PLANE_BACKWARD(TYPE, 8, 8, false); } \
-    else { if (parts > 1) MV_PLANE_BACKWARD(TYPE, 16, 8, true); else MV_PLANE_BACKWARD(TYPE, 16, 8, false); }         \
+    if (plane_small(p)) { if (parts > 1) MV_PLANE_BACKWARD(TYPE, 8, true); else MV_PLANE_BACKWARD(TYPE, 8, false); } \
+    else { if (parts > 1) MV_PLANE_BACKWARD(TYPE, 16, true); else MV_PLANE_BACKWARD(TYPE, 16, false); }         \
   } while (0)
   switch (dtype) {
     case MV_F32: MV_PLANE_BACKWARD_OF(float); break;

@@ -1122,9 +1122,9 @@ __global__ __launch_bounds__(THREADS, 4) void roi_resample_kernel(
 }
 
 // ---- taps straight from the caches -----------------------------------------------------------------
-// The persistent kernel above pays ~18 us per launch whatever the size (plans of up to 16 items on one
-// wavefront, a box through registers and LDS, one item after the other).  Small problems run this kernel instead: a
-// workgroup takes 1 / PARTS of one tile, and its lanes read their taps from the L1 / L2, the two x taps of
+// The persistent kernel above takes ~7 us before the size counts (plans of up to 16 items on one wavefront, a box through
+// registers and LDS, one item after the other).  Small problems run this kernel instead, ~4.7 us (launch_resample has
+// the rule): a workgroup takes 1 / PARTS of one tile, and its lanes read their taps from the L1 / L2, the two x taps of
 // a row in one load.  Items, plans, coordinates (relative to the same box origin), tap rules and blends are those
 // of the kernel above, so the outputs are the same bit for bit.
 // The two x taps of a row: elements `off` and `off` + 1 (bytes) of the buffer.
