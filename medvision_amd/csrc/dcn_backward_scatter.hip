@@ -18,7 +18,8 @@
 // 16-bit result.  Otherwise a 64-bit word per channel, scale from the global maxima.
 //
 // What bounds it: the LDS additions (six to seven 64-bit lanes a clock and compute unit) and the 64-byte atomics of the tiles
-// (21 G a second on the whole chip).
+// (21 G a second on the whole chip).  Busy, bf16 [2, 32 -> 64, 48^3] (32-bit sums, 496 us): vector issue 61 %, LDS 54 % (61 % of
+// that bank conflicts: cells at random places); fp16 [8, 256 -> 256, 100 x 152] (64-bit, 1185 us): 47 %, 37 %, texture addressers 39 %.
 #include "dcn_scatter.hpp"
 
 namespace mv {

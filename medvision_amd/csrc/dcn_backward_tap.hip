@@ -21,8 +21,9 @@
 // Corners that the LDS scatter does not take are listed when the records are made, and their 32 channels are added as
 // 128 contiguous bytes.
 // What bounds it: narrow layers the vector instructions of the samples (184 per 16 positions and 32 channels, and as many more
-// for everything else) and the latency of the gathers, wide ones the matrix cores and LDS, and everywhere the atomics of the far
-// corners (64 bytes per corner and 16 channels, 21 G of them a second at best).
+// for everything else; vector issue 56 %) and the latency of the gathers (50 % of the wavefronts' time in waits), wide ones LDS
+// (45 %, half of it bank conflicts; vector issue 25 %, matrix cores 17 %) and the same waits, and everywhere the atomics of the
+// far corners (64 bytes per corner and 16 channels, 21 G of them a second at best).
 //   (bf16 [2, 32 -> 64, 48^3]: 493 us; the data and weight kernels before it took 670 us.  fp16 images
 //   [8, 256 -> 256, 100 x 152]: 762 us, 4380 us before.  [1, 128 -> 128, 7 x 45 x 18]: 64 us, 790 us before.)
 #include "dcn_scatter.hpp"

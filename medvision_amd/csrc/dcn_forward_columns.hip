@@ -20,8 +20,9 @@
 // PT: 32 positions use a weight fragment twice; 16 give a layer of a few thousand positions twice the workgroups, whose
 // wavefronts then share the positions and split the pieces.  (64 positions: no faster for wide layers, 165 us against
 // 134 us for bf16 [2, 128 -> 64, 50 x 37 x 13].)
-// What bounds it: narrow layers the blend (a multiply-add per channel and corner) and the cache look-ups of the corners
-// (64 bytes a clock), wide ones the matrix cores; small layers the latency of the chain load - blend - product.
+// What bounds it: the cache look-ups of the corners (64 bytes a clock; 256 -> 256 channels: texture addressers 74 % busy, vector
+// issue 34 %, matrix cores 24 %), narrow layers the blend too (a multiply-add per channel and corner); small layers the latency of
+// the chain load - blend - product.
 //   (Images fp16 [8, 256 -> 256, 100 x 152]: 566 us with 16 positions per wavefront and the weights through LDS, 283 us now;
 //   bf16 [4, 256 -> 64, 121 x 21] stride 2: 83 us, 21 us now; bf16 [1, 128 -> 32, 6 x 22 x 34]: 100 us, 30 us now.)
 #include "dcn_mfma.hpp"

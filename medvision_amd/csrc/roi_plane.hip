@@ -16,12 +16,13 @@
 // one, columns in groups of four), so that large rois with a small sampling grid read only what they use.  A lane's
 // piece of a 16 x 16 piece of the box is one 16-byte load (16-bit tensors: 8 bytes), straight from the feature map.
 //   (1000 rois of 4 - 64 pixels, adaptive grid, 256 channels, 7 x 7 cells, fp32, [2, 256, 200, 304]: 480 us when the
-//   boxes went through LDS and three barriers per chunk of channels; 161 us now.)
+//   boxes went through LDS and three barriers per chunk of channels; 165 us now: matrix cores 47 % and texture addressers 58 %
+//   busy.)
 //
 // Backward, one workgroup = (16 x 16 pixels, some channels): it looks up the rois that touch its pixels, works out
 // its pixels' weights for eight rois at a time and adds roi after roi into accumulators that stay in registers.  No
 // atomics, no fp32 copy of the gradient, every pixel written once, sums in the order of the rois.
-//   (The same head: 1030 us with one atomic per touched pixel, roi and channel; 140 us now.)
+//   (The same head: 1030 us with one atomic per touched pixel, roi and channel; 145 us now: matrix cores 50 %, vector issue 32 %.)
 // What bounds them: the matrix cores (three 32-clock instructions per roi, tile and channel backward; 4 (x pieces + 1)
 // per row piece and channel forward) and the latency of the loads.
 #include <algorithm>
