@@ -1104,6 +1104,54 @@ def test_rotated_heads_backward_with_many_rois_and_channels(ops, oracle, dtype, 
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rotated,channels,rois_n,size,out,sr", [
+    (True, 32, 300, (18, 26, 30), (7, 7, 7), 2),      # box tiles, several channels per workgroup
+    (True, 32, 300, (26, 30), (14, 14), 3),
+    (False, 32, 60, (18, 26, 30), (7, 7, 7), 2),      # separable sums
+    (False, 32, 60, (26, 30), (7, 7), 0),             # images: pixels' owners, rois split over workgroups
+    (False, 8, 40, (200, 210), (5, 9), 2),            # the same, a workgroup per tile
+    (True, 3, 2, (20, 24, 28), (20, 24, 28), 1),      # resampling: tiles of the output
+])
+def test_raw_backward_adds_to_the_gradient(oracle, dtype, rotated, channels, rois_n, size, out, sr):
+    """``_C.*_backward`` and ``mv_roi_align_*_backward`` ADD to the gradient that they are given (the classes have it written),
+    which takes kernels of its own for heads; values that are not finite reach the same voxels as in the oracle."""
+    from medvision_amd import _C
+    nd = len(size)
+    g = wl.gen(700 + sum(size) + channels)
+    xyz = torch.tensor(size[::-1], dtype=torch.float32)
+    ext = torch.exp(torch.rand(rois_n, nd, generator=g) * math.log(30.0)) * 0.6      # 0.6 .. 18 voxels
+    ctr = torch.rand(rois_n, nd, generator=g) * xyz
+    if out == size:
+        ext, ctr = xyz.repeat(rois_n, 1), (xyz / 2).repeat(rois_n, 1)
+    image = torch.randint(0, 2, (rois_n, 1), generator=g).float()
+    if rotated:
+        angle = (torch.rand(rois_n, 3 if nd == 3 else 1, generator=g) * 2 - 1) * math.radians(40)
+        rois = torch.cat([image, ctr, ext, angle], 1)
+    else:
+        rois = torch.cat([image, ctr - ext / 2, ctr + ext / 2], 1)
+    run = getattr(_C, f"roi_align_{'rotated_' if rotated else ''}{nd}d_backward")
+    shape = (2, channels, *size)
+
+    def check(gy, start, what):
+        grad = start.to(DEV)
+        run(gy.to(DEV), rois.to(DEV), grad, *out, 1.0, sr, *((True, 1) if rotated else (1,)))
+        want = start.double() + oracle.roi_align_backward(gy, rois, shape, 1.0, sr, True, 1, rotated).reshape(shape)
+        got, ok = grad.cpu(), torch.isfinite(want)
+        # (the oracle's border samples carry 0 x infinity to voxels of weight 0, which the kernels leave out)
+        assert torch.isfinite(got[ok]).all() and torch.isfinite(got).all() == ok.all(), what
+        assert_close(got[ok], want[ok], BWD_TOL[dtype], what)
+
+    gy = torch.randn(rois_n, channels, *out, generator=g).to(dtype)
+    start = torch.randn(shape, generator=g).to(dtype)
+    check(gy, start, "added")
+    if rotated and out != size:
+        big = int(torch.argmax(ext.prod(dim=1)))
+        gy[big, 3].view(-1)[gy[big, 3].numel() // 2] = float("nan")
+        gy[(big + 1) % rois_n, 17].view(-1)[5] = float("inf")
+        check(gy, start, "NaN and infinite gradients")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("ndim,rotated,C,out", [(3, True, 24, (7, 7, 7)), (3, True, 72, (7, 7, 7)),
                                                 (2, True, 520, (14, 14)), (2, False, 32, (20, 20))])
 def test_heads_forward_from_channels_last_copy(ops, oracle, dtype, ndim, rotated, C, out):
