@@ -1,7 +1,8 @@
 // Channel padding for the matrix-core deformable-convolution kernels.
 //
-// Those kernels take channel counts that are multiples of 32 per convolution group, per deformable
-// group and per group of output channels (dcn3d_mfma.hip, dcn3d_mfma_backward.hip).  Any other layer
+// The backward's kernels take channel counts that are multiples of 32 per convolution group, per deformable
+// group and per group of output channels (dcn3d_mfma_backward.hip), the forward's input channels in whole 16-byte pieces per
+// group and output channels in multiples of 16 (dcn_forward_columns.hip).  Any other layer
 // (16, 24, 40, 48 ... channels, with any number of groups as long as convolution groups and
 // deformable groups nest) is run as the next larger layer that they do take: the input, the weight
 // and the output gradient get zero channels (forward: as copies in the caller's workspace; backward: in the passes that lay them
