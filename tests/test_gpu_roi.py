@@ -316,8 +316,9 @@ def test_pooled_kernels_with_large_boxes(ops, oracle, shape, out, sr, extent, dt
 def test_pooled_forward_with_dense_and_sparse_rois_in_one_call(ops, oracle, dtype, ndim):
     """Plain boxes from a fraction of a voxel to most of the feature map, grids of 1 and 2: a roi whose box
     holds more than half as many voxels as its samples have taps is read sparsely and takes its taps one
-    by one (on images four per sample, the absent slice left out), the others stage their box in LDS;
-    both kinds in one launch, 40 channels (matrix-core blocks and the remainder)."""
+    by one, the others stage their box in LDS;
+    both kinds in one launch, 40 channels (matrix-core blocks and the remainder).  (Images have kernels that list
+    the rows and columns that samples touch.)"""
     g = wl.gen(420 + ndim)
     size = (20, 72, 88)[3 - ndim:]
     out = (7,) * ndim
@@ -822,7 +823,8 @@ def test_pooled_boxes_wider_than_the_tap_tables(ops, oracle, dtype):
     """Few cells spread over many voxels: boxes of 70-100 voxels on one axis with 7 cells of 2
     samples, and of more than 258.  The separable backward kernel indexes its tap ranges by source
     voxel through a table of 260 entries and has to hand wider boxes to the per-output scatter (with
-    68 entries and no such hand-over it once ran off the table and never finished)."""
+    68 entries and no such hand-over it once ran off the table and never finished).  Images of four cells and more have
+    kernels of their own now; volumes beyond 258: the next test."""
     g = wl.gen(77)
     img = torch.randn(2, 6, 110, 120, generator=g).to(dtype)
     rois2 = torch.tensor([[0, 3.0, 5.0, 98.0, 60.0], [1, 10.5, 2.0, 105.0, 101.0], [0, 40.0, 40.0, 47.0, 46.0],
@@ -840,6 +842,25 @@ def test_pooled_boxes_wider_than_the_tap_tables(ops, oracle, dtype):
         y.backward(gy.to(DEV))
         want = oracle.roi_align_backward(gy, rois, feat.shape, 1.0, 2, True, 1, False)
         assert_close(x.grad, want, BWD_TOL[dtype], "backward")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_pooled_volumes_wider_than_the_tap_tables(ops, oracle, dtype, axis):
+    """The same on volumes, along each axis, on both sides of 258 voxels (images with such boxes have kernels of their own)."""
+    g = wl.gen(178 + axis)
+    size = [5, 5, 5]
+    size[axis] = 300
+    feat = torch.randn(1, 8, *size[::-1], generator=g).to(dtype)
+    rois = torch.tensor([[0, 0.5, 0.5, 0.5, 4.5, 4.5, 4.5]] * 4)
+    for i, (lo, hi) in enumerate(((4.0, 292.5), (20.0, 278.0), (-5.0, 310.0), (30.0, 50.0))):
+        rois[i, 1 + axis], rois[i, 4 + axis] = lo, hi
+    x = feat.to(DEV).requires_grad_(True)
+    y = ops.RoIAlign((3, 7, 9), 1.0, 2)(x, rois.to(DEV))
+    assert_close(y, oracle.roi_align_forward(feat, rois, (3, 7, 9), 1.0, 2, True, 1, False), FWD_TOL[dtype], "forward")
+    gy = torch.randn(y.shape, generator=g).to(dtype)
+    y.backward(gy.to(DEV))
+    assert_close(x.grad, oracle.roi_align_backward(gy, rois, feat.shape, 1.0, 2, True, 1, False), BWD_TOL[dtype], "backward")
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
@@ -1049,11 +1070,10 @@ def test_backward_of_finely_sampled_rois_with_gradients_of_one_sign(ops, oracle,
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("ndim", [3, 2])
 def test_rotated_heads_backward_with_many_rois_and_channels(ops, oracle, dtype, ndim):
-    """Enough rois x channels for a workgroup to own several channels: a block's samples are worked out
-    once and their taps kept in registers while the channels pass through the LDS tile.  Boxes from one
-    channel per pass (large rois) to all of a workgroup's channels side by side (small ones), more samples
-    per thread than are kept (grid 3, 14^2 cells), a NaN and an infinity in single channels (those
-    channels' terms go out one by one, the others' through the tile), zero gradients."""
+    """Hundreds of overlapping rois x 32 channels, which the voxels' owners take (the last part's three channels, and the raw
+    entry points of test_raw_backward_adds_to_the_gradient, the box tiles, where a workgroup owns several channels
+    and keeps a block's taps in registers): rois of a fraction of a voxel to most of the volume, grids of 2 and 3 and adaptive
+    ones, a NaN and an infinity in single channels, zero gradients."""
     g = wl.gen(650 + ndim)
     size = (18, 26, 30)[3 - ndim:]
     out = (7, 7, 7) if ndim == 3 else (14, 14)
