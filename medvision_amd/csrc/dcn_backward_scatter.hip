@@ -2,130 +2,244 @@
 //
 //   gx[corner_n(k, q), c] += w_n * mask * gcol[c, k, q],   gcol[c, k, q] = sum_o Wt[o, c, k] * gy[o, q]
 //
-// A workgroup owns a brick of positions and 16 (fp32: 8) channels; its sixteen wavefronts split the brick's groups of 32
-// positions and, where there are fewer than sixteen, the taps.  Two taps at a time: the lower half-wavefront works out tap k of
-// the group's positions, the upper half tap k + 1; gcol comes from the 16 x 16 MFMA with the channels as rows (fp32: the
-// eight channels of both taps), so a lane holds position l % 16 of a block and four channels.  Corners in the brick's tile are
-// integer additions to LDS; afterwards the tile's non-zero sums are added to the gradient buffer, one global atomic per
-// (voxel, channel) of the tile instead of one per (position, tap, corner, channel).
+// A workgroup owns a brick of positions and 16 channels (8 where 64-bit sums of 16 are beyond the LDS); its wavefronts split the
+// brick's groups of 32 positions and, where there are fewer groups than wavefronts, the taps.  Two taps at a time: every lane works
+// out one sample, a cell of the tile and the weights of its corners.  gcol comes from the 16 x 16 MFMA with the positions as rows, so
+// that a row of sixteen lanes holds sixteen channels of one position (eight of two taps): the sample's words reach them as DPP row
+// broadcasts, which the multiplications take as an operand, and an LDS addition meets four (eight) cells of 64 contiguous bytes.
+// Per term: multiply, convert, add.  Corners outside the tile or the volume have weight 0 in a cell that exists: no branches.
+//   (Channels as rows, a lane holding one position and four channels, needed the samples' words from LDS, a branch per corner
+//   and additions to 16 places: bf16 [2, 32 -> 64, 48^3] 496 us, now 338 us; fp16 [8, 256 -> 256, 100 x 152] 1185 us, now 500 us.)
+// Afterwards the tile's non-zero sums are added to the gradient buffer, one global atomic per (voxel, channel) of the tile
+// instead of one per (position, tap, corner, channel).
 //
-// NARROW (dense layers of 16-bit tensors, see dcn_scatter_plan): 32-bit sums.  (Two of them per 64-bit addition: 11.3 terms a clock and compute unit
-// against 10.3, and more vector instructions to make the words: 556 us against 504 us.)  They leave 30 - ceil(log2(positions * taps)) bits for a term (17 for 3 x 3 x 3 taps), so the scale comes from the data: a
-// first sweep over the brick's taps forms gcol alone (matrix cores, no geometry) and takes max |gcol| of the workgroup;
-// every term is then below max |gcol| * max |mask| < 2^ex and is rounded to a multiple of 2^(ex - shift) (adding
-// 1.5 * 2^23 in fp32 leaves round(x) in the low mantissa bits for |x| < 2^22).  The error of a voxel's sum stays below
-// terms * 2^(ex - shift - 1), about 2^-15 of the values it sums for the 3 x 3 x 3 layer — a sixteenth of the last bit of the
-// 16-bit result.  Otherwise a 64-bit word per channel, scale from the global maxima.
+// NARROW (dense layers of 16-bit tensors, see dcn_scatter_plan): 32-bit sums.  They leave 30 - ceil(log2(positions * taps)) bits for
+// a term (17 for 3 x 3 x 3 taps), so the scale comes from the data: a first sweep over the brick's taps forms gcol alone (matrix
+// cores, no geometry; 17 us of the 338) and takes max |gcol| of the workgroup; every term is then below max |gcol| * max |mask| <
+// 2^ex and is rounded to a multiple of 2^(ex - shift).  The error of a voxel's sum stays below terms * 2^(ex - shift - 1), about
+// 2^-15 of the values it sums for the 3 x 3 x 3 layer — a sixteenth of the last bit of the 16-bit result.  Otherwise a 64-bit word
+// per channel, scale from the global maxima.
 //
-// What bounds it: the LDS additions (six to seven 64-bit lanes a clock and compute unit) and the 64-byte atomics of the tiles
-// (21 G a second on the whole chip).  Busy, bf16 [2, 32 -> 64, 48^3] (32-bit sums, 496 us): vector issue 61 %, LDS 54 % (61 % of
-// that bank conflicts: cells at random places); fp16 [8, 256 -> 256, 100 x 152] (64-bit, 1185 us): 47 %, 37 %, texture addressers 39 %.
+// What bounds it: the LDS additions (64 lanes of 32 bits in 4 clocks, of 64 bits in 6, whatever the cells) behind phases that leave
+// the LDS idle, since a tile fills the compute unit: the first group's inputs, the sweep, the tile's atomics (40 us).  Busy: bf16
+// [2, 32 -> 64, 48^3] vector issue 52 %, LDS 40 %; fp16 [8, 256 -> 256, 100 x 152] 45 %, 26 %, texture addressers 39 %.
 #include "dcn_scatter.hpp"
 
 namespace mv {
 
 // Tiles of input voxels: their pitches are constants, so that the corners of a sample are immediate offsets (with pitches at run
 // time: 603 us against 504 us for bf16 [2, 32 -> 64, 48^3]).
-template <int D, int H, int W> struct Tile { static constexpr int TD = D, TH = H, TW = W, VOX = D * H * W, NC = D > 1 ? 8 : 4; };
+// Channels of a workgroup: 16, and 8 where 64-bit sums of 16 are beyond the LDS.
+template <int D, int H, int W> struct Tile {
+  static constexpr int TD = D, TH = H, TW = W, VOX = D * H * W, NC = D > 1 ? 8 : 4;
+  static constexpr bool WIDE = D == 1 && W > H;
+  template <bool NARROW> static constexpr int channels = VOX * 16 * (NARROW ? 4 : 8) <= 160 * 1024 ? 16 : 8;
+};
 constexpr int kScatterMinShift = 14;  // fewer bits per term: 64-bit words
 __host__ __device__ constexpr int scatter32_shift(int terms) {
   int bits = 0;
   while ((1L << bits) < terms) bits++;
-  return bits < 8 ? 22 : 30 - bits;   // (a term stays below 2^22)
+  return bits < 8 ? 22 : 30 - bits;
 }
-// sums between voxels: the channels of a workgroup, and one to spread the banks
-template <bool NARROW> constexpr int kScatterStride = NARROW ? 17 : 9;
 
-// KEEP: slices of grad_output (of 4 * kPiece output channels) that a wavefront keeps in registers over the taps: 4, or 8 with half
-// the wavefronts for wide layers, whose further slices cost 64 cache look-ups each for every tap.
+template <int... I, typename F> __device__ __forceinline__ void unrolled(std::integer_sequence<int, I...>, F f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+// The value that lane FROM of the lane's row of sixteen holds.  CH == 8: lane FROM for the row's lower half, FROM + 8 for the upper.
+template <int CH, int FROM> __device__ __forceinline__ int row_word(int v) {
+  constexpr int kRowBroadcast = 0x150;
+  if constexpr (CH == 16) return __builtin_amdgcn_mov_dpp(v, kRowBroadcast + FROM, 0xf, 0xf, true);
+  const int low = __builtin_amdgcn_mov_dpp(v, kRowBroadcast + FROM, 0xf, 0xf, true);
+  return __builtin_amdgcn_update_dpp(low, v, kRowBroadcast + (FROM + 8) % 16, 0xf, 0xc, false);
+}
+template <int CH, int FROM> __device__ __forceinline__ float row_value(float v) {
+  return __int_as_float(row_word<CH, FROM>(__float_as_int(v)));
+}
+// round(x) for |x| < 2^31 in one instruction
+__device__ __forceinline__ int round_word(float x) {
+  int r;
+  asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+  return r;
+}
+
+// A value that is the same in all lanes, in a scalar register
+__device__ __forceinline__ float uniform(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
+
+// One axis of a tile that starts at voxel `origin` and whose cells low .. high - 1 lie in the volume.
+struct TileAxis {
+  float origin, low, high, low1, high1;
+  __device__ __forceinline__ TileAxis(int first, int cells, int voxels)
+      : origin(uniform(static_cast<float>(first))), low(uniform(static_cast<float>(max(0, -first)))),
+        high(uniform(static_cast<float>(min(cells, voxels - first)))), low1(uniform(low - 1.f)), high1(uniform(high - 1.f)) {}
+  // The weights of two neighbouring cells of the tile, of which it returns the first.  A corner outside has weight 0: a sample on the
+  // tile's edge has its cells moved by one, any other one outside both weights 0 (NaN positions too), so that every cell exists.
+  template <int CELLS, typename P> __device__ __forceinline__ float sample(P p, float &w0, float &w1) const {
+    const P f = floor(p);
+    const float frac = static_cast<float>(p - f), z = static_cast<float>(f - static_cast<P>(origin));
+    const float u0 = z >= low && z < high ? 1.f - frac : 0.f, u1 = z >= low1 && z < high1 ? frac : 0.f;
+    const float first = fminf(fmaxf(z, 0.f), static_cast<float>(CELLS - 2));
+    const bool moved = z != first;
+    w0 = moved ? u1 : u0;
+    w1 = moved ? u0 : u1;
+    return first;
+  }
+};
+
+// KEEP: slices of grad_output (of 4 * kPiece output channels) that a wavefront keeps in registers over the taps: 2 or 4, or 8 with
+// half the wavefronts for wide layers, whose further slices cost 64 cache look-ups each for every tap.
 template <typename T, bool NARROW, typename S, int KEEP>
-__global__ __launch_bounds__(KEEP == 4 ? 1024 : 512) void dcn_backward_scatter_kernel(
+__global__ __launch_bounds__(KEEP <= 4 ? 1024 : 512) void dcn_backward_scatter_kernel(
     const T *__restrict__ off, const T *__restrict__ mask, const T *__restrict__ gyt,
     const T *__restrict__ wa, float *__restrict__ gxt, const DcnDims s, const ScatterShape shape,
     const unsigned *__restrict__ bounds) {
   using M = Mfma<T>;
   using P = typename std::conditional<(sizeof(T) == 2), float, double>::type;
-  constexpr int PC = M::kPiece, SL = 4 * PC, CH = NARROW ? 16 : 8, NC = S::NC, WAVES = KEEP == 4 ? 16 : 8;
+  constexpr int PC = M::kPiece, SL = 4 * PC, ES = sizeof(T), CH = S::template channels<NARROW>, NC = S::NC, ND = NC == 8 ? 3 : 2;
+  constexpr int WAVES = KEEP <= 4 ? 16 : 8;
+  constexpr int TAPS = CH == 16 ? 2 : 1;   // products per pair of taps
+  // positions of a group: 64 where eight slices of the weight come from the caches for every tap (with sixteen wavefronts of 32
+  // positions 620 us instead of 500 for fp16 [8, 256 -> 256, 100 x 152])
+  constexpr int SETS = KEEP == 8 && S::WIDE ? 2 : 1, BLOCKS = 2 * SETS, GROUP = 16 * BLOCKS;
   using Sum = typename std::conditional<NARROW, int, unsigned long long>::type;
-  constexpr int STRIDE = kScatterStride<NARROW>;
-  __shared__ Sum tile[S::VOX * STRIDE];
-  __shared__ float recs[WAVES][5][64];   // cell and corner bits, mask (times the scale), ld, lh, lw
+  constexpr int CELL = CH * static_cast<int>(sizeof(Sum));
+  __shared__ __attribute__((aligned(16))) Sum tile[S::VOX * CH];
   __shared__ unsigned wgmax;
   const ScatterScale scale = scatter_scale(bounds, shape.terms, mask != nullptr);
   if (!scale.valid) return;  // (a NaN or infinity somewhere: every corner went through the tap kernel)
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int n = lane % 32, half = lane / 32, p16 = lane % 16, j = lane / 16;
-  const unsigned brick = xcd_contiguous(blockIdx.x, gridDim.x);
-  const int bx = brick % shape.nbw, by = (brick / shape.nbw) % shape.nbh, bz = brick / (shape.nbw * shape.nbh);
-  const int c0 = blockIdx.y * CH, b = blockIdx.z;
+  const int p16 = lane % 16, j = lane / 16;
+  // the lane's own sample: position n of a group, the first or second tap of a pair
+  const int n = p16 / 4 % 2 * 16 + 4 * j + p16 % 4, half = p16 / 8;
+  // (the channel blocks of a brick next to each other on one XCD: they read the same grad_output and offsets)
+  const int turns = CH == 16 && KEEP == 8 ? shape.turns : 1;   // blocks of CH channels, one after the other
+  const unsigned id = xcd_contiguous(blockIdx.x, gridDim.x), shares_of_brick = s.Cin / (CH * turns), brick = id / shares_of_brick;
+  int c0 = static_cast<int>(id % shares_of_brick) * (CH * turns);
+  const int bx = brick % shape.nbw, by = brick / shape.nbw % shape.nbh, bz = brick / (shape.nbw * shape.nbh) % shape.nbd,
+            b = brick / (shape.nbw * shape.nbh * shape.nbd);
   const int dgi = c0 / s.cpd, g = c0 / s.cpg;
   const long bg = static_cast<long>(b) * s.dg + dgi;
   const int steps = s.opg / SL, cblocks = s.cpg / 16;
-  const int groups = (1 << (shape.bd + shape.bh + shape.bw)) / 32;   // of 32 positions
-  const int pwaves = min(groups, 8);                                 // wavefronts over the groups; the others over the taps
+  const int groups = (1 << (shape.bd + shape.bh + shape.bw)) / GROUP;
+  const int pwaves = min(groups, WAVES);   // wavefronts over the groups; the others over the taps
   const int share = wave / pwaves, shares = WAVES / pwaves;
   const int per = (s.K + shares - 1) / shares, k0 = min(share * per, s.K), k1 = min(s.K, k0 + per);
   const TileOrigin origin = tile_origin(s, shape, bz, by, bx);
 
-  for (int i = threadIdx.x; i < S::VOX * STRIDE; i += WAVES * 64) tile[i] = 0;
-  if (threadIdx.x == 0) wgmax = 0u;
-  __syncthreads();
-
   // position of brick index i, columns fastest
-  auto position = [&](int i, bool &live) {
+  struct Position { int d, h, w, q; bool live; };
+  auto position = [&](int i) {
+    Position p;
     const int od = (bz << shape.bd) + (i >> (shape.bh + shape.bw)), oh = (by << shape.bh) + ((i >> shape.bw) & ((1 << shape.bh) - 1)),
               ow = (bx << shape.bw) + (i & ((1 << shape.bw) - 1));
-    live = od < s.Do && oh < s.Ho && ow < s.Wo;
-    return (static_cast<long>(min(od, s.Do - 1)) * s.Ho + min(oh, s.Ho - 1)) * s.Wo + min(ow, s.Wo - 1);
+    p.live = od < s.Do && oh < s.Ho && ow < s.Wo;
+    p.d = min(od, s.Do - 1); p.h = min(oh, s.Ho - 1); p.w = min(ow, s.Wo - 1);
+    p.q = (p.d * s.Ho + p.h) * s.Wo + p.w;
+    return p;
   };
-  // grad_output of the lane's column in the two 16-position blocks of a group (MFMA B operand)
-  const T *grow[2];
-  bool glive[2];
-  u32x4 keep[2][KEEP];
+  // grad_output of the lane's row in the blocks of 16 positions of group `loaded` (MFMA A operand)
+  u32x4 keep[BLOCKS][KEEP];
+  auto gradient = [&](const Position &p, int st) {
+    return p.live && st < steps ? *reinterpret_cast<const u32x4 *>(gyt + (static_cast<long>(b) * s.Q + p.q) * s.Cout + g * s.opg + j * PC + st * SL)
+                                : u32x4{0u, 0u, 0u, 0u};
+  };
+  int loaded = -1;
+  bool some = false;   // (any position of the group exists)
   auto load_keep = [&](int pg) {
+    if (pg == loaded) return;
+    loaded = pg;
+    bool mine = false;
 #pragma unroll
-    for (int blk = 0; blk < 2; blk++) {
-      bool on;
-      const long qb = position(pg * 32 + blk * 16 + p16, on);
-      const T *from = gyt + (static_cast<long>(b) * s.Q + qb) * s.Cout + g * s.opg + j * PC;
+    for (int blk = 0; blk < BLOCKS; blk++) {
+      const Position p = position(pg * GROUP + blk * 16 + p16);
 #pragma unroll
-      for (int st = 0; st < KEEP; st++)
-        keep[blk][st] = on && st < steps ? *reinterpret_cast<const u32x4 *>(from + st * SL) : u32x4{0u, 0u, 0u, 0u};
-      grow[blk] = from;
-      glive[blk] = on;
+      for (int st = 0; st < KEEP; st++) keep[blk][st] = gradient(p, st);
+      mine = mine || p.live;
     }
+    some = __any(mine) != 0;
   };
-  // Rows of the weight of tap k: NARROW its 16 channels; else the 8 channels of tap k in rows 0 - 7 and of tap k + 1 in rows 8 - 15
-  // (zeros when that is not the wavefront's)
-  const long tap_stride = static_cast<long>(cblocks) * steps * 64 * PC;
-  const T *wrow = wa + (static_cast<long>(g) * s.K * cblocks + (c0 - g * s.cpg) / 16) * steps * (64 * PC) +
-                  (NARROW ? lane : j * 16 + p16 % 8 + (c0 - g * s.cpg) % 16) * PC + (NARROW ? 0 : p16 / 8 * tap_stride);
+  // Columns of the weight of tap k: the 16 channels; of eight channels tap k in columns 0 - 7 and tap k + 1 in columns 8 - 15.  No
+  // branches: slices that do not exist meet zeros of grad_output, the tap behind the wavefront's last one samples of weight 0 (and the
+  // buffer ends behind the last of all).
+  const int tap_bytes = s.cpg * s.opg * ES;
+  const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<T *>(wa + static_cast<long>(g) * s.K * s.cpg * s.opg), 0, s.K * tap_bytes, kRsrcFlags);
+  int cl = c0 - g * s.cpg;
+  const unsigned wlane = static_cast<unsigned>((CH == 16 ? lane : j * 16 + p16 % 8 + cl % 16) * 16 + (CH == 16 ? 0 : half * tap_bytes));
   auto load_weight = [&](int k, int st) {
-    const bool on = NARROW || k + p16 / 8 < k1;
-    return on && st < steps ? *reinterpret_cast<const u32x4 *>(wrow + k * tap_stride + static_cast<long>(st) * (64 * PC)) : u32x4{0u, 0u, 0u, 0u};
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, wlane, k * tap_bytes + (cl / 16 * steps + min(st, steps - 1)) * 1024, 0));
   };
-  // gcol of both blocks of the group (the further slices of wide layers are read again for every tap)
-  auto product = [&](const u32x4 (&w)[KEEP], int k, float4_t (&acc)[2]) {
-    acc[0] = acc[1] = float4_t{0.f, 0.f, 0.f, 0.f};
+  constexpr int AHEAD = SETS == 2 ? 4 : KEEP;   // slices requested behind the product before (the registers hold no more)
+  auto load_weights = [&](int k, u32x4 (&w)[AHEAD]) {
 #pragma unroll
-    for (int st = 0; st < KEEP; st++)
-      if (st < steps) {
-        acc[0] = M::run16(w[st], keep[0][st], acc[0]);
-        acc[1] = M::run16(w[st], keep[1][st], acc[1]);
-      }
+    for (int st = 0; st < AHEAD; st++) w[st] = load_weight(k, st);
+  };
+  // gcol of the blocks of the group (the further slices of wide layers are read again for every tap)
+  auto product = [&](const u32x4 (&w)[AHEAD], int k, int pg, float4_t (&acc)[BLOCKS]) {
+#pragma unroll
+    for (int blk = 0; blk < BLOCKS; blk++) acc[blk] = float4_t{0.f, 0.f, 0.f, 0.f};
+    u32x4 now[AHEAD], then[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++) now[i] = w[i];
+#pragma unroll
+    for (int from = 0; from < KEEP; from += AHEAD) {
+#pragma unroll
+      for (int i = 0; i < AHEAD; i++)
+        if (from + AHEAD + i < KEEP) then[i] = load_weight(k, from + AHEAD + i);
+      if (AHEAD < KEEP) __builtin_amdgcn_sched_barrier(0);   // (the registers hold no more of the weight)
+#pragma unroll
+      for (int i = 0; i < AHEAD; i++)
+#pragma unroll
+        for (int blk = 0; blk < BLOCKS; blk++) acc[blk] = M::run16(keep[blk][from + i], now[i], acc[blk]);
+      if (AHEAD < KEEP) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < AHEAD; i++) now[i] = then[i];
+    }
     for (int st = KEEP; KEEP > 4 && st < steps; st++) {
       const u32x4 wf = load_weight(k, st);
 #pragma unroll
-      for (int blk = 0; blk < 2; blk++) {
-        const u32x4 bf = glive[blk] ? *reinterpret_cast<const u32x4 *>(grow[blk] + st * SL) : u32x4{0u, 0u, 0u, 0u};
-        acc[blk] = M::run16(wf, bf, acc[blk]);
-      }
+      for (int blk = 0; blk < BLOCKS; blk++)
+        acc[blk] = M::run16(gradient(position(pg * GROUP + blk * 16 + p16), st), wf, acc[blk]);
     }
   };
-  auto load_weights = [&](int k, u32x4 (&w)[KEEP]) {
+  // ---- a group's samples -----------------------------------------------------------------------------------------
+  int bd[SETS], bh[SETS], bw[SETS];
+  unsigned at0[SETS];
+  bool live[SETS];
+  // offsets and mask as they are stored: requested a pair ahead, converted where they are used
+  T rd[SETS], rh[SETS], rw[SETS], rm[SETS];
+  const unsigned step = static_cast<unsigned>(s.Q) * ES;
+  auto request = [&](int k) {
+    const bool second = half && k + 1 < s.K;   // (beyond the last tap: the first of the pair)
+    const char *o = reinterpret_cast<const char *>(off + (bg * s.K + k) * ND * s.Q), *m = reinterpret_cast<const char *>(mask + (bg * s.K + k) * s.Q);
 #pragma unroll
-    for (int st = 0; st < KEEP; st++) w[st] = load_weight(k, st);
+    for (int e = 0; e < SETS; e++) {
+      const unsigned at = at0[e] + (second ? ND * step : 0u);
+      if (ND == 3) rd[e] = *reinterpret_cast<const T *>(o + at);
+      rh[e] = *reinterpret_cast<const T *>(o + (ND - 2) * static_cast<long>(step) + at);
+      rw[e] = *reinterpret_cast<const T *>(o + (ND - 1) * static_cast<long>(step) + at);
+      if (mask) rm[e] = *reinterpret_cast<const T *>(m + (at0[e] + (second ? step : 0u)));
+    }
   };
+  const int kfirst = min(k0, s.K - 1);   // (k0 == K: a share without taps)
+  auto open = [&](int pg) {
+#pragma unroll
+    for (int e = 0; e < SETS; e++) {
+      const Position own = position(pg * GROUP + e * 32 + n);
+      bd[e] = own.d * s.sd - s.pd; bh[e] = own.h * s.sh - s.ph; bw[e] = own.w * s.sw - s.pw;
+      at0[e] = static_cast<unsigned>(own.q) * ES;
+      live[e] = own.live;
+    }
+    request(kfirst);
+  };
+  u32x4 weights[AHEAD];   // of the next product, requested behind the one before
+
+  // The first group's inputs are on their way while the tile is cleared.
+  open(wave % pwaves);
+  load_keep(wave % pwaves);
+  load_weights(kfirst, weights);
+  for (int i = threadIdx.x; i < S::VOX * CELL / 16; i += WAVES * 64) reinterpret_cast<u32x4 *>(tile)[i] = u32x4{0u, 0u, 0u, 0u};
+  if (threadIdx.x == 0) wgmax = 0u;
+  __syncthreads();
 
   float up = 1.f, down = 1.f;
   if constexpr (NARROW) {
@@ -133,11 +247,11 @@ __global__ __launch_bounds__(KEEP == 4 ? 1024 : 512) void dcn_backward_scatter_k
     float top = 0.f;
     for (int pg = wave % pwaves; pg < groups; pg += pwaves) {
       load_keep(pg);
+      if (!some) continue;
       for (int k = k0; k < k1; k++) {
-        u32x4 w[KEEP];
-        load_weights(k, w);
-        float4_t acc[2];
-        product(w, k, acc);
+        float4_t acc[BLOCKS];
+        product(weights, k, pg, acc);
+        load_weights(k + 1 < k1 ? k + 1 : k0, weights);
 #pragma unroll
         for (int i = 0; i < 4; i++) top = fmaxf(top, fmaxf(fabsf(acc[0][i]), fabsf(acc[1][i])));
       }
@@ -153,182 +267,181 @@ __global__ __launch_bounds__(KEEP == 4 ? 1024 : 512) void dcn_backward_scatter_k
     up = ldexpf(1.f, shift - ex);
     down = ldexpf(1.f, ex - shift);
   }
-  constexpr float kMagic = 12582912.f;  // 1.5 * 2^23
-  float(*rec)[64] = recs[wave];
+  const TileAxis ad(origin.d, S::TD, s.D), ah(origin.h, S::TH, s.H), aw(origin.w, S::TW, s.W);
+  char *const sums = reinterpret_cast<char *>(tile) + p16 % CH * sizeof(Sum);
 
-  for (int pg = wave % pwaves; pg < groups; pg += pwaves) {
-    bool live;
-    const long q = position(pg * 32 + n, live);
-    const int ow = q % s.Wo, oh = (q / s.Wo) % s.Ho, od = q / (static_cast<long>(s.Wo) * s.Ho);
-    const int bd = od * s.sd - s.pd, bh = oh * s.sh - s.ph, bw = ow * s.sw - s.pw;
-    load_keep(pg);
-    int kt = k0 + half;  // the lane's own tap
-    const T *o = off + (bg * s.nd * s.K + static_cast<long>(s.nd) * kt) * s.Q + q;
-    const T *mk = mask ? mask + (bg * s.K + kt) * s.Q + q : nullptr;
-    int ki = kt / (s.kh * s.kw), kj = (kt / s.kw) % s.kh, kk = kt % s.kw;
-    P fd = P(0), fh = P(0), fw = P(0);
-    float fm = 1.f;
-    if (kt < k1) {
-      dcn_offsets(s, o, fd, fh, fw);
-      if (mk) fm = load(mk);
-    }
-    for (int k = k0; k < k1; k += 2) {
-      // weight pieces of the two taps (the taps' geometry below hides their latency)
-      u32x4 wpair[NARROW ? 2 : 1][KEEP];
+  const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
+      gxt + static_cast<long>(b) * s.P * s.Cin, 0, static_cast<int>(s.P * s.Cin * 4), kRsrcFlags);
+  constexpr int CELLS = 64 / CH, TURNS = (S::TW + CELLS - 1) / CELLS;   // cells of a turn
+  const int first = lane / CH;
+  const unsigned turn_bytes = static_cast<unsigned>(CELLS * s.Cin) * 4u, place = static_cast<unsigned>(first * s.Cin + lane % CH) * 4u;
+  for (int turn = 0; turn < turns; turn++) {
+    for (int pg = wave % pwaves; pg < groups; pg += pwaves) {
+      if (groups > pwaves) {
+        load_keep(pg);
+        if (pg != wave % pwaves || turn > 0) open(pg);
+      }
+      if (!some) continue;   // (positions beyond the output)
+      int kt = k0 + half;  // the lane's own tap
+      int ki = kt / (s.kh * s.kw), kj = (kt / s.kw) % s.kh, kk = kt % s.kw;
+      for (int k = k0; k < k1; k += 2) {
+        // the lane's samples: byte offset of the first cell, the corners' weights times the mask (and the scale)
+        int cell[SETS];
+        float w[SETS][NC];
 #pragma unroll
-      for (int u = 0; u < (NARROW ? 2 : 1); u++) load_weights(min(k + u, s.K - 1), wpair[u]);
-      {
-        P pd = fd + static_cast<P>(bd + ki * s.dd);
-        const P ph = fh + static_cast<P>(bh + kj * s.dh), pw = fw + static_cast<P>(bw + kk * s.dw);
-        if (NC == 4) pd = P(0);   // images: the only slice
-        const float m = fm;
-        const bool tap_on = kt < k1;
+        for (int e = 0; e < SETS; e++) {
+          float m = mask ? static_cast<float>(load(&rm[e])) : 1.f;
+          m = live[e] && kt < k1 ? (NARROW ? m * up : m) : 0.f;
+          float wd[2] = {1.f, 0.f}, wh[2], ww[2], at = 0.f;
+          if constexpr (ND == 3) at = ad.sample<S::TD>(static_cast<P>(load(&rd[e])) + static_cast<P>(bd[e] + ki * s.dd), wd[0], wd[1]);
+          const float ath = ah.sample<S::TH>(static_cast<P>(load(&rh[e])) + static_cast<P>(bh[e] + kj * s.dh), wh[0], wh[1]);
+          const float atw = aw.sample<S::TW>(static_cast<P>(load(&rw[e])) + static_cast<P>(bw[e] + kk * s.dw), ww[0], ww[1]);
+          at = fmaf(at, static_cast<float>(S::TH), ath);
+          cell[e] = static_cast<int>(fmaf(at, static_cast<float>(S::TW), atw)) * CELL;
+#pragma unroll
+          for (int c = 0; c < NC; c++) w[e][c] = m * wd[c >> 2] * wh[(c >> 1) & 1] * ww[c & 1];
+        }
+        request(k + 2 < k1 ? k + 2 : kfirst);
         kt += 2;
-        o += 2 * s.nd * s.Q;
-        if (mk) mk += 2 * s.Q;
 #pragma unroll
         for (int u = 0; u < 2; u++)
           if (++kk == s.kw) { kk = 0; if (++kj == s.kh) { kj = 0; ++ki; } }
-        if (kt < k1) {  // the next pair's offsets are in flight during this pair's adds
-          dcn_offsets(s, o, fd, fh, fw);
-          if (mk) fm = load(mk);
-        }
-        CornerTaps t;
-        corner_taps<P>(s, pd, ph, pw, live && tap_on, 1u, 0u, ~0u, t);
-        int first;
-        unsigned bits = tile_bits(shape, origin, static_cast<int>(floor(pd)), static_cast<int>(floor(ph)), static_cast<int>(floor(pw)), first);
-        unsigned inside = 0;
+        unrolled(std::make_integer_sequence<int, TAPS>{}, [&](auto uc) {
+          constexpr int u = decltype(uc)::value;
+          if (k + u >= k1) return;
+          float4_t acc[BLOCKS];
+          product(weights, k + u, pg, acc);
+          const int next = k + (CH == 16 ? u + 1 : 2);
+          load_weights(next < k1 ? next : kfirst, weights);
+          unrolled(std::make_integer_sequence<int, 8 * SETS>{}, [&](auto ic) {
+            constexpr int i = decltype(ic)::value, e = i / 8, FROM = u * 8 + i % 8;   // position 4 j + i % 4 of block i / 4
+            const float gv = acc[i / 4][i % 4];
+            char *const dst = sums + row_word<CH, FROM>(cell[e]);
+            const double gd = static_cast<double>(gv) * scale.up;
 #pragma unroll
-        for (int c = 0; c < NC; c++) inside |= t.at[c] != ~0u ? 1u << c : 0u;
-        bits &= inside;
-        rec[0][lane] = __uint_as_float(static_cast<unsigned>(first) * 256u + bits);
-        rec[1][lane] = NARROW ? m * up : m;
-        rec[2][lane] = t.ld; rec[3][lane] = t.lh; rec[4][lane] = t.lw;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-#pragma unroll
-      for (int u = 0; u < (NARROW ? 2 : 1); u++) {
-        if (k + u >= k1) break;
-        float4_t acc[2];
-        product(wpair[u], k + u, acc);
-#pragma unroll
-        for (int blk = 0; blk < 2; blk++) {
-          const int at = (NARROW ? u : j / 2) * 32 + blk * 16 + p16;
-          const int word = __float_as_int(rec[0][at]);
-          const float m = rec[1][at], ld = rec[2][at], lh = rec[3][at], lw = rec[4][at];
-          const unsigned bits = static_cast<unsigned>(word) & 255u;
-          const float wd[2] = {1.f - ld, ld}, wh[2] = {1.f - lh, lh}, ww[2] = {1.f - lw, lw};
-          // (NARROW: channel 4 j + r of a voxel is its sum j + 4 r, so that the lanes of neighbouring voxels use all banks)
-          // the lane's sums of the first corner (the record's cell may lie before the tile: its corners do not)
-          char *const cell0 = reinterpret_cast<char *>(tile) + ((word >> 8) * STRIDE + (NARROW ? j : 4 * (j % 2))) * static_cast<int>(sizeof(Sum));
-          float gv[4];
-          double gd[4];
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            gv[r] = acc[blk][r] * m;
-            if constexpr (!NARROW) gd[r] = static_cast<double>(gv[r]) * scale.up;
-          }
-#pragma unroll
-          for (int c = 0; c < NC; c++) {
-            const int ca = c >> 2, cb = (c >> 1) & 1, ce = c & 1;
-            if ((bits >> c) & 1u) {
-              const float wc = wd[ca] * wh[cb] * ww[ce];
-              Sum *dst = reinterpret_cast<Sum *>(cell0 + (ca * (S::TH * S::TW) + cb * S::TW + ce) * (STRIDE * static_cast<int>(sizeof(Sum))));
-#pragma unroll
-              for (int r = 0; r < 4; r++) {
-                if constexpr (NARROW)
-                  __hip_atomic_fetch_add(dst + 4 * r, __float_as_int(fmaf(wc, gv[r], kMagic)) - 0x4B400000, __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_WORKGROUP);
-                else
-                  __hip_atomic_fetch_add(dst + r, fixed_term(wc, gd[r]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-              }
+            for (int c = 0; c < NC; c++) {
+              Sum *const to = reinterpret_cast<Sum *>(dst + ((c >> 2) * (S::TH * S::TW) + ((c >> 1) & 1) * S::TW + (c & 1)) * CELL);
+              const float wc = row_value<CH, FROM>(w[e][c]);
+              if constexpr (NARROW) __hip_atomic_fetch_add(to, round_word(wc * gv), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+              else __hip_atomic_fetch_add(to, fixed_term(wc, gd), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
-          }
-        }
+          });
+        });
       }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
     }
-  }
-  __syncthreads();
-  // ---- the tile's voxels inside the volume go to the gradient buffer, all channels of a voxel at once -----------
-  const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
-      gxt + static_cast<long>(b) * s.P * s.Cin, 0, static_cast<int>(s.P * s.Cin * 4), kRsrcFlags);
-  const unsigned cin4 = static_cast<unsigned>(s.Cin) * 4u;
-  const int slot = threadIdx.x % CH, ch = NARROW ? slot % 4 * 4 + slot / 4 : slot;
-  for (int cell = threadIdx.x / CH; cell < S::VOX; cell += WAVES * 64 / CH) {
-    const int zw = cell % S::TW + origin.w, zh = cell / S::TW % S::TH + origin.h, zd = cell / (S::TW * S::TH) + origin.d;
-    const Sum sum = tile[cell * STRIDE + slot];
-    const float v = NARROW ? static_cast<float>(sum) * down
-                           : static_cast<float>(static_cast<double>(static_cast<long long>(sum)) * scale.down);
-    if (zd >= 0 && zd < s.D && zh >= 0 && zh < s.H && zw >= 0 && zw < s.W && v != 0.f)
-      __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(
-          v, gr, static_cast<unsigned>((zd * s.H + zh) * s.W + zw) * cin4 + static_cast<unsigned>(c0 + ch) * 4u, 0, 0);
+    if (turn + 1 < turns) {   // the next turn's first weights
+      cl += CH;
+      load_weights(kfirst, weights);
+    }
+    __syncthreads();
+    // ---- the tile's voxels inside the volume go to the gradient buffer, all channels of a voxel at once: a row of the tile per
+    // wavefront, whose place is then scalar arithmetic ------------------------------------------------------------
+    for (int row = wave; row < S::TD * S::TH; row += WAVES) {
+      const int zd = row / S::TH + origin.d, zh = row % S::TH + origin.h;
+      if (zd < 0 || zd >= s.D || zh < 0 || zh >= s.H) continue;
+      const unsigned at = static_cast<unsigned>(((zd * s.H + zh) * s.W + origin.w) * s.Cin + c0) * 4u + place;   // (may lie before the row)
+      Sum *const from = tile + row * S::TW * CH + lane;
+#pragma unroll
+      for (int u = 0; u < TURNS; u++) {
+        const int cell = u * CELLS + first, zw = cell + origin.w;
+        if (S::TW % CELLS && u == TURNS - 1 && cell >= S::TW) continue;
+        const Sum sum = from[u * 64];
+        if (turn + 1 < turns) from[u * 64] = 0;
+        const float v = NARROW ? static_cast<float>(sum) * down
+                               : static_cast<float>(static_cast<double>(static_cast<long long>(sum)) * scale.down);
+        if (zw >= 0 && zw < s.W && v != 0.f)
+          __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(v, gr, at + u * turn_bytes, 0, 0);
+      }
+    }
+    c0 += CH;
+    if (turn + 1 < turns) __syncthreads();
   }
 }
 
 using TileVolume = Tile<10, 14, 14>;    // 4 x 8 x 8 positions: two voxels to spare at stride 1
 using TileStrided = Tile<12, 12, 13>;   // 4 x 4 x 4 positions: stride 2, dilation
-using TileImage = Tile<1, 44, 44>;      // 32 x 32 positions (16 x 16 at stride 2)
-using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions, two workgroups on a compute unit
+using TileImage = Tile<1, 44, 44>;      // 32 x 32 positions, 32-bit sums
+using TileWide = Tile<1, 28, 44>;       // 16 x 32 positions (8 x 16 at stride 2), 64-bit sums
+using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions
 
 // The brick and its tile: the first of the list whose tile holds the reach of the brick's undeformed taps with two voxels to spare
 // on either side, or one, if none has two.  Images with fewer workgroups than compute units take a smaller brick (77 us ->
 // 35 us for [1, 256 -> 128, 27 x 58]); volumes do not (the halo of 4 x 4 x 4 positions is most of their tile: 117 us
-// against 78 us for [2, 16 -> 128, 7 x 19 x 32]).  False: no brick fits.
+// against 78 us for [2, 16 -> 128, 7 x 19 x 32]).  Images with 64-bit sums have smaller tiles of 16 channels instead of 44 x 44 of 8:
+// half the samples to work out, and 5.5 million requests of 64 bytes instead of 9.9 of 32 for [8, 256 -> 256, 100 x 152].  False:
+// no brick fits.
 //
 // Width of the sums: 32 bits round every term to 14 - 22 bits of the workgroup's largest, which is worth their speed in dense
 // layers alone (16-bit tensors, the first brick fits: unit strides, taps close together; up to 128 output channels).  bf16 training
-// step of [2, 32 -> 64, 48^3]: 1178 us, 1393 us with 64-bit sums.  Strided and wide layers have 64-bit sums, as good as fp32 ones:
-// where the output's gradient is 2^-14 of what it is elsewhere in the brick, 32 bits left them 2 - 20 % off.  Training steps, 32
-// against 64 bits: [8, 256 -> 256, 100 x 152] fp16 2315 / 2337 us; stride 2, [8, 128 -> 128, 100 x 152] 332 / 370 us and
-// [2, 32 -> 64, 48^3] 297 / 345 us.
+// step of [2, 32 -> 64, 48^3]: 1178 us, 1393 us with 64-bit sums (with the kernel before this one).  Strided and wide layers have 64-bit sums, as good as fp32 ones:
+// where the output's gradient is 2^-14 of what it is elsewhere in the brick, 32 bits left them 2 - 20 % off. 
 bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
   static const int volumes[2][6] = {{2, 3, 3, 10, 14, 14}, {2, 2, 2, 12, 12, 13}};
-  static const int images[4][6] = {{0, 5, 5, 1, 44, 44}, {0, 4, 4, 1, 28, 28}, {0, 4, 4, 1, 44, 44}, {0, 3, 3, 1, 28, 28}};
+  static const int dense_images[3][6] = {{0, 5, 5, 1, 44, 44}, {0, 4, 4, 1, 28, 28}, {0, 3, 3, 1, 28, 28}};
+  static const int images[4][6] = {{0, 4, 5, 1, 28, 44}, {0, 4, 4, 1, 28, 28}, {0, 3, 4, 1, 28, 44}, {0, 3, 3, 1, 28, 28}};
   const bool image = s.nd == 2;
   const int st[3] = {s.sd, s.sh, s.sw}, kn[3] = {s.kd, s.kh, s.kw}, dl[3] = {s.dd, s.dh, s.dw}, on[3] = {s.Do, s.Ho, s.Wo};
-  int best = -1;
-  bool dense = false;
-  for (int i = 0; i < (image ? 4 : 2); i++) {
-    const int *e = image ? images[i] : volumes[i];
-    long spare = 1 << 20, bricks = s.B;
-    for (int a = 0; a < 3; a++) {
-      const long extent = static_cast<long>((1 << e[a]) - 1) * st[a] + static_cast<long>(kn[a] - 1) * dl[a] + 1;
-      if (!image || a > 0) spare = std::min(spare, e[3 + a] - extent);
-      bricks *= (on[a] + (1 << e[a]) - 1) >> e[a];
+  // voxels to spare in a tile; workgroups
+  const auto spare_of = [&](const int *e) {
+    long spare = 1 << 20;
+    for (int a = image ? 1 : 0; a < 3; a++)
+      spare = std::min(spare, e[3 + a] - (static_cast<long>((1 << e[a]) - 1) * st[a] + static_cast<long>(kn[a] - 1) * dl[a] + 1));
+    return (1L << (e[0] + e[1] + e[2])) * s.K >= (1L << 20) ? -1 : spare;
+  };
+  const auto workgroups = [&](const int *e, int channels) {
+    long bricks = s.B;
+    for (int a = 0; a < 3; a++) bricks *= (on[a] + (1 << e[a]) - 1) >> e[a];
+    return bricks * (s.Cin / channels);
+  };
+  const auto choose = [&](const int (*list)[6], int count, int channels) {
+    int best = -1;
+    for (int i = 0; i < count; i++) {
+      const int *e = list[i];
+      const long spare = spare_of(e);
+      if (spare < 2) continue;
+      const int rank = (spare >= 4 ? 2 : 0) + (image && workgroups(e, channels) >= 256 ? 1 : 0);
+      if (rank <= best) continue;
+      best = rank;
+      shape = ScatterShape{e[0], e[1], e[2], e[3], e[4], e[5], 0, 0, 0, (1 << (e[0] + e[1] + e[2])) * s.K, 0, 1};
     }
-    if (spare < 2 || (1L << (e[0] + e[1] + e[2])) * s.K >= (1L << 20)) continue;
-    dense = dense || i == 0;
-    const int rank = (spare >= 4 ? 2 : 0) + (image && bricks * (s.Cin / (dtype == MV_F32 ? 8 : 16)) >= 256 ? 1 : 0);
-    if (rank <= best) continue;
-    best = rank;
-    shape = ScatterShape{e[0], e[1], e[2], e[3], e[4], e[5], 0, 0, (1 << (e[0] + e[1] + e[2])) * s.K, 0};
+    return best >= 0;
+  };
+  // (offsets and weights at 32-bit byte offsets from scalar bases)
+  if (s.Cin / 8 > 65535 || s.Q >= (1L << 28) || static_cast<long>(s.K) * s.cpg * s.opg * (dtype == MV_F32 ? 4 : 2) >= (1L << 31)) return false;
+  bool fits = false;
+  if (dtype != MV_F32 && s.opg <= 128 && spare_of(image ? dense_images[0] : volumes[0]) >= 2) {
+    fits = image ? choose(dense_images, 3, 16) : choose(volumes, 2, 16);
+    shape.narrow = fits && scatter32_shift(shape.terms) >= kScatterMinShift;
   }
-  if (best < 0 || s.Cin / 8 > 65535) return false;
-  shape.narrow = dense && dtype != MV_F32 && s.opg <= 128 && scatter32_shift(shape.terms) >= kScatterMinShift;
+  if (!shape.narrow) fits = image ? choose(images, 4, 16) : choose(volumes, 2, 8);
+  if (!fits) return false;
+  shape.nbd = (s.Do + (1 << shape.bd) - 1) >> shape.bd;
   shape.nbh = (s.Ho + (1 << shape.bh) - 1) >> shape.bh;
   shape.nbw = (s.Wo + (1 << shape.bw) - 1) >> shape.bw;
-  return static_cast<long>(shape.nbh) * shape.nbw * ((s.Do + (1 << shape.bd) - 1) >> shape.bd) < (1L << 31);
+  // wide images: 32 channels in two turns, which share grad_output, while that leaves four workgroups per compute unit
+  // (fp16 [8, 256 -> 256, 100 x 152]: 500 us, 575 us in one turn, four turns the same)
+  shape.turns = image && static_cast<double>(shape.nbd) * shape.nbh * shape.nbw * s.B * (s.Cin / 16) >= 2048 ? 2 : 1;
+  return static_cast<double>(shape.nbd) * shape.nbh * shape.nbw * s.B * (s.Cin / 8) < static_cast<double>(1L << 31);
 }
 
 template <typename T, typename S>
 static int scatter_launch(const void *off, const void *mask, const void *gyt, const void *wf, float *gxt, const DcnDims &s,
                           const ScatterShape &shape, const unsigned *bounds, hipStream_t stream) {
-  const int nbd = (s.Do + (1 << shape.bd) - 1) >> shape.bd;
-  const bool wide = s.opg > 4 * 64 / static_cast<int>(sizeof(T));
-  const dim3 grid(static_cast<unsigned>(nbd) * shape.nbh * shape.nbw, s.Cin / (shape.narrow ? 16 : 8), s.B);
+  const int slices = s.opg / (64 / static_cast<int>(sizeof(T)));
 #define MV_SCATTER(NARROWV, KEEPV)                                                                                    \
-  hipLaunchKernelGGL((dcn_backward_scatter_kernel<T, NARROWV, S, KEEPV>), grid, dim3(KEEPV == 4 ? 1024 : 512), 0, stream,     \
+  hipLaunchKernelGGL((dcn_backward_scatter_kernel<T, NARROWV, S, KEEPV>),                                              \
+                     dim3(static_cast<unsigned>(shape.nbd) * shape.nbh * shape.nbw * s.B * (s.Cin / (S::template channels<NARROWV> * (KEEPV == 8 ? shape.turns : 1)))), \
+                     dim3(KEEPV <= 4 ? 1024 : 512), 0, stream,                                                         \
                      static_cast<const T *>(off), static_cast<const T *>(mask), static_cast<const T *>(gyt),          \
                      static_cast<const T *>(wf), gxt, s, shape, bounds)
   if (shape.narrow) {
-    if constexpr (sizeof(T) == 2) MV_SCATTER(true, 4);   // (never wide)
-  } else {
-    if (wide) MV_SCATTER(false, 8); else MV_SCATTER(false, 4);
+    if constexpr (sizeof(T) == 2 && !std::is_same<S, TileWide>::value) {   // (never wide)
+      if (slices <= 2) MV_SCATTER(true, 2); else MV_SCATTER(true, 4);
+    }
+  } else if constexpr (!std::is_same<S, TileImage>::value) {
+    if (slices <= 2) MV_SCATTER(false, 2);
+    else if (slices <= 4) MV_SCATTER(false, 4);
+    else MV_SCATTER(false, 8);
   }
 #undef MV_SCATTER
   return check_launch("dcn_backward_scatter_kernel");
@@ -340,7 +453,8 @@ int dcn_scatter(const void *off, const void *mask, const void *gyt, const void *
 #define MV_SCATTER_AS(T)                                                                                              \
   (shape.th == TileVolume::TH ? MV_SCATTER_TILE(T, TileVolume)                                                          \
    : shape.th == TileStrided::TH ? MV_SCATTER_TILE(T, TileStrided)                                                      \
-   : shape.th == TileImage::TH ? MV_SCATTER_TILE(T, TileImage) : MV_SCATTER_TILE(T, TileSmall))
+   : shape.th == TileImage::TH ? MV_SCATTER_TILE(T, TileImage)                                                        \
+   : shape.tw == TileWide::TW ? MV_SCATTER_TILE(T, TileWide) : MV_SCATTER_TILE(T, TileSmall))
   if (dtype == MV_F16) return MV_SCATTER_AS(__half);
   if (dtype == MV_F32) return MV_SCATTER_AS(float);
   return MV_SCATTER_AS(__hip_bfloat16);

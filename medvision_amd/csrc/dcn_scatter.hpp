@@ -14,9 +14,10 @@ constexpr int kRsrcFlags = 0x00020000;
 // others are added to the gradient buffer by the tap kernel, 128 bytes per request.
 struct ScatterShape {
   int bd, bh, bw, td, th, tw;
-  int nbh, nbw;   // bricks per column and row of bricks
+  int nbd, nbh, nbw;   // bricks along the axes
   int terms;      // corners that a voxel of a tile can take: positions of the brick times taps
   int narrow;     // 32-bit sums instead of 64-bit ones (dcn_scatter_plan)
+  int turns;      // blocks of sixteen channels of a workgroup (wide images)
 };
 struct TileOrigin { int d, h, w; };
 __device__ __forceinline__ TileOrigin tile_origin(const DcnDims &s, const ScatterShape &t, int bz, int by, int bx) {

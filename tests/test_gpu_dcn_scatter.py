@@ -1,0 +1,59 @@
+"""The input's gradient of deformable layers at the edges of the LDS tiles that sum it, against the fp64 oracle: every brick and tile,
+counts of output channels around the slices that a wavefront keeps, samples on the tiles' and the input's borders."""
+import pytest
+import torch
+
+from parity import BWD_TOL, assert_close
+import workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def _gradient(oracle, dtype, batch, cin, cout, size, stride, groups, dg, offsets, seed):
+    if len(size) == 3:
+        from medvision_amd.ops.modulated_deform_conv_3d import modulated_deform_conv
+    else:
+        from medvision_amd.ops.modulated_deform_conv_2d import modulated_deform_conv
+    g = wl.gen(seed)
+    x, off, mask, w, b = wl.dcn_inputs(g, batch, cin, cout, size, 3, dg, groups, dtype, stride, 1, 1)
+    off = offsets(off, g).to(dtype)
+    leaves = [t.to(DEV).requires_grad_(True) for t in (x, off, mask, w, b)]
+    y = modulated_deform_conv(*leaves, stride, 1, 1, groups, dg)
+    gy = torch.randn(y.shape, generator=g).to(dtype)
+    y.backward(gy.to(DEV))
+    want = oracle.dcn3d_backward(x, off, mask, w, gy, True, stride, 1, 1, groups, dg)[0]
+    assert_close(leaves[0].grad, want, BWD_TOL[dtype], "input")
+
+
+def _borders(off, g):
+    """Whole and half voxels up to beyond the tiles, a few samples exactly one voxel outside, a few very far away."""
+    whole = torch.randint(-9, 10, off.shape, generator=g).float()
+    pick = torch.rand(off.shape, generator=g)
+    return torch.where(pick < 0.5, whole, torch.where(pick < 0.98, whole + 0.5, torch.where(pick < 0.99, -1.0, 3e4)))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("cin,cout,size,stride,groups,dg", [
+    (32, 32, (5, 9, 17), 1, 1, 1),        # volumes: a brick and a remainder along every axis
+    (64, 96, (4, 8, 9), 1, 1, 2),         # three slices of grad_output, two deformable groups
+    (32, 160, (6, 9, 10), 2, 1, 1),       # strided, more slices than four
+    (32, 64, (33, 35), 1, 1, 1),          # images: a brick of 32 x 32 (16 x 32) and a remainder
+    (64, 288, (17, 33), 1, 1, 1),         # more slices than eight
+    (64, 64, (31, 67), 2, 2, 2),          # strided, groups
+    (512, 32, (20, 20), 1, 1, 1),         # many channel blocks
+])
+def test_samples_on_borders(oracle, dtype, cin, cout, size, stride, groups, dg):
+    _gradient(oracle, dtype, 2, cin, cout, size, stride, groups, dg, _borders, cin + cout + sum(size))
+
+
+@pytest.mark.parametrize("dtype,batch,cout,size", [
+    (torch.float16, 64, 160, (5, 7)),     # 2048 workgroups, bricks of which most groups do not exist
+    (torch.bfloat16, 16, 160, (17, 33)),
+    (torch.float32, 64, 96, (5, 7)),
+    (torch.float16, 63, 160, (5, 7)),     # one image fewer: one block of channels per workgroup
+])
+def test_two_channel_blocks_per_workgroup(oracle, dtype, batch, cout, size):
+    """Wide images of 2048 and more workgroups of sixteen channels sum 32 channels in two turns."""
+    _gradient(oracle, dtype, batch, 512, cout, size, 1, 1, 1, lambda off, g: off, batch + sum(size))
