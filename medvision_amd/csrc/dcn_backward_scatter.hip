@@ -358,7 +358,11 @@ __global__ __launch_bounds__(KEEP <= 4 ? 1024 : 512) void dcn_backward_scatter_k
   }
 }
 
-using TileVolume = Tile<10, 14, 14>;    // 4 x 8 x 8 positions: two voxels to spare at stride 1
+// 4 x 8 x 8 positions at stride 1: six voxels to spare along d, four along h and w.  A voxel more on either side along d costs 20 % more of
+// the tile's atomics (10 us for bf16 [2, 32 -> 64, 48^3]) and leaves two thirds of the corners that the tap kernel adds one by
+// one (offsets of sigma = 2: 8.4 -> 5.7 %; that kernel 504 -> 462 us); 12 x 14 x 15 and 11 x 15 x 15 were no faster, layers of small offsets
+// do not change.
+using TileVolume = Tile<12, 14, 14>;
 using TileStrided = Tile<12, 12, 13>;   // 4 x 4 x 4 positions: stride 2, dilation
 using TileImage = Tile<1, 44, 44>;      // 32 x 32 positions, 32-bit sums
 using TileWide = Tile<1, 28, 44>;       // 16 x 32 positions (8 x 16 at stride 2), 64-bit sums
@@ -376,7 +380,7 @@ using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions
 // step of [2, 32 -> 64, 48^3]: 1178 us, 1393 us with 64-bit sums (with the kernel before this one).  Strided and wide layers have 64-bit sums, as good as fp32 ones:
 // where the output's gradient is 2^-14 of what it is elsewhere in the brick, 32 bits left them 2 - 20 % off. 
 bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
-  static const int volumes[2][6] = {{2, 3, 3, 10, 14, 14}, {2, 2, 2, 12, 12, 13}};
+  static const int volumes[2][6] = {{2, 3, 3, 12, 14, 14}, {2, 2, 2, 12, 12, 13}};
   static const int dense_images[3][6] = {{0, 5, 5, 1, 44, 44}, {0, 4, 4, 1, 28, 28}, {0, 3, 3, 1, 28, 28}};
   static const int images[4][6] = {{0, 4, 5, 1, 28, 44}, {0, 4, 4, 1, 28, 28}, {0, 3, 4, 1, 28, 44}, {0, 3, 3, 1, 28, 28}};
   const bool image = s.nd == 2;
