@@ -234,28 +234,25 @@ __device__ __forceinline__ void dcn_zero_f32_block(float *p, long n, const unsig
   for (long i = bid * 256L + threadIdx.x; i < n; i += nblocks * 256L) p[i] = 0.f;
 }
 
-// One pass over a slab of grad_output[b, o, .]: its sum into the fp32 bias accumulator and (`out`
-// given) its largest magnitude as a bit pattern into *out.  Workgroup = (o, b, slab of `slab_len`
-// positions); about 512 workgroups in all — enough loads in flight for the memory system, and few enough
-// for the atomics on the one word of the maximum, which retire one after the other (~10 ns each).
+// One pass over grad_output[b, o, .]: the sums of its rows into the fp32 bias accumulator and (`out` given) its largest magnitude as a
+// bit pattern into *out.  About 512 workgroups in all — enough loads in flight for the memory system, and few enough for the
+// atomics on the one word of the maximum, which retire one after the other (~10 ns each): a workgroup takes a slab of
+// `slab_len` positions of a row, or (`rows` > 0: many rows) each of its wavefronts `rows` whole rows.
+//   (2048 rows of 15 200 positions, fp16, a workgroup per row: 57 us; 27 us with a row per wavefront.)
+static long gy_rows(const DcnDims &s) { return static_cast<long>(s.Cout) * s.B; }
 static long gy_slab_len(const DcnDims &s) {
-  const long rows = static_cast<long>(s.Cout) * s.B;
-  const long slabs = std::max(1L, std::min((s.Q + 2047) / 2048, (512 + rows - 1) / rows));
+  const long rows = gy_rows(s), slabs = std::max(1L, std::min((s.Q + 2047) / 2048, (512 + rows - 1) / rows));
   return ((s.Q + slabs - 1) / slabs + 1023) / 1024 * 1024;
 }
-template <typename T>
-__device__ __forceinline__ void dcn_gy_sum_max_block(const T *__restrict__ gy, float *__restrict__ gb32, unsigned *out,
-                                                     const DcnDims s, const long slab_len, const unsigned bid) {
+static int gy_rows_per_wave(const DcnDims &s) {   // 0: slabs
+  const long rows = gy_rows(s);
+  return rows < 1024 ? 0 : static_cast<int>((rows + 2047) / 2048);
+}
+// sum and largest magnitude of src[q0 .. q_end), `threads` threads, PIECES independent 16-byte loads each
+template <typename T, int PIECES>
+__device__ __forceinline__ void gy_sum_max(const T *__restrict__ src, long q0, const long q_end, const int thread, const int threads,
+                                           float &v, float &m, bool &bad) {
   constexpr int V = 16 / static_cast<int>(sizeof(T));
-  __shared__ float sums[4];
-  const unsigned slabs = static_cast<unsigned>((s.Q + slab_len - 1) / slab_len);
-  const unsigned slab = bid % slabs, r = bid / slabs;
-  const int b = static_cast<int>(r % s.B), o = static_cast<int>(r / s.B);
-  const T *src = gy + (static_cast<long>(b) * s.Cout + o) * s.Q;
-  long q0 = static_cast<long>(slab) * slab_len;
-  const long q_end = min(q0 + slab_len, s.Q);
-  float v = 0.f, m = 0.f;
-  bool bad = false;
   auto take = [&](T e) {
     const float x = static_cast<float>(load(&e));
     v += x;
@@ -263,23 +260,46 @@ __device__ __forceinline__ void dcn_gy_sum_max_block(const T *__restrict__ gy, f
     m = fmaxf(m, fabsf(x));
   };
   if (reinterpret_cast<uintptr_t>(src + q0) % 16 == 0) {
-    // 16-byte pieces, four independent loads per lane and step
     const long groups = (q_end - q0) / V;
     const u32x4 *pieces = reinterpret_cast<const u32x4 *>(src + q0);
-    for (long i = threadIdx.x; i < groups; i += 1024) {
-      union { u32x4 u; T e[V]; } raw[4];
+    for (long i = thread; i < groups; i += PIECES * threads) {
+      union { u32x4 u; T e[V]; } raw[PIECES];
 #pragma unroll
-      for (int u = 0; u < 4; u++) raw[u].u = i + u * 256 < groups ? pieces[i + u * 256] : u32x4{0u, 0u, 0u, 0u};
+      for (int u = 0; u < PIECES; u++) raw[u].u = i + u * threads < groups ? pieces[i + u * threads] : u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-      for (int u = 0; u < 4; u++)
+      for (int u = 0; u < PIECES; u++)
 #pragma unroll
         for (int e = 0; e < V; e++) take(raw[u].e[e]);
     }
     q0 += groups * V;
   }
-  for (long q = q0 + threadIdx.x; q < q_end; q += 256) take(src[q]);
+  for (long q = q0 + thread; q < q_end; q += threads) take(src[q]);
+}
+template <typename T>
+__device__ __forceinline__ void dcn_gy_sum_max_block(const T *__restrict__ gy, float *__restrict__ gb32, unsigned *out,
+                                                     const DcnDims s, const long slab_len, const int rows, const unsigned bid) {
+  __shared__ float sums[4];
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  float v = 0.f, m = 0.f;
+  bool bad = false;
+  const long total = static_cast<long>(s.Cout) * s.B;
+  if (rows > 0) {
+    for (long r = (bid * 4L + wave) * rows, last = min(r + rows, total); r < last; r++) {   // (rows are [b][o])
+      v = 0.f;
+      gy_sum_max<T, 8>(gy + r * s.Q, 0, s.Q, lane, kWave, v, m, bad);
+      for (int sh = 32; sh > 0; sh >>= 1) v += __shfl_xor(v, sh);
+      if (lane == 0) atomicAdd(gb32 + r % s.Cout, v);
+    }
+    if (out) fold_max(bad ? 0x7fc00000u : __float_as_uint(m), out);
+    return;
+  }
+  const unsigned slabs = static_cast<unsigned>((s.Q + slab_len - 1) / slab_len);
+  const unsigned slab = bid % slabs, r = bid / slabs;
+  const int b = static_cast<int>(r % s.B), o = static_cast<int>(r / s.B);
+  const long q0 = static_cast<long>(slab) * slab_len;
+  gy_sum_max<T, 4>(gy + (static_cast<long>(b) * s.Cout + o) * s.Q, q0, min(q0 + slab_len, s.Q), threadIdx.x, 256, v, m, bad);
   for (int sh = 32; sh > 0; sh >>= 1) v += __shfl_xor(v, sh);
-  if (threadIdx.x % kWave == 0) sums[threadIdx.x / kWave] = v;
+  if (lane == 0) sums[wave] = v;
   if (out) fold_max(bad ? 0x7fc00000u : __float_as_uint(m), out);   // (contains the barrier)
   else __syncthreads();
   if (threadIdx.x == 0) atomicAdd(gb32 + o, (sums[0] + sums[1]) + (sums[2] + sums[3]));
@@ -318,12 +338,12 @@ __global__ __launch_bounds__(256) void dcn_backward_maxima_kernel(const T *__res
                                                                   const T *__restrict__ mask, const long nmask,
                                                                   const T *__restrict__ wt, const DcnDims s,
                                                                   unsigned *__restrict__ bounds, float *__restrict__ gb32,
-                                                                  const long slab_len, const unsigned gy_blocks,
+                                                                  const long slab_len, const int rows, const unsigned gy_blocks,
                                                                   const unsigned mask_blocks) {
   const unsigned id = blockIdx.x;
   if (id < gy_blocks) {
-    // with a bias gradient to form the pass over grad_output also sums it, a workgroup per (o, b, slab)
-    if (gb32) dcn_gy_sum_max_block<T>(gy, gb32, bounds, s, slab_len, id);
+    // with a bias gradient to form the pass over grad_output also sums it
+    if (gb32) dcn_gy_sum_max_block<T>(gy, gb32, bounds, s, slab_len, rows, id);
     else dcn_absmax_block<T>(gy, ngy, bounds, id, gy_blocks);
   } else if (id < gy_blocks + mask_blocks) dcn_absmax_block<T>(mask, nmask, bounds + 2, id - gy_blocks, mask_blocks);
   else dcn_weight_colsum_block<T>(wt, s, bounds + 1, id - gy_blocks - mask_blocks);
@@ -404,14 +424,15 @@ static int backward_run(const void *x, const void *off, const void *mask, const 
                      static_cast<const T *>(gy), gyt, static_cast<const T *>(wt), wb, gxt, nz, real, pad, j);
   if (tiles || want_bias) {
     const long slab_len = gy_slab_len(real);
-    const long sum_blocks = static_cast<long>(real.Cout) * s.B * ((s.Q + slab_len - 1) / slab_len);
+    const int rows = gy_rows_per_wave(real);
+    const long sum_blocks = rows > 0 ? (gy_rows(real) + 4L * rows - 1) / (4L * rows) : gy_rows(real) * ((s.Q + slab_len - 1) / slab_len);
     const unsigned gy_blocks = static_cast<unsigned>(want_bias ? sum_blocks : min((ngy + 8191) / 8192, 256L));
     const unsigned mask_blocks = mask && tiles ? static_cast<unsigned>(min((nmask + 8191) / 8192, 256L)) : 0u;
     const unsigned col_blocks = tiles ? static_cast<unsigned>((ncols + 63) / 64) : 0u;
     MV_REQUIRE(sum_blocks < (1L << 30), "grid too large");
     hipLaunchKernelGGL((dcn_backward_maxima_kernel<T>), dim3(gy_blocks + mask_blocks + col_blocks), dim3(256), 0, stream,
                        static_cast<const T *>(gy), ngy, static_cast<const T *>(mask), nmask, static_cast<const T *>(wt), real,
-                       tiles ? bounds : nullptr, want_bias ? *gb32 : nullptr, slab_len, gy_blocks, mask_blocks);
+                       tiles ? bounds : nullptr, want_bias ? *gb32 : nullptr, slab_len, rows, gy_blocks, mask_blocks);
   }
   int st = check_launch("dcn_backward_prepare_kernel");
   if (st) return st;
