@@ -90,21 +90,16 @@ __global__ __launch_bounds__(kClThreads) void roi_forward_cl_kernel(const T *__r
           const float lx = __shfl(rec_fx, from), ly = __shfl(rec_fy, from), lz = __shfl(rec_fz, from);
           if (at0 < 0 || !loads) continue;
           const unsigned at = static_cast<unsigned>(at0) + static_cast<unsigned>(c0) * ES;
-          auto take = [&](u32x4 r, float (&v)[V]) {
-            if constexpr (ES == 4) {
-              v[0] = __uint_as_float(r.x); v[1] = __uint_as_float(r.y); v[2] = __uint_as_float(r.z); v[3] = __uint_as_float(r.w);
-            } else {
-              union { u32x4 u; T e[8]; } w;
-              w.u = r;
-#pragma unroll
-              for (int i = 0; i < 8; i++) v[i] = static_cast<float>(load(&w.e[i]));
-            }
+          auto element = [](u32x4 r, int i) {
+            if constexpr (ES == 4) return __uint_as_float(r[i]);
+            union { u32x4 u; T e[V]; } x;
+            x.u = r;
+            return static_cast<float>(load(&x.e[i]));
           };
           if (p.order == 0) {
-            float v[V];
-            take(__builtin_amdgcn_raw_buffer_load_b128(xr, at, 0, 0), v);
+            const u32x4 r = __builtin_amdgcn_raw_buffer_load_b128(xr, at, 0, 0);
 #pragma unroll
-            for (int i = 0; i < V; i++) acc[i] += v[i];
+            for (int i = 0; i < V; i++) acc[i] += element(r, i);
             continue;
           }
           const unsigned dx = (step & 1u) ? cbytes : 0u, dy = (step & 2u) ? sy : 0u, dz = (step & 4u) ? sz : 0u;
@@ -113,13 +108,25 @@ __global__ __launch_bounds__(kClThreads) void roi_forward_cl_kernel(const T *__r
           for (int k = 0; k < 8; k++)
             raw[k] = __builtin_amdgcn_raw_buffer_load_b128(xr, at + ((k & 4) ? dz : 0u) + ((k & 2) ? dy : 0u) + ((k & 1) ? dx : 0u), 0, 0);
           const float hx = 1.f - lx, hy = 1.f - ly, hz = 1.f - lz;
-          float v[8][V];
+          if constexpr (ES == 4) {
 #pragma unroll
-          for (int k = 0; k < 8; k++) take(raw[k], v[k]);
+            for (int i = 0; i < V; i++) {
+              float v[8];
 #pragma unroll
-          for (int i = 0; i < V; i++)
-            acc[i] += hz * (hy * (hx * v[0][i] + lx * v[1][i]) + ly * (hx * v[2][i] + lx * v[3][i])) +
-                      lz * (hy * (hx * v[4][i] + lx * v[5][i]) + ly * (hx * v[6][i] + lx * v[7][i]));
+              for (int k = 0; k < 8; k++) v[k] = element(raw[k], i);
+              acc[i] += hz * (hy * (hx * v[0] + lx * v[1]) + ly * (hx * v[2] + lx * v[3])) +
+                        lz * (hy * (hx * v[4] + lx * v[5]) + ly * (hx * v[6] + lx * v[7]));
+            }
+          } else {
+            // one multiply-add per tap, which reads the 16-bit element as it is (bf16: a shift before it); blended axis by axis as above
+            // a tap costs two and a conversion: 84 % vector issue, now 61 %
+            const float w00 = hz * hy, w01 = hz * ly, w10 = lz * hy, w11 = lz * ly;
+            const float w[8] = {w00 * hx, w00 * lx, w01 * hx, w01 * lx, w10 * hx, w10 * lx, w11 * hx, w11 * lx};
+#pragma unroll
+            for (int k = 0; k < 8; k++)
+#pragma unroll
+              for (int i = 0; i < V; i++) acc[i] = fmaf(w[k], element(raw[k], i), acc[i]);
+          }
         }
       }
       if (cell_on && loads) {
@@ -167,9 +174,13 @@ int roi_forward_cl(const void *input, const void *rois, void *output, int dtype,
   cs.passes = (pieces + cs.lanes - 1) / cs.lanes;
   const long cells = static_cast<long>(p.od) * p.oh * p.ow;
   const int per_turn = (kClThreads / kWave) * cs.slots;   // cells a workgroup takes at a time
-  // a roi per workgroup when there are many; few rois are split so that ~1024 workgroups exist
-  long chunks = (1024 + p.R - 1) / p.R;
-  chunks = std::max(1L, std::min(chunks, (cells + per_turn - 1) / per_turn));
+  // Workgroups of about eight samples per lane, short enough to fill the chip evenly to the end (fp16, 1000 rotated rois x 64 channels x
+  // 7^3 cells, eight samples each: 172 us with two workgroups per roi, 141 with eleven), long enough for the roi's geometry (1181
+  // rois x 7^2 cells of one sample: 28 us with one, 37 with four); few rois are split so that ~1024 workgroups exist, many to 16 384.
+  const long grid_of = p.sampling_ratio > 0 ? p.sampling_ratio : 2, samples = p.ndim == 3 ? grid_of * grid_of * grid_of : grid_of * grid_of;
+  const long turns = (cells + per_turn - 1) / per_turn, least = std::max(1L, 8 / samples);   // turns of a workgroup
+  long chunks = std::max((1024 + p.R - 1L) / p.R, std::min((16384 + p.R - 1L) / p.R, turns / least));
+  chunks = std::max(1L, std::min(chunks, turns));
   cs.chunk = static_cast<int>(((cells + chunks - 1) / chunks + per_turn - 1) / per_turn * per_turn);
   cs.chunks = static_cast<int>((cells + cs.chunk - 1) / cs.chunk);
   const dim3 grid(cs.chunks, p.R), block(kClThreads);
