@@ -21,18 +21,21 @@
 // Corners that the LDS scatter does not take are listed when the records are made, and their 32 channels are added as
 // 128 contiguous bytes.
 // What bounds it: narrow layers the vector instructions of the samples (184 per 16 positions and 32 channels, and as many more
-// for everything else; vector issue 56 %) and the latency of the gathers (50 % of the wavefronts' time in waits), wide ones LDS
-// (45 %, half of it bank conflicts; vector issue 25 %, matrix cores 17 %) and the same waits, and everywhere the atomics of the
-// far corners (64 bytes per corner and 16 channels, 21 G of them a second at best).
-//   (bf16 [2, 32 -> 64, 48^3]: 493 us; the data and weight kernels before it took 670 us.  fp16 images
-//   [8, 256 -> 256, 100 x 152]: 762 us, 4380 us before.  [1, 128 -> 128, 7 x 45 x 18]: 64 us, 790 us before.)
+// for everything else; vector issue 68 %) and the latency of the gathers (47 % of the wavefronts' time in waits), wide ones LDS
+// (43 %; vector issue 29 %, matrix cores 20 %) and the same waits, and everywhere the atomics of the far corners (64 bytes per corner
+// and 16 channels, 21 G of them a second at best).
+//   (bf16 [2, 32 -> 64, 48^3]: 409 us; the data and weight kernels before it took 670 us.  fp16 images
+//   [8, 256 -> 256, 100 x 152]: 582 us, 4380 us before.  [1, 128 -> 128, 7 x 45 x 18]: 64 us, 790 us before.)
 #include "dcn_scatter.hpp"
+
+#include <algorithm>
 
 namespace mv {
 
-// One 16-byte piece (kPiece neighbouring channels of a position) of an LDS block [piece][position]: rows of 68 pieces, so that
-// both the four pieces of neighbouring positions and one piece of sixteen positions fall on different banks.
-constexpr int kTapTile = 64, kTapPitch = kTapTile + 4;   // positions per turn
+// One 16-byte piece (kPiece neighbouring channels of a position) of an LDS block [piece][position]: rows of 69 pieces, so that
+// eight pieces of a position, the four pieces of neighbouring positions and one piece of sixteen positions fall on different banks
+// (rows of 68: eight pieces of a position on four sets of banks; fp16 [8, 256 -> 256, 100 x 152] 616 us, 582 us with 69).
+constexpr int kTapTile = 64, kTapPitch = kTapTile + 5;   // positions per turn
 __device__ __forceinline__ int tap_slot(int piece, int position) { return piece * kTapPitch + position; }
 
 // Operand of a product over positions from such a block: row `block * 16 + lane % 16` (a channel), the kPiece positions
@@ -68,6 +71,11 @@ struct TapPiece { int k_first, taps, q_first, positions; };
 template <typename T, int NC, int OBW, int CBW>
 constexpr int TAP_WAVES = OBW * CBW >= 8 || (NC == 8 && (sizeof(T) == 4 || OBW >= 2)) ? 2 : OBW == 1 && CBW == 2 && sizeof(T) == 2 ? 4 : 3;
 
+// blocks of 16 channels of gcol per wavefront: two where that halves the reads of grad_output from LDS (a block of four positions each
+// would do too, but the registers leave room for two: fp16 [8, 256 -> 256, 100 x 152] 638 -> 616 us, four 740 us;
+// bf16 [2, 128 -> 128, 112 x 208] training step 312 -> 295 us)
+template <typename T, int NC, int OBW, int CBW> constexpr int TAP_BLOCKS = CBW == 4 ? 2 : 1;
+
 // OBW: blocks of 16 output channels per wavefront (every fourth block of the 64 * OBW rows from row0; layers with more rows
 // take several passes, gcol and all that follows from it being sums over them).  CBW: blocks of 16 input channels of a
 // chunk.  NC: corners, 8 for volumes, 4 for images.
@@ -92,11 +100,12 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
   const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int j = lane % 16, kc = lane / 16;   // matrix layout
   const int lj = lane / 4, lk = lane % 4;    // load layout
-  // (taps of one range next to each other, on one XCD: they gather the same part of x and read the same gy)
-  const int id = static_cast<int>(xcd_contiguous(blockIdx.x, gridDim.x)), k = piece.k_first + id % piece.taps;
-  const int dgi = blockIdx.y / chunks, part = blockIdx.y % chunks, b = blockIdx.z;
+  // (taps and chunks of one range next to each other, on one XCD: they gather the same part of x and read the same gy)
+  const unsigned wg = xcd_contiguous(blockIdx.x, gridDim.x), inner = piece.taps * s.dg * chunks, ranges = gridDim.x / (inner * s.B);
+  const int k = piece.k_first + static_cast<int>(wg % piece.taps), slice = static_cast<int>(wg / piece.taps % (s.dg * chunks));
+  const int dgi = slice / chunks, part = slice % chunks, b = static_cast<int>(wg / inner / ranges);
   const int c0 = dgi * s.cpd + part * CW, g = c0 / s.cpg;
-  const int within = id / piece.taps * range;   // < 2^31: within.. is a range of the piece
+  const int within = static_cast<int>(wg / inner % ranges) * range;   // < 2^31: within.. is a range of the piece
   const long q0 = piece.q_first + static_cast<long>(within);
   const int count = min(range, piece.positions - within);   // positions of the range
   const long bg = static_cast<long>(b) * s.dg + dgi;
@@ -107,15 +116,17 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
       gxt + static_cast<long>(b) * s.P * s.Cin, 0, static_cast<int>(s.P * s.Cin * 4), kRsrcFlags);
   const bool split = bounds && scatter_scale(bounds, shape.terms, mask != nullptr).valid;
 
-  // gcol: wavefront w forms the channels of block w % CBW for CBW blocks of sixteen positions; its rows of the weight stay
+  // gcol: a wavefront forms WB blocks of sixteen channels for CBW / WB blocks of sixteen positions; its rows of the weight stay
   // in registers for the whole range
-  const int wblock = wave % CBW, wfirst = wave / CBW * CBW;
-  u32x4 wreg[STEPS];
-  {
-    const T *src = wf + (((static_cast<long>(g) * s.K + k) * (s.cpg / 16) + (c0 - g * s.cpg) / 16 + wblock) * (s.opg / SL) + row0 / SL) * (64 * PC) + lane * PC;
+  constexpr int WB = TAP_BLOCKS<T, NC, OBW, CBW>, WP = CBW / WB;
+  const int wblock = wave % (CBW / WB) * WB, wfirst = wave / (CBW / WB) * WP;
+  u32x4 wreg[WB][STEPS];
+#pragma unroll
+  for (int w = 0; w < WB; w++) {
+    const T *src = wf + (((static_cast<long>(g) * s.K + k) * (s.cpg / 16) + (c0 - g * s.cpg) / 16 + wblock + w) * (s.opg / SL) + row0 / SL) * (64 * PC) + lane * PC;
 #pragma unroll
     for (int st = 0; st < STEPS; st++)
-      wreg[st] = st < steps ? *reinterpret_cast<const u32x4 *>(src + st * (64 * PC)) : u32x4{0u, 0u, 0u, 0u};
+      wreg[w][st] = st < steps ? *reinterpret_cast<const u32x4 *>(src + st * (64 * PC)) : u32x4{0u, 0u, 0u, 0u};
   }
   // grad_output of a tile, loaded a tile ahead where the registers allow it: thread t has piece t % NP of positions t / NP +
   // u * 256 / NP (positions and rows that do not exist: zeros)
@@ -226,16 +237,24 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
     gather(raw[0], 0);
     if (AHEAD) stage(tile + 1);   // (beyond the last one: zeros)
     {
-      float4_t gc[CBW];
+      float4_t gc[WB][WP];
 #pragma unroll
-      for (int n = 0; n < CBW; n++) gc[n] = float4_t{0.f, 0.f, 0.f, 0.f};
+      for (int w = 0; w < WB; w++)
+#pragma unroll
+        for (int n = 0; n < WP; n++) gc[w][n] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int st = 0; st < STEPS; st++)
 #pragma unroll
-        for (int n = 0; n < CBW; n++) gc[n] = M::run16(wreg[st], gyl[tap_slot(st * 4 + kc, (wfirst + n) * 16 + j)], gc[n]);
+        for (int n = 0; n < WP; n++) {
+          const u32x4 gy = gyl[tap_slot(st * 4 + kc, (wfirst + n) * 16 + j)];
 #pragma unroll
-      for (int n = 0; n < CBW; n++)
-        *reinterpret_cast<float4 *>(&gcol[(wfirst + n) * 16 + j][wblock * 16 + 4 * kc]) = make_float4(gc[n][0], gc[n][1], gc[n][2], gc[n][3]);
+          for (int w = 0; w < WB; w++) gc[w][n] = M::run16(wreg[w][st], gy, gc[w][n]);
+        }
+#pragma unroll
+      for (int w = 0; w < WB; w++)
+#pragma unroll
+        for (int n = 0; n < WP; n++)
+          *reinterpret_cast<float4 *>(&gcol[(wfirst + n) * 16 + j][(wblock + w) * 16 + 4 * kc]) = make_float4(gc[w][n][0], gc[w][n][1], gc[w][n][2], gc[w][n][3]);
     }
     __syncthreads();   // gcol is complete
     // sums over the lane's channels: differences along w (along h, d), value
@@ -396,18 +415,47 @@ bool dcn_tap_supported(const DcnDims &s, int dtype) {
   return s.Q < (1L << 31) && s.Cout <= 65536 && static_cast<long>(s.dg) * tap_chunks(s, dtype) <= 65535 && static_cast<long>(s.dg) * s.K <= 65535;
 }
 
+// Ranges of positions.  The workgroups of a launch do the same work, so that they should fill the places on the chip (`slots`) a whole
+// number of times: with about four workgroups per compute unit bf16 [2, 32 -> 64, 48^3] had 1458 workgroups on 1024 places (446 us,
+// now 1998: 411 us), fp16 [8, 256 -> 256, 100 x 152] 1152 on 512 (745 us, now 1440: 653 us).  Every workgroup costs a few tiles of
+// its own: the weight and the first offsets (as long as 1.5 tiles), and a block of the weight gradient, `block` fp32 atomics
+// at 64 bytes per request, 21 G a second, a tile taking 3.7 us.
+static long tap_ranges(long tiles, long others, long slots, long block) {
+  const double own = 1.5 + static_cast<double>(slots) * block / 16 / (21e9 * 3.7e-6);
+  long best = 0;
+  double least = 0.0;
+  const long first = (tiles + kTapRange / kTapTile - 1) / (kTapRange / kTapTile);
+  for (long per = std::min(tiles, kTapRange / kTapTile); per >= 1; per--) {
+    const long ranges = (tiles + per - 1) / per, rounds = (ranges * others + slots - 1) / slots;
+    const double cost = rounds * (per + own);
+    if (best == 0 || cost < least) { best = ranges; least = cost; }
+  }
+  return std::max(best, first);
+}
+
+// workgroups of an instance that the chip holds at a time (256 compute units; a property of the compiled kernel)
+template <typename T, int NC, int OBW, int CBW> static long tap_places() {
+  static const long places = [] {
+    int n = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void *>(&dcn_backward_tap_kernel<T, NC, OBW, CBW>), 256, 0) != hipSuccess)
+      (void)hipGetLastError();
+    return 256L * std::max(n, 1);
+  }();
+  return places;
+}
+
 template <typename T, int NC, int CBW>
 static int tap_launch(const T *xt, const T *off, const T *mask, const T *gyt, const T *wf, float *gxt, T *goff,
                       T *gmask, float *partial, float *gw, const DcnDims &s, const unsigned *bounds, const ScatterShape &shape, int dtype,
                       const TapPiece &piece, hipStream_t stream) {
   const int chunks = tap_chunks(s, dtype), shares = tap_shares(s, dtype);
-  // Positions of a workgroup: every one adds a block of the weight gradient to memory and fills LDS with a block of the
-  // weight, so as many as leave ~4 workgroups per compute unit.
+  const int rows = std::min(static_cast<int>(s.opg), s.opg <= 64 ? 64 : s.opg <= 128 || sizeof(T) == 4 ? 128 : 256);
   const long others = static_cast<long>(piece.taps) * s.dg * chunks * s.B, tiles = (piece.positions + static_cast<long>(kTapTile) - 1) / kTapTile;
-  const long want = std::max(1L, 1024 / others), per = std::min(std::max(1L, (tiles + want - 1) / want), kTapRange / kTapTile);
-  const long ranges = (tiles + per - 1) / per;
-  MV_REQUIRE(ranges * piece.taps < (1L << 31), "grid too large");
-  const dim3 grid(static_cast<unsigned>(ranges * piece.taps), static_cast<unsigned>(s.dg * chunks), s.B);
+  const long slots = s.opg <= 64 ? tap_places<T, NC, 1, CBW>() : s.opg <= 128 || sizeof(T) == 4 ? tap_places<T, NC, 2, CBW>()
+                                                                                                     : tap_places<T, NC, sizeof(T) == 2 ? 4 : 2, CBW>();
+  const long ranges = tap_ranges(tiles, others, slots, static_cast<long>(rows) * (16 * CBW)), per = (tiles + ranges - 1) / ranges;
+  MV_REQUIRE(static_cast<double>(ranges) * others < static_cast<double>(1L << 31), "grid too large");
+  const dim3 grid(static_cast<unsigned>(ranges * others));
   const int range = static_cast<int>(per * kTapTile);
 #define MV_TAP(OBWV, ROW)                                                                                               \
   hipLaunchKernelGGL((dcn_backward_tap_kernel<T, NC, OBWV, CBW>), grid, dim3(256), 0, stream, xt, off, mask, gyt, wf, gxt,     \
