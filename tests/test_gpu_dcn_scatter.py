@@ -23,8 +23,9 @@ def _gradient(oracle, dtype, batch, cin, cout, size, stride, groups, dg, offsets
     y = modulated_deform_conv(*leaves, stride, 1, 1, groups, dg)
     gy = torch.randn(y.shape, generator=g).to(dtype)
     y.backward(gy.to(DEV))
-    want = oracle.dcn3d_backward(x, off, mask, w, gy, True, stride, 1, 1, groups, dg)[0]
-    assert_close(leaves[0].grad, want, BWD_TOL[dtype], "input")
+    want = oracle.dcn3d_backward(x, off, mask, w, gy, True, stride, 1, 1, groups, dg)
+    assert_close(leaves[0].grad, want[0], BWD_TOL[dtype], "input")
+    assert_close(leaves[4].grad, want[4], BWD_TOL[dtype], "bias")   # (from 1024 rows of grad_output on several per workgroup)
 
 
 def _borders(off, g):
