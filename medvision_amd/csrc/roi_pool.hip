@@ -928,13 +928,13 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_forward_kernel(
 // gradient, already in the layout of the right-hand operand (column = channel, K = cell).  The
 // accumulator then holds, per lane, four neighbouring voxels of one box row for one channel: lanes
 // 0..15 are 16 neighbouring channels of the channels-last buffer, so an atomic instruction adds runs
-// of 64 contiguous bytes.  Wavefronts work on different channel blocks and share nothing but the
+// of 64 contiguous bytes.  Wavefronts work on different channel blocks or slices and share nothing but the
 // weights: no barrier after the set-up.
 constexpr int kPoolBwdRow = 72;   // fp16 elements per row of the transposed weights: 64 cells + pad
 template <typename T>
 __device__ inline void pool_backward_mfma(const T *__restrict__ src_any, float *__restrict__ dst_any, const RoiProblem &p,
                                           const PoolShared &sh, const float (&wd)[3][kDenseSrc][8],
-                                          unsigned char *lds, int c_count) {
+                                          unsigned char *lds, int c_count, int part, int parts) {
   using M = Mfma<T>;
   auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
   const int nx = uni(sh.ax[0].box_hi - sh.ax[0].box_lo + 1), ny = uni(sh.ax[1].box_hi - sh.ax[1].box_lo + 1),
@@ -987,8 +987,13 @@ __device__ inline void pool_backward_mfma(const T *__restrict__ src_any, float *
   // this roi's gradient rows of the block; reads beyond the block's channels return zeros
   const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<T *>(src), 0, c_count * cells * 2 + 16, 0x00020000);
-  const int blocks = (c_count + 15) / 16;
-  for (int blk = wave; blk < blocks; blk += kPoolThreads / kWave) {
+  // wavefronts side by side on channel blocks; where there are fewer blocks, several share a block's slices
+  constexpr int kWaves = kPoolThreads / kWave;
+  const int blocks = (c_count + 15) / 16, side = blocks == 1 ? 1 : blocks == 2 ? 2 : kWaves;
+  const int shares = parts * (kWaves / side), share = part * (kWaves / side) + wave / side;
+  const int z_first = nz * share / shares, z_last = nz * (share + 1) / shares;
+  if (z_first == z_last) return;
+  for (int blk = wave % side; blk < blocks; blk += side) {
     const int c = blk * 16 + col;
     const bool cv = c < c_count;
     // the lane's gradient pieces: cells quad * 8 .. + 7 (+ 32) of every pd of its channel
@@ -1017,7 +1022,7 @@ __device__ inline void pool_backward_mfma(const T *__restrict__ src_any, float *
     for (int pd = 0; pd < 8; pd++)
 #pragma unroll
       for (int ks = 0; ks < 2; ks++) g[pd][ks] &= keep[ks];
-    for (int z = 0; z < nz; z++) {
+    for (int z = z_first; z < z_last; z++) {
       float wz[8];
       {
         const float4 lo4 = *reinterpret_cast<const float4 *>(&wd[2][z][0]), hi4 = *reinterpret_cast<const float4 *>(&wd[2][z][4]);
@@ -1065,6 +1070,7 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
   __shared__ __attribute__((aligned(16))) unsigned char lds[kPoolLdsBytes];
   const unsigned n = blockIdx.x;
   const int c_begin = blockIdx.y * channels_per_block, c_end = min(c_begin + channels_per_block, p.C);
+  const int part = CL ? blockIdx.z : 0, parts = CL ? gridDim.z : 1;   // of the workgroups that share the box's slices
   // intermediates are fp32 here, so size the chunk with 4-byte box elements
   __shared__ __attribute__((aligned(16))) float wd[3][kDenseSrc][CELLS];
   PoolPlan plan = pool_setup<RT, CELLS>(sh, rois + static_cast<long>(n) * roi_columns(p.ndim, 0), p, sizeof(float), wd, true);
@@ -1087,13 +1093,13 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
   int zs = 0;
   if (plan.staged == 1 && !wide) {
     const long bx = sh.ax[0].box_hi - sh.ax[0].box_lo + 1, by = sh.ax[1].box_hi - sh.ax[1].box_lo + 1;
-    zs = sh.ax[2].box_hi - sh.ax[2].box_lo + 1;
+    zs = (sh.ax[2].box_hi - sh.ax[2].box_lo + parts) / parts;   // (the longest part)
     const bool box = !CL && dense;                         // planar sums from the dense matrices: the slab of the box itself is staged
     const long per_plane = (box ? by * bx * 4 : 0L) + (by * p.ow + static_cast<long>(p.oh) * p.ow) * 4;
     const int want = min(CL ? 16 : 4, c_end - c_begin);
     // (the set-up has counted a staged box: planar sums through the tap tables keep none, so that a plane of
     // an image that is larger than LDS still takes this path and not one atomic per tap of every sample)
-    if (!CL && !dense) plan.chunk = static_cast<int>(min(kPoolLdsBytes / (zs * per_plane + 16), 64L));
+    if ((!CL && !dense) || parts > 1) plan.chunk = static_cast<int>(min(kPoolLdsBytes / (zs * per_plane + 16), 64L));
     if (plan.chunk < want) {
       zs = static_cast<int>(min(max((kPoolLdsBytes / want - 16) / per_plane, 1L), static_cast<long>(zs)));
       plan.chunk = static_cast<int>(min(kPoolLdsBytes / (zs * per_plane + 16), 64L));
@@ -1103,7 +1109,7 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
   if (plan.staged == 0 || wide) {  // per-output scatter
     const int total = (c_end - c_begin) * cells;
     const int gz = p.ndim == 3 ? sh.g.grid[2] : 1, gy = sh.g.grid[1], gx = sh.g.grid[0];
-    for (int i = threadIdx.x; i < total; i += kPoolThreads) {
+    for (int i = part * kPoolThreads + threadIdx.x; i < total; i += parts * kPoolThreads) {
       const int pw = i % p.ow, ph = (i / p.ow) % p.oh, pd = (i / (p.ow * p.oh)) % p.od, c = i / cells;
       const float top = load(src + i) / static_cast<float>(sh.g.count);
       for (int iz = 0; iz < gz; iz++) {
@@ -1130,6 +1136,8 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
   const float inv_nxy = 1.f / (nx * ny), inv_nx = 1.f / nx, inv_ow = 1.f / p.ow,
               inv_ohw = 1.f / ohw, inv_nyow = 1.f / (ny * p.ow),
               inv_gx = 1.f / gx, inv_gy = 1.f / gy, inv_gz = 1.f / gz;
+  const int z_first = nz * part / parts, z_last = nz * (part + 1) / parts;
+  if (z_first == z_last) return;
   if (dense) {   // (the set-up has built the matrices)
     if constexpr (CL && CELLS == 8 && std::is_same<T, __half>::value && std::is_same<G, float>::value) {
       // matrix-core form: 32-bit offsets into the image's accumulation buffer and into this roi's
@@ -1142,15 +1150,15 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
       // than the tensor's last block)
       const long behind = (static_cast<long>(p.R) * p.C - (static_cast<long>(n) * p.C + c_end)) * cells * 2;
       if (fits && small && behind >= 16) {
-        pool_backward_mfma(src, dst_cl, p, sh, wd, lds, c_end - c_begin);
+        pool_backward_mfma(src, dst_cl, p, sh, wd, lds, c_end - c_begin, part, parts);
         return;
       }
     }
     const float inv_ow = 1.f / p.ow;
     for (int cb = c_begin; cb < c_end; cb += plan.chunk) {
       const int cs = min(plan.chunk, c_end - cb);
-      for (int z0 = 0; z0 < nz; z0 += zs) {   // slabs of box planes
-      const int nzs = min(zs, nz - z0);
+      for (int z0 = z_first; z0 < z_last; z0 += zs) {   // slabs of box planes
+      const int nzs = min(zs, z_last - z0);
       const int vol_s = nx * ny * nzs;
       const float inv_vol_s = 1.f / vol_s;
       float *t2 = reinterpret_cast<float *>(lds);      // [cs][nzs][oh][ow]
@@ -1233,8 +1241,8 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
   pool_first(sh);
   for (int cb = c_begin; cb < c_end; cb += plan.chunk) {
     const int cs = min(plan.chunk, c_end - cb);
-    for (int z0 = 0; z0 < nz; z0 += zs) {   // slabs of box planes
-    const int nzs = min(zs, nz - z0);
+    for (int z0 = z_first; z0 < z_last; z0 += zs) {   // slabs of box planes
+    const int nzs = min(zs, z_last - z0);
     const int vol_s = nx * ny * nzs;
     const float inv_vol_s = 1.f / vol_s, inv_nzsohw = 1.f / (nzs * ohw);
     float *t1 = reinterpret_cast<float *>(lds);       // [cs][nzs][ny][ow]
@@ -1532,10 +1540,21 @@ bool roi_pool_applies(int dtype, const RoiProblem &p) { return pool_applies(dtyp
 int roi_pool_backward(const void *grad_output, const void *rois, void *acc, int dtype,
                       const RoiProblem &p, hipStream_t s, bool channels_last) {
   if (!pool_applies(dtype, p)) return -1;
-  const int cpb = pool_channels_per_block(p);
+  // Channels-last sums of volumes: an atomic request takes as long for one channel as for sixteen, and the matrix
+  // instructions take sixteen in any case.  So a workgroup keeps at least that many, and where rois and channel blocks
+  // do not fill the chip, up to four workgroups share the slices of a box.  Kernel, fp16: 141 rois of 16 channels and 5^3
+  // cells 98 -> 20 us, 77 of 32 and 7^3 103 -> 26; fp32, 250 of 16 and 7^3 52 -> 27.  A part repeats the set-up of the
+  // box: none is added from 1024 workgroups on (1951 rois of 32 channels step in 121 us with one part and in 132 with
+  // two), and up to there the large boxes need them (807 rois of 32 channels, boxes of up to 21^3: 292 us with two,
+  // 325 with one).  32 channels per workgroup on the matrix cores, as of 1024 workgroups on: with 64, where no
+  // wavefronts share slices any more, 461 rois of 256 channels step in 611 us, not 515.
+  int cpb = pool_channels_per_block(p);
+  const bool share = channels_last && p.ndim == 3, mfma = dtype == MV_F16 && pool_small_cells(p);
+  if (share) cpb = std::max(cpb, std::min(p.C, mfma ? 32 : 16));
   const long cblocks = (p.C + cpb - 1) / cpb;
   if (cblocks > 65535) return -1;
-  const dim3 grid(p.R, static_cast<unsigned>(cblocks));
+  const long groups = p.R * cblocks, parts = share ? std::min((1023 + groups) / groups, 4L) : 1;
+  const dim3 grid(p.R, static_cast<unsigned>(cblocks), static_cast<unsigned>(parts));
   const float *r = static_cast<const float *>(rois);
   const bool small = pool_small_cells(p);
 #define MV_POOL_BACKWARD(TYPE, CLV)                                                          \

@@ -33,6 +33,32 @@ def test_fp32_plain(oracle, size, channels, rois, cells, ratio):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("size,channels,rois,cells,ratio,reach", [
+    ((5, 9, 11), 16, 4, (5, 5, 5), 2, 3),         # boxes of fewer slices than workgroups share them
+    ((1, 30, 34), 16, 6, (7, 7, 7), 1, 12),       # one slice
+    ((21, 13, 10), 17, 9, (7, 7, 7), 2, 18),      # a second block of one channel
+    ((14, 12, 9), 50, 30, (4, 3, 4), 0, 14),      # four blocks, a wavefront each
+    ((24, 30, 34), 40, 16, (6, 5, 7), 3, 40),     # boxes beyond the dense matrices
+    ((70, 12, 12), 20, 160, (2, 3, 2), 1, 90),    # boxes wider than the lists: sums per sample
+    ((16, 16, 18), 16, 400, (12, 9, 10), 1, 10),  # more than eight cells per axis, three workgroups per box
+    ((12, 12, 14), 16, 1023, (4, 4, 4), 2, 9),    # two workgroups per box
+    ((12, 12, 14), 16, 1024, (4, 4, 4), 2, 9),    # one
+])
+def test_plain_boxes_shared_by_workgroups(oracle, dtype, size, channels, rois, cells, ratio, reach):
+    from medvision_amd.ops.roi_align_nd import roi_align_3d
+    g = wl.gen(sum(size) + rois + channels)
+    at = torch.rand(rois, 3, generator=g) * torch.tensor(size[::-1]) * 1.2 - 2.0
+    boxes = torch.cat([torch.randint(0, 2, (rois, 1), generator=g).float(), at, at + torch.rand(rois, 3, generator=g) * reach], 1)
+    feat = torch.zeros(2, channels, *size, dtype=dtype)
+    x = feat.to(DEV).requires_grad_()
+    out = roi_align_3d(x, boxes.to(DEV), cells, 1.0, ratio, 1)
+    gy = torch.randn(out.shape, generator=g).to(dtype)
+    out.backward(gy.to(DEV))
+    want = oracle.roi_align_backward(gy, boxes, feat.shape, 1.0, ratio, True, 1, False)
+    assert_close(x.grad, want, BWD_TOL[dtype], "backward")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("size,channels,rois,cells,ratio,order,reach", [
     ((9, 11, 13), 8, 6, (4, 4, 4), 2, 1, 12),      # tiles with remainders, one group of channels
     ((8, 8, 12), 72, 20, (7, 7, 7), 0, 1, 9),      # rows of whole pieces, a second group with few channels
