@@ -395,13 +395,14 @@ __device__ inline void pool_forward_mfma(const T *__restrict__ src_any, T *__res
   // of a step are issued one step ahead, so they are in flight during the previous step's products
   // and stores.
   const int tiles = (c_count + 3) / 4;
+  const bool few = tiles <= kPoolThreads / kWave;   // a tile per wavefront
   struct Step { int tile, zg, k0; };
   struct Loaded { u32x2 va[2], vb[2]; };
   auto next_of = [&](Step st) {
     st.k0 += 32;
     if (st.k0 >= KP) {
       st.k0 = 0; st.zg += 2;
-      if (st.zg >= zgroups) { st.zg = 0; st.tile += st.tile % 2 == 0 ? 1 : 2 * (kPoolThreads / kWave) - 1; }
+      if (st.zg >= zgroups) { st.zg = 0; st.tile += few ? kPoolThreads / kWave : st.tile % 2 == 0 ? 1 : 2 * (kPoolThreads / kWave) - 1; }
     }
     return st;
   };
@@ -436,7 +437,7 @@ __device__ inline void pool_forward_mfma(const T *__restrict__ src_any, T *__res
   constexpr int kAhead = 3;
   Step q[kAhead];
   Loaded ld[kAhead];
-  q[0] = Step{2 * wave, 0, 0};   // tiles 2 w, 2 w + 1, then 2 (w + 4), ...: neighbours in memory back to back
+  q[0] = Step{few ? wave : 2 * wave, 0, 0};   // tiles 2 w, 2 w + 1, then 2 (w + 4), ...: neighbours in memory back to back
 #pragma unroll
   for (int u = 0; u < kAhead; u++) {
     if (u > 0) q[u] = next_of(q[u - 1]);
@@ -626,14 +627,32 @@ __device__ inline void pool_forward_mfma(const T *__restrict__ src_any, T *__res
   store_kept();
 }
 
+// Whether a roi's box most likely suits the matrix-core form (few rows times columns, not read sparsely): every
+// workgroup of the roi comes to the same answer, which settles the channels per workgroup and nothing else.
+template <typename RT>
+__device__ __forceinline__ bool pool_small_box(const RT *roi, const RoiProblem &p) {
+  const float scale = static_cast<float>(p.scale), grid = static_cast<float>(p.sampling_ratio);
+  const int nd = p.ndim;
+  auto extent = [&](int a, int size) { return fminf(fmaxf((roi[1 + nd + a] - roi[1 + a]) * scale, 1.f), static_cast<float>(size)); };
+  const float ex = extent(0, p.W), ey = extent(1, p.H), ez = nd == 3 ? extent(2, p.D) : 0.f;
+  if (!((ex + 5.f) * (ey + 2.f) <= kMfmaYx)) return false;
+  if (p.sampling_ratio <= 0) return true;
+  const float nx = grid * p.ow, ny = grid * p.oh, nz = nd == 3 ? grid * p.od : .5f;   // samples per axis
+  return (ex - ex / nx + 2.f) * (ey - ey / ny + 2.f) * (nd == 3 ? ez - ez / nz + 2.f : 1.f) <= 4.f * nx * ny * nz;
+}
+
 template <typename T, typename RT, int CELLS>
 __global__ __launch_bounds__(kPoolThreads) void roi_pool_forward_kernel(
     const T *__restrict__ feat, const RT *__restrict__ rois, T *__restrict__ out, const RoiProblem p,
-    const int channels_per_block, const T *__restrict__ blocked, const int Wb, const unsigned *__restrict__ order) {
+    const int channels_per_block, const int joined, const T *__restrict__ blocked, const int Wb,
+    const unsigned *__restrict__ order) {
   __shared__ PoolShared sh;
   __shared__ __attribute__((aligned(16))) unsigned char lds[kPoolLdsBytes];
   const unsigned n = order ? order[blockIdx.x] : blockIdx.x;   // (largest rois first, see pool_order_rois)
-  const int c_begin = blockIdx.y * channels_per_block, c_end = min(c_begin + channels_per_block, p.C);
+  int cpb = channels_per_block;   // small boxes: `joined` times as many
+  if (joined > 1 && pool_small_box(rois + static_cast<long>(n) * roi_columns(p.ndim, 0), p)) cpb *= joined;
+  if (static_cast<long>(blockIdx.y) * cpb >= p.C) return;   // (channels of a workgroup before)
+  const int c_begin = blockIdx.y * cpb, c_end = min(c_begin + cpb, p.C);
   __shared__ __attribute__((aligned(16))) float wd[3][kDenseSrc][CELLS];
   PoolPlan plan = pool_setup<RT, CELLS>(sh, rois + static_cast<long>(n) * roi_columns(p.ndim, 0), p, sizeof(T),
                                         CELLS == 8 ? wd : nullptr, true, true);
@@ -1414,7 +1433,8 @@ static bool pool_applies(int dtype, const RoiProblem &p) {
 // tables are built once per workgroup, so with many rois fewer, longer workgroups are cheaper) and
 // halved while there are too few workgroups to fill the compute units (few rois, few channels: a
 // workgroup walks its channels in LDS-sized chunks one after the other).
-// (`enough`: the number of workgroups that must remain when the channels per workgroup double)
+// (`enough`: the number of workgroups that must remain when the channels per workgroup double.  What few workgroups
+// lose to the set-up, the callers mend.)
 static int pool_channels_per_block(const RoiProblem &p, long enough = 6144) {
   int cpb = 32;
   while (cpb < 256 && cpb < p.C && static_cast<long>(p.R) * ((p.C + 2 * cpb - 1) / (2 * cpb)) >= enough) cpb *= 2;
@@ -1424,9 +1444,9 @@ static int pool_channels_per_block(const RoiProblem &p, long enough = 6144) {
 
 template <typename T, int CELLS>
 static void launch_pool_forward(const void *input, const float *r, void *output, const RoiProblem &p, int cpb,
-                                dim3 grid, hipStream_t s, const void *blocked = nullptr, const unsigned *order = nullptr) {
+                                dim3 grid, hipStream_t s, int joined = 1, const void *blocked = nullptr, const unsigned *order = nullptr) {
   hipLaunchKernelGGL((roi_pool_forward_kernel<T, float, CELLS>), grid, dim3(kPoolThreads), 0, s,
-                     static_cast<const T *>(input), r, static_cast<T *>(output), p, cpb,
+                     static_cast<const T *>(input), r, static_cast<T *>(output), p, cpb, joined,
                      static_cast<const T *>(blocked), p.W / 4, order);
 }
 
@@ -1511,7 +1531,17 @@ int roi_pool_forward(const void *input, const void *rois, void *output, int dtyp
   }
   // (from the blocked copy, in launch order, a workgroup's set-up weighs more than the balance of the
   // last wave of workgroups: 256 channels per workgroup from 3072 workgroups on, config 5 0.415 -> 0.39 ms)
-  const int cpb = pool_channels_per_block(p, blocked != nullptr && order != nullptr ? 3072 : 6144);
+  // A workgroup whose channels were halved for want of workgroups has idle wavefronts on the matrix cores (four channels
+  // each) and repeats the set-up and the weight products of its box.  There the boxes that suit the matrix cores take sixteen
+  // channels per workgroup and leave the others nothing to do; larger ones, of which a channel takes long, stay spread out
+  // over all of them, four channels each: 141 rois of 16 channels and 5^3 cells 29.5 -> 12 us, 369 of 32 and 7^3 35 -> 19 (27
+  // with eight each), 103 of 16 with boxes of up to 20^3 37 -> 24 (56 with sixteen).  The kernels without matrix cores, where
+  // all threads share a channel, gain from four (29 fp32 rois of 64 channels and 7^3 21 -> 11 us, 15 with eight).
+  int cpb = pool_channels_per_block(p, blocked != nullptr && order != nullptr ? 3072 : 6144), joined = 1;
+  if (pool_small_cells(p)) {
+    if (dtype == MV_F16) cpb = std::max(cpb, std::min(p.C, 4));
+    joined = std::max(std::min(p.C, dtype == MV_F16 ? 16 : 4) / cpb, 1);
+  }
   const long cblocks = (p.C + cpb - 1) / cpb;
   if (cblocks > 65535) return -1;
   const dim3 grid(p.R, static_cast<unsigned>(cblocks));
@@ -1519,15 +1549,15 @@ int roi_pool_forward(const void *input, const void *rois, void *output, int dtyp
   const bool small = pool_small_cells(p);
   switch (dtype) {
     case MV_F32:
-      small ? launch_pool_forward<float, 8>(input, r, output, p, cpb, grid, s)
+      small ? launch_pool_forward<float, 8>(input, r, output, p, cpb, grid, s, joined)
             : launch_pool_forward<float, 16>(input, r, output, p, cpb, grid, s);
       break;
     case MV_F16:
-      small ? launch_pool_forward<__half, 8>(input, r, output, p, cpb, grid, s, blocked, order)
+      small ? launch_pool_forward<__half, 8>(input, r, output, p, cpb, grid, s, joined, blocked, order)
             : launch_pool_forward<__half, 16>(input, r, output, p, cpb, grid, s);
       break;
     default:
-      small ? launch_pool_forward<__hip_bfloat16, 8>(input, r, output, p, cpb, grid, s)
+      small ? launch_pool_forward<__hip_bfloat16, 8>(input, r, output, p, cpb, grid, s, joined)
             : launch_pool_forward<__hip_bfloat16, 16>(input, r, output, p, cpb, grid, s);
   }
   return check_launch("roi_pool_forward_kernel");
@@ -1546,11 +1576,12 @@ int roi_pool_backward(const void *grad_output, const void *rois, void *acc, int 
   // cells 98 -> 20 us, 77 of 32 and 7^3 103 -> 26; fp32, 250 of 16 and 7^3 52 -> 27.  A part repeats the set-up of the
   // box: none is added from 1024 workgroups on (1951 rois of 32 channels step in 121 us with one part and in 132 with
   // two), and up to there the large boxes need them (807 rois of 32 channels, boxes of up to 21^3: 292 us with two,
-  // 325 with one).  32 channels per workgroup on the matrix cores, as of 1024 workgroups on: with 64, where no
-  // wavefronts share slices any more, 461 rois of 256 channels step in 611 us, not 515.
+  // 325 with one).  On the matrix cores 32 channels per workgroup where four parts of them fill the chip (with 64, where no
+  // wavefronts share slices any more, 461 rois of 256 channels step in 611 us, not 515; below that, 77 rois of 32
+  // channels: 37 us, with 16 per workgroup 26).
   int cpb = pool_channels_per_block(p);
   const bool share = channels_last && p.ndim == 3, mfma = dtype == MV_F16 && pool_small_cells(p);
-  if (share) cpb = std::max(cpb, std::min(p.C, mfma ? 32 : 16));
+  if (share) cpb = std::max(cpb, std::min(p.C, mfma && p.R * ((p.C + 31L) / 32) >= 256 ? 32 : 16));
   const long cblocks = (p.C + cpb - 1) / cpb;
   if (cblocks > 65535) return -1;
   const long groups = p.R * cblocks, parts = share ? std::min((1023 + groups) / groups, 4L) : 1;
