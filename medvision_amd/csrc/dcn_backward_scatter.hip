@@ -363,7 +363,10 @@ __global__ __launch_bounds__(KEEP <= 4 ? 1024 : 512) void dcn_backward_scatter_k
 // one (offsets of sigma = 2: 8.4 -> 5.7 %; that kernel 504 -> 462 us); 12 x 14 x 15 and 11 x 15 x 15 were no faster, layers of small offsets
 // do not change.
 using TileVolume = Tile<12, 14, 14>;
-using TileStrided = Tile<12, 12, 13>;   // 4 x 4 x 4 positions: stride 2, dilation
+using TileStrided = Tile<12, 12, 13>;   // 4 x 4 x 4 positions: dilation, 64-bit sums
+using TileDeep = Tile<9, 10, 14>;       // 4 x 4 x 8 positions, 64-bit sums of 16-bit tensors
+using TileDeepStrided = Tile<8, 12, 13>;   // 2 x 4 x 4 positions, the same at stride 2
+template <typename S> constexpr bool kDeep = std::is_same<S, TileDeep>::value || std::is_same<S, TileDeepStrided>::value;
 using TileImage = Tile<1, 44, 44>;      // 32 x 32 positions, 32-bit sums
 using TileWide = Tile<1, 28, 44>;       // 16 x 32 positions (8 x 16 at stride 2), 64-bit sums
 using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions
@@ -372,8 +375,14 @@ using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions
 // on either side, or one, if none has two.  Images with fewer workgroups than compute units take a smaller brick (77 us ->
 // 35 us for [1, 256 -> 128, 27 x 58]); volumes do not (the halo of 4 x 4 x 4 positions is most of their tile: 117 us
 // against 78 us for [2, 16 -> 128, 7 x 19 x 32]).  Images with 64-bit sums have smaller tiles of 16 channels instead of 44 x 44 of 8:
-// half the samples to work out, and 5.5 million requests of 64 bytes instead of 9.9 of 32 for [8, 256 -> 256, 100 x 152].  False:
-// no brick fits.
+// half the samples to work out, and 5.5 million requests of 64 bytes instead of 9.9 of 32 for [8, 256 -> 256, 100 x 152].  Where no
+// brick of images gives a workgroup to every compute unit, the one of most workgroups (fp32 [2, 128 -> 256, 36 x 18]: 48 of
+// 16 x 32 positions 131 us, 240 of 8 x 8 31 us).  Volumes of 16-bit tensors with 64-bit sums have
+// smaller tiles of 16 channels too, where they leave three voxels to spare: bf16 [4, 32 -> 128, 57 x 51 x 27] at stride 2 472 us
+// with 12 x 12 x 13 of 8, 407 us with 8 x 12 x 13 of 16 (the tap kernel, which adds the corners beyond the smaller bricks' tiles,
+// 236 -> 275 us).  fp32 ones would gain more ([4, 16 -> 16, 17 x 43 x 30] 343 us, 244 us with 9 x 10 x 14 of 16), but every
+// addition to memory rounds: their gradient would be 1.5e-7 (rms) off instead of 1.3e-7.  With 32-bit sums, where 16 channels fit
+// the larger tile, smaller ones only cost more halo (30 layers of fewer than 256 workgroups: 2 % slower).  False: no brick fits.
 //
 // Width of the sums: 32 bits round every term to 14 - 22 bits of the workgroup's largest, which is worth their speed in dense
 // layers alone (16-bit tensors, the first brick fits: unit strides, taps close together; up to 128 output channels).  bf16 training
@@ -381,6 +390,7 @@ using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions
 // where the output's gradient is 2^-14 of what it is elsewhere in the brick, 32 bits left them 2 - 20 % off. 
 bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
   static const int volumes[2][6] = {{2, 3, 3, 12, 14, 14}, {2, 2, 2, 12, 12, 13}};
+  static const int deep[2][6] = {{2, 2, 3, 9, 10, 14}, {1, 2, 2, 8, 12, 13}};
   static const int dense_images[3][6] = {{0, 5, 5, 1, 44, 44}, {0, 4, 4, 1, 28, 28}, {0, 3, 3, 1, 28, 28}};
   static const int images[4][6] = {{0, 4, 5, 1, 28, 44}, {0, 4, 4, 1, 28, 28}, {0, 3, 4, 1, 28, 44}, {0, 3, 3, 1, 28, 28}};
   const bool image = s.nd == 2;
@@ -399,13 +409,15 @@ bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
   };
   const auto choose = [&](const int (*list)[6], int count, int channels) {
     int best = -1;
+    const int *taken = nullptr;
     for (int i = 0; i < count; i++) {
       const int *e = list[i];
       const long spare = spare_of(e);
       if (spare < 2) continue;
       const int rank = (spare >= 4 ? 2 : 0) + (image && workgroups(e, channels) >= 256 ? 1 : 0);
-      if (rank <= best) continue;
+      if (rank < best || (rank == best && !(image && workgroups(taken, channels) < 256))) continue;
       best = rank;
+      taken = e;
       shape = ScatterShape{e[0], e[1], e[2], e[3], e[4], e[5], 0, 0, 0, (1 << (e[0] + e[1] + e[2])) * s.K, 0, 1};
     }
     return best >= 0;
@@ -417,7 +429,10 @@ bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
     fits = image ? choose(dense_images, 3, 16) : choose(volumes, 2, 16);
     shape.narrow = fits && scatter32_shift(shape.terms) >= kScatterMinShift;
   }
-  if (!shape.narrow) fits = image ? choose(images, 4, 16) : choose(volumes, 2, 8);
+  if (!shape.narrow) {
+    const int (*const small)[6] = image || dtype == MV_F32 ? nullptr : spare_of(deep[0]) >= 3 ? deep : spare_of(deep[1]) >= 3 ? deep + 1 : nullptr;
+    fits = image ? choose(images, 4, 16) : small ? choose(small, 1, 16) : choose(volumes, 2, 8);
+  }
   if (!fits) return false;
   shape.nbd = (s.Do + (1 << shape.bd) - 1) >> shape.bd;
   shape.nbh = (s.Ho + (1 << shape.bh) - 1) >> shape.bh;
@@ -439,10 +454,10 @@ static int scatter_launch(const void *off, const void *mask, const void *gyt, co
                      static_cast<const T *>(off), static_cast<const T *>(mask), static_cast<const T *>(gyt),          \
                      static_cast<const T *>(wf), gxt, s, shape, bounds)
   if (shape.narrow) {
-    if constexpr (sizeof(T) == 2 && !std::is_same<S, TileWide>::value) {   // (never wide)
+    if constexpr (sizeof(T) == 2 && !kDeep<S> && !S::WIDE) {   // (those have 64-bit sums)
       if (slices <= 2) MV_SCATTER(true, 2); else MV_SCATTER(true, 4);
     }
-  } else if constexpr (!std::is_same<S, TileImage>::value) {
+  } else if constexpr (!std::is_same<S, TileImage>::value && !(kDeep<S> && sizeof(T) == 4)) {   // (never of these)
     if (slices <= 2) MV_SCATTER(false, 2);
     else if (slices <= 4) MV_SCATTER(false, 4);
     else MV_SCATTER(false, 8);
@@ -455,7 +470,9 @@ int dcn_scatter(const void *off, const void *mask, const void *gyt, const void *
                 const ScatterShape &shape, const unsigned *bounds, int dtype, hipStream_t stream) {
 #define MV_SCATTER_TILE(T, S) scatter_launch<T, S>(off, mask, gyt, wf, gxt, s, shape, bounds, stream)
 #define MV_SCATTER_AS(T)                                                                                              \
-  (shape.th == TileVolume::TH ? MV_SCATTER_TILE(T, TileVolume)                                                          \
+  (shape.td == TileDeep::TD ? MV_SCATTER_TILE(T, TileDeep)                                                             \
+   : shape.td == TileDeepStrided::TD ? MV_SCATTER_TILE(T, TileDeepStrided)                                              \
+   : shape.th == TileVolume::TH ? MV_SCATTER_TILE(T, TileVolume)                                                          \
    : shape.th == TileStrided::TH ? MV_SCATTER_TILE(T, TileStrided)                                                      \
    : shape.th == TileImage::TH ? MV_SCATTER_TILE(T, TileImage)                                                        \
    : shape.tw == TileWide::TW ? MV_SCATTER_TILE(T, TileWide) : MV_SCATTER_TILE(T, TileSmall))

@@ -40,6 +40,8 @@ def _borders(off, g):
     (32, 32, (5, 9, 17), 1, 1, 1),        # volumes: a brick and a remainder along every axis
     (64, 96, (4, 8, 9), 1, 1, 2),         # three slices of grad_output, two deformable groups
     (32, 160, (6, 9, 10), 2, 1, 1),       # strided, more slices than four
+    (48, 16, (9, 5, 25), 1, 1, 1),        # bricks of 4 x 4 x 8 and a remainder along every axis
+    (16, 64, (9, 13, 17), 2, 1, 1),       # of 2 x 4 x 4, strided
     (32, 64, (33, 35), 1, 1, 1),          # images: a brick of 32 x 32 (16 x 32) and a remainder
     (64, 288, (17, 33), 1, 1, 1),         # more slices than eight
     (64, 64, (31, 67), 2, 2, 2),          # strided, groups
