@@ -13,11 +13,11 @@
 // Afterwards the tile's non-zero sums are added to the gradient buffer, one global atomic per (voxel, channel) of the tile
 // instead of one per (position, tap, corner, channel).
 //
-// NARROW (dense layers of 16-bit tensors, see dcn_scatter_plan): 32-bit sums.  They leave 30 - ceil(log2(positions * taps)) bits for
-// a term (17 for 3 x 3 x 3 taps), so the scale comes from the data: a first sweep over the brick's taps forms gcol alone (matrix
+// NARROW (dense layers of 16-bit tensors, see dcn_scatter_plan): 32-bit sums.  They leave 31 - log2(positions * taps) bits for
+// a term (18 for 3 x 3 x 3 taps), so the scale comes from the data: a first sweep over the brick's taps forms gcol alone (matrix
 // cores, no geometry; 17 us of the 338) and takes max |gcol| of the workgroup; every term is then below max |gcol| * max |mask| <
 // 2^ex and is rounded to a multiple of 2^(ex - shift).  The error of a voxel's sum stays below terms * 2^(ex - shift - 1), about
-// 2^-15 of the values it sums for the 3 x 3 x 3 layer — a sixteenth of the last bit of the 16-bit result.  Otherwise a 64-bit word
+// 2^-16 of the values it sums for the 3 x 3 x 3 layer — a thirty-second of the last bit of a bf16 result.  Otherwise a 64-bit word
 // per channel, scale from the global maxima.
 //
 // What bounds it: the LDS additions (64 lanes of 32 bits in 4 clocks, of 64 bits in 6, whatever the cells) behind phases that leave
@@ -35,11 +35,12 @@ template <int D, int H, int W> struct Tile {
   static constexpr bool WIDE = D == 1 && W > H;
   template <bool NARROW> static constexpr int channels = VOX * 16 * (NARROW ? 4 : 8) <= 160 * 1024 ? 16 : 8;
 };
-constexpr int kScatterMinShift = 14;  // fewer bits per term: 64-bit words
+constexpr int kScatter32Terms = 1 << 16;  // more (fewer than 14 bits each): 64-bit words
+// the largest shift <= 22 with terms * 2^shift < 2^31
 __host__ __device__ constexpr int scatter32_shift(int terms) {
-  int bits = 0;
-  while ((1L << bits) < terms) bits++;
-  return bits < 8 ? 22 : 30 - bits;
+  int shift = 22;
+  while (shift > 0 && (static_cast<long>(terms) << shift) > 0x7fffffffL) shift--;
+  return shift;
 }
 
 template <int... I, typename F> __device__ __forceinline__ void unrolled(std::integer_sequence<int, I...>, F f) {
@@ -427,7 +428,7 @@ bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
   bool fits = false;
   if (dtype != MV_F32 && s.opg <= 128 && spare_of(image ? dense_images[0] : volumes[0]) >= 2) {
     fits = image ? choose(dense_images, 3, 16) : choose(volumes, 2, 16);
-    shape.narrow = fits && scatter32_shift(shape.terms) >= kScatterMinShift;
+    shape.narrow = fits && shape.terms <= kScatter32Terms;
   }
   if (!shape.narrow) {
     const int (*const small)[6] = image || dtype == MV_F32 ? nullptr : spare_of(deep[0]) >= 3 ? deep : spare_of(deep[1]) >= 3 ? deep + 1 : nullptr;
