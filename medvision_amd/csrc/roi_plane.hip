@@ -262,8 +262,9 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void roi_plane_forward_kernel(con
     }
     return;
   }
-  const int m = lane % 16, q = lane / 16, mc = m < CELLS ? m : CELLS - 1;
-  const bool cell_lane = CELLS == 16 || m < CELLS;
+  constexpr int PAIR = 16 / CELLS, SUMS = kPlaneAtOnce / PAIR;   // channels side by side in the columns of the products
+  const int m = lane % 16, q = lane / 16, mc = m % CELLS, mine = m / CELLS;   // the lane's cell and its channel of the pair
+  const bool cell_lane = m < CELLS;
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int y_pieces = (rows + 15) / 16, x_pieces = (groups + 3) / 4;
   const int plane_bytes = static_cast<int>(plane) * ES;   // < 2^27, checked by the host
@@ -289,23 +290,30 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void roi_plane_forward_kernel(con
 #pragma unroll
     for (int c = 0; c < kPlaneAtOnce; c++) v[c] = plane_load_cells<T, 4>(rsrc, off, c * plane_bytes);
   };
-  f32x4_t sum[kPlaneAtOnce], t[kPlaneAtOnce];
+  f32x4_t sum[SUMS], t[SUMS];
   static_assert(kPlaneChannels <= 32 * kPlaneWaves * kPlaneAtOnce, "a bit for each of the wavefront's groups of channels");
   unsigned special = 0;   // the groups whose sums are not finite
   unsigned out_off[4];   // the lane's four outputs of a channel
 #pragma unroll
   for (int r = 0; r < 4; r++)
-    out_off[r] = m < p.ow && 4 * q + r < p.oh ? static_cast<unsigned>(((4 * q + r) * p.ow + m) * ES) : kPlaneNowhere;
+    out_off[r] = mc < p.ow && 4 * q + r < p.oh ? static_cast<unsigned>((mine * cells + (4 * q + r) * p.ow + mc) * ES) : kPlaneNowhere;
   auto columns = [&](const PlaneCells<T, 4> (&v)[kPlaneAtOnce], const Step &st, auto first) {
     const int g = st.xp * 4 + q;
-    float bx[4];
+    float bx[PAIR][4];   // of two channels, the weights meet the first one in columns 0 - 7 and the second one in columns 8 - 15
 #pragma unroll
-    for (int u = 0; u < 4; u++) bx[u] = cell_lane && g < groups ? wx[4 * g + u][mc] : 0.f;
+    for (int u = 0; u < 4; u++) {
+      const float w = g < groups ? wx[4 * g + u][mc] : 0.f;
+#pragma unroll
+      for (int i = 0; i < PAIR; i++) bx[i][u] = mine == i ? w : 0.f;
+    }
 #pragma unroll
     for (int u = 0; u < 4; u++)
 #pragma unroll
-      for (int c = 0; c < kPlaneAtOnce; c++)
-        t[c] = plane_product(load(&v[c].v[u]), bx[u], decltype(first)::value && u == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : t[c]);
+      for (int i = 0; i < PAIR; i++)
+#pragma unroll
+        for (int c = 0; c < SUMS; c++)
+          t[c] = plane_product(load(&v[c * PAIR + i].v[u]), bx[i][u],
+                               decltype(first)::value && u == 0 && i == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : t[c]);
   };
   auto row_sums = [&](const Step &st, auto first) {
     // register r of lane group q: listed row 16 yp + 4 q + r
@@ -318,7 +326,7 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void roi_plane_forward_kernel(con
 #pragma unroll
     for (int r = 0; r < 4; r++)
 #pragma unroll
-      for (int c = 0; c < kPlaneAtOnce; c++)
+      for (int c = 0; c < SUMS; c++)
         sum[c] = plane_product(ay[r], t[c][r], decltype(first)::value && r == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : sum[c]);
   };
   auto products = [&](const PlaneCells<T, 4> (&v)[kPlaneAtOnce], const Step &st) {
@@ -330,7 +338,7 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void roi_plane_forward_kernel(con
     if (st.yp + 1 < y_pieces) return;
     float check = 0.f;   // stays zero unless a sum is infinite or NaN
 #pragma unroll
-    for (int c = 0; c < kPlaneAtOnce; c++)
+    for (int c = 0; c < SUMS; c++)
 #pragma unroll
       for (int r = 0; r < 4; r++) check = fmaf(sum[c][r], 0.f, check);
     if (__ballot(!(check == 0.f)) != 0) {
@@ -341,9 +349,9 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void roi_plane_forward_kernel(con
         dst + static_cast<long>(st.c0) * cells, 0,
         __builtin_amdgcn_readfirstlane(min(kPlaneAtOnce, c_count - st.c0) * cells * ES), 0x00020000);
 #pragma unroll
-    for (int c = 0; c < kPlaneAtOnce; c++)   // (channels beyond the last one are beyond the buffer)
+    for (int c = 0; c < SUMS; c++)   // (channels beyond the last one are beyond the buffer)
 #pragma unroll
-      for (int r = 0; r < 4; r++) plane_store<T>(to, out_off[r], c * cells * ES, sum[c][r]);
+      for (int r = 0; r < 4; r++) plane_store<T>(to, out_off[r], c * PAIR * cells * ES, sum[c][r]);
   };
   // kPlaneSteps sets of load registers used in turn: the loads of the next kPlaneSteps - 1 steps are in flight
   Step step[kPlaneSteps];
