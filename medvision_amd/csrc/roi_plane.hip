@@ -5,7 +5,7 @@
 // wx[cell column], each the sum over the cell's samples on that axis, so that with G = the 7 x 7 cells of a channel
 //     forward  G = Wy box Wx^T,        backward  box += Wy^T G Wx
 // are two small matrix products per channel each.  They run on the fp32 matrix cores (16 x 16 x 4, exact fp32
-// products and sums).  A dense product gives 0 x infinity for a pixel or gradient that no sample's weight reaches, so
+// products and sums), the forward pass's first one on the 16-bit ones where the pixels are 16-bit (PlaneHalf).  A dense product gives 0 x infinity for a pixel or gradient that no sample's weight reaches, so
 // sums that come out not finite are formed again without the terms of weight 0 (one test per finished sum; the second
 // pass runs for such channels and tiles alone).  The accumulator of the first product is the right-hand operand of the second as it stands:
 // lane l holds column l % 16 and the four rows 4 (l / 16) + r, and a product's step r takes K = one row per lane
@@ -16,15 +16,16 @@
 // one, columns in groups of four), so that large rois with a small sampling grid read only what they use.  A lane's
 // piece of a 16 x 16 piece of the box is one 16-byte load (16-bit tensors: 8 bytes), straight from the feature map.
 //   (1000 rois of 4 - 64 pixels, adaptive grid, 256 channels, 7 x 7 cells, fp32, [2, 256, 200, 304]: 480 us when the
-//   boxes went through LDS and three barriers per chunk of channels; 165 us now: matrix cores 47 % and texture addressers 58 %
-//   busy.)
+//   boxes went through LDS and three barriers per chunk of channels; 157 us now (168 us with a channel per product, matrix cores 47 %
+//   and texture addressers 58 % busy).  fp16, 1613 rois of 3 - 25 pixels x 256 channels: 147 us with a channel per fp32 product, 122 us with
+//   two, 108 us with the first product on the 16-bit cores.)
 //
 // Backward, one workgroup = (16 x 16 pixels, some channels): it looks up the rois that touch its pixels, works out
 // its pixels' weights for eight rois at a time and adds roi after roi into accumulators that stay in registers.  No
 // atomics, no fp32 copy of the gradient, every pixel written once, sums in the order of the rois.
 //   (The same head: 1030 us with one atomic per touched pixel, roi and channel; 145 us now: matrix cores 50 %, vector issue 32 %.)
-// What bounds them: the matrix cores (three 32-clock instructions per roi, tile and channel backward; 4 (x pieces + 1)
-// per row piece and channel forward) and the latency of the loads.
+// What bounds them: the matrix cores (three 32-clock instructions per roi, tile and channel backward; 4 x pieces + 2
+// per row piece and channel forward, 4 with 16 cells) and the latency of the loads.
 #include <algorithm>
 
 #include "common.hpp"
@@ -41,6 +42,31 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ f32x4_t plane_product(float a, float b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
+
+// Four pixels of a 16-bit tensor, as they are stored, times four weights (K of a 16 x 16 x 16 product): the weights as
+// the sum of three 16-bit parts, of which two share a product of twice the K.  Every product is exact in fp32, and the
+// parts hold the weight's 24 bits (bf16) or leave less than 2^-28 (fp16, whose weights, at most 1, are kept times 2^14).
+template <typename T> struct PlaneHalf;
+template <> struct PlaneHalf<__half> {
+  using E = _Float16;
+  static constexpr float kScale = 16384.f;
+  typedef _Float16 v4 __attribute__((ext_vector_type(4)));
+  typedef _Float16 v8 __attribute__((ext_vector_type(8)));
+  static __device__ __forceinline__ f32x4_t two(v8 a, v8 b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+  static __device__ __forceinline__ f32x4_t one(v4 a, v4 b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0); }
+};
+template <> struct PlaneHalf<__hip_bfloat16> {
+  using E = __bf16;
+  static constexpr float kScale = 1.f;
+  typedef __bf16 v4 __attribute__((ext_vector_type(4)));
+  typedef __bf16 v8 __attribute__((ext_vector_type(8)));
+  typedef short s4 __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ f32x4_t two(v8 a, v8 b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+  static __device__ __forceinline__ f32x4_t one(v4 a, v4 b, f32x4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s4, a), __builtin_bit_cast(s4, b), c, 0, 0, 0);
+  }
+};
+template <> struct PlaneHalf<float> { static constexpr float kScale = 1.f; };
 
 // One axis of a plain roi: v(cell, sub) = start + cell * bin + (sub + .5) * step (local_coord's expression)
 struct PlaneAxis {
@@ -299,21 +325,54 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void roi_plane_forward_kernel(con
     out_off[r] = mc < p.ow && 4 * q + r < p.oh ? static_cast<unsigned>((mine * cells + (4 * q + r) * p.ow + mc) * ES) : kPlaneNowhere;
   auto columns = [&](const PlaneCells<T, 4> (&v)[kPlaneAtOnce], const Step &st, auto first) {
     const int g = st.xp * 4 + q;
-    float bx[PAIR][4];   // of two channels, the weights meet the first one in columns 0 - 7 and the second one in columns 8 - 15
+    // (of two channels, the weights meet the first one in columns 0 - 7 and the second one in columns 8 - 15)
+    if constexpr (ES == 2) {
+      using H = PlaneHalf<T>;
+      typename H::v8 high[PAIR];   // first and second parts
+      typename H::v4 low[PAIR];    // third parts
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const float w = g < groups ? wx[4 * g + u][mc] : 0.f;
+      for (int u = 0; u < 4; u++) {
+        const float w = g < groups ? wx[4 * g + u][mc] * H::kScale : 0.f;
+        const typename H::E first_part = static_cast<typename H::E>(w);
+        const float left = w - static_cast<float>(first_part);
+        const typename H::E second_part = static_cast<typename H::E>(left);
+        const typename H::E third_part = static_cast<typename H::E>(left - static_cast<float>(second_part));
 #pragma unroll
-      for (int i = 0; i < PAIR; i++) bx[i][u] = mine == i ? w : 0.f;
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++)
+        for (int i = 0; i < PAIR; i++) {
+          high[i][u] = mine == i ? first_part : static_cast<typename H::E>(0.f);
+          high[i][4 + u] = mine == i ? second_part : static_cast<typename H::E>(0.f);
+          low[i][u] = mine == i ? third_part : static_cast<typename H::E>(0.f);
+        }
+      }
 #pragma unroll
       for (int i = 0; i < PAIR; i++)
 #pragma unroll
-        for (int c = 0; c < SUMS; c++)
-          t[c] = plane_product(load(&v[c * PAIR + i].v[u]), bx[i][u],
-                               decltype(first)::value && u == 0 && i == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : t[c]);
+        for (int c = 0; c < SUMS; c++) {
+          const typename H::v4 a = __builtin_bit_cast(typename H::v4, v[c * PAIR + i]);
+          t[c] = H::two(__builtin_shufflevector(a, a, 0, 1, 2, 3, 0, 1, 2, 3), high[i],
+                        decltype(first)::value && i == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : t[c]);
+        }
+#pragma unroll
+      for (int i = 0; i < PAIR; i++)
+#pragma unroll
+        for (int c = 0; c < SUMS; c++) t[c] = H::one(__builtin_bit_cast(typename H::v4, v[c * PAIR + i]), low[i], t[c]);
+    } else {
+      float bx[PAIR][4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const float w = g < groups ? wx[4 * g + u][mc] : 0.f;
+#pragma unroll
+        for (int i = 0; i < PAIR; i++) bx[i][u] = mine == i ? w : 0.f;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int i = 0; i < PAIR; i++)
+#pragma unroll
+          for (int c = 0; c < SUMS; c++)
+            t[c] = plane_product(load(&v[c * PAIR + i].v[u]), bx[i][u],
+                                 decltype(first)::value && u == 0 && i == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : t[c]);
+    }
   };
   auto row_sums = [&](const Step &st, auto first) {
     // register r of lane group q: listed row 16 yp + 4 q + r
@@ -321,7 +380,7 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void roi_plane_forward_kernel(con
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       const int k = st.yp * 16 + 4 * q + r;
-      ay[r] = cell_lane && k < rows ? wy[k][mc] : 0.f;
+      ay[r] = cell_lane && k < rows ? wy[k][mc] * (1.f / PlaneHalf<T>::kScale) : 0.f;
     }
 #pragma unroll
     for (int r = 0; r < 4; r++)
