@@ -38,33 +38,31 @@ constexpr int kPlaneThreads = 256, kPlaneWaves = kPlaneThreads / kWave;
 constexpr int kPlaneTile = 16;       // pixels per side of a matrix piece
 constexpr unsigned kPlaneNowhere = 0x80000000u;   // beyond every buffer: the load returns zeros
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef unsigned plane_u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f32x4_t plane_product(float a, float b, f32x4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// Four pixels of a 16-bit tensor, as they are stored, times four weights (K of a 16 x 16 x 16 product): the weights as
-// the sum of three 16-bit parts, of which two share a product of twice the K.  Every product is exact in fp32, and the
-// parts hold the weight's 24 bits (bf16) or leave less than 2^-28 (fp16, whose weights, at most 1, are kept times 2^14).
+// Values of a 16-bit tensor, as they are stored, times fp32 weights, on the 16-bit matrix cores: a weight is the sum of
+// three 16-bit parts, which stand next to each other in K against the same values.  Every product is exact in fp32, and
+// the parts hold the weight's 24 bits (bf16) or leave less than 2^-28 (fp16, whose weights, at most 1, are kept times 2^14).
+// All products of a sum are 16 x 16 x 32 ones: where a 16 x 16 x 16 one took the result of a 16 x 16 x 32 one as its third
+// operand, the compiler left no wait between them, and it read the old registers.
 template <typename T> struct PlaneHalf;
 template <> struct PlaneHalf<__half> {
   using E = _Float16;
   static constexpr float kScale = 16384.f;
   typedef _Float16 v4 __attribute__((ext_vector_type(4)));
   typedef _Float16 v8 __attribute__((ext_vector_type(8)));
-  static __device__ __forceinline__ f32x4_t two(v8 a, v8 b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
-  static __device__ __forceinline__ f32x4_t one(v4 a, v4 b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0); }
+  static __device__ __forceinline__ f32x4_t product(v8 a, v8 b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 };
 template <> struct PlaneHalf<__hip_bfloat16> {
   using E = __bf16;
   static constexpr float kScale = 1.f;
   typedef __bf16 v4 __attribute__((ext_vector_type(4)));
   typedef __bf16 v8 __attribute__((ext_vector_type(8)));
-  typedef short s4 __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ f32x4_t two(v8 a, v8 b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
-  static __device__ __forceinline__ f32x4_t one(v4 a, v4 b, f32x4_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s4, a), __builtin_bit_cast(s4, b), c, 0, 0, 0);
-  }
+  static __device__ __forceinline__ f32x4_t product(v8 a, v8 b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 };
 template <> struct PlaneHalf<float> { static constexpr float kScale = 1.f; };
 
@@ -328,8 +326,7 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void roi_plane_forward_kernel(con
     // (of two channels, the weights meet the first one in columns 0 - 7 and the second one in columns 8 - 15)
     if constexpr (ES == 2) {
       using H = PlaneHalf<T>;
-      typename H::v8 high[PAIR];   // first and second parts
-      typename H::v4 low[PAIR];    // third parts
+      typename H::v8 part[2][PAIR];   // first and second parts; third parts
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         const float w = g < groups ? wx[4 * g + u][mc] * H::kScale : 0.f;
@@ -339,23 +336,23 @@ __global__ __launch_bounds__(kPlaneThreads, 4) void roi_plane_forward_kernel(con
         const typename H::E third_part = static_cast<typename H::E>(left - static_cast<float>(second_part));
 #pragma unroll
         for (int i = 0; i < PAIR; i++) {
-          high[i][u] = mine == i ? first_part : static_cast<typename H::E>(0.f);
-          high[i][4 + u] = mine == i ? second_part : static_cast<typename H::E>(0.f);
-          low[i][u] = mine == i ? third_part : static_cast<typename H::E>(0.f);
+          const typename H::E none = static_cast<typename H::E>(0.f);
+          part[0][i][u] = mine == i ? first_part : none;
+          part[0][i][4 + u] = mine == i ? second_part : none;
+          part[1][i][u] = mine == i ? third_part : none;
+          part[1][i][4 + u] = none;
         }
       }
 #pragma unroll
-      for (int i = 0; i < PAIR; i++)
+      for (int k = 0; k < 2; k++)
 #pragma unroll
-        for (int c = 0; c < SUMS; c++) {
-          const typename H::v4 a = __builtin_bit_cast(typename H::v4, v[c * PAIR + i]);
-          t[c] = H::two(__builtin_shufflevector(a, a, 0, 1, 2, 3, 0, 1, 2, 3), high[i],
-                        decltype(first)::value && i == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : t[c]);
-        }
+        for (int i = 0; i < PAIR; i++)
 #pragma unroll
-      for (int i = 0; i < PAIR; i++)
-#pragma unroll
-        for (int c = 0; c < SUMS; c++) t[c] = H::one(__builtin_bit_cast(typename H::v4, v[c * PAIR + i]), low[i], t[c]);
+          for (int c = 0; c < SUMS; c++) {
+            const typename H::v4 a = __builtin_bit_cast(typename H::v4, v[c * PAIR + i]);
+            t[c] = H::product(__builtin_shufflevector(a, a, 0, 1, 2, 3, 0, 1, 2, 3), part[k][i],
+                              decltype(first)::value && k == 0 && i == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : t[c]);
+          }
     } else {
       float bx[PAIR][4];
 #pragma unroll
