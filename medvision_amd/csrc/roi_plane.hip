@@ -5,7 +5,7 @@
 // wx[cell column], each the sum over the cell's samples on that axis, so that with G = the 7 x 7 cells of a channel
 //     forward  G = Wy box Wx^T,        backward  box += Wy^T G Wx
 // are two small matrix products per channel each.  They run on the fp32 matrix cores (16 x 16 x 4, exact fp32
-// products and sums), the forward pass's first one on the 16-bit ones where the pixels are 16-bit (PlaneHalf).  A dense product gives 0 x infinity for a pixel or gradient that no sample's weight reaches, so
+// products and sums), the first one on the 16-bit ones where the pixels or gradients are 16-bit (PlaneHalf).  A dense product gives 0 x infinity for a pixel or gradient that no sample's weight reaches, so
 // sums that come out not finite are formed again without the terms of weight 0 (one test per finished sum; the second
 // pass runs for such channels and tiles alone).  The accumulator of the first product is the right-hand operand of the second as it stands:
 // lane l holds column l % 16 and the four rows 4 (l / 16) + r, and a product's step r takes K = one row per lane
@@ -23,9 +23,10 @@
 // Backward, one workgroup = (16 x 16 pixels, some channels): it looks up the rois that touch its pixels, works out
 // its pixels' weights for eight rois at a time and adds roi after roi into accumulators that stay in registers.  No
 // atomics, no fp32 copy of the gradient, every pixel written once, sums in the order of the rois.
-//   (The same head: 1030 us with one atomic per touched pixel, roi and channel; 145 us now: matrix cores 50 %, vector issue 32 %.)
-// What bounds them: the matrix cores (three 32-clock instructions per roi, tile and channel backward; 4 x pieces + 2
-// per row piece and channel forward, 4 with 16 cells) and the latency of the loads.
+//   (The same head: 1030 us with one atomic per touched pixel, roi and channel; 145 us now: matrix cores 50 %, vector issue 32 %.  16-bit
+//   gradients, 14 x 14 cells: fp16 1499 rois x 256 channels 304 us with fp32 products, 207 us; bf16 1689 x 128 207 us, 143 us.)
+// What bounds them: the matrix cores (three 32-clock instructions per roi, tile and channel backward, eight with 16 cells; 4 x pieces + 2
+// per row piece and channel forward, + 4 with 16 cells; a first product of 16-bit values takes a quarter, forward, or less) and the latency of the loads.
 #include <algorithm>
 
 #include "common.hpp"
@@ -497,30 +498,54 @@ __global__ __launch_bounds__(kPlaneThreads, CELLS == 8 ? 4 : 2) void roi_plane_b
 #pragma unroll
     for (int i = 0; i < PIECES; i++) v[i] = plane_load_cells<T, STEPS>(rsrc, off, i * pair_bytes);
   };
+  // (a load that reaches past its row of cells brings the next row's, channel's or roi's: cleared, 0 x inf is not 0)
+  using Bits = typename std::conditional<ES * STEPS == 4, unsigned, unsigned long long>::type;   // of a 16-bit load
+  const Bits keep = have >= STEPS ? static_cast<Bits>(~0ull) : have <= 0 ? 0 : (static_cast<Bits>(1) << (16 * have)) - 1;
   auto add = [&](PlaneCells<T, STEPS> (&v)[PIECES], int bi) {
-    if constexpr (ES == 2) {
-      typename std::conditional<STEPS == 2, unsigned, unsigned long long>::type bits;
-#pragma unroll
-      for (int i = 0; i < PIECES; i++) {
-        __builtin_memcpy(&bits, &v[i], sizeof(bits));
-        bits >>= 16 * back;
-        __builtin_memcpy(&v[i], &bits, sizeof(bits));
-      }
-    }
+    using H = PlaneHalf<T>;
     float wx[STEPS], wy[STEPS];
 #pragma unroll
     for (int t = 0; t < STEPS; t++) {
-      wx[t] = weights[bi][0][m][pw + t];
-      wy[t] = weights[bi][1][m][q + 4 * t];
+      wx[t] = weights[bi][0][m][pw + t] * H::kScale;
+      wy[t] = weights[bi][1][m][q + 4 * t] * (1.f / H::kScale);
     }
     // (products of different channels next to each other: each waits for the one before it of its own channel)
     f32x4_t t[PIECES];
+    constexpr f32x4_t zero = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if constexpr (ES == 2) {
+      // the gradients stand twice (four times) in K, against the weights' parts
+      constexpr int PRODUCTS = STEPS / 2;
+      typename H::v8 parts[PRODUCTS];
 #pragma unroll
-    for (int k = 0; k < STEPS; k++)
+      for (int k = 0; k < STEPS; k++) {
+        const typename H::E first = static_cast<typename H::E>(wx[k]);
+        const float left = wx[k] - static_cast<float>(first);
+        const typename H::E second = static_cast<typename H::E>(left);
+        parts[0][k] = first;
+        parts[0][STEPS + k] = second;
+        if constexpr (STEPS == 2) parts[0][2 * STEPS + k] = static_cast<typename H::E>(left - static_cast<float>(second));
+        else parts[PRODUCTS - 1][k] = static_cast<typename H::E>(left - static_cast<float>(second));
+        parts[PRODUCTS - 1][8 - STEPS + k] = static_cast<typename H::E>(0.f);
+      }
 #pragma unroll
-      for (int i = 0; i < PIECES; i++)
-        // (a load that reaches past its row of cells brings the next row's, channel's or roi's: cleared, 0 x inf is not 0)
-        t[i] = plane_product(k < have ? load(&v[i].v[k]) : 0.f, wx[k], k == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : t[i]);
+      for (int k = 0; k < PRODUCTS; k++)
+#pragma unroll
+        for (int i = 0; i < PIECES; i++) {
+          Bits bits;
+          __builtin_memcpy(&bits, &v[i], sizeof(bits));
+          bits = (bits >> (16 * back)) & keep;
+          typename H::v8 g;
+          if constexpr (STEPS == 2) g = __builtin_bit_cast(typename H::v8, plane_u32x4{bits, bits, bits, bits});
+          else g = __builtin_bit_cast(typename H::v8, plane_u32x4{static_cast<unsigned>(bits), static_cast<unsigned>(bits >> 32), static_cast<unsigned>(bits), static_cast<unsigned>(bits >> 32)});
+          t[i] = H::product(g, parts[k], k == 0 ? zero : t[i]);
+        }
+    } else {
+#pragma unroll
+      for (int k = 0; k < STEPS; k++)
+#pragma unroll
+        for (int i = 0; i < PIECES; i++)
+          t[i] = plane_product(k < have ? load(&v[i].v[k]) : 0.f, wx[k], k == 0 ? zero : t[i]);
+    }
 #pragma unroll
     for (int s = 0; s < STEPS; s++)
 #pragma unroll
