@@ -396,13 +396,14 @@ __device__ inline void pool_forward_mfma(const T *__restrict__ src_any, T *__res
   // and stores.
   const int tiles = (c_count + 3) / 4;
   const bool few = tiles <= kPoolThreads / kWave;   // a tile per wavefront
+  const int after_even = few ? kPoolThreads / kWave : 1, after_odd = few ? kPoolThreads / kWave : 2 * (kPoolThreads / kWave) - 1;
   struct Step { int tile, zg, k0; };
   struct Loaded { u32x2 va[2], vb[2]; };
   auto next_of = [&](Step st) {
     st.k0 += 32;
     if (st.k0 >= KP) {
       st.k0 = 0; st.zg += 2;
-      if (st.zg >= zgroups) { st.zg = 0; st.tile += few ? kPoolThreads / kWave : st.tile % 2 == 0 ? 1 : 2 * (kPoolThreads / kWave) - 1; }
+      if (st.zg >= zgroups) { st.zg = 0; st.tile += st.tile % 2 == 0 ? after_even : after_odd; }
     }
     return st;
   };
@@ -950,7 +951,7 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_forward_kernel(
 // of 64 contiguous bytes.  Wavefronts work on different channel blocks or slices and share nothing but the
 // weights: no barrier after the set-up.
 constexpr int kPoolBwdRow = 72;   // fp16 elements per row of the transposed weights: 64 cells + pad
-template <typename T>
+template <typename T, bool SHARE>
 __device__ inline void pool_backward_mfma(const T *__restrict__ src_any, float *__restrict__ dst_any, const RoiProblem &p,
                                           const PoolShared &sh, const float (&wd)[3][kDenseSrc][8],
                                           unsigned char *lds, int c_count, int part, int parts) {
@@ -1008,11 +1009,15 @@ __device__ inline void pool_backward_mfma(const T *__restrict__ src_any, float *
       const_cast<T *>(src), 0, c_count * cells * 2 + 16, 0x00020000);
   // wavefronts side by side on channel blocks; where there are fewer blocks, several share a block's slices
   constexpr int kWaves = kPoolThreads / kWave;
-  const int blocks = (c_count + 15) / 16, side = blocks == 1 ? 1 : blocks == 2 ? 2 : kWaves;
-  const int shares = parts * (kWaves / side), share = part * (kWaves / side) + wave / side;
-  const int z_first = nz * share / shares, z_last = nz * (share + 1) / shares;
-  if (z_first == z_last) return;
-  for (int blk = wave % side; blk < blocks; blk += side) {
+  const int blocks = (c_count + 15) / 16, side = !SHARE || blocks > 2 ? kWaves : blocks;
+  int z_first = 0, z_last = nz;
+  if constexpr (SHARE) {
+    const int shares = parts * (kWaves / side), share = part * (kWaves / side) + wave / side;
+    z_first = nz * share / shares;
+    z_last = nz * (share + 1) / shares;
+    if (z_first == z_last) return;
+  }
+  for (int blk = SHARE ? wave % side : wave; blk < blocks; blk += SHARE ? side : kWaves) {
     const int c = blk * 16 + col;
     const bool cv = c < c_count;
     // the lane's gradient pieces: cells quad * 8 .. + 7 (+ 32) of every pd of its channel
@@ -1041,7 +1046,7 @@ __device__ inline void pool_backward_mfma(const T *__restrict__ src_any, float *
     for (int pd = 0; pd < 8; pd++)
 #pragma unroll
       for (int ks = 0; ks < 2; ks++) g[pd][ks] &= keep[ks];
-    for (int z = z_first; z < z_last; z++) {
+    for (int z = SHARE ? z_first : 0; z < (SHARE ? z_last : nz); z++) {
       float wz[8];
       {
         const float4 lo4 = *reinterpret_cast<const float4 *>(&wd[2][z][0]), hi4 = *reinterpret_cast<const float4 *>(&wd[2][z][4]);
@@ -1081,7 +1086,8 @@ __device__ inline void pool_backward_mfma(const T *__restrict__ src_any, float *
 // CL: the accumulation buffer is channels-last [N, D*H*W, C] (a workspace): the lanes of a wavefront
 // then add neighbouring channels of a voxel, contiguous bytes,
 // instead of one element in each of many rows (a scattered atomic moves a whole memory sector).
-template <typename T, typename G, typename RT, bool CL, int CELLS>
+// SHARE: gridDim.z workgroups share the slices of a box.
+template <typename T, typename G, typename RT, bool CL, int CELLS, bool SHARE>
 __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
     const T *__restrict__ gout, const RT *__restrict__ rois, G *__restrict__ gin, const RoiProblem p,
     const int channels_per_block) {
@@ -1089,7 +1095,7 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
   __shared__ __attribute__((aligned(16))) unsigned char lds[kPoolLdsBytes];
   const unsigned n = blockIdx.x;
   const int c_begin = blockIdx.y * channels_per_block, c_end = min(c_begin + channels_per_block, p.C);
-  const int part = CL ? blockIdx.z : 0, parts = CL ? gridDim.z : 1;   // of the workgroups that share the box's slices
+  const int part = SHARE ? blockIdx.z : 0, parts = SHARE ? gridDim.z : 1;
   // intermediates are fp32 here, so size the chunk with 4-byte box elements
   __shared__ __attribute__((aligned(16))) float wd[3][kDenseSrc][CELLS];
   PoolPlan plan = pool_setup<RT, CELLS>(sh, rois + static_cast<long>(n) * roi_columns(p.ndim, 0), p, sizeof(float), wd, true);
@@ -1155,8 +1161,8 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
   const float inv_nxy = 1.f / (nx * ny), inv_nx = 1.f / nx, inv_ow = 1.f / p.ow,
               inv_ohw = 1.f / ohw, inv_nyow = 1.f / (ny * p.ow),
               inv_gx = 1.f / gx, inv_gy = 1.f / gy, inv_gz = 1.f / gz;
-  const int z_first = nz * part / parts, z_last = nz * (part + 1) / parts;
-  if (z_first == z_last) return;
+  const int z_first = SHARE ? nz * part / parts : 0, z_last = SHARE ? nz * (part + 1) / parts : nz;
+  if (SHARE && z_first == z_last) return;
   if (dense) {   // (the set-up has built the matrices)
     if constexpr (CL && CELLS == 8 && std::is_same<T, __half>::value && std::is_same<G, float>::value) {
       // matrix-core form: 32-bit offsets into the image's accumulation buffer and into this roi's
@@ -1169,7 +1175,7 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
       // than the tensor's last block)
       const long behind = (static_cast<long>(p.R) * p.C - (static_cast<long>(n) * p.C + c_end)) * cells * 2;
       if (fits && small && behind >= 16) {
-        pool_backward_mfma(src, dst_cl, p, sh, wd, lds, c_end - c_begin, part, parts);
+        pool_backward_mfma<T, SHARE>(src, dst_cl, p, sh, wd, lds, c_end - c_begin, part, parts);
         return;
       }
     }
@@ -1450,10 +1456,10 @@ static void launch_pool_forward(const void *input, const float *r, void *output,
                      static_cast<const T *>(blocked), p.W / 4, order);
 }
 
-template <typename T, bool CL, int CELLS>
+template <typename T, bool CL, int CELLS, bool SHARE>
 static void launch_pool_backward(const void *grad_output, const float *r, void *acc, const RoiProblem &p, int cpb,
                                  dim3 grid, hipStream_t s) {
-  hipLaunchKernelGGL((roi_pool_backward_kernel<T, float, float, CL, CELLS>), grid, dim3(kPoolThreads), 0, s,
+  hipLaunchKernelGGL((roi_pool_backward_kernel<T, float, float, CL, CELLS, SHARE>), grid, dim3(kPoolThreads), 0, s,
                      static_cast<const T *>(grad_output), r, static_cast<float *>(acc), p, cpb);
 }
 
@@ -1584,26 +1590,28 @@ int roi_pool_backward(const void *grad_output, const void *rois, void *acc, int 
   if (share) cpb = std::max(cpb, std::min(p.C, mfma && p.R * ((p.C + 31L) / 32) >= 256 ? 32 : 16));
   const long cblocks = (p.C + cpb - 1) / cpb;
   if (cblocks > 65535) return -1;
-  const long groups = p.R * cblocks, parts = share ? std::min((1023 + groups) / groups, 4L) : 1;
+  // (larger blocks leave 1024 workgroups and more, and cost nothing where the kernel works out no shares: 5 us of 1190 for the
+  // training step of 4000 rois of 256 channels)
+  const bool shared = share && cpb <= 32;
+  const long groups = p.R * cblocks, parts = shared ? std::min((1023 + groups) / groups, 4L) : 1;
   const dim3 grid(p.R, static_cast<unsigned>(cblocks), static_cast<unsigned>(parts));
   const float *r = static_cast<const float *>(rois);
   const bool small = pool_small_cells(p);
-#define MV_POOL_BACKWARD(TYPE, CLV)                                                          \
-  (small ? launch_pool_backward<TYPE, CLV, 8>(grad_output, r, acc, p, cpb, grid, s)          \
-         : launch_pool_backward<TYPE, CLV, 16>(grad_output, r, acc, p, cpb, grid, s))
+#define MV_POOL_BACKWARD(TYPE, CLV, SHAREV)                                                          \
+  (small ? launch_pool_backward<TYPE, CLV, 8, SHAREV>(grad_output, r, acc, p, cpb, grid, s)          \
+         : launch_pool_backward<TYPE, CLV, 16, SHAREV>(grad_output, r, acc, p, cpb, grid, s))
+#define MV_POOL_BACKWARD_OF(TYPE)                                                                    \
+  do {                                                                                               \
+    if (shared) MV_POOL_BACKWARD(TYPE, true, true);                                                  \
+    else if (channels_last) MV_POOL_BACKWARD(TYPE, true, false);                                     \
+    else MV_POOL_BACKWARD(TYPE, false, false);                                                       \
+  } while (0)
   switch (dtype) {
-    case MV_F32:
-      if (channels_last) MV_POOL_BACKWARD(float, true);
-      else MV_POOL_BACKWARD(float, false);
-      break;
-    case MV_F16:
-      if (channels_last) MV_POOL_BACKWARD(__half, true);
-      else MV_POOL_BACKWARD(__half, false);
-      break;
-    default:
-      if (channels_last) MV_POOL_BACKWARD(__hip_bfloat16, true);
-      else MV_POOL_BACKWARD(__hip_bfloat16, false);
+    case MV_F32: MV_POOL_BACKWARD_OF(float); break;
+    case MV_F16: MV_POOL_BACKWARD_OF(__half); break;
+    default: MV_POOL_BACKWARD_OF(__hip_bfloat16);
   }
+#undef MV_POOL_BACKWARD_OF
 #undef MV_POOL_BACKWARD
   return check_launch("roi_pool_backward_kernel");
 }
