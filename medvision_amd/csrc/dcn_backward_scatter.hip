@@ -9,13 +9,13 @@
 // broadcasts, which the multiplications take as an operand, and an LDS addition meets four (eight) cells of 64 contiguous bytes.
 // Per term: multiply, convert, add.  Corners outside the tile or the volume have weight 0 in a cell that exists: no branches.
 //   (Channels as rows, a lane holding one position and four channels, needed the samples' words from LDS, a branch per corner
-//   and additions to 16 places: bf16 [2, 32 -> 64, 48^3] 496 us, now 338 us; fp16 [8, 256 -> 256, 100 x 152] 1185 us, now 500 us.)
+//   and additions to 16 places: bf16 [2, 32 -> 64, 48^3] 496 us, then 338 us (351 us with today's larger tile); fp16 [8, 256 -> 256, 100 x 152] 1185 us, now 500 us.)
 // Afterwards the tile's non-zero sums are added to the gradient buffer, one global atomic per (voxel, channel) of the tile
 // instead of one per (position, tap, corner, channel).
 //
 // NARROW (dense layers of 16-bit tensors, see dcn_scatter_plan): 32-bit sums.  They leave 31 - log2(positions * taps) bits for
 // a term (18 for 3 x 3 x 3 taps), so the scale comes from the data: a first sweep over the brick's taps forms gcol alone (matrix
-// cores, no geometry; 17 us of the 338) and takes max |gcol| of the workgroup; every term is then below max |gcol| * max |mask| <
+// cores, no geometry; 17 us) and takes max |gcol| of the workgroup; every term is then below max |gcol| * max |mask| <
 // 2^ex and is rounded to a multiple of 2^(ex - shift).  The error of a voxel's sum stays below terms * 2^(ex - shift - 1), about
 // 2^-16 of the values it sums for the 3 x 3 x 3 layer — a thirty-second of the last bit of a bf16 result.  Otherwise a 64-bit word
 // per channel, scale from the global maxima.

@@ -25,7 +25,7 @@
 // (43 %; vector issue 29 %, matrix cores 20 %) and the same waits, and everywhere the atomics of the far corners (64 bytes per corner
 // and 16 channels, 21 G of them a second at best).
 //   (bf16 [2, 32 -> 64, 48^3]: 409 us; the data and weight kernels before it took 670 us.  fp16 images
-//   [8, 256 -> 256, 100 x 152]: 582 us, 4380 us before.  [1, 128 -> 128, 7 x 45 x 18]: 64 us, 790 us before.)
+//   [8, 256 -> 256, 100 x 152]: 582 us, 4380 us before.  [1, 128 -> 128, 7 x 45 x 18]: 60 us, 790 us before.)
 #include "dcn_scatter.hpp"
 
 #include <algorithm>
