@@ -386,9 +386,25 @@ using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions
 // the larger tile, smaller ones only cost more halo (30 layers of fewer than 256 workgroups: 2 % slower).  False: no brick fits.
 //
 // Width of the sums: 32 bits round every term to 14 - 22 bits of the workgroup's largest, which is worth their speed in dense
-// layers alone (16-bit tensors, the first brick fits: unit strides, taps close together; up to 128 output channels).  bf16 training
+// layers alone (dcn_dense; 16-bit tensors, up to 128 output channels).  bf16 training
 // step of [2, 32 -> 64, 48^3]: 1178 us, 1393 us with 64-bit sums (with the kernel before this one).  Strided and wide layers have 64-bit sums, as good as fp32 ones:
-// where the output's gradient is 2^-14 of what it is elsewhere in the brick, 32 bits left them 2 - 20 % off. 
+// where the output's gradient is 2^-14 of what it is elsewhere in the brick, 32 bits left them 2 - 20 % off.
+
+// Voxels along one axis that the undeformed taps of neighbouring positions reach
+static long dcn_reach(int positions, int stride, int taps, int dilation) {
+  return (positions - 1L) * stride + (taps - 1L) * dilation + 1;
+}
+// Dense layers: unit strides and taps close together, a rule of the layer whatever the tiles hold (tiles that grew by two voxels
+// took layers of stride (2, 1, 1), dilation (3, 1, 1) and 7 x 3 x 3 taps with them, whose 32-bit sums were 14 - 18 % off there).
+static bool dcn_dense(const DcnDims &s) {
+  if (s.nd == 2) return dcn_reach(32, s.sh, s.kh, s.dh) <= 42 && dcn_reach(32, s.sw, s.kw, s.dw) <= 42;
+  return dcn_reach(4, s.sd, s.kd, s.dd) <= 8 && dcn_reach(8, s.sh, s.kh, s.dh) <= 12 && dcn_reach(8, s.sw, s.kw, s.dw) <= 12;
+}
+// Among them, volumes that take bricks of 4 x 8 x 8 positions.  Those whose taps reach further have bricks of 4 x 4 x 4 (also where the
+// larger tile would hold them): two bits more for a term, and one maximum for a quarter of the positions.
+static bool dcn_dense_large(const DcnDims &s) {
+  return dcn_reach(4, s.sd, s.kd, s.dd) <= 6 && dcn_reach(8, s.sh, s.kh, s.dh) <= 10 && dcn_reach(8, s.sw, s.kw, s.dw) <= 10;
+}
 bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
   static const int volumes[2][6] = {{2, 3, 3, 12, 14, 14}, {2, 2, 2, 12, 12, 13}};
   static const int deep[2][6] = {{2, 2, 3, 9, 10, 14}, {1, 2, 2, 8, 12, 13}};
@@ -426,8 +442,8 @@ bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
   // (offsets and weights at 32-bit byte offsets from scalar bases)
   if (s.Cin / 8 > 65535 || s.Q >= (1L << 28) || static_cast<long>(s.K) * s.cpg * s.opg * (dtype == MV_F32 ? 4 : 2) >= (1L << 31)) return false;
   bool fits = false;
-  if (dtype != MV_F32 && s.opg <= 128 && spare_of(image ? dense_images[0] : volumes[0]) >= 2) {
-    fits = image ? choose(dense_images, 3, 16) : choose(volumes, 2, 16);
+  if (dtype != MV_F32 && s.opg <= 128 && dcn_dense(s)) {
+    fits = image ? choose(dense_images, 3, 16) : choose(dcn_dense_large(s) ? volumes : volumes + 1, 1, 16);
     shape.narrow = fits && shape.terms <= kScatter32Terms;
   }
   if (!shape.narrow) {

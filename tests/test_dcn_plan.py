@@ -1,0 +1,53 @@
+"""The plan of the deformable backward's LDS sums (``dcn_scatter_plan``, host code): bricks, tiles and the width of the sums,
+asked of the built library without a GPU."""
+import ctypes
+import math
+
+import pytest
+
+from medvision_amd import _lib
+
+
+class _Dims(ctypes.Structure):   # DcnDims (csrc/dcn_common.hpp)
+    _fields_ = [(n, ctypes.c_int) for n in (
+        "B", "Cin", "D", "H", "W", "Cout", "kd", "kh", "kw", "sd", "sh", "sw", "pd", "ph", "pw", "dd", "dh", "dw",
+        "groups", "dg", "nd", "Do", "Ho", "Wo", "K", "cpg", "opg", "cpd")] + [("Q", ctypes.c_long), ("P", ctypes.c_long)]
+
+
+class _Shape(ctypes.Structure):   # ScatterShape (csrc/dcn_scatter.hpp)
+    _fields_ = [(n, ctypes.c_int) for n in (
+        "bd", "bh", "bw", "td", "th", "tw", "nbd", "nbh", "nbw", "terms", "narrow", "turns")]
+
+
+def _plan(code, batch, cin, cout, size, kernel=3, stride=1, dilation=1, padding=None):
+    """The plan of a layer, None where no brick fits."""
+    nd = len(size)
+    each = lambda v: (1,) * (3 - nd) + ((v,) * nd if isinstance(v, int) else tuple(v))
+    k, s, d, n = each(kernel), each(stride), each(dilation), (1,) * (3 - nd) + tuple(size)
+    p = tuple((a - 1) * b // 2 for a, b in zip(k, d)) if padding is None else (0,) * (3 - nd) + (padding,) * nd
+    out = [(n[a] + 2 * p[a] - (d[a] * (k[a] - 1) + 1)) // s[a] + 1 for a in range(3)]
+    dims = _Dims(batch, cin, *n, cout, *k, *s, *p, *d, 1, 1, nd, *out, math.prod(k), cin, cout, cin, math.prod(out), math.prod(n))
+    fn = _lib.load()._ZN2mv16dcn_scatter_planERKNS_7DcnDimsEiRNS_12ScatterShapeE
+    fn.restype, fn.argtypes = ctypes.c_bool, [ctypes.POINTER(_Dims), ctypes.c_int, ctypes.POINTER(_Shape)]
+    shape = _Shape()
+    return shape if fn(ctypes.byref(dims), code, ctypes.byref(shape)) else None
+
+
+@pytest.mark.parametrize("code", [_lib.MV_F16, _lib.MV_BF16])
+@pytest.mark.parametrize("kernel,stride,dilation,narrow,brick", [
+    (3, 1, 1, 1, (2, 3, 3)),
+    ((1, 3, 3), (2, 1, 1), 1, 1, (2, 2, 2)),      # every other slice, each by itself
+    (3, 1, (2, 1, 1), 1, (2, 2, 2)),               # 19 bits for a term, not the 18 of the larger brick
+    (3, (2, 1, 1), 1, 0, None),                    # strided
+    (3, 1, (3, 1, 1), 0, None),                    # taps far apart
+    ((7, 3, 3), 1, 1, 0, None),
+    (3, (1, 2, 1), 1, 0, None),
+    (3, 1, (1, 1, 3), 0, None),
+    (3, 2, 1, 0, None),
+])
+def test_width_of_the_sums_of_volumes(code, kernel, stride, dilation, narrow, brick):
+    """32-bit sums are for dense layers: with strides or taps far apart along any axis the sums have 64 bits, whatever the tiles hold."""
+    shape = _plan(code, 2, 32, 64, (48, 48, 48), kernel, stride, dilation)
+    assert shape.narrow == narrow
+    if brick:
+        assert (shape.bd, shape.bh, shape.bw) == brick

@@ -60,3 +60,39 @@ def test_samples_on_borders(oracle, dtype, cin, cout, size, stride, groups, dg):
 def test_two_channel_blocks_per_workgroup(oracle, dtype, batch, cout, size):
     """Wide images of 2048 and more workgroups of sixteen channels sum 32 channels in two turns."""
     _gradient(oracle, dtype, batch, 512, cout, size, 1, 1, 1, lambda off, g: off, batch + sum(size))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("kernel,stride,dilation", [
+    ((3, 3, 3), (2, 1, 1), (1, 1, 1)),
+    ((3, 3, 3), (1, 1, 1), (3, 1, 1)),
+    ((7, 3, 3), (1, 1, 1), (1, 1, 1)),
+])
+def test_small_gradients_beside_large_ones_along_one_axis(oracle, dtype, kernel, stride, dilation):
+    """Layers that are strided, dilated or deep along one axis alone sum the input's gradient in 64 bits too: where the output's
+    gradient is 2^-14 of what it is in the same brick, the sums are as good as anywhere (rounding of the result: 2^-11 / 2^-8)."""
+    from medvision_amd import _C
+    cin, cout, size = 32, 64, (9, 8, 40)
+    g = wl.gen(sum(kernel) + sum(stride) + sum(dilation))
+    pad = tuple((k - 1) * d // 2 for k, d in zip(kernel, dilation))
+    out = [(n + 2 * p - (d * (k - 1) + 1)) // s + 1 for n, p, d, k, s in zip(size, pad, dilation, kernel, stride)]
+    taps = kernel[0] * kernel[1] * kernel[2]
+    x = torch.randn(1, cin, *size, generator=g).to(dtype)
+    w = (torch.randn(cout, cin, *kernel, generator=g) / (cin * taps) ** 0.5).to(dtype)
+    off = (torch.rand(1, 3 * taps, *out, generator=g) - 0.5).to(dtype)
+    mask = torch.rand(1, taps, *out, generator=g).to(dtype)
+    gy = torch.randn(1, cout, *out, generator=g)
+    split = 20      # in the middle of a brick of eight columns
+    gy[..., :split] *= 2.0 ** -6
+    gy[..., split:] *= 2.0 ** 8
+    gy = gy.to(dtype)
+    ins = [t.to(DEV) for t in (x, w, torch.zeros(cout, dtype=dtype), off, mask)]
+    sums = [torch.zeros_like(t) for t in ins]
+    _C.modulated_deform_conv_3d_backward(ins[0], ins[1], ins[2], None, ins[3], ins[4], None, sums[0], sums[1], sums[2], sums[3], sums[4],
+                                         gy.to(DEV), *kernel, *stride, *pad, *dilation, 1, 1, True)
+    want = oracle.dcn3d_backward(x, off, mask, w, gy, True, stride, pad, dilation, 1, 1)[0].reshape(x.shape)
+    edge = split - 3      # columns that no position beyond the split reaches
+    got, want = sums[0].cpu().double()[..., :edge], want[..., :edge]
+    assert float(want.abs().max()) < 1.0       # nothing of the large ones
+    error = float((got - want).norm() / want.norm())
+    assert error < (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8), error
