@@ -368,7 +368,7 @@ using TileStrided = Tile<12, 12, 13>;   // 4 x 4 x 4 positions: dilation, 64-bit
 using TileDeep = Tile<9, 10, 14>;       // 4 x 4 x 8 positions, 64-bit sums of 16-bit tensors
 using TileDeepStrided = Tile<8, 12, 13>;   // 2 x 4 x 4 positions, the same at stride 2
 template <typename S> constexpr bool kDeep = std::is_same<S, TileDeep>::value || std::is_same<S, TileDeepStrided>::value;
-using TileImage = Tile<1, 44, 44>;      // 32 x 32 positions, 32-bit sums
+using TileImage = Tile<1, 44, 44>;      // 32 x 32 positions, 32-bit sums; 16 x 16 positions whose taps are far apart, 64-bit sums
 using TileWide = Tile<1, 28, 44>;       // 16 x 32 positions (8 x 16 at stride 2), 64-bit sums
 using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions
 
@@ -378,7 +378,9 @@ using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions
 // against 78 us for [2, 16 -> 128, 7 x 19 x 32]).  Images with 64-bit sums have smaller tiles of 16 channels instead of 44 x 44 of 8:
 // half the samples to work out, and 5.5 million requests of 64 bytes instead of 9.9 of 32 for [8, 256 -> 256, 100 x 152].  Where no
 // brick of images gives a workgroup to every compute unit, the one of most workgroups (fp32 [2, 128 -> 256, 36 x 18]: 48 of
-// 16 x 32 positions 131 us, 240 of 8 x 8 31 us).  Volumes of 16-bit tensors with 64-bit sums have
+// 16 x 32 positions 131 us, 240 of 8 x 8 31 us).  Images whose taps are too far apart for those (3 x 3 taps from dilation 9 on) have
+// 16 x 16 positions in 44 x 44 of 8 channels, up to dilation 13 (backward pass at dilation 12, with every corner left to the tap kernel
+// and with the tile: fp16 [2, 64 -> 64, 64 x 64] 142 and 121 us, [2, 256 -> 256, 64 x 64] 305 and 264 us).  Volumes of 16-bit tensors with 64-bit sums have
 // smaller tiles of 16 channels too, where they leave three voxels to spare: bf16 [4, 32 -> 128, 57 x 51 x 27] at stride 2 472 us
 // with 12 x 12 x 13 of 8, 407 us with 8 x 12 x 13 of 16 (the tap kernel, which adds the corners beyond the smaller bricks' tiles,
 // 236 -> 275 us).  fp32 ones would gain more ([4, 16 -> 16, 17 x 43 x 30] 343 us, 244 us with 9 x 10 x 14 of 16), but every
@@ -410,6 +412,7 @@ bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
   static const int deep[2][6] = {{2, 2, 3, 9, 10, 14}, {1, 2, 2, 8, 12, 13}};
   static const int dense_images[3][6] = {{0, 5, 5, 1, 44, 44}, {0, 4, 4, 1, 28, 28}, {0, 3, 3, 1, 28, 28}};
   static const int images[4][6] = {{0, 4, 5, 1, 28, 44}, {0, 4, 4, 1, 28, 28}, {0, 3, 4, 1, 28, 44}, {0, 3, 3, 1, 28, 28}};
+  static const int far_images[1][6] = {{0, 4, 4, 1, 44, 44}};
   const bool image = s.nd == 2;
   const int st[3] = {s.sd, s.sh, s.sw}, kn[3] = {s.kd, s.kh, s.kw}, dl[3] = {s.dd, s.dh, s.dw}, on[3] = {s.Do, s.Ho, s.Wo};
   // voxels to spare in a tile; workgroups
@@ -449,6 +452,8 @@ bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
   if (!shape.narrow) {
     const int (*const small)[6] = image || dtype == MV_F32 ? nullptr : spare_of(deep[0]) >= 3 ? deep : spare_of(deep[1]) >= 3 ? deep + 1 : nullptr;
     fits = image ? choose(images, 4, 16) : small ? choose(small, 1, 16) : choose(volumes, 2, 8);
+    const int taken[6] = {shape.bd, shape.bh, shape.bw, shape.td, shape.th, shape.tw};
+    if (image && (!fits || spare_of(taken) < 4) && spare_of(far_images[0]) >= (fits ? 4 : 2)) fits = choose(far_images, 1, 8);
   }
   if (!fits) return false;
   shape.nbd = (s.Do + (1 << shape.bd) - 1) >> shape.bd;
@@ -466,7 +471,8 @@ static int scatter_launch(const void *off, const void *mask, const void *gyt, co
   const int slices = s.opg / (64 / static_cast<int>(sizeof(T)));
 #define MV_SCATTER(NARROWV, KEEPV)                                                                                    \
   hipLaunchKernelGGL((dcn_backward_scatter_kernel<T, NARROWV, S, KEEPV>),                                              \
-                     dim3(static_cast<unsigned>(shape.nbd) * shape.nbh * shape.nbw * s.B * (s.Cin / (S::template channels<NARROWV> * (KEEPV == 8 ? shape.turns : 1)))), \
+                     dim3(static_cast<unsigned>(shape.nbd) * shape.nbh * shape.nbw * s.B *                              \
+                          (s.Cin / (S::template channels<NARROWV> * (KEEPV == 8 && S::template channels<NARROWV> == 16 ? shape.turns : 1)))), \
                      dim3(KEEPV <= 4 ? 1024 : 512), 0, stream,                                                         \
                      static_cast<const T *>(off), static_cast<const T *>(mask), static_cast<const T *>(gyt),          \
                      static_cast<const T *>(wf), gxt, s, shape, bounds)
@@ -474,7 +480,7 @@ static int scatter_launch(const void *off, const void *mask, const void *gyt, co
     if constexpr (sizeof(T) == 2 && !kDeep<S> && !S::WIDE) {   // (those have 64-bit sums)
       if (slices <= 2) MV_SCATTER(true, 2); else MV_SCATTER(true, 4);
     }
-  } else if constexpr (!std::is_same<S, TileImage>::value && !(kDeep<S> && sizeof(T) == 4)) {   // (never of these)
+  } else if constexpr (!(kDeep<S> && sizeof(T) == 4)) {   // (never of those)
     if (slices <= 2) MV_SCATTER(false, 2);
     else if (slices <= 4) MV_SCATTER(false, 4);
     else MV_SCATTER(false, 8);

@@ -51,3 +51,18 @@ def test_width_of_the_sums_of_volumes(code, kernel, stride, dilation, narrow, br
     assert shape.narrow == narrow
     if brick:
         assert (shape.bd, shape.bh, shape.bw) == brick
+
+
+@pytest.mark.parametrize("code", [_lib.MV_F32, _lib.MV_F16, _lib.MV_BF16])
+@pytest.mark.parametrize("cout", [64, 256])
+@pytest.mark.parametrize("kernel,stride,dilation", [
+    (3, 1, 9), (3, 1, 10), (3, 1, 12), (3, 1, 13), (3, 1, (12, 2)), (3, 1, (1, 12)), ((3, 5), (1, 2), (12, 1)),
+])
+def test_images_with_taps_far_apart_keep_their_tiles(code, cout, kernel, stride, dilation):
+    """A tile of 44 x 44 voxels holds the reach of 3 x 3 taps up to dilation 13: their corners are summed in LDS."""
+    shape = _plan(code, 2, 128, cout, (112, 208), kernel, stride, dilation)
+    assert shape is not None
+    st, dl, kn = ((v, v) if isinstance(v, int) else v for v in (stride, dilation, kernel))
+    spare = min(t - ((1 << b) - 1) * s - (k - 1) * d - 1
+                for t, b, s, k, d in zip((shape.th, shape.tw), (shape.bh, shape.bw), st, kn, dl))
+    assert spare >= (4 if max(dl) <= 12 else 2)

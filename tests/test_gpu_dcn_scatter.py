@@ -11,19 +11,19 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-def _gradient(oracle, dtype, batch, cin, cout, size, stride, groups, dg, offsets, seed):
+def _gradient(oracle, dtype, batch, cin, cout, size, stride, groups, dg, offsets, seed, dilation=1):
     if len(size) == 3:
         from medvision_amd.ops.modulated_deform_conv_3d import modulated_deform_conv
     else:
         from medvision_amd.ops.modulated_deform_conv_2d import modulated_deform_conv
     g = wl.gen(seed)
-    x, off, mask, w, b = wl.dcn_inputs(g, batch, cin, cout, size, 3, dg, groups, dtype, stride, 1, 1)
+    x, off, mask, w, b = wl.dcn_inputs(g, batch, cin, cout, size, 3, dg, groups, dtype, stride, dilation, dilation)
     off = offsets(off, g).to(dtype)
     leaves = [t.to(DEV).requires_grad_(True) for t in (x, off, mask, w, b)]
-    y = modulated_deform_conv(*leaves, stride, 1, 1, groups, dg)
+    y = modulated_deform_conv(*leaves, stride, dilation, dilation, groups, dg)
     gy = torch.randn(y.shape, generator=g).to(dtype)
     y.backward(gy.to(DEV))
-    want = oracle.dcn3d_backward(x, off, mask, w, gy, True, stride, 1, 1, groups, dg)
+    want = oracle.dcn3d_backward(x, off, mask, w, gy, True, stride, dilation, dilation, groups, dg)
     assert_close(leaves[0].grad, want[0], BWD_TOL[dtype], "input")
     assert_close(leaves[4].grad, want[4], BWD_TOL[dtype], "bias")   # (from 1024 rows of grad_output on several per workgroup)
 
@@ -49,6 +49,18 @@ def _borders(off, g):
 ])
 def test_samples_on_borders(oracle, dtype, cin, cout, size, stride, groups, dg):
     _gradient(oracle, dtype, 2, cin, cout, size, stride, groups, dg, _borders, cin + cout + sum(size))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("cin,cout,size,dilation,groups,dg", [
+    (32, 32, (33, 35), 10, 1, 1),         # a slice or two of grad_output, bricks of 16 x 16 and a remainder
+    (64, 96, (20, 50), 12, 1, 2),         # three (fp32: six), two deformable groups
+    (64, 288, (17, 40), 13, 1, 1),        # more slices than eight
+    (512, 160, (37, 21), 12, 1, 1),       # many channel blocks
+    (64, 64, (48, 30), 9, 2, 1),          # groups
+])
+def test_images_with_taps_far_apart(oracle, dtype, cin, cout, size, dilation, groups, dg):
+    _gradient(oracle, dtype, 2, cin, cout, size, 1, groups, dg, _borders, cin + cout + sum(size), dilation)
 
 
 @pytest.mark.parametrize("dtype,batch,cout,size", [
