@@ -368,9 +368,25 @@ using TileStrided = Tile<12, 12, 13>;   // 4 x 4 x 4 positions: dilation, 64-bit
 using TileDeep = Tile<9, 10, 14>;       // 4 x 4 x 8 positions, 64-bit sums of 16-bit tensors
 using TileDeepStrided = Tile<8, 12, 13>;   // 2 x 4 x 4 positions, the same at stride 2
 template <typename S> constexpr bool kDeep = std::is_same<S, TileDeep>::value || std::is_same<S, TileDeepStrided>::value;
-using TileImage = Tile<1, 44, 44>;      // 32 x 32 positions, 32-bit sums; 16 x 16 positions whose taps are far apart, 64-bit sums
+using TileImage = Tile<1, 44, 44>;      // 32 x 32 positions, 32-bit sums; 16 x 16 positions whose taps are further apart
 using TileWide = Tile<1, 28, 44>;       // 16 x 32 positions (8 x 16 at stride 2), 64-bit sums
 using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions
+
+// Voxels along one axis that the undeformed taps of neighbouring positions reach
+static long dcn_reach(int positions, int stride, int taps, int dilation) {
+  return (positions - 1L) * stride + (taps - 1L) * dilation + 1;
+}
+// Dense layers: positions and taps close together along every axis, a rule of the layer whatever the tiles hold (tiles that grew by two voxels
+// took layers of stride (2, 1, 1), dilation (3, 1, 1) and 7 x 3 x 3 taps with them, whose 32-bit sums were 14 - 18 % off there).
+static bool dcn_dense(const DcnDims &s) {
+  if (s.nd == 2) return dcn_reach(32, s.sh, s.kh, s.dh) <= 42 && dcn_reach(32, s.sw, s.kw, s.dw) <= 42;
+  return dcn_reach(4, s.sd, s.kd, s.dd) <= 8 && dcn_reach(8, s.sh, s.kh, s.dh) <= 12 && dcn_reach(8, s.sw, s.kw, s.dw) <= 12;
+}
+// Among them, volumes that take bricks of 4 x 8 x 8 positions.  Those whose taps reach further have bricks of 4 x 4 x 4 (also where the
+// larger tile would hold them): two bits more for a term, and one maximum for a quarter of the positions.
+static bool dcn_dense_large(const DcnDims &s) {
+  return dcn_reach(4, s.sd, s.kd, s.dd) <= 6 && dcn_reach(8, s.sh, s.kh, s.dh) <= 10 && dcn_reach(8, s.sw, s.kw, s.dw) <= 10;
+}
 
 // The brick and its tile: the first of the list whose tile holds the reach of the brick's undeformed taps with two voxels to spare
 // on either side, or one, if none has two.  Images with fewer workgroups than compute units take a smaller brick (77 us ->
@@ -379,7 +395,8 @@ using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions
 // half the samples to work out, and 5.5 million requests of 64 bytes instead of 9.9 of 32 for [8, 256 -> 256, 100 x 152].  Where no
 // brick of images gives a workgroup to every compute unit, the one of most workgroups (fp32 [2, 128 -> 256, 36 x 18]: 48 of
 // 16 x 32 positions 131 us, 240 of 8 x 8 31 us).  Images whose taps are too far apart for those (3 x 3 taps from dilation 9 on) have
-// 16 x 16 positions in 44 x 44 of 8 channels, up to dilation 13 (backward pass at dilation 12, with every corner left to the tap kernel
+// 16 x 16 positions in 44 x 44 (with 64-bit sums of 8 channels), up to dilation 13, and so have dense ones where 32 x 32 leave fewer than
+// four voxels to spare (fp16 [2, 128 -> 128, 112 x 120] at dilation 5, backward pass: 302 us with 8 x 8 positions in 28 x 28, 233 us; backward pass at dilation 12, with every corner left to the tap kernel
 // and with the tile: fp16 [2, 64 -> 64, 64 x 64] 142 and 121 us, [2, 256 -> 256, 64 x 64] 305 and 264 us).  Volumes of 16-bit tensors with 64-bit sums have
 // smaller tiles of 16 channels too, where they leave three voxels to spare: bf16 [4, 32 -> 128, 57 x 51 x 27] at stride 2 472 us
 // with 12 x 12 x 13 of 8, 407 us with 8 x 12 x 13 of 16 (the tap kernel, which adds the corners beyond the smaller bricks' tiles,
@@ -391,26 +408,10 @@ using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions
 // layers alone (dcn_dense; 16-bit tensors, up to 128 output channels).  bf16 training
 // step of [2, 32 -> 64, 48^3]: 1178 us, 1393 us with 64-bit sums (with the kernel before this one).  Strided and wide layers have 64-bit sums, as good as fp32 ones:
 // where the output's gradient is 2^-14 of what it is elsewhere in the brick, 32 bits left them 2 - 20 % off.
-
-// Voxels along one axis that the undeformed taps of neighbouring positions reach
-static long dcn_reach(int positions, int stride, int taps, int dilation) {
-  return (positions - 1L) * stride + (taps - 1L) * dilation + 1;
-}
-// Dense layers: unit strides and taps close together, a rule of the layer whatever the tiles hold (tiles that grew by two voxels
-// took layers of stride (2, 1, 1), dilation (3, 1, 1) and 7 x 3 x 3 taps with them, whose 32-bit sums were 14 - 18 % off there).
-static bool dcn_dense(const DcnDims &s) {
-  if (s.nd == 2) return dcn_reach(32, s.sh, s.kh, s.dh) <= 42 && dcn_reach(32, s.sw, s.kw, s.dw) <= 42;
-  return dcn_reach(4, s.sd, s.kd, s.dd) <= 8 && dcn_reach(8, s.sh, s.kh, s.dh) <= 12 && dcn_reach(8, s.sw, s.kw, s.dw) <= 12;
-}
-// Among them, volumes that take bricks of 4 x 8 x 8 positions.  Those whose taps reach further have bricks of 4 x 4 x 4 (also where the
-// larger tile would hold them): two bits more for a term, and one maximum for a quarter of the positions.
-static bool dcn_dense_large(const DcnDims &s) {
-  return dcn_reach(4, s.sd, s.kd, s.dd) <= 6 && dcn_reach(8, s.sh, s.kh, s.dh) <= 10 && dcn_reach(8, s.sw, s.kw, s.dw) <= 10;
-}
 bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
   static const int volumes[2][6] = {{2, 3, 3, 12, 14, 14}, {2, 2, 2, 12, 12, 13}};
   static const int deep[2][6] = {{2, 2, 3, 9, 10, 14}, {1, 2, 2, 8, 12, 13}};
-  static const int dense_images[3][6] = {{0, 5, 5, 1, 44, 44}, {0, 4, 4, 1, 28, 28}, {0, 3, 3, 1, 28, 28}};
+  static const int dense_images[4][6] = {{0, 5, 5, 1, 44, 44}, {0, 4, 4, 1, 28, 28}, {0, 4, 4, 1, 44, 44}, {0, 3, 3, 1, 28, 28}};
   static const int images[4][6] = {{0, 4, 5, 1, 28, 44}, {0, 4, 4, 1, 28, 28}, {0, 3, 4, 1, 28, 44}, {0, 3, 3, 1, 28, 28}};
   static const int far_images[1][6] = {{0, 4, 4, 1, 44, 44}};
   const bool image = s.nd == 2;
@@ -446,7 +447,7 @@ bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
   if (s.Cin / 8 > 65535 || s.Q >= (1L << 28) || static_cast<long>(s.K) * s.cpg * s.opg * (dtype == MV_F32 ? 4 : 2) >= (1L << 31)) return false;
   bool fits = false;
   if (dtype != MV_F32 && s.opg <= 128 && dcn_dense(s)) {
-    fits = image ? choose(dense_images, 3, 16) : choose(dcn_dense_large(s) ? volumes : volumes + 1, 1, 16);
+    fits = image ? choose(dense_images, 4, 16) : choose(dcn_dense_large(s) ? volumes : volumes + 1, 1, 16);
     shape.narrow = fits && shape.terms <= kScatter32Terms;
   }
   if (!shape.narrow) {

@@ -66,3 +66,12 @@ def test_images_with_taps_far_apart_keep_their_tiles(code, cout, kernel, stride,
     spare = min(t - ((1 << b) - 1) * s - (k - 1) * d - 1
                 for t, b, s, k, d in zip((shape.th, shape.tw), (shape.bh, shape.bw), st, kn, dl))
     assert spare >= (4 if max(dl) <= 12 else 2)
+
+
+@pytest.mark.parametrize("cout", [64, 128])
+@pytest.mark.parametrize("kernel,dilation", [(3, 5), (11, 1), ((3, 5), (5, 2))])
+def test_dense_images_of_far_reach(cout, kernel, dilation):
+    """Where 32 x 32 positions leave fewer than four voxels to spare, 16 x 16 in the same tile, not 8 x 8 in a smaller one."""
+    for code in (_lib.MV_F16, _lib.MV_BF16):
+        shape = _plan(code, 2, 128, cout, (112, 208), kernel, 1, dilation)
+        assert (shape.narrow, shape.bh, shape.bw, shape.th, shape.tw) == (1, 4, 4, 44, 44)
