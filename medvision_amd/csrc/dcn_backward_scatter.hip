@@ -369,8 +369,11 @@ using TileDeep = Tile<9, 10, 14>;       // 4 x 4 x 8 positions, 64-bit sums of 1
 using TileDeepStrided = Tile<8, 12, 13>;   // 2 x 4 x 4 positions, the same at stride 2
 template <typename S> constexpr bool kDeep = std::is_same<S, TileDeep>::value || std::is_same<S, TileDeepStrided>::value;
 using TileImage = Tile<1, 44, 44>;      // 32 x 32 positions, 32-bit sums; 16 x 16 positions whose taps are further apart
-using TileWide = Tile<1, 28, 44>;       // 16 x 32 positions (8 x 16 at stride 2), 64-bit sums
+using TileWide = Tile<1, 28, 44>;       // 16 x 32 positions (8 x 16 at stride 2), 64-bit sums of 16-bit tensors
 using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions
+struct TileSmallF32 : TileSmall {         // the same for fp32: two workgroups of 8 channels on a compute unit
+  template <bool NARROW> static constexpr int channels = 8;
+};
 
 // Voxels along one axis that the undeformed taps of neighbouring positions reach
 static long dcn_reach(int positions, int stride, int taps, int dilation) {
@@ -391,18 +394,25 @@ static bool dcn_dense_large(const DcnDims &s) {
 // The brick and its tile: the first of the list whose tile holds the reach of the brick's undeformed taps with two voxels to spare
 // on either side, or one, if none has two.  Images with fewer workgroups than compute units take a smaller brick (77 us ->
 // 35 us for [1, 256 -> 128, 27 x 58]); volumes do not (the halo of 4 x 4 x 4 positions is most of their tile: 117 us
-// against 78 us for [2, 16 -> 128, 7 x 19 x 32]).  Images with 64-bit sums have smaller tiles of 16 channels instead of 44 x 44 of 8:
-// half the samples to work out, and 5.5 million requests of 64 bytes instead of 9.9 of 32 for [8, 256 -> 256, 100 x 152].  Where no
-// brick of images gives a workgroup to every compute unit, the one of most workgroups (fp32 [2, 128 -> 256, 36 x 18]: 48 of
-// 16 x 32 positions 131 us, 240 of 8 x 8 31 us).  Images whose taps are too far apart for those (3 x 3 taps from dilation 9 on) have
-// 16 x 16 positions in 44 x 44 (with 64-bit sums of 8 channels), up to dilation 13, and so have dense ones where 32 x 32 leave fewer than
-// four voxels to spare (fp16 [2, 128 -> 128, 112 x 120] at dilation 5, backward pass: 302 us with 8 x 8 positions in 28 x 28, 233 us; backward pass at dilation 12, with every corner left to the tap kernel
-// and with the tile: fp16 [2, 64 -> 64, 64 x 64] 142 and 121 us, [2, 256 -> 256, 64 x 64] 305 and 264 us).  Volumes of 16-bit tensors with 64-bit sums have
-// smaller tiles of 16 channels too, where they leave three voxels to spare: bf16 [4, 32 -> 128, 57 x 51 x 27] at stride 2 472 us
-// with 12 x 12 x 13 of 8, 407 us with 8 x 12 x 13 of 16 (the tap kernel, which adds the corners beyond the smaller bricks' tiles,
-// 236 -> 275 us).  fp32 ones would gain more ([4, 16 -> 16, 17 x 43 x 30] 343 us, 244 us with 9 x 10 x 14 of 16), but every
-// addition to memory rounds: their gradient would be 1.5e-7 (rms) off instead of 1.3e-7.  With 32-bit sums, where 16 channels fit
-// the larger tile, smaller ones only cost more halo (30 layers of fewer than 256 workgroups: 2 % slower).  False: no brick fits.
+// against 78 us for [2, 16 -> 128, 7 x 19 x 32]).  False: no brick fits.
+//
+// 16-bit images with 64-bit sums have smaller tiles of 16 channels instead of 44 x 44 of 8: half the samples to work out, and
+// 5.5 million requests of 64 bytes instead of 9.9 of 32 for [8, 256 -> 256, 100 x 152].  Where no brick of 16-bit images gives a
+// workgroup to every compute unit, the one of most workgroups.  Taps too far apart for those tiles (3 x 3 taps from dilation 9 on)
+// have 16 x 16 positions in 44 x 44 of 8 channels, up to dilation 13 (backward pass at dilation 12, every corner left to the tap kernel
+// and with this tile: fp16 [2, 64 -> 64, 64 x 64] 142 and 121 us, [2, 256 -> 256, 64 x 64] 305 and 264 us); so have dense images,
+// with 16 channels, where 32 x 32 positions leave fewer than four voxels to spare (fp16 [2, 128 -> 128, 112 x 120] at dilation 5: 302 us
+// with 8 x 8 positions in 28 x 28, 233 us).
+//
+// Tensors of fp32 keep the largest bricks: every addition of a tile's sums to memory rounds.  Images, with the lists of 16-bit ones
+// ([1, 64 -> 64, 24 x 24] in 8 x 8 positions, not 32 x 32): gradient 1.56e-7 (rms) off instead of 1.53e-7, backward pass 100 instead
+// of 125 us, [2, 128 -> 128, 112 x 208] 658 instead of 730 us.  Volumes ([4, 16 -> 16, 17 x 43 x 30] with 9 x 10 x 14 of 16 channels): 1.5e-7
+// instead of 1.3e-7, 244 instead of 343 us.
+//
+// Volumes of 16-bit tensors with 64-bit sums have smaller tiles of 16 channels too, where they leave three voxels to spare:
+// bf16 [4, 32 -> 128, 57 x 51 x 27] at stride 2 472 us with 12 x 12 x 13 of 8, 407 us with 8 x 12 x 13 of 16 (the tap kernel, which
+// adds the corners beyond the smaller bricks' tiles, 236 -> 275 us).  With 32-bit sums, where 16 channels fit the larger tile, smaller ones
+// only cost more halo (30 layers of fewer than 256 workgroups: 2 % slower).
 //
 // Width of the sums: 32 bits round every term to 14 - 22 bits of the workgroup's largest, which is worth their speed in dense
 // layers alone (dcn_dense; 16-bit tensors, up to 128 output channels).  bf16 training
@@ -411,7 +421,7 @@ static bool dcn_dense_large(const DcnDims &s) {
 bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
   static const int volumes[2][6] = {{2, 3, 3, 12, 14, 14}, {2, 2, 2, 12, 12, 13}};
   static const int deep[2][6] = {{2, 2, 3, 9, 10, 14}, {1, 2, 2, 8, 12, 13}};
-  static const int dense_images[4][6] = {{0, 5, 5, 1, 44, 44}, {0, 4, 4, 1, 28, 28}, {0, 4, 4, 1, 44, 44}, {0, 3, 3, 1, 28, 28}};
+  static const int large_images[4][6] = {{0, 5, 5, 1, 44, 44}, {0, 4, 4, 1, 28, 28}, {0, 4, 4, 1, 44, 44}, {0, 3, 3, 1, 28, 28}};
   static const int images[4][6] = {{0, 4, 5, 1, 28, 44}, {0, 4, 4, 1, 28, 28}, {0, 3, 4, 1, 28, 44}, {0, 3, 3, 1, 28, 28}};
   static const int far_images[1][6] = {{0, 4, 4, 1, 44, 44}};
   const bool image = s.nd == 2;
@@ -436,7 +446,7 @@ bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
       const long spare = spare_of(e);
       if (spare < 2) continue;
       const int rank = (spare >= 4 ? 2 : 0) + (image && workgroups(e, channels) >= 256 ? 1 : 0);
-      if (rank < best || (rank == best && !(image && workgroups(taken, channels) < 256))) continue;
+      if (rank < best || (rank == best && !(image && dtype != MV_F32 && workgroups(taken, channels) < 256))) continue;
       best = rank;
       taken = e;
       shape = ScatterShape{e[0], e[1], e[2], e[3], e[4], e[5], 0, 0, 0, (1 << (e[0] + e[1] + e[2])) * s.K, 0, 1};
@@ -447,12 +457,12 @@ bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
   if (s.Cin / 8 > 65535 || s.Q >= (1L << 28) || static_cast<long>(s.K) * s.cpg * s.opg * (dtype == MV_F32 ? 4 : 2) >= (1L << 31)) return false;
   bool fits = false;
   if (dtype != MV_F32 && s.opg <= 128 && dcn_dense(s)) {
-    fits = image ? choose(dense_images, 4, 16) : choose(dcn_dense_large(s) ? volumes : volumes + 1, 1, 16);
+    fits = image ? choose(large_images, 4, 16) : choose(dcn_dense_large(s) ? volumes : volumes + 1, 1, 16);
     shape.narrow = fits && shape.terms <= kScatter32Terms;
   }
   if (!shape.narrow) {
     const int (*const small)[6] = image || dtype == MV_F32 ? nullptr : spare_of(deep[0]) >= 3 ? deep : spare_of(deep[1]) >= 3 ? deep + 1 : nullptr;
-    fits = image ? choose(images, 4, 16) : small ? choose(small, 1, 16) : choose(volumes, 2, 8);
+    fits = image ? (dtype == MV_F32 ? choose(large_images, 4, 8) : choose(images, 4, 16)) : small ? choose(small, 1, 16) : choose(volumes, 2, 8);
     const int taken[6] = {shape.bd, shape.bh, shape.bw, shape.td, shape.th, shape.tw};
     if (image && (!fits || spare_of(taken) < 4) && spare_of(far_images[0]) >= (fits ? 4 : 2)) fits = choose(far_images, 1, 8);
   }
@@ -481,7 +491,7 @@ static int scatter_launch(const void *off, const void *mask, const void *gyt, co
     if constexpr (sizeof(T) == 2 && !kDeep<S> && !S::WIDE) {   // (those have 64-bit sums)
       if (slices <= 2) MV_SCATTER(true, 2); else MV_SCATTER(true, 4);
     }
-  } else if constexpr (!(kDeep<S> && sizeof(T) == 4)) {   // (never of those)
+  } else if constexpr (!((kDeep<S> || S::WIDE) && sizeof(T) == 4)) {   // (never of those)
     if (slices <= 2) MV_SCATTER(false, 2);
     else if (slices <= 4) MV_SCATTER(false, 4);
     else MV_SCATTER(false, 8);
@@ -499,7 +509,8 @@ int dcn_scatter(const void *off, const void *mask, const void *gyt, const void *
    : shape.th == TileVolume::TH ? MV_SCATTER_TILE(T, TileVolume)                                                          \
    : shape.th == TileStrided::TH ? MV_SCATTER_TILE(T, TileStrided)                                                      \
    : shape.th == TileImage::TH ? MV_SCATTER_TILE(T, TileImage)                                                        \
-   : shape.tw == TileWide::TW ? MV_SCATTER_TILE(T, TileWide) : MV_SCATTER_TILE(T, TileSmall))
+   : shape.tw == TileWide::TW ? MV_SCATTER_TILE(T, TileWide)                                                            \
+                              : scatter_launch<T, std::conditional<sizeof(T) == 4, TileSmallF32, TileSmall>::type>(off, mask, gyt, wf, gxt, s, shape, bounds, stream))
   if (dtype == MV_F16) return MV_SCATTER_AS(__half);
   if (dtype == MV_F32) return MV_SCATTER_AS(float);
   return MV_SCATTER_AS(__hip_bfloat16);

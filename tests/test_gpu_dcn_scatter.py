@@ -108,3 +108,23 @@ def test_small_gradients_beside_large_ones_along_one_axis(oracle, dtype, kernel,
     assert float(want.abs().max()) < 1.0       # nothing of the large ones
     error = float((got - want).norm() / want.norm())
     assert error < (2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8), error
+
+
+@pytest.mark.parametrize("cin,cout,size,stride", [(64, 64, (24, 24), 1), (32, 288, (31, 20), 1), (64, 32, (32, 30), 2)])
+def test_fp32_images_of_one_brick_are_rounded_once(oracle, cin, cout, size, stride):
+    """Every addition of a tile's sums to the fp32 gradient rounds, so that fp32 images have bricks as large as the tiles hold while
+    no brick fills the chip.  Whole weights and gradients and offsets in eighths: the terms and their 64-bit sums are exact, and an
+    image of one brick is off by one rounding, 2^-24 of each value."""
+    from medvision_amd.ops.modulated_deform_conv_2d import modulated_deform_conv
+    g = wl.gen(cin + cout)
+    x, off, mask, w, b = wl.dcn_inputs(g, 2, cin, cout, size, 3, 1, 1, torch.float32, stride, 1, 1)
+    off = torch.randint(-24, 25, off.shape, generator=g) / 8.0
+    w = torch.randint(-127, 128, w.shape, generator=g).float()
+    leaves = [t.to(DEV).requires_grad_(True) for t in (x, off, torch.ones_like(mask), w, b)]
+    y = modulated_deform_conv(*leaves, stride, 1, 1, 1, 1)
+    gy = torch.randint(-2047, 2048, y.shape, generator=g).float()
+    y.backward(gy.to(DEV))
+    want = oracle.dcn3d_backward(x, off, torch.ones_like(mask), w, gy, True, stride, 1, 1, 1, 1)[0].reshape(x.shape)
+    error = (leaves[0].grad.cpu().double() - want).abs()
+    worst = float((error / want.abs().clamp(min=1e-9)).max())
+    assert worst <= 2.0 ** -24, worst * 2.0 ** 24
