@@ -90,4 +90,9 @@ __device__ __forceinline__ unsigned xcd_contiguous(unsigned id, unsigned count) 
   return id < per_xcd * 8 ? (id % 8) * per_xcd + id / 8 : id;
 }
 
+// Grids of very many workgroups: a dimension of a grid has fewer than 2^32 threads, so that beyond it the workgroups stand in
+// rows.  The last row may be longer than needed: kernels leave where linear_block() is not below the number of workgroups.
+dim3 linear_grid(long workgroups, int threads);
+__device__ __forceinline__ unsigned linear_block() { return blockIdx.y * gridDim.x + blockIdx.x; }
+
 }  // namespace mv

@@ -1,4 +1,4 @@
-// Error reporting and library identity.
+// Error reporting, library identity, launch grids.
 #include "common.hpp"
 
 namespace mv {
@@ -14,6 +14,11 @@ int fail(int status, const char *fmt, ...) {
   vsnprintf(last_error_buffer(), 512, fmt, ap);
   va_end(ap);
   return status;
+}
+
+dim3 linear_grid(long workgroups, int threads) {
+  const long row = ((1L << 32) - 1) / threads, rows = (workgroups + row - 1) / row;
+  return dim3(static_cast<unsigned>((workgroups + rows - 1) / rows), static_cast<unsigned>(rows));
 }
 
 }  // namespace mv

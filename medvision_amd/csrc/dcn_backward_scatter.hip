@@ -113,7 +113,9 @@ __global__ __launch_bounds__(KEEP <= 4 ? 1024 : 512) void dcn_backward_scatter_k
   const int n = p16 / 4 % 2 * 16 + 4 * j + p16 % 4, half = p16 / 8;
   // (the channel blocks of a brick next to each other on one XCD: they read the same grad_output and offsets)
   const int turns = CH == 16 && KEEP == 8 ? shape.turns : 1;   // blocks of CH channels, one after the other
-  const unsigned id = xcd_contiguous(blockIdx.x, gridDim.x), shares_of_brick = s.Cin / (CH * turns), brick = id / shares_of_brick;
+  const unsigned shares_of_brick = s.Cin / (CH * turns), workgroups = shape.nbd * shape.nbh * shape.nbw * s.B * shares_of_brick;
+  if (linear_block() >= workgroups) return;
+  const unsigned id = xcd_contiguous(linear_block(), workgroups), brick = id / shares_of_brick;
   int c0 = static_cast<int>(id % shares_of_brick) * (CH * turns);
   const int bx = brick % shape.nbw, by = brick / shape.nbw % shape.nbh, bz = brick / (shape.nbw * shape.nbh) % shape.nbd,
             b = brick / (shape.nbw * shape.nbh * shape.nbd);
@@ -482,8 +484,9 @@ static int scatter_launch(const void *off, const void *mask, const void *gyt, co
   const int slices = s.opg / (64 / static_cast<int>(sizeof(T)));
 #define MV_SCATTER(NARROWV, KEEPV)                                                                                    \
   hipLaunchKernelGGL((dcn_backward_scatter_kernel<T, NARROWV, S, KEEPV>),                                              \
-                     dim3(static_cast<unsigned>(shape.nbd) * shape.nbh * shape.nbw * s.B *                              \
-                          (s.Cin / (S::template channels<NARROWV> * (KEEPV == 8 && S::template channels<NARROWV> == 16 ? shape.turns : 1)))), \
+                     linear_grid(static_cast<long>(shape.nbd) * shape.nbh * shape.nbw * s.B *                           \
+                                     (s.Cin / (S::template channels<NARROWV> * (KEEPV == 8 && S::template channels<NARROWV> == 16 ? shape.turns : 1))), \
+                                 KEEPV <= 4 ? 1024 : 512),                                                              \
                      dim3(KEEPV <= 4 ? 1024 : 512), 0, stream,                                                         \
                      static_cast<const T *>(off), static_cast<const T *>(mask), static_cast<const T *>(gyt),          \
                      static_cast<const T *>(wf), gxt, s, shape, bounds)

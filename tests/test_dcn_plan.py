@@ -75,3 +75,30 @@ def test_dense_images_of_far_reach(cout, kernel, dilation):
     for code in (_lib.MV_F16, _lib.MV_BF16):
         shape = _plan(code, 2, 128, cout, (112, 208), kernel, 1, dilation)
         assert (shape.narrow, shape.bh, shape.bw, shape.th, shape.tw) == (1, 4, 4, 44, 44)
+
+
+class _Dim3(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_uint32) for n in "xyz"]
+
+
+def _grid(workgroups, threads):
+    fn = _lib.load()._ZN2mv11linear_gridEli
+    fn.restype, fn.argtypes = _Dim3, [ctypes.c_long, ctypes.c_int]
+    return fn(workgroups, threads)
+
+
+@pytest.mark.parametrize("threads", [256, 512, 1024])
+@pytest.mark.parametrize("workgroups", [1, 255, (1 << 22) - 1, 1 << 22, (1 << 22) + 1, 4239360, (1 << 24) - 1, 1 << 24, 19462005, (1 << 31) - 1])
+def test_grids_of_many_workgroups(workgroups, threads):
+    """A dimension of a grid has fewer than 2^32 threads: one row as long as that holds, then rows that leave no whole row idle."""
+    g = _grid(workgroups, threads)
+    assert g.x * threads < 1 << 32 and g.y <= 65535 and g.z == 1
+    assert g.x * g.y >= workgroups > g.x * (g.y - 1)
+    assert g.y == 1 or workgroups * threads >= 1 << 32
+
+
+def test_a_volume_of_more_workgroups_than_a_row():
+    """fp32 [16, 32 -> 32, 128 x 180 x 182] at dilation 2 has 4 239 360 workgroups of 1024 threads: the plan takes it."""
+    shape = _plan(_lib.MV_F32, 16, 32, 32, (128, 180, 182), 3, 1, 2)
+    assert shape.nbd * shape.nbh * shape.nbw * 16 * (32 // 8) == 4239360
+    assert _grid(4239360, 1024).y == 2
