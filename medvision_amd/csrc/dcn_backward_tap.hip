@@ -84,7 +84,7 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
     const T *__restrict__ xt, const T *__restrict__ off, const T *__restrict__ mask, const T *__restrict__ gyt,
     const T *__restrict__ wf, float *__restrict__ gxt, T *__restrict__ goff, T *__restrict__ gmask,
     float *__restrict__ partial, float *__restrict__ gw, const DcnDims s, const unsigned *__restrict__ bounds,
-    const ScatterShape shape, const int chunks, const int shares, const int range, const int row0, const TapPiece piece) {
+    const ScatterShape shape, const int chunks, const int shares, const int range, const unsigned ranges, const int row0, const TapPiece piece) {
   using M = Mfma<T>;
   using P = typename std::conditional<(sizeof(T) == 2), float, double>::type;  // position type
   constexpr int PC = M::kPiece, SL = 4 * PC, ES = sizeof(T), CW = 16 * CBW, ROWS = 64 * OBW;
@@ -101,7 +101,9 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
   const int j = lane % 16, kc = lane / 16;   // matrix layout
   const int lj = lane / 4, lk = lane % 4;    // load layout
   // (taps and chunks of one range next to each other, on one XCD: they gather the same part of x and read the same gy)
-  const unsigned wg = xcd_contiguous(blockIdx.x, gridDim.x), inner = piece.taps * s.dg * chunks, ranges = gridDim.x / (inner * s.B);
+  const unsigned inner = piece.taps * s.dg * chunks, workgroups = ranges * inner * s.B;
+  if (linear_block() >= workgroups) return;
+  const unsigned wg = xcd_contiguous(linear_block(), workgroups);
   const int k = piece.k_first + static_cast<int>(wg % piece.taps), slice = static_cast<int>(wg / piece.taps % (s.dg * chunks));
   const int dgi = slice / chunks, part = slice % chunks, b = static_cast<int>(wg / inner / ranges);
   const int c0 = dgi * s.cpd + part * CW, g = c0 / s.cpg;
@@ -459,11 +461,11 @@ static int tap_launch(const T *xt, const T *off, const T *mask, const T *gyt, co
   const long ranges = sizeof(T) == 4 ? (tiles + few - 1) / few : tap_ranges(tiles, others, slots, static_cast<long>(rows) * (16 * CBW));
   const long per = (tiles + ranges - 1) / ranges;
   MV_REQUIRE(static_cast<double>(ranges) * others < static_cast<double>(1L << 31), "grid too large");
-  const dim3 grid(static_cast<unsigned>(ranges * others));
+  const dim3 grid = linear_grid(ranges * others, 256);
   const int range = static_cast<int>(per * kTapTile);
 #define MV_TAP(OBWV, ROW)                                                                                               \
   hipLaunchKernelGGL((dcn_backward_tap_kernel<T, NC, OBWV, CBW>), grid, dim3(256), 0, stream, xt, off, mask, gyt, wf, gxt,     \
-                     goff, gmask, partial, gw, s, bounds, shape, chunks, shares, range, ROW, piece)
+                     goff, gmask, partial, gw, s, bounds, shape, chunks, shares, range, static_cast<unsigned>(ranges), ROW, piece)
   if (s.opg <= 64) {
     MV_TAP(1, 0);
   } else if (s.opg <= 128 || sizeof(T) == 4) {
