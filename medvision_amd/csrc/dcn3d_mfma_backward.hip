@@ -249,19 +249,22 @@ static int gy_rows_per_wave(const DcnDims &s) {   // 0: slabs
   const long rows = gy_rows(s);
   return rows < 1024 ? 0 : static_cast<int>((rows + 2047) / 2048);
 }
-// sum and largest magnitude of src[q0 .. q_end), `threads` threads, PIECES independent 16-byte loads each
+// sum and largest magnitude of src[q0 .. q_end), `threads` threads, PIECES independent 16-byte loads each, which have a sum each: an
+// addition of a chain rounds by as much as the chain has grown (fp32, 8 rows of 15 200 positions and 64 threads: the bias gradient is
+// off by 3.1e-7 (rms) with one sum per thread, 1.3e-7 with eight)
 template <typename T, int PIECES>
-__device__ __forceinline__ void gy_sum_max(const T *__restrict__ src, long q0, const long q_end, const int thread, const int threads,
-                                           float &v, float &m, bool &bad) {
+__device__ __forceinline__ float gy_sum_max(const T *__restrict__ src, const long q0, const long q_end, const int thread, const int threads,
+                                            float &m, bool &bad) {
   constexpr int V = 16 / static_cast<int>(sizeof(T));
-  auto take = [&](T e) {
+  float sum[PIECES] = {};
+  auto take = [&](T e, float &v) {
     const float x = static_cast<float>(load(&e));
     v += x;
     bad = bad || !(x == x);
     m = fmaxf(m, fabsf(x));
   };
   typedef unsigned int piece_t __attribute__((ext_vector_type(4), aligned(2)));   // (element alignment: the hardware takes it)
-  const long groups = (q_end - q0) / V;
+  const long groups = (q_end - q0) / V, rest = q0 + groups * V;
   const piece_t *pieces = reinterpret_cast<const piece_t *>(src + q0);
   for (long i = thread; i < groups; i += PIECES * threads) {
     union { u32x4 u; T e[V]; } raw[PIECES];
@@ -270,23 +273,26 @@ __device__ __forceinline__ void gy_sum_max(const T *__restrict__ src, long q0, c
 #pragma unroll
     for (int u = 0; u < PIECES; u++)
 #pragma unroll
-      for (int e = 0; e < V; e++) take(raw[u].e[e]);
+      for (int e = 0; e < V; e++) take(raw[u].e[e], sum[u]);
   }
-  q0 += groups * V;
-  for (long q = q0 + thread; q < q_end; q += threads) take(src[q]);
+  if (rest + thread < q_end) take(src[rest + thread], sum[0]);   // (fewer than V elements)
+#pragma unroll
+  for (int half = PIECES / 2; half > 0; half /= 2)
+#pragma unroll
+    for (int u = 0; u < half; u++) sum[u] += sum[u + half];
+  return sum[0];
 }
 template <typename T>
 __device__ __forceinline__ void dcn_gy_sum_max_block(const T *__restrict__ gy, float *__restrict__ gb32, unsigned *out,
                                                      const DcnDims s, const long slab_len, const int rows, const unsigned bid) {
   __shared__ float sums[4];
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  float v = 0.f, m = 0.f;
+  float m = 0.f;
   bool bad = false;
   const long total = static_cast<long>(s.Cout) * s.B;
   if (rows > 0) {
     for (long r = (bid * 4L + wave) * rows, last = min(r + rows, total); r < last; r++) {   // (rows are [b][o])
-      v = 0.f;
-      gy_sum_max<T, 8>(gy + r * s.Q, 0, s.Q, lane, kWave, v, m, bad);
+      float v = gy_sum_max<T, 8>(gy + r * s.Q, 0, s.Q, lane, kWave, m, bad);
       for (int sh = 32; sh > 0; sh >>= 1) v += __shfl_xor(v, sh);
       if (lane == 0) atomicAdd(gb32 + r % s.Cout, v);
     }
@@ -297,7 +303,7 @@ __device__ __forceinline__ void dcn_gy_sum_max_block(const T *__restrict__ gy, f
   const unsigned slab = bid % slabs, r = bid / slabs;
   const int b = static_cast<int>(r % s.B), o = static_cast<int>(r / s.B);
   const long q0 = static_cast<long>(slab) * slab_len;
-  gy_sum_max<T, 4>(gy + (static_cast<long>(b) * s.Cout + o) * s.Q, q0, min(q0 + slab_len, s.Q), threadIdx.x, 256, v, m, bad);
+  float v = gy_sum_max<T, 4>(gy + (static_cast<long>(b) * s.Cout + o) * s.Q, q0, min(q0 + slab_len, s.Q), threadIdx.x, 256, m, bad);
   for (int sh = 32; sh > 0; sh >>= 1) v += __shfl_xor(v, sh);
   if (lane == 0) sums[wave] = v;
   if (out) fold_max(bad ? 0x7fc00000u : __float_as_uint(m), out);   // (contains the barrier)

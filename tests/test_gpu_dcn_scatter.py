@@ -128,3 +128,21 @@ def test_fp32_images_of_one_brick_are_rounded_once(oracle, cin, cout, size, stri
     error = (leaves[0].grad.cpu().double() - want).abs()
     worst = float((error / want.abs().clamp(min=1e-9)).max())
     assert worst <= 2.0 ** -24, worst * 2.0 ** 24
+
+
+@pytest.mark.parametrize("size", [(120, 127), (101, 151)])      # rows at whole pieces of 16 bytes, rows at any element
+@pytest.mark.parametrize("batch,cout", [(8, 128), (2, 64)])     # 1024 rows, a wavefront each; slabs of rows
+def test_fp32_bias_of_long_rows(batch, cout, size):
+    """The bias gradient of fp32 layers is a sum in fp32, in chains of at most a 512th of a row.  A chain of n normal values rounds n times
+    at 0.4 * 2^-24 of the sum so far (rms), sqrt(n / 2) * 0.4 * 2^-24 of its result: 1e-7 of the sum of all chains for n = 30; the tree and
+    the atomics above add as much.  (Chains of a 64th of a row: 3e-7.)"""
+    from medvision_amd import _C
+    g = torch.Generator(DEV).manual_seed(sum(size))
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    ins = x, w, b, off, mask = rand(batch, 32, *size), rand(cout, 32, 1, 1), rand(cout), rand(batch, 2, *size), rand(batch, 1, *size)
+    gy, sums = rand(batch, cout, *size), [torch.zeros_like(t) for t in ins]
+    gx, gw, gb, goff, gmask = sums
+    _C.modulated_deform_conv_2d_backward(x, w, b, None, off, mask, None, gx, gw, gb, goff, gmask, gy, 1, 1, 1, 1, 0, 0, 1, 1, 1, 1, True)
+    want = gy.double().sum((0, 2, 3))
+    error = float((gb.double() - want).norm() / want.norm())
+    assert error < 2e-7, error
