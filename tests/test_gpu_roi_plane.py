@@ -86,3 +86,36 @@ def test_plane_heads_non_finite(oracle, dtype, size, channels, rois, cells, rati
 
     marks = (~torch.isfinite(gy)).to(dtype)
     compare(x.grad, spread(torch.where(marks > 0, 0.0, gy)), spread(marks) == 0, BWD_TOL[dtype], "backward")
+
+
+@pytest.mark.parametrize("dtype,exponents,normal", [(torch.float16, (-24, -15), -14), (torch.bfloat16, (-133, -126), -126)])
+@pytest.mark.parametrize("cells", [(7, 7), (14, 14)])
+def test_plane_heads_denormal_values(oracle, dtype, exponents, normal, cells):
+    """16-bit pixels and gradients go to the matrix cores as they are: values below the type's normal ones keep their bits.  Results are
+    off by half a unit in the last place (the smallest denormal's below 2^normal), and by 2^-16 of the terms' sum for weights whose
+    sample lies next to a decision of the sampler."""
+    from medvision_amd.ops.roi_align_nd import roi_align_2d
+    g = wl.gen(sum(cells))
+    rois, channels, size = 60, 34, (60, 70)
+    at = torch.rand(rois, 2, generator=g) * torch.tensor(size[::-1]) * 0.9
+    boxes = torch.cat([torch.randint(0, 2, (rois, 1), generator=g).float(), at, at + torch.rand(rois, 2, generator=g) * 30 + 1], 1)
+
+    def values(*shape):
+        e = exponents[0] + (exponents[1] - exponents[0]) * torch.rand(*shape, generator=g, dtype=torch.float64)
+        return (torch.exp2(e) * (torch.randint(0, 2, shape, generator=g) * 2 - 1)).to(dtype)
+
+    feat = values(2, channels, *size)
+    x = feat.to(DEV).requires_grad_()
+    out = roi_align_2d(x, boxes.to(DEV), cells, 1.0, 2, 1)
+    gy = values(*out.shape)
+    out.backward(gy.to(DEV))
+    half = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+
+    def check(got, of, name):
+        want, terms = of(False), of(True)
+        error = (got.detach().cpu().double() - want.reshape(got.shape)).abs().reshape(-1)
+        bound = half * want.abs().clamp(min=2.0 ** normal).reshape(-1) + 2.0 ** -16 * terms.reshape(-1)
+        assert float(want.abs().max()) > 0 and float((error / bound).max()) <= 1.0, name
+
+    check(out, lambda a: oracle.roi_align_forward(feat.abs() if a else feat, boxes, cells, 1.0, 2, True, 1, False), "forward")
+    check(x.grad, lambda a: oracle.roi_align_backward(gy.abs() if a else gy, boxes, feat.shape, 1.0, 2, True, 1, False), "backward")
