@@ -9,20 +9,21 @@
 // broadcasts, which the multiplications take as an operand, and an LDS addition meets four (eight) cells of 64 contiguous bytes.
 // Per term: multiply, convert, add.  Corners outside the tile or the volume have weight 0 in a cell that exists: no branches.
 //   (Channels as rows, a lane holding one position and four channels, needed the samples' words from LDS, a branch per corner
-//   and additions to 16 places: bf16 [2, 32 -> 64, 48^3] 496 us, then 338 us (351 us with today's larger tile); fp16 [8, 256 -> 256, 100 x 152] 1185 us, now 500 us.)
+//   and additions to 16 places: bf16 [2, 32 -> 64, 48^3] 496 us, then 338 us (348 us with today's larger tile); fp16 [8, 256 -> 256, 100 x 152] 1185 us, now 510 us.)
 // Afterwards the tile's non-zero sums are added to the gradient buffer, one global atomic per (voxel, channel) of the tile
 // instead of one per (position, tap, corner, channel).
 //
 // NARROW (dense layers of 16-bit tensors, see dcn_scatter_plan): 32-bit sums.  They leave 31 - log2(positions * taps) bits for
 // a term (18 for 3 x 3 x 3 taps), so the scale comes from the data: a first sweep over the brick's taps forms gcol alone (matrix
 // cores, no geometry; 17 us) and takes max |gcol| of the workgroup; every term is then below max |gcol| * max |mask| <
-// 2^ex and is rounded to a multiple of 2^(ex - shift).  The error of a voxel's sum stays below terms * 2^(ex - shift - 1), about
-// 2^-16 of the values it sums for the 3 x 3 x 3 layer — a thirty-second of the last bit of a bf16 result.  Otherwise a 64-bit word
+// 2^ex and is rounded to a multiple of 2^(ex - shift).  The error of a voxel's sum stays below terms * 2^(ex - shift - 1), whatever its own
+// size: 1.3 % of the workgroup's largest term for 3 x 3 x 3 taps if all roundings agreed.  With gradients of even size it is far less
+// (fp16 [2, 32 -> 64, 48^3], sigma = 2: 2.18e-4 rms of the gradient, of which rounding the result is 2.07e-4).  Otherwise a 64-bit word
 // per channel, scale from the global maxima.
 //
 // What bounds it: the LDS additions (64 lanes of 32 bits in 4 clocks, of 64 bits in 6, whatever the cells) behind phases that leave
 // the LDS idle, since a tile fills the compute unit: the first group's inputs, the sweep, the tile's atomics (40 us).  Busy: bf16
-// [2, 32 -> 64, 48^3] vector issue 52 %, LDS 40 %; fp16 [8, 256 -> 256, 100 x 152] 45 %, 26 %, texture addressers 39 %.
+// [2, 32 -> 64, 48^3] vector issue 51 %, LDS 40 %; fp16 [8, 256 -> 256, 100 x 152] 46 %, 28 %, texture addressers 37 %.
 #include "dcn_scatter.hpp"
 
 namespace mv {
@@ -400,7 +401,8 @@ static bool dcn_dense_large(const DcnDims &s) {
 //
 // 16-bit images with 64-bit sums have smaller tiles of 16 channels instead of 44 x 44 of 8: half the samples to work out, and
 // 5.5 million requests of 64 bytes instead of 9.9 of 32 for [8, 256 -> 256, 100 x 152].  Where no brick of 16-bit images gives a
-// workgroup to every compute unit, the one of most workgroups.  Taps too far apart for those tiles (3 x 3 taps from dilation 9 on)
+// workgroup to every compute unit, the one of most workgroups (backward passes of fp16 [2, 128 -> 256, 36 x 18] 150 -> 112 us,
+// [1, 64 -> 64, 24 x 24] 109 -> 72 us, [1, 256 -> 128, 27 x 58] 124 -> 109 us).  Taps too far apart for those tiles (3 x 3 taps from dilation 9 on)
 // have 16 x 16 positions in 44 x 44 of 8 channels, up to dilation 13 (backward pass at dilation 12, every corner left to the tap kernel
 // and with this tile: fp16 [2, 64 -> 64, 64 x 64] 142 and 121 us, [2, 256 -> 256, 64 x 64] 305 and 264 us); so have dense images,
 // with 16 channels, where 32 x 32 positions leave fewer than four voxels to spare (fp16 [2, 128 -> 128, 112 x 120] at dilation 5: 302 us
@@ -417,9 +419,10 @@ static bool dcn_dense_large(const DcnDims &s) {
 // only cost more halo (30 layers of fewer than 256 workgroups: 2 % slower).
 //
 // Width of the sums: 32 bits round every term to 14 - 22 bits of the workgroup's largest, which is worth their speed in dense
-// layers alone (dcn_dense; 16-bit tensors, up to 128 output channels).  bf16 training
-// step of [2, 32 -> 64, 48^3]: 1178 us, 1393 us with 64-bit sums (with the kernel before this one).  Strided and wide layers have 64-bit sums, as good as fp32 ones:
-// where the output's gradient is 2^-14 of what it is elsewhere in the brick, 32 bits left them 2 - 20 % off.
+// layers alone (dcn_dense; 16-bit tensors, up to 128 output channels).  Backward passes with 32 and with 64 bits: bf16 volumes
+// [2, 32 -> 64, 48^3] 838 and 1140 us, [2, 64 -> 64, 24 x 32 x 32] 436 and 553 us; fp16 images [2, 64 -> 128, 100 x 152] 173 - 189 and
+// 183 - 187 us, [2, 128 -> 128, 112 x 208] 283 - 304 and 290 - 297 us: no gain any more.  Strided and wide layers have 64-bit sums, as good as
+// fp32 ones: where the output's gradient is 2^-14 of what it is elsewhere in the brick, 32 bits left them 2 - 20 % off.
 bool dcn_scatter_plan(const DcnDims &s, int dtype, ScatterShape &shape) {
   static const int volumes[2][6] = {{2, 3, 3, 12, 14, 14}, {2, 2, 2, 12, 12, 13}};
   static const int deep[2][6] = {{2, 2, 3, 9, 10, 14}, {1, 2, 2, 8, 12, 13}};

@@ -21,11 +21,11 @@
 // Corners that the LDS scatter does not take are listed when the records are made, and their 32 channels are added as
 // 128 contiguous bytes.
 // What bounds it: narrow layers the vector instructions of the samples (184 per 16 positions and 32 channels, and as many more
-// for everything else; vector issue 68 %) and the latency of the gathers (47 % of the wavefronts' time in waits), wide ones LDS
-// (43 %; vector issue 29 %, matrix cores 20 %) and the same waits, and everywhere the atomics of the far corners (64 bytes per corner
+// for everything else; vector issue 68 %) and the latency of the gathers (48 % of the wavefronts' time in waits), wide ones LDS
+// (35 %; vector issue 31 %, matrix cores 21 %) and the same waits (49 %), and everywhere the atomics of the far corners (64 bytes per corner
 // and 16 channels, 21 G of them a second at best).
-//   (bf16 [2, 32 -> 64, 48^3]: 409 us; the data and weight kernels before it took 670 us.  fp16 images
-//   [8, 256 -> 256, 100 x 152]: 582 us, 4380 us before.  [1, 128 -> 128, 7 x 45 x 18]: 60 us, 790 us before.)
+//   (bf16 [2, 32 -> 64, 48^3]: 390 us; the data and weight kernels before it took 670 us.  fp16 images
+//   [8, 256 -> 256, 100 x 152]: 587 us, 4380 us before.  [1, 128 -> 128, 7 x 45 x 18]: 60 us, 790 us before.)
 #include "dcn_scatter.hpp"
 
 #include <algorithm>
@@ -421,7 +421,8 @@ bool dcn_tap_supported(const DcnDims &s, int dtype) {
 // number of times: with about four workgroups per compute unit bf16 [2, 32 -> 64, 48^3] had 1458 workgroups on 1024 places (446 us,
 // now 1998: 411 us), fp16 [8, 256 -> 256, 100 x 152] 1152 on 512 (745 us, now 1440: 653 us).  Every workgroup costs a few tiles of
 // its own: the weight and the first offsets (as long as 1.5 tiles), and a block of the weight gradient, `block` fp32 atomics
-// at 64 bytes per request, 21 G a second, a tile taking 3.7 us.  fp32 layers keep four workgroups per compute unit: each addition
+// at 64 bytes per request, 21 G a second, a tile taking 3.7 us (of those two layers; the ranges hardly depend on it: with 1 to 16 us the
+// backward passes of twelve layers of all instances differ by at most 4 %, most by 1).  fp32 layers keep four workgroups per compute unit: each addition
 // rounds their weight gradient (2.2e-7 rms of it with the ranges of 16-bit layers, 1.9e-7 with these, [2, 64 -> 128, 36 x 40]), at
 // 3 to 5 % of a training step.
 static long tap_ranges(long tiles, long others, long slots, long block) {

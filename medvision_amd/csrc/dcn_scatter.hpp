@@ -41,8 +41,8 @@ __device__ __forceinline__ unsigned tile_bits(const ScatterShape &t, const TileO
   return bits;
 }
 
-// The LDS sums are fixed point (LDS float atomics retire one lane at a time: 0.33 lanes a clock, 64-bit integer ones
-// six to seven).  Every term is w * mask * gcol with 0 <= w <= 1, so
+// The LDS sums are fixed point (LDS float atomics retire one lane at a time: 0.33 lanes a clock, 64-bit integer ones 6.4, or 10.7 where
+// sixteen lanes add to neighbouring words).  Every term is w * mask * gcol with 0 <= w <= 1, so
 //   |term| <= max|mask| * max|grad_output| * max_{c,k} sum_o |Wt[o,c,k]|  =: bound < 2^ex,
 // and a voxel takes at most one corner of each (position, tap) of the brick: positions * taps terms.
 // Terms are scaled by 2^(shift - ex), shift = min(50, 62 - ceil(log2(terms))), and rounded to

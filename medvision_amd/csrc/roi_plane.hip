@@ -16,14 +16,14 @@
 // one, columns in groups of four), so that large rois with a small sampling grid read only what they use.  A lane's
 // piece of a 16 x 16 piece of the box is one 16-byte load (16-bit tensors: 8 bytes), straight from the feature map.
 //   (1000 rois of 4 - 64 pixels, adaptive grid, 256 channels, 7 x 7 cells, fp32, [2, 256, 200, 304]: 480 us when the
-//   boxes went through LDS and three barriers per chunk of channels; 157 us now (168 us with a channel per product, matrix cores 47 %
-//   and texture addressers 58 % busy).  fp16, 1613 rois of 3 - 25 pixels x 256 channels: 147 us with a channel per fp32 product, 122 us with
+//   boxes went through LDS and three barriers per chunk of channels; 157 us now, matrix cores 42 % and texture addressers 58 % busy (168 us
+//   with a channel per product).  fp16, 1613 rois of 3 - 25 pixels x 256 channels: 147 us with a channel per fp32 product, 122 us with
 //   two, 108 us with the first product on the 16-bit cores.)
 //
 // Backward, one workgroup = (16 x 16 pixels, some channels): it looks up the rois that touch its pixels, works out
 // its pixels' weights for eight rois at a time and adds roi after roi into accumulators that stay in registers.  No
 // atomics, no fp32 copy of the gradient, every pixel written once, sums in the order of the rois.
-//   (The same head: 1030 us with one atomic per touched pixel, roi and channel; 145 us now: matrix cores 50 %, vector issue 32 %.  16-bit
+//   (The same head: 1030 us with one atomic per touched pixel, roi and channel; 147 us now: matrix cores 51 %, vector issue 32 %.  16-bit
 //   gradients, 14 x 14 cells: fp16 1499 rois x 256 channels 304 us with fp32 products, 207 us; bf16 1689 x 128 207 us, 143 us.)
 // What bounds them: the matrix cores (three 32-clock instructions per roi, tile and channel backward, eight with 16 cells; 4 x pieces + 2
 // per row piece and channel forward, + 4 with 16 cells; a first product of 16-bit values takes a quarter, forward, or less) and the latency of the loads.

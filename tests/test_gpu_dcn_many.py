@@ -12,7 +12,8 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("taps", [1, 3])
 def test_many_images_of_one_pixel(taps):
     """65535 images of one pixel and 1056 channels: 4.3 million workgroups of 1024 threads sum the gradient of the input, and with 3 x 3 taps
-    19 million of 256 threads form the others.  The pixel takes max(0, 1 - |p|) of every sample along each axis, so that all gradients are products of matrices, here in fp32."""
+    19 million of 256 threads form the others.  The pixel takes max(0, 1 - |p|) of every sample along each axis, so that all gradients are
+    products of matrices, here in fp32."""
     from medvision_amd import _C
     batch, cin, cout, dtype = 65535, 1056, 32, torch.float16
     g = torch.Generator(DEV).manual_seed(taps)

@@ -40,9 +40,12 @@ def _borders(off, g):
     (32, 32, (5, 9, 17), 1, 1, 1),        # volumes: a brick and a remainder along every axis
     (64, 96, (4, 8, 9), 1, 1, 2),         # three slices of grad_output, two deformable groups
     (32, 160, (6, 9, 10), 2, 1, 1),       # strided, more slices than four
-    (48, 16, (9, 5, 25), 1, 1, 1),        # bricks of 4 x 4 x 8 and a remainder along every axis
+    (48, 16, (9, 5, 25), 1, 1, 1),        # channel counts that are padded
+    (32, 160, (9, 5, 25), 1, 1, 1),       # wide: 16-bit ones in bricks of 4 x 4 x 8 and a remainder along every axis
     (16, 64, (9, 13, 17), 2, 1, 1),       # of 2 x 4 x 4, strided
-    (32, 64, (33, 35), 1, 1, 1),          # images: a brick of 32 x 32 (16 x 32) and a remainder
+    (32, 64, (33, 35), 1, 1, 1),          # images: a brick of 32 x 32 (few workgroups of 16-bit ones: of 8 x 8) and a remainder
+    (512, 32, (40, 37), 1, 1, 1),         # of 32 x 32 with 32-bit sums too
+    (512, 64, (33, 67), 2, 1, 1),         # of 8 x 16, strided (fp32: of 16 x 16)
     (64, 288, (17, 33), 1, 1, 1),         # more slices than eight
     (64, 64, (31, 67), 2, 2, 2),          # strided, groups
     (512, 32, (20, 20), 1, 1, 1),         # many channel blocks
@@ -70,7 +73,8 @@ def test_images_with_taps_far_apart(oracle, dtype, cin, cout, size, dilation, gr
     (torch.float16, 63, 160, (5, 7)),     # one image fewer: one block of channels per workgroup
 ])
 def test_two_channel_blocks_per_workgroup(oracle, dtype, batch, cout, size):
-    """Wide images of 2048 and more workgroups of sixteen channels sum 32 channels in two turns."""
+    """Wide 16-bit images of 2048 and more workgroups of sixteen channels sum 32 channels in two turns (fp32 ones have workgroups of eight
+    channels and one turn)."""
     _gradient(oracle, dtype, batch, 512, cout, size, 1, 1, 1, lambda off, g: off, batch + sum(size))
 
 
