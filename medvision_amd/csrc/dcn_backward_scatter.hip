@@ -374,7 +374,9 @@ template <typename S> constexpr bool kDeep = std::is_same<S, TileDeep>::value ||
 using TileImage = Tile<1, 44, 44>;      // 32 x 32 positions, 32-bit sums; 16 x 16 positions whose taps are further apart
 using TileWide = Tile<1, 28, 44>;       // 16 x 32 positions (8 x 16 at stride 2), 64-bit sums of 16-bit tensors
 using TileSmall = Tile<1, 28, 28>;      // 16 x 16 or 8 x 8 positions
-struct TileSmallF32 : TileSmall {         // the same for fp32: two workgroups of 8 channels on a compute unit
+// The same for fp32, 8 channels: twice the workgroups for the few large bricks that fp32 has (backward pass of [1, 256 -> 128, 27 x 58] 155 us,
+// 165 us with 16; with twice as many bricks 16 would be 3 - 5 % faster).
+struct TileSmallF32 : TileSmall {
   template <bool NARROW> static constexpr int channels = 8;
 };
 
