@@ -411,7 +411,7 @@ static bool dcn_dense_large(const DcnDims &s) {
 // with 8 x 8 positions in 28 x 28, 233 us).
 //
 // Tensors of fp32 keep the largest bricks: every addition of a tile's sums to memory rounds.  Images, with the lists of 16-bit ones
-// ([1, 64 -> 64, 24 x 24] in 8 x 8 positions, not 32 x 32): gradient 1.56e-7 (rms) off instead of 1.53e-7, backward pass 100 instead
+// ([1, 64 -> 64, 24 x 24] in 8 x 8 positions, not 32 x 32): gradient 1.56e-7 (rms) off instead of 1.52e-7, backward pass 100 instead
 // of 125 us, [2, 128 -> 128, 112 x 208] 658 instead of 730 us.  Volumes ([4, 16 -> 16, 17 x 43 x 30] with 9 x 10 x 14 of 16 channels): 1.5e-7
 // instead of 1.3e-7, 244 instead of 343 us.
 //

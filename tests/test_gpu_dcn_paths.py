@@ -48,6 +48,7 @@ def test_matrix_core_layers(oracle, dtype, cin, cout, size, stride, groups, dg):
     (32, 64, (48, 72), 1, 12),        # taps far apart
     (32, 64, (6, 20, 48), 2, 1),      # volumes, strided
     (32, 160, (5, 9, 48), 1, 1),
+    (32, 160, (5, 9, 40), 1, 1),      # (the split is in the middle of a brick)
 ])
 def test_small_gradients_beside_large_ones(oracle, dtype, cin, cout, size, stride, dilation):
     """The gradient of the input keeps fp32 sums in strided and wide layers: where the output's gradient is 2^-14 of what it
