@@ -1448,6 +1448,9 @@ static int pool_channels_per_block(const RoiProblem &p, long enough = 6144) {
   return cpb;
 }
 
+// workgroups with `cpb` channels each
+static long pool_groups(const RoiProblem &p, int cpb) { return static_cast<long>(p.R) * ((p.C + cpb - 1) / cpb); }
+
 template <typename T, int CELLS>
 static void launch_pool_forward(const void *input, const float *r, void *output, const RoiProblem &p, int cpb,
                                 dim3 grid, hipStream_t s, int joined = 1, const void *blocked = nullptr, const unsigned *order = nullptr) {
@@ -1538,15 +1541,17 @@ int roi_pool_forward(const void *input, const void *rois, void *output, int dtyp
   // (from the blocked copy, in launch order, a workgroup's set-up weighs more than the balance of the
   // last wave of workgroups: 256 channels per workgroup from 3072 workgroups on, config 5 0.415 -> 0.39 ms)
   // A workgroup whose channels were halved for want of workgroups has idle wavefronts on the matrix cores (four channels
-  // each) and repeats the set-up and the weight products of its box.  There the boxes that suit the matrix cores take sixteen
-  // channels per workgroup and leave the others nothing to do; larger ones, of which a channel takes long, stay spread out
-  // over all of them, four channels each: 141 rois of 16 channels and 5^3 cells 29.5 -> 12 us, 369 of 32 and 7^3 35 -> 19 (27
-  // with eight each), 103 of 16 with boxes of up to 20^3 37 -> 24 (56 with sixteen).  The kernels without matrix cores, where
-  // all threads share a channel, gain from four (29 fp32 rois of 64 channels and 7^3 21 -> 11 us, 15 with eight).
+  // each) and repeats the set-up and the weight products of its box.  There the boxes that suit the matrix cores take up to sixteen
+  // channels per workgroup, with the kernels without matrix cores, where all threads share a channel, up to four, and leave the other workgroups
+  // nothing to do; larger boxes, of which a channel takes long, stay spread out over all of them: fp16, 141 rois of 16 channels and 5^3 cells
+  // 27 -> 21 us, 103 of 16 with boxes of up to 20^3 38 -> 30; fp32, 29 of 64 and 7^3 27 -> 19.  One workgroup per compute unit has to
+  // remain: fewer only make the longest one longer (with sixteen and four channels in whatever number of workgroups, and four for the large
+  // boxes too, fp16, 14 x 32 x 7^3 18.5 -> 37 us; bf16, 5 x 16 11.9 -> 22.8).  Over 220 heads of 4 - 2000 rois and 1 - 256
+  // channels 1.10 - 1.13 times as fast as without joined channels, none slower by more than 6 % (1 us).
   int cpb = pool_channels_per_block(p, blocked != nullptr && order != nullptr ? 3072 : 6144), joined = 1;
   if (pool_small_cells(p)) {
-    if (dtype == MV_F16) cpb = std::max(cpb, std::min(p.C, 4));
     joined = std::max(std::min(p.C, dtype == MV_F16 ? 16 : 4) / cpb, 1);
+    while (joined > 1 && pool_groups(p, cpb * joined) < 256) joined /= 2;
   }
   const long cblocks = (p.C + cpb - 1) / cpb;
   if (cblocks > 65535) return -1;
