@@ -642,6 +642,12 @@ __device__ __forceinline__ bool pool_small_box(const RT *roi, const RoiProblem &
   return (ex - ex / nx + 2.f) * (ey - ey / ny + 2.f) * (nd == 3 ? ez - ez / nz + 2.f : 1.f) <= 4.f * nx * ny * nz;
 }
 
+// Slices of a volume's box, as its extent gives them: the same answer in every workgroup of the roi
+template <typename RT>
+__device__ __forceinline__ int pool_slices(const RT *roi, const RoiProblem &p) {
+  return static_cast<int>(fminf(fmaxf((roi[6] - roi[3]) * static_cast<float>(p.scale), 1.f), static_cast<float>(p.D))) + 1;
+}
+
 template <typename T, typename RT, int CELLS>
 __global__ __launch_bounds__(kPoolThreads) void roi_pool_forward_kernel(
     const T *__restrict__ feat, const RT *__restrict__ rois, T *__restrict__ out, const RoiProblem p,
@@ -1007,9 +1013,10 @@ __device__ inline void pool_backward_mfma(const T *__restrict__ src_any, float *
   // this roi's gradient rows of the block; reads beyond the block's channels return zeros
   const __amdgpu_buffer_rsrc_t gr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<T *>(src), 0, c_count * cells * 2 + 16, 0x00020000);
-  // wavefronts side by side on channel blocks; where there are fewer blocks, several share a block's slices
+  // wavefronts side by side on channel blocks; SHARE: on the slices of the one or two blocks (where the workgroups fill the chip not
+  // on fewer than five slices: each wavefront loads the block's gradient)
   constexpr int kWaves = kPoolThreads / kWave;
-  const int blocks = (c_count + 15) / 16, side = !SHARE || blocks > 2 ? kWaves : blocks;
+  const int blocks = (c_count + 15) / 16, side = !SHARE || (gridDim.z == 1 && nz < 5) ? kWaves : blocks;
   int z_first = 0, z_last = nz;
   if constexpr (SHARE) {
     const int shares = parts * (kWaves / side), share = part * (kWaves / side) + wave / side;
@@ -1086,7 +1093,7 @@ __device__ inline void pool_backward_mfma(const T *__restrict__ src_any, float *
 // CL: the accumulation buffer is channels-last [N, D*H*W, C] (a workspace): the lanes of a wavefront
 // then add neighbouring channels of a voxel, contiguous bytes,
 // instead of one element in each of many rows (a scattered atomic moves a whole memory sector).
-// SHARE: gridDim.z workgroups share the slices of a box.
+// SHARE: up to gridDim.z workgroups share the slices of a box, and wavefronts those of a block of channels.
 template <typename T, typename G, typename RT, bool CL, int CELLS, bool SHARE>
 __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
     const T *__restrict__ gout, const RT *__restrict__ rois, G *__restrict__ gin, const RoiProblem p,
@@ -1095,7 +1102,12 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
   __shared__ __attribute__((aligned(16))) unsigned char lds[kPoolLdsBytes];
   const unsigned n = blockIdx.x;
   const int c_begin = blockIdx.y * channels_per_block, c_end = min(c_begin + channels_per_block, p.C);
-  const int part = SHARE ? blockIdx.z : 0, parts = SHARE ? gridDim.z : 1;
+  int part = 0, parts = 1;
+  if (SHARE && gridDim.z > 1) {   // (at least three slices each: a part repeats the set-up)
+    part = blockIdx.z;
+    parts = min(static_cast<int>(gridDim.z), max(1, pool_slices(rois + static_cast<long>(n) * roi_columns(p.ndim, 0), p) / 3));
+    if (part >= parts) return;
+  }
   // intermediates are fp32 here, so size the chunk with 4-byte box elements
   __shared__ __attribute__((aligned(16))) float wd[3][kDenseSrc][CELLS];
   PoolPlan plan = pool_setup<RT, CELLS>(sh, rois + static_cast<long>(n) * roi_columns(p.ndim, 0), p, sizeof(float), wd, true);
@@ -1582,23 +1594,20 @@ int roi_pool_backward(const void *grad_output, const void *rois, void *acc, int 
                       const RoiProblem &p, hipStream_t s, bool channels_last) {
   if (!pool_applies(dtype, p)) return -1;
   // Channels-last sums of volumes: an atomic request takes as long for one channel as for sixteen, and the matrix
-  // instructions take sixteen in any case.  So a workgroup keeps at least that many, and where rois and channel blocks
-  // do not fill the chip, up to four workgroups share the slices of a box.  Kernel, fp16: 141 rois of 16 channels and 5^3
-  // cells 98 -> 20 us, 77 of 32 and 7^3 103 -> 26; fp32, 250 of 16 and 7^3 52 -> 27.  A part repeats the set-up of the
-  // box: none is added from 1024 workgroups on (1951 rois of 32 channels step in 121 us with one part and in 132 with
-  // two), and up to there the large boxes need them (807 rois of 32 channels, boxes of up to 21^3: 292 us with two,
-  // 325 with one).  On the matrix cores 32 channels per workgroup where four parts of them fill the chip (with 64, where no
-  // wavefronts share slices any more, 461 rois of 256 channels step in 611 us, not 515; below that, 77 rois of 32
-  // channels: 37 us, with 16 per workgroup 26).
+  // instructions take sixteen in any case.  So a workgroup keeps that many (without matrix cores fewer where that would leave few
+  // workgroups), and where rois and channel blocks do not fill the chip, up to four workgroups share the slices of a box; on the matrix
+  // cores wavefronts without a block of their own share those.  Backward passes without both and with them: fp16, 141 rois of 16
+  // channels and 5^3 cells 72 -> 28 us, 77 of 32 and 7^3 114 -> 44, 461 of 256 and 7^3 236 -> 206; fp32, 250 of 16 and 7^3 66 -> 30.  Both repeat
+  // work.  A part repeats the set-up of the box, so it has at least three slices (483 rois of one channel, boxes of 1 - 4 slices: 21.5 us in one part,
+  // 32.5 in three), and there is one from 1024 workgroups on; wavefronts repeat the loads of the gradient.  Over 220 heads of 4 - 2000
+  // rois and 1 - 256 channels 1.28 - 1.38 times as fast as without both, none slower by more than 8 % (3 us).
   int cpb = pool_channels_per_block(p);
   const bool share = channels_last && p.ndim == 3, mfma = dtype == MV_F16 && pool_small_cells(p);
-  if (share) cpb = std::max(cpb, std::min(p.C, mfma && p.R * ((p.C + 31L) / 32) >= 256 ? 32 : 16));
+  if (share) cpb = std::max(cpb, std::min(p.C, mfma || pool_groups(p, 16) >= 128 ? 16 : pool_groups(p, 8) >= 64 ? 8 : 4));
   const long cblocks = (p.C + cpb - 1) / cpb;
   if (cblocks > 65535) return -1;
-  // (larger blocks leave 1024 workgroups and more, and cost nothing where the kernel works out no shares: 5 us of 1190 for the
-  // training step of 4000 rois of 256 channels)
-  const bool shared = share && cpb <= 32;
-  const long groups = p.R * cblocks, parts = shared ? std::min((1023 + groups) / groups, 4L) : 1;
+  const long groups = p.R * cblocks, parts = share ? std::min((1023 + groups) / groups, 4L) : 1;
+  const bool shared = parts > 1 || (share && mfma && cpb <= 32);   // (more than one part: at most sixteen channels)
   const dim3 grid(p.R, static_cast<unsigned>(cblocks), static_cast<unsigned>(parts));
   const float *r = static_cast<const float *>(rois);
   const bool small = pool_small_cells(p);

@@ -34,11 +34,15 @@ def test_fp32_plain(oracle, size, channels, rois, cells, ratio):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("size,channels,rois,cells,ratio,reach", [
-    ((5, 9, 11), 16, 4, (5, 5, 5), 2, 3),         # boxes of fewer slices than workgroups share them
+    ((5, 9, 11), 16, 4, (5, 5, 5), 2, 3),         # boxes of too few slices to be shared
+    ((7, 9, 11), 16, 20, (5, 5, 5), 2, 7),        # about six slices: one or two workgroups
     ((1, 30, 34), 16, 6, (7, 7, 7), 1, 12),       # one slice
     ((21, 13, 10), 17, 9, (7, 7, 7), 2, 18),      # a second block of one channel
     ((14, 12, 9), 50, 30, (4, 3, 4), 0, 14),      # four blocks of sixteen channels, the last of two
-    ((12, 12, 14), 40, 300, (5, 5, 5), 2, 9),     # fp16: two blocks per workgroup, two wavefronts and two workgroups per box and block
+    ((12, 12, 14), 40, 300, (5, 5, 5), 2, 9),     # three blocks, the last of eight channels, two workgroups per box
+    ((12, 12, 14), 24, 30, (5, 5, 5), 2, 12),     # without matrix cores blocks of eight channels
+    ((9, 12, 14), 9, 7, (7, 5, 7), 2, 9),         # of four
+    ((12, 12, 14), 40, 520, (4, 3, 4), 2, 11),    # fp16: two blocks per workgroup, whose wavefronts share the slices of all but flat boxes
     ((24, 30, 34), 40, 16, (6, 5, 7), 3, 40),     # boxes beyond the dense matrices
     ((70, 12, 12), 20, 160, (2, 3, 2), 1, 90),    # boxes wider than the lists: sums per sample
     ((16, 16, 18), 16, 400, (12, 9, 10), 1, 10),  # more than eight cells per axis, three workgroups per box
