@@ -642,10 +642,47 @@ __device__ __forceinline__ bool pool_small_box(const RT *roi, const RoiProblem &
   return (ex - ex / nx + 2.f) * (ey - ey / ny + 2.f) * (nd == 3 ? ez - ez / nz + 2.f : 1.f) <= 4.f * nx * ny * nz;
 }
 
-// Slices of a volume's box, as its extent gives them: the same answer in every workgroup of the roi
+// Voxels of a roi's box, as its extent gives them, or that its samples reach, if those are fewer
 template <typename RT>
-__device__ __forceinline__ int pool_slices(const RT *roi, const RoiProblem &p) {
-  return static_cast<int>(fminf(fmaxf((roi[6] - roi[3]) * static_cast<float>(p.scale), 1.f), static_cast<float>(p.D))) + 1;
+__device__ __forceinline__ float pool_voxels(const RT *roi, const RoiProblem &p) {
+  const float scale = static_cast<float>(p.scale);
+  const int nd = p.ndim;
+  auto extent = [&](int a, int size) { return fminf(fmaxf((roi[1 + nd + a] - roi[1 + a]) * scale, 1.f), static_cast<float>(size)) + 1.f; };
+  const float voxels = extent(0, p.W) * extent(1, p.H) * (nd == 3 ? extent(2, p.D) : 1.f);
+  if (p.sampling_ratio <= 0) return voxels;
+  const float grid = static_cast<float>(p.sampling_ratio), plane = 4.f * grid * grid * static_cast<float>(p.oh * p.ow);
+  return fminf(voxels, nd == 3 ? 2.f * grid * static_cast<float>(p.od) * plane : plane);
+}
+
+// How the workgroups of a roi share its channels and the slices of its box, backward (roi_pool_backward): the same answer in every
+// workgroup of the roi, from the roi's extent.
+struct PoolShare {
+  int most, parts;    // channels of a workgroup, workgroups side by side on the slices: at most
+  int enough, many;   // workgroups per roi that are too few, and that are as many as pay for large boxes
+  int blocks;         // workgroups per roi that are launched
+};
+// In voxels times channels, of which a workgroup without matrix cores takes about 450 a microsecond behind a set-up of five: less than
+// kShareLeast is not worth a part of its own, more than kShareLarge makes the few workgroups of a small head its longest ones.
+constexpr float kShareLeast = 1500.f, kShareLarge = 4000.f;
+__host__ __device__ inline int pool_share_channels(const PoolShare &share, int channels, int parts, float voxels) {
+  int c = share.most;
+  for (; c > 1; c /= 2) {
+    const int groups = (channels + c - 1) / c * parts;
+    if (groups >= (c * voxels > kShareLarge * parts ? share.many : share.enough)) break;
+  }
+  return c;
+}
+// `matrix`: boxes that suit the matrix cores take all channels of their blocks at once
+template <typename RT>
+__device__ __forceinline__ void pool_share(const PoolShare &share, const RT *roi, const RoiProblem &p, bool matrix, int &channels, int &parts) {
+  // (a part repeats the set-up: at least three slices)
+  const int slices = static_cast<int>(fminf(fmaxf((roi[6] - roi[3]) * static_cast<float>(p.scale), 1.f), static_cast<float>(p.D))) + 1;
+  parts = min(share.parts, max(1, slices / 3));
+  channels = share.most;
+  if (matrix && pool_small_box(roi, p)) return;
+  const float voxels = pool_voxels(roi, p);
+  parts = max(1, min(parts, static_cast<int>(voxels * static_cast<float>(channels) * (1.f / kShareLeast))));
+  channels = pool_share_channels(share, p.C, parts, voxels);
 }
 
 template <typename T, typename RT, int CELLS>
@@ -960,7 +997,7 @@ constexpr int kPoolBwdRow = 72;   // fp16 elements per row of the transposed wei
 template <typename T, bool SHARE>
 __device__ inline void pool_backward_mfma(const T *__restrict__ src_any, float *__restrict__ dst_any, const RoiProblem &p,
                                           const PoolShared &sh, const float (&wd)[3][kDenseSrc][8],
-                                          unsigned char *lds, int c_count, int part, int parts) {
+                                          unsigned char *lds, int c_count, int part, int parts, bool alone) {
   using M = Mfma<T>;
   auto uni = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
   const int nx = uni(sh.ax[0].box_hi - sh.ax[0].box_lo + 1), ny = uni(sh.ax[1].box_hi - sh.ax[1].box_lo + 1),
@@ -1016,7 +1053,7 @@ __device__ inline void pool_backward_mfma(const T *__restrict__ src_any, float *
   // wavefronts side by side on channel blocks; SHARE: on the slices of the one or two blocks (where the workgroups fill the chip not
   // on fewer than five slices: each wavefront loads the block's gradient)
   constexpr int kWaves = kPoolThreads / kWave;
-  const int blocks = (c_count + 15) / 16, side = !SHARE || (gridDim.z == 1 && nz < 5) ? kWaves : blocks;
+  const int blocks = (c_count + 15) / 16, side = !SHARE || (alone && nz < 5) ? kWaves : blocks;
   int z_first = 0, z_last = nz;
   if constexpr (SHARE) {
     const int shares = parts * (kWaves / side), share = part * (kWaves / side) + wave / side;
@@ -1093,21 +1130,22 @@ __device__ inline void pool_backward_mfma(const T *__restrict__ src_any, float *
 // CL: the accumulation buffer is channels-last [N, D*H*W, C] (a workspace): the lanes of a wavefront
 // then add neighbouring channels of a voxel, contiguous bytes,
 // instead of one element in each of many rows (a scattered atomic moves a whole memory sector).
-// SHARE: up to gridDim.z workgroups share the slices of a box, and wavefronts those of a block of channels.
+// SHARE: up to share.parts workgroups share the slices of a box, and wavefronts those of a block of channels.
 template <typename T, typename G, typename RT, bool CL, int CELLS, bool SHARE>
 __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
     const T *__restrict__ gout, const RT *__restrict__ rois, G *__restrict__ gin, const RoiProblem p,
-    const int channels_per_block) {
+    const PoolShare share) {
   __shared__ PoolShared sh;
   __shared__ __attribute__((aligned(16))) unsigned char lds[kPoolLdsBytes];
   const unsigned n = blockIdx.x;
-  const int c_begin = blockIdx.y * channels_per_block, c_end = min(c_begin + channels_per_block, p.C);
-  int part = 0, parts = 1;
-  if (SHARE && gridDim.z > 1) {   // (at least three slices each: a part repeats the set-up)
-    part = blockIdx.z;
-    parts = min(static_cast<int>(gridDim.z), max(1, pool_slices(rois + static_cast<long>(n) * roi_columns(p.ndim, 0), p) / 3));
-    if (part >= parts) return;
+  int block = blockIdx.y, channels = share.most, part = 0, parts = 1;
+  if (SHARE && share.parts > 1) {
+    pool_share(share, rois + static_cast<long>(n) * roi_columns(p.ndim, 0), p, CELLS == 8 && std::is_same<T, __half>::value, channels, parts);
+    part = block % parts;
+    block /= parts;
+    if (static_cast<long>(block) * channels >= p.C) return;
   }
+  const int c_begin = block * channels, c_end = min(c_begin + channels, p.C);
   // intermediates are fp32 here, so size the chunk with 4-byte box elements
   __shared__ __attribute__((aligned(16))) float wd[3][kDenseSrc][CELLS];
   PoolPlan plan = pool_setup<RT, CELLS>(sh, rois + static_cast<long>(n) * roi_columns(p.ndim, 0), p, sizeof(float), wd, true);
@@ -1187,7 +1225,7 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_backward_kernel(
       // than the tensor's last block)
       const long behind = (static_cast<long>(p.R) * p.C - (static_cast<long>(n) * p.C + c_end)) * cells * 2;
       if (fits && small && behind >= 16) {
-        pool_backward_mfma<T, SHARE>(src, dst_cl, p, sh, wd, lds, c_end - c_begin, part, parts);
+        pool_backward_mfma<T, SHARE>(src, dst_cl, p, sh, wd, lds, c_end - c_begin, part, parts, share.parts == 1);
         return;
       }
     }
@@ -1472,10 +1510,10 @@ static void launch_pool_forward(const void *input, const float *r, void *output,
 }
 
 template <typename T, bool CL, int CELLS, bool SHARE>
-static void launch_pool_backward(const void *grad_output, const float *r, void *acc, const RoiProblem &p, int cpb,
-                                 dim3 grid, hipStream_t s) {
-  hipLaunchKernelGGL((roi_pool_backward_kernel<T, float, float, CL, CELLS, SHARE>), grid, dim3(kPoolThreads), 0, s,
-                     static_cast<const T *>(grad_output), r, static_cast<float *>(acc), p, cpb);
+static void launch_pool_backward(const void *grad_output, const float *r, void *acc, const RoiProblem &p,
+                                 const PoolShare &share, hipStream_t s) {
+  hipLaunchKernelGGL((roi_pool_backward_kernel<T, float, float, CL, CELLS, SHARE>), dim3(p.R, share.blocks), dim3(kPoolThreads), 0, s,
+                     static_cast<const T *>(grad_output), r, static_cast<float *>(acc), p, share);
 }
 
 // dense-matrix width of the kernel instance: 8 cells per axis when the output allows it
@@ -1594,26 +1632,36 @@ int roi_pool_backward(const void *grad_output, const void *rois, void *acc, int 
                       const RoiProblem &p, hipStream_t s, bool channels_last) {
   if (!pool_applies(dtype, p)) return -1;
   // Channels-last sums of volumes: an atomic request takes as long for one channel as for sixteen, and the matrix
-  // instructions take sixteen in any case.  So a workgroup keeps that many (without matrix cores fewer where that would leave few
-  // workgroups), and where rois and channel blocks do not fill the chip, up to four workgroups share the slices of a box; on the matrix
+  // instructions take sixteen in any case.  So a workgroup keeps that many (eight above 8 cells per axis, where LDS holds few planes of
+  // sixteen), and where rois and channel blocks do not fill the chip, up to four workgroups share the slices of a box; on the matrix
   // cores wavefronts without a block of their own share those.  Backward passes without both and with them: fp16, 141 rois of 16
-  // channels and 5^3 cells 72 -> 28 us, 77 of 32 and 7^3 114 -> 44, 461 of 256 and 7^3 236 -> 206; fp32, 250 of 16 and 7^3 66 -> 30.  Both repeat
-  // work.  A part repeats the set-up of the box, so it has at least three slices (483 rois of one channel, boxes of 1 - 4 slices: 21.5 us in one part,
-  // 32.5 in three), and there is one from 1024 workgroups on; wavefronts repeat the loads of the gradient.  Over 220 heads of 4 - 2000
-  // rois and 1 - 256 channels 1.28 - 1.38 times as fast as without both, none slower by more than 8 % (3 us).
-  int cpb = pool_channels_per_block(p);
-  const bool share = channels_last && p.ndim == 3, mfma = dtype == MV_F16 && pool_small_cells(p);
-  if (share) cpb = std::max(cpb, std::min(p.C, mfma || pool_groups(p, 16) >= 128 ? 16 : pool_groups(p, 8) >= 64 ? 8 : 4));
-  const long cblocks = (p.C + cpb - 1) / cpb;
+  // channels and 5^3 cells 72 -> 28 us, 77 of 32 and 7^3 114 -> 44, 461 of 256 and 7^3 236 -> 206; fp32, 250 of 16 and 7^3 66 -> 30.
+  // What that may cost: boxes of few slices have no parts, and in small heads sixteen channels of a large one last longer than all the
+  // rest (training steps, fp16, 13 rois x 27 channels x 7^3, boxes of up to 35 voxels a side: 83 us with two channels per workgroup, 218 with sixteen;
+  // fp32, 16 x 35 x 10^3, five slices: 60 and 108 us).  So a roi's workgroups settle their channels and parts by its box (pool_share):
+  // fewer channels below 256 workgroups of the head, or 512 where one has much to do: 61 and 69 us.  Heads whose blocks of eight
+  // channels fill the chip stay as they are without matrix cores (735 fp32 rois x 15 channels: 71 us, 77 in parts), and from 1024 workgroups on all do.
+  // Over 460 volume heads of 1 - 4000 rois and 1 - 256 channels a training step is 1.15 times as fast as without sharing, none slower by more than 8 % (a
+  // few us) but one by 13 %.
+  PoolShare share{pool_channels_per_block(p), 1, 0, 0, 0};
+  const bool mfma = dtype == MV_F16 && pool_small_cells(p), joint = channels_last && p.ndim == 3 && (mfma || share.most < 8);
+  if (joint) share.most = std::max(share.most, std::min(p.C, mfma || pool_small_cells(p) ? 16 : 8));
+  const long cblocks = (p.C + share.most - 1L) / share.most, groups = p.R * cblocks;
   if (cblocks > 65535) return -1;
-  const long groups = p.R * cblocks, parts = share ? std::min((1023 + groups) / groups, 4L) : 1;
-  const bool shared = parts > 1 || (share && mfma && cpb <= 32);   // (more than one part: at most sixteen channels)
-  const dim3 grid(p.R, static_cast<unsigned>(cblocks), static_cast<unsigned>(parts));
+  if (joint) share.parts = static_cast<int>(std::min((1023 + groups) / groups, 4L));
+  share.enough = (255 + p.R) / p.R;
+  share.many = (511 + p.R) / p.R;
+  share.blocks = static_cast<int>(cblocks);
+  for (int parts = 1; share.parts > 1 && parts <= share.parts; parts++) {
+    const int c = pool_share_channels(share, p.C, parts, INFINITY);
+    share.blocks = std::max(share.blocks, std::max((p.C + c - 1) / c, static_cast<int>(cblocks)) * parts);
+  }
+  const bool shared = share.parts > 1 || (joint && mfma && share.most <= 32);   // (more than one part: at most sixteen channels)
   const float *r = static_cast<const float *>(rois);
   const bool small = pool_small_cells(p);
 #define MV_POOL_BACKWARD(TYPE, CLV, SHAREV)                                                          \
-  (small ? launch_pool_backward<TYPE, CLV, 8, SHAREV>(grad_output, r, acc, p, cpb, grid, s)          \
-         : launch_pool_backward<TYPE, CLV, 16, SHAREV>(grad_output, r, acc, p, cpb, grid, s))
+  (small ? launch_pool_backward<TYPE, CLV, 8, SHAREV>(grad_output, r, acc, p, share, s)          \
+         : launch_pool_backward<TYPE, CLV, 16, SHAREV>(grad_output, r, acc, p, share, s))
 #define MV_POOL_BACKWARD_OF(TYPE)                                                                    \
   do {                                                                                               \
     if (shared) MV_POOL_BACKWARD(TYPE, true, true);                                                  \

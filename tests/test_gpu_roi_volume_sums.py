@@ -44,6 +44,9 @@ def test_fp32_plain(oracle, size, channels, rois, cells, ratio):
     ((9, 12, 14), 9, 7, (7, 5, 7), 2, 9),         # of four
     ((12, 12, 14), 40, 520, (4, 3, 4), 2, 11),    # fp16: two blocks per workgroup, whose wavefronts share the slices of all but flat boxes
     ((24, 30, 34), 40, 16, (6, 5, 7), 3, 40),     # boxes beyond the dense matrices
+    ((5, 40, 38), 35, 9, (10, 10, 10), 3, 36),    # wide boxes of few slices: one or two channels per workgroup, one or two parts
+    ((20, 30, 30), 19, 3, (7, 6, 7), 2, 28),      # fp16: boxes beyond the matrix cores beside small ones; channels and parts by the box
+    ((13, 24, 20), 29, 30, (9, 10, 9), 1, 24),    # more than eight cells: blocks of eight channels or fewer
     ((70, 12, 12), 20, 160, (2, 3, 2), 1, 90),    # boxes wider than the lists: sums per sample
     ((16, 16, 18), 16, 400, (12, 9, 10), 1, 10),  # more than eight cells per axis, three workgroups per box
     ((12, 12, 14), 16, 1023, (4, 4, 4), 2, 9),    # two workgroups per box
