@@ -662,8 +662,9 @@ struct PoolShare {
   int blocks;         // workgroups per roi that are launched
 };
 // In voxels times channels, of which a workgroup without matrix cores takes about 450 a microsecond behind a set-up of five: less than
-// kShareLeast is not worth a part of its own, more than kShareLarge makes the few workgroups of a small head its longest ones.
-constexpr float kShareLeast = 1500.f, kShareLarge = 4000.f;
+// kShareLeast is not worth a part of its own, more than kShareLarge makes the few workgroups of a small head its longest ones; forward, joined
+// channels of more than kShareJoined last longer than the set-ups that they save.
+constexpr float kShareLeast = 1500.f, kShareLarge = 4000.f, kShareJoined = 3000.f;
 __host__ __device__ inline int pool_share_channels(const PoolShare &share, int channels, int parts, float voxels) {
   int c = share.most;
   for (; c > 1; c /= 2) {
@@ -694,7 +695,15 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_forward_kernel(
   __shared__ __attribute__((aligned(16))) unsigned char lds[kPoolLdsBytes];
   const unsigned n = order ? order[blockIdx.x] : blockIdx.x;   // (largest rois first, see pool_order_rois)
   int cpb = channels_per_block;   // small boxes: `joined` times as many
-  if (joined > 1 && pool_small_box(rois + static_cast<long>(n) * roi_columns(p.ndim, 0), p)) cpb *= joined;
+  if (joined > 1) {
+    constexpr bool kMatrix = CELLS == 8 && std::is_same<T, __half>::value;
+    const RT *roi = rois + static_cast<long>(n) * roi_columns(p.ndim, 0);
+    if (pool_small_box(roi, p)) {
+      int times = joined;
+      while (!kMatrix && times > 1 && pool_voxels(roi, p) * static_cast<float>(cpb * times) > kShareJoined) times /= 2;
+      cpb *= times;
+    }
+  }
   if (static_cast<long>(blockIdx.y) * cpb >= p.C) return;   // (channels of a workgroup before)
   const int c_begin = blockIdx.y * cpb, c_end = min(c_begin + cpb, p.C);
   __shared__ __attribute__((aligned(16))) float wd[3][kDenseSrc][CELLS];
@@ -1594,10 +1603,11 @@ int roi_pool_forward(const void *input, const void *rois, void *output, int dtyp
   // each) and repeats the set-up and the weight products of its box.  There the boxes that suit the matrix cores take up to sixteen
   // channels per workgroup, with the kernels without matrix cores, where all threads share a channel, up to four, and leave the other workgroups
   // nothing to do; larger boxes, of which a channel takes long, stay spread out over all of them: fp16, 141 rois of 16 channels and 5^3 cells
-  // 27 -> 21 us, 103 of 16 with boxes of up to 20^3 38 -> 30; fp32, 29 of 64 and 7^3 27 -> 19.  One workgroup per compute unit has to
-  // remain: fewer only make the longest one longer (with sixteen and four channels in whatever number of workgroups, and four for the large
-  // boxes too, fp16, 14 x 32 x 7^3 18.5 -> 37 us; bf16, 5 x 16 11.9 -> 22.8).  Over 220 heads of 4 - 2000 rois and 1 - 256
-  // channels 1.10 - 1.13 times as fast as without joined channels, none slower by more than 6 % (1 us).
+  // 27 -> 21 us, 103 of 16 with boxes of up to 20^3 38 -> 30, 369 of 32 and 7^3 43 -> 32; fp32, 29 of 64 and 7^3 22 -> 13.  One workgroup per
+  // compute unit has to remain: fewer only make the longest one longer (with sixteen and four channels in whatever number of workgroups, and
+  // four for the large boxes too, fp16, 14 x 32 x 7^3 18.5 -> 37 us; bf16, 5 x 16 11.9 -> 22.8).  Without matrix cores no more channels are joined than
+  // the box has work for (kShareJoined): 947 fp32 rois of two channels, 8^3 cells and boxes of up to 32 x 18 x 32 take 46 us, joined 56; 55 of
+  // 18 and 7^3 18 and 27.
   int cpb = pool_channels_per_block(p, blocked != nullptr && order != nullptr ? 3072 : 6144), joined = 1;
   if (pool_small_cells(p)) {
     joined = std::max(std::min(p.C, dtype == MV_F16 ? 16 : 4) / cpb, 1);
