@@ -1172,7 +1172,7 @@ def test_raw_backward_adds_to_the_gradient(oracle, dtype, rotated, channels, roi
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("ndim,rotated,C,out", [(3, True, 24, (7, 7, 7)), (3, True, 72, (7, 7, 7)),
+@pytest.mark.parametrize("ndim,rotated,C,out", [(3, True, 24, (7, 7, 7)), (3, True, 72, (7, 7, 7)), (3, True, 16, (10, 9, 11)),
                                                 (2, True, 520, (14, 14)), (2, False, 32, (20, 20))])
 def test_heads_forward_from_channels_last_copy(ops, oracle, dtype, ndim, rotated, C, out):
     """Detection heads that the separable pooled kernels do not take (rotated boxes, more than 16 cells per
