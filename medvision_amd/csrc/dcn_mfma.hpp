@@ -6,6 +6,9 @@ namespace mv {
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
@@ -26,11 +29,10 @@ template <> struct Mfma<__half> {
     return __half2float(__ushort_as_half(static_cast<unsigned short>(w >> 16)));
   }
   static __device__ __forceinline__ float element(const u32x4 &r, int i) { return i % 2 ? hi(r[i / 2]) : lo(r[i / 2]); }
-  // two values rounded to nearest even and packed, in one instruction
+  // two values rounded to nearest even and packed, in one instruction (v_cvt_pk_f16_f32; not as inline assembly, around which the
+  // compiler leaves no wait for a matrix instruction that is still writing a or b)
   static __device__ __forceinline__ unsigned pack2(float a, float b) {
-    unsigned r;
-    asm("v_cvt_pk_f16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
+    return __builtin_bit_cast(unsigned, __builtin_convertvector((float2_t{a, b}), half2_t));
   }
   // v[0..7] += w * piece
   static __device__ __forceinline__ void fma_piece(float (&v)[8], float w, u32x4 r) {
@@ -49,11 +51,10 @@ template <> struct Mfma<__hip_bfloat16> {
   static __device__ __forceinline__ float lo(unsigned w) { return __uint_as_float(w << 16); }
   static __device__ __forceinline__ float hi(unsigned w) { return __uint_as_float(w & 0xffff0000u); }
   static __device__ __forceinline__ float element(const u32x4 &r, int i) { return i % 2 ? hi(r[i / 2]) : lo(r[i / 2]); }
-  // two values rounded to nearest even and packed, in one instruction
+  // two values rounded to nearest even and packed, in one instruction (v_cvt_pk_bf16_f32; not as inline assembly, around which the
+  // compiler leaves no wait for a matrix instruction that is still writing a or b)
   static __device__ __forceinline__ unsigned pack2(float a, float b) {
-    unsigned r;
-    asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
+    return __builtin_bit_cast(unsigned, __builtin_convertvector((float2_t{a, b}), bf16x2_t));
   }
   static __device__ __forceinline__ void fma_piece(float (&v)[8], float w, u32x4 r) {
     v[0] += w * lo(r.x); v[1] += w * hi(r.x); v[2] += w * lo(r.y); v[3] += w * hi(r.y);
