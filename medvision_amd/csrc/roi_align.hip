@@ -173,6 +173,10 @@ int roi_plane_forward(const void *input, const void *rois, void *output, int dty
 int roi_plane_backward_parts(int dtype, const RoiProblem &p);
 int roi_plane_backward(const void *grad_output, const void *rois, void *grad, float *acc, int dtype, const RoiProblem &p,
                        int parts, bool accumulate, hipStream_t s);
+// roi_brick_backward.hip: backward of 16-bit heads of plain boxes on volumes by the voxels' owners
+size_t roi_brick_workspace(int dtype, const RoiProblem &p);
+int roi_brick_backward(const void *grad_output, const void *rois, void *grad_input, int dtype, const RoiProblem &p, void *workspace,
+                       size_t capacity, hipStream_t s);
 // roi_own_backward.hip: backward of heads that the pooled kernels do not take (rotated boxes, large grids) by the voxels' owners
 bool roi_own_applies(int dtype, const RoiProblem &p);
 size_t roi_own_workspace(int dtype, const RoiProblem &p);
@@ -343,6 +347,10 @@ int roi_backward(const void *grad_output, const void *rois, void *grad_input, in
     if (st >= 0) return st || parts == 1 ? st : fold_sums();
   }
   // (a gradient to be added to keeps the kernel with atomics, and so does one without the workspace)
+  if (!accumulate) {
+    st = roi_brick_backward(grad_output, rois, grad_input, dtype, p, workspace, capacity, s);
+    if (st >= 0) return st;
+  }
   if (!accumulate && !roi_pool_applies(dtype, p)) {
     st = roi_own_backward(grad_output, rois, grad_input, dtype, p, workspace, capacity, s);
     if (st >= 0) return st;
@@ -557,7 +565,8 @@ size_t mv_roi_align_backward_write_workspace_bytes(int dtype, int ndim, int rota
   const bool any = batch > 0 && channels > 0 && p.D > 0 && height > 0 && width > 0 && num_rois > 0 && p.od > 0 && out_h > 0 && out_w > 0;
   if (any && mv::roi_backward_wants_sums(dtype, p)) return sizeof(float) * static_cast<size_t>(batch) * channels * p.D * height * width;
   const size_t sums = mv_roi_align_backward_workspace_bytes(dtype, batch, channels, depth, height, width);
-  if (!any || mv::roi_pool_applies(dtype, p)) return sums;
+  if (!any) return sums;
+  if (mv::roi_pool_applies(dtype, p)) return std::max(sums, mv::roi_brick_workspace(dtype, p));
   return std::max(sums, mv::roi_own_workspace(dtype, p));
 }
 

@@ -1,0 +1,656 @@
+// RoIAlign BACKWARD of plain boxes with few cells per axis (fp16 detection heads on volumes) by the voxels' owners: no global
+// atomics, no fp32 copy of the gradient to clear and to fold.  Same results as the reference's one-thread-per-output kernel
+// with eight atomicAdd per sample (csrc/cuda/roi_align_3d_cuda_kernel.cuh:90-202).
+//
+// A box's samples are separable, so a roi's share of the gradient is
+//     grad[z, y, x][c] += sum_pd Wz[z][pd] P[c, pd][y, x],   P[c, pd][y, x] = sum_(ph, pw) gout[c][pd][ph][pw] Wy[y][ph] Wx[x][pw]
+// with a short matrix per axis (up to 8 cells).  A wavefront owns a brick of 8 x 8 x 8 voxels and 16 channels: their sums are
+// accumulators.  It takes the rois that touch the brick one after the other.  Both sums are products on the matrix cores, for two
+// channels and 16 voxels (two rows of the brick) at a time:
+//   * P: rows (channel, pd), K = (ph, pw) with cells padded to rows of eight, so that a lane's 16-byte piece of the left operand is
+//     one row of cells as it lies in grad_output, and its piece of the right one a row of Wx times one number of Wy, formed in
+//     registers from the roi's tables, which a small launch before has left in memory.
+//   * over pd: rows (channel', z), K = (channel, pd), block-diagonal in the channel with Wz in the blocks: the accumulator of the
+//     first product is the right operand of the second as it stands.
+// The gradient of a roi's 16 channels is one run of memory of 10 KB or so.  It comes to LDS as it lies there (loads of its rows of
+// cells straight into registers, 16 bytes of 64 different cache lines each, kept the texture addressers 85 % busy: 800 us for
+// 4000 rois x 256 channels x 7^3), the next roi's while the present one's products run.  The order of the sums is the order of the rois.
+//
+// Two small launches before: the rois' tables, and the bricks' lists of rois.  The two wavefronts of a workgroup have neighbouring
+// bricks along x: rows of the gradient are written 32 bytes at a time (16 bytes of a single brick are 547 MB for a gradient of 226;
+// four bricks, 64 bytes, wait for the longest of four lists).
+#include "common.hpp"
+#include "roi_geometry.hpp"
+#include "sampling.hpp"
+#include "dcn_mfma.hpp"
+
+#include <algorithm>
+
+namespace mv {
+
+bool roi_pool_applies(int dtype, const RoiProblem &p);   // roi_pool.hip
+
+constexpr int kBrickThreads = 256, kBrickWaves = kBrickThreads / kWave;
+constexpr int kBrickCells = 8, kBrickChannels = 16;
+constexpr int kBrickTried = 4;                 // records that a thread fetches together
+constexpr int kBrickEdge = 8;                  // voxels of a brick along each axis
+constexpr int kBrickPad = 128;                 // bytes behind the copy of the last roi's gradient
+
+// What the tables kernel leaves about a roi: first and last voxel of its box per axis (low and high half; first > last: the roi
+// touches nothing) and the image.  Its tables are rows of eight fp32 weights, one per voxel along x, then y, then z, the axes
+// padded to whole bricks; only the rows of the bricks that the box touches are written.  A row of y holds cell c at
+// c % 4 * 2 + c / 4, the two cells of a lane side by side.
+struct BrickRoi { unsigned span[3]; int image; };
+
+__host__ __device__ inline int brick_up(int n) { return (n + kBrickEdge - 1) / kBrickEdge * kBrickEdge; }
+__host__ __device__ inline int brick_rows(const RoiProblem &p) { return brick_up(p.W) + brick_up(p.H) + brick_up(p.D); }
+// where the rows of y and z start
+__device__ __forceinline__ int brick_row_y(const RoiProblem &p) { return brick_up(p.W); }
+__device__ __forceinline__ int brick_row_z(const RoiProblem &p) { return brick_up(p.W) + brick_up(p.H); }
+
+// One workgroup per roi, a wavefront per axis; further ones copy the last roi's gradient to a place with room behind it (a row of
+// cells is read as 16 bytes, more than it may have behind it at the end of a tensor).
+__global__ __launch_bounds__(3 * kWave) void roi_brick_tables_kernel(const float *__restrict__ rois, BrickRoi *__restrict__ recs,
+                                                                     float *__restrict__ tables, const RoiProblem p,
+                                                                     const __half *__restrict__ last, __half *__restrict__ copy, const int slab) {
+  if (blockIdx.x >= static_cast<unsigned>(p.R)) {
+    const int at = ((blockIdx.x - p.R) * 3 * kWave + threadIdx.x) * 8, end = slab + kBrickPad / 2;
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      if (at + i < end) copy[at + i] = at + i < slab ? last[at + i] : store_cast<__half>(0.f);
+    return;
+  }
+  const int n = blockIdx.x, a = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+  const float *roi = rois + static_cast<long>(n) * roi_columns(3, 0);
+  const int image = static_cast<int>(roi[0]), nc = a == 0 ? p.ow : a == 1 ? p.oh : p.od, sz = a == 0 ? p.W : a == 1 ? p.H : p.D;
+  const bool empty = image < 0 || image >= p.N;
+  // (the expressions of build_geom; an extent of at least 1 has a grid of at least 1)
+  const double start = static_cast<double>(roi[1 + a]) * p.scale, ext = fmax(static_cast<double>(roi[4 + a]) * p.scale - start, 1.0);
+  const int grid = p.sampling_ratio > 0 ? p.sampling_ratio : static_cast<int>(ceil(ext / static_cast<double>(nc)));
+  const double bin = ext / static_cast<double>(nc), step = bin / static_cast<double>(grid), per = 1.0 / step;
+  auto tap = [&](int cell, int sub, int &lo, int &hi, float &frac) {   // (local_coord's expression)
+    const double v = start + cell * bin + static_cast<double>(static_cast<float>(sub) + .5f) * step;
+    return clamped_tap<float>(v, sz, lo, hi, frac, p.order);
+  };
+  // Positions grow with the sample, so the box runs from the first valid sample to the last: both are among the 64 from, and up to,
+  // the ones that this estimate gives (fmin and fmax make 0 and the last of a position that is not a number).
+  int first = 0x7fff, last_voxel = -1;
+  if (!empty) {
+    const long entries = static_cast<long>(nc) * grid;
+    const double top = static_cast<double>(entries - 1);
+    const long e0 = static_cast<long>(fmin(fmax(floor((-1.0 - start) * per - 0.5) - 2.0, 0.0), top));
+    const long e1 = static_cast<long>(fmax(fmin(ceil((sz - start) * per - 0.5) + 2.0, top), 0.0));
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const long e = i == 0 ? min(e0 + lane, entries - 1) : max(e1 - lane, 0L);
+      int lo, hi;
+      float frac;
+      int cell = 0;
+      long sub = e;
+      while (sub >= grid && cell + 1 < nc) { sub -= grid; cell++; }
+      if (tap(cell, static_cast<int>(sub), lo, hi, frac)) {
+        first = min(first, lo);
+        last_voxel = max(last_voxel, hi);
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 1; m < kWave; m *= 2) {
+    first = min(first, __shfl_xor(first, m));
+    last_voxel = max(last_voxel, __shfl_xor(last_voxel, m));
+  }
+  if (lane == 0) {
+    recs[n].span[a] = static_cast<unsigned>(first) | static_cast<unsigned>(max(last_voxel, 0)) << 16;
+    if (a == 0) recs[n].image = image;
+  }
+  const int cell = lane % kBrickCells;
+  const float inv = 1.f / static_cast<float>(grid);
+  float *rows = tables + (static_cast<long>(n) * brick_rows(p) + (a == 0 ? 0 : a == 1 ? brick_row_y(p) : brick_row_z(p))) * kBrickCells;
+  for (int r0 = first / kBrickEdge * kBrickEdge; r0 <= last_voxel; r0 += kWave / kBrickCells) {
+    const int row = r0 + lane / kBrickCells;
+    float w = 0.f;
+    if (cell < nc && row >= first && row <= last_voxel) {
+      // the cell's samples that can reach the row, a few more on either side
+      const double from = start + cell * bin, below = row == 0 ? -1.0 : row - 1.0, above = row >= sz - 2 ? sz : row + 1.0;
+      const int s0 = static_cast<int>(fmin(fmax(floor((below - from) * per - 0.5) - 2.0, 0.0), static_cast<double>(grid - 1)));
+      const int s1 = static_cast<int>(fmax(fmin(ceil((above - from) * per - 0.5) + 2.0, static_cast<double>(grid - 1)), 0.0));
+      for (int s = s0; s <= s1; s++) {
+        int lo, hi;
+        float frac;
+        if (!tap(cell, s, lo, hi, frac)) continue;
+        if (lo == row) w += (1.f - frac) * inv;
+        if (hi == row) w += frac * inv;
+      }
+    }
+    rows[row * kBrickCells + (a == 1 ? cell % 4 * 2 + cell / 4 : cell)] = w;
+  }
+}
+
+// The rois that touch a brick, in their order: a workgroup per brick.  An entry is the roi's number, with a bit for the upper
+// four rows of the brick and one for the lower four.
+constexpr unsigned kBrickUpper = 1u << 30, kBrickLower = 1u << 31;
+__global__ __launch_bounds__(kBrickThreads) void roi_brick_lists_kernel(const uint4 *__restrict__ recs, unsigned *__restrict__ lists,
+                                                                        unsigned *__restrict__ lengths, const int R, const int nx,
+                                                                        const int ny, const int nz) {
+  __shared__ unsigned counts[2][kBrickTried * kBrickWaves];
+  unsigned id = blockIdx.x;
+  unsigned *const list = lists + static_cast<long>(id) * R;
+  const int first[3] = {static_cast<int>(id % nx) * kBrickEdge, static_cast<int>(id / nx % ny) * kBrickEdge,
+                        static_cast<int>(id / nx / ny % nz) * kBrickEdge};
+  const int image = id / nx / ny / nz;
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  unsigned have = 0;
+  int turn = 0;
+  for (int base = 0; base < R; base += kBrickTried * kBrickThreads, turn ^= 1) {
+    uint4 rec[kBrickTried];
+    unsigned long hits[kBrickTried];
+#pragma unroll
+    for (int i = 0; i < kBrickTried; i++) rec[i] = recs[min(base + i * kBrickThreads + static_cast<int>(threadIdx.x), R - 1)];
+#pragma unroll
+    for (int i = 0; i < kBrickTried; i++) {
+      const int k = base + i * kBrickThreads + static_cast<int>(threadIdx.x);
+      const unsigned span[3] = {rec[i].x, rec[i].y, rec[i].z};
+      bool hit = k < R && static_cast<int>(rec[i].w) == image;
+#pragma unroll
+      for (int a = 0; a < 3; a++) {
+        const int lo = static_cast<int>(span[a] & 0xffffu) - first[a], hi = static_cast<int>(span[a] >> 16) - first[a];
+        hit = hit && lo <= hi && lo < kBrickEdge && hi >= 0;
+        if (a == 1) rec[i].x = static_cast<unsigned>(k) | (lo < kBrickEdge / 2 ? kBrickUpper : 0) | (hi >= kBrickEdge / 2 ? kBrickLower : 0);
+      }
+      hits[i] = __ballot(hit);
+      if (lane == 0) counts[turn][i * kBrickWaves + wave] = __popcll(hits[i]);
+    }
+    __syncthreads();   // (the counts of a turn are read before this barrier of the next one, and written again behind it)
+#pragma unroll
+    for (int i = 0; i < kBrickTried; i++)
+#pragma unroll
+      for (int w = 0; w < kBrickWaves; w++) {
+        if (w == wave && (hits[i] >> lane & 1)) list[have + __popcll(hits[i] & ((1UL << lane) - 1))] = rec[i].x;
+        have += counts[turn][i * kBrickWaves + w];
+      }
+  }
+  if (threadIdx.x == 0) lengths[id] = have;
+}
+
+// The operands of the products: the weights Wy Wx and the sums P are rounded once each (11 bits; P that overflows makes a sum that is
+// not finite, see brick_careful), Wz is the sum of two numbers.
+typedef _Float16 brick_half4 __attribute__((ext_vector_type(4)));
+struct BrickLeft { brick_half4 high, low; };
+__device__ __forceinline__ brick_half4 brick_pack(const float (&w)[4]) {
+  return __builtin_bit_cast(brick_half4, uint2{Mfma<__half>::pack2(w[0], w[1]), Mfma<__half>::pack2(w[2], w[3])});
+}
+__device__ __forceinline__ BrickLeft brick_left(const float (&w)[4]) {
+  BrickLeft l;
+  l.high = brick_pack(w);
+  float rest[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) rest[r] = w[r] - static_cast<float>(l.high[r]);
+  l.low = brick_pack(rest);
+  return l;
+}
+__device__ __forceinline__ float4_t brick_add(const BrickLeft &l, const float4_t &part, float4_t acc) {
+  const float p[4] = {part[0], part[1], part[2], part[3]};
+  const brick_half4 right = brick_pack(p);
+  acc = __builtin_amdgcn_mfma_f32_16x16x16f16(l.low, right, acc, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x16f16(l.high, right, acc, 0, 0, 0);
+}
+
+// A region whose sums come out not finite, done again term by term and without the terms of weight 0.  Thread: one (y, x) of the
+// region, its sums of eight channels and all slices in LDS.
+template <int LOG_WX>
+__device__ inline void brick_careful(const __half *__restrict__ gout, const BrickRoi *__restrict__ recs, const float *__restrict__ tables,
+                                     __half *__restrict__ grad, const RoiProblem &p, float *const sums, const int X0,
+                                     const int Y0, const int Z0, const int c_base, const int image) {
+  constexpr int TZ = kBrickEdge;
+  using M = Mfma<__half>;
+  constexpr int threads = kWave << LOG_WX;
+  const int lane = threadIdx.x % kWave, x = X0 + (threadIdx.x & ((8 << LOG_WX) - 1)), y = Y0 + (threadIdx.x >> (3 + LOG_WX));
+  const int cells = p.od * p.oh * p.ow, ohw = p.oh * p.ow;
+  float *const mine = sums + threadIdx.x;
+  for (int c0 = c_base; c0 < min(c_base + kBrickChannels, p.C); c0 += 8) {
+    const int cn = min(8, p.C - c0);
+    for (int i = 0; i < 8 * TZ; i++) mine[i * threads] = 0.f;
+    for (int base = 0; base < p.R; base += kWave) {
+      const BrickRoi rec = recs[min(base + lane, p.R - 1)];
+      const int first[3] = {X0, Y0, Z0}, extent[3] = {8 << LOG_WX, 8, TZ};
+      bool hit = base + lane < p.R && rec.image == image;
+#pragma unroll
+      for (int a = 0; a < 3; a++) {
+        const int lo = rec.span[a] & 0xffffu, hi = rec.span[a] >> 16;
+        hit = hit && lo <= hi && lo < first[a] + extent[a] && hi >= first[a];
+      }
+      for (unsigned long mask = __ballot(hit); mask != 0; mask &= mask - 1) {
+        const int i = __builtin_ctzl(mask), n = base + i;
+        unsigned span[3];
+#pragma unroll
+        for (int a = 0; a < 3; a++) span[a] = __builtin_amdgcn_readlane(rec.span[a], i);
+        if (x < static_cast<int>(span[0] & 0xffffu) || x > static_cast<int>(span[0] >> 16) ||
+            y < static_cast<int>(span[1] & 0xffffu) || y > static_cast<int>(span[1] >> 16))
+          continue;
+        const int z0 = max(static_cast<int>(span[2] & 0xffffu) - Z0, 0), z1 = min(static_cast<int>(span[2] >> 16) - Z0, TZ - 1);
+        const float *tab = tables + static_cast<long>(n) * brick_rows(p) * kBrickCells;
+        for (int c = 0; c < cn; c++)
+          for (int pd = 0; pd < p.od; pd++) {
+            const __half *g = gout + (static_cast<long>(n) * p.C + c0 + c) * cells + pd * ohw;
+            float part = 0.f;
+            for (int k = 0; k < ohw; k++) {
+              const int ph = k / p.ow, pw = k - ph * p.ow;
+              float w = tab[(brick_row_y(p) + y) * kBrickCells + ph % 4 * 2 + ph / 4] * tab[x * kBrickCells + pw];
+              w = M::lo(M::pack2(w, w));   // (as the products have it)
+              if (w != 0.f) part += w * load(g + k);
+            }
+            for (int z = z0; z <= z1; z++) {
+              const float w = tab[(brick_row_z(p) + Z0 + z) * kBrickCells + pd];
+              if (w != 0.f && part != 0.f) mine[(c * TZ + z) * threads] += w * part;
+            }
+          }
+      }
+    }
+    if (x < p.W && y < p.H)
+      for (int i = 0; i < cn * TZ; i++)
+        if (Z0 + i % TZ < p.D)
+          grad[(((static_cast<long>(image) * p.C + c0 + i / TZ) * p.D + Z0 + i % TZ) * p.H + y) * p.W + x] = store_cast<__half>(mine[i * threads]);
+  }
+}
+
+// What a workgroup works on: 1 << LOG_WX bricks side by side, 16 channels of an image; `part` of `parts` workgroups that share them.
+template <int LOG_WX>
+struct BrickPlace {
+  int X0, Y0, Z0, c_base, image, part;
+  long brick;      // the first one's number, among those of all images
+  int bricks;      // of them that there are
+  bool none;
+  __device__ __forceinline__ BrickPlace(const RoiProblem &p, const int nx, const int ny, const int nz, const int cblocks, const int parts,
+                                        const unsigned total) {
+    // eight runs of regions, one per die, neighbours one after the other: they read the same rois' gradients
+    const unsigned run = (total + 7) / 8;
+    unsigned id = (blockIdx.x % 8) * run + blockIdx.x / 8;
+    none = blockIdx.x / 8 >= run || id >= total;
+    part = id % parts; id /= parts;
+    const int rx = id % nx; id /= nx;
+    const int ry = id % ny; id /= ny;
+    const int rz = id % nz; id /= nz;
+    c_base = static_cast<int>(id % cblocks) * kBrickChannels;
+    image = id / cblocks;
+    X0 = rx * kBrickEdge << LOG_WX; Y0 = ry * kBrickEdge; Z0 = rz * kBrickEdge;
+    const int along = (p.W + kBrickEdge - 1) / kBrickEdge;
+    brick = ((static_cast<long>(image) * nz + rz) * ny + ry) * along + (rx << LOG_WX);
+    bricks = min(1 << LOG_WX, along - (rx << LOG_WX));
+  }
+};
+
+// The wavefronts' sums to the gradient.  acc[i][k], register r: channel 2 i + quad / 2, voxel z = quad % 2 * 4 + r, y = 2 k + col / 8,
+// x = col % 8 of the brick.
+template <int LOG_WX>
+__device__ __forceinline__ void brick_finish(const float4_t (&acc)[kBrickChannels / 2][4], const BrickPlace<LOG_WX> &at,
+                                             const __half *__restrict__ gout, const BrickRoi *__restrict__ recs,
+                                             const float *__restrict__ tables, __half *__restrict__ grad, const RoiProblem &p,
+                                             unsigned char *const lds, unsigned &special) {
+  constexpr int wxn = 1 << LOG_WX, RX = kBrickEdge << LOG_WX, TZ = kBrickEdge;
+  const int lane = threadIdx.x % kWave, bx = threadIdx.x / kWave * kBrickEdge, col = lane % 16, quad = lane / 16;
+  // a weight of zero times a gradient that is not finite is not a number
+  float check = 0.f;
+#pragma unroll
+  for (int i = 0; i < kBrickChannels / 2; i++)
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) check = fmaf(acc[i][k][r], 0.f, check);
+  if (__ballot(!(check == 0.f)) != 0 && lane == 0) special = 1;
+  __syncthreads();
+  if (special != 0) {
+    brick_careful<LOG_WX>(gout, recs, tables, grad, p, reinterpret_cast<float *>(lds), at.X0, at.Y0, at.Z0, at.c_base, at.image);
+    return;
+  }
+  // through LDS, so that rows of the region go out whole: [channel][z][y][x], a little room between channels against bank conflicts
+  __half *const stage = reinterpret_cast<__half *>(lds);
+  constexpr int channel = (TZ * 64 << LOG_WX) + 8;
+#pragma unroll
+  for (int i = 0; i < kBrickChannels / 2; i++)
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        stage[(2 * i + quad / 2) * channel + ((quad % 2 * 4 + r) * 8 + 2 * k + col / 8) * RX + bx + col % 8] =
+            store_cast<__half>(acc[i][k][r]);
+  __syncthreads();
+  constexpr int kPieces = kBrickChannels * wxn * TZ * 8;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < kPieces; i += kWave * wxn) {
+    const int px = i & (wxn - 1), row = (i >> LOG_WX) & (TZ * 8 - 1), cl = (i >> LOG_WX) / (TZ * 8);
+    const int y = at.Y0 + row % 8, z = at.Z0 + row / 8, x = at.X0 + px * 8;
+    if (at.c_base + cl >= p.C || y >= p.H || z >= p.D || x >= p.W) continue;
+    const u32x4 v = *reinterpret_cast<const u32x4 *>(stage + cl * channel + row * RX + px * 8);
+    __half *dst = grad + (((static_cast<long>(at.image) * p.C + at.c_base + cl) * p.D + z) * p.H + y) * p.W + x;
+    if (x + 8 <= p.W) {   // one store: global memory takes any alignment
+      typedef unsigned int V __attribute__((ext_vector_type(4), aligned(2)));
+      *reinterpret_cast<V *>(dst) = v;
+    } else {
+      __half e[8];
+      __builtin_memcpy(e, &v, sizeof(v));
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+        if (x + k < p.W) dst[k] = e[k];
+    }
+  }
+}
+
+// where part `k` of `parts` of a list begins
+__device__ __forceinline__ int brick_share(const int length, const int k, const int parts) {
+  return static_cast<int>(static_cast<long>(length) * k / parts);
+}
+
+template <int LOG_WX, bool SHARED>
+__global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
+    const __half *__restrict__ gout, const __half *__restrict__ last, const BrickRoi *__restrict__ recs, const float *__restrict__ tables,
+    const unsigned *__restrict__ lists, const unsigned *__restrict__ lengths, __half *__restrict__ grad, const RoiProblem p, const int nx,
+    const int ny, const int nz, const int cblocks, const unsigned total, const int pieces, const int ring, const int parts,
+    float4_t *__restrict__ partial) {
+  using M = Mfma<__half>;
+  // A ring of `ring` kilobytes and one more for each wavefront, for the rois' gradients, `pieces` of them each; at the end the sums.
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  __shared__ unsigned special;
+  const BrickPlace<LOG_WX> place(p, nx, ny, nz, cblocks, SHARED ? parts : 1, total);
+  if (place.none) return;
+  const int X0 = place.X0, Y0 = place.Y0, Z0 = place.Z0, c_base = place.c_base;
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int bx = wave * kBrickEdge;
+  const int col = lane % 16, quad = lane / 16;
+  const int cells = p.od * p.oh * p.ow, ohw = p.oh * p.ow;
+  const long slab = static_cast<long>(p.C) * cells;
+  const int rows = brick_rows(p);
+  unsigned char *const ring_lds = lds + wave * (ring + 1) * 1024;
+  // the lane's first row of cells (ph = quad) there, of channel col / 8 and plane col % 8 (beyond the last: any, its weights are 0),
+  // in elements; the second is four rows on
+  const int piece = col / 8 * cells + min(col % 8, p.od - 1) * ohw + quad * p.ow;
+
+  // and its places in a roi's tables
+  const int at_x = (X0 + bx + col % 8) * kBrickCells, at_y = (brick_row_y(p) + Y0 + col / 8) * kBrickCells + 2 * quad,
+            at_z = (brick_row_z(p) + Z0 + col % 8) * kBrickCells + quad % 2 * 4;
+  const bool own_block = col / 8 == quad / 2;
+
+  if (threadIdx.x == 0) special = 0;
+  __syncthreads();
+  // the brick's list, or this part of it; a wavefront beyond the last column of bricks has none
+  const long brick = place.brick + wave;
+  int have = wave < place.bricks ? static_cast<int>(lengths[brick]) : 0, begin = 0;
+  if (SHARED) {
+    begin = brick_share(have, place.part, parts);
+    have = brick_share(have, place.part + 1, parts) - begin;
+  }
+  const unsigned *const list = lists + brick * p.R + begin;
+  // [two channels][two rows of voxels]: z = quad % 2 * 4 + r of channel quad / 2 at voxel (y = col / 8, x = col % 8)
+  float4_t acc[kBrickChannels / 2][4];
+  {
+#pragma unroll
+    for (int i = 0; i < kBrickChannels / 2; i++)
+#pragma unroll
+      for (int k = 0; k < 4; k++) acc[i][k] = float4_t{0.f, 0.f, 0.f, 0.f};
+    if (have > 0) {
+      unsigned entries = list[min(lane, have - 1)];   // 64 at a time, one per lane
+      auto entry = [&](const int i) {
+        if (i % kWave == 0 && i > 0) {
+          entries = list[min(i + lane, have - 1)];
+          asm volatile("" : "+v"(entries));   // (a wait here and not where it is used, which would be one for all that is on its way)
+        }
+        return static_cast<unsigned>(__builtin_amdgcn_readlane(entries, i % kWave));
+      };
+      // what a lane needs of a roi's tables: its voxel's row of x, its rows' pairs of y, and four weights of z
+      struct Weights { float4 x0, x1; float2 y[4]; float4 z; };
+      auto fetch = [&](unsigned n, Weights &w) {
+        const float *tab = tables + static_cast<long>(n) * rows * kBrickCells;
+        const float4 *x = reinterpret_cast<const float4 *>(tab + at_x);
+        w.x0 = x[0];
+        w.x1 = x[1];
+#pragma unroll
+        for (int k = 0; k < 4; k++) w.y[k] = *reinterpret_cast<const float2 *>(tab + at_y + 2 * k * kBrickCells);
+        w.z = *reinterpret_cast<const float4 *>(tab + at_z);
+      };
+      // A roi's gradient of the 16 channels is one run of memory.  It comes to LDS as it is, 1024 bytes a load, from the 4-byte
+      // boundary before it; returns the elements between that and its start.
+      // Pieces `from` to `to` of it go to the ring's places from `at` on; the piece that comes to the first place when others are
+      // before it goes behind the last place too, so that what lies across the ring's end can be read in one.
+      struct Run { u32x4 src; int odd; };
+      auto run_of = [&](const unsigned of) {
+        const bool end = of == static_cast<unsigned>(p.R) - 1u;
+        const long from = (end ? 0L : of * slab) + static_cast<long>(c_base) * cells;   // in elements
+        const unsigned char *const start = reinterpret_cast<const unsigned char *>((end ? last : gout) + from);
+        const int odd = static_cast<int>(reinterpret_cast<unsigned long long>(start) & 2);
+        const long behind = (end ? slab * 2 + kBrickPad : p.R * slab * 2) - from * 2 + odd;
+        const unsigned long long base = reinterpret_cast<unsigned long long>(start - odd);
+        return Run{u32x4{static_cast<unsigned>(base), static_cast<unsigned>(base >> 32) & 0xffffu,
+                         static_cast<unsigned>(min(behind, 0x7ffffff0L)), 0x00020000u}, odd};
+      };
+      // (Written out: behind the compiler's own form every read of LDS waits for all the loads that are on their way to it.  The waits
+      // that it places for other loads count these among them, so that they are longer than they need be, never shorter.)
+      const unsigned ring_at = __builtin_amdgcn_readfirstlane(
+          static_cast<unsigned>(reinterpret_cast<unsigned long long>((__attribute__((address_space(3))) unsigned char *)ring_lds)));
+      auto to_lds = [&](const Run &run, const int piece_at, const int place) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     : : "s"(__builtin_amdgcn_readfirstlane(ring_at + place * 1024)), "v"(lane * 16 + piece_at * 1024), "s"(run.src) : "memory");
+      };
+      auto bring = [&](const Run &run, int place, const int from, const int to) {
+#pragma unroll 1
+        for (int i = from; i < to; i++) {
+          to_lds(run, i, place);
+          if (place == 0 && i > 0) to_lds(run, i, ring);
+          place = place + 1 == ring ? 0 : place + 1;
+        }
+        return place;
+      };
+      const int early = min(ring - pieces, pieces);   // pieces that come in before the present roi has been read
+      // Pairs of channels are read four ahead; behind the fourth of the last sweep the next roi's gradient may come in.
+      u32x4 slot[4][2];
+      auto read = [&](unsigned at, const unsigned end, u32x4 (&s)[2]) {   // (a roi begins before the end and is no longer than the ring)
+        typedef unsigned int V __attribute__((ext_vector_type(4), aligned(4)));
+        const unsigned char *const from = ring_lds + min(at, at - end);
+        s[0] = *reinterpret_cast<const V *>(from);
+        s[1] = *reinterpret_cast<const V *>(from + 8 * p.ow);
+      };
+      Weights w;
+      unsigned e = entry(0);
+      fetch(e & ~(kBrickUpper | kBrickLower), w);
+      Run here = run_of(e & ~(kBrickUpper | kBrickLower));
+      int first = 0, next_place = bring(here, 0, 0, pieces);   // in the ring: of the present roi, of the next
+      for (int done = 0; done < have; done++) {
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");   // the gradient is here, and the tables
+        asm volatile("" : "+v"(w.x0.x), "+v"(w.x0.y), "+v"(w.x0.z), "+v"(w.x0.w), "+v"(w.x1.x), "+v"(w.x1.y), "+v"(w.x1.z), "+v"(w.x1.w));
+        asm volatile("" : "+v"(w.y[0].x), "+v"(w.y[0].y), "+v"(w.y[1].x), "+v"(w.y[1].y), "+v"(w.y[2].x), "+v"(w.y[2].y), "+v"(w.y[3].x),
+                          "+v"(w.y[3].y), "+v"(w.z.x), "+v"(w.z.y), "+v"(w.z.z), "+v"(w.z.w));
+        const bool more = done + 1 < have;
+        const unsigned e2 = more ? entry(done + 1) : e, n2 = e2 & ~(kBrickUpper | kBrickLower);
+        const Run run2 = run_of(n2);
+        int first2 = next_place;
+        Weights w2;
+        fetch(n2, w2);
+        if (more) next_place = bring(run2, first2, 0, early);
+        const float ws[4] = {own_block ? w.z.x : 0.f, own_block ? w.z.y : 0.f, own_block ? w.z.z : 0.f, own_block ? w.z.w : 0.f};
+        const BrickLeft left = brick_left(ws);
+        const float xs[8] = {w.x0.x, w.x0.y, w.x0.z, w.x0.w, w.x1.x, w.x1.y, w.x1.z, w.x1.w};
+        const bool half[2] = {(e & kBrickUpper) != 0, (e & kBrickLower) != 0};
+        // (from the 4-byte boundary, and shifted after: 16 bytes at a 2-byte boundary take LDS 60 clocks, 660 instead of 380 us of all)
+        const unsigned at = (piece + here.odd / 2) / 2 * 4 + first * 1024, end = ring * 1024;
+        const unsigned shift = (piece + here.odd / 2) % 2 * 16;
+        const int pair = 4 * cells;   // bytes from two channels to the next
+#pragma unroll
+        for (int h = 0; h < 2; h++) {   // the upper and the lower four rows of the brick
+          if (!half[h]) continue;
+          u32x4 right[2][2];
+#pragma unroll
+          for (int k = 0; k < 2; k++)
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) {
+              const float y = ks == 0 ? w.y[2 * h + k].x : w.y[2 * h + k].y;
+              float f[8];
+#pragma unroll
+              for (int j = 0; j < 8; j++) f[j] = y * xs[j];
+              right[k][ks] = M::pack(f);
+            }
+#pragma unroll
+          for (int i = 0; i < 4; i++) read(at + i * pair, end, slot[i]);
+#pragma unroll
+          for (int i = 0; i < kBrickChannels / 2; i++) {
+            u32x4 g[2];
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++) {
+              const u32x4 v = slot[i % 4][ks];
+              g[ks] = u32x4{__builtin_amdgcn_alignbit(v.y, v.x, shift), __builtin_amdgcn_alignbit(v.z, v.y, shift),
+                            __builtin_amdgcn_alignbit(v.w, v.z, shift), v.w >> shift};
+            }
+            float4_t part[2] = {float4_t{0.f, 0.f, 0.f, 0.f}, float4_t{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+              for (int k = 0; k < 2; k++) part[k] = M::run16(g[ks], right[k][ks], part[k]);
+            if (i < 4) read(at + (i + 4) * pair, end, slot[i]);
+            if (i == 3 && (h == 1 || !half[1])) {
+#pragma unroll
+              for (int j = 0; j < 4; j++) asm volatile("" : "+v"(slot[j][0]), "+v"(slot[j][1]) : : "memory");   // they have been read
+              if (more) next_place = bring(run2, next_place, early, pieces);
+            }
+#pragma unroll
+            for (int k = 0; k < 2; k++) acc[i][2 * h + k] = brick_add(left, part[k], acc[i][2 * h + k]);
+          }
+        }
+        e = e2; w = w2; here = run2; first = first2;
+      }
+    }
+  }
+  if constexpr (SHARED) {
+    if (have == 0) return;
+    float4_t *const to = partial + ((brick * cblocks + c_base / kBrickChannels) * parts + place.part) * (kBrickChannels / 2 * 4 * kWave) + lane;
+#pragma unroll
+    for (int i = 0; i < kBrickChannels / 2; i++)
+#pragma unroll
+      for (int k = 0; k < 4; k++) to[(i * 4 + k) * kWave] = acc[i][k];
+  } else {
+    brick_finish<LOG_WX>(acc, place, gout, recs, tables, grad, p, lds, special);
+  }
+}
+
+// The sums of the parts.
+template <int LOG_WX>
+__global__ __launch_bounds__(kWave << LOG_WX) void roi_brick_fold_kernel(
+    const __half *__restrict__ gout, const BrickRoi *__restrict__ recs, const float *__restrict__ tables,
+    const unsigned *__restrict__ lengths, __half *__restrict__ grad, const RoiProblem p, const int nx, const int ny, const int nz,
+    const int cblocks, const unsigned total, const int parts, const float4_t *__restrict__ partial) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  __shared__ unsigned special;
+  const BrickPlace<LOG_WX> place(p, nx, ny, nz, cblocks, 1, total);
+  if (place.none) return;
+  if (threadIdx.x == 0) special = 0;
+  __syncthreads();
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int have = wave < place.bricks ? static_cast<int>(lengths[place.brick + wave]) : 0;
+  float4_t acc[kBrickChannels / 2][4];
+#pragma unroll
+  for (int i = 0; i < kBrickChannels / 2; i++)
+#pragma unroll
+    for (int k = 0; k < 4; k++) acc[i][k] = float4_t{0.f, 0.f, 0.f, 0.f};
+  const float4_t *from = partial + ((place.brick + wave) * cblocks + place.c_base / kBrickChannels) * parts * (kBrickChannels / 2 * 4 * kWave) + lane;
+  for (int part = 0; part < parts; part++, from += kBrickChannels / 2 * 4 * kWave) {
+    if (brick_share(have, part, parts) == brick_share(have, part + 1, parts)) continue;   // (left nothing)
+#pragma unroll
+    for (int i = 0; i < kBrickChannels / 2; i++)
+#pragma unroll
+      for (int k = 0; k < 4; k++) acc[i][k] += from[(i * 4 + k) * kWave];
+  }
+  brick_finish<LOG_WX>(acc, place, gout, recs, tables, grad, p, lds, special);
+}
+
+static size_t brick_tables_bytes(const RoiProblem &p) {
+  return (static_cast<size_t>(p.R) * brick_rows(p) * kBrickCells * sizeof(float) + 255) / 256 * 256;
+}
+
+static long brick_count(const RoiProblem &p) {
+  return static_cast<long>(p.N) * (brick_up(p.D) / kBrickEdge) * (brick_up(p.H) / kBrickEdge) * (brick_up(p.W) / kBrickEdge);
+}
+static long brick_waves(const RoiProblem &p) { return brick_count(p) * ((p.C + kBrickChannels - 1) / kBrickChannels); }
+
+// Workgroups that share a brick and 16 channels, for maps of fewer than 1024 such pairs whose bricks have many rois each; their sums go
+// through memory (64 KB for each) and another launch.  Forward and backward pass, one workgroup and this many: [4,64,11,27,28] with 3510 rois
+// of 7^3 cells 873 and 435 us, [2,83,24,29,25] with 484 of 4^3 271 and 190; [2,24,35,93,28] with 369 of 2^3, four rois per five bricks, 59 and 66.
+static int brick_parts(const RoiProblem &p) {
+  if (4L * p.R < 5 * brick_count(p)) return 1;
+  return static_cast<int>(std::max(std::min(2048 / brick_waves(p), 16L), 1L));
+}
+
+bool roi_brick_applies(int dtype, const RoiProblem &p) {
+  if (dtype != MV_F16 || p.ndim != 3 || p.od > kBrickCells || p.oh > kBrickCells || p.ow > kBrickCells || !roi_pool_applies(dtype, p)) return false;
+  if (p.D > 0x7fff || p.H > 0x7fff || p.W > 0x7fff) return false;
+  const long slab = static_cast<long>(p.C) * p.od * p.oh * p.ow * 2;   // bytes of a roi's gradient
+  if (slab < kBrickPad || slab + kBrickPad >= (1L << 31)) return false;
+  if (static_cast<long>(p.R) * brick_rows(p) * kBrickCells * 4 >= (1L << 31) || p.R >= (1 << 30)) return false;
+  // Small maps have too few bricks to fill the chip, and few channels leave most of a product idle; there the kernel that adds box by box is
+  // the faster one.  Forward and backward pass there -> here: [1,16,14,40,66] with 163 rois of 7^3 cells (90 bricks) 37 -> 54 us,
+  // [4,36,10,20,26] with 112 (96 bricks) 59 -> 72, [2,19,6,125,50] with 89 of 8^3 (224 bricks) 38 -> 42; [2,16,12,94,77] with 987 (480 bricks) 84 -> 77,
+  // [1,32,18,57,123] with 463 91 -> 83, [2,256,10,64,67] with 363 of 5^3 173 -> 130.  Over 240 heads of 1 - 4000 rois, 1 - 256 channels and up to
+  // 64 x 128 x 128 voxels 1.22 times as fast in geometric mean, the slowest 0.92.
+  return brick_count(p) * p.C >= 7680 && brick_waves(p) * 16 < (1L << 31) - 8;
+}
+
+static size_t brick_lists_bytes(const RoiProblem &p) { return (static_cast<size_t>(brick_count(p)) * (p.R + 1) * 4 + 255) / 256 * 256; }
+static size_t brick_partial_bytes(const RoiProblem &p) {
+  const int parts = brick_parts(p);
+  return parts > 1 ? static_cast<size_t>(brick_waves(p)) * parts * kBrickChannels * 512 * sizeof(float) : 0;
+}
+
+size_t roi_brick_workspace(int dtype, const RoiProblem &p) {
+  if (!roi_brick_applies(dtype, p)) return 0;
+  return brick_tables_bytes(p) + brick_lists_bytes(p) + brick_partial_bytes(p) + static_cast<size_t>(p.R) * sizeof(BrickRoi) +
+         static_cast<size_t>(p.C) * p.od * p.oh * p.ow * 2 + kBrickPad;
+}
+
+// Writes all of grad_input.  -1: not for these kernels, or a workspace that is too small for them.
+int roi_brick_backward(const void *grad_output, const void *rois, void *grad_input, int dtype, const RoiProblem &p, void *workspace,
+                       size_t capacity, hipStream_t s) {
+  if (!roi_brick_applies(dtype, p) || capacity < roi_brick_workspace(dtype, p) || reinterpret_cast<uintptr_t>(workspace) % 16 != 0) return -1;
+  float *const tables = static_cast<float *>(workspace);
+  unsigned *const lists = reinterpret_cast<unsigned *>(static_cast<char *>(workspace) + brick_tables_bytes(p));
+  unsigned *const lengths = lists + brick_count(p) * p.R;
+  float4_t *const partial = reinterpret_cast<float4_t *>(reinterpret_cast<char *>(lists) + brick_lists_bytes(p));
+  BrickRoi *const recs = reinterpret_cast<BrickRoi *>(reinterpret_cast<char *>(partial) + brick_partial_bytes(p));
+  __half *const copy = reinterpret_cast<__half *>(recs + p.R);
+  const int slab = p.C * p.od * p.oh * p.ow;
+  const int copies = (slab + kBrickPad / 2 + 3 * kWave * 8 - 1) / (3 * kWave * 8);
+  // (rows of eight cells have to lie at 4-byte boundaries: what a shift brings in is one cell short of that)
+  if (p.ow == kBrickCells && reinterpret_cast<uintptr_t>(grad_output) % 4 != 0) return -1;
+  // kilobytes of a roi's 16 channels (and behind them: a row of cells may be read as 16 bytes, and rows up to the eighth), and of a
+  // wavefront's ring: as much as lets eight wavefronts share a compute unit's LDS, or one roi's
+  const int pieces = (kBrickChannels * p.od * p.oh * p.ow * 2 + 2 + kBrickPad + 1023) / 1024;
+  const int ring = std::max(std::min(2 * pieces, 18), pieces);
+  const int log_wx = p.W > kBrickEdge ? 1 : 0;
+  const int nx = (p.W + (8 << log_wx) - 1) >> (3 + log_wx), ny = brick_up(p.H) / kBrickEdge, cblocks = (p.C + kBrickChannels - 1) / kBrickChannels;
+  const int nz = brick_up(p.D) / kBrickEdge;
+  const int parts = brick_parts(p);
+  const long regions = static_cast<long>(p.N) * cblocks * nz * ny * nx, total = regions * parts;
+  const float *const r = static_cast<const float *>(rois);
+  const __half *const g = static_cast<const __half *>(grad_output);
+  __half *const grad = static_cast<__half *>(grad_input);
+  const size_t sums = static_cast<size_t>(kBrickChannels) * ((512 << log_wx) + 8) * 2, rings = static_cast<size_t>(ring + 1) * 1024 << log_wx;
+  hipLaunchKernelGGL(roi_brick_tables_kernel, dim3(p.R + copies), dim3(3 * kWave), 0, s, r, recs, tables, p, g + static_cast<long>(p.R - 1) * slab,
+                     copy, slab);
+  hipLaunchKernelGGL(roi_brick_lists_kernel, dim3(static_cast<unsigned>(brick_count(p))), dim3(kBrickThreads), 0, s,
+                     reinterpret_cast<const uint4 *>(recs), lists, lengths, p.R, brick_up(p.W) / kBrickEdge, ny, nz);
+  auto grid = [](long n) { return dim3(static_cast<unsigned>((n + 7) / 8 * 8)); };
+#define MV_BRICK(LOG_WX, SHARED)                                                                                               \
+  hipLaunchKernelGGL((roi_brick_backward_kernel<LOG_WX, SHARED>), grid(total), dim3(kWave << LOG_WX), std::max(sums, rings), s, g, copy, recs, \
+                     tables, lists, lengths, grad, p, nx, ny, nz, cblocks, static_cast<unsigned>(total), pieces, ring, parts, partial)
+#define MV_BRICK_FOLD(LOG_WX)                                                                                                  \
+  hipLaunchKernelGGL((roi_brick_fold_kernel<LOG_WX>), grid(regions), dim3(kWave << LOG_WX), sums, s, g, recs, tables, lengths, grad, p, nx, ny, \
+                     nz, cblocks, static_cast<unsigned>(regions), parts, partial)
+  if (parts == 1) {
+    if (log_wx) MV_BRICK(1, false); else MV_BRICK(0, false);
+  } else if (log_wx) {
+    MV_BRICK(1, true);
+    MV_BRICK_FOLD(1);
+  } else {
+    MV_BRICK(0, true);
+    MV_BRICK_FOLD(0);
+  }
+#undef MV_BRICK
+#undef MV_BRICK_FOLD
+  return check_launch("roi_brick_backward_kernel");
+}
+
+}  // namespace mv

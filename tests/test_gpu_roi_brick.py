@@ -1,0 +1,94 @@
+"""Gradients of fp16 heads of plain boxes on volumes by the voxels' owners (roi_brick_backward.hip): remainders of bricks and
+channels, rows of cells at any alignment, shared bricks, gradients that are not finite, against the fp64 oracle."""
+import pytest
+import torch
+
+from parity import BWD_TOL, assert_close
+import workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+TOL = BWD_TOL[torch.float16]
+
+
+def boxes_of(g, images, size, rois, reach):
+    at = torch.rand(rois, 3, generator=g) * torch.tensor(size[::-1]) * 1.2 - 2.0
+    image = torch.randint(0, images, (rois, 1), generator=g).float()
+    return torch.cat([image, at, at + torch.rand(rois, 3, generator=g) * reach], 1)
+
+
+@pytest.mark.parametrize("images,channels,size,rois,cells,ratio,order,reach", [
+    (2, 128, (9, 17, 33), 60, (7, 7, 7), 2, 1, 12),     # a voxel beyond the bricks on every axis
+    (1, 320, (16, 24, 32), 9, (8, 8, 8), 2, 1, 20),     # whole bricks, rows of eight cells, a gradient that fills its ring
+    (4, 80, (40, 33, 8), 50, (5, 6, 7), 0, 1, 20),      # one brick along x
+    (2, 129, (9, 17, 33), 40, (5, 3, 7), 1, 1, 9),      # odd channels: gradients that start between two words
+    (2, 128, (9, 17, 33), 74, (4, 4, 4), 2, 1, 9),      # one workgroup per brick
+    (2, 128, (9, 17, 33), 300, (4, 4, 4), 2, 1, 9),     # four share one
+    (1, 128, (16, 16, 120), 700, (7, 1, 2), 3, 1, 9),   # the last of seven regions along x is half empty
+    (2, 128, (9, 17, 33), 1100, (2, 2, 2), 1, 1, 6),    # more rois than are tried at a time
+    (2, 144, (20, 30, 30), 20, (3, 5, 2), 2, 0, 14),    # nearest taps
+    (1, 256, (30, 30, 30), 6, (7, 7, 7), 1, 1, 200),    # boxes larger than the map
+    (3, 64, (41, 20, 40), 1, (1, 1, 1), 1, 1, 3),       # one cell
+])
+def test_bricks(oracle, images, channels, size, rois, cells, ratio, order, reach):
+    from medvision_amd.ops.roi_align_nd import roi_align_3d
+    g = wl.gen(sum(size) + rois + channels)
+    boxes = boxes_of(g, images, size, rois, reach)
+    x = torch.zeros(images, channels, *size, dtype=torch.float16, device=DEV, requires_grad=True)
+    out = roi_align_3d(x, boxes.to(DEV), cells, 1.0, ratio, order)
+    gy = torch.randn(out.shape, generator=g).half()
+    want = oracle.roi_align_backward(gy, boxes, x.shape, 1.0, ratio, True, order, False).reshape(x.shape)
+    # gradients at a word's start and between two words
+    for shift in (0, 1):
+        room = torch.zeros(gy.numel() + 1, dtype=torch.float16, device=DEV)
+        room[shift:shift + gy.numel()] = gy.flatten().to(DEV)
+        assert_close(torch.autograd.grad(out, x, room[shift:shift + gy.numel()].view(gy.shape), retain_graph=True)[0], want, TOL, f"shift {shift}")
+    # an infinite gradient reaches the voxels of its cell alone
+    gy[0, 0].view(-1)[0] = float("inf")
+    unit = torch.zeros(out.shape)
+    unit[0, 0].view(-1)[0] = 1.0
+    # (weights are rounded to 11 bits, 2^-25 at the least)
+    hit = oracle.roi_align_backward(unit, boxes, x.shape, 1.0, ratio, True, order, False).reshape(x.shape) > 1e-6
+    got = torch.autograd.grad(out, x, gy.to(DEV))[0].cpu().double()
+    assert not torch.isfinite(got[hit]).any()
+    assert_close(torch.where(hit, want, got), want, TOL, "finite part")
+
+
+def test_sums_beyond_fp16(oracle):
+    """Cells far smaller than a voxel: sums over y and x of gradients near the type's largest, which no fp16 number holds."""
+    from medvision_amd.ops.roi_align_nd import roi_align_3d
+    g = wl.gen(5)
+    size = (9, 17, 33)
+    at = torch.rand(6, 3, generator=g) * 6 + 1
+    boxes = torch.cat([torch.zeros(6, 1), at, at + 0.1], 1)
+    x = torch.zeros(2, 128, *size, dtype=torch.float16, device=DEV, requires_grad=True)
+    out = roi_align_3d(x, boxes.to(DEV), (7, 7, 7), 1.0, 2, 1)
+    gy = (torch.randn(out.shape, generator=g) * 3000).half()
+    want = oracle.roi_align_backward(gy, boxes, x.shape, 1.0, 2, True, 1, False).reshape(x.shape)
+    got = torch.autograd.grad(out, x, gy.to(DEV))[0].cpu().double()
+    fits = want.abs() < 60000
+    assert bool((got[~fits].abs() > 59000).all())
+    assert_close(torch.where(fits, got, want), want, TOL, "gradient")
+
+
+def test_keeps_to_its_workspace(oracle):
+    """With the room that the query asks for, and with the room that the older kernels need, which then run."""
+    from medvision_amd import _lib
+    lib, code = _lib.load(), _lib.MV_F16
+    g = wl.gen(3)
+    dims, rois, cells = (2, 128, 9, 17, 33), 300, 7
+    boxes = boxes_of(g, 2, dims[2:], rois, 9)
+    gy = torch.randn(rois, dims[1], cells, cells, cells, generator=g).half()
+    want = oracle.roi_align_backward(gy, boxes, dims, 1.0, 2, True, 1, False)
+    size = (code, 3, 0, *dims, rois, cells, cells, cells, 2, 1)
+    full, shared = lib.mv_roi_align_backward_write_workspace_bytes(*size), lib.mv_roi_align_backward_workspace_bytes(code, *dims)
+    assert full > shared
+    grad, d_gy, d_rois = torch.full(dims, 7.0, dtype=torch.float16, device=DEV), gy.to(DEV), boxes.to(DEV)
+    for given in (shared, full):
+        room = torch.full((full + 4096,), 0x5a, dtype=torch.uint8, device=DEV)
+        grad.fill_(7.0)
+        _lib.check(lib.mv_roi_align_backward_replace(_lib.ptr(d_gy), _lib.ptr(d_rois), _lib.ptr(grad), code, 3, 0, *dims, rois, cells, cells, cells,
+                                                     1.0, 2, 1, 1, _lib.ptr(room), given, _lib.stream_of(grad)))
+        assert bool((room[given:] == 0x5a).all())
+        assert_close(grad, want, TOL, f"{given} bytes")
