@@ -1,5 +1,5 @@
-// Matrix-core forward of deformable layers on large volumes with 32 or 64 channels per group (16-bit tensors): the taps are
-// worked out once per position and shared through LDS.  (dcn_forward_columns.hip: every other layer, the layouts of x and the
+// Matrix-core forward of deformable layers on large volumes with 32 (fp16: or 64) channels and 64 output channels per group (16-bit
+// tensors): the taps are worked out once per position and shared through LDS.  (dcn_forward_columns.hip: every other layer, the layouts of x and the
 // weights, and the plan that both share.)
 #include <cstdint>
 
@@ -49,10 +49,7 @@ __global__ __launch_bounds__(256, 5) void dcn_forward_shared_taps_kernel(
     const int ow = w0 + l % 8, oh = h0 + (l / 8) % bhy, od = d0 + l / (8 * bhy);
     return (ow < s.Wo && oh < s.Ho && od < s.Do) ? (static_cast<long>(od) * s.Ho + oh) * s.Wo + ow : -1;
   };
-  const int blocks = s.opg / 16;
-  const int chunks = (blocks + MB - 1) / MB;
-  const int g = blockIdx.y / chunks, mb0 = (blockIdx.y % chunks) * MB;
-  const int b = blockIdx.z;
+  const int g = blockIdx.y, b = blockIdx.z;
   const int dgi = g * s.cpg / s.cpd;
   const long bg = static_cast<long>(b) * s.dg + dgi;
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
@@ -92,14 +89,13 @@ __global__ __launch_bounds__(256, 5) void dcn_forward_shared_taps_kernel(
   // (in wf [block][tap][slice][lane]; taps beyond the last one are loaded and not used)
   constexpr int tap_bytes = SLICES * 64 * 16;
   const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<T *>(wf + static_cast<long>(g) * blocks * s.K * SLICES * (64 * PC)), 0, blocks * s.K * tap_bytes, 0x00020000);
+      const_cast<T *>(wf + static_cast<long>(g) * MB * s.K * SLICES * (64 * PC)), 0, MB * s.K * tap_bytes, 0x00020000);
   unsigned wsrc[WREG];
 #pragma unroll
   for (int i = 0; i < WREG; i++) {
     const int id = i * 256 + tid, t = id / WT, rem = id % WT;
     const int ln = rem % 64, m = (rem / 64) % MB, cc = rem / (64 * MB);
-    wsrc[i] = (id < TG * WT && mb0 + m < blocks) ? static_cast<unsigned>((((mb0 + m) * s.K + t) * SLICES + cc) * 1024 + ln * 16)
-                                                 : kOutside;
+    wsrc[i] = id < TG * WT ? static_cast<unsigned>(((m * s.K + t) * SLICES + cc) * 1024 + ln * 16) : kOutside;
   }
 
   float4_t acc[MB];
@@ -207,40 +203,42 @@ __global__ __launch_bounds__(256, 5) void dcn_forward_shared_taps_kernel(
   u32x2 braw[MB];
 #pragma unroll
   for (int m = 0; m < MB; m++)
-    braw[m] = __builtin_amdgcn_raw_buffer_load_b64(br, (g * s.opg + (mb0 + m) * 16 + kc * 4) * ES, 0, 0);
+    braw[m] = __builtin_amdgcn_raw_buffer_load_b64(br, (g * s.opg + m * 16 + kc * 4) * ES, 0, 0);
 #pragma unroll
   for (int m = 0; m < MB; m++) {
-    if (mb0 + m >= blocks) continue;
     const float bv[4] = {M::lo(braw[m].x), M::hi(braw[m].x), M::lo(braw[m].y), M::hi(braw[m].y)};
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      const int o = g * s.opg + (mb0 + m) * 16 + kc * 4 + r;
+      const int o = g * s.opg + m * 16 + kc * 4 + r;
       y[(static_cast<long>(b) * s.Cout + o) * s.Q + qo] = store_cast<T>(acc[m][r] + bv[r]);
     }
   }
 }
 
 // The layers that this kernel serves: volumes of many bricks (below four workgroups per compute unit the columns
-// kernel's smaller ones win: 44 us against 30 us for fp16 [4, 64 -> 64, 16 x 38 x 26], stride 2), all of a group's channels in one or
-// two slices of one deformable group, at least 64 output channels.  There it is the faster one: fp16 [2, 32 -> 64, 48^3] 159 us
-// against 185 us.
+// kernel's smaller ones win: 44 us against 30 us for fp16 [4, 64 -> 64, 16 x 38 x 26], stride 2), all of a group's channels in one
+// slice (fp16: or two) of one deformable group, and 64 output channels.  There it is the faster one: fp16 [2, 32 -> 64, 32^3] 57 us
+// against 64 us, bf16 55 and 63, fp16 [64 -> 64, 48^3] 152 and 159.  It repeats the samples for every 64 output channels, which the columns
+// kernel shares among 256 (bf16 [2, 32 -> 128, 32^3] 95 against 78 us, fp16 [2, 64 -> 256, 32^3] 279 and 162); bf16 with 64 channels leaves
+// it three wavefronts per SIMD (64 -> 64 48^3 192 against 167 us); and its bricks have to be full (fp16 [2, 32 -> 64, 37 x 29 x 33],
+// 73 % of the positions alive: 73 against 69 us; 64 -> 64 120 and 107; [4, 64 -> 64, 9 x 45 x 51], 77 %: 136 and 124).
 int dcn_shared_taps_forward(const void *xt, const void *off, const void *mask, const void *wf, const void *bias, void *y,
                             const DcnDims &s, int dtype, hipStream_t stream) {
-  const int slices = s.cpg / 32, blocks = s.opg / 16, chunks = (blocks + 3) / 4;
+  const int slices = s.cpg / 32;
   // bricks of 8 x 4 x 2 output voxels (8 x 8 of a single slice), one per workgroup
   const int bdz = s.Do > 1 ? 2 : 1, bhy = 8 / bdz;
   const long bricks = static_cast<long>((s.Wo + 7) / 8) * ((s.Ho + bhy - 1) / bhy) * ((s.Do + bdz - 1) / bdz);
-  if (s.nd != 3 || s.cpg % 32 || slices < 1 || slices > 2 || s.cpd % s.cpg || blocks < 4 || bricks * s.B < 1024 || bricks >= (1L << 31) ||
-      static_cast<long>(s.groups) * chunks > 65535 || 3L * s.K * s.Q * 2 >= (1L << 31) ||
-      static_cast<long>(s.K) * slices * blocks * 1024 >= (1L << 31))
+  if (s.nd != 3 || s.cpg % 32 || slices < 1 || slices > (dtype == MV_F16 ? 2 : 1) || s.cpd % s.cpg || s.opg != 64 || bricks * s.B < 1024 ||
+      s.Q * 20 < bricks * (64 * 17) || bricks >= (1L << 31) || s.groups > 65535 || 3L * s.K * s.Q * 2 >= (1L << 31) ||
+      static_cast<long>(s.K) * slices * 4 * 1024 >= (1L << 31))
     return -1;
-  const dim3 grid(static_cast<unsigned>(bricks), s.groups * chunks, s.B), block(256);
+  const dim3 grid(static_cast<unsigned>(bricks), s.groups, s.B), block(256);
 #define MV_SHARED_TAPS(T, SLICES)                                                                                     \
   hipLaunchKernelGGL((dcn_forward_shared_taps_kernel<T, SLICES>), grid, block, 0, stream, static_cast<const T *>(xt), \
                      static_cast<const T *>(off), static_cast<const T *>(mask), static_cast<const T *>(wf),           \
                      static_cast<const T *>(bias), static_cast<T *>(y), s)
   if (dtype == MV_F16) { if (slices == 1) MV_SHARED_TAPS(__half, 1); else MV_SHARED_TAPS(__half, 2); }
-  else { if (slices == 1) MV_SHARED_TAPS(__hip_bfloat16, 1); else MV_SHARED_TAPS(__hip_bfloat16, 2); }
+  else MV_SHARED_TAPS(__hip_bfloat16, 1);
 #undef MV_SHARED_TAPS
   return check_launch("dcn_forward_shared_taps_kernel");
 }

@@ -11,21 +11,26 @@
 // lanes of a position fetch four neighbouring pieces, usually one cache line, together.  Weights in fragment order
 // (workspace): a wavefront's operand is one coalesced 16-byte load per lane.
 //
-// Workgroup = PT positions x up to 64 * OBW output channels, four wavefronts:
+// Workgroup = PT positions x up to 16 * W * OBW output channels, W wavefronts:
 //   records   a thread works out one (unit, position): the corners' byte offsets and weights (times the mask) go
-//             to LDS, 256 of them at a time; a unit is a tap of one deformable group.  Their offsets are requested a window ahead.
-//   samples   an item = 16 positions x 4 pieces: load, blend, write the piece to LDS.  The corners of the next item are on
+//             to LDS, 64 * W of them at a time; a unit is a tap of one deformable group.  Their offsets are requested a window ahead.
+//   samples   an item = 64 / LP positions x LP pieces: load, blend, write the piece to LDS.  The corners of the next item are on
 //             their way while one is blended, also across the product in between.
 //   product   16 pieces of K against the wavefront's rows of the weight, v_mfma_f32_16x16x32 (fp32: 16x16x4).
-// PT: 32 positions use a weight fragment twice; 16 give a layer of a few thousand positions twice the workgroups, whose
-// wavefronts then share the positions and split the pieces.  (64 positions: no faster for wide layers, 165 us against
-// 134 us for bf16 [2, 128 -> 64, 50 x 37 x 13].)
-// What bounds it: the cache look-ups of the corners (64 bytes a clock; 256 -> 256 channels: texture addressers 74 % busy, vector
-// issue 34 %, matrix cores 24 %), narrow layers the blend too (a multiply-add per channel and corner); small layers the latency of
-// the chain load - blend - product.
-//   (Images fp16 [8, 256 -> 256, 100 x 152]: 566 us with 16 positions per wavefront and the weights through LDS, 283 us now;
+// LP: the cache takes a load by the 128-byte lines that it touches (4.6 clocks each when they come from the L2, whatever is read of them), so
+// eight neighbouring lanes read a whole line of a corner where its channels are that many (fp16 [8, 256 -> 256, 100 x 152] 274 -> 249 us
+// with 64 positions, fp16 [2, 128 -> 64, 24^3] 98 -> 90, fp32 243 -> 217); four, half a line, elsewhere.
+// PT, W: 32 positions use a weight fragment twice; 16 give a layer of a few thousand positions twice the workgroups, whose
+// wavefronts then share the positions and split the pieces.  Wide images take 64 positions and eight wavefronts, which halves the reads of the
+// weights, two thirds of the cache's work ([8, 256 -> 256, 100 x 152] fp16 298 -> 274 us, with LP = 8 299 -> 245; fp32, batch 4,
+// 715 -> 648); the rule is at the launch.  (128 positions of sixteen wavefronts: 292 us, one workgroup per compute unit waits at
+// its barriers; volumes, whose eight corners leave too few registers, fp16 [128 -> 256, 16 x 16 x 90] 127 us with 32 positions and 139 with 64.)
+// What bounds it: the look-ups of the corners and weights in the vector caches, narrow layers the blend too (a multiply-add per channel and
+// corner); small layers the latency of the chain load - blend - product.
+//   (Images fp16 [8, 256 -> 256, 100 x 152]: 566 us with 16 positions per wavefront and the weights through LDS;
 //   bf16 [4, 256 -> 64, 121 x 21] stride 2: 83 us, 21 us now; bf16 [1, 128 -> 32, 6 x 22 x 34]: 100 us, 30 us now.)
 #include "dcn_mfma.hpp"
+#include <algorithm>
 
 namespace mv {
 
@@ -83,24 +88,26 @@ __global__ __launch_bounds__(256) void dcn_columns_layout_kernel(const U *__rest
 // ---- the layer ---------------------------------------------------------------------------------------------------------
 constexpr int kColPieces = 16;   // pieces of a product: four K steps
 
-template <typename T, int NC, int PT, int OBW>
-__global__ __launch_bounds__(256, OBW == 4 && (PT == 32 || NC == 8) ? 2 : (OBW == 1 ? 4 : 3)) void dcn_forward_columns_kernel(
+template <typename T, int NC, int PT, int OBW, int W, int LP>
+__global__ __launch_bounds__(kWave * W, W == 8 ? 4 : OBW == 4 && (PT == 32 || NC == 8) ? 2 : (OBW == 1 ? 4 : 3)) void dcn_forward_columns_kernel(
     const T *__restrict__ xt, const T *__restrict__ off, const T *__restrict__ mask, const T *__restrict__ wf,
     const T *__restrict__ bias, T *__restrict__ y, const DcnDims s) {
   using M = Mfma<T>;
   using P = typename std::conditional<(sizeof(T) == 2), float, double>::type;  // position type
-  constexpr int PC = M::kPiece, ES = sizeof(T), PG = PT / 16, TG = 256 / PT;   // position groups; units of a window
+  constexpr int PC = M::kPiece, ES = sizeof(T), PG = PT / 16, TG = kWave * W / PT;   // position groups; units of a window
   constexpr int PIECES = kColPieces, KS = PIECES / 4;
-  constexpr int ITEMS = KS * PG / 4;                                           // items of a wavefront per product
+  constexpr int ITEMS = KS * PG / W;                                           // items of a wavefront per product
   constexpr unsigned kOutside = 0x80000000u;                                   // beyond the buffer: such loads return zeros
-  constexpr int RW = 2 * NC + 4, PITCH = PT + 4;   // (records 4 dwords further apart than they are long: banks)
+  constexpr int RW = 2 * NC + 4, PITCH = PT + (LP == 8 ? 1 : 4);   // (records 4 dwords further apart than they are long, a position's pieces: banks)
+  constexpr int LG = PT * LP / kWave, LS = W / LG;   // items side by side on the positions; groups of LP pieces a wavefront is on at a time
+  static_assert(LG * LS == W && ITEMS * W * kWave == PT * kColPieces && kColPieces % (LS * LP) == 0, "items of a product are shared out evenly");
   __shared__ __attribute__((aligned(16))) unsigned rec[TG * PT][RW];           // [unit][position]: at[NC], mask * w[NC]
   __shared__ u32x4 col[2][PIECES * PITCH];                                 // [piece][position]
   const int tid = threadIdx.x, lane = tid % kWave, wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int j = lane % 16, kc = lane / 16;   // matrix layout
-  const int lj = lane / 4, lk = lane % 4;    // load layout
-  const int row_chunks = (s.opg + 64 * OBW - 1) / (64 * OBW);
-  const int g = blockIdx.y / row_chunks, row0 = blockIdx.y % row_chunks * (64 * OBW), b = blockIdx.z;
+  const int lj = lane / LP, lk = lane % LP;  // load layout
+  const int row_chunks = (s.opg + 16 * W * OBW - 1) / (16 * W * OBW);
+  const int g = blockIdx.y / row_chunks, row0 = blockIdx.y % row_chunks * (16 * W * OBW), b = blockIdx.z;
   // (an XCD takes a contiguous eighth of the positions: its L2 then holds an eighth of the input and the offsets' reach)
   const long q0 = static_cast<long>(xcd_contiguous(blockIdx.x, gridDim.x)) * PT;
   const int dgn = s.cpd < s.cpg ? s.cpg / s.cpd : 1, dg0 = g * s.cpg / s.cpd;
@@ -142,16 +149,16 @@ __global__ __launch_bounds__(256, OBW == 4 && (PT == 32 || NC == 8) ? 2 : (OBW =
     }
   };
 
-  // ---- samples: item i of a product: slot = wave + 4 i, positions 16 * (slot % PG), quadruple slot / PG of the product's pieces;
-  // a wavefront's items form one sequence over the window, 4 / PG quadruples apart ------------------------------------
-  const int p = wave % PG * 16 + lj;         // (slot % PG is the same for all of them)
-  const bool whole = up % 4 == 0;            // a quadruple belongs to one unit
-  const int quads = up / 4;                  // per unit (`whole`)
+  // ---- samples: item i of a product: slot = wave + W i, positions 64 / LP * (slot % LG), group slot / LG of LP pieces of the
+  // product; a wavefront's items form one sequence over the window, LS groups apart -----------------------------------
+  const int p = wave % LG * (kWave / LP) + lj;   // (slot % LG is the same for all of them)
+  const bool whole = LP == 8 || up % 4 == 0;     // a group of pieces belongs to one unit
+  const int per_unit = up / LP;              // (`whole`)
   // (division by the pieces of a unit: the high half of a product, exact while piece * up < 2^32)
   const unsigned magic = up == 1 ? 0u : 0xffffffffu / static_cast<unsigned>(up) + 1u;
   u32x4 raw[NC];
   const unsigned *rnow = nullptr;            // the record of the item on its way
-  int nu = 0, nr = 0;                        // the next item: unit of the window and quadruple of it (`whole`), or quadruple of the window
+  int nu = 0, nr = 0;                        // the next item: unit of the window and group of it (`whole`), or group of the window
   auto gather = [&](int window, int limit) {
     unsigned add;
     int scalar_add = g * s.cpg * ES;
@@ -159,16 +166,16 @@ __global__ __launch_bounds__(256, OBW == 4 && (PT == 32 || NC == 8) ? 2 : (OBW =
       const int u = min(nu, min(TG, units - window) - 1);   // (past the last one: loaded for nothing)
       rnow = rec[u * PT + p];
       add = static_cast<unsigned>(lk) * 16u;
-      scalar_add += nr * 64;
+      scalar_add += nr * (16 * LP);
       if (dgn > 1) scalar_add += (window + u) % dgn * (s.cpd * ES);
-      nr += 4 / PG;
-      while (nr >= quads) { nr -= quads; nu++; }
+      nr += LS;
+      while (nr >= per_unit) { nr -= per_unit; nu++; }
     } else {
       const int piece = min(nr * 4 + lk, limit - 1);
       const int u = up == 1 ? piece : static_cast<int>(__umulhi(static_cast<unsigned>(piece), magic)), r = piece - u * up;
       rnow = rec[u * PT + p];
       add = static_cast<unsigned>((dgn == 1 ? r * PC : (window + u) % dgn * s.cpd + r * PC) * ES);
-      nr += 4 / PG;
+      nr += LS;
     }
 #pragma unroll
     for (int c = 0; c < NC; c += 4) {
@@ -179,7 +186,7 @@ __global__ __launch_bounds__(256, OBW == 4 && (PT == 32 || NC == 8) ? 2 : (OBW =
   };
   // `left`: pieces of the window from this product's first one on
   auto blend = [&](int left, int i, u32x4 *to) {
-    const int piece = (wave / PG + i * (4 / PG)) * 4 + lk;
+    const int piece = (wave / LG + i * LS) * LP + lk;
     float v[PC];
 #pragma unroll
     for (int e = 0; e < PC; e++) v[e] = 0.f;
@@ -202,7 +209,7 @@ __global__ __launch_bounds__(256, OBW == 4 && (PT == 32 || NC == 8) ? 2 : (OBW =
   const T *wsrc[OBW];
 #pragma unroll
   for (int o = 0; o < OBW; o++)   // (blocks beyond the last one repeat it; their products are not used)
-    wsrc[o] = wf + (static_cast<long>(g) * blocks + min(row0 / 16 + o * 4 + wave, blocks - 1)) * steps_all * (64 * PC) + lane * PC;
+    wsrc[o] = wf + (static_cast<long>(g) * blocks + min(row0 / 16 + o * W + wave, blocks - 1)) * steps_all * (64 * PC) + lane * PC;
 
   request(0);
   int buf = 0;
@@ -213,8 +220,8 @@ __global__ __launch_bounds__(256, OBW == 4 && (PT == 32 || NC == 8) ? 2 : (OBW =
     __syncthreads();
     const int limit = min(TG, units - window) * up, step0 = window * up / 4;   // (TG is a multiple of four)
     nu = 0;
-    nr = wave / PG;
-    if (whole) while (nr >= quads) { nr -= quads; nu++; }
+    nr = wave / LG;
+    if (whole) while (nr >= per_unit) { nr -= per_unit; nu++; }
     gather(window, limit);
     for (int first = 0; first < limit; first += PIECES) {
       u32x4 a[OBW][KS];
@@ -244,7 +251,7 @@ __global__ __launch_bounds__(256, OBW == 4 && (PT == 32 || NC == 8) ? 2 : (OBW =
   // accumulator register r of lane l: output channel 4 * (l / 16) + r of its block, position l % 16 of its group
 #pragma unroll
   for (int o = 0; o < OBW; o++) {
-    const int row = row0 + (o * 4 + wave) * 16 + 4 * kc;
+    const int row = row0 + (o * W + wave) * 16 + 4 * kc;
     if (row >= s.opg) continue;
     float bv[4];
 #pragma unroll
@@ -308,23 +315,42 @@ static int columns_run(const void *x, const void *off, const void *mask, const v
   auto groups_of = [&](int p, int o) { return (s.Q + p - 1) / p * s.B * s.groups * ((s.opg + 64 * o - 1) / (64 * o)); };
   if (groups_of(pt, obw) < 512) pt = 16;
   while (obw > 1 && groups_of(pt, obw) < 256) obw /= 2;
+  // 16-byte pieces of a corner that a load takes from each position: eight, whole 128-byte lines, where a unit's channels allow it.
+  const bool eights = std::min(s.cpd, s.cpg) % (8 * Mfma<T>::kPiece) == 0;
+  // Wide images: 64 positions and eight wavefronts per workgroup, as long as enough of them remain.  Their time goes in steps of 256
+  // workgroups: fp16 [256 -> 256, 64 x n] 44 against 40 us with n = 128, 46 and 51 with 160, 49 and 65 with 224, 66 and 64 with 300, 68 and 88 with 450,
+  // 100 and 119 with 700; fp32, bound by its products too, 326 and 277 us with 350, 330 and 367 with 450, 489 and 452 with 520, 494 and 537 with 700.
+  const bool wide = NC == 4 && s.opg > 128 && groups_of(64, 4) >= (sizeof(T) == 2 ? 160 : 640);
+  if (wide) pt = 64;
   const long qblocks = (s.Q + pt - 1) / pt;
   const long rows = static_cast<long>(s.groups) * ((s.opg + 64 * obw - 1) / (64 * obw));
   MV_REQUIRE(qblocks < (1L << 31) && rows <= 65535, "grid too large");
-  const dim3 grid(static_cast<unsigned>(qblocks), static_cast<unsigned>(rows), s.B), block(256);
-#define MV_COLUMNS(PTV, OBWV)                                                                                          \
-  hipLaunchKernelGGL((dcn_forward_columns_kernel<T, NC, PTV, OBWV>), grid, block, 0, stream, xt, static_cast<const T *>(off), \
-                     static_cast<const T *>(mask), wf, static_cast<const T *>(bias), static_cast<T *>(y), s)
+  const dim3 grid(static_cast<unsigned>(qblocks), static_cast<unsigned>(rows), s.B);
+#define MV_COLUMNS_LP(PTV, OBWV, WV, LPV)                                                                              \
+  hipLaunchKernelGGL((dcn_forward_columns_kernel<T, NC, PTV, OBWV, WV, LPV>), grid, dim3(kWave * WV), 0, stream, xt,     \
+                     static_cast<const T *>(off), static_cast<const T *>(mask), wf, static_cast<const T *>(bias), static_cast<T *>(y), s)
+#define MV_COLUMNS(PTV, OBWV, WV)                                                                                      \
+  do {                                                                                                                 \
+    if (eights) MV_COLUMNS_LP(PTV, OBWV, WV, 8);                                                                       \
+    else MV_COLUMNS_LP(PTV, OBWV, WV, 4);                                                                              \
+  } while (0)
 #define MV_COLUMNS_PT(PTV)                                                                                             \
   do {                                                                                                                 \
-    if (obw == 1) MV_COLUMNS(PTV, 1);                                                                                  \
-    else if (obw == 2) MV_COLUMNS(PTV, 2);                                                                             \
-    else MV_COLUMNS(PTV, 4);                                                                                           \
+    if (obw == 1) MV_COLUMNS(PTV, 1, 4);                                                                               \
+    else if (obw == 2) MV_COLUMNS(PTV, 2, 4);                                                                          \
+    else MV_COLUMNS(PTV, 4, 4);                                                                                        \
   } while (0)
-  if (pt == 32) MV_COLUMNS_PT(32);
-  else MV_COLUMNS_PT(16);
+  bool launched = false;
+  if constexpr (NC == 4) {
+    if (wide) { MV_COLUMNS(64, 2, 8); launched = true; }
+  }
+  if (!launched) {
+    if (pt == 32) MV_COLUMNS_PT(32);
+    else MV_COLUMNS_PT(16);
+  }
 #undef MV_COLUMNS_PT
 #undef MV_COLUMNS
+#undef MV_COLUMNS_LP
   return check_launch("dcn_forward_columns_kernel");
 }
 

@@ -104,3 +104,26 @@ def test_offset_gradient_of_nearly_equal_corners(oracle, cin, cout, size):
     largest = (terms.reshape(1, taps, *size) * delta)[(slice(None), slice(None), *inside[2:])]
     worst = float((((got - want).abs() - 2.0 ** -11 * want.abs()) / largest).max())
     assert worst <= 2.0 ** -22, worst
+
+
+@pytest.mark.parametrize("dtype,batch,cin,cout,size,groups,dg", [
+    (torch.float16, 1, 64, 144, (101, 103), 1, 1),      # 64 positions, rows of 256 with a remainder, a last tile of 35 positions
+    (torch.bfloat16, 2, 128, 272, (73, 71), 1, 2),      # two passes over the rows, a unit of one line
+    (torch.float16, 1, 80, 144, (103, 101), 1, 1),      # units of ten pieces: no whole lines
+    (torch.float32, 1, 32, 144, (203, 202), 1, 1),
+    (torch.float16, 1, 64, 32, (5, 7, 11), 1, 1),       # 16 positions
+    (torch.float32, 2, 96, 160, (6, 9, 11), 1, 3),
+    (torch.bfloat16, 2, 128, 96, (9, 33, 30), 2, 1),    # 32 positions, groups of 48 rows
+])
+def test_columns_of_whole_lines(oracle, dtype, batch, cin, cout, size, groups, dg):
+    """Corners read by whole cache lines (units of 128 bytes and multiples) and by halves, tiles of 16, 32 and 64 positions."""
+    if len(size) == 3:
+        from medvision_amd.ops.modulated_deform_conv_3d import modulated_deform_conv
+    else:
+        from medvision_amd.ops.modulated_deform_conv_2d import modulated_deform_conv
+    g = wl.gen(cin + cout + sum(size))
+    x, off, mask, w, b = wl.dcn_inputs(g, batch, cin, cout, size, 3, dg, groups, dtype, 1, 1, 1)
+    off = off * 1.5
+    with torch.no_grad():
+        y = modulated_deform_conv(*[t.to(DEV) for t in (x, off, mask, w, b)], 1, 1, 1, groups, dg)
+    assert_close(y, oracle.dcn3d_forward(x, off, mask, w, b, 1, 1, 1, groups, dg), FWD_TOL[dtype], "forward")
