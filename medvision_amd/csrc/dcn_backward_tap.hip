@@ -25,7 +25,8 @@
 // (35 %; vector issue 31 %, matrix cores 21 %) and the same waits (49 %), and everywhere the atomics of the far corners (64 bytes per corner
 // and 16 channels, 21 G of them a second at best).
 //   (bf16 [2, 32 -> 64, 48^3]: 390 us; the data and weight kernels before it took 670 us.  fp16 images
-//   [8, 256 -> 256, 100 x 152]: 587 us, 4380 us before.  [1, 128 -> 128, 7 x 45 x 18]: 60 us, 790 us before.)
+//   [8, 256 -> 256, 100 x 152]: 538 us, 587 with
+//   grad_output of a tile loaded when it begins, 4380 before.  [1, 128 -> 128, 7 x 45 x 18]: 60 us, 790 us before.)
 #include "dcn_scatter.hpp"
 
 #include <algorithm>
@@ -130,7 +131,8 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
     for (int st = 0; st < STEPS; st++)
       wreg[w][st] = st < steps ? *reinterpret_cast<const u32x4 *>(src + st * (64 * PC)) : u32x4{0u, 0u, 0u, 0u};
   }
-  // grad_output of a tile, loaded a tile ahead where the registers allow it: thread t has piece t % NP of positions t / NP +
+  // grad_output of a tile, loaded a tile ahead where the registers allow it, elsewhere during the tile's last product, when those of the
+  // corners are free (loads at the start of the tile had nothing to hide behind: the step above 1456 -> 1407 us): thread t has piece t % NP of positions t / NP +
   // u * 256 / NP (positions and rows that do not exist: zeros)
   constexpr bool AHEAD = STAGED <= 4;
   constexpr int NP = ROWS / PC;
@@ -208,12 +210,11 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
     else if (lk + s.nd >= 3) tout = goff + (bg * s.nd * s.K + s.nd * k + lk + s.nd - 3) * s.Q + q0 + p;
   }
   if (tid < kRecs) request(0);
-  if (AHEAD) stage(0);
+  stage(0);
   const int tiles = (count + kTapTile - 1) / kTapTile;
   for (int tile = 0; tile < tiles; tile++) {
     const int half = tile & 1;
     __syncthreads();   // the tile before has been read
-    if (!AHEAD) stage(tile);
     keep();
     if (half == 0 && tid < kRecs) {
       publish(tile * kTapTile);
@@ -323,6 +324,18 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
     }
 #undef MV_QUAD
     __syncthreads();   // the tile's column values are complete
+    // ---- far corners: 32 lanes add an entry's channels, 32 at a time -------------------------------------------------
+    const int far = __builtin_amdgcn_readfirstlane(far_count[half]), n = tid % 32;
+    for (int i = tid / 32; i < far; i += 8) {
+      const uint2 entry = far_list[half][i];
+      const float w = __uint_as_float(entry.y);
+      const float *src = gcol[entry.x & 63u];
+      const unsigned base = (entry.x & ~127u) + static_cast<unsigned>(c0 + n) * 4u;
+#pragma unroll
+      for (int c = 0; c < CW; c += 32)
+        __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(w * src[c + n], gr, base + c * 4u, 0, 0);
+    }
+    if (!AHEAD) stage(tile + 1);   // (beyond the last one: zeros)
     // ---- gw += gy col^T, a quarter of the rows per wavefront -------------------------------------------------------
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) {
@@ -335,17 +348,6 @@ __global__ __launch_bounds__(256, (TAP_WAVES<T, NC, OBW, CBW>)) void dcn_backwar
 #pragma unroll
         for (int o = 0; o < OBW; o++) acc[o][c] = M::run16(a[o], bf, acc[o][c]);
       }
-    }
-    // ---- far corners: 32 lanes add an entry's channels, 32 at a time -------------------------------------------------
-    const int far = __builtin_amdgcn_readfirstlane(far_count[half]), n = tid % 32;
-    for (int i = tid / 32; i < far; i += 8) {
-      const uint2 entry = far_list[half][i];
-      const float w = __uint_as_float(entry.y);
-      const float *src = gcol[entry.x & 63u];
-      const unsigned base = (entry.x & ~127u) + static_cast<unsigned>(c0 + n) * 4u;
-#pragma unroll
-      for (int c = 0; c < CW; c += 32)
-        __builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(w * src[c + n], gr, base + c * 4u, 0, 0);
     }
   }
   // accumulator register r of lane l: output channel 4 * (l / 16) + r of its block, input channel l % 16
