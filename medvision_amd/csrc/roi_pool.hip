@@ -54,12 +54,13 @@ struct PoolShared {
 // The tap entries of one output cell (grid <= kTapRegs samples) in registers; unused entries have
 // weight 0 and index 0.
 constexpr int kTapRegs = 2;
-struct TapRegs {
-  int lo[kTapRegs], hi[kTapRegs];
-  float wlo[kTapRegs], whi[kTapRegs];
+template <int N>
+struct TapRegsOf {
+  int lo[N], hi[N];
+  float wlo[N], whi[N];
   __device__ __forceinline__ void load(const AxisTaps &t, int cell) {
 #pragma unroll
-    for (int s = 0; s < kTapRegs; s++) {
+    for (int s = 0; s < N; s++) {
       const bool on = s < t.grid;
       const int e = on ? cell * t.grid + s : 0;
       lo[s] = on ? t.lo[e] : 0; hi[s] = on ? t.hi[e] : 0;
@@ -71,7 +72,7 @@ struct TapRegs {
   __device__ __forceinline__ float apply(const E *row, int stride) const {
     float acc = 0.f;
 #pragma unroll
-    for (int s = 0; s < kTapRegs; s++)
+    for (int s = 0; s < N; s++)
       acc += wlo[s] * load_any(row + lo[s] * stride) + whi[s] * load_any(row + hi[s] * stride);
     return acc;
   }
@@ -79,10 +80,12 @@ struct TapRegs {
   static __device__ __forceinline__ float load_any(const __half *p) { return mv::load(p); }
   static __device__ __forceinline__ float load_any(const __hip_bfloat16 *p) { return mv::load(p); }
 };
+using TapRegs = TapRegsOf<kTapRegs>;
 
 struct PoolPlan {
   int staged;      // 1: LDS path, 0: per-output gather, -1: every output is zero
   int chunk;       // channels per LDS pass
+  long voxels;     // of a staged box
 };
 
 static_assert(kPoolEntries % kWave == 0, "one wavefront builds the tap table of one axis, kPoolEntries / kWave entries per lane");
@@ -97,7 +100,8 @@ constexpr int kDenseSrc = 32;   // source voxels per axis of the dense weight ma
 // gather / scatter paths.  One barrier.
 template <typename RT, int CELLS>
 __device__ inline PoolPlan pool_setup(PoolShared &sh, const RT *roi, const RoiProblem &p, size_t elem_bytes,
-                                      float (*wd)[kDenseSrc][CELLS], bool slabs = false, bool sparse_gather = false) {
+                                      float (*wd)[kDenseSrc][CELLS], bool slabs = false, bool sparse_gather = false,
+                                      const int lds_bytes = kPoolLdsBytes) {
   const int nd = p.ndim;
   const int cells[3] = {p.ow, p.oh, p.od};
   const int size[3] = {p.W, p.H, p.D};
@@ -105,7 +109,7 @@ __device__ inline PoolPlan pool_setup(PoolShared &sh, const RT *roi, const RoiPr
   // extents and sampling grids of all axes (every lane the same): they decide the path
   double start[3], ext[3];
   int grid[3], entries[3];
-  PoolPlan plan{1, 0};
+  PoolPlan plan{1, 0, 0};
   if (b < 0 || b >= p.N) plan.staged = -1;
 #pragma unroll
   for (int a = 0; a < 3; a++) {
@@ -208,6 +212,7 @@ __device__ inline PoolPlan pool_setup(PoolShared &sh, const RT *roi, const RoiPr
     if (sh.ax[k].box_hi < 0) plan.staged = -1;  // no valid sample on this axis
     vol *= sh.ax[k].box_hi - sh.ax[k].box_lo + 1;
   }
+  plan.voxels = vol;
   if (plan.staged != 1) return plan;
   if (sparse_gather) {
     // A box that holds more than half as many voxels as the roi's samples have taps is read sparsely (bins
@@ -222,7 +227,7 @@ __device__ inline PoolPlan pool_setup(PoolShared &sh, const RT *roi, const RoiPr
   {
     const long nz = sh.ax[2].box_hi - sh.ax[2].box_lo + 1, ny = sh.ax[1].box_hi - sh.ax[1].box_lo + 1;
     const long per_channel = vol * static_cast<long>(elem_bytes) + (nz * ny * p.ow + nz * p.oh * p.ow) * 4 + 16;
-    const long chunk = kPoolLdsBytes / per_channel;
+    const long chunk = lds_bytes / per_channel;
     if (chunk < 1 && !slabs) plan.staged = 0;   // (a caller that works in slabs of box planes sizes them itself)
     plan.chunk = static_cast<int>(min(chunk, 64L));
   }
@@ -686,29 +691,251 @@ __device__ __forceinline__ void pool_share(const PoolShare &share, const RT *roi
   channels = pool_share_channels(share, p.C, parts, voxels);
 }
 
-template <typename T, typename RT, int CELLS>
-__global__ __launch_bounds__(kPoolThreads) void roi_pool_forward_kernel(
+// Forward pass of a large box, up to eight cells per axis: a wavefront per output plane and channel, no barriers.  The cells of a
+// plane pd need only the few slices that its samples touch.  Per unit (pd, channel)
+//   z   a lane loads its voxels of the touched slices of the box, coalesced along the rows, and blends the slices in registers: to LDS;
+//   x   eight rows times eight cells per turn: the row's taps from LDS, their sum to LDS;
+//   y   a lane per cell (ph, pw): the taps of its column, and the cell goes out.
+// The wavefronts share the tap tables, the rest of the LDS is their own, and the first voxels of a wavefront's next unit are on their way
+// while it contracts one.  (Whole boxes staged per workgroup, with three barriers per LDS-sized chunk of channels, took 21 us for each
+// channel of a box of 9504 voxels: 38 us for 128 fp32 rois x 16 channels x 7^3 with boxes of 4 - 24 voxels a side, 21 us now; 259 x 256, up to 23 voxels, 407 -> 230;
+// 3361 x 32, up to 22, 427 -> 280; bf16, 2228 x 16, up to 17, 109 -> 97.)
+// Slices of weight 0 are not read.
+constexpr int kPlanePer = 12, kPlaneBox = kPlanePer * kWave;   // voxels of a slab of rows: per lane, and in all
+constexpr int kPlaneRows = 64;                                 // rows of a slab
+constexpr int kPlaneLds = (kPlaneBox + kPlaneRows + kPlaneRows * 8) * 4;   // bytes per wavefront
+static_assert(kPlaneLds * (kPoolThreads / kWave) <= 30 * 1024, "room for four wavefronts");
+
+__device__ __forceinline__ void pool_wave_sync() {   // LDS of one wavefront is in order: only the compiler has to keep it
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <typename T>
+__device__ inline void pool_forward_planes(const T *__restrict__ src, T *__restrict__ dst, const RoiProblem &p, const PoolShared &sh,
+                                           unsigned char *lds, const int channels) {
+  const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  constexpr int waves = kPoolThreads / kWave;
+  float *const box = reinterpret_cast<float *>(lds + wave * kPlaneLds), *const rows = box + kPlaneBox + kPlaneRows;
+  const AxisTaps &xt = sh.ax[0], &yt = sh.ax[1], &zt = sh.ax[2];
+  const auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+  const int gx = uniform(xt.grid), gy = uniform(yt.grid), gz = uniform(zt.grid);
+  const int nx = uniform(xt.box_hi - xt.box_lo) + 1, ny = uniform(yt.box_hi - yt.box_lo) + 1;
+  const int ph = lane / 8, pw = lane % 8, ohw = p.oh * p.ow, cells = p.od * ohw, units = p.od * channels;
+  const bool live = ph < p.oh && pw < p.ow;
+  const long plane = static_cast<long>(p.H) * p.W, volume = plane * p.D;
+  const T *const corner = src + uniform(zt.box_lo) * plane + static_cast<long>(uniform(yt.box_lo)) * p.W + uniform(xt.box_lo);
+  T *const cell = dst + ph * p.ow + pw;
+  const int ex = min(pw, p.ow - 1) * gx, ey = min(ph, p.oh - 1) * gy;   // the lane's first entries
+  constexpr int REGS = 4;
+  const bool few = gx <= 2 && gy <= 2, some = gx <= REGS && gy <= REGS;
+  TapRegsOf<REGS> tx, ty;
+  tx.load(xt, min(pw, p.ow - 1));
+  ty.load(yt, min(ph, p.oh - 1));
+
+  const int pitch = nx | 1, slab = min(min(kPlaneBox / nx, kPlaneRows), ny);   // (odd: rows on different banks)
+  const float inv_nx = 1.f / static_cast<float>(nx);
+  unsigned from[kPlanePer];   // the lane's voxels of a slab: in a slice, and in LDS
+  int to[kPlanePer];
+  auto prepare = [&](int y0, int count) {
+#pragma unroll
+    for (int u = 0; u < kPlanePer; u++) {
+      const int k = min(lane + u * kWave, count - 1), y = fdiv(k, inv_nx), x = k - y * nx;   // (past the end: the last one again)
+      from[u] = static_cast<unsigned>((y0 + y) * p.W + x);
+      to[u] = y * pitch + x;
+    }
+  };
+  // lane k: weight of slice first + k of the box for the cells of plane pd
+  int first = 0, plane_of = -1;
+  float wz = 0.f;
+  auto weights = [&](int pd) {
+    const int e = pd * gz + min(lane, gz - 1);
+    const int lo = zt.lo[e], hi = zt.hi[e];
+    const float a = lane < gz ? zt.wlo[e] : 0.f, c = lane < gz ? zt.whi[e] : 0.f;
+    const unsigned long long valid = __ballot(a != 0.f || c != 0.f);
+    first = valid ? __builtin_amdgcn_readlane(lo, __builtin_ctzll(valid)) : 0;
+    wz = 0.f;
+    for (int s = 0; s < gz; s++) {
+      const float ws = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(a), s)), wt = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(c), s));
+      wz += (__builtin_amdgcn_readlane(lo, s) - first == lane ? ws : 0.f) + (__builtin_amdgcn_readlane(hi, s) - first == lane ? wt : 0.f);
+    }
+    plane_of = pd;
+  };
+  // Four slices at a time.  Where fewer are left, the first one stands in for the others and its weight is shared out, by powers of two:
+  // no sum has a term of weight 0.
+  struct Slices { int at[4]; float w[4]; };
+  auto next_slices = [&](unsigned long long &left) {
+    Slices s;
+    const int n = min(static_cast<int>(__popcll(left)), 4);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      s.at[k] = k < n ? __builtin_ctzll(left) : s.at[0];
+      s.w[k] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wz), s.at[k])) * (k == 0 ? (n == 4 ? 1.f : n == 1 ? .25f : .5f) : k < n ? 1.f : n == 3 ? .5f : .25f);
+      if (k < n) left &= left - 1;
+    }
+    return s;
+  };
+  float raw[2][4][4];   // [set][slice][voxel]
+  auto request = [&](float (&r)[4][4], const T *base, const Slices &s, int u0) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const T *const slice = base + s.at[k] * plane;
+#pragma unroll
+      for (int u = 0; u < 4; u++) r[k][u] = load(slice + from[u0 + u]);
+    }
+  };
+  auto put = [&](const float (&r)[4][4], const Slices &s, int u0) {
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      float v = s.w[0] * r[0][u];
+#pragma unroll
+      for (int k = 1; k < 4; k++) v = fmaf(s.w[k], r[k][u], v);
+      box[to[u0 + u]] = v;
+    }
+  };
+  // (more than four slices: added to what the first four have left)
+  auto put_more = [&](const T *base, unsigned long long left, int count) {
+    while (left) {
+      const Slices s = next_slices(left);
+#pragma unroll
+      for (int u0 = 0; u0 < kPlanePer; u0 += 4) {
+        if (u0 * kWave >= count) break;
+        request(raw[0], base, s, u0);
+        float v[4];
+        pool_wave_sync();
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = box[to[u0 + u]];
+        pool_wave_sync();   // (lanes past the end share the last voxel)
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+#pragma unroll
+          for (int k = 0; k < 4; k++) v[u] = fmaf(s.w[k], raw[0][k][u], v[u]);
+          box[to[u0 + u]] = v[u];
+        }
+      }
+    }
+  };
+  auto along_x = [&](int n_rows) {
+    for (int r = ph; r < n_rows; r += 8) {   // (ph, pw as row and cell)
+      const float *line = box + r * pitch;
+      float sum = 0.f;
+      if (some) {
+#pragma unroll
+        for (int s = 0; s < REGS; s++)
+          if (s < 2 || !few) sum += tx.wlo[s] * line[tx.lo[s]] + tx.whi[s] * line[tx.hi[s]];
+      } else {
+        for (int s = 0; s < gx; s++) sum += xt.wlo[ex + s] * line[xt.lo[ex + s]] + xt.whi[ex + s] * line[xt.hi[ex + s]];
+      }
+      rows[r * 8 + pw] = sum;
+    }
+  };
+  auto along_y = [&](int y0, int n_rows) {   // the share of rows y0 ..
+    float sum = 0.f;
+    auto add = [&](int lo, int hi, float wlo, float whi) {
+      if (static_cast<unsigned>(lo - y0) < static_cast<unsigned>(n_rows)) sum += wlo * rows[(lo - y0) * 8 + pw];
+      if (static_cast<unsigned>(hi - y0) < static_cast<unsigned>(n_rows)) sum += whi * rows[(hi - y0) * 8 + pw];
+    };
+    if (some) {
+#pragma unroll
+      for (int s = 0; s < REGS; s++)
+        if (s < 2 || !few) add(ty.lo[s], ty.hi[s], ty.wlo[s], ty.whi[s]);
+    } else {
+      for (int s = 0; s < gy; s++) add(yt.lo[ey + s], yt.hi[ey + s], yt.wlo[ey + s], yt.whi[ey + s]);
+    }
+    return sum;
+  };
+
+  Slices now;
+  const T *base = nullptr;
+  unsigned long long left = 0;
+  bool empty = false;
+  auto begin = [&](int u) {   // units: the channels of a plane next to each other
+    const int pd = u / channels, c = u - pd * channels;
+    if (pd != plane_of) weights(pd);
+    left = __ballot(wz != 0.f);
+    empty = left == 0;   // (the plane is outside: its cells are zero, whatever slice 0 holds)
+    if (empty) left = 1;
+    base = corner + c * volume + first * plane;
+    now = next_slices(left);
+  };
+  auto store = [&](int u, float sum) {
+    const int pd = u / channels, c = u - pd * channels;
+    if (live) cell[static_cast<long>(c) * cells + pd * ohw] = store_cast<T>(sum);
+  };
+  const int count = slab * nx;
+  if (slab == ny) {
+    prepare(0, count);
+    if (wave < units) {
+      begin(wave);
+      request(raw[0], base, now, 0);
+    }
+    for (int u = wave; u < units; u += waves) {
+      if (count > 4 * kWave) request(raw[1], base, now, 4);
+      put(raw[0], now, 0);
+      if (count > 8 * kWave) request(raw[0], base, now, 8);
+      if (count > 4 * kWave) put(raw[1], now, 4);
+      if (count > 8 * kWave) put(raw[0], now, 8);
+      if (left) put_more(base, left, count);
+      pool_wave_sync();
+      const bool none = empty;
+      if (u + waves < units) {
+        begin(u + waves);
+        request(raw[0], base, now, 0);
+      }
+      along_x(ny);
+      pool_wave_sync();
+      const float sum = along_y(0, ny);
+      store(u, none ? 0.f : sum);
+      pool_wave_sync();
+    }
+    return;
+  }
+  for (int u = wave; u < units; u += waves) {
+    begin(u);
+    float sum = 0.f;
+    for (int y0 = 0; y0 < ny; y0 += slab) {
+      const int n_rows = min(slab, ny - y0), voxels = n_rows * nx;
+      prepare(y0, voxels);
+#pragma unroll
+      for (int u0 = 0; u0 < kPlanePer; u0 += 4) {
+        if (u0 * kWave >= voxels) break;
+        request(raw[0], base, now, u0);
+        put(raw[0], now, u0);
+      }
+      if (left) put_more(base, left, voxels);
+      pool_wave_sync();
+      along_x(n_rows);
+      pool_wave_sync();
+      sum += along_y(y0, n_rows);
+      pool_wave_sync();
+    }
+    store(u, empty ? 0.f : sum);
+  }
+}
+
+constexpr int kPoolLdsFour = 30 * 1024;   // four workgroups on a compute unit
+
+template <typename T, typename RT, int CELLS, int LDS>
+__global__ __launch_bounds__(kPoolThreads, LDS == kPoolLdsFour ? 4 : 1) void roi_pool_forward_kernel(
     const T *__restrict__ feat, const RT *__restrict__ rois, T *__restrict__ out, const RoiProblem p,
     const int channels_per_block, const int joined, const T *__restrict__ blocked, const int Wb,
     const unsigned *__restrict__ order) {
   __shared__ PoolShared sh;
-  __shared__ __attribute__((aligned(16))) unsigned char lds[kPoolLdsBytes];
+  __shared__ __attribute__((aligned(16))) unsigned char lds[LDS];
   const unsigned n = order ? order[blockIdx.x] : blockIdx.x;   // (largest rois first, see pool_order_rois)
   int cpb = channels_per_block;   // small boxes: `joined` times as many
-  if (joined > 1) {
+  const RT *const roi = rois + static_cast<long>(n) * roi_columns(p.ndim, 0);
+  if (joined > 1 && pool_small_box(roi, p)) {
     constexpr bool kMatrix = CELLS == 8 && std::is_same<T, __half>::value;
-    const RT *roi = rois + static_cast<long>(n) * roi_columns(p.ndim, 0);
-    if (pool_small_box(roi, p)) {
-      int times = joined;
-      while (!kMatrix && times > 1 && pool_voxels(roi, p) * static_cast<float>(cpb * times) > kShareJoined) times /= 2;
-      cpb *= times;
-    }
+    int times = joined;
+    while (!kMatrix && times > 1 && pool_voxels(roi, p) * static_cast<float>(cpb * times) > kShareJoined) times /= 2;
+    cpb *= times;
   }
   if (static_cast<long>(blockIdx.y) * cpb >= p.C) return;   // (channels of a workgroup before)
   const int c_begin = blockIdx.y * cpb, c_end = min(c_begin + cpb, p.C);
   __shared__ __attribute__((aligned(16))) float wd[3][kDenseSrc][CELLS];
   PoolPlan plan = pool_setup<RT, CELLS>(sh, rois + static_cast<long>(n) * roi_columns(p.ndim, 0), p, sizeof(T),
-                                        CELLS == 8 ? wd : nullptr, true, true);
+                                        CELLS == 8 ? wd : nullptr, true, true, LDS);
   const int cells = p.od * p.oh * p.ow;
   const long plane = static_cast<long>(p.D) * p.H * p.W;
   T *dst = out + (static_cast<long>(n) * p.C + c_begin) * cells;
@@ -718,6 +945,21 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_forward_kernel(
     return;
   }
   const T *src = feat + (static_cast<long>(sh.g.batch) * p.C + c_begin) * plane;
+  if constexpr (CELLS == 8 && !std::is_same<T, __half>::value) {
+    // A large box by wavefronts on their own (a plane's samples are one per lane, its slices too, and a row fits the wavefront's LDS).
+    // Smaller ones are better off with whole boxes, whose slices are read once for all planes: 296 bf16 rois x 32 channels of up to 11 voxels
+    // a side 27 us, 34 us with 1000 voxels as the limit; 565 fp32 rois x 128 channels of up to 15 voxels a side 180 us without, 119 us with 1200
+    // and 169 us with 3000.  fp16 boxes beyond the matrix cores' form would gain too, but those within it lose 2 % to the scalar registers
+    // that this branch costs the kernel.
+    constexpr long kPlanesFrom = sizeof(T) == 4 ? 1200 : 1800;
+    if (__builtin_expect(plan.staged == 1 && plan.voxels >= kPlanesFrom, 0)) {
+      const int nx = sh.ax[0].box_hi - sh.ax[0].box_lo + 1, ny = sh.ax[1].box_hi - sh.ax[1].box_lo + 1, nz = sh.ax[2].box_hi - sh.ax[2].box_lo + 1;
+      if (p.ndim == 3 && sh.ax[2].grid <= kWave && nz <= kWave && nx <= kPlaneBox) {
+        pool_forward_planes<T>(src, dst, p, sh, lds, c_end - c_begin);
+        return;
+      }
+    }
+  }
   if (plan.staged == 1 && plan.chunk < 1) {
     // A box too large for LDS with all its planes is worked through in slabs of planes: x and y are
     // contracted per slab, and the z contraction adds each slab's share to sums kept per output.
@@ -733,7 +975,7 @@ __global__ __launch_bounds__(kPoolThreads) void roi_pool_forward_kernel(
     // per slab the passes were 20 - 30 % slower — 200 rois of 24 - 32 voxels x 256 channels, grid 4: 7.0 -> 5.0 ms)
     for (int c = gx * gy * gz > 27 ? 1 : 0; c >= 1 && cs == 0; c >>= 1) {
       const int cn = min(c, c_end - c_begin);
-      const long planes = (kPoolLdsBytes - 32 - cn * static_cast<long>(cells) * 4) / (cn * per_plane);
+      const long planes = (LDS - 32 - cn * static_cast<long>(cells) * 4) / (cn * per_plane);
       if (planes >= 1) { cs = cn; zs = static_cast<int>(min(planes, static_cast<long>(nz))); }
     }
     if (cs == 0) {
@@ -1510,10 +1752,10 @@ static int pool_channels_per_block(const RoiProblem &p, long enough = 6144) {
 // workgroups with `cpb` channels each
 static long pool_groups(const RoiProblem &p, int cpb) { return static_cast<long>(p.R) * ((p.C + cpb - 1) / cpb); }
 
-template <typename T, int CELLS>
+template <typename T, int CELLS, int LDS = kPoolLdsBytes>
 static void launch_pool_forward(const void *input, const float *r, void *output, const RoiProblem &p, int cpb,
                                 dim3 grid, hipStream_t s, int joined = 1, const void *blocked = nullptr, const unsigned *order = nullptr) {
-  hipLaunchKernelGGL((roi_pool_forward_kernel<T, float, CELLS>), grid, dim3(kPoolThreads), 0, s,
+  hipLaunchKernelGGL((roi_pool_forward_kernel<T, float, CELLS, LDS>), grid, dim3(kPoolThreads), 0, s,
                      static_cast<const T *>(input), r, static_cast<T *>(output), p, cpb, joined,
                      static_cast<const T *>(blocked), p.W / 4, order);
 }
@@ -1609,18 +1851,31 @@ int roi_pool_forward(const void *input, const void *rois, void *output, int dtyp
   // the box has work for (kShareJoined): 947 fp32 rois of two channels, 8^3 cells and boxes of up to 32 x 18 x 32 take 46 us, joined 56; 55 of
   // 18 and 7^3 18 and 27.
   int cpb = pool_channels_per_block(p, blocked != nullptr && order != nullptr ? 3072 : 6144), joined = 1;
+  // Without matrix cores a head of few rois and channels takes as few channels per workgroup as let all workgroups run at a time: four on a
+  // compute unit with 30 KB for the boxes (LDS), three with 40 KB (223 fp32 rois x 32 channels 18.6 us with 1784 workgroups, 11.8 with 892; 16 bf16 x 256, 1024
+  // workgroups, 12.9 and 10.8).  From nine channels each on, large boxes would last longer than the rounds that this saves.
+  bool four = false;
+  if (p.ndim == 3 && dtype != MV_F16 && pool_small_cells(p) && p.R <= 1024) {
+    int fit = 1;
+    while (fit <= 8 && pool_groups(p, fit) > 1024) fit++;
+    if (fit <= 8) {
+      cpb = fit;
+      four = pool_groups(p, fit) > 768;
+    }
+  }
   if (pool_small_cells(p)) {
     joined = std::max(std::min(p.C, dtype == MV_F16 ? 16 : 4) / cpb, 1);
     while (joined > 1 && pool_groups(p, cpb * joined) < 256) joined /= 2;
   }
+  const bool small = pool_small_cells(p);
   const long cblocks = (p.C + cpb - 1) / cpb;
   if (cblocks > 65535) return -1;
   const dim3 grid(p.R, static_cast<unsigned>(cblocks));
   const float *r = static_cast<const float *>(rois);
-  const bool small = pool_small_cells(p);
   switch (dtype) {
     case MV_F32:
-      small ? launch_pool_forward<float, 8>(input, r, output, p, cpb, grid, s, joined)
+      four ? launch_pool_forward<float, 8, kPoolLdsFour>(input, r, output, p, cpb, grid, s, joined)
+      : small ? launch_pool_forward<float, 8>(input, r, output, p, cpb, grid, s, joined)
             : launch_pool_forward<float, 16>(input, r, output, p, cpb, grid, s);
       break;
     case MV_F16:
@@ -1628,7 +1883,8 @@ int roi_pool_forward(const void *input, const void *rois, void *output, int dtyp
             : launch_pool_forward<__half, 16>(input, r, output, p, cpb, grid, s);
       break;
     default:
-      small ? launch_pool_forward<__hip_bfloat16, 8>(input, r, output, p, cpb, grid, s, joined)
+      four ? launch_pool_forward<__hip_bfloat16, 8, kPoolLdsFour>(input, r, output, p, cpb, grid, s, joined)
+      : small ? launch_pool_forward<__hip_bfloat16, 8>(input, r, output, p, cpb, grid, s, joined)
             : launch_pool_forward<__hip_bfloat16, 16>(input, r, output, p, cpb, grid, s);
   }
   return check_launch("roi_pool_forward_kernel");
