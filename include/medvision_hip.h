@@ -280,6 +280,14 @@ int mv_deform_warp_2d(const void *img, const void *offset, void *output, int dty
 int mv_deform_warp_3d(const void *img, const void *offset, void *output, int dtype, int batch,
                       int channels, int depth, int height, int width, int order, void *stream);
 
+/* The same warp on volumes by the field that the order-3 affine engine gives for a control grid [B, 3, grid_d, grid_h, grid_w]
+ * (float32) over the window [border, points - border] of each axis (aug_cuda/aug_spatial.py:560-600), without that field in
+ * memory: order 1 (the field rounded to the image's dtype), MV_I32: order 0.  ..._applies: whether the kernel takes these
+ * sizes (0: upsample and warp in two calls).                                                                              */
+int mv_elastic_warp_3d_applies(int dtype, int batch, int depth, int height, int width, int grid_d, int grid_h, int grid_w, float border);
+int mv_elastic_warp_3d(const void *img, const void *grid, void *output, int dtype, int batch, int channels, int depth, int height,
+                       int width, int grid_d, int grid_h, int grid_w, float border, void *stream);
+
 /* ---- augmentation DCN in general ----------------------------------------------------------------
  * replaces deform_2d / deform_3d  csrc/deform_2d.h, csrc/deform_3d.h:27 (vision.cpp:71-72; host
  * csrc/cuda_aug/deform_3d_cuda.cu:43-152, kernel csrc/cuda_aug/deform_3d_cuda_kernel.cuh:8-89) for

@@ -76,6 +76,8 @@ SIGNATURES = {
     "mv_dcn2d_backward_write": (_i, [_p] * 10 + [_SHAPE2_P, _i, _p, _p]),
     "mv_deform_warp_2d": (_i, [_p, _p, _p, _i] + [_i] * 4 + [_i, _p]),
     "mv_deform_warp_3d": (_i, [_p, _p, _p, _i] + [_i] * 5 + [_i, _p]),
+    "mv_elastic_warp_3d_applies": (_i, [_i] * 8 + [ctypes.c_float]),
+    "mv_elastic_warp_3d": (_i, [_p, _p, _p] + [_i] * 9 + [ctypes.c_float, _p]),
     "mv_deform_conv_3d": (_i, [_p] * 6 + [_i, _i, _p]),
     "mv_deform_conv_2d": (_i, [_p] * 6 + [_i, _i, _p]),
     "mv_upload": (_i, [_p, _p, _sz, _p]),

@@ -386,7 +386,7 @@ class CudaRandomElasticDeformation(CudaAugBase):
         self.INTER_ORDER = order                       # of the control grid's upsampling
         self.num_locked_borders = 2
         assert max_displacement <= 1.0
-        self.tmp_params = None
+        self._forget_field()
 
     def __repr__(self):
         return (f'{self.__class__.__name__}(p={self.p}, num_control_points={self.num_control_points}, '
@@ -396,8 +396,23 @@ class CudaRandomElasticDeformation(CudaAugBase):
     def canBackward(self):
         return True
 
+    def _forget_field(self):
+        self._field = self._device_grid = self._field_device = None
+
+    @property
+    def tmp_params(self):
+        """The dense field of the present draw, on the device of the last image; None before there is one."""
+        if self._field is None and self._field_device is not None:
+            self.dense_field(self._field_device)
+        return self._field
+
+    @tmp_params.setter
+    def tmp_params(self, field):
+        self._forget_field()
+        self._field = field
+
     def _forward_params(self, result):
-        self.tmp_params = None
+        self._forget_field()
         self._init_params(result)
         grid = self.to_tuple(self.num_control_points, self.dim)
         cell = np.array(self.image_shape) / (np.array(grid) - 1)
@@ -414,30 +429,52 @@ class CudaRandomElasticDeformation(CudaAugBase):
         result[self.key_name] = self.params
 
     def _backward_params(self, result):
-        self.tmp_params = None
+        self._forget_field()
         self._init_params(result)
         params = result.pop(self.key_name, None)
         if params is not None:
             self.params = -params
 
+    def _control_grid(self):
+        """[batch, component, *grid]: half of the control points' displacements."""
+        coarse = self.params if self.batched else self.params[None]
+        if coarse.dtype.kind != 'f':
+            coarse = coarse.astype(np.float32)
+        return np.moveaxis(coarse, -1, 1) / 2
+
     def dense_field(self, device):
         """[dim, *image_shape] displacements (z, y, x components) -- the batch stage: [batch, dim,
         *image_shape] -- cached per draw."""
-        if self.tmp_params is None:
-            coarse = self.params if self.batched else self.params[None]
-            if coarse.dtype.kind != 'f':
-                coarse = coarse.astype(np.float32)
-            grid = np.moveaxis(coarse, -1, 1) / 2          # [batch, component, *grid]
+        if self._field is None:
+            grid = self._control_grid()
             shape_xyz = grid.shape[2:][::-1]
             roi = geometry.window_rois(self.dim, [1.5] * self.dim, [s - 1.5 for s in shape_xyz],
                                        index=np.arange(grid.shape[0]))
             fn = affine_2d if self.dim == 2 else affine_3d
             dense = fn(native.upload(grid, device), native.upload(roi, device),
                        tuple(self.image_shape), 1, 1, True, self.INTER_ORDER)
-            self.tmp_params = dense if self.batched else dense.squeeze(0)
-        return self.tmp_params
+            self._field = dense if self.batched else dense.squeeze(0)
+        return self._field
+
+    def _warp_from_grid(self, image, order):
+        """[batch, channel, *image_shape] warped without a dense field in memory; None where there is one already, or the kernel
+        does not take these sizes or types."""
+        labels = image.dtype == torch.int32
+        if (self._field is not None or self.dim != 3 or self.INTER_ORDER != 3 or not image.is_cuda or order != (0 if labels else 1)
+                or tuple(image.shape[2:]) != tuple(self.image_shape)):
+            return None
+        if self._device_grid is None or self._device_grid.device != image.device:
+            grid = self._control_grid()
+            if grid.dtype != np.float32:
+                return None
+            self._device_grid = native.upload(grid, image.device)
+        return native.elastic_warp(image, self._device_grid, 1.5)
 
     def elastic_transform(self, image, order=1):
+        self._field_device = image.device
+        out = self._warp_from_grid(image if self.batched else image.unsqueeze(0), order)
+        if out is not None:
+            return out if self.batched else out.squeeze(0)
         field = self.dense_field(image.device)
         fn = apply_offset_2d if self.dim == 2 else apply_offset_3d
         if not self.batched:

@@ -469,6 +469,31 @@ Tensor deform_warp(const Tensor &img_in, const Tensor &offset_in, double given_o
   return out;
 }
 
+// A volume [B,C,D,H,W] warped by the field that its control grids [B,3,z,y,x] give over the window [border, points - border]; nothing
+// where that has to be done in two calls.
+std::optional<Tensor> elastic_warp(const Tensor &img_in, const Tensor &grid, double border) {
+  const py::gil_scoped_release no_gil;
+  const at::NoGradGuard no_grad;
+  if (!img_in.is_cuda() || img_in.dim() != 5 || grid.dim() != 5 || grid.device() != img_in.device() || grid.scalar_type() != at::kFloat ||
+      grid.size(0) != img_in.size(0) || grid.size(1) != 3 || img_in.numel() == 0)
+    return std::nullopt;
+  const auto type = img_in.scalar_type();
+  if (type != at::kInt && type != at::kFloat && type != at::kHalf && type != at::kBFloat16) return std::nullopt;
+  for (const Tensor &t : {img_in, grid})
+    for (int64_t n : t.sizes())
+      if (n > std::numeric_limits<int>::max()) return std::nullopt;
+  const int code = type == at::kInt ? static_cast<int>(MV_I32) : dtype_code(img_in);
+  const auto d = five_dims(img_in.sizes(), 3);
+  const auto g = five_dims(grid.sizes(), 3);
+  const float edge = static_cast<float>(border);
+  if (!mv_elastic_warp_3d_applies(code, d[0], d[2], d[3], d[4], g[2], g[3], g[4], edge)) return std::nullopt;
+  const c10::DeviceGuard guard(img_in.device());
+  const Tensor img = img_in.contiguous(), points = grid.contiguous();
+  const Tensor out = at::empty_like(img);
+  check(mv_elastic_warp_3d(ptr(img), ptr(points), ptr(out), code, d[0], d[1], d[2], d[3], d[4], g[2], g[3], g[4], edge, stream_of(img)));
+  return out;
+}
+
 // ---- helpers of the augmentation stages ----------------------------------------------------------------------------
 // A host array (rois, a control grid) on the device, without waiting for what is queued there.  float64 stays float64,
 // every other type becomes float32.
@@ -505,6 +530,7 @@ PYBIND11_MODULE(_native, m) {
   m.def("modulated_deform_conv", &modulated_deform_conv);
   m.def("deform_conv", &deform_conv);
   m.def("deform_warp", &deform_warp);
+  m.def("elastic_warp", &elastic_warp);
   m.def("upload", &upload);
   m.def("peak_mib", &peak_mib);
 }

@@ -289,3 +289,48 @@ def test_int32_label_maps_are_sampled_as_they_are(dim, size, out):
     assert int((got != 0).sum()) > got.numel() // 4
     with pytest.raises((RuntimeError, AssertionError)):
         fn(seg.to(DEV), rois, out, 1.0, 1, True, 1)    # int32 at order 1
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("batch,channels,size,points", [
+    (1, 1, (33, 41, 97), (8, 8, 8)),       # tiles with remainders on every axis
+    (2, 3, (8, 8, 32), (4, 5, 6)),         # one tile; several rows of control points per voxel
+    (1, 2, (7, 9, 5), (9, 7, 16)),         # less than a tile, most points along x
+    (1, 1, (64, 1, 2), (10, 4, 4)),        # axes of one and two voxels
+])
+def test_elastic_warp_without_a_field(batch, channels, size, points, dtype):
+    """The warp from the control grid against the two calls that it stands for, images and labels."""
+    from medvision_amd._lib import native
+    from medvision_amd.ops import affine_3d, apply_offset_3d
+    g = wl.gen(sum(size) + sum(points))
+    grid = (torch.rand(batch, 3, *points, generator=g) * 2 - 1) * torch.tensor([2.0, 5.0, 9.0]).view(1, 3, 1, 1, 1)
+    img = torch.randn(batch, channels, *size, generator=g).to(dtype).to(DEV)
+    seg = torch.randint(0, 7, (batch, channels, *size), generator=g, dtype=torch.int32).to(DEV)
+    n = torch.tensor(points[::-1], dtype=torch.float32)
+    rois = torch.stack([torch.tensor([b, *(n / 2), *(n - 3), 0, 0, 0]) for b in range(batch)])
+    field = affine_3d(grid.to(DEV), rois.to(DEV), size, 1, 1, True, 3)
+    got = native.elastic_warp(img, grid.to(DEV), 1.5)
+    want = apply_offset_3d(img, field.to(dtype))
+    # (the last bit of a displacement may differ, and with it a rounding of it: 2^-11 / 2^-8 of a few voxels)
+    assert_close(got, want, {torch.float32: 1e-5, torch.float16: 4e-3, torch.bfloat16: 3e-2}[dtype], "image")
+    # (fp32 sums differ in their last bits; rounded to 11 bits, one in 2^12 of such differences can show, to 8 bits fewer)
+    assert dtype == torch.float32 or float((got != want).float().mean()) < 8 * 2.0 ** -12
+    labels = native.elastic_warp(seg, grid.to(DEV), 1.5)
+    assert labels.dtype == torch.int32 and float((labels != apply_offset_3d(seg, field, 0)).float().mean()) < 1e-4
+    assert native.elastic_warp(img.double(), grid.to(DEV), 1.5) is None
+    assert native.elastic_warp(img, grid.to(DEV)[..., :3], 1.5) is None           # a window of nothing
+    assert native.elastic_warp(img, torch.zeros(batch, 3, 4, 17, 4, device=DEV), 1.5) is None
+
+
+def test_elastic_stage_keeps_a_given_field(aug):
+    """A dense field that is there already is the one that is applied; one that nobody asked for is made when it is read."""
+    img = torch.randn(1, 12, 14, 16).to(DEV)
+    stage = aug.CudaRandomElasticDeformation(1.0, 7, 0.9)
+    np.random.seed(3)
+    stage._forward_params({"img": img, "img_dim": 3})
+    first = stage.elastic_transform(img)
+    field = stage.tmp_params
+    assert field.shape == (3, 12, 14, 16) and stage.tmp_params is field
+    assert_close(stage.elastic_transform(img), first, 1e-5, "from the field")
+    stage.tmp_params = torch.zeros_like(field)
+    assert torch.equal(stage.elastic_transform(img), img)
