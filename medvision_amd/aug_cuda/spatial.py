@@ -33,6 +33,9 @@ class _Resampler:
     def _out_size(self):
         raise NotImplementedError
 
+    def _uploaded_rois(self, device):
+        return native.upload(self._rois(), device)
+
     def _skip(self):
         return False
 
@@ -40,13 +43,13 @@ class _Resampler:
         assert tensor.is_cuda, 'image should be cuda'
         lead = 2 if self.batched else 1
         assert tensor.ndim == self.dim + lead, 'image should be [batch,] channel, **dim'
-        fn = affine_2d if self.dim == 2 else affine_3d
         rois = getattr(self, '_device_rois', None)
         if rois is None or rois.device != tensor.device:
-            rois = self._device_rois = native.upload(self._rois(), tensor.device)
-        batch = tensor if self.batched else tensor.unsqueeze(0)
-        out = fn(batch, rois, tuple(int(v) for v in self._out_size()), 1.0, sampling_ratio, True, order)
-        return out if self.batched else out.squeeze(0)
+            rois = self._device_rois = self._uploaded_rois(tensor.device)
+        size = tuple(int(v) for v in self._out_size())
+        if not self.batched:
+            return native.affine_sample(self.dim, tensor, rois, size, sampling_ratio, order)
+        return native.affine(self.dim, tensor, rois, size, 1.0, sampling_ratio, True, order)
 
     def _labels(self, seg, sampling_ratio):
         """Order 0 on a label map.  The reference resamples a float copy and converts back
@@ -116,6 +119,12 @@ class CudaResize(_Resampler, CudaAugBase):
 
     def _rois(self):
         return geometry.frame_rois(self.image_shape, self.batch)
+
+    def _uploaded_rois(self, device):
+        if self.batched or getattr(self._rois, '__func__', None) is not CudaResize._rois:
+            return super()._uploaded_rois(device)
+        none = [0.0] * self.dim
+        return native.window_roi(self.dim, none, self.image_shape[::-1], [1.0] * self.dim, none, 0.0, device)
 
     def _out_size(self):
         return [int(s * f) for s, f in zip(self.image_shape, self.params)]
@@ -190,6 +199,14 @@ class CudaRandomAffine(_Resampler, CudaAugBase):
     def _rois(self):
         start, end = self._window()
         return geometry.window_rois(self.dim, start, end, *self._affine(), index=np.arange(self.batch))
+
+    def _uploaded_rois(self, device):
+        # (the arrays of one row cost 6 us on the host, the native form 1)
+        scales, shifts, rotate = self._affine()
+        if self.batched or getattr(self._rois, '__func__', None) is not CudaRandomAffine._rois or len(rotate) != 1:
+            return super()._uploaded_rois(device)
+        start, end = self._window()
+        return native.window_roi(self.dim, start, end, scales, shifts, rotate[0], device)
 
     def _out_size(self):
         return self.image_shape
@@ -419,10 +436,11 @@ class CudaRandomElasticDeformation(CudaAugBase):
         inner = tuple(slice(self.num_locked_borders, n - self.num_locked_borders) for n in grid)
         fields = []
         for _ in range(self.batch):      # one draw per sample, in sample order
-            coarse = 2 * np.random.rand(*grid, self.dim).astype(np.float32) - 1
+            # (all points are drawn, as in the reference; the locked ones are not used)
+            coarse = 2 * np.random.rand(*grid, self.dim)[inner].astype(np.float32) - 1
             coarse *= self.max_displacement * cell / 2          # per component (z, y, x)
-            locked = np.zeros_like(coarse)
-            locked[inner] = coarse[inner]
+            locked = np.zeros((*grid, self.dim), np.float32)
+            locked[inner] = coarse
             fields.append(locked)
         # per-sample stage: [*grid, dim]; batch stage: [batch, *grid, dim]
         self.params = np.array(fields) if self.batched else fields[0]
@@ -457,24 +475,24 @@ class CudaRandomElasticDeformation(CudaAugBase):
         return self._field
 
     def _warp_from_grid(self, image, order):
-        """[batch, channel, *image_shape] warped without a dense field in memory; None where there is one already, or the kernel
-        does not take these sizes or types."""
+        """The image warped without a dense field in memory; None where there is one already, or the kernel does not take these
+        sizes or types."""
         labels = image.dtype == torch.int32
         if (self._field is not None or self.dim != 3 or self.INTER_ORDER != 3 or not image.is_cuda or order != (0 if labels else 1)
-                or tuple(image.shape[2:]) != tuple(self.image_shape)):
+                or image.shape[2 if self.batched else 1:] != tuple(self.image_shape)):
             return None
         if self._device_grid is None or self._device_grid.device != image.device:
             grid = self._control_grid()
             if grid.dtype != np.float32:
                 return None
             self._device_grid = native.upload(grid, image.device)
-        return native.elastic_warp(image, self._device_grid, 1.5)
+        return native.elastic_warp(image, self._device_grid, 1.5)   # (a sample: as a batch of one)
 
     def elastic_transform(self, image, order=1):
         self._field_device = image.device
-        out = self._warp_from_grid(image if self.batched else image.unsqueeze(0), order)
+        out = self._warp_from_grid(image, order)
         if out is not None:
-            return out if self.batched else out.squeeze(0)
+            return out
         field = self.dense_field(image.device)
         fn = apply_offset_2d if self.dim == 2 else apply_offset_3d
         if not self.batched:

@@ -260,6 +260,11 @@ Tensor affine(int ndim, const Tensor &features, const Tensor &rois, const py::ob
   return roi_forward(c, features, rois, Tensor());
 }
 
+// The same for a sample [C, *spatial] as for a batch of one
+Tensor affine_sample(int ndim, const Tensor &sample, const Tensor &rois, const py::object &out_size, double sampling_ratio, double order) {
+  return affine(ndim, sample.unsqueeze(0), rois, out_size, 1.0, sampling_ratio, true, order).squeeze(0);
+}
+
 // ---- deformable convolution -----------------------------------------------------------------------------------------
 struct DcnCall {
   int nd, groups, dg;
@@ -469,11 +474,13 @@ Tensor deform_warp(const Tensor &img_in, const Tensor &offset_in, double given_o
   return out;
 }
 
-// A volume [B,C,D,H,W] warped by the field that its control grids [B,3,z,y,x] give over the window [border, points - border]; nothing
-// where that has to be done in two calls.
-std::optional<Tensor> elastic_warp(const Tensor &img_in, const Tensor &grid, double border) {
+// A volume [B,C,D,H,W], or a sample [C,D,H,W] as a batch of one, warped by the field that its control grids [B,3,z,y,x] give over the
+// window [border, points - border]; nothing where that has to be done in two calls.
+std::optional<Tensor> elastic_warp(const Tensor &given, const Tensor &grid, double border) {
   const py::gil_scoped_release no_gil;
   const at::NoGradGuard no_grad;
+  const bool sample = given.dim() == 4;
+  const Tensor img_in = sample ? given.unsqueeze(0) : given;
   if (!img_in.is_cuda() || img_in.dim() != 5 || grid.dim() != 5 || grid.device() != img_in.device() || grid.scalar_type() != at::kFloat ||
       grid.size(0) != img_in.size(0) || grid.size(1) != 3 || img_in.numel() == 0)
     return std::nullopt;
@@ -491,7 +498,7 @@ std::optional<Tensor> elastic_warp(const Tensor &img_in, const Tensor &grid, dou
   const Tensor img = img_in.contiguous(), points = grid.contiguous();
   const Tensor out = at::empty_like(img);
   check(mv_elastic_warp_3d(ptr(img), ptr(points), ptr(out), code, d[0], d[1], d[2], d[3], d[4], g[2], g[3], g[4], edge, stream_of(img)));
-  return out;
+  return sample ? out.squeeze(0) : out;
 }
 
 // ---- helpers of the augmentation stages ----------------------------------------------------------------------------
@@ -515,6 +522,30 @@ Tensor upload(const py::array &given, const at::Device &device) {
   return out;
 }
 
+// The roi of one window of one sample, as geometry.window_rois has it (its float32 arithmetic, in its order), on the device
+Tensor window_roi(int dim, const std::vector<double> &start, const std::vector<double> &end, const std::vector<double> &scales,
+                  const std::vector<double> &shifts, double rotate, const at::Device &device) {
+  const size_t n = static_cast<size_t>(dim);
+  MVB_CHECK((dim == 2 || dim == 3) && start.size() == n && end.size() == n && scales.size() == n && shifts.size() == n,
+            "expected one value per axis");
+  float row[10] = {};
+  const int columns = dim == 2 ? 6 : 10;
+  for (size_t a = 0; a < n; a++) {
+    const float s = static_cast<float>(start[a]), e = static_cast<float>(end[a]), scale = static_cast<float>(scales[a]), shift = static_cast<float>(shifts[a]);
+    const float extent = e - s, middle = (s + e) / 2.f, moved = extent * shift;
+    row[1 + a] = middle - moved / scale;
+    row[1 + n + a] = extent / scale;
+  }
+  row[columns - 1] = static_cast<float>(rotate);
+  const py::gil_scoped_release no_gil;
+  const at::NoGradGuard no_grad;
+  const c10::OptionalDeviceGuard guard(device.is_cuda() ? std::optional<at::Device>(device) : std::nullopt);
+  const Tensor out = at::empty({1, columns}, at::TensorOptions().dtype(at::kFloat).device(device));
+  if (device.is_cuda()) check(mv_upload(row, ptr(out), columns * sizeof(float), stream_of(out)));
+  else std::memcpy(out.data_ptr(), row, columns * sizeof(float));
+  return out;
+}
+
 // torch.cuda.max_memory_allocated() in MiB, without building the whole tree of statistics (18 us)
 double peak_mib() {
   auto *allocator = c10::hip::HIPCachingAllocator::get();
@@ -527,10 +558,12 @@ double peak_mib() {
 PYBIND11_MODULE(_native, m) {
   m.def("roi_align", &roi_align);
   m.def("affine", &affine);
+  m.def("affine_sample", &affine_sample);
   m.def("modulated_deform_conv", &modulated_deform_conv);
   m.def("deform_conv", &deform_conv);
   m.def("deform_warp", &deform_warp);
   m.def("elastic_warp", &elastic_warp);
   m.def("upload", &upload);
+  m.def("window_roi", &window_roi);
   m.def("peak_mib", &peak_mib);
 }

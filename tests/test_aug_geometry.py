@@ -125,3 +125,19 @@ def test_elastic_field_keeps_the_control_grids_type(grid, dtype):
         stage.params = params[:points, :points, :points]
         field = stage.dense_field(torch.device("cuda"))
         assert field.dtype == dtype and field.shape == (3, 20, 24, 28)
+
+
+def test_native_window_rois_are_the_arrays_rows():
+    """The roi of one window, built natively, has the bits of geometry.window_rois."""
+    from medvision_amd._lib import native
+    rng = np.random.default_rng(8)
+    for k in range(200):
+        dim = 2 + k % 2
+        start = [int(v) for v in rng.integers(0, 40, dim)] if k % 3 else [0.0] * dim
+        end = [s + float(v) for s, v in zip(start, rng.uniform(0.1, 300, dim))]
+        scales, shifts, rotate = list(rng.uniform(0.5, 1.7, dim)), [rng.uniform(-0.3, 0.3) for _ in range(dim)], rng.uniform(-4, 4)
+        want = geometry.window_rois(dim, start, end, scales, shifts, [rotate], index=np.arange(1))
+        got = native.window_roi(dim, start, end, scales, shifts, rotate, torch.device("cpu"))
+        assert got.dtype == torch.float32 and np.array_equal(got.numpy(), want)
+    with pytest.raises(RuntimeError):
+        native.window_roi(3, [0.0] * 3, [1.0] * 3, [1.0] * 2, [0.0] * 3, 0.0, torch.device("cpu"))
