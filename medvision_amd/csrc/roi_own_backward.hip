@@ -19,10 +19,11 @@
 // channels; summed in LDS boxes per roi and added to memory, the boxes' scan and 64-byte global atomics (21 G a second)
 // took the time.  Here the additions are products (70 GFLOP with what the tiles' padding wastes), the corner weights are
 // added once per sample instead of once per channel, and what bounds the kernel is the samples' arithmetic (every
-// cell is worked out by each of the ~10 tiles it reaches) and the conversion of the tables: vector issue 65 %, waits 46 % of the
-// wavefronts' time, LDS 9 %, matrix cores 3 %.
+// cell is worked out by each of the ~10 tiles it reaches) and the conversion of the tables: vector issue 70 %, waits 40 % of the
+// wavefronts' time, LDS 14 %.  A sample's eight corners are added without branches, those outside the tile as zeros, and in tiles off the image's border
+// its voxels are its position's floor: 358 us, 440 with a branch per corner and the clamped taps everywhere.
 // Small tiles: a tile's products are dense, and cells that reach it fill a larger one less.
-// Training step of 1000 rois with 7^3 cells on [2,64,48,96,96] fp16: 2080 -> 700 us, of which this kernel takes 444 us (26 us for
+// Training step of 1000 rois with 7^3 cells on [2,64,48,96,96] fp16: 2080 -> 550 us, of which this kernel takes 358 us (26 us for
 // the layout; the box kernel, its fp32 sums and their fold took 1.8 ms).
 #include "common.hpp"
 #include "roi_geometry.hpp"
@@ -159,6 +160,13 @@ __global__ __launch_bounds__(256) void roi_own_layout_kernel(const U *__restrict
 __device__ __forceinline__ void own_wave_sync() {   // LDS of one wavefront is in order: only the compiler has to keep it
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
+}
+
+// round(x) for 0 <= x < 2^31 in one instruction
+__device__ __forceinline__ unsigned own_round(float x) {
+  unsigned r;
+  asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+  return r;
 }
 
 typedef float own_acc __attribute__((ext_vector_type(16)));
@@ -315,6 +323,8 @@ __global__ __launch_bounds__(kOwnThreads, 3) void roi_own_backward_kernel(const 
   const double mid[3] = {t0[0] + 0.5 * (TX - 1), t0[1] + 0.5 * (TY - 1), t0[2] + 0.5 * (TZ - 1)};
   constexpr double ext[3] = {0.5 * (TX - 1), 0.5 * (TY - 1), 0.5 * (TZ - 1)};
 
+  // No sample that reaches the tile is moved onto the image's border (order 1).
+  const bool interior = p.order == 1 && t0[0] > 0 && t0[0] + TX < p.W && t0[1] > 0 && t0[1] + TY < p.H && (TZ == 1 || (t0[2] > 0 && t0[2] + TZ < p.D));
   if (threadIdx.x == 0) special = 0;
   bool any = false;   // the tile has a roi (the same for all threads)
 
@@ -462,6 +472,8 @@ __global__ __launch_bounds__(kOwnThreads, 3) void roi_own_backward_kernel(const 
             const unsigned cx = packed & 1023u, cy = (packed >> 10) & 1023u, cz = packed >> 20;
             if (part == 0) rows[columns + k] = n * cells + (cz * p.oh + cy) * p.ow + cx;
             unsigned *const column = table + columns + k;
+            unsigned *const aside = column + (part & 15) * kOwnPitch;   // (lanes of one cell apart; 15 voxels and the farthest corner are in the table)
+            static_assert(15 + ((TZ > 1 ? TY : 0) + 1) * TX + 1 < kOwnVoxels, "room for every corner");
             const double bx = g.start[0] + cx * g.bin[0], by = g.start[1] + cy * g.bin[1], bz = g.start[2] + cz * g.bin[2];
             for (int s = part; s < count; s += parts) {
               int s1, s2;
@@ -481,20 +493,37 @@ __global__ __launch_bounds__(kOwnThreads, 3) void roi_own_backward_kernel(const 
                 ry = g.rot[3] * x + g.rot[4] * y + g.rot[5] * z + g.centre[1];
                 rz = p.ndim == 3 ? g.rot[6] * x + g.rot[7] * y + g.rot[8] * z + g.centre[2] : 0.0;
               }
-              int xi[2], yi[2], zi[2];
-              float fx, fy, fz;
-              if (!clamped_tap<float>(rz, p.D, zi[0], zi[1], fz, p.order) || !clamped_tap<float>(ry, p.H, yi[0], yi[1], fy, p.order) ||
-                  !clamped_tap<float>(rx, p.W, xi[0], xi[1], fx, p.order))
-                continue;
+              // the first of the sample's two voxels along each axis, in the tile, and the fraction to the second one
+              int ix, iy, iz = 0;
+              float fx, fy, fz = 0.f;
+              bool inside = true;
+              if (interior) {
+                const double gx = floor(rx), gy = floor(ry), gz = floor(rz);
+                fx = static_cast<float>(rx - gx); fy = static_cast<float>(ry - gy);
+                ix = static_cast<int>(gx) - t0[0]; iy = static_cast<int>(gy) - t0[1];
+                if (TZ > 1) {
+                  fz = static_cast<float>(rz - gz);
+                  iz = static_cast<int>(gz) - t0[2];
+                }
+              } else {
+                int hi;   // (the next voxel, or the same with a fraction of 0)
+                inside = clamped_tap<float>(rz, p.D, iz, hi, fz, p.order) && clamped_tap<float>(ry, p.H, iy, hi, fy, p.order) &&
+                         clamped_tap<float>(rx, p.W, ix, hi, fx, p.order);
+                ix -= t0[0]; iy -= t0[1]; iz -= t0[2];
+              }
+              const auto in = [&](int i, int n, float w) { return inside && static_cast<unsigned>(i) < static_cast<unsigned>(n) && w != 0.f; };
               const float wx[2] = {1.f - fx, fx}, wy[2] = {1.f - fy, fy}, wz[2] = {1.f - fz, fz};
+              const bool ox[2] = {in(ix, TX, wx[0]), in(ix + 1, TX, wx[1])}, oy[2] = {in(iy, TY, wy[0]), in(iy + 1, TY, wy[1])},
+                         oz[2] = {in(iz, TZ, wz[0]), in(iz + 1, TZ, wz[1])};
+              unsigned *const first_corner = column + ((iz * TY + iy) * TX + ix) * kOwnPitch;
+              // (corners outside the tile, or of weight 0, add nothing to a place that exists: no branches)
 #pragma unroll
-              for (int c = 0; c < 8; c++) {
-                const unsigned vx = xi[c & 1] - t0[0], vy = yi[(c >> 1) & 1] - t0[1], vz = zi[c >> 2] - t0[2];
-                const float w = wz[c >> 2] * wy[(c >> 1) & 1] * wx[c & 1];
-                if (vx < TX && vy < TY && vz < TZ && w != 0.f)
-                  __hip_atomic_fetch_add(column + ((vz * TY + vy) * TX + vx) * kOwnPitch,
-                                         max(static_cast<unsigned>(__float2int_rn(w * quanta)), 1u), __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_WORKGROUP);
+              for (int c = 0; c < (TZ > 1 ? 8 : 4); c++) {
+                const int bx_ = c & 1, by_ = (c >> 1) & 1, bz_ = c >> 2;
+                const bool on = ox[bx_] && oy[by_] && oz[bz_];
+                unsigned *const to = (on ? first_corner : aside) + ((bz_ * TY + by_) * TX + bx_) * kOwnPitch;
+                const unsigned term = max(own_round(wz[bz_] * wy[by_] * wx[bx_] * quanta), 1u);
+                __hip_atomic_fetch_add(to, on ? term : 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
               }
             }
           }
