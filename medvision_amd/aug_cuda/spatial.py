@@ -395,6 +395,8 @@ class CudaRandomElasticDeformation(CudaAugBase):
     """Random displacements on a coarse control grid (two locked border layers), upsampled to a
     dense field with the order-3 affine engine and applied with the displacement-field warp."""
 
+    _field = _device_grid = _field_device = None       # (also of stages pickled before they had these)
+
     def __init__(self, p, num_control_points=8, max_displacement=0.8, order=3):
         super().__init__()
         self.p = p
@@ -412,6 +414,12 @@ class CudaRandomElasticDeformation(CudaAugBase):
     @property
     def canBackward(self):
         return True
+
+    def __setstate__(self, state):
+        state = dict(state)
+        if 'tmp_params' in state:
+            state['_field'] = state.pop('tmp_params')
+        self.__dict__.update(state)
 
     def _forget_field(self):
         self._field = self._device_grid = self._field_device = None

@@ -433,7 +433,7 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
           static_cast<unsigned>(reinterpret_cast<unsigned long long>((__attribute__((address_space(3))) unsigned char *)ring_lds)));
       auto to_lds = [&](const Run &run, const int piece_at, const int place) {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                     : : "s"(__builtin_amdgcn_readfirstlane(ring_at + place * 1024)), "v"(lane * 16 + piece_at * 1024), "s"(run.src) : "memory");
+                     : : "s"(__builtin_amdgcn_readfirstlane(ring_at + place * 1024)), "v"(lane * 16 + piece_at * 1024), "s"(run.src) : "memory", "m0");
       };
       auto bring = [&](const Run &run, int place, const int from, const int to) {
 #pragma unroll 1
@@ -606,16 +606,21 @@ static size_t brick_partial_bytes(const RoiProblem &p) {
   return parts > 1 ? static_cast<size_t>(brick_waves(p)) * parts * kBrickChannels * 512 * sizeof(float) : 0;
 }
 
+// Lists grow with rois times bricks: where they would take more than 256 MB and more than the fp32 copy of the gradient of the kernel
+// with atomics (more than 512 rois per channel on large maps), that kernel stays.
 size_t roi_brick_workspace(int dtype, const RoiProblem &p) {
   if (!roi_brick_applies(dtype, p)) return 0;
-  return brick_tables_bytes(p) + brick_lists_bytes(p) + brick_partial_bytes(p) + static_cast<size_t>(p.R) * sizeof(BrickRoi) +
-         static_cast<size_t>(p.C) * p.od * p.oh * p.ow * 2 + kBrickPad;
+  const size_t bytes = brick_tables_bytes(p) + brick_lists_bytes(p) + brick_partial_bytes(p) + static_cast<size_t>(p.R) * sizeof(BrickRoi) +
+                       static_cast<size_t>(p.C) * p.od * p.oh * p.ow * 2 + kBrickPad;
+  const size_t copy = static_cast<size_t>(p.N) * p.C * p.D * p.H * p.W * sizeof(float);
+  return bytes <= std::max(copy, static_cast<size_t>(256) << 20) ? bytes : 0;
 }
 
 // Writes all of grad_input.  -1: not for these kernels, or a workspace that is too small for them.
 int roi_brick_backward(const void *grad_output, const void *rois, void *grad_input, int dtype, const RoiProblem &p, void *workspace,
                        size_t capacity, hipStream_t s) {
-  if (!roi_brick_applies(dtype, p) || capacity < roi_brick_workspace(dtype, p) || reinterpret_cast<uintptr_t>(workspace) % 16 != 0) return -1;
+  const size_t wanted = roi_brick_workspace(dtype, p);
+  if (wanted == 0 || capacity < wanted || reinterpret_cast<uintptr_t>(workspace) % 16 != 0) return -1;
   float *const tables = static_cast<float *>(workspace);
   unsigned *const lists = reinterpret_cast<unsigned *>(static_cast<char *>(workspace) + brick_tables_bytes(p));
   unsigned *const lengths = lists + brick_count(p) * p.R;

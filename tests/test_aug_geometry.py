@@ -141,3 +141,18 @@ def test_native_window_rois_are_the_arrays_rows():
         assert got.dtype == torch.float32 and np.array_equal(got.numpy(), want)
     with pytest.raises(RuntimeError):
         native.window_roi(3, [0.0] * 3, [1.0] * 3, [1.0] * 2, [0.0] * 3, 0.0, torch.device("cpu"))
+
+
+def test_elastic_stage_restored_from_an_older_state():
+    """A state that holds the dense field under its public name, and a stage that never ran."""
+    import pickle
+    import numpy as np
+    from medvision_amd.aug_cuda import CudaRandomElasticDeformation
+    stage = CudaRandomElasticDeformation(1.0, 6, 0.5)
+    old = {k: v for k, v in stage.__dict__.items() if k not in ('_field', '_device_grid', '_field_device')}
+    for field in (None, np.ones(3)):
+        again = CudaRandomElasticDeformation.__new__(CudaRandomElasticDeformation)
+        again.__setstate__({**old, 'tmp_params': field})
+        assert again.tmp_params is field and again._field is field
+        assert again._device_grid is None
+    assert pickle.loads(pickle.dumps(stage)).tmp_params is None

@@ -1,0 +1,21 @@
+"""Scratch memory of the backward pass of fp16 heads on volumes: lists of rois per brick do not outgrow the kernel with atomics."""
+import pytest
+
+from medvision_amd import _lib
+
+
+@pytest.mark.parametrize("dims,rois,lists", [
+    ((2, 256, 24, 96, 96), 4000, True),
+    ((1, 16, 64, 128, 128), 4000, True),        # 2048 bricks
+    ((1, 16, 256, 256, 256), 8000, True),       # 32768 bricks: 1.05 GB of lists, a copy of 1.07 GB
+    ((1, 16, 256, 256, 256), 8300, False),
+    ((8, 16, 64, 128, 128), 60000, False),      # 3.9 GB of lists
+])
+def test_lists_are_no_larger_than_the_copy(dims, rois, lists):
+    lib, code = _lib.load(), _lib.MV_F16
+    copy = lib.mv_roi_align_backward_workspace_bytes(code, *dims)
+    asked = lib.mv_roi_align_backward_write_workspace_bytes(code, 3, 0, *dims, rois, 7, 7, 7, 2, 1)
+    assert asked <= max(copy, 256 << 20)
+    assert asked >= copy
+    if not lists:
+        assert asked == copy
