@@ -433,7 +433,7 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
           static_cast<unsigned>(reinterpret_cast<unsigned long long>((__attribute__((address_space(3))) unsigned char *)ring_lds)));
       auto to_lds = [&](const Run &run, const int piece_at, const int place) {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                     : : "s"(__builtin_amdgcn_readfirstlane(ring_at + place * 1024)), "v"(lane * 16 + piece_at * 1024), "s"(run.src) : "memory", "m0");
+                     : : "s"(__builtin_amdgcn_readfirstlane(ring_at + place * 1024)), "v"(lane * 16 + piece_at * 1024), "s"(run.src) : "memory");
       };
       auto bring = [&](const Run &run, int place, const int from, const int to) {
 #pragma unroll 1
@@ -578,12 +578,18 @@ static long brick_count(const RoiProblem &p) {
 }
 static long brick_waves(const RoiProblem &p) { return brick_count(p) * ((p.C + kBrickChannels - 1) / kBrickChannels); }
 
-// Workgroups that share a brick and 16 channels, for maps of fewer than 1024 such pairs whose bricks have many rois each; their sums go
-// through memory (64 KB for each) and another launch.  Forward and backward pass, one workgroup and this many: [4,64,11,27,28] with 3510 rois
-// of 7^3 cells 873 and 435 us, [2,83,24,29,25] with 484 of 4^3 271 and 190; [2,24,35,93,28] with 369 of 2^3, four rois per five bricks, 59 and 66.
+// Workgroups that share a brick and 16 channels, for maps of few such pairs whose bricks have many rois each (a roi is one serial chain for a
+// wavefront); their sums go through memory (32 KB for a wavefront) and another launch.  2048 wavefronts run at a time.  Forward and backward
+// pass, one workgroup and as many as make 2048 wavefronts: [4,64,11,27,28] with 3510 rois of 7^3 cells 873 and 435 us, [2,83,24,29,25] with 484
+// of 4^3 271 and 190; [2,24,35,93,28] with 369 of 2^3, four rois per five bricks, 59 and 66.
+// Lists differ in length, and the longest is the end of the launch: 4096 wavefronts, half as long, even that out where lists are long.  2048 and
+// 4096: [1,128,36,27,46] with 2424 rois of 4^3, 20 per brick, 530 and 403 us, [1,128,9,76,38] with 2543 of 7^3, 25 per brick, 575 and 453,
+// [1,128,12,48,65] with 932 of 5^3, 9 per brick, 331 and 315; [1,64,22,57,38] with 243 of 7^3, 2 per brick, 80 and 89, [2,32,19,95,25] with 568, 2
+// per brick, 70 and 78.
 static int brick_parts(const RoiProblem &p) {
   if (4L * p.R < 5 * brick_count(p)) return 1;
-  return static_cast<int>(std::max(std::min(2048 / brick_waves(p), 16L), 1L));
+  const long wavefronts = p.R >= 8 * brick_count(p) ? 4096 : 2048;
+  return static_cast<int>(std::max(std::min(wavefronts / brick_waves(p), 16L), 1L));
 }
 
 bool roi_brick_applies(int dtype, const RoiProblem &p) {

@@ -92,3 +92,19 @@ def test_keeps_to_its_workspace(oracle):
                                                      1.0, 2, 1, 1, _lib.ptr(room), given, _lib.stream_of(grad)))
         assert bool((room[given:] == 0x5a).all())
         assert_close(grad, want, TOL, f"{given} bytes")
+
+
+@pytest.mark.parametrize("images,channels,size,rois", [
+    (1, 128, (32, 40, 64), 1300),    # 1280 pairs of a brick and 16 channels: three workgroups each
+    (1, 128, (32, 40, 64), 1279),    # one roi short of eight per brick: one
+    (1, 256, (9, 16, 17), 110),      # the most that share one
+])
+def test_more_workgroups_share_bricks_of_many_rois(oracle, images, channels, size, rois):
+    from medvision_amd.ops.roi_align_nd import roi_align_3d
+    g = wl.gen(rois)
+    boxes = boxes_of(g, images, size, rois, 7)
+    x = torch.zeros(images, channels, *size, dtype=torch.float16, device=DEV, requires_grad=True)
+    out = roi_align_3d(x, boxes.to(DEV), (2, 3, 2), 1.0, 1, 1)
+    gy = torch.randn(out.shape, generator=g).half()
+    want = oracle.roi_align_backward(gy, boxes, x.shape, 1.0, 1, True, 1, False).reshape(x.shape)
+    assert_close(torch.autograd.grad(out, x, gy.to(DEV))[0], want, TOL, "gradient")
