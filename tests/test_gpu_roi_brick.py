@@ -108,3 +108,39 @@ def test_more_workgroups_share_bricks_of_many_rois(oracle, images, channels, siz
     gy = torch.randn(out.shape, generator=g).half()
     want = oracle.roi_align_backward(gy, boxes, x.shape, 1.0, 1, True, 1, False).reshape(x.shape)
     assert_close(torch.autograd.grad(out, x, gy.to(DEV))[0], want, TOL, "gradient")
+
+
+@pytest.mark.parametrize("scale", [1e-5, 1e-6])
+def test_small_gradients(oracle, scale):
+    """Gradients in the subnormal range: the result's own rounding (half a step of 2^-24) is what may be left, with the same again
+    for the sums' operands."""
+    from medvision_amd.ops.roi_align_nd import roi_align_3d
+    g = wl.gen(8)
+    boxes = boxes_of(g, 1, (24, 40, 40), 300, 12)
+    x = torch.zeros(1, 128, 24, 40, 40, dtype=torch.float16, device=DEV, requires_grad=True)
+    out = roi_align_3d(x, boxes.to(DEV), (7, 7, 7), 1.0, 2, 1)
+    gy = (torch.randn(out.shape, generator=g) * scale).half()
+    want = torch.as_tensor(oracle.roi_align_backward(gy, boxes, x.shape, 1.0, 2, True, 1, False)).double().reshape(x.shape)
+    got = torch.autograd.grad(out, x, gy.to(DEV))[0].cpu().double()
+    own = (want.half().double() - want).norm()
+    # (weights of 11 bits, twice: below 1e-3 of the result)
+    assert (got - want).norm() <= 1.1 * own + 1e-3 * want.norm()
+
+
+def test_gradients_beyond_their_scale(oracle):
+    """Large gradients in some cells of a roi and ordinary ones in the rest."""
+    from medvision_amd.ops.roi_align_nd import roi_align_3d
+    g = wl.gen(9)
+    boxes = boxes_of(g, 2, (9, 17, 33), 60, 12)
+    x = torch.zeros(2, 128, 9, 17, 33, dtype=torch.float16, device=DEV, requires_grad=True)
+    out = roi_align_3d(x, boxes.to(DEV), (7, 7, 7), 1.0, 2, 1)
+    gy = torch.randn(out.shape, generator=g).half()
+    gy[::3, ::5] *= 4000
+    want = oracle.roi_align_backward(gy, boxes, x.shape, 1.0, 2, True, 1, False).reshape(x.shape)
+    got = torch.autograd.grad(out, x, gy.to(DEV))[0].cpu().double()
+    want = torch.as_tensor(want).double()
+    fits = want.abs() < 60000
+    assert_close(torch.where(fits, got, want), want, TOL, "gradient")
+    ordinary = torch.ones(128, dtype=torch.bool)
+    ordinary[::5] = False
+    assert_close(got[:, ordinary], want[:, ordinary], TOL, "channels of ordinary gradients")
