@@ -494,8 +494,8 @@ __global__ __launch_bounds__(kOwnThreads, 3) void roi_own_backward_kernel(const 
                 rz = p.ndim == 3 ? g.rot[6] * x + g.rot[7] * y + g.rot[8] * z + g.centre[2] : 0.0;
               }
               // the first of the sample's two voxels along each axis, in the tile, and the fraction to the second one
-              int ix, iy, iz = 0;
-              float fx, fy, fz = 0.f;
+              int ix = 0, iy = 0, iz = 0;
+              float fx = 0.f, fy = 0.f, fz = 0.f;
               bool inside = true;
               if (interior) {
                 const double gx = floor(rx), gy = floor(ry), gz = floor(rz);
@@ -723,9 +723,14 @@ bool roi_own_applies(int dtype, const RoiProblem &p) {
   const double per_voxel = static_cast<double>(cells) * p.R / (static_cast<double>(p.N) * p.D * p.H * p.W);
   if (p.ndim == 3 && (dtype == MV_F32 ? p.C < 64 && per_voxel > 2.0 : p.C < 32 && per_voxel > 8.0)) return false;
   // Rois far apart on a large fp32 map with one sample a cell (or an adaptive grid, which often is one): most of the time is the
-  // writing of zeros, and the fill before the atomics does that faster.  [4,128,36,101,44], adaptive: 16 rois 155 us there, 186
-  // here; 120 rois 349, 382; 494 rois (0.27 cells per voxel) 949, 916.
-  if (p.ndim == 3 && dtype == MV_F32 && p.sampling_ratio < 2 && per_voxel < 0.25 && own_tiles(p) * own_groups(p) > 4096) return false;
+  // writing of zeros, and the fill before the atomics does that faster.  What the atomics cost is the voxels of the boxes, whatever their
+  // cells, so the line is in rois per voxel: of 46 drawn training steps with boxes of 1 - 24 voxels all 28 from 1 / 1600 on are faster here, 1.05 -
+  // 2.6 times ([2,256,17,72,115], 760 rois of 4^3 cells, 750 -> 481 us; [4,128,36,120,39], 347 of 7^3, 867 -> 739; [4,32,31,61,109], 1012 of
+  // 5^3, 459 -> 323), those below 1 / 2000 mostly not ([4,128,28,55,117], 231 of 7^3, 467 -> 520; [4,256,37,107,87], 266 of 5^3, 1276 -> 1484).
+  // The error against 64 bits is a third (1.0e-7 and 3.2e-7, six of them).
+  const double voxels = static_cast<double>(p.N) * p.D * p.H * p.W;
+  if (p.ndim == 3 && dtype == MV_F32 && p.sampling_ratio < 2 && per_voxel < 0.25 && p.R * 1600.0 < voxels && own_tiles(p) * own_groups(p) > 4096)
+    return false;
   return own_tiles(p) * own_groups(p) < (1L << 31) - 8 && cells * p.R / 32 * own_groups(p) < (1L << 30);
 }
 
