@@ -290,6 +290,38 @@ size_t dcn_columns_workspace_bytes(const DcnDims &s, int dtype) {
          columns_align(static_cast<size_t>(s.Cout / 16) * columns_steps(s, static_cast<int>(16 / es)) * 1024);
 }
 
+// images (the kernels with four corners)
+static bool columns_image(const DcnDims &s) { return s.nd == 2 && s.D == 1 && s.kd == 1 && s.pd == 0; }
+
+// What a workgroup takes: `positions` of an image or volume, `waves` wavefronts of `blocks` blocks of 16 output channels each; the grid is
+// tiles x chunks x samples.
+struct ColumnsPlan {
+  int positions, waves, blocks;
+  long tiles, chunks;
+};
+
+void dcn_columns_plan(const DcnDims &s, int dtype, ColumnsPlan &plan) {
+  // Positions per workgroup: 32 as long as that gives every compute unit two workgroups, otherwise 16; then fewer output
+  // channels per workgroup (each share repeats the samples) until there is one for every compute unit.
+  int pt = 32, obw = s.opg <= 64 ? 1 : (s.opg <= 128 ? 2 : 4);
+  auto groups_of = [&](int p, int o) { return (s.Q + p - 1) / p * s.B * s.groups * ((s.opg + 64 * o - 1) / (64 * o)); };
+  if (groups_of(pt, obw) < 512) pt = 16;
+  while (obw > 1 && groups_of(pt, obw) < 256) obw /= 2;
+  // Wide images: 64 positions and eight wavefronts per workgroup, as long as enough of them remain.  Their time goes in steps of 256
+  // workgroups: fp16 [256 -> 256, 64 x n] 44 against 40 us with n = 128, 46 and 51 with 160, 49 and 65 with 224, 66 and 64 with 300, 68 and 88 with 450,
+  // 100 and 119 with 700; fp32, bound by its products too, 326 and 277 us with 350, 330 and 367 with 450, 489 and 452 with 520, 494 and 537 with 700.
+  // Not where their last tile holds much that does not exist (small images in large batches: fp16 [200, 256 -> 256] of 7 x 7 43 us and 65 with 32,
+  // 10 x 10 64 and 87; of 5 x 5, as long as 7 x 7 there, 36 with 32, 4 x 4 24).
+  const long positions64 = (s.Q + 63) / 64 * 64, positions32 = (s.Q + 31) / 32 * 32;
+  const bool wide = columns_image(s) && s.opg > 128 && groups_of(64, 4) >= (dtype == MV_F32 ? 640 : 160) && positions64 * 8 <= positions32 * 9;
+  plan.positions = wide ? 64 : pt;
+  plan.waves = wide ? 8 : 4;
+  plan.blocks = wide ? 2 : obw;
+  const int rows = 16 * plan.waves * plan.blocks;   // (as the kernel has it: its groups and chunks are numbered by them)
+  plan.tiles = (s.Q + plan.positions - 1) / plan.positions;
+  plan.chunks = s.groups * static_cast<long>((s.opg + rows - 1) / rows);
+}
+
 template <typename T, int NC>
 static int columns_run(const void *x, const void *off, const void *mask, const void *wt, const void *bias, void *y,
                        const DcnDims &s, void *workspace, hipStream_t stream) {
@@ -309,54 +341,36 @@ static int columns_run(const void *x, const void *off, const void *mask, const v
     st = dcn_shared_taps_forward(xt, off, mask, wf, bias, y, s, sizeof(T) == 2 && std::is_same<T, __half>::value ? MV_F16 : MV_BF16, stream);
     if (st >= 0) return st;
   }
-  // Positions per workgroup: 32 as long as that gives every compute unit two workgroups, otherwise 16; then fewer output
-  // channels per workgroup (each share repeats the samples) until there is one for every compute unit.
-  int pt = 32, obw = s.opg <= 64 ? 1 : (s.opg <= 128 ? 2 : 4);
-  auto groups_of = [&](int p, int o) { return (s.Q + p - 1) / p * s.B * s.groups * ((s.opg + 64 * o - 1) / (64 * o)); };
-  if (groups_of(pt, obw) < 512) pt = 16;
-  while (obw > 1 && groups_of(pt, obw) < 256) obw /= 2;
+  ColumnsPlan plan;
+  dcn_columns_plan(s, sizeof(T) == 2 ? MV_F16 : MV_F32, plan);
+  MV_REQUIRE(plan.tiles < (1L << 31) && plan.chunks <= 65535, "grid too large");
+  const dim3 grid(static_cast<unsigned>(plan.tiles), static_cast<unsigned>(plan.chunks), s.B);
   // 16-byte pieces of a corner that a load takes from each position: eight, whole 128-byte lines, where a unit's channels allow it.
   const bool eights = std::min(s.cpd, s.cpg) % (8 * Mfma<T>::kPiece) == 0;
-  // Wide images: 64 positions and eight wavefronts per workgroup, as long as enough of them remain.  Their time goes in steps of 256
-  // workgroups: fp16 [256 -> 256, 64 x n] 44 against 40 us with n = 128, 46 and 51 with 160, 49 and 65 with 224, 66 and 64 with 300, 68 and 88 with 450,
-  // 100 and 119 with 700; fp32, bound by its products too, 326 and 277 us with 350, 330 and 367 with 450, 489 and 452 with 520, 494 and 537 with 700.
-  const bool wide = NC == 4 && s.opg > 128 && groups_of(64, 4) >= (sizeof(T) == 2 ? 160 : 640);
-  if (wide) pt = 64;
-  const long qblocks = (s.Q + pt - 1) / pt;
-  const long rows = static_cast<long>(s.groups) * ((s.opg + 64 * obw - 1) / (64 * obw));
-  MV_REQUIRE(qblocks < (1L << 31) && rows <= 65535, "grid too large");
-  const dim3 grid(static_cast<unsigned>(qblocks), static_cast<unsigned>(rows), s.B);
 #define MV_COLUMNS_LP(PTV, OBWV, WV, LPV)                                                                              \
   hipLaunchKernelGGL((dcn_forward_columns_kernel<T, NC, PTV, OBWV, WV, LPV>), grid, dim3(kWave * WV), 0, stream, xt,     \
                      static_cast<const T *>(off), static_cast<const T *>(mask), wf, static_cast<const T *>(bias), static_cast<T *>(y), s)
 #define MV_COLUMNS(PTV, OBWV, WV)                                                                                      \
-  do {                                                                                                                 \
+  if (plan.positions == PTV && plan.blocks == OBWV && plan.waves == WV) {                                              \
     if (eights) MV_COLUMNS_LP(PTV, OBWV, WV, 8);                                                                       \
     else MV_COLUMNS_LP(PTV, OBWV, WV, 4);                                                                              \
-  } while (0)
-#define MV_COLUMNS_PT(PTV)                                                                                             \
-  do {                                                                                                                 \
-    if (obw == 1) MV_COLUMNS(PTV, 1, 4);                                                                               \
-    else if (obw == 2) MV_COLUMNS(PTV, 2, 4);                                                                          \
-    else MV_COLUMNS(PTV, 4, 4);                                                                                        \
-  } while (0)
-  bool launched = false;
-  if constexpr (NC == 4) {
-    if (wide) { MV_COLUMNS(64, 2, 8); launched = true; }
+    return check_launch("dcn_forward_columns_kernel");                                                                 \
   }
-  if (!launched) {
-    if (pt == 32) MV_COLUMNS_PT(32);
-    else MV_COLUMNS_PT(16);
-  }
-#undef MV_COLUMNS_PT
+  if constexpr (NC == 4) { MV_COLUMNS(64, 2, 8) }
+  MV_COLUMNS(32, 1, 4)
+  MV_COLUMNS(32, 2, 4)
+  MV_COLUMNS(32, 4, 4)
+  MV_COLUMNS(16, 1, 4)
+  MV_COLUMNS(16, 2, 4)
+  MV_COLUMNS(16, 4, 4)
 #undef MV_COLUMNS
 #undef MV_COLUMNS_LP
-  return check_launch("dcn_forward_columns_kernel");
+  return fail(MV_INVALID_ARGUMENT, "no kernel for this plan");
 }
 
 int dcn_columns_forward(const void *x, const void *off, const void *mask, const void *wt, const void *bias, void *y,
                         const DcnDims &s, int dtype, void *workspace, hipStream_t stream) {
-  const bool image = s.nd == 2 && s.D == 1 && s.kd == 1 && s.pd == 0;
+  const bool image = columns_image(s);
 #define MV_COLUMNS_AS(T) \
   (image ? columns_run<T, 4>(x, off, mask, wt, bias, y, s, workspace, stream) : columns_run<T, 8>(x, off, mask, wt, bias, y, s, workspace, stream))
   if (dtype == MV_F16) return MV_COLUMNS_AS(__half);

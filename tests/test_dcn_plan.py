@@ -102,3 +102,36 @@ def test_a_volume_of_more_workgroups_than_a_row():
     shape = _plan(_lib.MV_F32, 16, 32, 32, (128, 180, 182), 3, 1, 2)
     assert shape.nbd * shape.nbh * shape.nbw * 16 * (32 // 8) == 4239360
     assert _grid(4239360, 1024).y == 2
+
+
+class _Columns(ctypes.Structure):   # ColumnsPlan (csrc/dcn_forward_columns.hip)
+    _fields_ = [(n, ctypes.c_int) for n in ("positions", "waves", "blocks")] + [(n, ctypes.c_long) for n in ("tiles", "chunks")]
+
+
+def _columns(code, batch, cin, cout, size, groups):
+    nd = len(size)
+    kernel, n = (1,) * (3 - nd) + (3,) * nd, (1,) * (3 - nd) + tuple(size)
+    pad = tuple(k // 2 for k in kernel)
+    dims = _Dims(batch, cin, *n, cout, *kernel, 1, 1, 1, *pad, 1, 1, 1, groups, 1, nd, *n, math.prod(kernel), cin // groups, cout // groups, cin,
+                 math.prod(n), math.prod(n))
+    fn = _lib.load()._ZN2mv16dcn_columns_planERKNS_7DcnDimsEiRNS_11ColumnsPlanE
+    fn.restype, fn.argtypes = None, [ctypes.POINTER(_Dims), ctypes.c_int, ctypes.POINTER(_Columns)]
+    plan = _Columns()
+    fn(ctypes.byref(dims), code, ctypes.byref(plan))
+    return plan
+
+
+@pytest.mark.parametrize("code", [_lib.MV_F32, _lib.MV_F16, _lib.MV_BF16])
+@pytest.mark.parametrize("groups", [1, 2, 3])
+@pytest.mark.parametrize("rows", [16, 64, 80, 128, 144, 256, 272, 512, 528])
+def test_columns_grid_covers_the_layer_once(code, groups, rows):
+    """The workgroups that start are those that the kernel numbers: its tiles of positions and, per group, its chunks of output channels."""
+    kernels = {(16, 4, 1), (16, 4, 2), (16, 4, 4), (32, 4, 1), (32, 4, 2), (32, 4, 4)}
+    for size in [(1, 1), (3, 3), (4, 4), (17, 1), (5, 5), (7, 7), (8, 8), (9, 9), (14, 14), (33, 47), (100, 152), (2, 2, 4), (5, 7, 11), (48, 48, 48)]:
+        q = math.prod(size)
+        for batch in [*range(1, 20), *range(20, 700, 7), 1024, 4096]:
+            plan = _columns(code, batch, 32 * groups, rows * groups, size, groups)
+            what = f"{size} x {batch}"
+            assert (plan.positions, plan.waves, plan.blocks) in kernels | ({(64, 8, 2)} if len(size) == 2 else set()), what
+            assert plan.tiles == -(-q // plan.positions), what
+            assert plan.chunks == groups * -(-rows // (16 * plan.waves * plan.blocks)), what

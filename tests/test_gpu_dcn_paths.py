@@ -127,3 +127,19 @@ def test_columns_of_whole_lines(oracle, dtype, batch, cin, cout, size, groups, d
     with torch.no_grad():
         y = modulated_deform_conv(*[t.to(DEV) for t in (x, off, mask, w, b)], 1, 1, 1, groups, dg)
     assert_close(y, oracle.dcn3d_forward(x, off, mask, w, b, 1, 1, 1, groups, dg), FWD_TOL[dtype], "forward")
+
+
+@pytest.mark.parametrize("dtype,batch,cin,cout,size", [
+    (torch.float16, 192, 32, 144, (4, 4)),      # few positions, many images: workgroups of fewer rows
+    (torch.bfloat16, 96, 32, 272, (3, 4)),
+    (torch.float16, 200, 16, 256, (3, 3)),
+    (torch.float16, 200, 16, 256, (7, 7)),      # 64 positions, of which 49
+    (torch.bfloat16, 300, 16, 144, (9, 9)),     # 32 positions: 64 would leave more than an eighth idle
+])
+def test_many_small_images(oracle, dtype, batch, cin, cout, size):
+    from medvision_amd.ops.modulated_deform_conv_2d import modulated_deform_conv
+    g = wl.gen(batch + cin + cout + sum(size))
+    x, off, mask, w, b = wl.dcn_inputs(g, batch, cin, cout, size, 3, 1, 1, dtype, 1, 1, 1)
+    with torch.no_grad():
+        y = modulated_deform_conv(*[t.to(DEV) for t in (x, off, mask, w, b)], 1, 1, 1, 1, 1)
+    assert_close(y, oracle.dcn3d_forward(x, off, mask, w, b, 1, 1, 1, 1, 1), FWD_TOL[dtype], "forward")
