@@ -172,34 +172,37 @@ __global__ __launch_bounds__(kBrickThreads) void roi_brick_lists_kernel(const ui
   if (threadIdx.x == 0) lengths[id] = have;
 }
 
-// The operands of the products: the weights Wy Wx and the sums P are rounded once each (11 bits; P that overflows makes a sum that is
-// not finite, see brick_careful), Wz is the sum of two numbers, side by side in K.  Where the first product's K has room, below eight rows of
-// cells, rows stand in it twice, the second time with what the rounding left of their weights.  Error against 64 bits, 40 heads (2.07e-4 of it
-// the result's own rounding): four rows 2.94e-4, seven 3.52e-4; 3.59e-4 without (12 of 812 us less), and 3.57e-4 with box-by-box sums, which
-// round twice as well.
-// P of small gradients would be a subnormal number of a few bits, so the weights Wy Wx stand there kBrickScale times as large.  A brick whose
-// sums do not come out finite with that is done again without.  (Gradients of 1e-5: error 5.6e-3 without it, 3.17e-3 with, of which 3.15e-3 is the
-// result's own rounding; box-by-box sums 4.2e-3.  64 and a look at every P, so that nothing is done twice: 860 instead of 820 us.)
-constexpr float kBrickScale = 16.f;
+// The operands of the products are fp16 numbers.  The weights Wy Wx and Wz are rounded to them (11 bits); where the first product's K has room,
+// below eight rows of cells, rows stand in it twice, the second time with what the rounding left of their weights.  The sums P stand in the
+// second product's K as two numbers, the second one what the first has left: they keep 22 bits.
+// Everything is scaled so that neither the largest nor the smallest gradients need a second look: Wy Wx by kBrickWeight, the first number of P by
+// 1 / 128 (64 cells of the type's largest still fit), its rest by kBrickWeight, and Wz by what makes the products' sum the result.
+// Error against 64 bits of heads with boxes up to 12 voxels (2.07e-4 of it the result's own rounding): four rows 2.86e-4, seven 3.45e-4,
+// eight 3.53e-4; box-by-box sums 3.61e-4.  Gradients of 1e-5: 2.17e-3 (own 2.15e-3), box by box 3.02e-3.  4000 rois x 256 channels x 7^3, forward and
+// backward pass, 494 us with P as one number, 544 with two; but with one number small gradients are lost unless it is scaled up, and where that
+// overflows the brick had to be done again (30 ms for gradients of 4000, 558 us now).
+constexpr float kBrickWeight = 16.f;
 typedef _Float16 brick_half4 __attribute__((ext_vector_type(4)));
-struct BrickLeft { brick_half4 high, low; };
 __device__ __forceinline__ brick_half4 brick_pack(const float (&w)[4]) {
   return __builtin_bit_cast(brick_half4, uint2{Mfma<__half>::pack2(w[0], w[1]), Mfma<__half>::pack2(w[2], w[3])});
 }
-__device__ __forceinline__ BrickLeft brick_left(const float (&w)[4]) {
-  BrickLeft l;
-  l.high = brick_pack(w);
-  float rest[4];
-#pragma unroll
-  for (int r = 0; r < 4; r++) rest[r] = w[r] - static_cast<float>(l.high[r]);
-  l.low = brick_pack(rest);
-  return l;
+__device__ __forceinline__ u32x4 brick_pair(const brick_half4 a, const brick_half4 b) {
+  const uint2 x = __builtin_bit_cast(uint2, a), y = __builtin_bit_cast(uint2, b);
+  return u32x4{x.x, x.y, y.x, y.y};
 }
-__device__ __forceinline__ float4_t brick_add(const BrickLeft &l, const float4_t &part, float4_t acc) {
-  const float p[4] = {part[0], part[1], part[2], part[3]};
-  const brick_half4 right = brick_pack(p);
-  const uint2 r = __builtin_bit_cast(uint2, right), lo = __builtin_bit_cast(uint2, l.low), hi = __builtin_bit_cast(uint2, l.high);
-  return Mfma<__half>::run16(u32x4{hi.x, hi.y, lo.x, lo.y}, u32x4{r.x, r.y, r.x, r.y}, acc);
+__device__ __forceinline__ u32x4 brick_left(const float (&w)[4]) {
+  const float large[4] = {w[0] * 128.f, w[1] * 128.f, w[2] * 128.f, w[3] * 128.f};
+  const float small[4] = {w[0] / kBrickWeight, w[1] / kBrickWeight, w[2] / kBrickWeight, w[3] / kBrickWeight};
+  return brick_pair(brick_pack(large), brick_pack(small));
+}
+__device__ __forceinline__ u32x4 brick_right(const float4_t &part) {
+  constexpr float kDown = 1.f / (128.f * kBrickWeight);
+  const float v[4] = {part[0] * kDown, part[1] * kDown, part[2] * kDown, part[3] * kDown};
+  brick_half4 high = brick_pack(v), rest;
+  asm("" : "+v"(high));   // (or the compiler forms it a second time, element by element, for the rest)
+#pragma unroll
+  for (int r = 0; r < 4; r++) rest[r] = static_cast<_Float16>(__builtin_fmaf(static_cast<float>(high[r]), -1.f / kDown, part[r]));
+  return brick_pair(high, rest);
 }
 
 // A region whose sums come out not finite, done again term by term and without the terms of weight 0.  Thread: one (y, x) of the
@@ -396,12 +399,11 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
   const unsigned *const list = lists + brick * p.R + begin;
   // [two channels][two rows of voxels]: z = quad % 2 * 4 + r of channel quad / 2 at voxel (y = col / 8, x = col % 8)
   float4_t acc[kBrickChannels / 2][4];
-#pragma unroll 1
-  for (float scale = kBrickScale;; scale = 1.f) {
 #pragma unroll
-    for (int i = 0; i < kBrickChannels / 2; i++)
+  for (int i = 0; i < kBrickChannels / 2; i++)
 #pragma unroll
-      for (int k = 0; k < 4; k++) acc[i][k] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int k = 0; k < 4; k++) acc[i][k] = float4_t{0.f, 0.f, 0.f, 0.f};
+  {
     if (have > 0) {
       unsigned entries = list[min(lane, have - 1)];   // 64 at a time, one per lane
       auto entry = [&](const int i) {
@@ -481,7 +483,7 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
         fetch(n2, w2);
         if (more) next_place = bring(run2, first2, 0, early);
         const float ws[4] = {own_block ? w.z.x : 0.f, own_block ? w.z.y : 0.f, own_block ? w.z.z : 0.f, own_block ? w.z.w : 0.f};
-        const BrickLeft left = brick_left(ws);
+        const u32x4 left = brick_left(ws);
         const float xs[8] = {w.x0.x, w.x0.y, w.x0.z, w.x0.w, w.x1.x, w.x1.y, w.x1.z, w.x1.w};
         const bool half[2] = {(e & kBrickUpper) != 0, (e & kBrickLower) != 0};
         // (from the 4-byte boundary, and shifted after: 16 bytes at a 2-byte boundary take LDS 60 clocks, 660 instead of 380 us of all)
@@ -496,7 +498,7 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
           for (int k = 0; k < 2; k++)
 #pragma unroll
             for (int ks = 0; ks < 2; ks++) {
-              const float y = (ks == 0 ? w.y[2 * h + k].x : w.y[2 * h + k].y) * scale;
+              const float y = (ks == 0 ? w.y[2 * h + k].x : w.y[2 * h + k].y) * kBrickWeight;
               float f[8];
 #pragma unroll
               for (int j = 0; j < 8; j++) f[j] = y * xs[j];
@@ -530,19 +532,12 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
               if (more) next_place = bring(run2, next_place, early, pieces);
             }
 #pragma unroll
-            for (int k = 0; k < 2; k++) acc[i][2 * h + k] = brick_add(left, part[k], acc[i][2 * h + k]);
+            for (int k = 0; k < 2; k++) acc[i][2 * h + k] = M::run16(left, brick_right(part[k]), acc[i][2 * h + k]);
           }
         }
         e = e2; w = w2; here = run2; first = first2;
       }
     }
-    if (scale == 1.f) break;
-    if (!brick_finite(acc)) continue;
-#pragma unroll
-    for (int i = 0; i < kBrickChannels / 2; i++)
-#pragma unroll
-      for (int k = 0; k < 4; k++) acc[i][k] *= 1.f / kBrickScale;
-    break;
   }
   if constexpr (SHARED) {
     if (have == 0) return;

@@ -144,3 +144,24 @@ def test_gradients_beyond_their_scale(oracle):
     ordinary = torch.ones(128, dtype=torch.bool)
     ordinary[::5] = False
     assert_close(got[:, ordinary], want[:, ordinary], TOL, "channels of ordinary gradients")
+
+
+@pytest.mark.parametrize("cells", [(4, 4, 4), (7, 7, 7), (8, 8, 8)])
+def test_small_gradients_beside_large_ones(oracle, cells):
+    """Channels of gradients near the type's largest beside channels in the subnormal range, in the same bricks: what may be left of the
+    small ones is the result's own rounding, with weights of 11 bits, twice (below 1e-3 of the result)."""
+    from medvision_amd.ops.roi_align_nd import roi_align_3d
+    g = wl.gen(11)
+    boxes = boxes_of(g, 1, (24, 40, 40), 300, 12)
+    x = torch.zeros(1, 128, 24, 40, 40, dtype=torch.float16, device=DEV, requires_grad=True)
+    out = roi_align_3d(x, boxes.to(DEV), cells, 1.0, 2, 1)
+    gy = torch.randn(out.shape, generator=g) * 1e-5
+    gy[:, ::5] *= 1e9
+    gy = gy.half()
+    assert bool(torch.isfinite(gy).all()) and float(gy.abs().max()) > 3e4
+    want = torch.as_tensor(oracle.roi_align_backward(gy, boxes, x.shape, 1.0, 2, True, 1, False)).double().reshape(x.shape)
+    got = torch.autograd.grad(out, x, gy.to(DEV))[0].cpu().double()
+    small = torch.ones(128, dtype=torch.bool)
+    small[::5] = False
+    own = (want[:, small].half().double() - want[:, small]).norm()
+    assert (got[:, small] - want[:, small]).norm() <= 1.1 * own + 1e-3 * want[:, small].norm()
