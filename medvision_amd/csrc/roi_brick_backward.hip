@@ -205,62 +205,23 @@ __device__ __forceinline__ u32x4 brick_right(const float4_t &part) {
   return brick_pair(high, rest);
 }
 
-// A region whose sums come out not finite, done again term by term and without the terms of weight 0.  Thread: one (y, x) of the
-// region, its sums of eight channels and all slices in LDS.
-template <int LOG_WX>
-__device__ inline void brick_careful(const __half *__restrict__ gout, const BrickRoi *__restrict__ recs, const float *__restrict__ tables,
-                                     __half *__restrict__ grad, const RoiProblem &p, float *const sums, const int X0,
-                                     const int Y0, const int Z0, const int c_base, const int image) {
-  constexpr int TZ = kBrickEdge;
-  using M = Mfma<__half>;
-  constexpr int threads = kWave << LOG_WX;
-  const int lane = threadIdx.x % kWave, x = X0 + (threadIdx.x & ((8 << LOG_WX) - 1)), y = Y0 + (threadIdx.x >> (3 + LOG_WX));
-  const int cells = p.od * p.oh * p.ow, ohw = p.oh * p.ow;
-  float *const mine = sums + threadIdx.x;
-  for (int c0 = c_base; c0 < min(c_base + kBrickChannels, p.C); c0 += 8) {
-    const int cn = min(8, p.C - c0);
-    for (int i = 0; i < 8 * TZ; i++) mine[i * threads] = 0.f;
-    for (int base = 0; base < p.R; base += kWave) {
-      const BrickRoi rec = recs[min(base + lane, p.R - 1)];
-      const int first[3] = {X0, Y0, Z0}, extent[3] = {8 << LOG_WX, 8, TZ};
-      bool hit = base + lane < p.R && rec.image == image;
-#pragma unroll
-      for (int a = 0; a < 3; a++) {
-        const int lo = rec.span[a] & 0xffffu, hi = rec.span[a] >> 16;
-        hit = hit && lo <= hi && lo < first[a] + extent[a] && hi >= first[a];
-      }
-      for (unsigned long mask = __ballot(hit); mask != 0; mask &= mask - 1) {
-        const int i = __builtin_ctzl(mask), n = base + i;
-        unsigned span[3];
-#pragma unroll
-        for (int a = 0; a < 3; a++) span[a] = __builtin_amdgcn_readlane(rec.span[a], i);
-        if (x < static_cast<int>(span[0] & 0xffffu) || x > static_cast<int>(span[0] >> 16) ||
-            y < static_cast<int>(span[1] & 0xffffu) || y > static_cast<int>(span[1] >> 16))
-          continue;
-        const int z0 = max(static_cast<int>(span[2] & 0xffffu) - Z0, 0), z1 = min(static_cast<int>(span[2] >> 16) - Z0, TZ - 1);
-        const float *tab = tables + static_cast<long>(n) * brick_rows(p) * kBrickCells;
-        for (int c = 0; c < cn; c++)
-          for (int pd = 0; pd < p.od; pd++) {
-            const __half *g = gout + (static_cast<long>(n) * p.C + c0 + c) * cells + pd * ohw;
-            float part = 0.f;
-            for (int k = 0; k < ohw; k++) {
-              const int ph = k / p.ow, pw = k - ph * p.ow;
-              float w = tab[(brick_row_y(p) + y) * kBrickCells + ph % 4 * 2 + ph / 4] * tab[x * kBrickCells + pw];
-              w = M::lo(M::pack2(w, w));   // (as the products have it)
-              if (w != 0.f) part += w * load(g + k);
-            }
-            for (int z = z0; z <= z1; z++) {
-              const float w = tab[(brick_row_z(p) + Z0 + z) * kBrickCells + pd];
-              if (w != 0.f && part != 0.f) mine[(c * TZ + z) * threads] += w * part;
-            }
-          }
-      }
-    }
-    if (x < p.W && y < p.H)
-      for (int i = 0; i < cn * TZ; i++)
-        if (Z0 + i % TZ < p.D)
-          grad[(((static_cast<long>(image) * p.C + c0 + i / TZ) * p.D + Z0 + i % TZ) * p.H + y) * p.W + x] = store_cast<__half>(mine[i * threads]);
-  }
+// A weight of zero times a gradient that is not finite is not a number, and it would reach every voxel of the brick.  Sums that do not come out finite
+// are formed again, in turns: what the positive infinities reach (1 stands for them), what the negative ones do, and the sums without any of
+// them; a gradient that is not a number counts as both.  The turns' results add up, inf - inf = NaN.  Turns that nothing is there for are left
+// out: gradients that are all NaN, or all the same infinity, take one.  (4000 rois x 256 channels x 7^3, forward and backward pass 550 us: with one
+// infinity 530 us, all NaN 1.3 ms, infinities of both signs alone 2.4; term by term in fp32, without a product, one infinity took 17.7 ms.)
+enum BrickTurn { kBrickAll, kBrickPlus, kBrickMinus, kBrickFinite };
+constexpr unsigned kBrickHasPlus = 2, kBrickHasMinus = 4, kBrickHasNan = 8, kBrickHasFinite = 16;   // what a brick's gradients have
+struct BrickKinds { unsigned plus = 0, minus = 0, nan = 0, finite = 0; };   // not 0: there are some
+// A word of two gradients in a turn
+__device__ __forceinline__ unsigned brick_screen(const unsigned v, const int turn, BrickKinds &has) {
+  const unsigned special = ((v & 0x7c007c00u) + 0x04000400u) & 0x80008000u;   // (a sign bit each, as all of these)
+  const unsigned nan = special & ((v & 0x03ff03ffu) + 0x7fff7fffu), inf = special ^ nan;
+  const unsigned finite = v & ~(special | (special - (special >> 15)));
+  has.plus |= inf & ~v; has.minus |= inf & v; has.nan |= nan; has.finite |= finite & 0x7fff7fffu;
+  if (turn == kBrickFinite) return finite;
+  const unsigned on = nan | (inf & (turn == kBrickPlus ? ~v : v));
+  return (on >> 1) - (on >> 5);   // (0x4000 - 0x0400: 1)
 }
 
 // What a workgroup works on: 1 << LOG_WX bricks side by side, 16 channels of an image; `part` of `parts` workgroups that share them.
@@ -302,21 +263,14 @@ __device__ __forceinline__ bool brick_finite(const float4_t (&acc)[kBrickChannel
 }
 
 // The wavefronts' sums to the gradient.  acc[i][k], register r: channel 2 i + quad / 2, voxel z = quad % 2 * 4 + r, y = 2 k + col / 8,
-// x = col % 8 of the brick.
+// x = col % 8 of the brick.  Not `sums`: `mark` where a sum is positive, 0 elsewhere.  Not `first`: added to what is there.
 template <int LOG_WX>
-__device__ __forceinline__ void brick_finish(const float4_t (&acc)[kBrickChannels / 2][4], const BrickPlace<LOG_WX> &at,
-                                             const __half *__restrict__ gout, const BrickRoi *__restrict__ recs,
-                                             const float *__restrict__ tables, __half *__restrict__ grad, const RoiProblem &p,
-                                             unsigned char *const lds, unsigned &special) {
+__device__ __forceinline__ void brick_finish(const float4_t (&acc)[kBrickChannels / 2][4], const BrickPlace<LOG_WX> &at, __half *__restrict__ grad,
+                                             const RoiProblem &p, unsigned char *const lds, const bool sums, const float mark, const bool first) {
   constexpr int wxn = 1 << LOG_WX, RX = kBrickEdge << LOG_WX, TZ = kBrickEdge;
-  const int lane = threadIdx.x % kWave, bx = threadIdx.x / kWave * kBrickEdge, col = lane % 16, quad = lane / 16;
-  // (a weight of zero times a gradient that is not finite is not a number)
-  if (!brick_finite(acc) && lane == 0) special = 1;
-  __syncthreads();
-  if (special != 0) {
-    brick_careful<LOG_WX>(gout, recs, tables, grad, p, reinterpret_cast<float *>(lds), at.X0, at.Y0, at.Z0, at.c_base, at.image);
-    return;
-  }
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));   // (nothing of this is formed before a brick's turns and kept)
+  const int lane = tid % kWave, bx = tid / kWave * kBrickEdge, col = lane % 16, quad = lane / 16;
   // through LDS, so that rows of the region go out whole: [channel][z][y][x], a little room between channels against bank conflicts
   __half *const stage = reinterpret_cast<__half *>(lds);
   constexpr int channel = (TZ * 64 << LOG_WX) + 8;
@@ -327,17 +281,17 @@ __device__ __forceinline__ void brick_finish(const float4_t (&acc)[kBrickChannel
 #pragma unroll
       for (int r = 0; r < 4; r++)
         stage[(2 * i + quad / 2) * channel + ((quad % 2 * 4 + r) * 8 + 2 * k + col / 8) * RX + bx + col % 8] =
-            store_cast<__half>(acc[i][k][r]);
+            store_cast<__half>(sums ? acc[i][k][r] : acc[i][k][r] > 0.f ? mark : 0.f);
   __syncthreads();
   constexpr int kPieces = kBrickChannels * wxn * TZ * 8;
 #pragma unroll 4
-  for (int i = threadIdx.x; i < kPieces; i += kWave * wxn) {
+  for (int i = tid; i < kPieces; i += kWave * wxn) {
     const int px = i & (wxn - 1), row = (i >> LOG_WX) & (TZ * 8 - 1), cl = (i >> LOG_WX) / (TZ * 8);
     const int y = at.Y0 + row % 8, z = at.Z0 + row / 8, x = at.X0 + px * 8;
     if (at.c_base + cl >= p.C || y >= p.H || z >= p.D || x >= p.W) continue;
     const u32x4 v = *reinterpret_cast<const u32x4 *>(stage + cl * channel + row * RX + px * 8);
     __half *dst = grad + (((static_cast<long>(at.image) * p.C + at.c_base + cl) * p.D + z) * p.H + y) * p.W + x;
-    if (x + 8 <= p.W) {   // one store: global memory takes any alignment
+    if (first && x + 8 <= p.W) {   // one store: global memory takes any alignment
       typedef unsigned int V __attribute__((ext_vector_type(4), aligned(2)));
       *reinterpret_cast<V *>(dst) = v;
     } else {
@@ -345,7 +299,7 @@ __device__ __forceinline__ void brick_finish(const float4_t (&acc)[kBrickChannel
       __builtin_memcpy(e, &v, sizeof(v));
 #pragma unroll
       for (int k = 0; k < 8; k++)
-        if (x + k < p.W) dst[k] = e[k];
+        if (x + k < p.W) dst[k] = first ? e[k] : store_cast<__half>(load(dst + k) + load(&e[k]));
     }
   }
 }
@@ -357,10 +311,9 @@ __device__ __forceinline__ int brick_share(const int length, const int k, const 
 
 template <int LOG_WX, bool SHARED>
 __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
-    const __half *__restrict__ gout, const __half *__restrict__ last, const BrickRoi *__restrict__ recs, const float *__restrict__ tables,
-    const unsigned *__restrict__ lists, const unsigned *__restrict__ lengths, __half *__restrict__ grad, const RoiProblem p, const int nx,
-    const int ny, const int nz, const int cblocks, const unsigned total, const int pieces, const int ring, const int parts,
-    float4_t *__restrict__ partial) {
+    const __half *__restrict__ gout, const __half *__restrict__ last, const float *__restrict__ tables, const unsigned *__restrict__ lists,
+    const unsigned *__restrict__ lengths, __half *__restrict__ grad, const RoiProblem p, const int nx, const int ny, const int nz,
+    const int cblocks, const unsigned total, const int pieces, const int ring, const int parts, float4_t *__restrict__ partial) {
   using M = Mfma<__half>;
   // A ring of `ring` kilobytes and one more for each wavefront, for the rois' gradients, `pieces` of them each; at the end the sums.
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -399,11 +352,13 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
   const unsigned *const list = lists + brick * p.R + begin;
   // [two channels][two rows of voxels]: z = quad % 2 * 4 + r of channel quad / 2 at voxel (y = col / 8, x = col % 8)
   float4_t acc[kBrickChannels / 2][4];
+  unsigned bits = 0;   // 1: the sums are not all finite; then what the gradients have
+#pragma unroll 1
+  for (int turn = kBrickAll;;) {
 #pragma unroll
-  for (int i = 0; i < kBrickChannels / 2; i++)
+    for (int i = 0; i < kBrickChannels / 2; i++)
 #pragma unroll
-    for (int k = 0; k < 4; k++) acc[i][k] = float4_t{0.f, 0.f, 0.f, 0.f};
-  {
+      for (int k = 0; k < 4; k++) acc[i][k] = float4_t{0.f, 0.f, 0.f, 0.f};
     if (have > 0) {
       unsigned entries = list[min(lane, have - 1)];   // 64 at a time, one per lane
       auto entry = [&](const int i) {
@@ -465,6 +420,22 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
         s[0] = *reinterpret_cast<const V *>(from);
         s[1] = *reinterpret_cast<const V *>(from + to_second);
       };
+      // the present roi's gradient as a turn has it, in LDS
+      auto screen = [&](int place, const int turn) {
+        BrickKinds has;
+#pragma unroll 2
+        for (int i = 0; i < pieces; i++) {
+          u32x4 *const at = reinterpret_cast<u32x4 *>(ring_lds + place * 1024) + lane;
+          u32x4 v = *at;
+#pragma unroll
+          for (int j = 0; j < 4; j++) v[j] = brick_screen(v[j], turn, has);
+          *at = v;
+          if (place == 0 && i > 0) at[ring * 64] = v;
+          place = place + 1 == ring ? 0 : place + 1;
+        }
+        const auto any = [](const unsigned word, const unsigned bit) { return __ballot(word != 0) != 0 ? bit : 0u; };
+        bits |= any(has.plus, kBrickHasPlus) | any(has.minus, kBrickHasMinus) | any(has.nan, kBrickHasNan) | any(has.finite, kBrickHasFinite);
+      };
       Weights w;
       unsigned e = entry(0);
       fetch(e & ~(kBrickUpper | kBrickLower), w);
@@ -475,6 +446,7 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
         asm volatile("" : "+v"(w.x0.x), "+v"(w.x0.y), "+v"(w.x0.z), "+v"(w.x0.w), "+v"(w.x1.x), "+v"(w.x1.y), "+v"(w.x1.z), "+v"(w.x1.w));
         asm volatile("" : "+v"(w.y[0].x), "+v"(w.y[0].y), "+v"(w.y[1].x), "+v"(w.y[1].y), "+v"(w.y[2].x), "+v"(w.y[2].y), "+v"(w.y[3].x),
                           "+v"(w.y[3].y), "+v"(w.z.x), "+v"(w.z.y), "+v"(w.z.z), "+v"(w.z.w));
+        if (turn != kBrickAll) screen(first, turn);
         const bool more = done + 1 < have;
         const unsigned e2 = more ? entry(done + 1) : e, n2 = e2 & ~(kBrickUpper | kBrickLower);
         const Run run2 = run_of(n2);
@@ -538,31 +510,62 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
         e = e2; w = w2; here = run2; first = first2;
       }
     }
-  }
-  if constexpr (SHARED) {
-    if (have == 0) return;
-    float4_t *const to = partial + ((brick * cblocks + c_base / kBrickChannels) * parts + place.part) * (kBrickChannels / 2 * 4 * kWave) + lane;
+    if (turn == kBrickAll && !brick_finite(acc)) bits = 1;
+    if constexpr (SHARED) {
+      if (have == 0) return;
+    } else {   // (both wavefronts take the same turns: they leave their sums together)
+      if (bits != 0 && lane == 0) atomicOr(&special, bits);
+      __syncthreads();
+      bits = __builtin_amdgcn_readfirstlane(special);
+    }
+    if (turn == kBrickAll && bits != 0) {
+      turn = kBrickPlus;
+      continue;
+    }
+    const bool infinite = (bits & (kBrickHasPlus | kBrickHasMinus)) != 0;
+    const bool sums = turn == kBrickAll || turn == kBrickFinite, first = turn == kBrickAll || turn == kBrickPlus;
+    const float mark = turn == kBrickMinus ? -INFINITY : infinite ? INFINITY : NAN;   // for what the turn's gradients reach
+    if constexpr (SHARED) {
+      float4_t *to =
+          partial + ((brick * cblocks + c_base / kBrickChannels) * parts + place.part) * (kBrickChannels / 2 * 4 * kWave) + lane;
+      asm volatile("" : "+v"(to));   // (the addresses are not formed before the turns and kept)
+      if (turn == kBrickAll) {
 #pragma unroll
-    for (int i = 0; i < kBrickChannels / 2; i++)
+        for (int i = 0; i < kBrickChannels / 2; i++)
 #pragma unroll
-      for (int k = 0; k < 4; k++) to[(i * 4 + k) * kWave] = acc[i][k];
-  } else {
-    brick_finish<LOG_WX>(acc, place, gout, recs, tables, grad, p, lds, special);
+          for (int k = 0; k < 4; k++) to[(i * 4 + k) * kWave] = acc[i][k];
+      } else {
+#pragma unroll
+        for (int i = 0; i < kBrickChannels / 2; i++)
+#pragma unroll
+          for (int k = 0; k < 4; k++) {
+            float4_t sum = acc[i][k];
+#pragma unroll
+            for (int r = 0; r < 4; r++) sum[r] = sums ? sum[r] : sum[r] > 0.f ? mark : 0.f;
+            if (!first) sum += to[0];
+            to[0] = sum;
+            to += kWave;
+            asm volatile("" : "+v"(to) : : "memory");   // (one after the other: together they take more registers than there are)
+          }
+      }
+    } else {
+      brick_finish<LOG_WX>(acc, place, grad, p, lds, sums, mark, first);
+    }
+    if (turn == kBrickPlus && infinite && (bits & (kBrickHasMinus | kBrickHasNan))) turn = kBrickMinus;
+    else if (turn != kBrickAll && turn != kBrickFinite && (bits & kBrickHasFinite)) turn = kBrickFinite;
+    else return;
+    if constexpr (!SHARED) __syncthreads();   // the sums have been read and are in memory
   }
 }
 
 // The sums of the parts.
 template <int LOG_WX>
 __global__ __launch_bounds__(kWave << LOG_WX) void roi_brick_fold_kernel(
-    const __half *__restrict__ gout, const BrickRoi *__restrict__ recs, const float *__restrict__ tables,
     const unsigned *__restrict__ lengths, __half *__restrict__ grad, const RoiProblem p, const int nx, const int ny, const int nz,
     const int cblocks, const unsigned total, const int parts, const float4_t *__restrict__ partial) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  __shared__ unsigned special;
   const BrickPlace<LOG_WX> place(p, nx, ny, nz, cblocks, 1, total);
   if (place.none) return;
-  if (threadIdx.x == 0) special = 0;
-  __syncthreads();
   const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int have = wave < place.bricks ? static_cast<int>(lengths[place.brick + wave]) : 0;
   float4_t acc[kBrickChannels / 2][4];
@@ -578,7 +581,7 @@ __global__ __launch_bounds__(kWave << LOG_WX) void roi_brick_fold_kernel(
 #pragma unroll
       for (int k = 0; k < 4; k++) acc[i][k] += from[(i * 4 + k) * kWave];
   }
-  brick_finish<LOG_WX>(acc, place, gout, recs, tables, grad, p, lds, special);
+  brick_finish<LOG_WX>(acc, place, grad, p, lds, true, 0.f, true);
 }
 
 static size_t brick_tables_bytes(const RoiProblem &p) {
@@ -668,11 +671,11 @@ int roi_brick_backward(const void *grad_output, const void *rois, void *grad_inp
                      reinterpret_cast<const uint4 *>(recs), lists, lengths, p.R, brick_up(p.W) / kBrickEdge, ny, nz);
   auto grid = [](long n) { return dim3(static_cast<unsigned>((n + 7) / 8 * 8)); };
 #define MV_BRICK(LOG_WX, SHARED)                                                                                               \
-  hipLaunchKernelGGL((roi_brick_backward_kernel<LOG_WX, SHARED>), grid(total), dim3(kWave << LOG_WX), std::max(sums, rings), s, g, copy, recs, \
-                     tables, lists, lengths, grad, p, nx, ny, nz, cblocks, static_cast<unsigned>(total), pieces, ring, parts, partial)
+  hipLaunchKernelGGL((roi_brick_backward_kernel<LOG_WX, SHARED>), grid(total), dim3(kWave << LOG_WX), std::max(sums, rings), s, g, copy, tables, \
+                     lists, lengths, grad, p, nx, ny, nz, cblocks, static_cast<unsigned>(total), pieces, ring, parts, partial)
 #define MV_BRICK_FOLD(LOG_WX)                                                                                                  \
-  hipLaunchKernelGGL((roi_brick_fold_kernel<LOG_WX>), grid(regions), dim3(kWave << LOG_WX), sums, s, g, recs, tables, lengths, grad, p, nx, ny, \
-                     nz, cblocks, static_cast<unsigned>(regions), parts, partial)
+  hipLaunchKernelGGL((roi_brick_fold_kernel<LOG_WX>), grid(regions), dim3(kWave << LOG_WX), sums, s, lengths, grad, p, nx, ny, nz, \
+                     cblocks, static_cast<unsigned>(regions), parts, partial)
   if (parts == 1) {
     if (log_wx) MV_BRICK(1, false); else MV_BRICK(0, false);
   } else if (log_wx) {

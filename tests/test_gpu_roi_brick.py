@@ -1,5 +1,7 @@
 """Gradients of fp16 heads of plain boxes on volumes by the voxels' owners (roi_brick_backward.hip): remainders of bricks and
 channels, rows of cells at any alignment, shared bricks, gradients that are not finite, against the fp64 oracle."""
+import ctypes
+
 import pytest
 import torch
 
@@ -165,3 +167,51 @@ def test_small_gradients_beside_large_ones(oracle, cells):
     small[::5] = False
     own = (want[:, small].half().double() - want[:, small]).norm()
     assert (got[:, small] - want[:, small]).norm() <= 1.1 * own + 1e-3 * want[:, small].norm()
+
+
+class _Problem(ctypes.Structure):   # RoiProblem (csrc/roi_geometry.hpp)
+    _fields_ = ([(n, ctypes.c_int) for n in ("ndim", "rotated", "N", "C", "D", "H", "W", "R", "od", "oh", "ow")] + [("scale", ctypes.c_double)] +
+                [(n, ctypes.c_int) for n in ("sampling_ratio", "aligned", "order")] + [(n, ctypes.c_uint) for n in ("per_roi", "chunks")])
+
+
+def bricks_apply(dims, rois, cells, ratio=2):
+    """Whether the bricks' kernels serve a head."""
+    from medvision_amd import _lib
+    fn = _lib.load()._ZN2mv19roi_brick_workspaceEiRKNS_10RoiProblemE
+    fn.restype, fn.argtypes = ctypes.c_size_t, [ctypes.c_int, ctypes.POINTER(_Problem)]
+    problem = _Problem(3, 0, *dims, rois, *cells, 1.0, ratio, 1, 1, dims[1] * cells[0] * cells[1] * cells[2], 1)
+    return fn(_lib.MV_F16, ctypes.byref(problem)) > 0
+
+
+@pytest.mark.parametrize("size,rois", [((9, 17, 33), 60), ((9, 17, 33), 480), ((40, 33, 8), 60), ((40, 33, 8), 480)])
+@pytest.mark.parametrize("kind", ["plus", "minus", "both", "nan", "all inf", "all nan"])
+def test_gradients_that_are_not_finite(oracle, size, rois, kind):
+    """One workgroup per brick and several, one brick along x and several: infinities reach their voxels with their sign, both signs and NaN as
+    NaN, every other voxel keeps its sum."""
+    from medvision_amd.ops.roi_align_nd import roi_align_3d
+    g = wl.gen(rois + size[2])
+    channels = 160
+    assert bricks_apply((2, channels, *size), rois, (4, 5, 4))
+    boxes = boxes_of(g, 2, size, rois, 9)
+    x = torch.zeros(2, channels, *size, dtype=torch.float16, device=DEV, requires_grad=True)
+    out = roi_align_3d(x, boxes.to(DEV), (4, 5, 4), 1.0, 2, 1)
+    gy = torch.randn(out.shape, generator=g).half()
+    draw = torch.rand(gy.shape, generator=g)
+    if kind.startswith("all"):
+        gy = torch.full_like(gy, float("inf")) * torch.sign(gy) if kind == "all inf" else torch.full_like(gy, float("nan"))
+    else:
+        few = draw < 2e-4
+        value = {"plus": torch.full_like(draw, float("inf")), "minus": torch.full_like(draw, -float("inf")), "nan": torch.full_like(draw, float("nan")),
+                 "both": torch.where(draw < 1e-4, float("inf"), -float("inf"))}[kind]
+        gy = torch.where(few, value.half(), gy)
+    reach = lambda of: torch.as_tensor(oracle.roi_align_backward(of.half(), boxes, x.shape, 1.0, 2, True, 1, False)).reshape(x.shape)
+    plus, minus = reach((gy == float("inf")) | gy.isnan()), reach((gy == -float("inf")) | gy.isnan())
+    finite = reach(torch.where(gy.isfinite(), gy, 0))
+    got = torch.autograd.grad(out, x, gy.to(DEV))[0].cpu().double()
+    sure, none = 1e-6, 0.0   # (weights between: too small for 16 bits)
+    assert bool(got[(plus > sure) & (minus > sure)].isnan().all())
+    assert bool((got[(plus > sure) & (minus == none)] == float("inf")).all())
+    assert bool((got[(plus == none) & (minus > sure)] == -float("inf")).all())
+    apart = (plus == none) & (minus == none)
+    assert_close(torch.where(apart, got, finite.double()), finite, TOL, "finite part")
+    assert kind.startswith("all") or float(apart.float().mean()) > 0.2
