@@ -399,8 +399,9 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
       const unsigned ring_at = __builtin_amdgcn_readfirstlane(
           static_cast<unsigned>(reinterpret_cast<unsigned long long>((__attribute__((address_space(3))) unsigned char *)ring_lds)));
       auto to_lds = [&](const Run &run, const int piece_at, const int place) {
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                     : : "s"(__builtin_amdgcn_readfirstlane(ring_at + place * 1024)), "v"(lane * 16 + piece_at * 1024), "s"(run.src) : "memory");
+        unsigned kept;   // (m0 is the compiler's own: it cannot be named as changed, so it gets back what it had)
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
+                     : "=&s"(kept) : "s"(__builtin_amdgcn_readfirstlane(ring_at + place * 1024)), "v"(lane * 16 + piece_at * 1024), "s"(run.src) : "memory");
       };
       auto bring = [&](const Run &run, int place, const int from, const int to) {
 #pragma unroll 1
