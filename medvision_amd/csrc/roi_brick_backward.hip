@@ -37,10 +37,11 @@ constexpr int kBrickEdge = 8;                  // voxels of a brick along each a
 constexpr int kBrickPad = 128;                 // bytes behind the copy of the last roi's gradient
 
 // What the tables kernel leaves about a roi: first and last voxel of its box per axis (low and high half; first > last: the roi
-// touches nothing) and the image.  Its tables are rows of eight fp32 weights, one per voxel along x, then y, then z, the axes
+// touches nothing; bit 15: more samples than a wavefront has lanes) and the image.  Its tables are rows of eight fp32 weights, one per voxel along x, then y, then z, the axes
 // padded to whole bricks; only the rows of the bricks that the box touches are written.  A row of y holds cell c at
 // c % 4 * 2 + c / 4, the two cells of a lane side by side; where there is no cell c + 4, cell c stands there too.
 struct BrickRoi { unsigned span[3]; int image; };
+constexpr unsigned kBrickMany = 0x8000u;
 
 __host__ __device__ inline int brick_up(int n) { return (n + kBrickEdge - 1) / kBrickEdge * kBrickEdge; }
 __host__ __device__ inline int brick_rows(const RoiProblem &p) { return brick_up(p.W) + brick_up(p.H) + brick_up(p.D); }
@@ -100,7 +101,8 @@ __global__ __launch_bounds__(3 * kWave) void roi_brick_tables_kernel(const float
     last_voxel = max(last_voxel, __shfl_xor(last_voxel, m));
   }
   if (lane == 0) {
-    recs[n].span[a] = static_cast<unsigned>(first) | static_cast<unsigned>(max(last_voxel, 0)) << 16;
+    const bool many = static_cast<long>(nc) * grid > kWave;
+    recs[n].span[a] = static_cast<unsigned>(first) | (many ? kBrickMany : 0u) | static_cast<unsigned>(max(last_voxel, 0)) << 16;
     if (a == 0) recs[n].image = image;
   }
   const int cell = a == 1 && lane % kBrickCells >= max(nc, 4) ? lane % kBrickCells - 4 : lane % kBrickCells;
@@ -127,8 +129,22 @@ __global__ __launch_bounds__(3 * kWave) void roi_brick_tables_kernel(const float
 }
 
 // The rois that touch a brick, in their order: a workgroup per brick.  An entry is the roi's number, with a bit for the upper
-// four rows of the brick and one for the lower four.
-constexpr unsigned kBrickUpper = 1u << 30, kBrickLower = 1u << 31;
+// four rows of the brick, one for the lower four, and one for the form with all bits (see brick_exact).
+constexpr unsigned kBrickUpper = 1u << 30, kBrickLower = 1u << 31, kBrickExact = 1u << 29, kBrickNumber = kBrickExact - 1;
+
+// Whether a roi's gradient has all bits of its weights: those that the kernel which adds box by box works out in fp32, not as products of 16-bit
+// numbers (a slice that does not fit its operand, boxes or samples beyond its tables, and what its loads would reach past the tensor's end).
+__device__ __forceinline__ bool brick_exact(const unsigned (&span)[3]) {
+  int extent[3];
+  bool many = false;
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+    extent[a] = static_cast<int>(span[a] >> 16) - static_cast<int>(span[a] & 0x7fffu) + 1;
+    many = many || (span[a] & kBrickMany) || extent[a] > 32;
+  }
+  return many || extent[1] * ((extent[0] + 3) & ~3) > 224;
+}
+
 __global__ __launch_bounds__(kBrickThreads) void roi_brick_lists_kernel(const uint4 *__restrict__ recs, unsigned *__restrict__ lists,
                                                                         unsigned *__restrict__ lengths, const int R, const int nx,
                                                                         const int ny, const int nz) {
@@ -153,10 +169,11 @@ __global__ __launch_bounds__(kBrickThreads) void roi_brick_lists_kernel(const ui
       bool hit = k < R && static_cast<int>(rec[i].w) == image;
 #pragma unroll
       for (int a = 0; a < 3; a++) {
-        const int lo = static_cast<int>(span[a] & 0xffffu) - first[a], hi = static_cast<int>(span[a] >> 16) - first[a];
+        const int lo = static_cast<int>(span[a] & 0x7fffu) - first[a], hi = static_cast<int>(span[a] >> 16) - first[a];
         hit = hit && lo <= hi && lo < kBrickEdge && hi >= 0;
         if (a == 1) rec[i].x = static_cast<unsigned>(k) | (lo < kBrickEdge / 2 ? kBrickUpper : 0) | (hi >= kBrickEdge / 2 ? kBrickLower : 0);
       }
+      if (brick_exact(span)) rec[i].x |= kBrickExact;
       hits[i] = __ballot(hit);
       if (lane == 0) counts[turn][i * kBrickWaves + wave] = __popcll(hits[i]);
     }
@@ -172,16 +189,20 @@ __global__ __launch_bounds__(kBrickThreads) void roi_brick_lists_kernel(const ui
   if (threadIdx.x == 0) lengths[id] = have;
 }
 
-// The operands of the products are fp16 numbers.  The weights Wy Wx and Wz are rounded to them (11 bits); where the first product's K has room,
-// below eight rows of cells, rows stand in it twice, the second time with what the rounding left of their weights.  The sums P stand in the
-// second product's K as two numbers, the second one what the first has left: they keep 22 bits.
-// Everything is scaled so that neither the largest nor the smallest gradients need a second look: Wy Wx by kBrickWeight, the first number of P by
-// 1 / 128 (64 cells of the type's largest still fit), its rest by kBrickWeight, and Wz by what makes the products' sum the result.
-// Error against 64 bits of heads with boxes up to 12 voxels (2.07e-4 of it the result's own rounding): four rows 2.86e-4, seven 3.45e-4,
-// eight 3.53e-4; box-by-box sums 3.61e-4.  Gradients of 1e-5: 2.17e-3 (own 2.15e-3), box by box 3.02e-3.  4000 rois x 256 channels x 7^3, forward and
-// backward pass, 494 us with P as one number, 544 with two; but with one number small gradients are lost unless it is scaled up, and where that
-// overflows the brick had to be done again (30 ms for gradients of 4000, 558 us now).
-constexpr float kBrickWeight = 16.f;
+// The operands of the products are fp16 numbers.  In the ordinary form the weights Wy Wx and the sums P are rounded to them once (11 bits) and Wz is
+// two numbers side by side in K.  Where the first product's K has room, below eight rows of cells, rows stand in it twice, the second time with
+// what the rounding left of their weights.  Wy Wx is scaled by kBrickWeight, so that P of small gradients is not a subnormal number of a few bits.
+// In the form with all bits (22 of them) Wy Wx, P and Wz are all two numbers, what is left of a weight in products of its own; the first number of
+// P is scaled down to 1 / 128 (64 cells of the type's largest fit), its rest up again, and Wz by what makes the products' sum the result.  It is
+// for rois whose gradients the kernel that adds box by box works out in fp32 (brick_exact), and for bricks whose sums overflow in the ordinary form
+// (|P| > 16376).
+// Error against 64 bits (2.07e-4 of it the result's own rounding) here and box by box, 200 rois of up to 12 voxels: four rows 2.93e-4 and 3.61e-4,
+// seven 3.53e-4 and 3.62e-4, eight 3.59e-4 and 3.60e-4; 100 rois of 16 - 24 voxels: 2.07e-4 with all bits (3.5e-4 without) and 2.07e-4; gradients of
+// 1e-5 2.24e-3 (own 2.15e-3) and 3.02e-3.
+// Backward pass of 4000 rois x 256 channels x 7^3: 500 us (box by box 795); with P as two numbers for all rois, so that no values need a second time,
+// 555, and 1000 rois of 4^3 x 128 98 and 115 (box by box 151).  Gradients of 4000 throughout, where all bricks do: 1.6 ms.  100 rois of 16 - 24 voxels
+// x 128 x 7^3: 220 us with all bits, 135 without, 399 box by box.
+constexpr float kBrickWeight = 4.f, kBrickExactWeight = 16.f;
 typedef _Float16 brick_half4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ brick_half4 brick_pack(const float (&w)[4]) {
   return __builtin_bit_cast(brick_half4, uint2{Mfma<__half>::pack2(w[0], w[1]), Mfma<__half>::pack2(w[2], w[3])});
@@ -190,13 +211,24 @@ __device__ __forceinline__ u32x4 brick_pair(const brick_half4 a, const brick_hal
   const uint2 x = __builtin_bit_cast(uint2, a), y = __builtin_bit_cast(uint2, b);
   return u32x4{x.x, x.y, y.x, y.y};
 }
-__device__ __forceinline__ u32x4 brick_left(const float (&w)[4]) {
-  const float large[4] = {w[0] * 128.f, w[1] * 128.f, w[2] * 128.f, w[3] * 128.f};
-  const float small[4] = {w[0] / kBrickWeight, w[1] / kBrickWeight, w[2] / kBrickWeight, w[3] / kBrickWeight};
-  return brick_pair(brick_pack(large), brick_pack(small));
+struct BrickLeft { brick_half4 value, rest; };
+__device__ __forceinline__ BrickLeft brick_left(const float (&w)[4], const float scale) {
+  const float v[4] = {w[0] * scale, w[1] * scale, w[2] * scale, w[3] * scale};
+  BrickLeft l;
+  l.value = brick_pack(v);
+  float rest[4];
+#pragma unroll
+  for (int r = 0; r < 4; r++) rest[r] = v[r] - static_cast<float>(l.value[r]);
+  l.rest = brick_pack(rest);
+  return l;
 }
-__device__ __forceinline__ u32x4 brick_right(const float4_t &part) {
-  constexpr float kDown = 1.f / (128.f * kBrickWeight);
+__device__ __forceinline__ u32x4 brick_sums(const float4_t &part) {
+  const float v[4] = {part[0], part[1], part[2], part[3]};
+  const brick_half4 sums = brick_pack(v);
+  return brick_pair(sums, sums);
+}
+__device__ __forceinline__ u32x4 brick_sums_exact(const float4_t &part) {
+  constexpr float kDown = 1.f / (128.f * kBrickExactWeight);
   const float v[4] = {part[0] * kDown, part[1] * kDown, part[2] * kDown, part[3] * kDown};
   brick_half4 high = brick_pack(v), rest;
   asm("" : "+v"(high));   // (or the compiler forms it a second time, element by element, for the rest)
@@ -205,23 +237,23 @@ __device__ __forceinline__ u32x4 brick_right(const float4_t &part) {
   return brick_pair(high, rest);
 }
 
-// A weight of zero times a gradient that is not finite is not a number, and it would reach every voxel of the brick.  Sums that do not come out finite
-// are formed again, in turns: what the positive infinities reach (1 stands for them), what the negative ones do, and the sums without any of
-// them; a gradient that is not a number counts as both.  The turns' results add up, inf - inf = NaN.  Turns that nothing is there for are left
-// out: gradients that are all NaN, or all the same infinity, take one.  (4000 rois x 256 channels x 7^3, forward and backward pass 550 us: with one
-// infinity 530 us, all NaN 1.3 ms, infinities of both signs alone 2.4; term by term in fp32, without a product, one infinity took 17.7 ms.)
-enum BrickTurn { kBrickAll, kBrickPlus, kBrickMinus, kBrickFinite };
-constexpr unsigned kBrickHasPlus = 2, kBrickHasMinus = 4, kBrickHasNan = 8, kBrickHasFinite = 16;   // what a brick's gradients have
-struct BrickKinds { unsigned plus = 0, minus = 0, nan = 0, finite = 0; };   // not 0: there are some
+// Sums that do not come out finite are formed again, with all bits and in turns.  (A weight of zero times a gradient that is not finite is not a
+// number, and it would reach every voxel of the brick.)  First the sums without such gradients, then what the positive infinities reach (1 stands
+// for them), then what the negative ones do; a gradient that is not a number counts as both.  The turns' results add up, inf - inf = NaN.  (4000 rois
+// x 256 channels x 7^3 with one infinity 500 us, all NaN 2.2 ms, infinities of both signs alone 3.4; term by term in fp32, without a product, one
+// infinity took 17.7 ms.)
+enum BrickTurn { kBrickAll, kBrickFinite, kBrickPlus, kBrickMinus };
+constexpr unsigned kBrickHasPlus = 2, kBrickHasMinus = 4, kBrickHasNan = 8;   // what a brick's gradients have
+struct BrickKinds { unsigned plus = 0, minus = 0, nan = 0, now = 0; };        // not 0: there are some (`now`: for the present turn)
 // A word of two gradients in a turn
 __device__ __forceinline__ unsigned brick_screen(const unsigned v, const int turn, BrickKinds &has) {
   const unsigned special = ((v & 0x7c007c00u) + 0x04000400u) & 0x80008000u;   // (a sign bit each, as all of these)
   const unsigned nan = special & ((v & 0x03ff03ffu) + 0x7fff7fffu), inf = special ^ nan;
-  const unsigned finite = v & ~(special | (special - (special >> 15)));
-  has.plus |= inf & ~v; has.minus |= inf & v; has.nan |= nan; has.finite |= finite & 0x7fff7fffu;
-  if (turn == kBrickFinite) return finite;
+  has.plus |= inf & ~v; has.minus |= inf & v; has.nan |= nan;
   const unsigned on = nan | (inf & (turn == kBrickPlus ? ~v : v));
-  return (on >> 1) - (on >> 5);   // (0x4000 - 0x0400: 1)
+  const unsigned now = turn == kBrickFinite ? v & ~(special | (special - (special >> 15))) : (on >> 1) - (on >> 5);   // (0x4000 - 0x0400: 1)
+  has.now |= now & 0x7fff7fffu;
+  return now;
 }
 
 // What a workgroup works on: 1 << LOG_WX bricks side by side, 16 channels of an image; `part` of `parts` workgroups that share them.
@@ -263,10 +295,10 @@ __device__ __forceinline__ bool brick_finite(const float4_t (&acc)[kBrickChannel
 }
 
 // The wavefronts' sums to the gradient.  acc[i][k], register r: channel 2 i + quad / 2, voxel z = quad % 2 * 4 + r, y = 2 k + col / 8,
-// x = col % 8 of the brick.  Not `sums`: `mark` where a sum is positive, 0 elsewhere.  Not `first`: added to what is there.
+// x = col % 8 of the brick.  Not `first`: `mark` where a sum is positive is added to what is there.
 template <int LOG_WX>
 __device__ __forceinline__ void brick_finish(const float4_t (&acc)[kBrickChannels / 2][4], const BrickPlace<LOG_WX> &at, __half *__restrict__ grad,
-                                             const RoiProblem &p, unsigned char *const lds, const bool sums, const float mark, const bool first) {
+                                             const RoiProblem &p, unsigned char *const lds, const bool first, const float mark) {
   constexpr int wxn = 1 << LOG_WX, RX = kBrickEdge << LOG_WX, TZ = kBrickEdge;
   int tid = threadIdx.x;
   asm volatile("" : "+v"(tid));   // (nothing of this is formed before a brick's turns and kept)
@@ -281,7 +313,7 @@ __device__ __forceinline__ void brick_finish(const float4_t (&acc)[kBrickChannel
 #pragma unroll
       for (int r = 0; r < 4; r++)
         stage[(2 * i + quad / 2) * channel + ((quad % 2 * 4 + r) * 8 + 2 * k + col / 8) * RX + bx + col % 8] =
-            store_cast<__half>(sums ? acc[i][k][r] : acc[i][k][r] > 0.f ? mark : 0.f);
+            store_cast<__half>(first ? acc[i][k][r] : acc[i][k][r] > 0.f ? mark : 0.f);
   __syncthreads();
   constexpr int kPieces = kBrickChannels * wxn * TZ * 8;
 #pragma unroll 4
@@ -302,6 +334,13 @@ __device__ __forceinline__ void brick_finish(const float4_t (&acc)[kBrickChannel
         if (x + k < p.W) dst[k] = first ? e[k] : store_cast<__half>(load(dst + k) + load(&e[k]));
     }
   }
+}
+
+// the lane's number, worked out where it is used: kept, it would be one register too many
+__device__ __forceinline__ int brick_lane() {
+  int lane;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+  return lane;
 }
 
 // where part `k` of `parts` of a list begins
@@ -332,13 +371,9 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
   // in elements; the second is four rows on, or the same
   const int piece = col / 8 * cells + min(col % 8, p.od - 1) * ohw + quad * p.ow;
 
-  // and its places in a roi's tables
-  const int at_x = (X0 + bx + col % 8) * kBrickCells, at_y = (brick_row_y(p) + Y0 + col / 8) * kBrickCells + 2 * quad,
-            at_z = (brick_row_z(p) + Z0 + col % 8) * kBrickCells + quad % 2 * 4;
   const bool own_block = col / 8 == quad / 2;
   const bool twice = quad + 4 >= p.oh;   // the lane's second row is its first again
   const unsigned to_second = twice ? 0 : 8 * p.ow;
-  const float taken = twice ? -1.f : 0.f;
 
   if (threadIdx.x == 0) special = 0;
   __syncthreads();
@@ -360,10 +395,10 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
 #pragma unroll
       for (int k = 0; k < 4; k++) acc[i][k] = float4_t{0.f, 0.f, 0.f, 0.f};
     if (have > 0) {
-      unsigned entries = list[min(lane, have - 1)];   // 64 at a time, one per lane
+      unsigned entries = list[min(brick_lane(), have - 1)];   // 64 at a time, one per lane
       auto entry = [&](const int i) {
         if (i % kWave == 0 && i > 0) {
-          entries = list[min(i + lane, have - 1)];
+          entries = list[min(i + brick_lane(), have - 1)];
           asm volatile("" : "+v"(entries));   // (a wait here and not where it is used, which would be one for all that is on its way)
         }
         return static_cast<unsigned>(__builtin_amdgcn_readlane(entries, i % kWave));
@@ -371,12 +406,16 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
       // what a lane needs of a roi's tables: its voxel's row of x, its rows' pairs of y, and four weights of z
       struct Weights { float4 x0, x1; float2 y[4]; float4 z; };
       auto fetch = [&](unsigned n, Weights &w) {
-        const float *tab = tables + static_cast<long>(n) * rows * kBrickCells;
+        // (its places there, in bytes)
+        const unsigned at = brick_lane(), c = at % 16, q = at / 16;
+        const unsigned at_x = (X0 + bx + c % 8) * (kBrickCells * 4), at_y = (brick_row_y(p) + Y0 + c / 8) * (kBrickCells * 4) + q * 8,
+                       at_z = (brick_row_z(p) + Z0 + c % 8) * (kBrickCells * 4) + q % 2 * 16;
+        const char *tab = reinterpret_cast<const char *>(tables + static_cast<long>(n) * rows * kBrickCells);
         const float4 *x = reinterpret_cast<const float4 *>(tab + at_x);
         w.x0 = x[0];
         w.x1 = x[1];
 #pragma unroll
-        for (int k = 0; k < 4; k++) w.y[k] = *reinterpret_cast<const float2 *>(tab + at_y + 2 * k * kBrickCells);
+        for (int k = 0; k < 4; k++) w.y[k] = *reinterpret_cast<const float2 *>(tab + (at_y + 2 * k * kBrickCells * 4));
         w.z = *reinterpret_cast<const float4 *>(tab + at_z);
       };
       // A roi's gradient of the 16 channels is one run of memory.  It comes to LDS as it is, 1024 bytes a load, from the 4-byte
@@ -398,16 +437,17 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
       // that it places for other loads count these among them, so that they are longer than they need be, never shorter.)
       const unsigned ring_at = __builtin_amdgcn_readfirstlane(
           static_cast<unsigned>(reinterpret_cast<unsigned long long>((__attribute__((address_space(3))) unsigned char *)ring_lds)));
-      auto to_lds = [&](const Run &run, const int piece_at, const int place) {
+      auto to_lds = [&](const Run &run, const int at, const int place) {
         unsigned kept;   // (m0 is the compiler's own: it cannot be named as changed, so it gets back what it had)
         asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
-                     : "=&s"(kept) : "s"(__builtin_amdgcn_readfirstlane(ring_at + place * 1024)), "v"(lane * 16 + piece_at * 1024), "s"(run.src) : "memory");
+                     : "=&s"(kept) : "s"(__builtin_amdgcn_readfirstlane(ring_at + place * 1024)), "v"(at), "s"(run.src) : "memory");
       };
       auto bring = [&](const Run &run, int place, const int from, const int to) {
+        int at = brick_lane() * 16 + from * 1024;
 #pragma unroll 1
-        for (int i = from; i < to; i++) {
-          to_lds(run, i, place);
-          if (place == 0 && i > 0) to_lds(run, i, ring);
+        for (int i = from; i < to; i++, at += 1024) {
+          to_lds(run, at, place);
+          if (place == 0 && i > 0) to_lds(run, at, ring);
           place = place + 1 == ring ? 0 : place + 1;
         }
         return place;
@@ -421,12 +461,13 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
         s[0] = *reinterpret_cast<const V *>(from);
         s[1] = *reinterpret_cast<const V *>(from + to_second);
       };
-      // the present roi's gradient as a turn has it, in LDS
+      // the present roi's gradient as a turn has it, in LDS; whether there is anything
       auto screen = [&](int place, const int turn) {
         BrickKinds has;
+        unsigned char *const mine = ring_lds + brick_lane() * 16;
 #pragma unroll 2
         for (int i = 0; i < pieces; i++) {
-          u32x4 *const at = reinterpret_cast<u32x4 *>(ring_lds + place * 1024) + lane;
+          u32x4 *const at = reinterpret_cast<u32x4 *>(mine + place * 1024);
           u32x4 v = *at;
 #pragma unroll
           for (int j = 0; j < 4; j++) v[j] = brick_screen(v[j], turn, has);
@@ -435,55 +476,73 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
           place = place + 1 == ring ? 0 : place + 1;
         }
         const auto any = [](const unsigned word, const unsigned bit) { return __ballot(word != 0) != 0 ? bit : 0u; };
-        bits |= any(has.plus, kBrickHasPlus) | any(has.minus, kBrickHasMinus) | any(has.nan, kBrickHasNan) | any(has.finite, kBrickHasFinite);
+        bits |= any(has.plus, kBrickHasPlus) | any(has.minus, kBrickHasMinus) | any(has.nan, kBrickHasNan);
+        return any(has.now, 1u) != 0;
       };
       Weights w;
       unsigned e = entry(0);
-      fetch(e & ~(kBrickUpper | kBrickLower), w);
-      Run here = run_of(e & ~(kBrickUpper | kBrickLower));
+      fetch(e & kBrickNumber, w);
+      Run here = run_of(e & kBrickNumber);
       int first = 0, next_place = bring(here, 0, 0, pieces);   // in the ring: of the present roi, of the next
       for (int done = 0; done < have; done++) {
         asm volatile("s_waitcnt vmcnt(0)" : : : "memory");   // the gradient is here, and the tables
         asm volatile("" : "+v"(w.x0.x), "+v"(w.x0.y), "+v"(w.x0.z), "+v"(w.x0.w), "+v"(w.x1.x), "+v"(w.x1.y), "+v"(w.x1.z), "+v"(w.x1.w));
         asm volatile("" : "+v"(w.y[0].x), "+v"(w.y[0].y), "+v"(w.y[1].x), "+v"(w.y[1].y), "+v"(w.y[2].x), "+v"(w.y[2].y), "+v"(w.y[3].x),
                           "+v"(w.y[3].y), "+v"(w.z.x), "+v"(w.z.y), "+v"(w.z.z), "+v"(w.z.w));
-        if (turn != kBrickAll) screen(first, turn);
+        const bool idle = turn != kBrickAll && !screen(first, turn);
         const bool more = done + 1 < have;
-        const unsigned e2 = more ? entry(done + 1) : e, n2 = e2 & ~(kBrickUpper | kBrickLower);
+        const unsigned e2 = more ? entry(done + 1) : e, n2 = e2 & kBrickNumber;
         const Run run2 = run_of(n2);
         int first2 = next_place;
         Weights w2;
         fetch(n2, w2);
         if (more) next_place = bring(run2, first2, 0, early);
         const float ws[4] = {own_block ? w.z.x : 0.f, own_block ? w.z.y : 0.f, own_block ? w.z.z : 0.f, own_block ? w.z.w : 0.f};
-        const u32x4 left = brick_left(ws);
         const float xs[8] = {w.x0.x, w.x0.y, w.x0.z, w.x0.w, w.x1.x, w.x1.y, w.x1.z, w.x1.w};
-        const bool half[2] = {(e & kBrickUpper) != 0, (e & kBrickLower) != 0};
         // (from the 4-byte boundary, and shifted after: 16 bytes at a 2-byte boundary take LDS 60 clocks, 660 instead of 380 us of all)
         const unsigned at = (piece + here.odd / 2) / 2 * 4 + first * 1024, end = ring * 1024;
         const unsigned shift = (piece + here.odd / 2) % 2 * 16;
         const int pair = 4 * cells;   // bytes from two channels to the next
+        const BrickLeft left = brick_left(ws, 1.f / kBrickWeight);
+        const u32x4 left_both = brick_pair(left.value, left.rest);
+        const bool upper = !idle && (e & kBrickUpper) != 0, lower = !idle && (e & kBrickLower) != 0;
+        // Two pairs of rows of voxels, or with all bits (EXACT) one, whose operands take as many registers.  `over`: the roi's last sweep.
+        auto sweep = [&](auto k0_, auto exact_, const bool over) {
+          constexpr bool EXACT = decltype(exact_)::value;
+          constexpr int K0 = decltype(k0_)::value, KN = EXACT ? 1 : 2, FORMS = EXACT ? 2 : 1;
+          unsigned from = at, second = to_second;
+          asm volatile("" : "+v"(second));
+          const float taken = second == 0 ? -1.f : 0.f;   // the second row is the first again
+          float weight = EXACT ? kBrickExactWeight : kBrickWeight;
+          u32x4 right[FORMS][KN][2], left_value{}, left_rest{};   // the second form: what the rounding left of the first
+          if constexpr (EXACT) {
+            asm volatile("" : "+v"(from), "+v"(weight));   // (nothing below is formed for several sweeps and kept: that takes more registers than there are)
+            const BrickLeft l = brick_left(ws, 128.f), small = brick_left(ws, 1.f / kBrickExactWeight);
+            left_value = brick_pair(l.value, small.value);
+            left_rest = brick_pair(l.rest, small.rest);
+          }
 #pragma unroll
-        for (int h = 0; h < 2; h++) {   // the upper and the lower four rows of the brick
-          if (!half[h]) continue;
-          u32x4 right[2][2];
-#pragma unroll
-          for (int k = 0; k < 2; k++)
+          for (int k = 0; k < KN; k++)
 #pragma unroll
             for (int ks = 0; ks < 2; ks++) {
-              const float y = (ks == 0 ? w.y[2 * h + k].x : w.y[2 * h + k].y) * kBrickWeight;
+              const float y = (ks == 0 ? w.y[K0 + k].x : w.y[K0 + k].y) * weight;
               float f[8];
 #pragma unroll
               for (int j = 0; j < 8; j++) f[j] = y * xs[j];
-              right[k][ks] = M::pack(f);
+              right[0][k][ks] = M::pack(f);
               if (ks == 1) {
 #pragma unroll
-                for (int j = 0; j < 8; j++) f[j] = fmaf(M::element(right[k][1], j), taken, f[j]);
-                right[k][1] = M::pack(f);
+                for (int j = 0; j < 8; j++) f[j] = fmaf(M::element(right[0][k][1], j), taken, f[j]);
+                right[0][k][1] = M::pack(f);
+              }
+              if constexpr (EXACT) {   // (the first row's stand in the second one's place already where that is free)
+#pragma unroll
+                for (int j = 0; j < 8; j++) f[j] = (f[j] - M::element(right[0][k][ks], j)) * (ks == 0 ? 1.f + taken : 1.f);
+                right[FORMS - 1][k][ks] = M::pack(f);
               }
             }
 #pragma unroll
-          for (int i = 0; i < 4; i++) read(at + i * pair, end, slot[i]);
+          for (int i = 0; i < 4; i++) read(from + i * pair, end, slot[i]);
 #pragma unroll
           for (int i = 0; i < kBrickChannels / 2; i++) {
             u32x4 g[2];
@@ -493,21 +552,48 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
               g[ks] = u32x4{__builtin_amdgcn_alignbit(v.y, v.x, shift), __builtin_amdgcn_alignbit(v.z, v.y, shift),
                             __builtin_amdgcn_alignbit(v.w, v.z, shift), v.w >> shift};
             }
-            float4_t part[2] = {float4_t{0.f, 0.f, 0.f, 0.f}, float4_t{0.f, 0.f, 0.f, 0.f}};
+            float4_t part[KN];
 #pragma unroll
-            for (int ks = 0; ks < 2; ks++)
+            for (int k = 0; k < KN; k++) part[k] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-              for (int k = 0; k < 2; k++) part[k] = M::run16(g[ks], right[k][ks], part[k]);
-            if (i < 4) read(at + (i + 4) * pair, end, slot[i]);
-            if (i == 3 && (h == 1 || !half[1])) {
+            for (int form = FORMS - 1; form >= 0; form--)
+#pragma unroll
+              for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+                for (int k = 0; k < KN; k++) part[k] = M::run16(g[ks], right[form][k][ks], part[k]);
+            if (i < 4) read(from + (i + 4) * pair, end, slot[i]);
+            if (i == 3 && over) {
 #pragma unroll
               for (int j = 0; j < 4; j++) asm volatile("" : "+v"(slot[j][0]), "+v"(slot[j][1]) : : "memory");   // they have been read
               if (more) next_place = bring(run2, next_place, early, pieces);
             }
 #pragma unroll
-            for (int k = 0; k < 2; k++) acc[i][2 * h + k] = M::run16(left, brick_right(part[k]), acc[i][2 * h + k]);
+            for (int k = 0; k < KN; k++) {
+              if constexpr (EXACT) {
+                const u32x4 sums = brick_sums_exact(part[k]);
+                acc[i][K0 + k] = M::run16(left_value, sums, M::run16(left_rest, sums, acc[i][K0 + k]));
+              } else {
+                acc[i][K0 + k] = M::run16(left_both, brick_sums(part[k]), acc[i][K0 + k]);
+              }
+            }
           }
+        };
+        // (one condition after the other, not two branches of one: where those meet, all sums are copied)
+        using std::integral_constant;
+        const bool exact = turn == kBrickFinite || (e & kBrickExact) != 0 || ((e & kBrickNumber) == static_cast<unsigned>(p.R) - 1u && c_base + kBrickChannels >= p.C);
+        if (!exact && upper) sweep(integral_constant<int, 0>(), std::false_type(), !lower);
+        if (!exact && lower) sweep(integral_constant<int, 2>(), std::false_type(), true);
+        unsigned all_bits = __builtin_amdgcn_readfirstlane(exact ? 1 : 0);
+        asm volatile("" : "+s"(all_bits));
+        if (all_bits != 0 && upper) {
+          sweep(integral_constant<int, 0>(), std::true_type(), false);
+          sweep(integral_constant<int, 1>(), std::true_type(), !lower);
         }
+        if (all_bits != 0 && lower) {
+          sweep(integral_constant<int, 2>(), std::true_type(), false);
+          sweep(integral_constant<int, 3>(), std::true_type(), true);
+        }
+        if (idle && more) next_place = bring(run2, next_place, early, pieces);
         e = e2; w = w2; here = run2; first = first2;
       }
     }
@@ -515,20 +601,19 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
     if constexpr (SHARED) {
       if (have == 0) return;
     } else {   // (both wavefronts take the same turns: they leave their sums together)
-      if (bits != 0 && lane == 0) atomicOr(&special, bits);
+      if (bits != 0 && brick_lane() == 0) atomicOr(&special, bits);
       __syncthreads();
       bits = __builtin_amdgcn_readfirstlane(special);
     }
     if (turn == kBrickAll && bits != 0) {
-      turn = kBrickPlus;
+      turn = kBrickFinite;
       continue;
     }
-    const bool infinite = (bits & (kBrickHasPlus | kBrickHasMinus)) != 0;
-    const bool sums = turn == kBrickAll || turn == kBrickFinite, first = turn == kBrickAll || turn == kBrickPlus;
-    const float mark = turn == kBrickMinus ? -INFINITY : infinite ? INFINITY : NAN;   // for what the turn's gradients reach
+    const bool infinite = (bits & (kBrickHasPlus | kBrickHasMinus)) != 0, first = turn <= kBrickFinite;
+    const float mark = turn == kBrickMinus ? -INFINITY : infinite ? INFINITY : NAN;   // for what the later turns' gradients reach
     if constexpr (SHARED) {
       float4_t *to =
-          partial + ((brick * cblocks + c_base / kBrickChannels) * parts + place.part) * (kBrickChannels / 2 * 4 * kWave) + lane;
+          partial + ((brick * cblocks + c_base / kBrickChannels) * parts + place.part) * (kBrickChannels / 2 * 4 * kWave) + brick_lane();
       asm volatile("" : "+v"(to));   // (the addresses are not formed before the turns and kept)
       if (turn == kBrickAll) {
 #pragma unroll
@@ -542,7 +627,7 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
           for (int k = 0; k < 4; k++) {
             float4_t sum = acc[i][k];
 #pragma unroll
-            for (int r = 0; r < 4; r++) sum[r] = sums ? sum[r] : sum[r] > 0.f ? mark : 0.f;
+            for (int r = 0; r < 4; r++) sum[r] = first ? sum[r] : sum[r] > 0.f ? mark : 0.f;
             if (!first) sum += to[0];
             to[0] = sum;
             to += kWave;
@@ -550,10 +635,10 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
           }
       }
     } else {
-      brick_finish<LOG_WX>(acc, place, grad, p, lds, sums, mark, first);
+      brick_finish<LOG_WX>(acc, place, grad, p, lds, first, mark);
     }
-    if (turn == kBrickPlus && infinite && (bits & (kBrickHasMinus | kBrickHasNan))) turn = kBrickMinus;
-    else if (turn != kBrickAll && turn != kBrickFinite && (bits & kBrickHasFinite)) turn = kBrickFinite;
+    if (turn == kBrickFinite && (bits & (kBrickHasPlus | kBrickHasNan))) turn = kBrickPlus;
+    else if ((turn == kBrickFinite || (turn == kBrickPlus && infinite)) && (bits & (kBrickHasMinus | kBrickHasNan))) turn = kBrickMinus;
     else return;
     if constexpr (!SHARED) __syncthreads();   // the sums have been read and are in memory
   }
@@ -582,7 +667,7 @@ __global__ __launch_bounds__(kWave << LOG_WX) void roi_brick_fold_kernel(
 #pragma unroll
       for (int k = 0; k < 4; k++) acc[i][k] += from[(i * 4 + k) * kWave];
   }
-  brick_finish<LOG_WX>(acc, place, grad, p, lds, true, 0.f, true);
+  brick_finish<LOG_WX>(acc, place, grad, p, lds, true, 0.f);
 }
 
 static size_t brick_tables_bytes(const RoiProblem &p) {
@@ -613,7 +698,7 @@ bool roi_brick_applies(int dtype, const RoiProblem &p) {
   if (p.D > 0x7fff || p.H > 0x7fff || p.W > 0x7fff) return false;
   const long slab = static_cast<long>(p.C) * p.od * p.oh * p.ow * 2;   // bytes of a roi's gradient
   if (slab < kBrickPad || slab + kBrickPad >= (1L << 31)) return false;
-  if (static_cast<long>(p.R) * brick_rows(p) * kBrickCells * 4 >= (1L << 31) || p.R >= (1 << 30)) return false;
+  if (static_cast<long>(p.R) * brick_rows(p) * kBrickCells * 4 >= (1L << 31) || p.R >= (1 << 29)) return false;
   // Small maps have too few bricks to fill the chip, and few channels leave most of a product idle; there the kernel that adds box by box is
   // the faster one.  Forward and backward pass there -> here: [1,16,14,40,66] with 163 rois of 7^3 cells (90 bricks) 37 -> 54 us,
   // [4,36,10,20,26] with 112 (96 bricks) 59 -> 72, [2,19,6,125,50] with 89 of 8^3 (224 bricks) 38 -> 42; [2,16,12,94,77] with 987 (480 bricks) 84 -> 77,
