@@ -693,6 +693,11 @@ static int brick_parts(const RoiProblem &p) {
   return static_cast<int>(std::max(std::min(wavefronts / brick_waves(p), 16L), 1L));
 }
 
+// Kilobytes of a roi's 16 channels (and behind them: a row of cells may be read as 16 bytes, and rows up to the eighth), and of a wavefront's
+// ring: as much as lets eight wavefronts share a compute unit's LDS, or one roi's
+static int brick_pieces(const RoiProblem &p) { return (kBrickChannels * p.od * p.oh * p.ow * 2 + 2 + kBrickPad + 1023) / 1024; }
+static int brick_ring(const RoiProblem &p) { return std::max(std::min(2 * brick_pieces(p), 18), brick_pieces(p)); }
+
 bool roi_brick_applies(int dtype, const RoiProblem &p) {
   if (dtype != MV_F16 || p.ndim != 3 || p.od > kBrickCells || p.oh > kBrickCells || p.ow > kBrickCells || !roi_pool_applies(dtype, p)) return false;
   if (p.D > 0x7fff || p.H > 0x7fff || p.W > 0x7fff) return false;
@@ -704,6 +709,10 @@ bool roi_brick_applies(int dtype, const RoiProblem &p) {
   // [4,36,10,20,26] with 112 (96 bricks) 59 -> 72, [2,19,6,125,50] with 89 of 8^3 (224 bricks) 38 -> 42; [2,16,12,94,77] with 987 (480 bricks) 84 -> 77,
   // [1,32,18,57,123] with 463 91 -> 83, [2,256,10,64,67] with 363 of 5^3 173 -> 130.  Over 240 heads of 1 - 4000 rois, 1 - 256 channels and up to
   // 64 x 128 x 128 voxels 1.22 times as fast in geometric mean, the slowest 0.92.
+  // Gradients that fill a wavefront's ring: hardly any of the next roi's comes in beside the present one's products, so that long lists take twice
+  // as long as others.  500 such heads (8^3 cells), box by box / here: below two rois for five bricks 1.30 (from 4096 wavefronts on) to 0.90 (below
+  // 800), up to five for four 1.08 to 0.76, beyond 0.80 - 0.87 ([4,128,48,60,21] with 3808 rois 1215 and 1946 us).
+  if (brick_ring(p) < brick_pieces(p) + 4 && 5L * p.R >= 2 * brick_count(p)) return false;
   return brick_count(p) * p.C >= 7680 && brick_waves(p) * 16 < (1L << 31) - 8;
 }
 
@@ -738,10 +747,7 @@ int roi_brick_backward(const void *grad_output, const void *rois, void *grad_inp
   const int copies = (slab + kBrickPad / 2 + 3 * kWave * 8 - 1) / (3 * kWave * 8);
   // (rows of eight cells have to lie at 4-byte boundaries: what a shift brings in is one cell short of that)
   if (p.ow == kBrickCells && reinterpret_cast<uintptr_t>(grad_output) % 4 != 0) return -1;
-  // kilobytes of a roi's 16 channels (and behind them: a row of cells may be read as 16 bytes, and rows up to the eighth), and of a
-  // wavefront's ring: as much as lets eight wavefronts share a compute unit's LDS, or one roi's
-  const int pieces = (kBrickChannels * p.od * p.oh * p.ow * 2 + 2 + kBrickPad + 1023) / 1024;
-  const int ring = std::max(std::min(2 * pieces, 18), pieces);
+  const int pieces = brick_pieces(p), ring = brick_ring(p);
   const int log_wx = p.W > kBrickEdge ? 1 : 0;
   const int nx = (p.W + (8 << log_wx) - 1) >> (3 + log_wx), ny = brick_up(p.H) / kBrickEdge, cblocks = (p.C + kBrickChannels - 1) / kBrickChannels;
   const int nz = brick_up(p.D) / kBrickEdge;

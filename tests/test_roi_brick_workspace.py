@@ -19,3 +19,16 @@ def test_lists_are_no_larger_than_the_copy(dims, rois, lists):
     assert asked >= copy
     if not lists:
         assert asked == copy
+
+
+@pytest.mark.parametrize("cells,rois,served", [
+    ((7, 7, 7), 4000, True),
+    ((7, 7, 8), 4000, True),      # 13 kilobytes of a ring of 18
+    ((8, 8, 8), 4000, False),     # 17 of them: box by box
+    ((7, 8, 8), 4000, False),
+    ((8, 8, 8), 345, True),       # fewer than two rois for five of the 864 bricks
+    ((8, 8, 8), 346, False),
+])
+def test_gradients_that_fill_their_ring(cells, rois, served):
+    from test_gpu_roi_brick import bricks_apply
+    assert bricks_apply((2, 256, 24, 96, 96), rois, cells) == served
