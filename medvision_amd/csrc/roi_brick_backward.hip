@@ -336,11 +336,12 @@ __device__ __forceinline__ void brick_finish(const float4_t (&acc)[kBrickChannel
   }
 }
 
-// the lane's number, worked out where it is used: kept, it would be one register too many
+// the lane's number, worked out where it is used: kept, it would be one register too many.  (The instructions are the compiler's own: around
+// inline assembly it leaves no wait for a matrix instruction that still reads or writes the register that the result gets.)
 __device__ __forceinline__ int brick_lane() {
-  int lane;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
-  return lane;
+  unsigned none = 0;
+  asm volatile("" : "+s"(none));
+  return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, none));
 }
 
 // where part `k` of `parts` of a list begins
@@ -438,8 +439,10 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
       const unsigned ring_at = __builtin_amdgcn_readfirstlane(
           static_cast<unsigned>(reinterpret_cast<unsigned long long>((__attribute__((address_space(3))) unsigned char *)ring_lds)));
       auto to_lds = [&](const Run &run, const int at, const int place) {
-        unsigned kept;   // (m0 is the compiler's own: it cannot be named as changed, so it gets back what it had)
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
+        // (m0 is the compiler's own: it cannot be named as changed, so it gets back what it had; and there are five waits before the load, what it
+        // needs where the compiler has just fetched its scalars from vector registers)
+        unsigned kept;
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 4\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
                      : "=&s"(kept) : "s"(__builtin_amdgcn_readfirstlane(ring_at + place * 1024)), "v"(at), "s"(run.src) : "memory");
       };
       auto bring = [&](const Run &run, int place, const int from, const int to) {
@@ -593,7 +596,10 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
           sweep(integral_constant<int, 2>(), std::true_type(), false);
           sweep(integral_constant<int, 3>(), std::true_type(), true);
         }
-        if (idle && more) next_place = bring(run2, next_place, early, pieces);
+        if (idle && more) {
+          asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");   // the screened gradient has been written: its places may be taken
+          next_place = bring(run2, next_place, early, pieces);
+        }
         e = e2; w = w2; here = run2; first = first2;
       }
     }
