@@ -28,6 +28,9 @@ def test_lists_are_no_larger_than_the_copy(dims, rois, lists):
     ((7, 8, 8), 4000, False),
     ((8, 8, 8), 345, True),       # fewer than two rois for five of the 864 bricks
     ((8, 8, 8), 346, False),
+    ((4, 4, 4), 4000, True),      # small gradients: two fit their ring, however small it is
+    ((5, 5, 5), 4000, True),
+    ((2, 2, 2), 4000, True),
 ])
 def test_gradients_that_fill_their_ring(cells, rois, served):
     from test_gpu_roi_brick import bricks_apply
