@@ -696,7 +696,7 @@ static long brick_waves(const RoiProblem &p) { return brick_count(p) * ((p.C + k
 static int brick_parts(const RoiProblem &p) {
   if (4L * p.R < 5 * brick_count(p)) return 1;
   const long wavefronts = p.R >= 8 * brick_count(p) ? 4096 : 2048;
-  return static_cast<int>(std::max(std::min(wavefronts / brick_waves(p), 16L), 1L));
+  return static_cast<int>(std::max(wavefronts / brick_waves(p), 1L));   // (at most eight: roi_brick_applies asks for 480 pairs)
 }
 
 // Kilobytes of a roi's 16 channels (and behind them: a row of cells may be read as 16 bytes, and rows up to the eighth), and of a wavefront's

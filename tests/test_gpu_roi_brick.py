@@ -243,3 +243,21 @@ def test_large_boxes_keep_their_bits(oracle, size, rois, cells, ratio, low, high
     got = torch.autograd.grad(out, x, gy.to(DEV))[0].cpu().double()
     own = (want.half().double() - want).norm()
     assert (got - want).norm() <= 1.01 * own + 1e-5 * want.norm()
+
+
+@pytest.mark.parametrize("images,channels,size,rois", [
+    (2, 128, (9, 17, 33), 480),      # eight share a brick, the most
+    (4, 80, (40, 33, 8), 130),       # one brick along x: four share it
+    (4, 80, (40, 33, 8), 800),       # eight
+])
+def test_shared_bricks(oracle, images, channels, size, rois):
+    from medvision_amd.ops.roi_align_nd import roi_align_3d
+    g = wl.gen(rois + channels)
+    dims, cells = (images, channels, *size), (3, 4, 5)
+    assert bricks_apply(dims, rois, cells)
+    boxes = boxes_of(g, images, size, rois, 9)
+    x = torch.zeros(dims, dtype=torch.float16, device=DEV, requires_grad=True)
+    out = roi_align_3d(x, boxes.to(DEV), cells, 1.0, 2, 1)
+    gy = torch.randn(out.shape, generator=g).half()
+    want = oracle.roi_align_backward(gy, boxes, x.shape, 1.0, 2, True, 1, False).reshape(x.shape)
+    assert_close(torch.autograd.grad(out, x, gy.to(DEV))[0], want, TOL, "gradient")
