@@ -45,16 +45,19 @@ __device__ __forceinline__ ElasticTaps elastic_taps(int i, int n, int points, do
 }
 
 // The taps of position i + off on an axis of `size` voxels, those of clamped_tap on the open interval (-1, size), without 64-bit
-// arithmetic: i + floor(off) is the position's floor, and off - floor(off) its fraction, rounded once.
-__device__ __forceinline__ bool elastic_tap(int i, float off, int size, int &lo, int &hi, float &frac) {
+// arithmetic: i + floor(off) is the position's floor, and off - floor(off) its fraction, rounded once.  `nearest`: the voxel at order 0, by the
+// fraction as it is before that rounding (floor(off) + 0.5 is a number of 32 bits, so the comparison is exact).
+__device__ __forceinline__ bool elastic_tap(int i, float off, int size, int &lo, int &hi, float &frac, int &nearest) {
   const float f = floorf(off);
   const bool near = fabsf(off) < 1e6f;   // (farther is outside, and not a number too)
   const int base = i + static_cast<int>(near ? f : 0.f);
   frac = off - f;
   const bool inside = near && base < size && (base >= 0 || (base == -1 && frac > 0.f));
-  if (base < 0 || base >= size - 1) frac = 0.f;
+  const bool border = base < 0 || base >= size - 1;
+  if (border) frac = 0.f;
   lo = min(max(base, 0), size - 1);
   hi = min(lo + 1, size - 1);
+  nearest = !border && off > f + 0.5f ? hi : lo;
   return inside;
 }
 
@@ -117,15 +120,13 @@ __global__ __launch_bounds__(kElThreads, 6) void elastic_warp_kernel(const T *__
       }
     }
     const int z = z0 + k;
-    int zi[2], yi[2], xi[2];
+    int zi[2], yi[2], xi[2], zn, yn, xn;
     float lz, lh, lw;
-    const bool live_z = elastic_tap(z, off[0], s.D, zi[0], zi[1], lz), live_y = elastic_tap(y, off[1], s.H, yi[0], yi[1], lh),
-               live = elastic_tap(x, off[2], s.W, xi[0], xi[1], lw) && live_z && live_y;
+    const bool live_z = elastic_tap(z, off[0], s.D, zi[0], zi[1], lz, zn), live_y = elastic_tap(y, off[1], s.H, yi[0], yi[1], lh, yn),
+               live = elastic_tap(x, off[2], s.W, xi[0], xi[1], lw, xn) && live_z && live_y;
     const unsigned q = static_cast<unsigned>((z * s.H + y) * s.W + x);
     if constexpr (std::is_same<T, int>::value) {
-      // (the low voxel where 1 - fraction >= 0.5)
-      const unsigned from = static_cast<unsigned>(((1.f - lz >= 0.5f ? zi[0] : zi[1]) * s.H + (1.f - lh >= 0.5f ? yi[0] : yi[1])) * s.W +
-                                                  (1.f - lw >= 0.5f ? xi[0] : xi[1]));
+      const unsigned from = static_cast<unsigned>((zn * s.H + yn) * s.W + xn);
       for (int ch = 0; ch < s.C; ch++) {
         const long plane = (static_cast<long>(b) * s.C + ch) * P;
         (out + plane)[q] = live ? (img + plane)[from] : 0;

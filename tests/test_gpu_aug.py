@@ -334,3 +334,27 @@ def test_elastic_stage_keeps_a_given_field(aug):
     assert_close(stage.elastic_transform(img), first, 1e-5, "from the field")
     stage.tmp_params = torch.zeros_like(field)
     assert torch.equal(stage.elastic_transform(img), img)
+
+
+def test_elastic_warp_labels_next_to_ties():
+    """Displacements a bit from half a voxel, at control points (where the upsampling gives them as they are): the voxel that the fp64 fraction picks."""
+    from medvision_amd._lib import native
+    g = wl.gen(17)
+    batch, size, points = 256, (2, 2, 5), (7, 7, 13)       # voxel i lies on control point 2 i + 2
+    bit = 2.0 ** -25
+    steps = torch.tensor([s * (k + 0.5 + e) for s in (1, -1) for k in (0, 1) for e in (-2 * bit, -bit, 0.0, bit, 2 * bit)] + [0.0, 1e-30, -1e-30])
+    grid = steps[torch.randint(0, len(steps), (batch, 3, *points), generator=g)].float()
+    seg = torch.randint(1, 1 << 20, (batch, 1, *size), generator=g, dtype=torch.int32)
+    where = torch.stack(torch.meshgrid(*[torch.arange(n) for n in size], indexing="ij"))
+    at = where + grid.double()[:, :, 2::2, 2::2, 2::2][:, :, :size[0], :size[1], :size[2]]
+    live = torch.ones(batch, *size, dtype=torch.bool)
+    index = []
+    for a in range(3):
+        p = at[:, a]
+        live &= (p > -1) & (p < size[a])
+        p = p.clamp(0, size[a] - 1)
+        low = p.floor()
+        index.append(torch.where(1 - (p - low) >= 0.5, low, low + 1).long())
+    want = torch.where(live, seg[torch.arange(batch).view(-1, 1, 1, 1), 0, index[0], index[1], index[2]], 0)
+    got = native.elastic_warp(seg.to(DEV), grid.to(DEV), 1.5)
+    assert got is not None and torch.equal(got[:, 0].cpu(), want)
