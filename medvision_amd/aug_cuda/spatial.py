@@ -483,10 +483,10 @@ class CudaRandomElasticDeformation(CudaAugBase):
         return self._field
 
     def _warp_from_grid(self, image, order):
-        """The image warped without a dense field in memory; None where there is one already, or the kernel does not take these
-        sizes or types."""
+        """The image warped without a dense field in memory; None where there is one already or a subclass gives its own, or the kernel
+        does not take these sizes or types."""
         labels = image.dtype == torch.int32
-        if (self._field is not None or self.dim != 3 or self.INTER_ORDER != 3 or not image.is_cuda or order != (0 if labels else 1)
+        if (getattr(self.dense_field, '__func__', None) is not CudaRandomElasticDeformation.dense_field or self._field is not None or self.dim != 3 or self.INTER_ORDER != 3 or not image.is_cuda or order != (0 if labels else 1)
                 or image.shape[2 if self.batched else 1:] != tuple(self.image_shape)):
             return None
         if self._device_grid is None or self._device_grid.device != image.device:

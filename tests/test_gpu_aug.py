@@ -358,3 +358,27 @@ def test_elastic_warp_labels_next_to_ties():
     want = torch.where(live, seg[torch.arange(batch).view(-1, 1, 1, 1), 0, index[0], index[1], index[2]], 0)
     got = native.elastic_warp(seg.to(DEV), grid.to(DEV), 1.5)
     assert got is not None and torch.equal(got[:, 0].cpu(), want)
+
+
+@pytest.mark.parametrize("batched", [False, True])
+def test_elastic_stage_applies_a_subclass_field(aug, batched):
+    """A subclass, or an instance, with a dense field of its own: images and labels are warped by that one."""
+    base = aug.BatchCudaRandomElasticDeformation if batched else aug.CudaRandomElasticDeformation
+    size = (12, 14, 16)
+
+    def moved(self, device):
+        field = torch.zeros((2, 3, *size) if batched else (3, *size), device=device)
+        field[..., 2, :, :, :] = 1.0     # one voxel along x
+        return field
+
+    class Own(base):
+        dense_field = moved
+
+    img = torch.randn((2, 1, *size) if batched else (1, *size)).to(DEV)
+    seg = torch.randint(0, 9, img.shape, dtype=torch.int32).to(DEV)
+    for stage in (Own(1.0, 7, 0.9), base(1.0, 7, 0.9)):
+        if type(stage) is base:
+            stage.dense_field = lambda device: moved(None, device)
+        stage._forward_params({"img": img, "img_dim": 3})
+        for got, given in ((stage.elastic_transform(img), img), (stage.elastic_transform(seg, order=0), seg)):
+            assert torch.equal(got[..., :-1], given[..., 1:]) and not bool(got[..., -1].any())
