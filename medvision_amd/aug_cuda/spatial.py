@@ -201,12 +201,15 @@ class CudaRandomAffine(_Resampler, CudaAugBase):
         return geometry.window_rois(self.dim, start, end, *self._affine(), index=np.arange(self.batch))
 
     def _uploaded_rois(self, device):
-        # (the arrays of one row cost 6 us on the host, the native form 1)
-        scales, shifts, rotate = self._affine()
-        if self.batched or getattr(self._rois, '__func__', None) is not CudaRandomAffine._rois or len(rotate) != 1:
-            return super()._uploaded_rois(device)
-        start, end = self._window()
-        return native.window_roi(self.dim, start, end, scales, shifts, rotate[0], device)
+        # (the arrays of one row cost 6 us on the host, the native form 1; it takes a flat row of each, window_rois scalars and tables too)
+        if not self.batched and getattr(self._rois, '__func__', None) is CudaRandomAffine._rois:
+            (start, end), (scales, shifts, rotate) = self._window(), self._affine()
+            try:
+                angle, = rotate
+                return native.window_roi(self.dim, start, end, scales, shifts, angle, device)
+            except (TypeError, ValueError, RuntimeError):
+                pass
+        return super()._uploaded_rois(device)
 
     def _out_size(self):
         return self.image_shape

@@ -156,3 +156,31 @@ def test_elastic_stage_restored_from_an_older_state():
         assert again.tmp_params is field and again._field is field
         assert again._device_grid is None
     assert pickle.loads(pickle.dumps(stage)).tmp_params is None
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("values", [
+    (1.25, 0.1, 0.3),                                                            # scalars, as window_rois takes them
+    ([1.25] * 3, 0.1, [0.3]),
+    (np.array([1.1, 1.2, 1.3]), np.array([0.1, -0.2, 0.05]), np.array([0.3])),
+    (np.float32(1.25), [0.1, 0.0, np.float32(0.2)], 1),
+    ([[1.1, 1.2, 1.3]], [[0.1, -0.2, 0.05]], [[0.3]]),                           # rows of a table
+    ([1.1, 1.2, 1.3], np.array([[0.1, -0.2, 0.05]]), np.array(0.3)),
+])
+def test_affine_stage_takes_what_window_rois_takes(dim, values):
+    """Scalars, rows and tables from a stage's parameters: the roi of geometry.window_rois."""
+    from medvision_amd.aug_cuda import CudaRandomAffine
+
+    def cut(v):
+        if isinstance(v, list):
+            return [cut(x) for x in v] if isinstance(v[0], list) else v[:dim]
+        return v[..., :dim] if isinstance(v, np.ndarray) and v.ndim else v
+
+    class Given(CudaRandomAffine):
+        def _affine(self):
+            return tuple(cut(v) for v in values)
+
+    stage = Given(1.0, 0.2, 0.1, 30)
+    stage._init_params({"img": torch.zeros(1, *(12, 14, 16)[:dim]), "img_dim": dim})
+    got = stage._uploaded_rois(torch.device("cpu"))
+    assert np.array_equal(got.cpu().numpy(), stage._rois())
