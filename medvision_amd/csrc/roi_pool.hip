@@ -1853,15 +1853,16 @@ int roi_pool_forward(const void *input, const void *rois, void *output, int dtyp
   int cpb = pool_channels_per_block(p, blocked != nullptr && order != nullptr ? 3072 : 6144), joined = 1;
   // Without matrix cores a head of few rois and channels takes as few channels per workgroup as let all workgroups run at a time: four on a
   // compute unit with 30 KB for the boxes (LDS), three with 40 KB (223 fp32 rois x 32 channels 18.6 us with 1784 workgroups, 11.8 with 892; 16 bf16 x 256, 1024
-  // workgroups, 12.9 and 10.8).  From nine channels each on, large boxes would last longer than the rounds that this saves.
+  // workgroups, 12.9 and 10.8).  From nine channels each on, large boxes would last longer than the rounds that this saves, and with two or three
+  // a head's largest box lasts longer by as much as is saved (454 heads: 1.00 and 1.04 times as fast in the mean, one in seven slower by 5 - 30 %): those keep their workgroups, with 30 KB
+  // where that saves a round of them (128 fp32 rois x 16 channels 26.0 and 21.7 us).
   bool four = false;
   if (p.ndim == 3 && dtype != MV_F16 && pool_small_cells(p) && p.R <= 1024) {
     int fit = 1;
     while (fit <= 8 && pool_groups(p, fit) > 1024) fit++;
-    if (fit <= 8) {
-      cpb = fit;
-      four = pool_groups(p, fit) > 768;
-    }
+    if (fit > 3 && fit <= 8) cpb = fit;
+    const long groups = pool_groups(p, cpb);
+    four = fit <= 8 && (groups + 1023) / 1024 < (groups + 767) / 768;
   }
   if (pool_small_cells(p)) {
     joined = std::max(std::min(p.C, dtype == MV_F16 ? 16 : 4) / cpb, 1);
