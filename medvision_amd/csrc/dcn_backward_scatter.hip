@@ -57,10 +57,11 @@ template <int CH, int FROM> __device__ __forceinline__ int row_word(int v) {
 template <int CH, int FROM> __device__ __forceinline__ float row_value(float v) {
   return __int_as_float(row_word<CH, FROM>(__float_as_int(v)));
 }
-// round(x) for |x| < 2^31 in one instruction
+// round(x) for |x| < 2^31 in one instruction (in the register of x: around inline assembly the compiler leaves no wait for a matrix instruction
+// that still reads a register which the result would get)
 __device__ __forceinline__ int round_word(float x) {
-  int r;
-  asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+  int r = __float_as_int(x);
+  asm("v_cvt_rpi_i32_f32 %0, %0" : "+v"(r));
   return r;
 }
 

@@ -162,10 +162,11 @@ __device__ __forceinline__ void own_wave_sync() {   // LDS of one wavefront is i
   __builtin_amdgcn_wave_barrier();
 }
 
-// round(x) for 0 <= x < 2^31 in one instruction
+// round(x) for 0 <= x < 2^31 in one instruction (in the register of x: around inline assembly the compiler leaves no wait for a matrix instruction
+// that still reads a register which the result would get)
 __device__ __forceinline__ unsigned own_round(float x) {
-  unsigned r;
-  asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+  unsigned r = __float_as_uint(x);
+  asm("v_cvt_rpi_i32_f32 %0, %0" : "+v"(r));
   return r;
 }
 
