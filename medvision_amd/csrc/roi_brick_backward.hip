@@ -439,20 +439,22 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
       const unsigned ring_at = __builtin_amdgcn_readfirstlane(
           static_cast<unsigned>(reinterpret_cast<unsigned long long>((__attribute__((address_space(3))) unsigned char *)ring_lds)));
       auto to_lds = [&](const Run &run, const int at, const int place) {
-        // (m0 is the compiler's own: it cannot be named as changed, so it gets back what it had; and there are five waits before the load, what it
-        // needs where the compiler has just fetched its scalars from vector registers)
-        unsigned kept;
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 4\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
-                     : "=&s"(kept) : "s"(__builtin_amdgcn_readfirstlane(ring_at + place * 1024)), "v"(at), "s"(run.src) : "memory");
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     : : "s"(__builtin_amdgcn_readfirstlane(ring_at + place * 1024)), "v"(at), "s"(run.src) : "memory");
       };
       auto bring = [&](const Run &run, int place, const int from, const int to) {
         int at = brick_lane() * 16 + from * 1024;
+        // (m0 is the compiler's own: it cannot be named as changed, so it gets back what it had; and five waits before the loads, what they need
+        // where the compiler has just fetched their scalars from vector registers)
+        unsigned kept;
+        asm volatile("s_mov_b32 %0, m0\n\ts_nop 4" : "=s"(kept) : "s"(run.src));
 #pragma unroll 1
         for (int i = from; i < to; i++, at += 1024) {
           to_lds(run, at, place);
           if (place == 0 && i > 0) to_lds(run, at, ring);
           place = place + 1 == ring ? 0 : place + 1;
         }
+        asm volatile("s_mov_b32 m0, %0" : : "s"(kept));
         return place;
       };
       const int early = min(ring - pieces, pieces);   // pieces that come in before the present roi has been read
