@@ -719,8 +719,10 @@ bool roi_brick_applies(int dtype, const RoiProblem &p) {
   // 64 x 128 x 128 voxels 1.22 times as fast in geometric mean, the slowest 0.92.
   // Gradients that fill a wavefront's ring: hardly any of the next roi's comes in beside the present one's products, so that long lists take twice
   // as long as others.  500 such heads (8^3 cells), box by box / here: below two rois for five bricks 1.30 (from 4096 wavefronts on) to 0.90 (below
-  // 800), up to five for four 1.08 to 0.76, beyond 0.80 - 0.87 ([4,128,48,60,21] with 3808 rois 1215 and 1946 us).
-  if (brick_ring(p) < std::min(2 * brick_pieces(p), brick_pieces(p) + 4) && 5L * p.R >= 2 * brick_count(p)) return false;
+  // 800), up to five for four 1.05 from 2048 wavefronts on and 0.76 - 0.95 below, beyond 0.80 - 0.87 ([4,128,48,60,21] with 3808 rois 1215 and 1946 us).
+  if (brick_ring(p) < std::min(2 * brick_pieces(p), brick_pieces(p) + 4) &&
+      (brick_waves(p) >= 2048 ? 4L * p.R >= 5 * brick_count(p) : 5L * p.R >= 2 * brick_count(p)))
+    return false;
   return brick_count(p) * p.C >= 7680 && brick_waves(p) * 16 < (1L << 31) - 8;
 }
 

@@ -26,8 +26,8 @@ def test_lists_are_no_larger_than_the_copy(dims, rois, lists):
     ((7, 7, 8), 4000, True),      # 13 kilobytes of a ring of 18
     ((8, 8, 8), 4000, False),     # 17 of them: box by box
     ((7, 8, 8), 4000, False),
-    ((8, 8, 8), 345, True),       # fewer than two rois for five of the 864 bricks
-    ((8, 8, 8), 346, False),
+    ((8, 8, 8), 1079, True),      # fewer than five rois for four of the 864 bricks
+    ((8, 8, 8), 1080, False),
     ((4, 4, 4), 4000, True),      # small gradients: two fit their ring, however small it is
     ((5, 5, 5), 4000, True),
     ((2, 2, 2), 4000, True),
@@ -35,3 +35,10 @@ def test_lists_are_no_larger_than_the_copy(dims, rois, lists):
 def test_gradients_that_fill_their_ring(cells, rois, served):
     from test_gpu_roi_brick import bricks_apply
     assert bricks_apply((2, 256, 24, 96, 96), rois, cells) == served
+
+
+@pytest.mark.parametrize("rois,served", [(28, True), (29, False)])
+def test_gradients_that_fill_their_ring_on_small_maps(rois, served):
+    """1152 pairs of a brick and 16 channels: two rois for five of the 72 bricks."""
+    from test_gpu_roi_brick import bricks_apply
+    assert bricks_apply((1, 256, 24, 32, 48), rois, (8, 8, 8)) == served
