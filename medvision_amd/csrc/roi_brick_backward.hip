@@ -715,8 +715,9 @@ bool roi_brick_applies(int dtype, const RoiProblem &p) {
   // Small maps have too few bricks to fill the chip, and few channels leave most of a product idle; there the kernel that adds box by box is
   // the faster one.  Forward and backward pass there -> here: [1,16,14,40,66] with 163 rois of 7^3 cells (90 bricks) 37 -> 54 us,
   // [4,36,10,20,26] with 112 (96 bricks) 59 -> 72, [2,19,6,125,50] with 89 of 8^3 (224 bricks) 38 -> 42; [2,16,12,94,77] with 987 (480 bricks) 84 -> 77,
-  // [1,32,18,57,123] with 463 91 -> 83, [2,256,10,64,67] with 363 of 5^3 173 -> 130.  Over 240 heads of 1 - 4000 rois, 1 - 256 channels and up to
-  // 64 x 128 x 128 voxels 1.22 times as fast in geometric mean, the slowest 0.92.
+  // [1,32,18,57,123] with 463 91 -> 83, [2,256,10,64,67] with 363 of 5^3 173 -> 130.  Over 2500 heads of 16 - 4000 rois, 2^3 - 8^3 cells, 16 - 256 channels
+  // and up to 64 x 128 x 128 voxels 1.20 times as fast in geometric mean (1.05 below 800 pairs of a brick and 16 channels, 1.42 from 4096 on), one in
+  // twenty-five slower by more than a tenth.  (The small ones stay for their values too: box by box, zero times an infinity reaches the whole box.)
   // Gradients that fill a wavefront's ring: hardly any of the next roi's comes in beside the present one's products, so that long lists take twice
   // as long as others.  500 such heads (8^3 cells), box by box / here: below two rois for five bricks 1.30 (from 4096 wavefronts on) to 0.90 (below
   // 800), up to five for four 1.05 from 2048 wavefronts on and 0.76 - 0.95 below, beyond 0.80 - 0.87 ([4,128,48,60,21] with 3808 rois 1215 and 1946 us).
