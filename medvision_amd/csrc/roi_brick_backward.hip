@@ -192,17 +192,24 @@ __global__ __launch_bounds__(kBrickThreads) void roi_brick_lists_kernel(const ui
 // The operands of the products are fp16 numbers.  In the ordinary form the weights Wy Wx and the sums P are rounded to them once (11 bits) and Wz is
 // two numbers side by side in K.  Where the first product's K has room, below eight rows of cells, rows stand in it twice, the second time with
 // what the rounding left of their weights.  Wy Wx is scaled by kBrickWeight, so that P of small gradients is not a subnormal number of a few bits.
-// In the form with all bits (22 of them) Wy Wx, P and Wz are all two numbers, what is left of a weight in products of its own; the first number of
-// P is scaled down to 1 / 128 (64 cells of the type's largest fit), its rest up again, and Wz by what makes the products' sum the result.  It is
-// for rois whose gradients the kernel that adds box by box works out in fp32 (brick_exact), and for bricks whose sums overflow in the ordinary form
-// (|P| > 16376).
+// In the form with all bits (22 of them) Wy Wx, P and Wz are all two numbers, what is left of a weight in products of its own.  It is for rois whose
+// gradients the kernel that adds box by box works out in fp32 (brick_exact): P is kept four times as large and its rest 256 times, so that gradients
+// of 1e-5 lose nothing.  Bricks whose sums overflow with that or in the ordinary form (|P| > 16376) have the form too: the first number of P is scaled
+// down to 1 / 128 (64 cells of the type's largest fit), its rest up to 16.  Wz is scaled by what makes the products' sum the result.
 // Error against 64 bits (2.07e-4 of it the result's own rounding) here and box by box, 200 rois of up to 12 voxels: four rows 2.93e-4 and 3.61e-4,
 // seven 3.53e-4 and 3.62e-4, eight 3.59e-4 and 3.60e-4; 100 rois of 16 - 24 voxels: 2.07e-4 with all bits (3.5e-4 without) and 2.07e-4; gradients of
-// 1e-5 2.24e-3 (own 2.15e-3) and 3.02e-3.
+// 1e-5 2.24e-3 (own 2.15e-3) and 3.02e-3, on 100 rois of 16 - 24 voxels 8.27e-3 both, all of it the result's own (8.32e-3 with the scales for large sums).
 // Backward pass of 4000 rois x 256 channels x 7^3: 500 us (box by box 795); with P as two numbers for all rois, so that no values need a second time,
 // 555, and 1000 rois of 4^3 x 128 98 and 115 (box by box 151).  Gradients of 4000 throughout, where all bricks do: 1.6 ms.  100 rois of 16 - 24 voxels
-// x 128 x 7^3: 220 us with all bits, 135 without, 399 box by box.
-constexpr float kBrickWeight = 4.f, kBrickExactWeight = 16.f;
+// x 128 x 7^3: 220 us with all bits, 125 without, 403 box by box.
+constexpr float kBrickWeight = 4.f;
+// The form with all bits: factors of Wy Wx, of the first number of P from what these give, back to that, and of Wz for the two numbers
+struct BrickScales {
+  float weight, down, up, value, rest;
+  __device__ __forceinline__ explicit BrickScales(const bool large)
+      : weight(large ? 16.f : 256.f), down(large ? 1.f / 2048 : 1.f / 64), up(large ? 2048.f : 64.f), value(large ? 128.f : 1.f / 4),
+        rest(large ? 1.f / 16 : 1.f / 256) {}
+};
 typedef _Float16 brick_half4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ brick_half4 brick_pack(const float (&w)[4]) {
   return __builtin_bit_cast(brick_half4, uint2{Mfma<__half>::pack2(w[0], w[1]), Mfma<__half>::pack2(w[2], w[3])});
@@ -227,13 +234,12 @@ __device__ __forceinline__ u32x4 brick_sums(const float4_t &part) {
   const brick_half4 sums = brick_pack(v);
   return brick_pair(sums, sums);
 }
-__device__ __forceinline__ u32x4 brick_sums_exact(const float4_t &part) {
-  constexpr float kDown = 1.f / (128.f * kBrickExactWeight);
-  const float v[4] = {part[0] * kDown, part[1] * kDown, part[2] * kDown, part[3] * kDown};
+__device__ __forceinline__ u32x4 brick_sums_exact(const float4_t &part, const BrickScales &scales) {
+  const float v[4] = {part[0] * scales.down, part[1] * scales.down, part[2] * scales.down, part[3] * scales.down};
   brick_half4 high = brick_pack(v), rest;
   asm("" : "+v"(high));   // (or the compiler forms it a second time, element by element, for the rest)
 #pragma unroll
-  for (int r = 0; r < 4; r++) rest[r] = static_cast<_Float16>(__builtin_fmaf(static_cast<float>(high[r]), -1.f / kDown, part[r]));
+  for (int r = 0; r < 4; r++) rest[r] = static_cast<_Float16>(__builtin_fmaf(static_cast<float>(high[r]), -scales.up, part[r]));
   return brick_pair(high, rest);
 }
 
@@ -511,6 +517,7 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
         const BrickLeft left = brick_left(ws, 1.f / kBrickWeight);
         const u32x4 left_both = brick_pair(left.value, left.rest);
         const bool upper = !idle && (e & kBrickUpper) != 0, lower = !idle && (e & kBrickLower) != 0;
+        const BrickScales scales(turn != kBrickAll);
         // Two pairs of rows of voxels, or with all bits (EXACT) one, whose operands take as many registers.  `over`: the roi's last sweep.
         auto sweep = [&](auto k0_, auto exact_, const bool over) {
           constexpr bool EXACT = decltype(exact_)::value;
@@ -518,11 +525,11 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
           unsigned from = at, second = to_second;
           asm volatile("" : "+v"(second));
           const float taken = second == 0 ? -1.f : 0.f;   // the second row is the first again
-          float weight = EXACT ? kBrickExactWeight : kBrickWeight;
+          float weight = EXACT ? scales.weight : kBrickWeight;
           u32x4 right[FORMS][KN][2], left_value{}, left_rest{};   // the second form: what the rounding left of the first
           if constexpr (EXACT) {
             asm volatile("" : "+v"(from), "+v"(weight));   // (nothing below is formed for several sweeps and kept: that takes more registers than there are)
-            const BrickLeft l = brick_left(ws, 128.f), small = brick_left(ws, 1.f / kBrickExactWeight);
+            const BrickLeft l = brick_left(ws, scales.value), small = brick_left(ws, scales.rest);
             left_value = brick_pair(l.value, small.value);
             left_rest = brick_pair(l.rest, small.rest);
           }
@@ -575,7 +582,7 @@ __global__ __launch_bounds__(kWave << LOG_WX, 2) void roi_brick_backward_kernel(
 #pragma unroll
             for (int k = 0; k < KN; k++) {
               if constexpr (EXACT) {
-                const u32x4 sums = brick_sums_exact(part[k]);
+                const u32x4 sums = brick_sums_exact(part[k], scales);
                 acc[i][K0 + k] = M::run16(left_value, sums, M::run16(left_rest, sums, acc[i][K0 + k]));
               } else {
                 acc[i][K0 + k] = M::run16(left_both, brick_sums(part[k]), acc[i][K0 + k]);

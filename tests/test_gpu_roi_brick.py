@@ -245,6 +245,49 @@ def test_large_boxes_keep_their_bits(oracle, size, rois, cells, ratio, low, high
     assert (got - want).norm() <= 1.01 * own + 1e-5 * want.norm()
 
 
+@pytest.mark.parametrize("rois,cells,low,high", [
+    (100, (7, 7, 7), 15, 24),
+    (100, (4, 5, 4), 15, 24),
+    (60, (7, 7, 7), 20, 38),
+])
+def test_large_boxes_keep_the_bits_of_small_gradients(oracle, rois, cells, low, high):
+    """Gradients of 1e-5: the results are subnormal numbers, and what is left of the sums' bits may not show beside their rounding (a tenth of it at
+    the most, half a hundredth of the error; less than half of that allowed)."""
+    from medvision_amd.ops.roi_align_nd import roi_align_3d
+    g = wl.gen(rois + sum(cells) + high)
+    dims = (1, 128, 24, 40, 40)
+    assert bricks_apply(dims, rois, cells)
+    extent = (torch.rand(rois, 3, generator=g) * (high - low) + low).minimum(torch.tensor([40., 40., 24.]))
+    at = torch.rand(rois, 3, generator=g) * (torch.tensor([40., 40., 24.]) - extent)
+    boxes = torch.cat([torch.zeros(rois, 1), at, at + extent], 1)
+    x = torch.zeros(dims, dtype=torch.float16, device=DEV, requires_grad=True)
+    out = roi_align_3d(x, boxes.to(DEV), cells, 1.0, 2, 1)
+    gy = (torch.randn(out.shape, generator=g) * 1e-5).half()
+    want = torch.as_tensor(oracle.roi_align_backward(gy, boxes, dims, 1.0, 2, True, 1, False)).double().reshape(dims)
+    got = torch.autograd.grad(out, x, gy.to(DEV))[0].cpu().double()
+    own = (want.half().double() - want).norm()
+    assert (got - want).norm() <= 1.002 * own
+
+
+def test_long_boxes_of_large_gradients(oracle):
+    """Boxes of all bits whose sums over rows go beyond fp16 (several cells per voxel on two axes, several voxels per cell on the third)."""
+    from medvision_amd.ops.roi_align_nd import roi_align_3d
+    g = wl.gen(41)
+    dims, rois, cells = (1, 128, 40, 24, 40), 12, (7, 7, 7)
+    assert bricks_apply(dims, rois, cells)
+    extent = torch.rand(rois, 3, generator=g) * torch.tensor([1.5, 1.5, 5.0]) + torch.tensor([1.5, 1.5, 33.0])
+    at = torch.rand(rois, 3, generator=g) * (torch.tensor([40., 24., 40.]) - extent)
+    boxes = torch.cat([torch.zeros(rois, 1), at, at + extent], 1)
+    x = torch.zeros(dims, dtype=torch.float16, device=DEV, requires_grad=True)
+    out = roi_align_3d(x, boxes.to(DEV), cells, 1.0, 2, 1)
+    gy = (torch.randn(out.shape, generator=g) * 8000).half()
+    want = torch.as_tensor(oracle.roi_align_backward(gy, boxes, dims, 1.0, 2, True, 1, False)).double().reshape(dims)
+    assert 16376 < want.abs().max() < 65000
+    got = torch.autograd.grad(out, x, gy.to(DEV))[0].cpu().double()
+    own = (want.half().double() - want).norm()
+    assert (got - want).norm() <= 1.01 * own + 1e-5 * want.norm()
+
+
 @pytest.mark.parametrize("images,channels,size,rois", [
     (2, 128, (9, 17, 33), 480),      # eight share a brick, the most
     (4, 80, (40, 33, 8), 130),       # one brick along x: four share it
